@@ -1,0 +1,564 @@
+"""The work that a program built on this framework has it do, as cases that can be timed and compared.
+
+A case is a model with random weights in a runner and ONE pass over it through the public entry points
+(:meth:`ModelRunner.step`, :meth:`Engine.generate`).  Kinds of pass:
+
+``decode``    one new token for every request of a batch whose earlier tokens are in the cache (the tokens are given, as
+              in replay and scoring; the contexts grow by one with every pass, as they do in use)
+``prefill``   one prompt, whole or in portions, up to the logits of its last token; then its pages go back
+``mixed``     a step of continuous batching: single tokens of running requests beside a portion of a new prompt
+``generate``  prompts through the scheduler and the sampler until every request has its new tokens, and then the
+              logits of the generated tokens in one scoring pass
+
+Models: the Llama 3 family's shapes and a small one, and two of the other architectures at the sizes that the benchmark
+gives them: Fanidra (a gated linear memory, differential attention in chunks, convolutions over time) and, in float32,
+Zekalorn (a delta rule, attention with a learned bias, routed experts; in bfloat16 a router's close calls fall either way by
+rounding alone, so that two correct implementations cannot be compared).
+"""
+import math
+import random
+
+import torch
+
+import nanoinfer_amd  # noqa: F401  (registers the architectures)
+from nanoinfer_amd.engine.llm import Engine
+from nanoinfer_amd.engine.runner import ModelRunner, StepEntry
+from nanoinfer_amd.engine.scheduler import EngineConfig
+from nanoinfer_amd.registry import architecture_of
+from nanoinfer_amd.sampling.params import SamplingParams
+from nanoinfer_amd.weights.loader import expected_tensors
+
+F64 = torch.float64
+PAGE = 16
+GROWTH = 3072          # decode passes for which a state has pages and tokens; then its requests start over
+
+
+# ---------------------------------------------------------------- models
+
+def _llama(hidden, layers, heads, kv_heads, head_dim, inter, vocab, factor, original, positions, tied):
+    return {"architectures": ["LlamaForCausalLM"], "model_type": "llama", "hidden_size": hidden, "num_hidden_layers": layers,
+            "num_attention_heads": heads, "num_key_value_heads": kv_heads, "head_dim": head_dim, "intermediate_size": inter,
+            "vocab_size": vocab, "rms_norm_eps": 1e-5, "rope_theta": 500000.0,
+            "rope_scaling": {"rope_type": "llama3", "factor": factor, "low_freq_factor": 1.0, "high_freq_factor": 4.0,
+                             "original_max_position_embeddings": original},
+            "max_position_embeddings": positions, "tie_word_embeddings": tied, "hidden_act": "silu"}
+
+
+def _fanidra():
+    memory = {"type": "hgrn2", "mixer": {"heads": 16, "dim": 128, "vdim": 128}}
+    attn = {"type": "attention", "mixer": {"heads": 16, "kv_heads": 4, "dim": 64, "vdim": 128, "scale": 64 ** -0.5, "diff": 0.4,
+                                           "conv": 4, "softcap": 30.0, "mask": {"size": 1024}, "rot": {"base": 500000.0, "dims": 64}}}
+    return {"architecture": "Fanidra", "vocab": 128256, "width": 2048, "embedding": {"scale": 2048 ** 0.5}, "norm": {"eps": 1e-5},
+            "residual_mult": 0.7, "canon": {"taps": 3},
+            "layers": [dict(memory if i % 2 == 0 else attn, mlp={"ff": 8192, "kind": "dense"}) for i in range(8)]}
+
+
+def _zekalorn():
+    delta = {"type": "channel_delta", "mixer": {"heads": 16, "kv_heads": 16, "dim": 128, "vdim": 128, "conv": 4,
+                                                "decay_rank": 64, "gate_rank": 64}}
+    attn = {"type": "attention", "mixer": {"heads": 32, "kv_heads": 8, "dim": 64, "vdim": 64, "scale": 64 ** -0.5,
+                                           "bias_max": 4096.0, "bias_rows": 64, "q_temp": {"coef": 0.1, "every": 1024}}}
+    dense = {"kind": "dense", "ff": 8192}
+    routed = {"kind": "moe", "expert": {"ff": 1024}, "router": {"experts": 16, "top": 4}}
+    pattern = [(delta, dense), (delta, routed), (delta, dense), (attn, routed)]
+    return {"architecture": "Zekalorn", "vocab": 128256, "width": 2048, "max_positions": 12288,
+            "embedding": {"scale": 2048 ** 0.5}, "norm": {"eps": 1e-5}, "token_side": {"dim": 64},
+            "layers": [dict(pattern[i % 4][0], mlp=pattern[i % 4][1]) for i in range(8)]}
+
+
+MODELS = {"llama-1b": lambda: _llama(2048, 16, 32, 8, 64, 8192, 128256, 32.0, 8192, 131072, True),
+          "llama-3b": lambda: _llama(3072, 28, 24, 8, 128, 8192, 128256, 32.0, 8192, 131072, True),
+          "llama-small": lambda: _llama(192, 3, 6, 1, 32, 512, 1000, 4.0, 64, 512, False),
+          "fanidra": _fanidra, "zekalorn": _zekalorn}
+
+# (name ending, mean, standard deviation) of the random weights; the first that fits counts
+RULES = {"llama": (("norm.weight", 1.0, 0.05), ("", 0.0, 0.02)),
+         "Fanidra": ((".norm1", 1.0, 0.1), (".norm2", 1.0, 0.1), ("final.norm", 1.0, 0.1), (".lq1", 0.0, 0.2), (".lk1", 0.0, 0.2),
+                     (".lq2", 0.0, 0.2), (".lk2", 0.0, 0.2), (".f.b", 1.0, 0.5), (".lower", 0.3, 0.05), (".conv", 0.0, 0.4),
+                     (".canon1", 0.0, 0.3), ("embed", 0.0, 0.3), ("norm", 1.0, 0.05), ("", 0.0, 0.05)),
+         "Zekalorn": (("A_log", -1.0, 0.5), ("dt_bias", 0.0, 0.5), (".conv", 0.0, 0.4), ("pos", 0.0, 0.3), ("side.embed", 0.0, 1.0),
+                      (".rel", 0.0, 0.5), ("embed", 0.0, 0.08), ("norm1", 1.0, 0.05), ("norm", 1.0, 0.05), ("", 0.0, 0.05))}
+
+
+def _config(case):
+    return MODELS[case["model"]]()
+
+
+def _spec(cfg):
+    arch = architecture_of(cfg)
+    return arch.build_spec(arch.config_from_dict(cfg))
+
+
+def _weights(case, cfg):
+    """Checkpoint tensors by name, on the GPU: matrices in the compute type, vectors in float32.  A model's weights do not
+    depend on the seed; what a program brings anew, the tokens, does."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    rules = RULES[cfg.get("architecture", "llama")]
+    store = torch.bfloat16 if case["dtype"] == "bfloat16" else torch.float32
+    out = {}
+    for name, shape in expected_tensors(_spec(cfg)).items():
+        mean, std = next((m, s) for end, m, s in rules if name.endswith(end))
+        t = torch.randn(shape, generator=g, device="cuda", dtype=torch.float32).mul_(std).add_(mean)
+        out[name] = t.to(store) if len(shape) > 1 else t
+    return out
+
+
+# ---------------------------------------------------------------- the cases
+
+def listed():
+    return [
+        # the smallest calls: five short prompts through the scheduler and the sampler of a small model
+        {"name": "generate, small model", "kind": "generate", "model": "llama-small", "dtype": "float32", "requests": 5, "longest": 200,
+         "portion": 32, "new": 16, "temperature": 0.8},
+        # one person chatting
+        {"name": "decode, one request", "kind": "decode", "model": "llama-1b", "dtype": "bfloat16", "batch": 1, "context": 700},
+        # a few requests with prompts of two thousand tokens: the benchmark's headline
+        {"name": "decode, 8 requests", "kind": "decode", "model": "llama-1b", "dtype": "bfloat16", "batch": 8, "context": 2200},
+        # a loaded server: many requests of very unequal length
+        {"name": "decode, 64 requests", "kind": "decode", "model": "llama-1b", "dtype": "bfloat16", "batch": 64, "context": 2100},
+        # long documents in the context
+        {"name": "decode, long contexts", "kind": "decode", "model": "llama-1b", "dtype": "bfloat16", "batch": 4, "context": 33000},
+        # a prompt of odd length in one portion
+        {"name": "prefill, 1999 tokens", "kind": "prefill", "model": "llama-1b", "dtype": "bfloat16", "tokens": 1999, "portion": 2048},
+        # continuous batching: running requests beside a portion of a new prompt
+        {"name": "mixed, 31 + 481", "kind": "mixed", "model": "llama-1b", "dtype": "bfloat16", "batch": 31, "context": 1100, "tokens": 481},
+        # the reference's own precision, at the next size of the family, and a prompt in portions
+        {"name": "decode, 3B float32", "kind": "decode", "model": "llama-3b", "dtype": "float32", "batch": 8, "context": 1300},
+        {"name": "prefill, float32", "kind": "prefill", "model": "llama-1b", "dtype": "float32", "tokens": 1700, "portion": 512},
+        # another architecture: a recurrent memory, convolutions, differential attention
+        {"name": "decode, Fanidra", "kind": "decode", "model": "fanidra", "dtype": "bfloat16", "batch": 8, "context": 1500},
+        {"name": "prefill, Fanidra", "kind": "prefill", "model": "fanidra", "dtype": "bfloat16", "tokens": 2045, "portion": 2048},
+        # a delta rule, attention with a bias by distance, routed experts
+        {"name": "prefill, Zekalorn float32", "kind": "prefill", "model": "zekalorn", "dtype": "float32", "tokens": 1500, "portion": 2048},
+    ]
+
+
+def _spread(rng, low, high):
+    """A whole number between ``low`` and ``high``, evenly over its logarithm."""
+    return int(round(math.exp(rng.uniform(math.log(low), math.log(high)))))
+
+
+def draw(rng):
+    kind = rng.choice(("decode", "decode", "prefill", "prefill", "mixed", "generate"))
+    if kind == "generate":
+        return {"kind": kind, "model": "llama-small", "dtype": "float32", "requests": rng.randint(1, 8),
+                "longest": rng.randint(20, 300), "portion": rng.choice((16, 32, 64, 300)), "new": rng.randint(4, 24),
+                "temperature": rng.choice((0.0, 0.8))}
+    model, dtype = rng.choice((("llama-1b", "bfloat16"), ("llama-1b", "bfloat16"), ("llama-1b", "float32"), ("llama-3b", "bfloat16"),
+                               ("llama-3b", "float32"), ("fanidra", "bfloat16"), ("fanidra", "float32"), ("zekalorn", "float32")))
+    if kind == "prefill":
+        return {"kind": kind, "model": model, "dtype": dtype, "tokens": _spread(rng, 40, 700 if model == "llama-3b" and dtype == "float32" else 1700),
+                "portion": rng.choice((256, 512, 2048))}
+    batch = _spread(rng, 1, 64)
+    if kind == "mixed":
+        return {"kind": kind, "model": model, "dtype": dtype, "batch": min(batch, 40), "context": _spread(rng, 100, 1300),
+                "tokens": _spread(rng, 17, 700)}
+    # a batch's contexts together stay under those of the listed cases
+    longest = 7000 if model in ("fanidra", "zekalorn") else 33000
+    return {"kind": kind, "model": model, "dtype": dtype, "batch": batch, "context": _spread(rng, 60, max(300, min(longest, 60000 // batch)))}
+
+
+def _contexts(case):
+    """Tokens in the cache of every request of the batch before the first pass: unequal, the longest as named."""
+    r, c = random.Random(case["batch"] * 100003 + case["context"]), case["context"]
+    return [c] + [r.randint(max(8, c // 2 if case["batch"] <= 8 else c // 12), c) for _ in range(case["batch"] - 1)]
+
+
+def _inputs(case, seed):
+    """Token ids from the seed: uniform over the vocabulary, as the benchmark draws them."""
+    cfg = _config(case)
+    vocab = cfg.get("vocab_size", cfg.get("vocab"))
+    r = random.Random(seed * 7919 + 13)
+
+    def ids(n):
+        return r.choices(range(vocab), k=n)
+
+    if case["kind"] == "generate":
+        longest = case["longest"]
+        return {"prompts": [ids(max(1, longest * (i + 1) // case["requests"] - (3 * i) % 5)) for i in range(case["requests"])]}
+    got = {"prompt": ids(case.get("tokens", 0))}
+    if "batch" in case:
+        got["cached"] = [ids(n) for n in _contexts(case)]
+        got["next"] = ids(case["batch"])
+        got["more"] = ids(GROWTH)
+    return got
+
+
+class State:
+    """What a program keeps between passes: its runner, its requests and the tokens that it feeds them."""
+
+    def __init__(self, case, inputs, runner, engine=None):
+        self.case, self.inputs, self.runner, self.engine = case, inputs, runner, engine
+        self.passes = 0
+
+    def fill(self):
+        """The requests' earlier tokens into the cache, in portions of at most 2,048."""
+        for i, toks in enumerate(self.inputs["cached"]):
+            self.runner.release(i)
+            for at in range(0, len(toks), 2048):
+                self.runner.step([StepEntry(i, toks[at:at + 2048], [])])
+        self.passes = 0
+
+    def singles(self):
+        """One token for every running request."""
+        if self.passes == GROWTH:
+            self.fill()
+        first = self.inputs["next"] if self.passes == 0 else None
+        k, more = self.passes, self.inputs["more"]
+        self.passes += 1
+        return [StepEntry(i, [first[i] if first else more[(k + 37 * i) % GROWTH]], [0]) for i in range(self.case["batch"])]
+
+
+def prepare(case, seed):
+    cfg = _config(case)
+    inputs = _inputs(case, seed)
+    tensors = _weights(case, cfg)
+    if case["kind"] == "generate":
+        tokens = sum(len(p) + 2 * case["new"] + 2 * PAGE for p in inputs["prompts"]) * 2
+        requests = 2 * case["requests"]
+    else:
+        tokens = len(inputs["prompt"]) + 2 * PAGE + sum(len(c) + GROWTH + 2 * PAGE for c in inputs.get("cached", ()))
+        requests = case.get("batch", 0) + 2
+    runner = ModelRunner.from_spec(_spec(cfg), tensors, dtype=case["dtype"], page_size=PAGE, max_tokens=tokens, max_requests=requests)
+    engine = None
+    if case["kind"] == "generate":
+        engine = Engine(config=EngineConfig(dtype=case["dtype"], block_size=PAGE, num_cache_blocks=tokens // PAGE, max_sequences=requests,
+                                            prefill_chunk_size=case["portion"]), runner=runner, ignore_eos=True)
+    state = State(case, inputs, runner, engine)
+    if "cached" in inputs:
+        state.fill()
+    return state
+
+
+def run(state):
+    case, runner, inputs = state.case, state.runner, state.inputs
+    if case["kind"] == "decode":
+        return runner.step(state.singles())
+    if case["kind"] == "mixed":
+        n = case["tokens"]
+        return runner.step(state.singles() + [StepEntry("new", inputs["prompt"], [n - 1])], end=["new"])
+    if case["kind"] == "prefill":
+        toks, portion = inputs["prompt"], case["portion"]
+        for at in range(0, len(toks), portion):
+            part = toks[at:at + portion]
+            last = at + portion >= len(toks)
+            logits = runner.step([StepEntry("prompt", part, [len(part) - 1] if last else [])], end=["prompt"] if last else [])
+        return logits
+    params = SamplingParams(temperature=case["temperature"], seed=7)
+    done = state.engine.generate(inputs["prompts"], max_new_tokens=case["new"], params=params)
+    state.engine.scheduler.clear_finished()
+    scored = runner.step([StepEntry(("score", i), r.prompt + r.tokens[:-1], list(range(len(r.prompt) - 1, len(r.prompt) + case["new"] - 1)))
+                          for i, r in enumerate(done)], end=[("score", i) for i in range(len(done))])
+    return {"tokens": torch.tensor([r.tokens for r in done]), "logits": scored}
+
+
+# ---------------------------------------------------------------- what a pass cannot do without
+
+def _sizes(cfg):
+    """(numbers in the layers' matrices that a token uses, numbers of the layers in all, numbers of the head, per layer with
+    attention: (its score and value channels of all heads, cached numbers a token, chunk of positions or None), numbers of
+    state a request)."""
+    total = used = 0
+    for name, shape in expected_tensors(_spec(cfg)).items():
+        if name in ("embed", "pos", "side.embed", "head", "lm_head.weight", "model.embed_tokens.weight"):
+            continue
+        n = math.prod(shape)
+        total += n
+        used += n // 4 if ".mlp.e" in name else n
+    if "hidden_size" in cfg:
+        attn = [(2 * cfg["num_attention_heads"] * cfg["head_dim"], 2 * cfg["num_key_value_heads"] * cfg["head_dim"], None)] * cfg["num_hidden_layers"]
+        return used, total, cfg["vocab_size"] * cfg["hidden_size"], attn, 0
+    attn, state = [], 0
+    for layer in cfg["layers"]:
+        m = layer["mixer"]
+        if layer["type"] == "attention":
+            maps = 2 if "diff" in m else 1
+            attn.append((maps * m["heads"] * (m["dim"] + m["vdim"]), m["kv_heads"] * (maps * m["dim"] + m["vdim"]), m.get("mask", {}).get("size")))
+        else:
+            state += m["heads"] * m["dim"] * m["vdim"]
+    return used, total, cfg["vocab"] * cfg["width"], attn, state
+
+
+def work(case):
+    cfg = _config(case)
+    el = 2 if case["dtype"] == "bfloat16" else 4
+    used, total, head, attn, state = _sizes(cfg)
+    vocab = cfg.get("vocab_size", cfg.get("vocab"))
+    lengths = []                                   # (tokens before, new tokens, rows of logits) of every request
+    if case["kind"] == "generate":
+        prompts = _inputs(case, 0)["prompts"]
+        lengths = [(0, len(p) + case["new"], case["new"]) for p in prompts]
+    else:
+        if "tokens" in case:
+            lengths.append((0, case["tokens"], 1))
+        lengths += [(c, 1, 1) for c in (_contexts(case) if "batch" in case else [])]
+    tokens, rows = sum(n for _, n, _ in lengths), sum(r for _, _, r in lengths)
+    flops = 2.0 * used * tokens + 2.0 * head * rows
+    size = min(total, used * tokens) * el + head * el + rows * vocab * 4.0
+    for channels, cached, chunk in attn:
+        for before, n, _ in lengths:
+            keys = sum(min(p + 1, p % chunk + 1 if chunk else p + 1) for p in range(before, before + n))
+            flops += 2.0 * channels * keys
+            size += cached * el * (n + (before % chunk if chunk else before))
+    flops += 6.0 * state * tokens
+    size += 8.0 * state * sum(1 if before == 0 else 2 for before, _, _ in lengths) / 2
+    return {"bytes": size, "flops": flops}
+
+
+def tolerance(case):
+    """Measured against :func:`exact`: float32 6e-7 (small model) to 1e-4 (28 layers, where the rotation's angles in float32
+    count), bfloat16 2e-3 (Fanidra) to 2e-2 (16 layers) and 4e-2 (28 layers)."""
+    if case["dtype"] == "float32":
+        return {"rel": 2e-4, "max": 4e-3, "differ": 0.01}
+    return {"rel": 1e-2 if case["model"] == "fanidra" else 3e-2, "max": 0.5, "differ": 0.01}
+
+
+# ---------------------------------------------------------------- the same in 64 bits, in plain torch
+
+def _rms(x, eps):
+    return x / torch.sqrt((x * x).mean(-1, keepdim=True) + eps)
+
+
+def _silu(z):
+    return z * torch.sigmoid(z)
+
+
+def _gelu(z):
+    return 0.5 * z * (1.0 + torch.tanh(math.sqrt(2.0 / math.pi) * (z + 0.044715 * z ** 3)))
+
+
+def _by_rows(fn, x, rows=16384):
+    return torch.cat([fn(x[i:i + rows]) for i in range(0, x.shape[0], rows)])
+
+
+def _attend(q, k, v, scale, bias=None, cap=None, chunk=None):
+    """q [T, H, dk], k [T, G, dk], v [T, G, dv] of one sequence -> [T, H, dv]; ``bias`` [T, H] by distance."""
+    T, H, G = q.shape[0], q.shape[1], k.shape[1]
+    k, v = (t.repeat_interleave(H // G, dim=1).permute(1, 0, 2).contiguous() for t in (k, v))
+    pos, out = torch.arange(T, device=q.device), []
+    for at in range(0, T, 512):
+        here = pos[at:at + 512]
+        first = (at // chunk) * chunk if chunk else 0
+        stop = min(T, at + 512)
+        s = q[at:stop].permute(1, 0, 2) @ k[:, first:stop].transpose(1, 2).contiguous() * scale
+        if cap is not None:
+            s = cap * torch.tanh(s / cap)
+        back = here[:, None] - pos[None, first:stop]
+        if bias is not None:
+            s = s + bias[back.clamp(min=0)].permute(2, 0, 1)
+        seen = back >= 0
+        if chunk:
+            seen &= (here // chunk)[:, None] == (pos // chunk)[None, first:stop]
+        p = torch.softmax(s.masked_fill(~seen, -math.inf), dim=-1)
+        out.append((p @ v[:, first:stop]).permute(1, 0, 2))
+    return torch.cat(out)
+
+
+def _conv(u, taps, spans):
+    """Causal convolution over time of every sequence, one filter a channel: the last tap meets the row itself."""
+    out = torch.zeros_like(u)
+    for a, b in spans:
+        for j in range(taps.shape[1]):
+            back = taps.shape[1] - 1 - j
+            if b - a > back:
+                out[a + back:b] += taps[:, j] * u[a:b - back]
+    return out
+
+
+def _padded(x, spans):
+    """[N, ...] rows of all sequences -> [longest, sequences, ...], zeros behind a sequence's end."""
+    out = x.new_zeros((max(b - a for a, b in spans), len(spans)) + x.shape[1:])
+    for s, (a, b) in enumerate(spans):
+        out[:b - a, s] = x[a:b]
+    return out
+
+
+def _unpadded(x, spans):
+    return torch.cat([x[:b - a, s] for s, (a, b) in enumerate(spans)])
+
+
+def _llama_exact(cfg, get, ids, spans):
+    H, G, hd, eps = cfg["num_attention_heads"], cfg["num_key_value_heads"], cfg["head_dim"], cfg["rms_norm_eps"]
+    sc = cfg["rope_scaling"]
+    f = cfg["rope_theta"] ** (-2.0 * torch.arange(hd // 2, dtype=F64, device="cuda") / hd)
+    wave, orig = 2.0 * math.pi / f, sc["original_max_position_embeddings"]
+    smooth = (orig / wave - sc["low_freq_factor"]) / (sc["high_freq_factor"] - sc["low_freq_factor"])
+    blend = (1.0 - smooth) * f / sc["factor"] + smooth * f
+    f = torch.where(wave >= orig / sc["low_freq_factor"], f / sc["factor"], torch.where(wave > orig / sc["high_freq_factor"], blend, f))
+    pos = torch.cat([torch.arange(b - a, device="cuda") for a, b in spans]).to(F64)
+    cos, sin = torch.cos(pos[:, None] * f)[:, None], torch.sin(pos[:, None] * f)[:, None]
+
+    def turn(t):
+        a, b = t[..., :hd // 2], t[..., hd // 2:]
+        return torch.cat([a * cos - b * sin, b * cos + a * sin], dim=-1)
+
+    x = get("model.embed_tokens.weight")[ids]
+    for i in range(cfg["num_hidden_layers"]):
+        pre = f"model.layers.{i}."
+        n = _rms(x, eps) * get(pre + "input_layernorm.weight")
+        q, k, v = (n @ get(pre + f"self_attn.{p}_proj.weight").t() for p in "qkv")
+        q, k, v = turn(q.view(-1, H, hd)), turn(k.view(-1, G, hd)), v.view(-1, G, hd)
+        y = torch.cat([_attend(q[a:b], k[a:b], v[a:b], hd ** -0.5) for a, b in spans])
+        x = x + y.reshape(-1, H * hd) @ get(pre + "self_attn.o_proj.weight").t()
+        norm, gate, up, down = (get(pre + p) for p in ("post_attention_layernorm.weight", "mlp.gate_proj.weight", "mlp.up_proj.weight",
+                                                       "mlp.down_proj.weight"))
+
+        def ff(r):
+            m = _rms(r, eps) * norm
+            return r + (_silu(m @ gate.t()) * (m @ up.t())) @ down.t()
+        x = _by_rows(ff, x)
+    return _rms(x, eps) * get("model.norm.weight"), get("model.embed_tokens.weight" if cfg["tie_word_embeddings"] else "lm_head.weight")
+
+
+def _fanidra_exact(cfg, get, ids, spans):
+    eps, mult = cfg["norm"]["eps"], cfg["residual_mult"]
+    pos = torch.cat([torch.arange(b - a, device="cuda") for a, b in spans]).to(F64)
+    x = get("embed")[ids] * cfg["embedding"]["scale"]
+    for i, layer in enumerate(cfg["layers"]):
+        pre, m = f"l{i}.", layer["mixer"]
+        h = x + _conv(x, get(pre + "canon1"), spans)
+        if layer["type"] == "attention":
+            H, G, dk, dv = m["heads"], m["kv_heads"], m["dim"], m["vdim"]
+            q, k, v = (_conv(h @ get(f"{pre}mix.{p}").t(), get(f"{pre}mix.{p}.conv"), spans) for p in "qkv")
+            half = m["rot"]["dims"] // 2
+            f = m["rot"]["base"] ** (-torch.arange(half, dtype=F64, device="cuda") / half)
+            cos, sin = torch.cos(pos[:, None] * f)[:, None, None], torch.sin(pos[:, None] * f)[:, None, None]
+
+            def turned(t, heads, norm):
+                t = (_rms(t.view(-1, heads, 2, dk), eps) * get(norm)).clone()
+                a, b = t[..., 0:2 * half:2].clone(), t[..., 1:2 * half:2].clone()
+                t[..., 0:2 * half:2], t[..., 1:2 * half:2] = a * cos - b * sin, b * cos + a * sin
+                return t
+            q, k, v = turned(q, H, pre + "mix.q.norm"), turned(k, G, pre + "mix.k.norm"), v.reshape(-1, G, dv)
+            lam = math.exp(float((get(pre + "mix.lq1") * get(pre + "mix.lk1")).sum())) \
+                - math.exp(float((get(pre + "mix.lq2") * get(pre + "mix.lk2")).sum())) + m["diff"]
+            maps = [torch.cat([_attend(q[a:b, :, j], k[a:b, :, j], v[a:b], m["scale"], cap=m["softcap"], chunk=m["mask"]["size"])
+                               for a, b in spans]) for j in (0, 1)]
+            y = _rms(maps[0] - lam * maps[1], eps) * (1.0 - m["diff"])
+        else:
+            H, dk, dv = m["heads"], m["dim"], m["vdim"]
+            low = get(pre + "mix.lower")
+            gate = low + (1.0 - low) * torch.sigmoid(h @ get(pre + "mix.f").t() + get(pre + "mix.f.b"))
+            q, gate, v = (_padded(t.view(-1, H, dk), spans) for t in (_silu(h @ get(pre + "mix.q").t()), gate, h @ get(pre + "mix.v").t()))
+            S, y = torch.zeros(len(spans), H, dk, dv, dtype=F64, device="cuda"), torch.zeros_like(v)
+            for t in range(v.shape[0]):
+                S.mul_(gate[t][..., None]).add_((1.0 - gate[t])[..., None] * v[t][..., None, :])
+                y[t] = (S * q[t][..., None]).sum(-2)
+            y = _rms(_unpadded(y, spans), eps) * get(pre + "mix.norm")
+        x = x + mult * get(pre + "norm1") * _rms(y.reshape(x.shape[0], -1) @ get(pre + "mix.o").t(), eps)
+        gate, up, down = (get(f"{pre}mlp.{p}") for p in ("gate", "up", "down"))
+        x = _by_rows(lambda r: r + mult * get(pre + "norm2") * _rms((_gelu(r @ gate.t()) * (r @ up.t())) @ down.t(), eps), x)
+    return _rms(x, eps) * get("final.norm"), get("head")
+
+
+def _zekalorn_exact(cfg, get, ids, spans):
+    eps, dim = cfg["norm"]["eps"], cfg["token_side"]["dim"]
+    pos = torch.cat([torch.arange(b - a, device="cuda") for a, b in spans])
+    x = get("embed")[ids] * cfg["embedding"]["scale"] + get("pos")[pos]
+    side = get("side.embed")[ids] if "side.embed" in get.names else None
+    for i, layer in enumerate(cfg["layers"]):
+        pre, m = f"l{i}.", layer["mixer"]
+        n = _rms(x, eps) * get(pre + "norm1")
+        H, G, dk, dv = m["heads"], m["kv_heads"], m["dim"], m["vdim"]
+        q, k, v = (n @ get(f"{pre}mix.{p}").t() for p in "qkv")
+        if layer["type"] == "attention":
+            factor = 1.0 + m["q_temp"]["coef"] * torch.log(((pos + 1) // m["q_temp"]["every"] + 1).to(F64))
+            rel = get(pre + "mix.rel")
+            rows, half = rel.shape[0], rel.shape[0] // 2
+            d = range(max(b - a for a, b in spans))
+            bucket = [j if j < half else min(rows - 1, half + int(math.floor(math.log(j / half) / math.log(m["bias_max"] / half) * (rows - half))))
+                      for j in d]
+            bias = rel[torch.tensor(bucket, device="cuda")]
+            q, k, v = q.view(-1, H, dk) * factor[:, None, None], k.view(-1, G, dk), v.view(-1, G, dv)
+            y = torch.cat([_attend(q[a:b], k[a:b], v[a:b], m["scale"], bias=bias) for a, b in spans])
+        else:
+            q, k, v = (_silu(_conv(t, get(f"{pre}mix.{p}.conv"), spans)) for p, t in zip("qkv", (q, k, v)))
+            q, k, v = q.view(-1, G, dk), k.view(-1, G, dk), v.view(-1, H, dv)
+            q, k = (t / torch.sqrt((t * t).sum(-1, keepdim=True) + 1e-6) for t in (q, k))
+            q, k = (q * dk ** -0.5).repeat_interleave(H // G, 1), k.repeat_interleave(H // G, 1)
+            beta = torch.sigmoid(n @ get(pre + "mix.b").t())
+            wide = (n @ get(pre + "mix.a1").t()) @ get(pre + "mix.a2").t() + get(pre + "mix.dt_bias")
+            decay = torch.exp(-torch.exp(get(pre + "mix.A_log"))[:, None] * torch.nn.functional.softplus(wide, threshold=700.0).view(-1, H, dk))
+            gate = torch.sigmoid((n @ get(pre + "mix.g1").t()) @ get(pre + "mix.g2").t()).view(-1, H, dv)
+            q, k, v, beta, decay = (_padded(t, spans) for t in (q, k, v, beta, decay))
+            S, y = torch.zeros(len(spans), H, dk, dv, dtype=F64, device="cuda"), torch.zeros_like(v)
+            for t in range(v.shape[0]):
+                S.mul_(decay[t][..., None])
+                u = beta[t][..., None] * (v[t] - (S * k[t][..., None]).sum(-2))
+                S.add_(k[t][..., None] * u[..., None, :])
+                y[t] = (S * q[t][..., None]).sum(-2)
+            y = _rms(_unpadded(y, spans), eps) * get(pre + "mix.norm") * gate
+        y = y.reshape(x.shape[0], -1) @ get(pre + "mix.o").t()
+        mlp = layer["mlp"]
+        if mlp["kind"] == "dense":
+            y = y + (_silu(n @ get(pre + "mlp.gate").t()) * (n @ get(pre + "mlp.up").t())) @ get(pre + "mlp.down").t()
+        else:
+            z, chosen = torch.topk(n @ get(pre + "mlp.router").t(), mlp["router"]["top"], dim=-1)
+            mix = torch.softmax(z, dim=-1)
+            for e in range(mlp["router"]["experts"]):
+                row, col = torch.nonzero(chosen == e, as_tuple=True)
+                hid = torch.relu(n[row] @ get(f"{pre}mlp.e{e}.up").t()) ** 2
+                y.index_add_(0, row, mix[row, col][:, None] * (hid @ get(f"{pre}mlp.e{e}.down").t()))
+        x = x + y
+        if side is not None:
+            own = side[:, i * dim:(i + 1) * dim]
+            x = x + _rms((_gelu(x @ get(pre + "side.gate").t()) * own) @ get(pre + "side.proj").t(), eps) * get(pre + "side.norm")
+    return _rms(x, eps) * get("final.norm"), get("head")
+
+
+PLAIN = {"llama": _llama_exact, "Fanidra": _fanidra_exact, "Zekalorn": _zekalorn_exact}
+
+
+class _Get:
+    """A tensor by name in 64 bits, made when it is asked for."""
+
+    def __init__(self, tensors):
+        self.tensors, self.names = tensors, set(tensors)
+
+    def __call__(self, name):
+        return self.tensors[name].to(F64)
+
+
+def _logits(cfg, get, sequences, last):
+    """Logits of the ``last`` last tokens of every sequence, [sequences * last, vocab]."""
+    ids = torch.tensor([t for s in sequences for t in s], device="cuda")
+    spans, at = [], 0
+    for s in sequences:
+        spans.append((at, at + len(s)))
+        at += len(s)
+    x, head = PLAIN[cfg.get("architecture", "llama")](cfg, get, ids, spans)
+    rows = torch.cat([x[b - last:b] for _, b in spans])
+    return rows @ head.t()
+
+
+def _uniform(seed, count):
+    """The engine's number in (0, 1] for a request's draw: a finaliser over its seed and the tokens that it has so far."""
+    m = (1 << 64) - 1
+    x = (seed * 0x9E3779B97F4A7C15 + (count + 1) * 0xD1B54A32D192ED03 + 0x2545F4914F6CDD1D) & m
+    for shift, mul in ((30, 0xBF58476D1CE4E5B9), (27, 0x94D049BB133111EB)):
+        x = ((x ^ (x >> shift)) * mul) & m
+    return (((x ^ (x >> 31)) >> 40) + 1) / float(1 << 24)
+
+
+def exact(case, seed):
+    cfg, inputs = _config(case), _inputs(case, seed)
+    get = _Get(_weights(case, cfg))
+    if case["kind"] == "generate":
+        sequences = [list(p) for p in inputs["prompts"]]
+        for k in range(case["new"]):
+            z = _logits(cfg, get, sequences, 1)
+            if case["temperature"] > 0:
+                mass = torch.softmax(z / case["temperature"], dim=-1).cumsum(-1)
+                ids = (mass < _uniform(7, k) * mass[:, -1:]).sum(-1)
+            else:
+                ids = z.argmax(-1)
+            for s, t in zip(sequences, ids.tolist()):
+                s.append(t)
+        new = case["new"]
+        return {"tokens": torch.tensor([s[-new:] for s in sequences]), "logits": _logits(cfg, get, [s[:-1] for s in sequences], new)}
+    sequences = [c + [t] for c, t in zip(inputs.get("cached", ()), inputs.get("next", ()))]
+    if inputs["prompt"]:
+        sequences.append(inputs["prompt"])
+    if sum(len(s) ** 2 for s in sequences) > 6e8 or sum(map(len, sequences)) > 80000:
+        return None          # over twenty seconds
+    return _logits(cfg, get, sequences, 1)
