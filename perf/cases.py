@@ -108,28 +108,28 @@ def _weights(case, cfg):
 def listed():
     return [
         # the smallest calls: five short prompts through the scheduler and the sampler of a small model
-        {"name": "generate, small model", "kind": "generate", "model": "llama-small", "dtype": "float32", "requests": 5, "longest": 200,
+        {"name": "generate small model", "kind": "generate", "model": "llama-small", "dtype": "float32", "requests": 5, "longest": 200,
          "portion": 32, "new": 16, "temperature": 0.8},
         # one person chatting
-        {"name": "decode, one request", "kind": "decode", "model": "llama-1b", "dtype": "bfloat16", "batch": 1, "context": 700},
+        {"name": "decode one request", "kind": "decode", "model": "llama-1b", "dtype": "bfloat16", "batch": 1, "context": 700},
         # a few requests with prompts of two thousand tokens: the benchmark's headline
-        {"name": "decode, 8 requests", "kind": "decode", "model": "llama-1b", "dtype": "bfloat16", "batch": 8, "context": 2200},
+        {"name": "decode 8 requests", "kind": "decode", "model": "llama-1b", "dtype": "bfloat16", "batch": 8, "context": 2200},
         # a loaded server: many requests of very unequal length
-        {"name": "decode, 64 requests", "kind": "decode", "model": "llama-1b", "dtype": "bfloat16", "batch": 64, "context": 2100},
+        {"name": "decode 64 requests", "kind": "decode", "model": "llama-1b", "dtype": "bfloat16", "batch": 64, "context": 2100},
         # long documents in the context
-        {"name": "decode, long contexts", "kind": "decode", "model": "llama-1b", "dtype": "bfloat16", "batch": 4, "context": 33000},
+        {"name": "decode long contexts", "kind": "decode", "model": "llama-1b", "dtype": "bfloat16", "batch": 4, "context": 33000},
         # a prompt of odd length in one portion
-        {"name": "prefill, 1999 tokens", "kind": "prefill", "model": "llama-1b", "dtype": "bfloat16", "tokens": 1999, "portion": 2048},
+        {"name": "prefill 1999 tokens", "kind": "prefill", "model": "llama-1b", "dtype": "bfloat16", "tokens": 1999, "portion": 2048},
         # continuous batching: running requests beside a portion of a new prompt
-        {"name": "mixed, 31 + 481", "kind": "mixed", "model": "llama-1b", "dtype": "bfloat16", "batch": 31, "context": 1100, "tokens": 481},
+        {"name": "mixed 31 + 481", "kind": "mixed", "model": "llama-1b", "dtype": "bfloat16", "batch": 31, "context": 1100, "tokens": 481},
         # the reference's own precision, at the next size of the family, and a prompt in portions
-        {"name": "decode, 3B float32", "kind": "decode", "model": "llama-3b", "dtype": "float32", "batch": 8, "context": 1300},
-        {"name": "prefill, float32", "kind": "prefill", "model": "llama-1b", "dtype": "float32", "tokens": 1700, "portion": 512},
+        {"name": "decode 3B float32", "kind": "decode", "model": "llama-3b", "dtype": "float32", "batch": 8, "context": 1300},
+        {"name": "prefill float32", "kind": "prefill", "model": "llama-1b", "dtype": "float32", "tokens": 1700, "portion": 512},
         # another architecture: a recurrent memory, convolutions, differential attention
-        {"name": "decode, Fanidra", "kind": "decode", "model": "fanidra", "dtype": "bfloat16", "batch": 8, "context": 1500},
-        {"name": "prefill, Fanidra", "kind": "prefill", "model": "fanidra", "dtype": "bfloat16", "tokens": 2045, "portion": 2048},
+        {"name": "decode Fanidra", "kind": "decode", "model": "fanidra", "dtype": "bfloat16", "batch": 8, "context": 1500},
+        {"name": "prefill Fanidra", "kind": "prefill", "model": "fanidra", "dtype": "bfloat16", "tokens": 2045, "portion": 2048},
         # a delta rule, attention with a bias by distance, routed experts
-        {"name": "prefill, Zekalorn float32", "kind": "prefill", "model": "zekalorn", "dtype": "float32", "tokens": 1500, "portion": 2048},
+        {"name": "prefill Zekalorn float32", "kind": "prefill", "model": "zekalorn", "dtype": "float32", "tokens": 1500, "portion": 2048},
     ]
 
 
