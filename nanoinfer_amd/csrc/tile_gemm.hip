@@ -1,0 +1,285 @@
+// Matrix products of many rows in float32: y[M, N] = x[M, K] . W[N, K]^T, where the time is the time of the matrix
+// cores.
+//
+// gfx950 multiplies float32 operands at 157 TFLOP/s and bfloat16 operands at sixteen times that.  A float32 number is
+// the sum of three bfloat16 numbers (24 bits of significand are three times 8):  x = xh + xm + xl, exactly, with xh cut
+// off x and xm rounded from the rest.  Of the nine products of two such sums the six largest are taken,
+//     xl wh + xh wl + xm wm + xm wh + xh wm + xh wh,
+// each product exact and added up in float32 by the matrix cores; the three left out are below 2^-24 of |x||w|, less than the rounding of one
+// float32 addition.  Six bfloat16 instructions take 3/8 of the time of the float32 ones they replace.
+//
+// A workgroup owns BM rows of x and BN rows of W.  Both come from global memory as float32, BK at a time, wait in
+// registers while the slab before them is multiplied, are taken apart there and written to LDS as three planes side by
+// side; a row of a slab takes 3 * BK * 2 bytes and 16 more, so that the 16-byte reads of any eight neighbouring rows
+// meet all banks.  LDS holds two slabs: one is read by the matrix instructions while the other is written.
+// A matrix whose tiles would leave compute units idle is cut along K into shares, whose float32 sums a second kernel
+// adds in their order.
+//
+// What bounds it is the matrix cores under load: a workgroup alone works at a rate that on 256 units were 1.82 PFLOP/s
+// of bfloat16 products, all of them together reach 1.2 to 1.32 (the library's bfloat16 product of 8,192^3 1.41), as the
+// clock falls.  Measured against the library's float32 product (us): [512, 2048] x [16384, 2048] 271 -> 163, 1,999 rows
+// 936 -> 611 (220 TFLOP/s), 512 rows x [2048, 8192] 135 -> 94.  Tiles: the larger the tile, the fewer reads of LDS and
+// numbers taken apart a product; 256 x 256 runs at 220 TFLOP/s, 128 x 256 at 197, the smaller ones at 165 and fill the
+// chip where there are few rows.
+//
+// Values that are not finite come out as NaN (an infinity less itself has no rest).
+#include "common.h"
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float floatx16_t __attribute__((ext_vector_type(16)));
+
+#define TG_XCDS 8
+
+// Workgroups are dealt to the eight XCDs in turn; this gives each XCD a run of neighbouring tiles, so that the
+// workgroups that read the same rows of W find them in one L2.
+__device__ __forceinline__ int tile_of_block(int id, int total) {
+    const int q = total / TG_XCDS, r = total % TG_XCDS, xcd = id % TG_XCDS, slot = id / TG_XCDS;
+    return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + slot;
+}
+
+// Four float32 numbers as three times four bfloat16 numbers that add up to them.
+__device__ __forceinline__ void split3(const float4 a, uint2& h, uint2& m, uint2& l) {
+    const float v[4] = {a.x, a.y, a.z, a.w};
+    uint32_t hw[2], mw[2], lw[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t u0 = __float_as_uint(v[2 * i]), u1 = __float_as_uint(v[2 * i + 1]);
+        hw[i] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);                 // the upper halves of both
+        const float r0 = v[2 * i] - __uint_as_float(u0 & 0xffff0000u);
+        const float r1 = v[2 * i + 1] - __uint_as_float(u1 & 0xffff0000u);
+        mw[i] = pack_bf16x2(r0, r1);
+        lw[i] = pack_bf16x2(r0 - __uint_as_float(mw[i] << 16), r1 - __uint_as_float(mw[i] & 0xffff0000u));
+    }
+    h = make_uint2(hw[0], hw[1]);
+    m = make_uint2(mw[0], mw[1]);
+    l = make_uint2(lw[0], lw[1]);
+}
+
+// What a workgroup's operands wait for.  AHEAD: the operands of a slab are read from LDS while the slab before is
+// multiplied, in a second set of registers (a product of 32 workgroups 121 -> 113 us); the largest tile has no room for
+// that set and reads them when their slab begins.
+enum { TG_STORE = 0, TG_GATED = 1 };
+
+// EPI TG_STORE: out[share][m][n] (shares > 1: float32 sums of every share).  TG_GATED: W is [gate; up] stacked, N its
+// rows; blocks of 32 columns of a tile come from the two halves in turn, so that a lane holds gate and up of the same
+// output; out[m][n] = act(gate) * up, N / 2 wide.
+template <int BM, int BN, int WM, int WN, bool AHEAD, int EPI>
+__global__ __launch_bounds__(WM * WN * WAVE) void split_gemm_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                    float* __restrict__ out, int M, int N, int K, int kper,
+                                                                    int mtiles, int ntiles, GatedUnit act) {
+    constexpr int THREADS = WM * WN * WAVE;
+    constexpr int BK = 16;
+    constexpr int ROWB = 3 * BK * 2 + 16;               // bytes of a row of a slab
+    constexpr int SLAB = (BM + BN) * ROWB;
+    constexpr int TMB = BM / WM / 32, TNB = BN / WN / 32;
+    constexpr int CPR = BK / 4;                         // chunks of four numbers a row
+    constexpr int CA = BM * CPR / THREADS, CB = BN * CPR / THREADS, CH = CA + CB;
+    static_assert(BM * CPR % THREADS == 0 && BN * CPR % THREADS == 0, "whole chunks a thread");
+    __shared__ __attribute__((aligned(16))) char lds[2 * SLAB];
+
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE;
+    const int t = tile_of_block(blockIdx.x, mtiles * ntiles);
+    const int m0 = (t % mtiles) * BM, nt = t / mtiles;
+    const int share = blockIdx.y;
+    const int kbeg = share * kper, kend = min(K, kbeg + kper);
+    const int half = N / 2;
+
+    const float* src[CH];
+    int dst[CH];
+    const int kc = (tid % CPR) * 4;                     // the same for all chunks of a thread
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const bool isx = c < CA;
+        const int r = (tid + (isx ? c : c - CA) * THREADS) / CPR;
+        if (isx) {
+            src[c] = x + static_cast<size_t>(min(m0 + r, M - 1)) * K;
+            dst[c] = r * ROWB + kc * 2;
+        } else {
+            int n;
+            if constexpr (EPI == TG_GATED) {
+                const int n_out = min(nt * (BN / 2) + (r / 64) * 32 + (r & 31), half - 1);
+                n = ((r >> 5) & 1) * half + n_out;
+            } else {
+                n = min(nt * BN + r, N - 1);
+            }
+            src[c] = w + static_cast<size_t>(n) * K;
+            dst[c] = (BM + r) * ROWB + kc * 2;
+        }
+    }
+    struct Raw { float4 v[CH]; };
+    struct Frags { bf16x8_t a[3][TMB], b[3][TNB]; };
+    auto fetch = [&](Raw& s, int k0) {
+        const int k = k0 + kc < kend ? k0 + kc : kbeg;   // a chunk is inside a share or outside it
+#pragma unroll
+        for (int c = 0; c < CH; ++c) s.v[c] = *reinterpret_cast<const float4*>(src[c] + k);
+    };
+    auto put = [&](const Raw& s, int c, int buf, int k0) {
+        uint2 h, m, l;
+        split3(s.v[c], h, m, l);
+        if (k0 + kc >= kend) h = m = l = make_uint2(0, 0);
+        char* p = lds + buf + dst[c];
+        *reinterpret_cast<uint2*>(p) = h;
+        *reinterpret_cast<uint2*>(p + BK * 2) = m;
+        *reinterpret_cast<uint2*>(p + BK * 4) = l;
+    };
+    const int wm = wave / WN, wn = wave % WN;
+    const int aoff = (wm * (BM / WM) + (lane & 31)) * ROWB + (lane >> 5) * 16;
+    const int boff = (BM + wn * (BN / WN) + (lane & 31)) * ROWB + (lane >> 5) * 16;
+    auto read = [&](Frags& f, int buf) {
+#pragma unroll
+        for (int p = 2; p >= 0; --p) {
+#pragma unroll
+            for (int i = 0; i < TMB; ++i) f.a[p][i] = *reinterpret_cast<const bf16x8_t*>(lds + buf + aoff + 32 * i * ROWB + p * BK * 2);
+#pragma unroll
+            for (int j = 0; j < TNB; ++j) f.b[p][j] = *reinterpret_cast<const bf16x8_t*>(lds + buf + boff + 32 * j * ROWB + p * BK * 2);
+        }
+    };
+    floatx16_t acc[TMB][TNB];
+#pragma unroll
+    for (int i = 0; i < TMB; ++i)
+#pragma unroll
+        for (int j = 0; j < TNB; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+    // one slab: its operands are in registers; the next slab's are read, the one behind that is taken apart and written
+    auto step = [&](int k0, const Frags& now, Frags& next, Raw& raw, int rd, int wr) {
+        if constexpr (AHEAD) read(next, rd);
+        constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};      // the small products first
+#pragma unroll
+        for (int g = 0; g < 6; ++g) {
+#pragma unroll
+            for (int i = 0; i < TMB; ++i)
+#pragma unroll
+                for (int j = 0; j < TNB; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(now.a[PA[g]][i], now.b[PB[g]][j], acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int c = 0; c < CH; ++c)
+                if (c >= g * CH / 6 && c < (g + 1) * CH / 6) put(raw, c, wr, k0 + 2 * BK);
+        }
+        fetch(raw, k0 + 4 * BK);
+        // a matrix instruction occupies its pipe for 32 cycles: room for a read, three vector instructions and a write
+#pragma unroll
+        for (int g = 0; g < 6 * TMB * TNB; ++g) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+            __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+        }
+        __syncthreads();
+    };
+    Raw r0, r1;
+    Frags f0, f1;
+    fetch(r0, kbeg);
+    fetch(r1, kbeg + BK);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) put(r0, c, 0, kbeg);
+    if constexpr (AHEAD) {
+#pragma unroll
+        for (int c = 0; c < CH; ++c) put(r1, c, SLAB, kbeg + BK);
+        fetch(r0, kbeg + 2 * BK);
+        fetch(r1, kbeg + 3 * BK);
+    } else {
+        fetch(r0, kbeg + 2 * BK);
+    }
+    __syncthreads();
+    if constexpr (AHEAD) {
+        read(f0, 0);
+        __syncthreads();
+        for (int k0 = kbeg; k0 < kend; k0 += 2 * BK) {      // (a slab past the end is zeros)
+            step(k0, f0, f1, r0, SLAB, 0);
+            step(k0 + BK, f1, f0, r1, 0, SLAB);
+        }
+    } else {
+        for (int k0 = kbeg; k0 < kend; k0 += 2 * BK) {
+            read(f0, 0);
+            step(k0 - BK, f0, f0, r1, 0, SLAB);
+            read(f0, SLAB);
+            step(k0, f0, f0, r0, 0, 0);
+        }
+    }
+
+    const int cols = EPI == TG_GATED ? half : N;
+    float* base = out + static_cast<size_t>(share) * M * cols;
+#pragma unroll
+    for (int i = 0; i < TMB; ++i) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int m = m0 + wm * (BM / WM) + 32 * i + 8 * (e / 4) + 4 * (lane >> 5) + (e & 3);
+            if (m >= M) continue;
+            if constexpr (EPI == TG_GATED) {
+#pragma unroll
+                for (int j = 0; j < TNB / 2; ++j) {
+                    const int n = nt * (BN / 2) + wn * (BN / WN / 2) + 32 * j + (lane & 31);
+                    if (n < cols) base[static_cast<size_t>(m) * cols + n] = act.value(acc[i][2 * j][e], acc[i][2 * j + 1][e]);
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < TNB; ++j) {
+                    const int n = nt * BN + wn * (BN / WN) + 32 * j + (lane & 31);
+                    if (n < cols) base[static_cast<size_t>(m) * cols + n] = act.plain(acc[i][j][e]);
+                }
+            }
+        }
+    }
+}
+
+// out[i] = the sum of the shares' n numbers, in their order; V at a time (n is a multiple of V).
+template <int V>
+__global__ __launch_bounds__(256) void add_shares_kernel(const float* __restrict__ parts, float* __restrict__ out, size_t n, int shares,
+                                                         GatedUnit act) {
+    const size_t i = (static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x) * V;
+    if (i >= n) return;
+    float s[V], v[V];
+    VecIO<float, V>::load(parts + i, s);
+    for (int p = 1; p < shares; ++p) {
+        VecIO<float, V>::load(parts + static_cast<size_t>(p) * n + i, v);
+#pragma unroll
+        for (int j = 0; j < V; ++j) s[j] += v[j];
+    }
+#pragma unroll
+    for (int j = 0; j < V; ++j) s[j] = act.plain(s[j]);
+    VecIO<float, V>::store(out + i, s);
+}
+
+template <int BM, int BN, int WM, int WN, bool AHEAD>
+static int launch_split(const float* x, const float* w, float* out, float* parts, int M, int N, int K, int shares, int kper, int epi,
+                        GatedUnit act, hipStream_t stream) {
+    const int cols = epi == TG_GATED ? N / 2 : N, per = epi == TG_GATED ? BN / 2 : BN;
+    const int mt = (M + BM - 1) / BM, nt = (cols + per - 1) / per;
+    const dim3 grid(mt * nt, shares);
+    if (epi == TG_GATED) {
+        auto kernel = split_gemm_kernel<BM, BN, WM, WN, AHEAD, TG_GATED>;
+        kernel<<<grid, WM * WN * WAVE, 0, stream>>>(x, w, out, M, N, K, K, mt, nt, act);
+    } else {
+        auto kernel = split_gemm_kernel<BM, BN, WM, WN, AHEAD, TG_STORE>;
+        GatedUnit none;
+        kernel<<<grid, WM * WN * WAVE, 0, stream>>>(x, w, shares > 1 ? parts : out, M, N, K, kper, mt, nt, shares > 1 ? none : act);
+        if (shares > 1) {
+            const size_t n = static_cast<size_t>(M) * N;
+            if (n % 4 == 0) add_shares_kernel<4><<<static_cast<unsigned>((n / 4 + 255) / 256), 256, 0, stream>>>(parts, out, n, shares, act);
+            else add_shares_kernel<1><<<static_cast<unsigned>((n + 255) / 256), 256, 0, stream>>>(parts, out, n, shares, act);
+        }
+    }
+    return NI_LAUNCH_RESULT();
+}
+
+// tile: 0 = 64 x 64, 1 = 128 x 128, 2 = 128 x 256, 3 = 256 x 256 (rows of x, rows of W)
+NI_EXPORT int ni_split_gemm(const void* x, const void* w, void* out, void* parts, int M, int N, int K, int tile, int shares, int kper,
+                            int gated, int activation, int squared, void* stream) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 4 || shares < 1 || (shares > 1 && (gated || !parts || kper <= 0 || kper % 16 || static_cast<long>(shares - 1) * kper >= K)) || (gated && N % 2))
+        return static_cast<int>(hipErrorInvalidValue);
+    GatedUnit act = GatedUnit::of(activation);
+    act.squared = squared != 0;
+    const float *xf = static_cast<const float*>(x), *wf = static_cast<const float*>(w);
+    float *of = static_cast<float*>(out), *pf = static_cast<float*>(parts);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (shares == 1) kper = K;
+    switch (tile) {
+        case 0: return launch_split<64, 256, 1, 4, true>(xf, wf, of, pf, M, N, K, shares, kper, gated, act, s);
+        case 1: return launch_split<128, 128, 2, 2, true>(xf, wf, of, pf, M, N, K, shares, kper, gated, act, s);
+        case 2: return launch_split<128, 256, 2, 4, true>(xf, wf, of, pf, M, N, K, shares, kper, gated, act, s);
+        case 3: return launch_split<256, 256, 2, 4, false>(xf, wf, of, pf, M, N, K, shares, kper, gated, act, s);
+        default: return static_cast<int>(hipErrorInvalidValue);
+    }
+}

@@ -1151,6 +1151,8 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
         if out is None:
             out = torch.empty(x.shape[0], rows.shape[0], dtype=out_dtype, device=x.device)
         return skinny_gemm(x, weight, out)
+    if split_wins(x, rows) and out_dtype == torch.float32:
+        return split_gemm(x, rows, out)
     rows_t = weight.rows_t if isinstance(weight, Weight) else rows.t()
     global _library_calls
     _library_calls += 1
@@ -1177,6 +1179,13 @@ def linear_swiglu(x, weight_gate_up, activation: str = "silu") -> torch.Tensor:
     if isinstance(x, NormedInput) or (skinny_wins(x.shape[0], x.shape[1], x.dtype, weight_gate_up)
                                       and (x.shape[0] <= SKINNY_BEST_ROWS or inter % 16 == 0)):
         return skinny_gemm(x, weight_gate_up, out, swiglu=True, activation=activation)
+    rows, _ = _rows_and_tiles(weight_gate_up)
+    if split_wins(x, rows):
+        M, N, K = x.shape[0], 2 * inter, x.shape[1]
+        # in one kernel, or cut along K with the SwiGLU kernel behind it (which moves 12 bytes an output at 4 TB/s)
+        if split_plan(M, N, K, True)[2] <= split_plan(M, N, K)[2] + 4.0 + 12.0 * M * inter / 4e6:
+            return split_gemm(x, rows, out, gated=activation)
+        return swiglu(split_gemm(x, rows), out, activation)
     global _library_calls
     _library_calls += 1
     rows_t = weight_gate_up.rows_t if isinstance(weight_gate_up, Weight) else weight_gate_up.t()
@@ -1189,6 +1198,9 @@ def linear_relu2(x, weight) -> torch.Tensor:
     if skinny_wins(x.shape[0], x.shape[1], x.dtype, weight):
         out = torch.empty(x.shape[0], weight.shape[0], dtype=x.dtype, device=x.device)
         return skinny_gemm(x, weight, out, activation="relu2")
+    rows, _ = _rows_and_tiles(weight)
+    if split_wins(x, rows):
+        return split_gemm(x, rows, squared=True)
     return experts_act(linear(x, weight), None, weight.shape[0], "relu2")
 
 
@@ -1201,6 +1213,8 @@ def require_gpu() -> torch.device:
 torch.backends.cuda.matmul.allow_tf32 = False
 torch.backends.cudnn.allow_tf32 = False
 
+# products of many rows on the matrix cores
+from .tile import split_gemm, split_plan, split_wins, tile_lib  # noqa: E402,F401
 # sums onto the residual stream, routed experts, the gated delta rule, attention with a bias by distance
 from .stream import (BIAS_ATTENTION_MFMA_FROM, DELTA_RUN_FROM, EXPERTS_FEW_ROWS, add_rmsnormed, add_vector,  # noqa: E402,F401
                      bias_attention, bias_attention_lib, bias_attention_mfma, bias_attention_mfma_rows, bias_attention_rows, bias_attention_runs, bias_attention_bf16_tokens, bias_attention_token_runs, delta_rule, delta_rule_lib, embed_scaled, experts_act, experts_few,

@@ -1,0 +1,81 @@
+"""Python face of the kernels in ``csrc/tile_gemm.hip``: products of many rows on the matrix cores, and the rules by
+which a product goes there, how it is cut into tiles and shares, and where the library's product stays."""
+from __future__ import annotations
+
+import ctypes
+import functools
+from typing import Optional, Tuple
+
+import torch
+
+from ..csrc import build as _build
+from . import GATED_ACTIVATIONS, KernelError, _check, _gpu, _load, _ptr, _stream
+
+COMPUTE_UNITS = 256
+
+# Tiles of the float32 product: rows of x, rows of W, workgroups a compute unit holds, and the microseconds that 16
+# elements of K take a workgroup when every unit is full and when it is alone (the matrix cores lower their clock under
+# load).  Fitted to sweeps of 65 to 2,048 rows over the layer sizes of the 1B, 3B and 8B shapes, where the plan that
+# :func:`split_plan` takes is within 4 % of the best of all tiles and shares.
+SPLIT_TILES = ((64, 256, 2, 1.67, 0.76), (128, 128, 2, 1.48, 0.66), (128, 256, 1, 1.36, 0.88), (256, 256, 1, 2.38, 1.64))
+
+
+def tile_lib() -> ctypes.CDLL:
+    return _load(_build.TILE_GEMM)
+
+
+def _split_cost(M: int, N: int, K: int, tile: int, shares: int) -> float:
+    """Microseconds of a float32 product with this tile and this many shares, by the figures above; the kernel that adds
+    the shares moves them at 4 TB/s."""
+    bm, bn, held, loaded, alone = SPLIT_TILES[tile]
+    full, rest = divmod(-(-M // bm) * -(-N // bn) * shares, COMPUTE_UNITS * held)
+    steps = -(-K // (16 * shares))
+    cost = 7.0 + full * loaded * steps + (alone + (loaded - alone) * rest / (COMPUTE_UNITS * held)) * steps * (rest > 0)
+    return cost + (3.5 + (shares + 1) * M * N * 4 / 4e6 if shares > 1 else 0.0)
+
+
+@functools.lru_cache(maxsize=4096)
+def split_plan(M: int, N: int, K: int, gated: bool = False) -> Tuple[int, int, float]:
+    """(tile, shares, estimated microseconds).  ``gated``: the product whose epilogue makes gate and up one output, which
+    is not cut along K."""
+    cost, tile, shares = min((_split_cost(M, N, K, t, s), t, s) for t in range(len(SPLIT_TILES))
+                             for s in ((1,) if gated else range(1, 17)) if s == 1 or K // s >= 128)
+    return tile, shares, cost
+
+
+def split_wins(x: torch.Tensor, rows: torch.Tensor) -> bool:
+    """Whether ``x . rows^T`` goes to the float32 product of :func:`split_gemm`: more rows than the skinny product takes
+    and work enough to pay for its start (some 8 us from the first load to the first matrix instruction).  Measured in
+    recorded launches against the library's float32 product (us, library : this): 512 rows on [16384, 2048] 243 : 163,
+    on [2048, 8192] 135 : 94, on [3072, 2048] 58 : 46, on [2048, 2048] 39 : 38; 164 rows on [3072, 3072] 42 : 39, on
+    [3072, 2048] 28 : 30, on [2048, 2048] 20 : 26: the line lies at 2.2 GFLOP."""
+    M, K = x.shape
+    return (x.dtype == torch.float32 and M > 64 and K % 4 == 0 and 2.0 * M * rows.shape[0] * K >= 2.2e9 and x.is_contiguous()
+            and rows.is_contiguous() and x.data_ptr() % 16 == 0 and rows.data_ptr() % 16 == 0)
+
+
+def split_gemm(x: torch.Tensor, rows: torch.Tensor, out: Optional[torch.Tensor] = None, gated: Optional[str] = None, squared: bool = False,
+               plan: Optional[Tuple[int, int]] = None) -> torch.Tensor:
+    """``x . rows^T`` for float32 ``x`` [M, K] and ``rows`` [N, K] by six bfloat16 products of the operands' three parts
+    (against 64 bits 0.9 times the error of the library's float32 product, less with shares).  ``gated``: an activation's
+    name; ``rows`` is [gate; up] stacked and the result ``act(gate) * up`` [M, N / 2].  ``squared``: ``relu(.)^2``.
+    ``plan``: another (tile, shares) than :func:`split_plan`'s."""
+    M, K = x.shape
+    N = rows.shape[0]
+    _gpu(x, "x", torch.float32)
+    _gpu(rows, "w", torch.float32, (N, K))
+    if gated is not None and (N % 2 or squared):
+        raise KernelError("a gated product takes a stacked matrix and no other activation")
+    cols = N if gated is None else N // 2
+    if out is None:
+        out = torch.empty(M, cols, dtype=torch.float32, device=x.device)
+    _gpu(out, "out", torch.float32, (M, cols))
+    if K % 4 or x.data_ptr() % 16 or rows.data_ptr() % 16:
+        raise KernelError(f"rows of {K} float32 elements at this address are not aligned to 16 bytes")
+    tile, shares = plan or split_plan(M, N, K, gated is not None)[:2]
+    per = -(-K // (16 * shares)) * 16
+    shares = -(-K // per)                                   # no share is empty
+    parts = torch.empty(shares, M, N, dtype=torch.float32, device=x.device) if shares > 1 else None
+    _check(tile_lib().ni_split_gemm(_ptr(x), _ptr(rows), _ptr(out), _ptr(parts), M, N, K, tile, shares, per, int(gated is not None),
+                                    GATED_ACTIVATIONS[gated or "silu"], int(squared), _stream()), "split_gemm")
+    return out

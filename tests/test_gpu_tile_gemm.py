@@ -1,0 +1,90 @@
+"""The products of many rows (``csrc/tile_gemm.hip``) alone: every tile at its edges, every epilogue, shares, and the
+error beside the library's float32 product."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def K():
+    from nanoinfer_amd import kernels
+    return kernels
+
+
+def operands(M, N, Kd, seed=0, spread=0):
+    g = torch.Generator().manual_seed(seed)
+    x, w = torch.randn(M, Kd, generator=g), torch.randn(N, Kd, generator=g)
+    if spread:      # rows of very different size: powers of two, so that the sums' relative errors stay what they are
+        x *= 2.0 ** torch.randint(-spread, spread + 1, (M, 1), generator=g)
+    return x.cuda(), w.cuda()
+
+
+def close(got, x, w):
+    """Every number within the bound of a float32 sum of 6 K exact products: (6 K + 8) roundings of at most 2^-24 of
+    sum |x||w| each (the three products left out are below one of them)."""
+    want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    assert bool(((got.double() - want).abs() <= (6 * x.shape[1] + 8) * 2.0 ** -24 * size).all())
+    return float((got.double() - want).norm() / want.norm())
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("M,N,Kd,shares", [(1, 1, 4, 1), (63, 255, 20, 1), (64, 256, 16, 1), (65, 257, 36, 1), (129, 130, 100, 1),
+                                           (257, 513, 132, 1), (300, 258, 300, 2), (70, 77, 1036, 3), (256, 128, 2048, 16)])
+def test_split_gemm_at_the_edges_of_its_tiles(K, tile, M, N, Kd, shares):
+    x, w = operands(M, N, Kd, seed=M + N + Kd, spread=30)
+    out = torch.full((M + 1, N), 7.0, device="cuda")
+    K.split_gemm(x, w, out[:M], plan=(tile, shares))
+    close(out[:M], x, w)
+    assert bool((out[M] == 7.0).all())                       # nothing behind the last row
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("M,inter", [(65, 1), (64, 32), (130, 100), (129, 129), (257, 300)])
+def test_split_gemm_gated_and_squared(K, tile, M, inter):
+    x, w = operands(M, 2 * inter, 68, seed=inter)
+    z = K.split_gemm(x, w, plan=(tile, 1))
+    for act in ("silu", "gelu_tanh"):
+        # the epilogue applies what the kernel of its own applies to the same float32 sums
+        got = K.split_gemm(x, w, gated=act, plan=(tile, 1))
+        assert torch.allclose(got, K.swiglu(z, torch.empty_like(got), act), rtol=1e-6, atol=0)
+    assert torch.equal(K.split_gemm(x, w, squared=True, plan=(tile, 1)), torch.relu(z) ** 2)
+    assert torch.equal(K.split_gemm(x, w, squared=True, plan=(tile, 2)), torch.relu(K.split_gemm(x, w, plan=(tile, 2))) ** 2)
+
+
+@pytest.mark.parametrize("M,N,Kd", [(65, 16384, 2048), (512, 2048, 8192), (512, 3072, 3072), (1000, 2500, 700)])
+def test_products_of_many_float32_rows_are_no_less_exact_than_the_librarys(K, M, N, Kd):
+    x, w = operands(M, N, Kd)
+    assert K.split_wins(x, w)
+    calls = K.library_calls()
+    ours = close(K.linear(x, w), x, w)
+    assert K.library_calls() == calls
+    assert ours <= 1.05 * close(torch.mm(x, w.t()), x, w)     # measured 0.6 to 0.9
+    g = K.linear_swiglu(x, w)
+    want = torch.nn.functional.silu(x.double() @ w[:N // 2].double().t()) * (x.double() @ w[N // 2:].double().t())
+    assert float((g.double() - want).norm() / want.norm()) <= 1e-5
+    assert K.library_calls() == calls
+
+
+def test_rows_that_are_not_finite_stay_so_and_touch_no_other(K):
+    x, w = operands(130, 300, 64)
+    x[3, 5], x[70, 0], x[129, 63] = float("inf"), float("nan"), float("-inf")
+    got = K.split_gemm(x, w)
+    bad = torch.zeros(130, dtype=torch.bool)
+    bad[[3, 70, 129]] = True
+    assert not bool(torch.isfinite(got[bad.cuda()]).any())
+    close(got[~bad.cuda()], x[~bad.cuda()], w)
+
+
+def test_what_split_gemm_does_not_take(K):
+    x, w = operands(70, 64, 64)
+    for bad in (lambda: K.split_gemm(x[:, :62].contiguous(), w[:, :62].contiguous()), lambda: K.split_gemm(x.bfloat16(), w.bfloat16()),
+                lambda: K.split_gemm(x, w[:, :60].contiguous()), lambda: K.split_gemm(x.view(-1)[1:1 + 69 * 64].view(69, 64), w),
+                lambda: K.split_gemm(x, w[:63], gated="silu"), lambda: K.split_gemm(x.t(), w)):
+        with pytest.raises(K.KernelError):
+            bad()
+    big, wide = operands(600, 1024, 2048)
+    calls = K.library_calls()                                 # rows that are no whole run of memory, or not aligned: the library's product
+    assert K.linear(big.t().contiguous().t(), wide).shape == (600, 1024)
+    assert K.linear(torch.randn(600 * 2048 + 1, device="cuda")[1:].view(600, 2048), wide).shape == (600, 1024)
+    assert K.library_calls() == calls + 2
