@@ -63,10 +63,23 @@ enum { TG_STORE = 0, TG_GATED = 1 };
 // EPI TG_STORE: out[share][m][n] (shares > 1: float32 sums of every share).  TG_GATED: W is [gate; up] stacked, N its
 // rows; blocks of 32 columns of a tile come from the two halves in turn, so that a lane holds gate and up of the same
 // output; out[m][n] = act(gate) * up, N / 2 wide.
-template <int BM, int BN, int WM, int WN, bool AHEAD, int EPI>
+//
+// GROUPED: the rows of x belong to groups (the tokens of one expert each), every group has N rows of W of its own.  The
+// rows of group e stand at the places offsets[e] .. offsets[e + 1] - 1; place p takes row rows[p] of x (rows null: row p).
+// No tile spans two groups.  How many tiles the groups need is known on the device alone: the grid is the most that so
+// many rows in so many groups can need, and a workgroup without a tile ends at once.
+struct Groups {
+    const int32_t* offsets;      // [count + 1]
+    const int32_t* rows;         // [places], or null
+    int count;
+    size_t wstride;              // numbers from one group's rows of W to the next group's
+    int ldw;                     // numbers from one row of W to the next
+};
+
+template <int BM, int BN, int WM, int WN, bool AHEAD, int EPI, bool GROUPED>
 __global__ __launch_bounds__(WM * WN * WAVE) void split_gemm_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                     float* __restrict__ out, int M, int N, int K, int kper,
-                                                                    int mtiles, int ntiles, GatedUnit act) {
+                                                                    int mtiles, int ntiles, GatedUnit act, Groups groups) {
     constexpr int THREADS = WM * WN * WAVE;
     constexpr int BK = 16;
     constexpr int ROWB = 3 * BK * 2 + 16;               // bytes of a row of a slab
@@ -79,7 +92,23 @@ __global__ __launch_bounds__(WM * WN * WAVE) void split_gemm_kernel(const float*
 
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE;
     const int t = tile_of_block(blockIdx.x, mtiles * ntiles);
-    const int m0 = (t % mtiles) * BM, nt = t / mtiles;
+    int m0 = (t % mtiles) * BM, ldw = K;
+    const int nt = t / mtiles;
+    if constexpr (GROUPED) {
+        int tile = t % mtiles, e = 0, begin = 0, end = 0;
+        for (; e < groups.count; ++e) {
+            begin = groups.offsets[e];
+            end = groups.offsets[e + 1];
+            const int tiles = (end - begin + BM - 1) / BM;
+            if (tile < tiles) break;
+            tile -= tiles;
+        }
+        if (e == groups.count) return;
+        m0 = begin + tile * BM;
+        M = end;                                        // the last place of this group and one
+        w += e * groups.wstride;
+        ldw = groups.ldw;
+    }
     const int share = blockIdx.y;
     const int kbeg = share * kper, kend = min(K, kbeg + kper);
     const int half = N / 2;
@@ -92,7 +121,10 @@ __global__ __launch_bounds__(WM * WN * WAVE) void split_gemm_kernel(const float*
         const bool isx = c < CA;
         const int r = (tid + (isx ? c : c - CA) * THREADS) / CPR;
         if (isx) {
-            src[c] = x + static_cast<size_t>(min(m0 + r, M - 1)) * K;
+            int row = min(m0 + r, M - 1);
+            if constexpr (GROUPED)
+                if (groups.rows) row = groups.rows[row];
+            src[c] = x + static_cast<size_t>(row) * K;
             dst[c] = r * ROWB + kc * 2;
         } else {
             int n;
@@ -102,7 +134,7 @@ __global__ __launch_bounds__(WM * WN * WAVE) void split_gemm_kernel(const float*
             } else {
                 n = min(nt * BN + r, N - 1);
             }
-            src[c] = w + static_cast<size_t>(n) * K;
+            src[c] = w + static_cast<size_t>(n) * ldw;
             dst[c] = (BM + r) * ROWB + kc * 2;
         }
     }
@@ -249,12 +281,12 @@ static int launch_split(const float* x, const float* w, float* out, float* parts
     const int mt = (M + BM - 1) / BM, nt = (cols + per - 1) / per;
     const dim3 grid(mt * nt, shares);
     if (epi == TG_GATED) {
-        auto kernel = split_gemm_kernel<BM, BN, WM, WN, AHEAD, TG_GATED>;
-        kernel<<<grid, WM * WN * WAVE, 0, stream>>>(x, w, out, M, N, K, K, mt, nt, act);
+        auto kernel = split_gemm_kernel<BM, BN, WM, WN, AHEAD, TG_GATED, false>;
+        kernel<<<grid, WM * WN * WAVE, 0, stream>>>(x, w, out, M, N, K, K, mt, nt, act, Groups{});
     } else {
-        auto kernel = split_gemm_kernel<BM, BN, WM, WN, AHEAD, TG_STORE>;
+        auto kernel = split_gemm_kernel<BM, BN, WM, WN, AHEAD, TG_STORE, false>;
         GatedUnit none;
-        kernel<<<grid, WM * WN * WAVE, 0, stream>>>(x, w, shares > 1 ? parts : out, M, N, K, kper, mt, nt, shares > 1 ? none : act);
+        kernel<<<grid, WM * WN * WAVE, 0, stream>>>(x, w, shares > 1 ? parts : out, M, N, K, kper, mt, nt, shares > 1 ? none : act, Groups{});
         if (shares > 1) {
             const size_t n = static_cast<size_t>(M) * N;
             if (n % 4 == 0) add_shares_kernel<4><<<static_cast<unsigned>((n / 4 + 255) / 256), 256, 0, stream>>>(parts, out, n, shares, act);
@@ -280,6 +312,112 @@ NI_EXPORT int ni_split_gemm(const void* x, const void* w, void* out, void* parts
         case 1: return launch_split<128, 128, 2, 2, true>(xf, wf, of, pf, M, N, K, shares, kper, gated, act, s);
         case 2: return launch_split<128, 256, 2, 4, true>(xf, wf, of, pf, M, N, K, shares, kper, gated, act, s);
         case 3: return launch_split<256, 256, 2, 4, false>(xf, wf, of, pf, M, N, K, shares, kper, gated, act, s);
+        default: return static_cast<int>(hipErrorInvalidValue);
+    }
+}
+
+// ---------------------------------------------------------------- routed experts, every token with its own experts alone
+// Every token has `top` entries (expert, weight).  The lists put the entries in the order of their experts, and an
+// expert's entries in the order of the tokens: one workgroup an expert counts the entries of the experts before its own
+// and then sets down its own, both in one order for all runs.  An entry that names no expert below E (an expert without
+// matrices) stands in no list, its place is -1.
+#define LIST_THREADS 1024
+__global__ __launch_bounds__(LIST_THREADS) void expert_lists_kernel(const int32_t* __restrict__ chosen, const float* __restrict__ mix,
+                                                                    int entries, int top, int E, int32_t* __restrict__ offsets,
+                                                                    int32_t* __restrict__ rows, float* __restrict__ weights,
+                                                                    int32_t* __restrict__ place) {
+    constexpr int NW = LIST_THREADS / WAVE;
+    __shared__ int counts[NW];
+    const int e = blockIdx.x, lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+    int before = 0;
+    for (int i = threadIdx.x; i < entries; i += LIST_THREADS) {
+        const int c = chosen[i];
+        before += c >= 0 && c < e;
+        if (e == 0 && (c < 0 || c >= E)) place[i] = -1;
+    }
+    __shared__ float scratch[16];
+    int at = static_cast<int>(block_sum(static_cast<float>(before), scratch));      // whole numbers below 2^24
+    if (threadIdx.x == 0) offsets[e] = at;
+    for (int i0 = 0; i0 < entries; i0 += LIST_THREADS) {
+        const int i = i0 + threadIdx.x;
+        const bool mine = i < entries && chosen[i] == e;
+        const unsigned long long votes = __ballot(mine);
+        __syncthreads();
+        if (lane == 0) counts[wave] = __popcll(votes);
+        __syncthreads();
+        int ahead = 0, all = 0;
+#pragma unroll
+        for (int v = 0; v < NW; ++v) {
+            ahead += v < wave ? counts[v] : 0;
+            all += counts[v];
+        }
+        if (mine) {
+            const int p = at + ahead + __popcll(votes & ((1ull << lane) - 1));
+            rows[p] = i / top;
+            weights[p] = mix[i];
+            place[i] = p;
+        }
+        at += all;
+    }
+    if (e == E - 1 && threadIdx.x == 0) offsets[E] = at;
+}
+
+// out[t, :] = the sum of what a token's entries gave, in the order of its entries
+template <int V>
+__global__ __launch_bounds__(256) void gather_entries_kernel(const float* __restrict__ y, const int32_t* __restrict__ place,
+                                                             float* __restrict__ out, int d, int top) {
+    const int t = blockIdx.x, c = (blockIdx.y * 256 + threadIdx.x) * V;
+    if (c >= d) return;
+    float s[V], v[V];
+#pragma unroll
+    for (int j = 0; j < V; ++j) s[j] = 0.f;
+    for (int k = 0; k < top; ++k) {
+        const int p = place[t * top + k];
+        if (p < 0) continue;
+        VecIO<float, V>::load(y + static_cast<size_t>(p) * d + c, v);
+#pragma unroll
+        for (int j = 0; j < V; ++j) s[j] += v[j];
+    }
+    VecIO<float, V>::store(out + static_cast<size_t>(t) * d + c, s);
+}
+
+NI_EXPORT int ni_expert_lists(const void* chosen, const void* mix, int T, int top, int E, void* offsets, void* rows, void* weights, void* place,
+                              void* stream) {
+    if (T <= 0 || top <= 0 || E <= 0 || static_cast<long>(T) * top >= (1 << 24)) return static_cast<int>(hipErrorInvalidValue);
+    expert_lists_kernel<<<E, LIST_THREADS, 0, static_cast<hipStream_t>(stream)>>>((const int32_t*)chosen, (const float*)mix, T * top, top, E,
+                                                                                  (int32_t*)offsets, (int32_t*)rows, (float*)weights, (int32_t*)place);
+    return NI_LAUNCH_RESULT();
+}
+
+NI_EXPORT int ni_gather_entries(const void* y, const void* place, void* out, int T, int d, int top, void* stream) {
+    if (T <= 0 || d <= 0 || top <= 0) return static_cast<int>(hipErrorInvalidValue);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (d % 4 == 0) gather_entries_kernel<4><<<dim3(T, (d / 4 + 255) / 256), 256, 0, s>>>((const float*)y, (const int32_t*)place, (float*)out, d, top);
+    else gather_entries_kernel<1><<<dim3(T, (d + 255) / 256), 256, 0, s>>>((const float*)y, (const int32_t*)place, (float*)out, d, top);
+    return NI_LAUNCH_RESULT();
+}
+
+template <int BM, int BN, int WM, int WN, bool AHEAD>
+static int launch_grouped(const float* x, const float* w, float* out, int places, int N, int K, const Groups& groups, hipStream_t stream) {
+    const int mt = places / BM + groups.count, nt = (N + BN - 1) / BN;      // at most: sum of ceil(rows / BM)
+    split_gemm_kernel<BM, BN, WM, WN, AHEAD, TG_STORE, true><<<dim3(mt * nt, 1), WM * WN * WAVE, 0, stream>>>(x, w, out, places, N, K, K, mt, nt,
+                                                                                                       GatedUnit{}, groups);
+    return NI_LAUNCH_RESULT();
+}
+
+// out[p, n] = x[rows[p], :] . W[group of p][n, :] for every place p of the groups' lists
+NI_EXPORT int ni_split_gemm_grouped(const void* x, const void* w, void* out, int places, int N, int K, const void* offsets, const void* rows,
+                                    int count, size_t wstride, int ldw, int tile, void* stream) {
+    if (places <= 0 || N <= 0 || K <= 0 || K % 4 || ldw < K || ldw % 4 || wstride % 4 || count <= 0) return static_cast<int>(hipErrorInvalidValue);
+    const Groups g{static_cast<const int32_t*>(offsets), static_cast<const int32_t*>(rows), count, wstride, ldw};
+    const float *xf = static_cast<const float*>(x), *wf = static_cast<const float*>(w);
+    float* of = static_cast<float*>(out);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    switch (tile) {
+        case 0: return launch_grouped<64, 256, 1, 4, true>(xf, wf, of, places, N, K, g, s);
+        case 1: return launch_grouped<128, 128, 2, 2, true>(xf, wf, of, places, N, K, g, s);
+        case 2: return launch_grouped<128, 256, 2, 4, true>(xf, wf, of, places, N, K, g, s);
+        case 3: return launch_grouped<256, 256, 2, 4, false>(xf, wf, of, places, N, K, g, s);
         default: return static_cast<int>(hipErrorInvalidValue);
     }
 }

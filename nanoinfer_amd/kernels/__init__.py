@@ -1214,7 +1214,7 @@ torch.backends.cuda.matmul.allow_tf32 = False
 torch.backends.cudnn.allow_tf32 = False
 
 # products of many rows on the matrix cores
-from .tile import split_gemm, split_plan, split_wins, tile_lib  # noqa: E402,F401
+from .tile import experts_grouped, experts_grouped_wins, split_gemm, split_plan, split_wins, tile_lib  # noqa: E402,F401
 # sums onto the residual stream, routed experts, the gated delta rule, attention with a bias by distance
 from .stream import (BIAS_ATTENTION_MFMA_FROM, DELTA_RUN_FROM, EXPERTS_FEW_ROWS, add_rmsnormed, add_vector,  # noqa: E402,F401
                      bias_attention, bias_attention_lib, bias_attention_mfma, bias_attention_mfma_rows, bias_attention_rows, bias_attention_runs, bias_attention_bf16_tokens, bias_attention_token_runs, delta_rule, delta_rule_lib, embed_scaled, experts_act, experts_few,

@@ -424,9 +424,9 @@ class RoutedExperts(Part):
     correction [experts + identity] (absent: none): added to the scores that choose the experts and the groups, never to the weights.
 
     The experts' matrices are laid side by side, up [E * ff, d] (gated: [E * 2 ff, d], an expert's gate rows and then
-    its up rows) and down [d, E * ff].  For a few rows only the chosen experts' rows are read; for many, all experts
-    run as two dense products with the mix of an expert that was not chosen at zero, which the matrix cores do
-    faster than a gather would here.  With a shared expert, and in steps of many rows with identity experts, the result is
+    its up rows) and down [d, E * ff].  For a few rows only the chosen experts' rows are read.  For many rows in float32 every
+    expert multiplies its own tokens' rows where that is estimated to be faster (``K.experts_grouped_wins``); else all experts
+    run as two dense products with the mix of an expert that was not chosen at zero.  With a shared expert, and in steps of many rows with identity experts, the result is
     two or three float32 addends [n, T, d], which the next norm sums in float32."""
 
     graph_safe = True
@@ -492,6 +492,12 @@ class RoutedExperts(Part):
         if few:
             y = K.experts_few(x, self.w_up.rows, self.w_down.rows, chosen, mix, self.ff, self.activation, None if out is None else out[0],
                               limit=self.limit, slope=self.slope)
+        elif K.experts_grouped_wins(x, self.w_up.rows, self.w_down.rows, self.top, self.E):
+            y = K.experts_grouped(x, self.w_up.rows, self.w_down.rows, chosen, mix, self.E,
+                                  lambda up, weights: K.experts_act(up, weights, self.ff, self.activation, self.limit, self.slope),
+                                  out=None if out is None else out[0])
+            if self.identity:
+                K.identity_experts(x, mix_all, self.E, out[more])
         else:
             act = K.experts_act(K.linear(x, self.w_up), mix_all, self.ff, self.activation, self.limit, self.slope)
             y = K.linear(act, self.w_down, out_dtype=torch.float32, out=None if out is None else out[0])

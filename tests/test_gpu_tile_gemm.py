@@ -88,3 +88,33 @@ def test_what_split_gemm_does_not_take(K):
     assert K.linear(big.t().contiguous().t(), wide).shape == (600, 1024)
     assert K.linear(torch.randn(600 * 2048 + 1, device="cuda")[1:].view(600, 2048), wide).shape == (600, 1024)
     assert K.library_calls() == calls + 2
+
+
+@pytest.mark.parametrize("T,d,ff,E,top,kind", [(1, 4, 4, 1, 1, "any"), (65, 36, 20, 5, 2, "any"), (300, 64, 132, 16, 4, "any"), (257, 68, 64, 7, 3, "one"),
+                                               (130, 40, 36, 6, 2, "identity"), (1500, 128, 64, 16, 4, "any")])
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+def test_every_expert_multiplies_its_own_tokens(K, monkeypatch, tile, T, d, ff, E, top, kind):
+    """Lists of every shape (an expert without tokens, one with all, entries that name no expert), whole against 64 bits."""
+    from nanoinfer_amd.kernels import tile as tiles
+    monkeypatch.setattr(tiles, "_grouped_plan", lambda *a: (0.0, tile))
+    g = torch.Generator().manual_seed(T + d)
+    x, up, down = torch.randn(T, d, generator=g), torch.randn(E * ff, d, generator=g), torch.randn(d, E * ff, generator=g)
+    total = E + (3 if kind == "identity" else 0)
+    chosen = torch.stack([torch.randperm(total, generator=g)[:top] for _ in range(T)]).int()
+    if kind == "one":                  # one expert has every token, the last has none
+        chosen[:, 0] = 2
+        chosen[:, 1:] = torch.tensor([0, 4])
+    mix = torch.rand(T, top, generator=g)
+    want, size = torch.zeros(T, d, dtype=torch.float64), torch.zeros(T, d, dtype=torch.float64)
+    for t in range(T):
+        for k in range(top):
+            e = int(chosen[t, k])
+            if e < E:
+                u, n = up[e * ff:(e + 1) * ff].double(), down[:, e * ff:(e + 1) * ff].double()
+                hid = mix[t, k].double() * torch.relu(u @ x[t].double()) ** 2
+                want[t] += n @ hid
+                size[t] += n.abs() @ (mix[t, k].double() * (u.abs() @ x[t].double().abs()) ** 2)
+    got = K.experts_grouped(x.cuda(), up.cuda(), down.cuda(), chosen.cuda(), mix.cuda(), E,
+                            lambda z, w: K.experts_act(z, w, ff, "relu2")).cpu().double()
+    # two products and a square, each a float32 sum: (2 (6 d + 8) + (6 ff + 8) + top + 4) roundings of the sums of sizes
+    assert bool(((got - want).abs() <= (12 * d + 6 * ff + 28 + top) * 2.0 ** -24 * size + 1e-30).all())
