@@ -27,6 +27,8 @@
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx16_t __attribute__((ext_vector_type(16)));
+typedef float floatx4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 #define TG_XCDS 8
 
@@ -257,8 +259,8 @@ __global__ __launch_bounds__(WM * WN * WAVE) void split_gemm_kernel(const float*
 }
 
 // out[i] = the sum of the shares' n numbers, in their order; V at a time (n is a multiple of V).
-template <int V>
-__global__ __launch_bounds__(256) void add_shares_kernel(const float* __restrict__ parts, float* __restrict__ out, size_t n, int shares,
+template <typename T, int V>
+__global__ __launch_bounds__(256) void add_shares_kernel(const float* __restrict__ parts, T* __restrict__ out, size_t n, int shares,
                                                          GatedUnit act) {
     const size_t i = (static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x) * V;
     if (i >= n) return;
@@ -271,11 +273,11 @@ __global__ __launch_bounds__(256) void add_shares_kernel(const float* __restrict
     }
 #pragma unroll
     for (int j = 0; j < V; ++j) s[j] = act.plain(s[j]);
-    VecIO<float, V>::store(out + i, s);
+    VecIO<T, V>::store(out + i, s);
 }
 
 template <int BM, int BN, int WM, int WN, bool AHEAD>
-static int launch_split(const float* x, const float* w, float* out, float* parts, int M, int N, int K, int shares, int kper, int epi,
+static int launch_split(const float* x, const float* w, float* out, int M, int N, int K, int shares, int kper, int epi,
                         GatedUnit act, hipStream_t stream) {
     const int cols = epi == TG_GATED ? N / 2 : N, per = epi == TG_GATED ? BN / 2 : BN;
     const int mt = (M + BM - 1) / BM, nt = (cols + per - 1) / per;
@@ -285,35 +287,235 @@ static int launch_split(const float* x, const float* w, float* out, float* parts
         kernel<<<grid, WM * WN * WAVE, 0, stream>>>(x, w, out, M, N, K, K, mt, nt, act, Groups{});
     } else {
         auto kernel = split_gemm_kernel<BM, BN, WM, WN, AHEAD, TG_STORE, false>;
-        GatedUnit none;
-        kernel<<<grid, WM * WN * WAVE, 0, stream>>>(x, w, shares > 1 ? parts : out, M, N, K, kper, mt, nt, shares > 1 ? none : act, Groups{});
-        if (shares > 1) {
-            const size_t n = static_cast<size_t>(M) * N;
-            if (n % 4 == 0) add_shares_kernel<4><<<static_cast<unsigned>((n / 4 + 255) / 256), 256, 0, stream>>>(parts, out, n, shares, act);
-            else add_shares_kernel<1><<<static_cast<unsigned>((n + 255) / 256), 256, 0, stream>>>(parts, out, n, shares, act);
-        }
+        kernel<<<grid, WM * WN * WAVE, 0, stream>>>(x, w, out, M, N, K, kper, mt, nt, act, Groups{});
     }
     return NI_LAUNCH_RESULT();
 }
 
-// tile: 0 = 64 x 64, 1 = 128 x 128, 2 = 128 x 256, 3 = 256 x 256 (rows of x, rows of W)
-NI_EXPORT int ni_split_gemm(const void* x, const void* w, void* out, void* parts, int M, int N, int K, int tile, int shares, int kper,
+// tile: 0 = 64 x 256, 1 = 128 x 128, 2 = 128 x 256, 3 = 256 x 256 (rows of x, rows of W).  shares > 1: `out` takes the sums of every
+// share of kper columns
+NI_EXPORT int ni_split_gemm(const void* x, const void* w, void* out, int M, int N, int K, int tile, int shares, int kper,
                             int gated, int activation, int squared, void* stream) {
-    if (M <= 0 || N <= 0 || K <= 0 || K % 4 || shares < 1 || (shares > 1 && (gated || !parts || kper <= 0 || kper % 16 || static_cast<long>(shares - 1) * kper >= K)) || (gated && N % 2))
+    if (M <= 0 || N <= 0 || K <= 0 || K % 4 || shares < 1 || (shares > 1 && (gated || squared || kper <= 0 || kper % 16 || static_cast<long>(shares - 1) * kper >= K)) || (gated && N % 2))
         return static_cast<int>(hipErrorInvalidValue);
     GatedUnit act = GatedUnit::of(activation);
     act.squared = squared != 0;
     const float *xf = static_cast<const float*>(x), *wf = static_cast<const float*>(w);
-    float *of = static_cast<float*>(out), *pf = static_cast<float*>(parts);
+    float* of = static_cast<float*>(out);
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (shares == 1) kper = K;
     switch (tile) {
-        case 0: return launch_split<64, 256, 1, 4, true>(xf, wf, of, pf, M, N, K, shares, kper, gated, act, s);
-        case 1: return launch_split<128, 128, 2, 2, true>(xf, wf, of, pf, M, N, K, shares, kper, gated, act, s);
-        case 2: return launch_split<128, 256, 2, 4, true>(xf, wf, of, pf, M, N, K, shares, kper, gated, act, s);
-        case 3: return launch_split<256, 256, 2, 4, false>(xf, wf, of, pf, M, N, K, shares, kper, gated, act, s);
+        case 0: return launch_split<64, 256, 1, 4, true>(xf, wf, of, M, N, K, shares, kper, gated, act, s);
+        case 1: return launch_split<128, 128, 2, 2, true>(xf, wf, of, M, N, K, shares, kper, gated, act, s);
+        case 2: return launch_split<128, 256, 2, 4, true>(xf, wf, of, M, N, K, shares, kper, gated, act, s);
+        case 3: return launch_split<256, 256, 2, 4, false>(xf, wf, of, M, N, K, shares, kper, gated, act, s);
         default: return static_cast<int>(hipErrorInvalidValue);
     }
+}
+
+// ---------------------------------------------------------------- bfloat16, 65 and more rows, the re-tiled matrix
+// y[M, N] = x[M, K] . W[N, K]^T with W in the order in which the products of decode steps stream it ([tile of 16
+// rows][piece of 64 columns][lane][32 bytes]): a lane's 32 bytes of a piece are two operands of
+// v_mfma_f32_16x16x32_bf16, so W goes from memory into registers and never through LDS.  Only x does: LDS is what a
+// product with both operands there runs out of (a 256 x 256 tile of such a kernel kept the matrix cores busy 52 % of
+// the time with LDS at 46 % of its cycles and its barriers between).
+//
+// A workgroup is WN wavefronts side by side, each with TN tiles of W of its own and all BM rows of x; nothing of W is
+// loaded twice in a workgroup.  x comes in slabs of 64 columns, three of them in LDS: one is multiplied, the next is
+// complete, the third is written from registers that were loaded a slab earlier.  A half piece (32 columns) of W is
+// loaded two halves before its turn, into the registers of the half before: three sets take turns.  Behind the
+// products of each 16 rows of x their operand of the next half is read, so that reads of LDS run beside the products
+// all the time and no operand is held twice.  W is the A operand: a lane then has four neighbouring columns of a row
+// of y and stores them at once.
+//
+// Measured (us; the library's product, with SwiGLU its kernel too : this): 512 rows on [16384, 2048] with SwiGLU
+// 41.5 : 35.3, on [2048, 8192] 29.4 : 25.5, on [3072, 2048] 14.6 : 15.1, on [2048, 2048] 12.0 : 11.9; 128 rows
+// 21 : 16.5, 18.5 : 12.4, 12.8 : 8.3, 9.4 : 6.4.  Raising a wavefront's priority while it multiplies (s_setprio) was
+// worth 39.6 -> 34.2.  Past 512 rows (1,024 with SwiGLU) the library's 256 x 256 tiles are ahead (1.27 PFLOP/s at 2,048 rows
+// against 1.06).
+template <int N> struct Num { static constexpr int value = N; };
+
+template <int WN, int TM, int TN, int MINW, int EPI, typename OUT>
+__global__ __launch_bounds__(WN * WAVE, MINW) void tiled_gemm_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                                                                    OUT* __restrict__ out, int M, int N, int K, int per,
+                                                                    int mtiles, int ntiles, GatedUnit act) {
+    constexpr int THREADS = WN * WAVE, BM = TM * 16, BNT = WN * TN;      // BNT: tiles of W a workgroup
+    constexpr int ROWB = 128 + 16, SLAB = BM * ROWB;
+    constexpr int CX = BM * 8 / THREADS;
+    __shared__ __attribute__((aligned(16))) char lds[3 * SLAB];
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE;
+    const int t = tile_of_block(blockIdx.x, mtiles * ntiles);
+    const int m0 = (t % mtiles) * BM, nt = t / mtiles, share = blockIdx.y;
+    const int pieces = K / 64, pbeg = share * per, pend = min(pieces, pbeg + per);
+    const auto xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(x), 0, M * K * 2, 0x00020000);
+    // x: 16 bytes a thread and chunk, eight neighbouring threads a row
+    int xsrc[CX], xdst[CX];
+#pragma unroll
+    for (int c = 0; c < CX; ++c) {
+        const int i = tid + c * THREADS, r = i >> 3;
+        xsrc[c] = min(m0 + r, M - 1) * K * 2 + (i & 7) * 16;
+        xdst[c] = r * ROWB + (i & 7) * 16;
+    }
+    // W: tile, piece, lane, 32 bytes
+    const int all = (N + 15) / 16;
+    int wt[TN];                  // bytes from the start of W
+    const auto wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(w), 0, all * pieces * 2048, 0x00020000);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        int n;
+        if constexpr (EPI == TG_GATED) {       // the first half of a wave's tiles are gate rows, the other half the up rows of the same outputs
+            const int o = min(nt * (BNT / 2) + wave * (TN / 2) + j % (TN > 1 ? TN / 2 : 1), all / 2 - 1);
+            n = (j / (TN > 1 ? TN / 2 : 1)) * (all / 2) + o;
+        } else {
+            n = min(nt * BNT + wave * TN + j, all - 1);
+        }
+        wt[j] = (n * pieces * 64 + lane) * 32;
+    }
+    const int xoff = (lane & 15) * ROWB + (lane >> 4) * 32;
+    u32x4_t xs[CX], wreg[3][TN];
+    bf16x8_t xf[TM];
+    floatx4_t acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    auto fetch = [&](int p) {
+        const int at = min(p, pend - 1) * 128;
+#pragma unroll
+        for (int c = 0; c < CX; ++c) xs[c] = __builtin_amdgcn_raw_buffer_load_b128(xr, xsrc[c], at, 0);
+    };
+    auto put = [&](int buf) {
+#pragma unroll
+        for (int c = 0; c < CX; ++c) *reinterpret_cast<u32x4_t*>(lds + buf + xdst[c]) = xs[c];
+    };
+    auto weights = [&](u32x4_t (&r)[TN], int h) {        // half h of the share: piece pbeg + h / 2
+        const int at = min(pbeg + (h >> 1), pend - 1) * 2048 + (h & 1) * 16;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) r[j] = __builtin_amdgcn_raw_buffer_load_b128(wr, wt[j], at, 0);
+    };
+    auto read = [&](int i, int buf, int half) {
+        xf[i] = *reinterpret_cast<const bf16x8_t*>(lds + buf + xoff + i * 16 * ROWB + half * 16);
+    };
+    fetch(pbeg);
+    weights(wreg[0], 0);
+    weights(wreg[1], 1);
+    put(0);
+    fetch(pbeg + 1);
+    put(SLAB);
+    fetch(pbeg + 2);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < TM; ++i) read(i, 0, 0);
+    // half a piece: its operands are in registers; the next half's rows of x are read behind each row of tiles
+    auto half = [&](const u32x4_t (&now)[TN], u32x4_t (&ahead)[TN], int h, int buf, int which) {
+        weights(ahead, h + 2);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, now[j]), xf[i], acc[i][j], 0, 0, 0);
+            read(i, buf, which);
+        }
+        __builtin_amdgcn_s_setprio(0);
+    };
+    // three pieces a turn: three slabs of x and three half pieces of W take turns
+    auto piece = [&](auto B, int p) {
+        constexpr int b = decltype(B)::value;                 // p % 3 counted from the share's first piece
+        constexpr int h = 2 * b % 3;
+        const int at = 2 * (p - pbeg);
+        put((b + 2) % 3 * SLAB);
+        fetch(p + 3);
+        half(wreg[h], wreg[(h + 2) % 3], at, b * SLAB, 1);
+        half(wreg[(h + 1) % 3], wreg[h], at + 1, (b + 1) % 3 * SLAB, 0);
+        __syncthreads();
+    };
+
+    int p = pbeg;
+    for (; p + 3 <= pend; p += 3) {
+        piece(Num<0>{}, p);
+        piece(Num<1>{}, p + 1);
+        piece(Num<2>{}, p + 2);
+    }
+    if (p < pend) piece(Num<0>{}, p);
+    if (p + 1 < pend) piece(Num<1>{}, p + 1);
+
+    const int cols = EPI == TG_GATED ? N / 2 : N;
+    OUT* base = out + static_cast<size_t>(share) * M * cols;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const int m = m0 + i * 16 + (lane & 15);
+        if (m >= M) continue;
+        constexpr int OT = EPI == TG_GATED && TN > 1 ? TN / 2 : TN;
+#pragma unroll
+        for (int j = 0; j < OT; ++j) {
+            const int n = (nt * (BNT * OT / TN) + wave * OT + j) * 16 + (lane >> 4) * 4;
+            if (n >= cols) continue;
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = EPI == TG_GATED ? act.rough(acc[i][j][e], acc[i][j + TN - OT][e]) : act.plain(acc[i][j][e]);
+            store_packed<OUT, 4>(base + static_cast<size_t>(m) * cols + n, v);
+        }
+    }
+}
+
+template <int WN, int TM, int TN, int MINW>
+static int launch_tiled(const bf16_t* x, const bf16_t* w, void* out, int M, int N, int K, int shares, int per, int epi, int f32, GatedUnit act,
+                        hipStream_t stream) {
+    constexpr int BM = TM * 16, BNT = WN * TN, T = WN * WAVE;
+    const int tiles = (N + 15) / 16, mt = (M + BM - 1) / BM;
+    if (epi == TG_GATED) {
+        if constexpr (TN > 1) {
+            const int nt = (tiles / 2 + BNT / 2 - 1) / (BNT / 2);
+            tiled_gemm_kernel<WN, TM, TN, MINW, TG_GATED, bf16_t><<<dim3(mt * nt), T, 0, stream>>>(x, w, static_cast<bf16_t*>(out), M, N, K, per, mt, nt, act);
+            return NI_LAUNCH_RESULT();
+        }
+        return static_cast<int>(hipErrorInvalidValue);
+    }
+    const int nt = (tiles + BNT - 1) / BNT;
+    const dim3 grid(mt * nt, shares);
+    if (f32) tiled_gemm_kernel<WN, TM, TN, MINW, TG_STORE, float><<<grid, T, 0, stream>>>(x, w, static_cast<float*>(out), M, N, K, per, mt, nt, act);
+    else tiled_gemm_kernel<WN, TM, TN, MINW, TG_STORE, bf16_t><<<grid, T, 0, stream>>>(x, w, static_cast<bf16_t*>(out), M, N, K, per, mt, nt, act);
+    return NI_LAUNCH_RESULT();
+}
+
+// tile: 0 = 128 x 256, 1 = 128 x 128, 2 = 64 x 128, 3 = 64 x 64 (rows of x, columns of y).  shares > 1: `out` takes float32 sums
+// of every share of `per` pieces; f32: float32 results
+NI_EXPORT int ni_tiled_gemm(const void* x, const void* w, void* out, int M, int N, int K, int tile, int shares, int per, int gated, int f32,
+                            int activation, int squared, void* stream) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 64 || N % 4 || shares < 1 || per < 1 || (shares > 1 && (!f32 || squared)) ||
+        static_cast<long>(shares - 1) * per >= K / 64 || static_cast<long>(shares) * per < K / 64 || (gated && (N % 32 || shares > 1 || f32)) ||
+        static_cast<long>(M) * K >= 1l << 30 || static_cast<long>(N + 15) * K >= 1l << 30)
+        return static_cast<int>(hipErrorInvalidValue);
+    GatedUnit act = GatedUnit::of(activation);
+    act.squared = squared != 0;
+    const bf16_t *xb = static_cast<const bf16_t*>(x), *wb = static_cast<const bf16_t*>(w);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    switch (tile) {
+        case 0: return launch_tiled<8, 8, 2, 2>(xb, wb, out, M, N, K, shares, per, gated, f32, act, s);
+        case 1: return launch_tiled<4, 8, 2, 2>(xb, wb, out, M, N, K, shares, per, gated, f32, act, s);
+        case 2: return launch_tiled<4, 4, 2, 4>(xb, wb, out, M, N, K, shares, per, gated, f32, act, s);
+        case 3: return launch_tiled<4, 4, 1, 4>(xb, wb, out, M, N, K, shares, per, gated, f32, act, s);
+        default: return static_cast<int>(hipErrorInvalidValue);
+    }
+}
+
+// out[i] = (relu of, squared,) the sum of `shares` times n float32 numbers, in their order
+NI_EXPORT int ni_add_shares(const void* parts, void* out, size_t n, int shares, int squared, int dtype, void* stream) {
+    if (n == 0 || shares < 1) return static_cast<int>(hipErrorInvalidValue);
+    GatedUnit act;
+    act.squared = squared != 0;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const unsigned v = n % 4 == 0 ? 4 : 1, blocks = static_cast<unsigned>((n / v + 255) / 256);
+    const float* pf = static_cast<const float*>(parts);
+    if (dtype == 0) {
+        if (v == 4) add_shares_kernel<float, 4><<<blocks, 256, 0, s>>>(pf, static_cast<float*>(out), n, shares, act);
+        else add_shares_kernel<float, 1><<<blocks, 256, 0, s>>>(pf, static_cast<float*>(out), n, shares, act);
+    } else {
+        if (v == 4) add_shares_kernel<bf16_t, 4><<<blocks, 256, 0, s>>>(pf, static_cast<bf16_t*>(out), n, shares, act);
+        else add_shares_kernel<bf16_t, 1><<<blocks, 256, 0, s>>>(pf, static_cast<bf16_t*>(out), n, shares, act);
+    }
+    return NI_LAUNCH_RESULT();
 }
 
 // ---------------------------------------------------------------- routed experts, every token with its own experts alone

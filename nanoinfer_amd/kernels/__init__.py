@@ -2,8 +2,8 @@
 on the host, that operand shapes, types and devices are what each kernel and its grid assume.
 
 There is no fallback: when a library cannot be built or loaded, or a tensor is not on the GPU,
-the call raises.  Matrix products are the one thing taken from a library (``torch.matmul`` ->
-rocBLAS/hipBLASLt), as the reference takes them from cuBLAS (src/op/kernels/cuda/matmul_kernel.cu:76-86).
+the call raises.  Matrix products of many bfloat16 rows are the one thing taken from a library (``torch.matmul`` ->
+rocBLAS/hipBLASLt), as the reference takes its products from cuBLAS (src/op/kernels/cuda/matmul_kernel.cu:76-86).
 """
 from __future__ import annotations
 
@@ -1094,10 +1094,11 @@ def skinny_qkv_rope(x, w_qkv, positions: torch.Tensor, cos: torch.Tensor,
 
 
 def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optional[torch.Tensor] = None,
-           pending: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None, leave: Optional[NormSpec] = None):
+           pending: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None, leave: Optional[NormSpec] = None,
+           addends: bool = False):
     """``x . weight^T`` with ``weight`` stored [out, in].  Few rows go to the hand-written skinny
-    product; many rows to the library (rocBLAS/hipBLASLt), where float32 inputs are multiplied in
-    true float32 (the reduced-precision matrix modes of the library are switched off at import).
+    product, more of them to the tiled products (:func:`tiled_wins`, :func:`split_wins`), the rest to the library
+    (rocBLAS/hipBLASLt; its reduced-precision matrix modes for float32 are switched off at import).
     ``out_dtype`` float32 keeps the float32 accumulators of a bfloat16 product.  ``x`` may be a
     :class:`NormedInput` where :func:`norm_prologue_ok` holds.  With ``residual`` (the float32
     residual stream, where :func:`residual_epilogue_ok` holds) the product is added into it and
@@ -1108,7 +1109,8 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
     output type) instead of a new tensor.  ``leave`` (with ``residual``, where :func:`leaves_scaled_ok`
     holds; ignored elsewhere): the norm that stands behind the stream; the product then runs whole and
     returns a :class:`ScaledInput` for that norm.  ``x`` may itself be a :class:`ScaledInput` where
-    :func:`takes_scaled_ok` holds."""
+    :func:`takes_scaled_ok` holds.  ``addends``: a product of many rows may come back as float32 addends
+    [S, M, N] (its K range cut into S shares), for a norm that adds them to the stream itself."""
     rows, _ = _rows_and_tiles(weight)
     if out is not None and (isinstance(x, (NormedInput, ScaledInput)) or residual is not None):
         raise KernelError("out= goes with a plain product")
@@ -1152,7 +1154,9 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
             out = torch.empty(x.shape[0], rows.shape[0], dtype=out_dtype, device=x.device)
         return skinny_gemm(x, weight, out)
     if split_wins(x, rows) and out_dtype == torch.float32:
-        return split_gemm(x, rows, out)
+        return split_gemm(x, rows, out, addends=addends)
+    if tiled_wins(x, weight) and (out is None or out.data_ptr() % 16 == 0):
+        return tiled_gemm(x, weight, out_dtype, out, addends=addends)
     rows_t = weight.rows_t if isinstance(weight, Weight) else rows.t()
     global _library_calls
     _library_calls += 1
@@ -1186,6 +1190,8 @@ def linear_swiglu(x, weight_gate_up, activation: str = "silu") -> torch.Tensor:
         if split_plan(M, N, K, True)[2] <= split_plan(M, N, K)[2] + 4.0 + 12.0 * M * inter / 4e6:
             return split_gemm(x, rows, out, gated=activation)
         return swiglu(split_gemm(x, rows), out, activation)
+    if tiled_wins(x, weight_gate_up, gated=True):
+        return tiled_gemm(x, weight_gate_up, out=out, gated=activation)
     global _library_calls
     _library_calls += 1
     rows_t = weight_gate_up.rows_t if isinstance(weight_gate_up, Weight) else weight_gate_up.t()
@@ -1201,6 +1207,8 @@ def linear_relu2(x, weight) -> torch.Tensor:
     rows, _ = _rows_and_tiles(weight)
     if split_wins(x, rows):
         return split_gemm(x, rows, squared=True)
+    if tiled_wins(x, weight):
+        return tiled_gemm(x, weight, squared=True)
     return experts_act(linear(x, weight), None, weight.shape[0], "relu2")
 
 
@@ -1214,7 +1222,8 @@ torch.backends.cuda.matmul.allow_tf32 = False
 torch.backends.cudnn.allow_tf32 = False
 
 # products of many rows on the matrix cores
-from .tile import experts_grouped, experts_grouped_wins, split_gemm, split_plan, split_wins, tile_lib  # noqa: E402,F401
+from .tile import (experts_grouped, experts_grouped_wins, split_gemm, split_plan, split_wins, tile_lib, tiled_gemm, tiled_plan,  # noqa: E402,F401
+                   tiled_wins)
 # sums onto the residual stream, routed experts, the gated delta rule, attention with a bias by distance
 from .stream import (BIAS_ATTENTION_MFMA_FROM, DELTA_RUN_FROM, EXPERTS_FEW_ROWS, add_rmsnormed, add_vector,  # noqa: E402,F401
                      bias_attention, bias_attention_lib, bias_attention_mfma, bias_attention_mfma_rows, bias_attention_rows, bias_attention_runs, bias_attention_bf16_tokens, bias_attention_token_runs, delta_rule, delta_rule_lib, embed_scaled, experts_act, experts_few,

@@ -9,7 +9,7 @@ from typing import Optional, Tuple
 import torch
 
 from ..csrc import build as _build
-from . import GATED_ACTIVATIONS, KernelError, _check, _gpu, _load, _ptr, _stream
+from . import GATED_ACTIVATIONS, KernelError, _check, _gpu, _load, _ptr, _stream, dtype_code
 
 COMPUTE_UNITS = 256
 
@@ -56,11 +56,12 @@ def split_wins(x: torch.Tensor, rows: torch.Tensor) -> bool:
 
 
 def split_gemm(x: torch.Tensor, rows: torch.Tensor, out: Optional[torch.Tensor] = None, gated: Optional[str] = None, squared: bool = False,
-               plan: Optional[Tuple[int, int]] = None) -> torch.Tensor:
+               plan: Optional[Tuple[int, int]] = None, addends: bool = False) -> torch.Tensor:
     """``x . rows^T`` for float32 ``x`` [M, K] and ``rows`` [N, K] by six bfloat16 products of the operands' three parts
     (against 64 bits 0.9 times the error of the library's float32 product, less with shares).  ``gated``: an activation's
     name; ``rows`` is [gate; up] stacked and the result ``act(gate) * up`` [M, N / 2].  ``squared``: ``relu(.)^2``.
-    ``plan``: another (tile, shares) than :func:`split_plan`'s."""
+    ``plan``: another (tile, shares) than :func:`split_plan`'s.  ``addends``: where the product is cut along K its shares come
+    back as they are, [shares, M, N], for a norm that adds them."""
     M, K = x.shape
     N = rows.shape[0]
     _gpu(x, "x", torch.float32)
@@ -68,17 +69,111 @@ def split_gemm(x: torch.Tensor, rows: torch.Tensor, out: Optional[torch.Tensor] 
     if gated is not None and (N % 2 or squared):
         raise KernelError("a gated product takes a stacked matrix and no other activation")
     cols = N if gated is None else N // 2
-    if out is None:
-        out = torch.empty(M, cols, dtype=torch.float32, device=x.device)
-    _gpu(out, "out", torch.float32, (M, cols))
     if K % 4 or x.data_ptr() % 16 or rows.data_ptr() % 16:
         raise KernelError(f"rows of {K} float32 elements at this address are not aligned to 16 bytes")
     tile, shares = plan or split_plan(M, N, K, gated is not None)[:2]
     per = -(-K // (16 * shares)) * 16
     shares = -(-K // per)                                   # no share is empty
-    parts = torch.empty(shares, M, N, dtype=torch.float32, device=x.device) if shares > 1 else None
-    _check(tile_lib().ni_split_gemm(_ptr(x), _ptr(rows), _ptr(out), _ptr(parts), M, N, K, tile, shares, per, int(gated is not None),
-                                    GATED_ACTIVATIONS[gated or "silu"], int(squared), _stream()), "split_gemm")
+    if shares > 1:
+        parts = torch.empty(shares, M, N, dtype=torch.float32, device=x.device)
+    elif out is None:
+        out = torch.empty(M, cols, dtype=torch.float32, device=x.device)
+    if out is not None:
+        _gpu(out, "out", torch.float32, (M, cols))
+    _check(tile_lib().ni_split_gemm(_ptr(x), _ptr(rows), _ptr(parts if shares > 1 else out), M, N, K, tile, shares, per, int(gated is not None),
+                                    GATED_ACTIVATIONS[gated or "silu"], int(squared and shares == 1), _stream()), "split_gemm")
+    if shares > 1:
+        return parts if addends else _add_shares(parts, torch.float32, out, squared)
+    return out
+
+
+def _add_shares(parts: torch.Tensor, dtype: torch.dtype, out: Optional[torch.Tensor], squared: bool) -> torch.Tensor:
+    """The shares [S, M, N] of a product added in their order, in ``out`` or a new tensor of that type."""
+    S, M, N = parts.shape
+    if out is None:
+        out = torch.empty(M, N, dtype=dtype, device=parts.device)
+    _check(tile_lib().ni_add_shares(_ptr(parts), _ptr(out), ctypes.c_size_t(M * N), S, int(squared), dtype_code(dtype), _stream()), "add_shares")
+    return out
+
+
+# ---------------------------------------------------------------- bfloat16 on the re-tiled matrix
+
+# As SPLIT_TILES, for 64 columns of K, with the microseconds before the first and behind the last of them.  Fitted to sweeps
+# of 65 to 1,024 rows over the layer sizes of the 1B, 3B and 8B shapes: the plan taken is the best of all tiles and
+# shares or within 6 % of it in four cases of five, within 21 % in all.
+TILED_TILES = ((128, 256, 1, 0.87, 0.57, 7.4), (128, 128, 2, 1.02, 0.23, 5.8), (64, 128, 4, 1.23, 0.13, 4.8), (64, 64, 5, 0.98, 0.11, 4.1))
+
+
+def _tiled_cost(M: int, N: int, K: int, tile: int, shares: int, gated: bool, addends: bool) -> float:
+    bm, bn, held, loaded, alone, fixed = TILED_TILES[tile]
+    full, rest = divmod(-(-M // bm) * -(-N // bn) * shares, COMPUTE_UNITS * held)
+    per = -(-(K // 64) // shares)
+    cost = fixed + full * loaded * per + (alone + (loaded - alone) * rest / (COMPUTE_UNITS * held)) * per * (rest > 0)
+    cost = max(cost + (shares > 1) * shares * M * N * 4 / 8e6, 3.0 + N * K * 2 / 5e6)
+    if shares > 1:      # the shares are read again, by the norm behind them or by a kernel that adds them
+        cost += shares * M * N * 4 / 5e6 + (0.5 if addends else 3.0)
+    return cost
+
+
+@functools.lru_cache(maxsize=4096)
+def tiled_plan(M: int, N: int, K: int, gated: bool = False, addends: bool = False) -> Tuple[int, int]:
+    """(tile, shares) of :func:`tiled_gemm`."""
+    return min((_tiled_cost(M, N, K, t, s, gated, addends), t, s) for t in range(3 if gated else 4)
+               for s in ((1,) if gated else (1, 2, 3, 4, 6, 8)) if s == 1 or K // s >= 256)[1:]
+
+
+TILED_ROWS = 512            # rows up to which the product on the re-tiled matrix beats the library's or ties with it
+TILED_ROWS_GATED = 1024     # the same with SwiGLU in the epilogue, up to 70 GFLOP
+
+
+def tiled_wins(x: torch.Tensor, weight, gated: bool = False) -> bool:
+    """Whether a bfloat16 product goes to :func:`tiled_gemm`: from 65 rows (the skinny product's end) to 512, or 1,024 with
+    SwiGLU in the epilogue; beyond, the library's product is faster by itself (us, library : this, [16384, 2048] with
+    SwiGLU at 1,024 rows 73 : 66, at 2,048 120 : 130; [2048, 8192] at 512 rows 29 : 26, at 1,500 54 : 59).  Up to there it also costs
+    the host a launch of some 5 us in place of the library's 20, which is what a step launched kernel by kernel waits for."""
+    tiles = getattr(weight, "tiles", None)
+    if x.dtype != torch.bfloat16 or tiles is None:
+        return False
+    M, K = x.shape
+    N = weight.rows.shape[0]
+    most = TILED_ROWS_GATED if gated and 2.0 * M * N * K <= 70e9 else TILED_ROWS
+    return (64 < M <= most and K % 64 == 0 and N % (32 if gated else 4) == 0 and (N + 15) * K < 1 << 30 and x.is_contiguous()
+            and x.data_ptr() % 16 == 0)
+
+
+def tiled_gemm(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None, out: Optional[torch.Tensor] = None, gated: Optional[str] = None,
+               squared: bool = False, addends: bool = False, plan: Optional[Tuple[int, int]] = None) -> torch.Tensor:
+    """``x . weight^T`` for bfloat16 ``x`` [M, K] and a re-tiled :class:`Weight` [N, K], in bfloat16 or (``out_dtype``) float32.
+    ``gated``, ``squared``, ``addends`` and ``plan`` as for :func:`split_gemm`."""
+    M, K = x.shape
+    tiles = getattr(weight, "tiles", None)
+    if tiles is None:
+        raise KernelError("this product takes a re-tiled matrix")
+    N = weight.rows.shape[0]
+    out_dtype = out_dtype or x.dtype
+    _gpu(x, "x", torch.bfloat16, (M, weight.rows.shape[1]))
+    _gpu(tiles, "tiles", torch.bfloat16)
+    if gated is not None and (N % 32 or squared or out_dtype != torch.bfloat16):
+        raise KernelError("a gated product takes a stacked matrix of whole tiles, no other activation, and gives bfloat16")
+    if K % 64 or N % 4 or x.data_ptr() % 16 or M * K >= 1 << 30 or (N + 15) * K >= 1 << 30 or tiles.numel() != (N + 15) // 16 * 16 * K:
+        raise KernelError(f"tiled_gemm does not take [{M}, {K}] x [{N}, {K}]")
+    cols = N if gated is None else N // 2
+    tile, shares = plan or tiled_plan(M, N, K, gated is not None, addends)
+    per = -(-(K // 64) // shares)
+    shares = -(-(K // 64) // per)
+    if out is not None:
+        _gpu(out, "out", out_dtype, (M, cols))
+        if out.data_ptr() % 16:
+            raise KernelError("out is not aligned to 16 bytes")
+    if shares > 1:
+        parts = torch.empty(shares, M, N, dtype=torch.float32, device=x.device)
+    elif out is None:
+        out = torch.empty(M, cols, dtype=out_dtype, device=x.device)
+    _check(tile_lib().ni_tiled_gemm(_ptr(x), _ptr(tiles), _ptr(parts if shares > 1 else out), M, N, K, tile, shares, per, int(gated is not None),
+                                    int(shares > 1 or out_dtype == torch.float32), GATED_ACTIVATIONS[gated or "silu"],
+                                    int(squared and shares == 1), _stream()), "tiled_gemm")
+    if shares > 1:
+        return parts if addends else _add_shares(parts, out_dtype, out, squared)
     return out
 
 

@@ -405,7 +405,12 @@ class Attention(Part):
             return K.skinny_gemm_merged(ws, nsplit, T, self.H, self.hd, self.w_o, y)
         return K.linear(attended, self.w_o, residual=residual, pending=carried, leave=leave)
 
-    def forward(self, x, ctx, cache: LayerCache, residual: Optional[torch.Tensor] = None, leave=None):
+    @property
+    def leaves_addends(self) -> bool:
+        """Whether ``forward`` takes ``addends=True``: the result may then be float32 addends [S, T, d]."""
+        return type(self).forward is Attention.forward and type(self).output is Attention.output
+
+    def forward(self, x, ctx, cache: LayerCache, residual: Optional[torch.Tensor] = None, leave=None, addends: bool = False):
         T = x.shape[0]
         carried = getattr(x, "pending", None)       # addends of the residual stream that came with a normed input
         if carried is not None and residual is None:
@@ -413,6 +418,8 @@ class Attention(Part):
         qkv = self.project_rotate_write(x, ctx, cache)
         leave_runs = type(self).output is Attention.output      # a replaced output stage gets the merged rows
         attended = self.attend(qkv, ctx, cache, leave_runs=leave_runs)
+        if addends and residual is None and not isinstance(attended, tuple):
+            return K.linear(attended, self.w_o, addends=True)
         if leave is not None:
             return self.output(attended, T, residual, carried, leave)
         return self.output(attended, T, residual, carried)
@@ -465,11 +472,16 @@ class SwiGLU(Part):
         """``silu(W_gate x) * (W_up x)``: what the down product takes (for a part that places that product's result itself)."""
         return K.linear_swiglu(x, self.w_gate_up)
 
-    def forward(self, x, ctx, residual: Optional[torch.Tensor] = None, leave=None):
+    @property
+    def leaves_addends(self) -> bool:
+        """Whether ``forward`` takes ``addends=True``: the result may then be float32 addends [S, T, d]."""
+        return type(self).forward is SwiGLU.forward
+
+    def forward(self, x, ctx, residual: Optional[torch.Tensor] = None, leave=None, addends: bool = False):
         carried = getattr(x, "pending", None)       # addends of the residual stream that came with a normed input
         if carried is not None and residual is None:
             raise K.KernelError("pending addends of the residual stream need residual=h to go into")
-        return K.linear(self.hidden(x), self.w_down, residual=residual, pending=carried, leave=leave)
+        return K.linear(self.hidden(x), self.w_down, residual=residual, pending=carried, leave=leave, addends=addends and residual is None)
 
 
 # ------------------------------------------------------------------ block
@@ -556,7 +568,7 @@ class PreNormBlock(Block):
             spec = self._deferred(self.ffn_norm, self.mixer, self.ffn, T)
             a = self.mixer.forward(x, ctx, cache, residual=h, **({} if spec is None else {"leave": spec}))
         else:
-            a = self._addend(self.mixer.forward(x, ctx, cache))
+            a = self._addend(self.mixer.forward(x, ctx, cache, **self._may_leave(self.mixer)))
         x = self._normed_input(self.ffn_norm, self.ffn, h, a)
         adds = getattr(self.ffn, "adds_residual", None)
         if adds is not None and adds(T):
@@ -564,8 +576,14 @@ class PreNormBlock(Block):
             spec = leave if (leave is not None and leaves is not None and leaves(T)) else None
             f = self.ffn.forward(x, ctx, residual=h, **({} if spec is None else {"leave": spec}))
         else:
-            f = self._addend(self.ffn.forward(x, ctx))
+            f = self._addend(self.ffn.forward(x, ctx, **self._may_leave(self.ffn)))
         return h, f
+
+    @staticmethod
+    def _may_leave(part) -> dict:
+        """What tells a part that knows of it that its result may come as float32 addends: whatever norm stands behind
+        gets them through :func:`pending_for`."""
+        return {"addends": True} if getattr(part, "leaves_addends", False) else {}
 
     def _addend(self, y):
         """What a part returned, as the next norm takes it: a float32 result [T, d] of a part that keeps its

@@ -118,3 +118,63 @@ def test_every_expert_multiplies_its_own_tokens(K, monkeypatch, tile, T, d, ff, 
                             lambda z, w: K.experts_act(z, w, ff, "relu2")).cpu().double()
     # two products and a square, each a float32 sum: (2 (6 d + 8) + (6 ff + 8) + top + 4) roundings of the sums of sizes
     assert bool(((got - want).abs() <= (12 * d + 6 * ff + 28 + top) * 2.0 ** -24 * size + 1e-30).all())
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("M,N,Kd,shares", [(1, 4, 64, 1), (63, 60, 128, 1), (65, 68, 192, 1), (129, 260, 256, 1), (257, 132, 320, 1),
+                                           (130, 516, 448, 2), (200, 96, 1024, 3), (64, 256, 2048, 8)])
+def test_tiled_gemm_at_the_edges_of_its_tiles(K, tile, M, N, Kd, shares):
+    x, w = (t.bfloat16() for t in operands(M, N, Kd, seed=M + N + Kd, spread=20))
+    weight = K.Weight(w)
+    for dtype in (torch.float32, torch.bfloat16):
+        out = torch.full((M + 1, N), 7.0, device="cuda", dtype=dtype)
+        K.tiled_gemm(x, weight, dtype, out[:M], plan=(tile, shares))
+        want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+        # K exact products in a float32 sum (K + 8 roundings), and the rounding of the result
+        bound = (Kd + 8) * 2.0 ** -24 * size + (2.0 ** -8 * want.abs() if dtype == torch.bfloat16 else 0)
+        assert bool(((out[:M].double() - want).abs() <= bound).all()), dtype
+        assert bool((out[M] == 7.0).all())
+    if shares > 1:
+        parts = K.tiled_gemm(x, weight, plan=(tile, shares), addends=True)
+        assert parts.dtype == torch.float32 and parts.dim() == 3
+        total = parts[0].clone()
+        for p in parts[1:]:
+            total += p
+        assert torch.equal(total, K.tiled_gemm(x, weight, torch.float32, plan=(tile, shares)))
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2])
+@pytest.mark.parametrize("M,inter", [(65, 16), (64, 32), (130, 112), (129, 144)])
+def test_tiled_gemm_gated_and_squared(K, tile, M, inter):
+    x, w = (t.bfloat16() for t in operands(M, 2 * inter, 192, seed=inter))
+    weight = K.Weight(w)
+    z = K.tiled_gemm(x, weight, torch.float32, plan=(tile, 1))
+    for act in ("silu", "gelu_tanh"):
+        want = K.swiglu(z, torch.empty(M, inter, device="cuda"), act)
+        got = K.tiled_gemm(x, weight, gated=act, plan=(tile, 1)).float()
+        # one rounding to bfloat16, and the hardware's exponential (2^-20 of the value)
+        assert bool(((got - want).abs() <= (2.0 ** -8 + 2.0 ** -18) * want.abs() + 1e-30).all())
+    for shares in (1, 2):
+        whole = K.tiled_gemm(x, weight, torch.float32, plan=(tile, shares))
+        assert torch.equal(K.tiled_gemm(x, weight, torch.float32, squared=True, plan=(tile, shares)), torch.relu(whole) ** 2)
+
+
+def test_where_bfloat16_products_go(K):
+    """65 to 512 rows (1,024 with SwiGLU) of a re-tiled matrix are multiplied here, the library is not asked; what the kernel
+    cannot take goes to the library as before."""
+    x, w = (t.bfloat16() for t in operands(600, 512, 256))
+    weight, odd = K.Weight(w), K.Weight(w[:511].contiguous())
+    calls = K.library_calls()
+    K.linear(x[:65], weight), K.linear(x[:512], weight, out_dtype=torch.float32), K.linear_swiglu(x, weight), K.linear_relu2(x[:100], weight)
+    assert K.library_calls() == calls
+    aside = torch.empty(600 * 512 + 1, device="cuda", dtype=torch.bfloat16)[1:].view(600, 512)
+    for n, f in enumerate((lambda: K.linear(x, weight), lambda: K.linear(x[:100], odd), lambda: K.linear(x[:100], w),
+                           lambda: K.linear(x[:100], K.Weight(w, tiled=False)), lambda: K.linear(x[:100, :200].contiguous(), K.Weight(w[:, :200].contiguous())),
+                           lambda: K.linear(x[:100], weight, out=aside[:100]))):
+        got = f()
+        assert K.library_calls() == calls + n + 1 and bool(torch.isfinite(got).all())
+    for bad in (lambda: K.tiled_gemm(x.float(), weight), lambda: K.tiled_gemm(x, w), lambda: K.tiled_gemm(x[:, :128].contiguous(), weight),
+                lambda: K.tiled_gemm(x, odd), lambda: K.tiled_gemm(x, K.Weight(w[:48].contiguous()), gated="silu"),
+                lambda: K.tiled_gemm(x[:100], weight, out=aside[:100])):
+        with pytest.raises(K.KernelError):
+            bad()
