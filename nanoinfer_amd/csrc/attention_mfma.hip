@@ -245,7 +245,7 @@ void mfma_attention_kernel(
         // inside the loop would have to be waited for before its rows can be asked for, and that
         // wait, being in order, would drain every row load still in flight.
         constexpr int TBL_MAX = 1024;
-        __shared__ int32_t tbl[TBL_MAX];
+        __shared__ __attribute__((aligned(16))) int32_t tbl[TBL_MAX];
         int key_lo = 0, key_hi = 0, lp0 = 0;              // keys of the current segment, and its first page
         // the first key any row of the tile may read: keys before it (the steps start at a multiple of
         // KSTEP) may lie in pages that a window has passed and given back, and are never loaded
@@ -566,9 +566,14 @@ void mfma_decode_kernel(
     static_assert(KSTEP * VROW * 2 >= 16 * HD * 4, "a wavefront's V tile is reused for its 16 x HD partial output");
 
     // Uncut key ranges of many tokens: the chip holds the grid two workgroups a compute unit, u and u + half the grid,
-    // which is the same x in the lower and the upper half of y.  The upper half takes the tokens from the far end, so
-    // that a caller who brings the tokens in the order of their contexts gets a long and a short one on every unit.
-    const int t = (gridDim.z == 1 && gridDim.y > 1 && 2 * blockIdx.y >= gridDim.y) ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
+    // which is the same x in the lower and the upper half of y.  In the order of their contexts, longest first, the upper
+    // half takes the tokens from the far end: a long and a short one on every unit (64 requests of 175 to 2,100 tokens in
+    // no order 41 -> 33 us, in order 31.6).
+    constexpr int TBL_MAX = 1024;
+    __shared__ __attribute__((aligned(16))) int32_t tbl[TBL_MAX];
+    int t = (gridDim.z == 1 && gridDim.y > 1 && 2 * blockIdx.y >= gridDim.y) ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
+    if (gridDim.z == 1 && gridDim.y > 1 && gridDim.x > 1 && gridDim.x <= RANKED_TOKENS && gridDim.x * gridDim.y <= RANKED_GROUPS)
+        t = token_by_length(positions, gridDim.x, t, tbl);
     const int G = H / KVH;
     const int chunks = (G + 15) / 16;
     const int g = blockIdx.y / chunks;
@@ -595,8 +600,6 @@ void mfma_decode_kernel(
     const int32_t* table = block_table + static_cast<size_t>(seq) * table_stride;
     auto page_of = [&](int key) { return POW2 ? (key >> page_shift) : key / page_size; };
     auto slot_of = [&](int key) { return POW2 ? (key & (page_size - 1)) : key % page_size; };
-    constexpr int TBL_MAX = 1024;
-    __shared__ int32_t tbl[TBL_MAX];
     int key_lo = 0, key_hi = 0, lp0 = 0;
     auto row_address = [&](int key) -> size_t {
         // clamped to keys the token may read: those before `lo` may lie in pages already given back

@@ -69,7 +69,7 @@ __global__ __launch_bounds__(MA_WAVES * WAVE) void mfma_attention_f32_kernel(
     __shared__ __attribute__((aligned(16))) float ksm[2][KSTEP][ROW];
     __shared__ __attribute__((aligned(16))) float vsm[2][KSTEP][ROW];
     constexpr int TBL_MAX = 1024;
-    __shared__ int32_t tbl[TBL_MAX];
+    __shared__ __attribute__((aligned(16))) int32_t tbl[TBL_MAX];
 
     // As many workgroups as the chip holds at once; the tiles come sorted by the keys they walk,
     // longest first, and workgroup w takes tiles w, 2P-1-w, 2P+w, ... (P workgroups in x).
@@ -373,12 +373,14 @@ __global__ __launch_bounds__(DEC_WAVES * WAVE) void mfma_decode_f32_kernel(
     __shared__ __attribute__((aligned(16))) float so[NW][16][HD];      // the wavefronts' outputs, met at the end
     __shared__ float sm_ml[NW][16][2];
     constexpr int TBL_MAX = 1024;
-    __shared__ int32_t tbl[TBL_MAX];
+    __shared__ __attribute__((aligned(16))) int32_t tbl[TBL_MAX];
 
     // (uncut key ranges of many tokens: a compute unit holds workgroups u and u + half the grid, the same x in the
-    // lower and the upper half of y; the upper half takes the tokens from the far end, so that tokens that come in
-    // the order of their contexts put a long and a short one on every unit)
-    const int t = (gridDim.z == 1 && gridDim.y > 1 && 2 * blockIdx.y >= gridDim.y) ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
+    // lower and the upper half of y; in the order of their contexts the upper half takes the tokens from the far end:
+    // a long and a short one on every unit)
+    int t = (gridDim.z == 1 && gridDim.y > 1 && 2 * blockIdx.y >= gridDim.y) ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
+    if (gridDim.z == 1 && gridDim.y > 1 && gridDim.x > 1 && gridDim.x <= RANKED_TOKENS && gridDim.x * gridDim.y <= RANKED_GROUPS)
+        t = token_by_length(positions, gridDim.x, t, tbl);
     const int G = H / KVH;
     const int chunks = (G + 15) / 16;
     const int g = blockIdx.y / chunks;

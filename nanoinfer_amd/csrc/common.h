@@ -227,6 +227,44 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
     return total;
 }
 
+// The token of a decode step that this workgroup takes: the one whose position is the `want`-th largest (of equal
+// positions the one that comes first).  Where every token's keys are walked by workgroups of their own, two of them on a
+// compute unit, who gets which token is what the time depends on: a long and a short one on every unit.  The caller's order
+// says nothing about the lengths, so each workgroup ranks the tokens itself, a thread a token against all others in `pos`
+// (LDS, 16-byte aligned, room for n rounded up to 4); nothing of it where they already come in order.  All threads call it.
+__device__ __forceinline__ int token_by_length(const int32_t* __restrict__ positions, int n, int want, int32_t* pos) {
+    bool disordered = false;
+    const int padded = (n + 3) & ~3;
+    for (int i = threadIdx.x; i < padded; i += blockDim.x) {
+        const int p = i < n ? positions[i] : -1;             // (no position is negative)
+        pos[i] = p;
+        disordered |= i + 1 < n && positions[i + 1] > p;
+    }
+    __shared__ int found;
+    if (threadIdx.x == 0) found = want;
+    if (__syncthreads_or(disordered)) {
+        for (int i = threadIdx.x; i < n; i += blockDim.x) {
+            const int mine = pos[i];
+            int rank = 0;
+#pragma unroll 4
+            for (int j = 0; j < padded; j += 4) {
+                const int4 v = *reinterpret_cast<const int4*>(pos + j);
+                // before this one: a larger position, or the same position and a smaller index
+                rank += v.x + (j < i) > mine;
+                rank += v.y + (j + 1 < i) > mine;
+                rank += v.z + (j + 2 < i) > mine;
+                rank += v.w + (j + 3 < i) > mine;
+            }
+            if (rank == want) found = i;
+        }
+        __syncthreads();
+    }
+    return __builtin_amdgcn_readfirstlane(found);
+}
+// Workgroups of such a grid up to which it is worth it (two on each of 256 units), and tokens that it takes at most.
+#define RANKED_GROUPS 512
+#define RANKED_TOKENS 256
+
 // What a gated hidden unit gives from its gate g and its up value u: g sigmoid(a g + b g^3) u.  (1, 0) is silu(g) u;
 // gelu in its tanh form is 0.5 g (1 + tanh y) = g sigmoid(2 y) with y = sqrt(2 / pi) (g + 0.044715 g^3).
 struct GatedUnit {
