@@ -1067,6 +1067,12 @@ __global__ __launch_bounds__(GV_THREADS) void skinny_rows_kernel(const T* __rest
         if (rope.slot_mapping) rope.slot_mapping += row0;
         if (defer.ss_in != nullptr) defer.ss_in += static_cast<size_t>(row0) * defer.parts;
         M = min(M - row0, ROWS);
+    } else if constexpr (EPI == EPI_STORE || EPI == EPI_SWIGLU) {
+        // more rows than one workgroup holds (a small matrix): the same
+        const int row0 = static_cast<int>(blockIdx.z) * ROWS;
+        x += static_cast<size_t>(row0) * K;
+        y += static_cast<size_t>(row0) * (EPI == EPI_SWIGLU ? I : N);
+        M = min(M - row0, ROWS);
     }
     unsigned char* slab = lds + wave * SLAB;
 
@@ -1335,6 +1341,15 @@ static int launch_mb(const void* x, const void* W, void* y, int M, int N, int K,
         // two, three or four blocks of sixteen rows: what a workgroup brings of x into its LDS grows with them
         // (dealt out only while that is still at most one workgroup a compute unit: the 160 pairs of tiles of the 3B
         // shape as 320 workgroups of 32 rows took 15.0 us at 64 rows, the 192 pairs of the 8B shape as 384 22.3 us)
+        if constexpr (EPI == EPI_STORE || EPI == EPI_SWIGLU) {
+            // more than 64 rows, for small matrices: 32 rows a workgroup while that is one workgroup a compute unit, else 64
+            if (M > 64) {
+                if (defer.ss_in != nullptr) return -11;
+                const int tiles = ((EPI == EPI_SWIGLU ? I : N) + 15) / 16;
+                if (static_cast<long>(tiles) * ((M + 31) / 32) <= 256) return launch_rows<T, TOUT, 2, EPI>(x, W, y, M, N, K, I, 1, stream, rope, 1, defer);
+                return launch_rows<T, TOUT, 4, EPI>(x, W, y, M, N, K, I, 1, stream, rope, 1, defer);
+            }
+        }
         const bool dealt = EPI == EPI_ROPE && ((N + 31) / 32) * ((M + 31) / 32) <= 256;
         if constexpr (EPI == EPI_ROPE) {
             // up to 32 rows of a matrix of few pairs of tiles (96 at the 1B shape): 16 rows a workgroup
@@ -1381,7 +1396,8 @@ static int launch_normed(const NormArgs& norm, const void* W, void* y, int M, in
 // epilogue: 0 store in the input type, 1 store float32, 2 SwiGLU (W is [2I, K], y is [M, I]),
 // 3 add into y, the float32 residual stream [M, N] (tiled W), 4 as 2 with gelu (tanh) in silu's place, 5 store relu(.)^2 in the
 // input type.
-// K must be a multiple of 16 bytes' worth of elements x 2 (bf16: 16, f32: 8); M <= 64.
+// K must be a multiple of 16 bytes' worth of elements x 2 (bf16: 16, f32: 8); M <= 64, or any M for small re-tiled matrices
+// (epilogues that store: every 32 or 64 rows stream the matrix anew).
 // tiled: W is in the re-tiled order described at the top (swiglu then needs N/2 to be a multiple of 16).
 // pend, n_pend (epilogue 3, at most 16 rows): float32 [n_pend, M, N] that y has not received yet and that are
 // added before the product, y = ((y + pend[0]) + pend[1] ...) + x . W^T; null, 0: none.
@@ -1398,7 +1414,7 @@ NI_EXPORT int ni_skinny_gemm(const void* x, const void* W, void* y, int M, int N
                              int tiled, int dtype, const void* pend, int n_pend, void* xn, const void* next_w, void* ss,
                              int parts, float eps, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (M > 64) return -1;
+    if (M > 64 && (!tiled || epilogue == 3 || M > 65535 * 32)) return -1;
     const int el = dtype == 0 ? 8 : 16;
     if (K % el != 0) return -2;
     const int I = N / 2;

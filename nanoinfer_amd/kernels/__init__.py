@@ -564,6 +564,28 @@ def skinny_wins(M: int, K: int, dtype: torch.dtype, weight=None) -> bool:
         # [28672, 4096] 122.8 : 103.6 and 197.7 : 141.9; [4096, 14336] 72.3 : 57.9 and 107.5 : 86.2
         return K <= 2048 and (M <= 32 or weight.rows.shape[0] < 8192)
     return M <= 32 or K <= 4096
+
+
+def _plain(x: torch.Tensor) -> bool:
+    """Whether the rows of x are one run of memory that starts at 16 bytes: what a kernel with wide loads takes."""
+    return x.is_contiguous() and x.data_ptr() % 16 == 0
+
+
+def skinny_deals(M: int, N: int, K: int, dtype: torch.dtype, weight) -> bool:
+    """Whether a product of more rows than the skinny kernel holds still goes there, 32 or 64 rows a workgroup: a small re-tiled
+    matrix (N: the columns of the result), whose library product takes 5 us and more (tens where its rule finds a kernel
+    of one workgroup), while every compute unit has at most one workgroup.  Measured in recorded launches (us, library : this):
+    float32 [192, 512] at 100 rows 49 : 4.4, [1024, 192] at 256 rows 5.5 : 4.9, at 448 6.3 : 6.4, [1024, 512] at 100 rows
+    6.5 : 4.8, at 160 6.7 : 7.0, [128, 2048] 7.3 : 8.9; bfloat16 [1024, 1024] at 256 rows 5.8 : 5.5, at 448 7.0 : 7.5,
+    [16, 2048] at 1,500 rows 5.6 : 4.7, [1024, 2048] at 256 rows 7.6 : 7.5."""
+    if not (isinstance(weight, Weight) and weight.tiles is not None and K % (8 if dtype == torch.float32 else 16) == 0):
+        return False
+    tiles = (N + 15) // 16
+    if dtype == torch.float32:
+        return (K <= 512 and tiles * ((M + 63) // 64) <= 256) or (K <= 1024 and tiles * ((M + 31) // 32) <= 256)
+    return K <= 2048 and tiles * ((M + 63) // 64) <= 256
+
+
 FUSE_NORMS = True           # residual sums and norms ride on the skinny products of a decode step where they can
 ADDENDS_IN_PROLOGUE = True  # the shares of a cut product are added by the next normalising prologue and residual epilogue
 MERGE_IN_PRODUCT = True     # the key runs of a decode step's attention are merged by the output product where it can
@@ -879,7 +901,8 @@ def _check_normed(x: NormedInput, Kd: int) -> None:
 
 def skinny_gemm(x, weight, out: torch.Tensor, swiglu: bool = False, residual: bool = False,
                 pending: Optional[torch.Tensor] = None, leave: Optional[NormSpec] = None, activation: str = "silu"):
-    """``x . weight^T`` for at most 64 rows of ``x``, streaming ``weight`` once (MFMA).  ``out``
+    """``x . weight^T`` for at most 64 rows of ``x`` (any number with a re-tiled matrix and a plain ``x`` and epilogue: every
+    64 or 32 of them stream it anew), streaming ``weight`` once (MFMA).  ``out``
     may be float32 for bfloat16 inputs.  With ``swiglu`` the weight is a stacked [2I, K] matrix
     (gate rows, then up rows) and ``out`` [M, I] receives ``silu(gate) * up`` (``activation`` "gelu_tanh": gelu in its
     tanh form in silu's place, for a plain ``x``); without it, ``activation`` "relu2" stores ``relu(x . weight^T)^2`` in the
@@ -897,7 +920,9 @@ def skinny_gemm(x, weight, out: torch.Tensor, swiglu: bool = False, residual: bo
     _gpu(rows, "weight", dtype)
     if not (rows.shape[1] == Kd):
         raise KernelError(f"skinny_gemm: {tuple(x.shape)} x {tuple(rows.shape)}^T")
-    if not (skinny_ok(M, Kd, dtype)):
+    # (more rows than a workgroup holds are dealt out to several: a given x, a re-tiled matrix and an epilogue that stores)
+    dealt = M > SKINNY_MAX_ROWS and tiles is not None and not (normed or scaled or residual or (swiglu and (N // 2) % 16))
+    if not (skinny_ok(min(M, SKINNY_MAX_ROWS) if dealt else M, Kd, dtype)):
         raise KernelError(f"skinny_gemm does not take M={M}, K={Kd} in {dtype}")
     if swiglu and tiles is not None and (N // 2) % 16:
         tiles = None          # gate and up halves do not start on tile boundaries: stream the rows as stored
@@ -1149,11 +1174,13 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
     out_dtype = out_dtype or x.dtype
     if out is not None:
         _gpu(out, "out", out_dtype, (x.shape[0], rows.shape[0]))
-    if skinny_wins(x.shape[0], x.shape[1], x.dtype, weight):
+    M, Kd = x.shape
+    if skinny_wins(M, Kd, x.dtype, weight) if M <= SKINNY_MAX_ROWS else (
+            skinny_deals(M, rows.shape[0], Kd, x.dtype, weight) and _plain(x) and (out is None or out.data_ptr() % 16 == 0)):
         if out is None:
-            out = torch.empty(x.shape[0], rows.shape[0], dtype=out_dtype, device=x.device)
+            out = torch.empty(M, rows.shape[0], dtype=out_dtype, device=x.device)
         return skinny_gemm(x, weight, out)
-    if split_wins(x, rows) and out_dtype == torch.float32:
+    if out_dtype == torch.float32 and split_wins(x, rows):
         return split_gemm(x, rows, out, addends=addends)
     if tiled_wins(x, weight) and (out is None or out.data_ptr() % 16 == 0):
         return tiled_gemm(x, weight, out_dtype, out, addends=addends)
@@ -1180,14 +1207,15 @@ def linear_swiglu(x, weight_gate_up, activation: str = "silu") -> torch.Tensor:
     if isinstance(x, ScaledInput) and not swiglu_takes_scaled(x.shape[0], x.shape[1], x.dtype, weight_gate_up):
         raise KernelError("this product cannot take a scaled input")
     # (past 16 rows only a matrix whose halves start on tile boundaries is streamed re-tiled)
-    if isinstance(x, NormedInput) or (skinny_wins(x.shape[0], x.shape[1], x.dtype, weight_gate_up)
-                                      and (x.shape[0] <= SKINNY_BEST_ROWS or inter % 16 == 0)):
+    M, Kd = x.shape
+    if isinstance(x, NormedInput) or ((skinny_wins(M, Kd, x.dtype, weight_gate_up) if M <= SKINNY_MAX_ROWS else
+                                       (skinny_deals(M, inter, Kd, x.dtype, weight_gate_up) and _plain(x)))
+                                      and (M <= SKINNY_BEST_ROWS or inter % 16 == 0)):
         return skinny_gemm(x, weight_gate_up, out, swiglu=True, activation=activation)
     rows, _ = _rows_and_tiles(weight_gate_up)
     if split_wins(x, rows):
-        M, N, K = x.shape[0], 2 * inter, x.shape[1]
         # in one kernel, or cut along K with the SwiGLU kernel behind it (which moves 12 bytes an output at 4 TB/s)
-        if split_plan(M, N, K, True)[2] <= split_plan(M, N, K)[2] + 4.0 + 12.0 * M * inter / 4e6:
+        if split_plan(M, 2 * inter, Kd, True)[2] <= split_plan(M, 2 * inter, Kd)[2] + 4.0 + 12.0 * M * inter / 4e6:
             return split_gemm(x, rows, out, gated=activation)
         return swiglu(split_gemm(x, rows), out, activation)
     if tiled_wins(x, weight_gate_up, gated=True):
@@ -1201,8 +1229,9 @@ def linear_swiglu(x, weight_gate_up, activation: str = "silu") -> torch.Tensor:
 def linear_relu2(x, weight) -> torch.Tensor:
     """``relu(x . weight^T)^2`` in the type of ``x``: fused into the product for few rows, product then an elementwise kernel
     for many."""
-    if skinny_wins(x.shape[0], x.shape[1], x.dtype, weight):
-        out = torch.empty(x.shape[0], weight.shape[0], dtype=x.dtype, device=x.device)
+    M, Kd = x.shape
+    if skinny_wins(M, Kd, x.dtype, weight) if M <= SKINNY_MAX_ROWS else (skinny_deals(M, weight.shape[0], Kd, x.dtype, weight) and _plain(x)):
+        out = torch.empty(M, weight.shape[0], dtype=x.dtype, device=x.device)
         return skinny_gemm(x, weight, out, activation="relu2")
     rows, _ = _rows_and_tiles(weight)
     if split_wins(x, rows):

@@ -162,17 +162,18 @@ def test_tiled_gemm_gated_and_squared(K, tile, M, inter):
 def test_where_bfloat16_products_go(K):
     """65 to 512 rows (1,024 with SwiGLU) of a re-tiled matrix are multiplied here, the library is not asked; what the kernel
     cannot take goes to the library as before."""
-    x, w = (t.bfloat16() for t in operands(600, 512, 256))
-    weight, odd = K.Weight(w), K.Weight(w[:511].contiguous())
+    x, w = (t.bfloat16() for t in operands(600, 2080, 256))
+    weight, odd = K.Weight(w), K.Weight(w[:2079].contiguous())
     calls = K.library_calls()
-    K.linear(x[:65], weight), K.linear(x[:512], weight, out_dtype=torch.float32), K.linear_swiglu(x, weight), K.linear_relu2(x[:100], weight)
+    K.linear(x[:65], weight), K.linear(x[:512], weight, out_dtype=torch.float32), K.linear_swiglu(x, weight), K.linear_relu2(x[:200], weight)
     assert K.library_calls() == calls
-    aside = torch.empty(600 * 512 + 1, device="cuda", dtype=torch.bfloat16)[1:].view(600, 512)
-    for n, f in enumerate((lambda: K.linear(x, weight), lambda: K.linear(x[:100], odd), lambda: K.linear(x[:100], w),
-                           lambda: K.linear(x[:100], K.Weight(w, tiled=False)), lambda: K.linear(x[:100, :200].contiguous(), K.Weight(w[:, :200].contiguous())),
-                           lambda: K.linear(x[:100], weight, out=aside[:100]))):
+    aside = torch.empty(600 * 2080 + 1, device="cuda", dtype=torch.bfloat16)[1:].view(600, 2080)
+    for n, f in enumerate((lambda: K.linear(x, weight), lambda: K.linear(x[:200], odd), lambda: K.linear(x[:100], w),
+                           lambda: K.linear(x[:100], K.Weight(w, tiled=False)), lambda: K.linear(x[:200, :200].contiguous(), K.Weight(w[:, :200].contiguous())),
+                           lambda: K.linear(x[:200], weight, out=aside[:200]), lambda: K.linear(x[:70], weight, out=aside[:70]),
+                           lambda: K.linear(x.view(-1)[1:1 + 70 * 256].view(70, 256), weight))):
         got = f()
-        assert K.library_calls() == calls + n + 1 and bool(torch.isfinite(got).all())
+        assert K.library_calls() == calls + n + 1 and bool(torch.isfinite(got).all()), n
     for bad in (lambda: K.tiled_gemm(x.float(), weight), lambda: K.tiled_gemm(x, w), lambda: K.tiled_gemm(x[:, :128].contiguous(), weight),
                 lambda: K.tiled_gemm(x, odd), lambda: K.tiled_gemm(x, K.Weight(w[:48].contiguous()), gated="silu"),
                 lambda: K.tiled_gemm(x[:100], weight, out=aside[:100])):
