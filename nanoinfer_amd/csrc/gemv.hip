@@ -192,6 +192,20 @@ __device__ __forceinline__ void store_exact4(bf16_t* p, const float (&v)[4]) {
                 static_cast<uint32_t>(f32_to_bf16_bits(v[2])) | (static_cast<uint32_t>(f32_to_bf16_bits(v[3])) << 16)};
 }
 
+// The rotation epilogue's columns are pairs (j, j + hd/2) of one head; the pairs of all heads are numbered through, and a
+// workgroup owns the R from wg * R.  Where R divides a head's pairs the head is the same for the whole workgroup.
+struct RopePair { int head, j; };
+template <int R>
+__device__ __forceinline__ RopePair rope_pair(int wg, int local, int hd) {
+    if constexpr (16 % R == 0) {
+        const int per_head = hd / (2 * R);
+        return {wg / per_head, (wg % per_head) * R + local};
+    } else {
+        const int pair = wg * R + local;
+        return {pair / (hd / 2), pair % (hd / 2)};
+    }
+}
+
 struct EpiEarly {
     bool have = false;       // the values below are those of item threadIdx.x
     int pos = 0, slot = -1;  // rotation: the row's position and cache slot
@@ -201,21 +215,21 @@ struct EpiEarly {
 };
 
 // The first half for the rotation epilogue (position and slot of the thread's row), the whole for the residual one.
-template <int EPI, int NT, int HALVES>
+template <int EPI, int NT, int R>
 __device__ __forceinline__ void epi_early_first(EpiEarly& e, const void* y, int M, int N, const RopeArgs& rope,
                                                 const float* pend, int n_pend, const float* next_w = nullptr) {
     const int item = threadIdx.x;
-    const int wg = blockIdx.x / HALVES, wg_half = blockIdx.x % HALVES;
+    const int wg = blockIdx.x;
     if constexpr (EPI == EPI_ROPE) {
         const int n_local = item % 16, m = item / 16;
-        if (item >= 16 * 16 || m >= M || (HALVES == 2 && (n_local >> 3) != wg_half)) return;
+        if (item >= 16 * 16 || m >= M || n_local >= R || 2 * (wg * R + n_local) >= N) return;
         e.have = true;
         e.pos = rope.positions[m];
         if (rope.slot_mapping) e.slot = rope.slot_mapping[m];
     } else if constexpr (EPI == EPI_RESIDUAL) {
         const int n_in = item % (NT * 16), m = item / (NT * 16);
-        const int n = wg * NT * 16 + n_in;
-        if (item >= 16 * NT * 16 || m >= M || n >= N || (HALVES == 2 && ((n_in % 16) >> 3) != wg_half)) return;
+        const int n = (wg * NT + n_in / 16) * R + n_in % 16;
+        if (item >= 16 * NT * 16 || m >= M || n >= N || n_in % 16 >= R) return;
         e.have = true;
         const float* dst = static_cast<const float*>(y) + static_cast<size_t>(m) * N + n;
         e.a = *dst;
@@ -228,14 +242,13 @@ __device__ __forceinline__ void epi_early_first(EpiEarly& e, const void* y, int 
     }
 }
 // The second half for the rotation epilogue, once the position has arrived: cos and sin of the thread's pair.
-template <int EPI, int HALVES>
+template <int EPI, int R>
 __device__ __forceinline__ void epi_early_second(EpiEarly& e, const RopeArgs& rope) {
     if constexpr (EPI == EPI_ROPE) {
         if (!e.have) return;
-        const int wg = blockIdx.x / HALVES;
-        const int per_head = rope.hd / 32;
-        if (wg / per_head >= rope.H + rope.KVH) return;       // values do not turn
-        const int j = (wg % per_head) * 16 + static_cast<int>(threadIdx.x) % 16;
+        const RopePair at_pair = rope_pair<R>(blockIdx.x, static_cast<int>(threadIdx.x) % 16, rope.hd);
+        if (at_pair.head >= rope.H + rope.KVH) return;       // values do not turn
+        const int j = at_pair.j;
         const size_t at = static_cast<size_t>(e.pos) * (rope.hd / 2) + j;
         e.a = rope.cos_t[at];
         e.b = rope.sin_t[at];
@@ -244,17 +257,16 @@ __device__ __forceinline__ void epi_early_second(EpiEarly& e, const RopeArgs& ro
 
 // What follows the main loop of both kernels: the wavefronts' partial sums meet in LDS and the
 // epilogue stores them.
-// HALVES == 2: two workgroups share the tiles that one would own; the first stores the first eight
-// columns of every tile, the second the others (each has multiplied only its own rows of W).
-template <typename T, typename TOUT, int MB, int NT, int EPI, int WV = GV_WAVES, bool EXT = false, int HALVES = 1>
+// R: the rows of W (columns of the result, pairs with rotation) that each tile of the workgroup holds, in its
+// first R columns.
+template <typename T, typename TOUT, int MB, int NT, int EPI, int WV = GV_WAVES, bool EXT = false, int R = 16>
 __device__ __forceinline__ void skinny_finish(const floatx4_t (&acc)[NT][MB], TOUT* __restrict__ y, int M, int N, int I,
                                               const RopeArgs& rope, float* ext = nullptr, const float* pend = nullptr,
                                               int n_pend = 0, const EpiEarly* early = nullptr,
                                               const DeferArgs& defer = DeferArgs{}, const float* factors = nullptr) {
     const int tid = threadIdx.x;
     const int wave = tid / WAVE, lane = tid % WAVE;
-    const int wg = blockIdx.x / HALVES;
-    const int wg_half = blockIdx.x % HALVES;      // which eight columns of every tile are this workgroup's
+    const int wg = blockIdx.x;
     // partial sums of the wavefronts meet in LDS: red[wave][tile][lane * 4 + i]; in memory of the
     // function's own, or (EXT) in memory the kernel has no other use for any more
     typedef float (*Red)[NT * MB][WAVE * 4];
@@ -285,7 +297,7 @@ __device__ __forceinline__ void skinny_finish(const floatx4_t (&acc)[NT][MB], TO
         // workgroup spent longer here than on a quarter of its matrix).  The four values are columns n0 .. n0 + 3 of row m;
         // a gate tile and its up tile are taken by the same thread.  (The rotation epilogue, 32 rows a workgroup, was
         // no faster this way and keeps the items below.)
-        static_assert(HALVES == 1, "halved tiles come with one block of rows");
+        static_assert(R == 16, "tiles of fewer rows of W come with one block of rows");
         if constexpr (DEFERS) {
             if (defer.xn != nullptr) {
                 // The stream's new values and what the next norm needs of them (see DeferArgs): h * w in the compute
@@ -414,14 +426,13 @@ __device__ __forceinline__ void skinny_finish(const floatx4_t (&acc)[NT][MB], TO
         }
     }
     if constexpr (EPI == EPI_ROPE) {
-        const int per_head = rope.hd / 32;
-        const int head = wg / per_head;                 // among H query, KVH key, KVH value heads
-        const int j0 = (wg % per_head) * 16;            // first of this workgroup's 16 pairs
         const int half = rope.hd / 2;
         for (int item = tid; item < MB * 16 * 16; item += WV * WAVE) {
             const int n_local = item % 16;
             const int m = item / 16;
-            if (m >= M || (HALVES == 2 && (n_local >> 3) != wg_half)) continue;
+            if (m >= M || n_local >= R || 2 * (wg * R + n_local) >= N) continue;
+            const RopePair at_pair = rope_pair<R>(wg, n_local, rope.hd);
+            const int head = at_pair.head, j = at_pair.j;      // the head among H query, KVH key, KVH value heads
             const int mb = m / 16, m_local = m % 16;
             const int src = ((n_local / 4) * 16 + m_local) * 4 + (n_local % 4);
             float x0 = 0.f, x1 = 0.f;
@@ -431,7 +442,6 @@ __device__ __forceinline__ void skinny_finish(const floatx4_t (&acc)[NT][MB], TO
                 x1 += red[w][1 * MB + mb][src];
             }
             if (scaled) { const float f = factor_of(m); x0 *= f; x1 *= f; }
-            const int j = j0 + n_local;
             const bool ready = early != nullptr && early->have && item == tid;      // asked for while W was streaming
             if (head < rope.H + rope.KVH) {             // queries and keys turn, values do not
                 float c, sn;
@@ -472,7 +482,6 @@ __device__ __forceinline__ void skinny_finish(const floatx4_t (&acc)[NT][MB], TO
         return;
     }
     constexpr int NOUT = (EPI == EPI_SWIGLU) ? NT / 2 : NT;      // output tiles of the workgroup
-    const int out_n0 = wg * NOUT * 16;
     const int out_width = (EPI == EPI_SWIGLU) ? I : N;
     if constexpr (EPI == EPI_RESIDUAL) {
         if (defer.xn != nullptr) {
@@ -482,16 +491,15 @@ __device__ __forceinline__ void skinny_finish(const floatx4_t (&acc)[NT][MB], TO
             // goes through the same code (lanes without a row or a column add zero and store nothing).
             constexpr int ROWW = NT * 16;
             static_assert(ROWW <= WAVE && WAVE % ROWW == 0, "the items of a row lie within a wavefront");
-            static_assert(HALVES == 1 || NT == 1, "halved tiles come one to a workgroup");
-            const int parts = gridDim.x;          // with HALVES == 2 every half of a tile is a part of its own
+            const int parts = gridDim.x;
             for (int base = 0; base < MB * 16 * ROWW; base += WV * WAVE) {
                 const int item = base + tid;
                 if (item - lane >= MB * 16 * ROWW) break;           // the whole wavefront is past the items
                 const int n_in = item % ROWW, m = item / ROWW;
                 const int ot = n_in / 16, n_local = n_in % 16;
                 const int mb = m / 16, m_local = m % 16;
-                const int n = out_n0 + n_in;
-                const bool live = m < M && n < N && (HALVES == 1 || (n_local >> 3) == wg_half);
+                const int n = (wg * NT + ot) * R + n_local;
+                const bool live = m < M && n < N && n_local < R;
                 float sq = 0.f;
                 if (live) {
                     const int src = ((n_local / 4) * 16 + m_local) * 4 + (n_local % 4);
@@ -521,8 +529,8 @@ __device__ __forceinline__ void skinny_finish(const floatx4_t (&acc)[NT][MB], TO
                 }
 #pragma unroll
                 for (int off = ROWW / 2; off > 0; off >>= 1) sq += __shfl_xor(sq, off, WAVE);
-                // (a half tile that lies past the matrix's last column still writes its part: zero)
-                if (n_in == (HALVES == 2 ? wg_half * 8 : 0) && m < M)
+                // (a workgroup that lies past the matrix's last column still writes its part: zero)
+                if (n_in == 0 && m < M)
                     defer.ss_out[static_cast<size_t>(m) * parts + blockIdx.x] = sq;
             }
             return;
@@ -533,8 +541,8 @@ __device__ __forceinline__ void skinny_finish(const floatx4_t (&acc)[NT][MB], TO
         const int m = item / (NOUT * 16);
         const int ot = n_in / 16, n_local = n_in % 16;
         const int mb = m / 16, m_local = m % 16;
-        const int n = out_n0 + n_in;
-        if (m >= M || n >= out_width || (HALVES == 2 && (n_local >> 3) != wg_half)) continue;
+        const int n = (wg * NOUT + ot) * R + n_local;
+        if (m >= M || n >= out_width || n_local >= R) continue;
         const int src = ((n_local / 4) * 16 + m_local) * 4 + (n_local % 4);
         float v;
         if (EPI == EPI_SWIGLU) {
@@ -659,16 +667,15 @@ __global__ __launch_bounds__(GV_THREADS) void skinny_gemm_kernel(const T* __rest
 // few lanes: read in that layout, h and the norm's weights take twice the load instructions of W
 // itself.  Staged, the workgroup reads every element once with full loads, normalises, rounds, and
 // leaves the rows in LDS, from where the lanes pick their operands.
-// HALVES == 2: a matrix of few tiles is streamed by twice the workgroups, each taking eight of a
-// tile's sixteen rows (the lanes of the other eight load the same rows again, which costs no
-// memory traffic, and their columns of the product are not stored).  A compute unit alone draws
-// about 37 GB/s from memory, so a launch of fewer workgroups than compute units cannot stream at
-// the chip's rate.
+// R: rows of W that a tile of the workgroup holds, sixteen or fewer.  The matrix takes as long as the compute unit that
+// has most of it, so where whole tiles would leave some units with more than others the rows are dealt out in smaller
+// tiles (decode_shape).  The lanes past R load the tile's row R - 1 again, which costs no memory traffic (but the texture
+// path the same time as a whole tile: the launch must stay one workgroup a compute unit), and their columns are not stored.
 // PEND (staged normalising prologue only): h comes with addends it has not received yet, which the prologue
 // adds to its rows.  A kernel of its own, because the addends wait in registers beside the rows of h while the
 // first pieces of W are asked for: for eight rows that is 172 registers instead of 120, one workgroup a compute
 // unit instead of two, which the products without addends should not pay.
-template <typename T, typename TOUT, int NT, int EPI, int XP, int WV, int SR, int HALVES = 1, int PRO = PRO_NORM, bool PEND = false>
+template <typename T, typename TOUT, int NT, int EPI, int XP, int WV, int SR, int R = 16, int PRO = PRO_NORM, bool PEND = false>
 __global__ __launch_bounds__(WV * WAVE) void skinny_decode_kernel(const T* __restrict__ x, const T* __restrict__ W,
                                                                    TOUT* __restrict__ y, int M, int N, int K, int I,
                                                                    RopeArgs rope, NormArgs norm, int splits, DeferArgs defer) {
@@ -687,10 +694,7 @@ __global__ __launch_bounds__(WV * WAVE) void skinny_decode_kernel(const T* __res
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;      // the same in every lane: say so
     const int r = lane % 16, kg = lane / 16;
-    const int wg = blockIdx.x / HALVES;
-    // the lane of the re-tiled matrix that this lane reads: its own, or with HALVES == 2 the one of this
-    // workgroup's half that has the same row modulo eight
-    const int wlane = HALVES == 1 ? lane : kg * 16 + ((r & 7) | (static_cast<int>(blockIdx.x % HALVES) << 3));
+    const int wg = blockIdx.x;
     const int pieces = (K + CH - 1) / CH;
     // with splits > 1 (no prologue) workgroup (x, y) multiplies the y-th share of the pieces and stores its sums in the y-th [M, N] of y
     const int share = (pieces + splits - 1) / splits;
@@ -698,19 +702,31 @@ __global__ __launch_bounds__(WV * WAVE) void skinny_decode_kernel(const T* __res
     y += static_cast<size_t>(blockIdx.y) * M * N;
     EpiEarly early;         // what the epilogue will read, asked for before W (not behind the merging prologue's many
                             // loads, where it gained nothing: the o product of one row 6.6 -> 7.3 us)
-    if constexpr (PRO == PRO_NORM) epi_early_first<EPI, NT, HALVES>(early, y, M, N, rope, norm.pend, norm.n_pend, defer.w);
+    if constexpr (PRO == PRO_NORM) epi_early_first<EPI, NT, R>(early, y, M, N, rope, norm.pend, norm.n_pend, defer.w);
 
     const T* wrow[NT];      // first byte of this lane in piece 0 of each tile
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-        int col0 = (EPI == EPI_SWIGLU) ? (wg * (NT / 2) + nt / 2) * 16 : (wg * NT + nt) * 16;
-        if (EPI == EPI_ROPE) {
-            const int per_head = rope.hd / 32;
-            col0 = (wg / per_head) * rope.hd + (wg % per_head) * 16 + nt * (rope.hd / 2);
-        }
-        const int shift = (EPI == EPI_SWIGLU && (nt % 2)) ? I : 0;
         const int limit = (N + 15) / 16 - 1;         // a workgroup's last tiles may lie past the matrix: read the last one, store nothing
-        wrow[nt] = W + static_cast<size_t>(min((col0 + shift) / 16, limit)) * pieces * (WAVE * EL) + wlane * EL;
+        int tile, tile_row = r;                      // this lane's row of W
+        if constexpr (R == 16) {
+            int col0 = (EPI == EPI_SWIGLU) ? (wg * (NT / 2) + nt / 2) * 16 : (wg * NT + nt) * 16;
+            if (EPI == EPI_ROPE) {
+                const RopePair first = rope_pair<R>(wg, 0, rope.hd);
+                col0 = first.head * rope.hd + first.j + nt * (rope.hd / 2);
+            }
+            tile = (col0 + ((EPI == EPI_SWIGLU && (nt % 2)) ? I : 0)) / 16;
+        } else {
+            static_assert(EPI != EPI_SWIGLU, "gate and up tiles are whole");
+            int n = (wg * NT + nt) * R + min(r, R - 1);
+            if (EPI == EPI_ROPE) {
+                const RopePair mine = rope_pair<R>(wg, min(r, R - 1), rope.hd);
+                n = mine.head * rope.hd + mine.j + nt * (rope.hd / 2);
+            }
+            tile = n / 16;
+            tile_row = n % 16;
+        }
+        wrow[nt] = W + static_cast<size_t>(min(tile, limit)) * pieces * (WAVE * EL) + (kg * 16 + tile_row) * EL;
     }
 
     floatx4_t acc[NT][1];
@@ -986,7 +1002,7 @@ __global__ __launch_bounds__(WV * WAVE) void skinny_decode_kernel(const T* __res
                 xn[p / PT][p % PT][0].from_floats(f);
             }
         }
-        epi_early_second<EPI, HALVES>(early, rope);      // behind the first trip of W; the position has arrived long ago
+        epi_early_second<EPI, R>(early, rope);      // behind the first trip of W; the position has arrived long ago
 #pragma unroll
         for (int t = 0; t < TRIPS; t += 2) {
             const int c = wave + t * STRIDE;
@@ -1006,7 +1022,7 @@ __global__ __launch_bounds__(WV * WAVE) void skinny_decode_kernel(const T* __res
         };
         Piece<T> xb_a[PT][1], xb_b[PT][1];
         load_x(p_begin + wave, xb_a);
-        epi_early_second<EPI, HALVES>(early, rope);      // behind the first trip of W and x (waits for the position only)
+        epi_early_second<EPI, R>(early, rope);      // behind the first trip of W and x (waits for the position only)
         if constexpr (EPI != EPI_RESIDUAL) take.settle(defer, M, wave, lane, factors);
         for (int c = p_begin + wave; c < p_end; c += 2 * STRIDE) {
             if (c + STRIDE < p_end) { load_w(c + STRIDE, wa_b); load_x(c + STRIDE, xb_b); }
@@ -1017,10 +1033,10 @@ __global__ __launch_bounds__(WV * WAVE) void skinny_decode_kernel(const T* __res
     }
     if constexpr (SHARE_LDS) {
         __syncthreads();                   // every wavefront has taken its operands from the staged rows
-        skinny_finish<T, TOUT, 1, NT, EPI, WV, true, HALVES>(acc, y, M, N, I, rope, reinterpret_cast<float*>(staged_rows),
+        skinny_finish<T, TOUT, 1, NT, EPI, WV, true, R>(acc, y, M, N, I, rope, reinterpret_cast<float*>(staged_rows),
                                                              norm.pend, norm.n_pend, &early, defer, factors);
     } else {
-        skinny_finish<T, TOUT, 1, NT, EPI, WV, false, HALVES>(acc, y, M, N, I, rope, nullptr, norm.pend, norm.n_pend, &early,
+        skinny_finish<T, TOUT, 1, NT, EPI, WV, false, R>(acc, y, M, N, I, rope, nullptr, norm.pend, norm.n_pend, &early,
                                                               defer, factors);
     }
 }
@@ -1187,14 +1203,38 @@ static int launch_nt(const void* x, const void* W, void* y, int M, int N, int K,
     return NI_LAUNCH_RESULT();
 }
 
-// Workgroups: a launch of no more than this many is doubled by halving the tiles.  A halved workgroup issues the loads of a
-// whole tile (the lanes of the other eight rows ask for the same bytes again, and a vector load costs the texture path the
-// same time whatever it fetches), so the doubled launch must still be one workgroup a compute unit: 160 pairs of tiles
-// as 320 halves put two on a quarter of the units and took 15.2 us where the 160 whole ones take 9 (the 3B shape's
-// [5120, 3072] with rotation at eight rows).
-#define HALVE_BELOW 128
 #define WIDE_BELOW 256        // workgroups: a product of one tile a workgroup and no more workgroups than this takes sixteen wavefronts
-#define HALVE_RESIDUAL_FROM 4096      // (the whole product onto the residual stream: from rows of this many elements)
+#define RESIDUAL_HALVES_FROM 4096     // elements of a row from which a whole product onto the stream is dealt out in half tiles
+#define DEAL_UNITS 256        // compute units the rows of W are dealt out to
+
+// How the decode kernel deals out the rows of W: tiles of a workgroup, and rows of W in each (16, or fewer).
+// The stacked [q; k; v] matrices of 2,560 and 3,072 pairs or 5,120 and 6,144 rows are no whole number of tiles for every
+// compute unit: some units took two workgroups where the others took one, and the launch lasted as long as those.  Dealt
+// out evenly, one workgroup of sixteen wavefronts a unit (before : now, us, at 1 / 8 / 16 rows):
+//   stored [5120, 3072] float32 19.6 : 16.4, 21.1 : 17.2, 24.7 : 19.0, bfloat16 9.1 : 7.9, 10.8 : 8.5, 13.2 : 9.8;
+//   [6144, 4096] float32 27.1 : 22.8, 28.4 : 24.5, 32.1 : 27.3, bfloat16 10.1 : 9.5, 11.4 : 10.1, 13.6 : 11.5;
+//   [4112, 2048] float32 13.1 : 11.3 ... 15.5 : 14.0, bfloat16 6.3 : 5.4 ... 8.3 : 6.8; [7000, 2048] 8 rows 16.7 : 15.7, 8.3 : 7.8;
+//   with rotation, 40 heads of 128 over 3,072 float32 20.6 : 17.6, 22.0 : 19.4, 23.5 : 20.8 (bfloat16 within 0.3);
+//   48 over 4,096 float32 26.2 : 23.6, 27.6 : 25.3.
+// A matrix of 2,049 to 4,096 rows keeps its whole tiles ([3072, 8192] as 256 workgroups of twelve rows: float32 26.4 : 25.2
+// at eight rows, bfloat16 9.6 : 10.1 at one), and so does a product in shares, whose grid the caller has chosen.
+// Eight wavefronts with half pairs, whose sums are then those of the matrix as stored.
+// Half tiles for a product of long rows onto the stream that leaves the next norm's input behind, and so cannot be cut
+// along K to fill the chip; half pairs for the few pairs of a small model (96 workgroups at the 1B shape).
+struct DecodeShape { int nt, r; };
+static DecodeShape decode_shape(int epi, int N, int K, int nt, bool given_x, bool whole, bool leaves) {
+    if (epi == EPI_SWIGLU) return {nt >= 4 ? 4 : 2, 16};
+    if (epi == EPI_ROPE) {
+        const int pairs = N / 2, each = (pairs + DEAL_UNITS - 1) / DEAL_UNITS;
+        return {2, each <= 8 ? 8 : !given_x ? 16 : each <= 10 ? 10 : each <= 12 ? 12 : 16};
+    }
+    nt = nt >= 4 ? 4 : nt >= 2 ? 2 : 1;
+    if (nt != 1 || !given_x || !whole) return {nt, 16};
+    const int each = (N + DEAL_UNITS - 1) / DEAL_UNITS;
+    if (epi == EPI_RESIDUAL && leaves && each <= 8 && K >= RESIDUAL_HALVES_FROM) return {1, 8};
+    if (epi == EPI_STORE && K >= 2048 && each > 16 && each <= 28) return {2, each <= 20 ? 10 : each <= 24 ? 12 : 14};
+    return {1, 16};
+}
 
 // The decode kernel: NT as launch_nt chooses it.  XP: pieces per wavefront of the normalising prologue, 0 without.
 template <typename T, typename TOUT, int EPI, int XP>
@@ -1215,71 +1255,72 @@ static int launch_decode(const void* x, const void* W, void* y, int M, int N, in
         }
     }
     const int out_width = (EPI == EPI_SWIGLU) ? I : N;
-    const int tiles = (out_width + 15) / 16;
-    bool defer_mismatch = false;       // the caller sized the sums of squares for another number of workgroups
-    auto run = [&](auto nt_tag) {
-        constexpr int NTc = decltype(nt_tag)::value;
-        constexpr int NOUT = (EPI == EPI_SWIGLU) ? NTc / 2 : NTc;
-        const int grid = (tiles + NOUT - 1) / NOUT;
-        // The stacked [q; k; v] matrix with rotation gives a workgroup two tiles (the partners of a
-        // rotation), which leaves a small model few workgroups (96 at the 1B shape): then two
-        // workgroups share every pair of tiles.  (For one tile a workgroup, 128 workgroups against
-        // 256, the same was measured and gained nothing: not compiled.)
-        // A whole product of long rows onto the residual stream (one that leaves the next norm's input behind, and
-        // so cannot be cut along K to fill the chip) is doubled the same way.
-        constexpr bool CAN_HALVE = EPI == EPI_ROPE || (EPI == EPI_RESIDUAL && NTc == 1 && XP == 0);
-        const bool halve = CAN_HALVE && grid <= HALVE_BELOW &&
-                           (EPI == EPI_ROPE || (K >= HALVE_RESIDUAL_FROM && splits == 1 && defer.xn != nullptr &&
-                                                2 * grid <= DEFER_PARTS_MAX));
-        if (defer.xn != nullptr && defer.parts != grid * (halve ? 2 : 1)) { defer_mismatch = true; return; }
-        auto launch = [&](auto wv_tag, auto sr_tag, auto halves_tag) {
-            constexpr int WVc = decltype(wv_tag)::value, SRc = decltype(sr_tag)::value, Hc = decltype(halves_tag)::value;
+    const DecodeShape shape = decode_shape(EPI, N, K, NT, XP == 0, splits == 1, defer.xn != nullptr);
+    int status = 0;
+    auto run = [&](auto nt_tag, auto r_tag) {
+        constexpr int NTc = decltype(nt_tag)::value, Rc = decltype(r_tag)::value;
+        constexpr int PER_WG = (EPI == EPI_SWIGLU || EPI == EPI_ROPE ? NTc / 2 : NTc) * Rc;      // columns, pairs of columns
+        const int grid = ((EPI == EPI_ROPE ? out_width / 2 : out_width) + PER_WG - 1) / PER_WG;
+        if (defer.xn != nullptr && defer.parts != grid) { status = -11; return; }       // sized for another number of workgroups
+        auto launch = [&](auto wv_tag, auto sr_tag) {
+            constexpr int WVc = decltype(wv_tag)::value, SRc = decltype(sr_tag)::value;
             if constexpr (XP > 0 && SRc > 0) {
                 if (norm.n_pend > 0) {
-                    skinny_decode_kernel<T, TOUT, NTc, EPI, XP, WVc, SRc, Hc, PRO_NORM, true>
-                        <<<dim3(grid * Hc, splits), WVc * WAVE, 0, stream>>>((const T*)x, (const T*)W, (TOUT*)y, M, N, K, I,
-                                                                              rope, norm, splits, defer);
+                    skinny_decode_kernel<T, TOUT, NTc, EPI, XP, WVc, SRc, Rc, PRO_NORM, true>
+                        <<<dim3(grid, splits), WVc * WAVE, 0, stream>>>((const T*)x, (const T*)W, (TOUT*)y, M, N, K, I,
+                                                                         rope, norm, splits, defer);
                     return;
                 }
             }
-            skinny_decode_kernel<T, TOUT, NTc, EPI, XP, WVc, SRc, Hc><<<dim3(grid * Hc, splits), WVc * WAVE, 0, stream>>>(
+            skinny_decode_kernel<T, TOUT, NTc, EPI, XP, WVc, SRc, Rc><<<dim3(grid, splits), WVc * WAVE, 0, stream>>>(
                 (const T*)x, (const T*)W, (TOUT*)y, M, N, K, I, rope, norm, splits, defer);
         };
-        using One = std::integral_constant<int, 1>;
-        using Two = std::integral_constant<int, 2>;
         using Waves8 = std::integral_constant<int, GV_WAVES>;
-        auto with_halves = [&](auto wv_tag, auto sr_tag) {
-            if constexpr (CAN_HALVE) {
-                if (halve) { launch(wv_tag, sr_tag, Two{}); return; }
-            }
-            launch(wv_tag, sr_tag, One{});
-        };
-        if constexpr (XP == 0 && NTc == 1) {
-            // rows of 2,048 elements or more in few workgroups: sixteen wavefronts each
+        if constexpr (XP == 0 && (NTc == 1 || (Rc != 16 && Rc != 8))) {
+            // rows of 2,048 elements or more in no more workgroups than compute units: sixteen wavefronts each
             if (grid <= WIDE_BELOW && K >= 2048) {
-                with_halves(std::integral_constant<int, 16>{}, std::integral_constant<int, 0>{});
+                launch(std::integral_constant<int, 16>{}, std::integral_constant<int, 0>{});
                 return;
             }
         }
         if constexpr ((XP == 4 || (XP == 8 && std::is_same<T, float>::value)) && NTc <= 2) {
             // up to eight rows: the prologue staged through LDS (its rows and the partial sums both fit),
             // compiled for 1, 4 and 8 rows
-            if (M == 1) { with_halves(Waves8{}, std::integral_constant<int, 1>{}); return; }
-            if (M <= 4) { with_halves(Waves8{}, std::integral_constant<int, 4>{}); return; }
-            if (M <= 8) { with_halves(Waves8{}, std::integral_constant<int, 8>{}); return; }
+            if (M == 1) { launch(Waves8{}, std::integral_constant<int, 1>{}); return; }
+            if (M <= 4) { launch(Waves8{}, std::integral_constant<int, 4>{}); return; }
+            if (M <= 8) { launch(Waves8{}, std::integral_constant<int, 8>{}); return; }
         }
-        with_halves(Waves8{}, std::integral_constant<int, 0>{});
+        launch(Waves8{}, std::integral_constant<int, 0>{});
     };
-    if constexpr (EPI != EPI_ROPE) {
-        if (NT >= 4) { run(std::integral_constant<int, 4>{}); return defer_mismatch ? -11 : NI_LAUNCH_RESULT(); }
+    using C1 = std::integral_constant<int, 1>;
+    using C2 = std::integral_constant<int, 2>;
+    using C4 = std::integral_constant<int, 4>;
+    using R8 = std::integral_constant<int, 8>;
+    using R10 = std::integral_constant<int, 10>;
+    using R12 = std::integral_constant<int, 12>;
+    using R14 = std::integral_constant<int, 14>;
+    using R16 = std::integral_constant<int, 16>;
+    if constexpr (EPI == EPI_ROPE) {
+        if (shape.r == 8) run(C2{}, R8{});
+        else if (XP == 0 && shape.r == 10) { if constexpr (XP == 0) run(C2{}, R10{}); }
+        else if (XP == 0 && shape.r == 12) { if constexpr (XP == 0) run(C2{}, R12{}); }
+        else run(C2{}, R16{});
+    } else if (shape.nt == 4) {
+        run(C4{}, R16{});
+    } else if (shape.nt == 2) {
+        if constexpr (XP == 0 && EPI == EPI_STORE) {
+            if (shape.r == 10) { run(C2{}, R10{}); return status != 0 ? status : NI_LAUNCH_RESULT(); }
+            if (shape.r == 12) { run(C2{}, R12{}); return status != 0 ? status : NI_LAUNCH_RESULT(); }
+            if (shape.r == 14) { run(C2{}, R14{}); return status != 0 ? status : NI_LAUNCH_RESULT(); }
+        }
+        run(C2{}, R16{});
+    } else if constexpr (EPI != EPI_SWIGLU) {
+        if constexpr (XP == 0 && EPI == EPI_RESIDUAL) {
+            if (shape.r == 8) { run(C1{}, R8{}); return status != 0 ? status : NI_LAUNCH_RESULT(); }
+        }
+        run(C1{}, R16{});
     }
-    if constexpr (EPI == EPI_SWIGLU || EPI == EPI_ROPE) {
-        run(std::integral_constant<int, 2>{});
-    } else {
-        if (NT >= 2) run(std::integral_constant<int, 2>{});
-        else run(std::integral_constant<int, 1>{});
-    }
-    return defer_mismatch ? -11 : NI_LAUNCH_RESULT();
+    return status != 0 ? status : NI_LAUNCH_RESULT();
 }
 
 // The kernel for 17 to 64 rows: MB blocks of 16 rows, NT as launch_nt chooses it, within the eight
@@ -1323,12 +1364,14 @@ static int launch_rows(const void* x, const void* W, void* y, int M, int N, int 
 // Workgroups of a product onto the residual stream of M rows and N columns, which is how many sums of squares
 // a row gets where the product leaves them behind for the next norm (DeferArgs): the launchers above, mirrored.
 static int residual_parts(int M, int N, int K, int tiles_per_group) {
+    if (M <= 16) {
+        const DecodeShape shape = decode_shape(EPI_RESIDUAL, N, K, tiles_per_group, true, true, true);
+        return (N + shape.nt * shape.r - 1) / (shape.nt * shape.r);
+    }
     const int tiles = (N + 15) / 16;
     int nt = tiles_per_group >= 4 ? 4 : tiles_per_group >= 2 ? 2 : 1;
     if (M > 32 && nt == 4) nt = 2;       // three and four blocks of sixteen rows hold at most two tiles a workgroup
-    const int grid = (tiles + nt - 1) / nt;
-    if (M > 16) return grid * nt;        // past sixteen rows every tile leaves its own sums
-    return (nt == 1 && grid <= HALVE_BELOW && 2 * grid <= DEFER_PARTS_MAX && K >= HALVE_RESIDUAL_FROM) ? 2 * grid : grid;
+    return (tiles + nt - 1) / nt * nt;   // past sixteen rows every tile leaves its own sums
 }
 
 template <typename T, typename TOUT, int EPI>
@@ -1528,7 +1571,7 @@ static int launch_merged(const NormArgs& merge, const void* W, void* y, int M, i
     if (defer.ss_in != nullptr || (defer.xn != nullptr && EPI != EPI_RESIDUAL)) return -11;
     auto go = [&](auto sr_tag) {
         constexpr int SRc = decltype(sr_tag)::value;
-        skinny_decode_kernel<bf16_t, TOUT, 1, EPI, 4, GV_WAVES, SRc, 1, PRO_MERGE><<<tiles, GV_THREADS, 0, stream>>>(
+        skinny_decode_kernel<bf16_t, TOUT, 1, EPI, 4, GV_WAVES, SRc, 16, PRO_MERGE><<<tiles, GV_THREADS, 0, stream>>>(
             nullptr, (const bf16_t*)W, (TOUT*)y, M, N, K, 0, RopeArgs{}, merge, 1, defer);
     };
     if (M == 1) go(std::integral_constant<int, 1>{});

@@ -1059,14 +1059,16 @@ def qkv_rope_ok(M: int, K: int, hd: int, rotary_dim: int, dtype: torch.dtype) ->
     return skinny_ok(M, K, dtype) and hd % 32 == 0 and rotary_dim == hd
 
 
-def qkv_rope_wins(M: int, K: int, dtype: torch.dtype) -> bool:
+def qkv_rope_wins(M: int, K: int, dtype: torch.dtype, weight=None) -> bool:
     """Whether that fused product is also faster than the library's product and the rotation kernel behind it.
     In bfloat16 always (17 to 64 rows of the 1B / 3B / 8B shapes: 7.2 : 12.9, 13.0 : 16.5, 20.7 : 21.8 us at 64 rows).
-    In float32 for rows of up to 2,048 elements, and for up to 16 rows of 4,096 or more: the 3B shape's
-    [5120, 3072] takes 29.5 : 22.4 at 8 rows and 41.2 : 33.1 at 64 (a float32 decode step of that shape at batch 8:
-    4.72 ms fused, 4.62 with the library), the 8B shape's [6144, 4096] 28.1 : 27.9 and 56.2 : 43.1 (a step at batch 8:
-    7.91 ms fused, 8.13 with the library; at batch 64 the library gains)."""
-    return dtype != torch.float32 or K <= 2048 or (M <= SKINNY_BEST_ROWS and K >= 4096)
+    In float32 for rows of up to 2,048 elements, and for up to 16 rows of any length with a re-tiled matrix, whose rows
+    are dealt out evenly over the compute units (the 3B shape's [5120, 3072] takes 19.4 us at 8 rows where the product and
+    the rotation kernel take 17.2 and 4.7, and at 16 rows 20.8 : 19.0 and 4.7), or of 4,096 or more with one as stored
+    (the 8B shape's [6144, 4096]: a step at batch 8 7.91 ms fused, 8.13 with the library).  Past 16 rows the library
+    gains: 41.2 : 33.1 and 56.2 : 43.1 at 64 rows."""
+    return dtype != torch.float32 or K <= 2048 or (M <= SKINNY_BEST_ROWS and
+                                                   (K >= 4096 or (isinstance(weight, Weight) and weight.tiles is not None)))
 
 
 def skinny_qkv_rope(x, w_qkv, positions: torch.Tensor, cos: torch.Tensor,

@@ -291,7 +291,7 @@ class Attention(Part):
             return False
         tables = self.position.tables()
         return (tables is not None and K.qkv_rope_ok(T, d, self.hd, 2 * tables[0].shape[1], dtype)
-                and K.qkv_rope_wins(T, d, dtype))
+                and K.qkv_rope_wins(T, d, dtype, self.w_qkv))
 
     def takes_normed(self, T: int) -> bool:
         """Whether ``forward`` takes the norm before it as a prologue of its first product for T tokens."""
