@@ -89,6 +89,72 @@ template <> struct Piece<float> {
     }
 };
 
+// Products of one tile of sixteen rows of W with the rows of x, summed over the pieces a wavefront takes.  COLS: the rows
+// of x there can be.  16: the accumulator of the 16 x 16 instructions as it is.  4 or 8, float32 only: a
+// v_mfma_f32_4x4x1_f32 multiplies sixteen blocks of 4 x 4 in 8 cycles, where the 16 x 16 x 4 instruction, whose rows of x
+// past those that exist are waste, takes 32.  The lanes of a piece as they are make the blocks: block (kg, r / 4) holds
+// four rows at the k of kg, and four rows of x, the lanes 4 h .. 4 h + 3 of kg, are handed to the four blocks of kg by the
+// instruction itself (cbsz, abid).  The four sums over kg meet at the end.  (The rows of x have to stay where they are,
+// each in its own lane with the lanes behind them on the last: loaded anew for every block the same lines are asked for
+// four times, and [3072, 8192] took 25.5 us at four rows where this takes 22.0 and the 16 x 16 instructions 24.4.)
+// Measured, 16 x 16 : 4 x 4, us: the head [128256, 3072] at 1 / 4 / 8 rows 302 : 268, 320 : 270, 339 : 281 (5.6 TB/s),
+// [128256, 2048] 197 : 194, 206 : 192, 216 : 193; [3072, 8192] 23.7 : 20.9, 24.4 : 22.0, 26.5 : 24.8; [5120, 3072] 16.5 : 14.7,
+// 17.1 : 15.2, 17.6 : 16.4; stacked [16384, 3072] 39.2 : 37.3, 38.8 : 37.3, 39.9 : 38.2; [2048, 2048] 7.8 : 7.3, 8.2 : 7.8, 8.7 : 8.7.
+// Eight rows of short rows of W lose at the end what they gain ([576, 192] 3.6 : 3.8): 16 x 16 there (with_cols).  Nine to
+// twelve rows the same way, a third instruction, gain nothing (head 358 : 351 and 229 : 239, [5120, 3072] 19.2 : 21.0).
+// A sum is of a quarter of the terms, four of them added: no less exact ([3072, 8192] 5.2e-7 : 2.5e-7 of the largest).
+template <typename T, int COLS>
+struct TileSum {
+    floatx4_t v = {0.f, 0.f, 0.f, 0.f};
+    // one piece of x with the pieces of the workgroup's NT tiles
+    template <int NT>
+    static __device__ __forceinline__ void add(TileSum (&sum)[NT][1], const Piece<T> (&a)[NT], const Piece<T>& b) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) sum[nt][0].v = Piece<T>::mma(a[nt], b, sum[nt][0].v);
+    }
+    // sums[lane * 4 + i]: the layout the epilogues read, D[n][m] at lane (n / 4) * 16 + m, register n % 4
+    __device__ __forceinline__ void leave(float* sums, int lane) const {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sums[lane * 4 + i] = v[i];
+    }
+};
+__device__ __forceinline__ float sum_over_kg(float x) {      // lanes r, r + 16, r + 32, r + 48
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+template <int COLS> struct FewRowsSum {
+    floatx4_t v[COLS / 4];         // lane (kg, r): row r of W with the rows 4 h + i of x, over the k of kg
+    __device__ __forceinline__ FewRowsSum() {
+#pragma unroll
+        for (int h = 0; h < COLS / 4; ++h) v[h] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    template <int NT, typename Sum>
+    static __device__ __forceinline__ void add(Sum (&sum)[NT][1], const Piece<float> (&w)[NT], const Piece<float>& x) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                floatx4_t (&c)[COLS / 4] = sum[nt][0].v;
+                c[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(x.v[i], w[nt].v[i], c[0], 2, 0, 0);
+                if constexpr (COLS > 4) c[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(x.v[i], w[nt].v[i], c[1], 2, 1, 0);
+            }
+    }
+    __device__ __forceinline__ void leave(float* sums, int lane) const {
+        const int r = lane % 16, kg = lane / 16;
+#pragma unroll
+        for (int h = 0; h < COLS / 4; ++h)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float s = sum_over_kg(v[h][i]);
+                if (kg == h) sums[((r / 4) * 16 + 4 * h + i) * 4 + r % 4] = s;
+            }
+    }
+};
+template <> struct TileSum<float, 4> : FewRowsSum<4> {};
+template <> struct TileSum<float, 8> : FewRowsSum<8> {};
+
 enum { EPI_STORE = 0, EPI_SWIGLU = 1, EPI_ROPE = 2, EPI_RESIDUAL = 3 };
 
 // The normalising prologue's inputs.
@@ -259,8 +325,8 @@ __device__ __forceinline__ void epi_early_second(EpiEarly& e, const RopeArgs& ro
 // epilogue stores them.
 // R: the rows of W (columns of the result, pairs with rotation) that each tile of the workgroup holds, in its
 // first R columns.
-template <typename T, typename TOUT, int MB, int NT, int EPI, int WV = GV_WAVES, bool EXT = false, int R = 16>
-__device__ __forceinline__ void skinny_finish(const floatx4_t (&acc)[NT][MB], TOUT* __restrict__ y, int M, int N, int I,
+template <typename T, typename TOUT, int MB, int NT, int EPI, int WV = GV_WAVES, bool EXT = false, int R = 16, int COLS = 16>
+__device__ __forceinline__ void skinny_finish(const TileSum<T, COLS> (&acc)[NT][MB], TOUT* __restrict__ y, int M, int N, int I,
                                               const RopeArgs& rope, float* ext = nullptr, const float* pend = nullptr,
                                               int n_pend = 0, const EpiEarly* early = nullptr,
                                               const DeferArgs& defer = DeferArgs{}, const float* factors = nullptr) {
@@ -280,9 +346,7 @@ __device__ __forceinline__ void skinny_finish(const floatx4_t (&acc)[NT][MB], TO
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) red[wave][nt * MB + mb][lane * 4 + i] = acc[nt][mb][i];
+        for (int mb = 0; mb < MB; ++mb) acc[nt][mb].leave(red[wave][nt * MB + mb], lane);
     __syncthreads();
     // the row's factor where the product stands behind a norm whose division it makes itself (1 otherwise)
     const bool scaled = EPI != EPI_RESIDUAL && factors != nullptr && defer.ss_in != nullptr;
@@ -584,7 +648,7 @@ __device__ __forceinline__ void skinny_finish(const floatx4_t (&acc)[NT][MB], TO
     }
 }
 
-template <typename T, typename TOUT, int MB, int NT, int EPI>
+template <typename T, typename TOUT, int MB, int NT, int EPI, int COLS = 16>
 __global__ __launch_bounds__(GV_THREADS) void skinny_gemm_kernel(const T* __restrict__ x, const T* __restrict__ W,
                                                                  TOUT* __restrict__ y, int M, int N, int K, int I,
                                                                  RopeArgs rope, GatedUnit glu) {
@@ -618,11 +682,8 @@ __global__ __launch_bounds__(GV_THREADS) void skinny_gemm_kernel(const T* __rest
         xrow[mb] = x + static_cast<size_t>(min(m, M - 1)) * K;
     }
 
-    floatx4_t acc[NT][MB];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb) acc[nt][mb] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    static_assert(COLS == 16 || MB == 1, "several blocks of rows are whole");
+    TileSum<T, COLS> acc[NT][MB];
 
     // PT pieces per trip, all their loads issued before the first multiply, to keep enough bytes in
     // flight; the wavefront covers pieces [first + wave * per_wave, ...) of its K range in order.
@@ -646,15 +707,19 @@ __global__ __launch_bounds__(GV_THREADS) void skinny_gemm_kernel(const T* __rest
         }
 #pragma unroll
         for (int u = 0; u < PT; ++u)
+            if constexpr (MB == 1) {
+                TileSum<T, COLS>::add(acc, wa[u], xb[u][0]);
+            } else {
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
+                for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-                for (int mb = 0; mb < MB; ++mb) acc[nt][mb] = Piece<T>::mma(wa[u][nt], xb[u][mb], acc[nt][mb]);
+                    for (int mb = 0; mb < MB; ++mb) acc[nt][mb].v = Piece<T>::mma(wa[u][nt], xb[u][mb], acc[nt][mb].v);
+            }
     }
 
     DeferArgs defer;
     defer.glu = glu;
-    skinny_finish<T, TOUT, MB, NT, EPI>(acc, y, M, N, I, rope, nullptr, nullptr, 0, nullptr, defer);
+    skinny_finish<T, TOUT, MB, NT, EPI, GV_WAVES, false, 16, COLS>(acc, y, M, N, I, rope, nullptr, nullptr, 0, nullptr, defer);
 }
 
 // The decode step's kernel: at most 16 rows, W re-tiled (and zero-padded to whole pieces, so a lane
@@ -675,7 +740,7 @@ __global__ __launch_bounds__(GV_THREADS) void skinny_gemm_kernel(const T* __rest
 // adds to its rows.  A kernel of its own, because the addends wait in registers beside the rows of h while the
 // first pieces of W are asked for: for eight rows that is 172 registers instead of 120, one workgroup a compute
 // unit instead of two, which the products without addends should not pay.
-template <typename T, typename TOUT, int NT, int EPI, int XP, int WV, int SR, int R = 16, int PRO = PRO_NORM, bool PEND = false>
+template <typename T, typename TOUT, int NT, int EPI, int XP, int WV, int SR, int R = 16, int PRO = PRO_NORM, bool PEND = false, int COLS = 16>
 __global__ __launch_bounds__(WV * WAVE) void skinny_decode_kernel(const T* __restrict__ x, const T* __restrict__ W,
                                                                    TOUT* __restrict__ y, int M, int N, int K, int I,
                                                                    RopeArgs rope, NormArgs norm, int splits, DeferArgs defer) {
@@ -729,9 +794,7 @@ __global__ __launch_bounds__(WV * WAVE) void skinny_decode_kernel(const T* __res
         wrow[nt] = W + static_cast<size_t>(min(tile, limit)) * pieces * (WAVE * EL) + (kg * 16 + tile_row) * EL;
     }
 
-    floatx4_t acc[NT][1];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[nt][0] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    TileSum<T, COLS> acc[NT][1];
 
     // PT pieces per trip; trip t of a wavefront covers pieces wave + (t * PT + u) * 8.  Two trips are
     // in registers at a time, in two fixed sets (A and B): one is multiplied while the other's loads
@@ -752,14 +815,12 @@ __global__ __launch_bounds__(WV * WAVE) void skinny_decode_kernel(const T* __res
     auto multiply = [&](int c, const Piece<T> (&wa)[PT][NT], const Piece<T> (&xb)[PT][1]) {
 #pragma unroll
         for (int u = 0; u < PT; ++u) {
-            if (c + u * WV < p_end) {
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) acc[nt][0] = Piece<T>::mma(wa[u][nt], xb[u][0], acc[nt][0]);
-            }
+            if (c + u * WV < p_end) TileSum<T, COLS>::add(acc, wa[u], xb[u][0]);
         }
     };
 
     Piece<T> wa_a[PT][NT], wa_b[PT][NT];
+    static_assert(COLS == 16 || XP == 0 || SR > 0, "a prologue that is not staged takes whole blocks");
     const int row = min(r, M - 1);       // columns of rows that do not exist are computed from the last row and not stored
     if constexpr (XP > 0) {
         // Normalising prologue: this lane's elements of its row of h for every piece of the wavefront
@@ -1033,10 +1094,10 @@ __global__ __launch_bounds__(WV * WAVE) void skinny_decode_kernel(const T* __res
     }
     if constexpr (SHARE_LDS) {
         __syncthreads();                   // every wavefront has taken its operands from the staged rows
-        skinny_finish<T, TOUT, 1, NT, EPI, WV, true, R>(acc, y, M, N, I, rope, reinterpret_cast<float*>(staged_rows),
+        skinny_finish<T, TOUT, 1, NT, EPI, WV, true, R, COLS>(acc, y, M, N, I, rope, reinterpret_cast<float*>(staged_rows),
                                                              norm.pend, norm.n_pend, &early, defer, factors);
     } else {
-        skinny_finish<T, TOUT, 1, NT, EPI, WV, false, R>(acc, y, M, N, I, rope, nullptr, norm.pend, norm.n_pend, &early,
+        skinny_finish<T, TOUT, 1, NT, EPI, WV, false, R, COLS>(acc, y, M, N, I, rope, nullptr, norm.pend, norm.n_pend, &early,
                                                               defer, factors);
     }
 }
@@ -1104,11 +1165,7 @@ __global__ __launch_bounds__(GV_THREADS) void skinny_rows_kernel(const T* __rest
         const int limit = (N + 15) / 16 - 1;         // a workgroup's last tiles may lie past the matrix: read the last one, store nothing
         wrow[nt] = W + static_cast<size_t>(min((col0 + shift) / 16, limit)) * pieces * (WAVE * EL) + lane * EL;
     }
-    floatx4_t acc[NT][MB];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb) acc[nt][mb] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    TileSum<T, 16> acc[NT][MB];
 
     // pieces past the end of a row are read from its last piece and not multiplied: no load is under a branch
     auto load_w = [&](int c, Piece<T> (&wa)[NT]) {
@@ -1148,7 +1205,7 @@ __global__ __launch_bounds__(GV_THREADS) void skinny_rows_kernel(const T* __rest
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-            for (int mb = 0; mb < MB; ++mb) acc[nt][mb] = Piece<T>::mma(wa[nt], xb[mb], acc[nt][mb]);
+            for (int mb = 0; mb < MB; ++mb) acc[nt][mb].v = Piece<T>::mma(wa[nt], xb[mb], acc[nt][mb].v);
     };
 
     Piece<T> wa_a[NT], wa_b[NT];
@@ -1179,6 +1236,18 @@ __global__ __launch_bounds__(GV_THREADS) void skinny_rows_kernel(const T* __rest
                                                   defer, factors);
 }
 
+// Calls f with the number of rows of x its kernel is to be compiled for (TileSum): by the rows and the length of a row
+// alone, so that every kernel takes a product's sums in the same order.
+#define EIGHT_COLS_ABOVE 1024      // elements of a row; also what four pieces a wavefront of a normalising prologue hold
+template <typename T, typename F>
+static void with_cols(int M, int K, F f) {
+    if constexpr (std::is_same<T, float>::value) {
+        if (M <= 4) { f(std::integral_constant<int, 4>{}); return; }
+        if (M <= 8 && K > EIGHT_COLS_ABOVE) { f(std::integral_constant<int, 8>{}); return; }
+    }
+    f(std::integral_constant<int, 16>{});
+}
+
 template <typename T, typename TOUT, int MB, int EPI>
 static int launch_nt(const void* x, const void* W, void* y, int M, int N, int K, int I, int NT,
                      hipStream_t stream, RopeArgs rope = RopeArgs{}, GatedUnit glu = GatedUnit{}) {
@@ -1188,7 +1257,12 @@ static int launch_nt(const void* x, const void* W, void* y, int M, int N, int K,
         constexpr int NTc = decltype(nt_tag)::value;
         constexpr int NOUT = (EPI == EPI_SWIGLU) ? NTc / 2 : NTc;
         const int grid = (tiles + NOUT - 1) / NOUT;
-        skinny_gemm_kernel<T, TOUT, MB, NTc, EPI><<<grid, GV_THREADS, 0, stream>>>((const T*)x, (const T*)W, (TOUT*)y, M, N, K, I, rope, glu);
+        auto with = [&](auto cols_tag) {
+            skinny_gemm_kernel<T, TOUT, MB, NTc, EPI, decltype(cols_tag)::value><<<grid, GV_THREADS, 0, stream>>>(
+                (const T*)x, (const T*)W, (TOUT*)y, M, N, K, I, rope, glu);
+        };
+        if constexpr (MB == 1) with_cols<T>(M, K, with);
+        else with(std::integral_constant<int, 16>{});
     };
     // NT * MB fragments of partial sums share 64 KB of LDS: at most 8
     if constexpr (MB <= 2 && EPI != EPI_ROPE) {
@@ -1206,6 +1280,13 @@ static int launch_nt(const void* x, const void* W, void* y, int M, int N, int K,
 #define WIDE_BELOW 256        // workgroups: a product of one tile a workgroup and no more workgroups than this takes sixteen wavefronts
 #define RESIDUAL_HALVES_FROM 4096     // elements of a row from which a whole product onto the stream is dealt out in half tiles
 #define DEAL_UNITS 256        // compute units the rows of W are dealt out to
+
+// The rows of x that a kernel with a prologue of XP pieces a wavefront staged for SR rows is compiled for (0: not staged):
+// as with_cols has it.
+template <typename T>
+constexpr int staged_cols(int SR, int XP) {
+    return !std::is_same<T, float>::value || SR == 0 ? 16 : SR <= 4 ? 4 : XP * GV_WAVES * 32 > EIGHT_COLS_ABOVE ? 8 : 16;
+}
 
 // How the decode kernel deals out the rows of W: tiles of a workgroup, and rows of W in each (16, or fewer).
 // The stacked [q; k; v] matrices of 2,560 and 3,072 pairs or 5,120 and 6,144 rows are no whole number of tiles for every
@@ -1266,14 +1347,19 @@ static int launch_decode(const void* x, const void* W, void* y, int M, int N, in
             constexpr int WVc = decltype(wv_tag)::value, SRc = decltype(sr_tag)::value;
             if constexpr (XP > 0 && SRc > 0) {
                 if (norm.n_pend > 0) {
-                    skinny_decode_kernel<T, TOUT, NTc, EPI, XP, WVc, SRc, Rc, PRO_NORM, true>
+                    skinny_decode_kernel<T, TOUT, NTc, EPI, XP, WVc, SRc, Rc, PRO_NORM, true, staged_cols<T>(SRc, XP)>
                         <<<dim3(grid, splits), WVc * WAVE, 0, stream>>>((const T*)x, (const T*)W, (TOUT*)y, M, N, K, I,
                                                                          rope, norm, splits, defer);
                     return;
                 }
             }
-            skinny_decode_kernel<T, TOUT, NTc, EPI, XP, WVc, SRc, Rc><<<dim3(grid, splits), WVc * WAVE, 0, stream>>>(
-                (const T*)x, (const T*)W, (TOUT*)y, M, N, K, I, rope, norm, splits, defer);
+            auto with = [&](auto cols_tag) {
+                skinny_decode_kernel<T, TOUT, NTc, EPI, XP, WVc, SRc, Rc, PRO_NORM, false, decltype(cols_tag)::value>
+                    <<<dim3(grid, splits), WVc * WAVE, 0, stream>>>((const T*)x, (const T*)W, (TOUT*)y, M, N, K, I, rope, norm,
+                                                                     splits, defer);
+            };
+            if constexpr (XP == 0) with_cols<T>(M, K, with);
+            else with(std::integral_constant<int, staged_cols<T>(SRc, XP)>{});
         };
         using Waves8 = std::integral_constant<int, GV_WAVES>;
         if constexpr (XP == 0 && (NTc == 1 || (Rc != 16 && Rc != 8))) {
