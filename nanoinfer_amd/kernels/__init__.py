@@ -408,7 +408,8 @@ def build_q_tiles(q_start, q_len, context_len, tile_tokens: int):
     return [x for t in tiles for x in t]
 
 
-def mfma_splits(n_tiles: int, kv_heads: int, group: int, max_keys: int) -> int:
+def mfma_splits(n_tiles: int, kv_heads: int, group: int, max_keys: int, hd: int = 64,
+                dtype: torch.dtype = torch.bfloat16) -> int:
     """Into how many runs the matrix-core kernel cuts the keys of every tile.  Cutting costs a
     second kernel that merges the runs, and float32 partial results in between: a step with many
     tiles is cut only into runs of 2,048 keys or more, up to about a thousand workgroups (measured
@@ -416,9 +417,28 @@ def mfma_splits(n_tiles: int, kv_heads: int, group: int, max_keys: int) -> int:
     every compute unit (2,048 tokens in tiles of 32 at contexts of 4,096 / 8,192 / 32,768: 88 / 180 / 721 us
     uncut, 99 / 192 / 741 in two runs; 1,024 tokens, one tile a unit: 75 / 142 uncut, 64 / 114 in two);
     a step with fewer tiles than the chip has compute units, into runs of 512 keys or more until
-    every unit has one."""
+    every unit has one.
+
+    In float32 a key costs sixteen times the matrix instructions and the merge is the same, so a cut pays much sooner:
+    runs of 32 keys or more, up to two workgroups a compute unit, whose wavefronts then multiply while others take
+    exponentials (a workgroup alone on a unit leaves one wavefront on each matrix core).  A workgroup more than that
+    where two would be left uneven: three runs up to 256 tiles of head size 64 or less, two up to 512 tiles (1,024 of
+    small heads, whose workgroups are small).  Measured, uncut and by the rule above : by this one, us: head size 64,
+    8 kv heads, 60 tokens at 900 keys 77.9 : 24.8; 164 at 1,700 82.5 : 57.1; 256 at 256 / 1,024 27.5 : 23.2,
+    56.1 : 47.3; 512 at 512 / 1,024 / 1,536 / 4,096 49.6 : 46.4, 91.4 : 74.8, 132 : 102, 243 : 231; 1,024 at 1,024 95.6 : 90.0
+    (2,048 at 2,048: 255 uncut, 268 in two); head size 128, 60 at 900 138.5 : 41.7, 164 at 1,700 141.5 : 105.9, 512 at 1,536
+    234 : 198, 1,024 at 1,024 178.5 : 168.0 (in three 220); head size 32, one kv head, 32 at 500 keys 30.9 : 10.6; head size 256,
+    2 kv heads, 256 at 256 86.5 : 35.0, 1,024 at 1,024 185.8 : 129.5.  Under 256 keys the cut gains less than the launch of the
+    merge costs a host that is behind (32 tokens at 200 keys 16.2 : 10 us, but five prompts through a small model 7.2 : 7.4 ms)."""
     hpt = _heads_per_tile(group)
     items = max(1, n_tiles * kv_heads * ((group + hpt - 1) // hpt))
+    if dtype == torch.float32:
+        runs = 2 * COMPUTE_UNITS // items
+        if hd <= 64 and 1 <= runs <= 2 and (runs + 1) * items <= 3 * COMPUTE_UNITS:
+            runs += 1
+        if runs <= 1 and items > COMPUTE_UNITS and items <= (2 if hd > 48 else 4) * COMPUTE_UNITS:
+            runs = 2
+        return int(max(1, min(runs, max_keys // 32 if max_keys >= 256 else 1, 16)))
     many = min(1024 // items if items < 2 * COMPUTE_UNITS else 1, max_keys // 2048)
     few = min(COMPUTE_UNITS // items, max_keys // 512)
     return int(max(1, min(max(many, few), 16)))

@@ -365,7 +365,7 @@ class Attention(Part):
             tiles = ctx.q_tiles(tile_tokens)
         if tiles is not None:
             if nsplit is None:
-                nsplit = K.mfma_splits(tiles.shape[0], self.KVH, self.H // self.KVH, max_keys)
+                nsplit = K.mfma_splits(tiles.shape[0], self.KVH, self.H // self.KVH, max_keys, self.hd, dtype)
             ws = ctx.workspace(T * self.H * nsplit * (self.hd + 2)) if nsplit > 1 else None
             K.mfma_attention(qkv, cache.kpool, cache.vpool, cache.block_table, tiles, out, self.H, self.KVH, self.hd,
                              self.scale, self.window, nsplit, ws, tile_tokens)
