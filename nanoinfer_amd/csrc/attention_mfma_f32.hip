@@ -53,6 +53,14 @@ __device__ __forceinline__ float lanes4(float x, bool take_max) {
     return take_max ? fmaxf(s, t) : s + t;
 }
 
+__device__ __forceinline__ float quads4(float x, bool take_max) {
+    // over the four lanes r, r + 4, r + 8, r + 12 of sixteen (row_ror:4, then row_ror:8): maximum or sum
+    float y = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x124, 0xf, 0xf, false));
+    x = take_max ? fmaxf(x, y) : x + y;
+    y = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xf, 0xf, false));
+    return take_max ? fmaxf(x, y) : x + y;
+}
+
 template <bool POW2>
 __global__ __launch_bounds__(MA_WAVES * WAVE) void mfma_attention_f32_kernel(
     const float* __restrict__ q, int q_stride, const float* __restrict__ kpool, const float* __restrict__ vpool,
@@ -357,7 +365,19 @@ NI_EXPORT int ni_mfma_attention_f32(const void* q, int q_stride, const void* kpo
 #define DEC_KEYS 16
 #define DEC_DEPTH 2
 
-template <bool POW2>
+//
+// FEW (up to four query heads a kv head, the usual group): rows of a 16 x 16 product past those heads are waste, and a
+// step of sixteen keys at head size 128 is 64 instructions of 32 cycles one behind the other on a wavefront that has its
+// matrix core to itself.  v_mfma_f32_4x4x1_f32 multiplies sixteen blocks of 4 x 4 in 8 cycles: block (kg, r / 4) is four
+// keys or dims by four heads.
+//   scores: A lane (r, kg) as above, B the head r % 4 at the same dims; lane (r, kg) gets the keys 4 * (r/4) + i of its head,
+//     one quarter of the dims, and the four kg are added up.
+//   output: A lane (r, kg) holds dims (4*kg + r%4)*HD/16 .. of key 4 * (r/4) + i, B its own weights; every r / 4 sums its own
+//     keys, and they meet at the end.
+// Measured, 16 x 16 : 4 x 4, us with the merge: 8 tokens of 774 to 1,300 keys, head size 128, 24 heads on 8, in one / two /
+// four runs 39.7 : 33.3, 27.7 : 24.4, 21.8 : 20.5 (68 MB; a run of 325 keys a compute unit is what remains); head size 64, 32 on 8,
+// 8 tokens of up to 2,200 keys in two / four runs 24.9 : 21.2, 17.3 : 17.0, 40 tokens of up to 1,300 uncut 37.7 : 34.2.
+template <bool POW2, bool FEW>
 __global__ __launch_bounds__(DEC_WAVES * WAVE) void mfma_decode_f32_kernel(
     const float* __restrict__ q, int q_stride, const float* __restrict__ kpool, const float* __restrict__ vpool,
     const int32_t* __restrict__ block_table, int table_stride, const int32_t* __restrict__ seq_of_token,
@@ -370,8 +390,9 @@ __global__ __launch_bounds__(DEC_WAVES * WAVE) void mfma_decode_f32_kernel(
     constexpr int QK = HD / 4;                     // MFMAs of the first product per step; floats of Q and of a key a lane holds
     constexpr int DB = HD / 16;                    // MFMAs of the second product per 4 keys
     constexpr int DEPTH = DEC_DEPTH;
-    __shared__ __attribute__((aligned(16))) float so[NW][16][HD];      // the wavefronts' outputs, met at the end
-    __shared__ float sm_ml[NW][16][2];
+    constexpr int ROWS = FEW ? 4 : 16;
+    __shared__ __attribute__((aligned(16))) float so[NW][ROWS][HD];      // the wavefronts' outputs, met at the end
+    __shared__ float sm_ml[NW][ROWS][2];
     constexpr int TBL_MAX = 1024;
     __shared__ __attribute__((aligned(16))) int32_t tbl[TBL_MAX];
 
@@ -388,7 +409,9 @@ __global__ __launch_bounds__(DEC_WAVES * WAVE) void mfma_decode_f32_kernel(
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
     const int r = lane % 16, kg = lane / 16;
-    const int hh = chunk * 16 + r;                 // this lane's row: a query head of the group
+    const int hh = chunk * 16 + r % ROWS;          // this lane's row: a query head of the group
+    const int key4 = 4 * (FEW ? r / 4 : kg);       // first of the lane's four keys of a step
+    const int dims = (FEW ? 4 * kg + r % 4 : r) * DB;      // first of the dims it loads of their values
     const bool row_ok = hh < G;
     const int head = g * G + hh;
 
@@ -434,7 +457,7 @@ __global__ __launch_bounds__(DEC_WAVES * WAVE) void mfma_decode_f32_kernel(
     auto load_rows = [&](int ks, StepRows& rows) {
         VecIO<float, QK>::load(kpool + row_address(ks + r) + kg * QK, rows.k);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) VecIO<float, DB>::load(vpool + row_address(ks + 4 * kg + i) + r * DB, rows.v[i]);
+        for (int i = 0; i < 4; ++i) VecIO<float, DB>::load(vpool + row_address(ks + key4 + i) + dims, rows.v[i]);
     };
 
     StepRows ring[DEPTH];
@@ -455,10 +478,17 @@ __global__ __launch_bounds__(DEC_WAVES * WAVE) void mfma_decode_f32_kernel(
         auto step = [&](int j, StepRows& rows) {
             const int ks = key_lo + (wave + j * NW) * KS;
             if (j < mine) {
-                // 1. scores: this lane gets row r, keys ks + 4*kg + i
+                // 1. scores: this lane gets its row's keys ks + key4 + i
                 floatx4_t st = floatx4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int j1 = 0; j1 < QK; ++j1) st = __builtin_amdgcn_mfma_f32_16x16x4f32(rows.k[j1], qf[j1], st, 0, 0, 0);
+                for (int j1 = 0; j1 < QK; ++j1) {
+                    if constexpr (FEW) st = __builtin_amdgcn_mfma_f32_4x4x1f32(rows.k[j1], qf[j1], st, 0, 0, 0);
+                    else st = __builtin_amdgcn_mfma_f32_16x16x4f32(rows.k[j1], qf[j1], st, 0, 0, 0);
+                }
+                if constexpr (FEW) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) st[i] = lanes4(st[i], false);
+                }
                 const bool inner = ks >= lo && ks + KS - 1 <= pos;
                 float sc[4];
                 float lane_max = NEG_BIG;
@@ -466,7 +496,7 @@ __global__ __launch_bounds__(DEC_WAVES * WAVE) void mfma_decode_f32_kernel(
                 for (int i = 0; i < 4; ++i) {
                     float v = st[i];
                     if (!inner) {
-                        const int key = ks + 4 * kg + i;
+                        const int key = ks + key4 + i;
                         v = (key <= pos && key >= lo) ? v : NEG_BIG;
                     }
                     sc[i] = v;
@@ -474,7 +504,7 @@ __global__ __launch_bounds__(DEC_WAVES * WAVE) void mfma_decode_f32_kernel(
                 }
                 // 2. a row whose scores have risen far above its reference: move it, rescale what was summed
                 if (__any(lane_max - REF_SLACK > m_ref)) {
-                    const float mx = lanes4(lane_max, true);
+                    const float mx = FEW ? quads4(lane_max, true) : lanes4(lane_max, true);
                     const bool move = mx > 0.5f * NEG_BIG && mx > m_ref + REF_SLACK;
                     const float m_new = move ? mx : m_ref;
                     const float corr = move ? expf(m_ref - m_new) : 1.0f;
@@ -483,14 +513,17 @@ __global__ __launch_bounds__(DEC_WAVES * WAVE) void mfma_decode_f32_kernel(
 #pragma unroll
                     for (int db = 0; db < DB; ++db) o[db] *= corr;
                 }
-                // 3. weights, and O^T += V^T . P^T for the keys {4*kg + i} of MFMA i
+                // 3. weights, and O^T += V^T . P^T for the keys {key4 + i} of MFMA i
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     float p = expf(sc[i] - m_ref);
                     if (!inner) p = sc[i] > 0.5f * NEG_BIG ? p : 0.f;
                     l_lane += p;
 #pragma unroll
-                    for (int db = 0; db < DB; ++db) o[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(rows.v[i][db], p, o[db], 0, 0, 0);
+                    for (int db = 0; db < DB; ++db) {
+                        if constexpr (FEW) o[db] = __builtin_amdgcn_mfma_f32_4x4x1f32(rows.v[i][db], p, o[db], 0, 0, 0);
+                        else o[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(rows.v[i][db], p, o[db], 0, 0, 0);
+                    }
                 }
             }
             load_rows(ks + DEPTH * NW * KS, rows);
@@ -504,12 +537,15 @@ __global__ __launch_bounds__(DEC_WAVES * WAVE) void mfma_decode_f32_kernel(
 
     // wavefronts meet: every one leaves (reference, sum) of its rows and its 16 x HD output in LDS; this lane
     // holds dims (4*kg + i)*DB + db of its row in o[db][i]
-    const float l = lanes4(l_lane, false);
-    if (kg == 0) { sm_ml[wave][r][0] = m_ref; sm_ml[wave][r][1] = l; }
+    const float l = FEW ? quads4(l_lane, false) : lanes4(l_lane, false);
+    if (kg == 0 && r < ROWS) { sm_ml[wave][r][0] = m_ref; sm_ml[wave][r][1] = l; }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int db = 0; db < DB; ++db) so[wave][r][(4 * kg + i) * DB + db] = o[db][i];
+        for (int db = 0; db < DB; ++db) {
+            const float v = FEW ? quads4(o[db][i], false) : o[db][i];
+            if (r < ROWS) so[wave][r][(4 * kg + i) * DB + db] = v;
+        }
     __syncthreads();
     const int rows_here = min(16, G - chunk * 16);
     for (int idx = tid; idx < rows_here * HD; idx += THREADS) {
@@ -552,7 +588,8 @@ NI_EXPORT int ni_mfma_token_attention_f32(const void* q, int q_stride, const voi
     int page_shift = 0;
     while (pow2 && (1 << page_shift) < page_size) ++page_shift;
     dim3 grid(T_tokens, KVH * chunks, nsplit);
-    auto kernel = pow2 ? mfma_decode_f32_kernel<true> : mfma_decode_f32_kernel<false>;
+    auto kernel = G <= 4 ? (pow2 ? mfma_decode_f32_kernel<true, true> : mfma_decode_f32_kernel<false, true>)
+                         : (pow2 ? mfma_decode_f32_kernel<true, false> : mfma_decode_f32_kernel<false, false>);
     kernel<<<grid, DEC_WAVES * WAVE, 0, stream>>>(
         (const float*)q, q_stride, (const float*)kpool, (const float*)vpool, (const int32_t*)block_table, table_stride,
         (const int32_t*)seq_of_token, (const int32_t*)positions, (float*)out, (float*)part_o, (float*)part_ml, H, KVH,
