@@ -2,8 +2,8 @@
 on the host, that operand shapes, types and devices are what each kernel and its grid assume.
 
 There is no fallback: when a library cannot be built or loaded, or a tensor is not on the GPU,
-the call raises.  Matrix products of many bfloat16 rows are the one thing taken from a library (``torch.matmul`` ->
-rocBLAS/hipBLASLt), as the reference takes its products from cuBLAS (src/op/kernels/cuda/matmul_kernel.cu:76-86).
+the call raises.  Matrix products that none of the kernels here takes or wins (over 512 bfloat16 rows, float32 ones of more
+than 64 rows and under 2.2 GFLOP) are the one thing taken from a library (``torch.matmul`` -> rocBLAS/hipBLASLt), as the reference takes its products from cuBLAS (src/op/kernels/cuda/matmul_kernel.cu:76-86).
 """
 from __future__ import annotations
 
