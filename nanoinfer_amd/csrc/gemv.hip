@@ -774,13 +774,15 @@ __global__ __launch_bounds__(WV * WAVE) void skinny_decode_kernel(const T* __res
     for (int nt = 0; nt < NT; ++nt) {
         const int limit = (N + 15) / 16 - 1;         // a workgroup's last tiles may lie past the matrix: read the last one, store nothing
         int tile, tile_row = r;                      // this lane's row of W
-        if constexpr (R == 16) {
-            int col0 = (EPI == EPI_SWIGLU) ? (wg * (NT / 2) + nt / 2) * 16 : (wg * NT + nt) * 16;
+        if constexpr (16 % R == 0) {                 // one tile of the matrix, the same for the whole workgroup
+            int col0 = (EPI == EPI_SWIGLU) ? (wg * (NT / 2) + nt / 2) * 16 : (wg * NT + nt) * R;
             if (EPI == EPI_ROPE) {
                 const RopePair first = rope_pair<R>(wg, 0, rope.hd);
                 col0 = first.head * rope.hd + first.j + nt * (rope.hd / 2);
             }
-            tile = (col0 + ((EPI == EPI_SWIGLU && (nt % 2)) ? I : 0)) / 16;
+            col0 += (EPI == EPI_SWIGLU && (nt % 2)) ? I : 0;
+            tile = col0 / 16;
+            if constexpr (R < 16) tile_row = col0 % 16 + min(r, R - 1);
         } else {
             static_assert(EPI != EPI_SWIGLU, "gate and up tiles are whole");
             int n = (wg * NT + nt) * R + min(r, R - 1);
