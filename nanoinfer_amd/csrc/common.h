@@ -265,13 +265,17 @@ __device__ __forceinline__ int token_by_length(const int32_t* __restrict__ posit
 #define RANKED_GROUPS 512
 #define RANKED_TOKENS 256
 
+// The bounds of hidden units.  NaN passes them (fmaxf and fminf would make it the bound: a number out of none).
+__device__ __forceinline__ float at_least(float v, float low) { return v < low ? low : v; }
+__device__ __forceinline__ float at_most(float v, float high) { return v > high ? high : v; }
+
 // What a gated hidden unit gives from its gate g and its up value u: g sigmoid(a g + b g^3) u.  (1, 0) is silu(g) u;
 // gelu in its tanh form is 0.5 g (1 + tanh y) = g sigmoid(2 y) with y = sqrt(2 / pi) (g + 0.044715 g^3).
 struct GatedUnit {
     float a = 1.f, b = 0.f;
     bool squared = false;          // (a product without a gate) a result v is stored as relu(v)^2
     __device__ __forceinline__ float plain(float v) const {
-        const float r = fmaxf(v, 0.f);
+        const float r = at_least(v, 0.f);
         return squared ? r * r : v;
     }
     __device__ __forceinline__ float value(float g, float u) const { return g / (1.0f + expf(-(g * (a + b * (g * g))))) * u; }

@@ -1002,7 +1002,7 @@ __global__ void experts_act_kernel(const T* __restrict__ up, const float* __rest
     const float w = mix_all ? mix_all[t * mix_stride + e] : 1.f;
     float v = 0.f;
     if (w != 0.f) {
-        const float u = fmaxf(ld(up + i), 0.f);
+        const float u = at_least(ld(up + i), 0.f);
         v = w * (u * u);
     }
     st(act + i, v);
@@ -1025,7 +1025,7 @@ __global__ void experts_act_vec_kernel(const T* __restrict__ up, const float* __
         VecIO<T, 8>::load(up + i, v);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const float u = fmaxf(v[j], 0.f);
+            const float u = at_least(v[j], 0.f);
             v[j] = w * (u * u);
         }
     } else {
@@ -1044,8 +1044,8 @@ struct GluForm {
 
 __device__ __forceinline__ float glu_value(float g, float u, const GluForm f) {
     if (f.form == 2) {
-        g = fminf(g, f.limit);
-        u = fminf(fmaxf(u, -f.limit), f.limit);
+        g = at_most(g, f.limit);
+        u = at_most(at_least(u, -f.limit), f.limit);
         return g / (1.0f + expf(-f.slope * g)) * (u + 1.0f);
     }
     return g / (1.0f + expf(-g)) * u;
@@ -1193,7 +1193,7 @@ __global__ void experts_up_few_kernel(const T* __restrict__ x, const T* __restri
             if constexpr (GATED) {
                 a = glu_value(s[u], s[R + u], form);
             } else {
-                a = fmaxf(s[u], 0.f);
+                a = at_least(s[u], 0.f);
                 a = a * a;
             }
             hid[static_cast<size_t>(pair) * ff + i0 + u] = a;
