@@ -22,7 +22,10 @@
 // numbers taken apart a product; 256 x 256 runs at 220 TFLOP/s, 128 x 256 at 197, the smaller ones at 165 and fill the
 // chip where there are few rows.
 //
-// Values that are not finite come out as NaN (an infinity less itself has no rest).
+// An infinity less itself has no rest: what it takes part in comes out of the matrix cores as NaN.  Numbers of the result
+// that are not finite are therefore worked out again from the float32 operands (plain_dot), each by the lane that holds
+// it, and are what a float32 product gives: infinities with their sign, NaN where there is no answer.  Finite results
+// pay one multiplication.
 #include "common.h"
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -37,6 +40,20 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ int tile_of_block(int id, int total) {
     const int q = total / TG_XCDS, r = total % TG_XCDS, xcd = id % TG_XCDS, slot = id / TG_XCDS;
     return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + slot;
+}
+
+// The float32 numbers a and b multiplied and added up one after the other, in 64 bits; NaN is its own end.
+__device__ __forceinline__ float plain_dot(const float* __restrict__ a, const float* __restrict__ b, int count) {
+    double s = 0.0;
+#pragma nounroll
+    for (int k = 0; k < count && s == s; k += 4) {
+        const float4 u = *reinterpret_cast<const float4*>(a + k), v = *reinterpret_cast<const float4*>(b + k);
+        s += static_cast<double>(u.x) * v.x;
+        s += static_cast<double>(u.y) * v.y;
+        s += static_cast<double>(u.z) * v.z;
+        s += static_cast<double>(u.w) * v.w;
+    }
+    return static_cast<float>(s);
 }
 
 // Four float32 numbers as three times four bfloat16 numbers that add up to them.
@@ -235,11 +252,13 @@ __global__ __launch_bounds__(WM * WN * WAVE) void split_gemm_kernel(const float*
 
     const int cols = EPI == TG_GATED ? half : N;
     float* base = out + static_cast<size_t>(share) * M * cols;
+    auto row_of = [&](int i, int e) { return m0 + wm * (BM / WM) + 32 * i + 8 * (e / 4) + 4 * (lane >> 5) + (e & 3); };
+    float zero = 0.f;                // NaN once a number that this lane holds is not finite
 #pragma unroll
     for (int i = 0; i < TMB; ++i) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-            const int m = m0 + wm * (BM / WM) + 32 * i + 8 * (e / 4) + 4 * (lane >> 5) + (e & 3);
+            const int m = row_of(i, e);
             if (m >= M) continue;
             if constexpr (EPI == TG_GATED) {
 #pragma unroll
@@ -253,6 +272,37 @@ __global__ __launch_bounds__(WM * WN * WAVE) void split_gemm_kernel(const float*
                     const int n = nt * BN + wn * (BN / WN) + 32 * j + (lane & 31);
                     if (n < cols) base[static_cast<size_t>(m) * cols + n] = act.plain(acc[i][j][e]);
                 }
+            }
+#pragma unroll
+            for (int j = 0; j < TNB; ++j) zero = fmaf(acc[i][j][e], 0.f, zero);
+        }
+    }
+    if (zero != 0.f) {
+        constexpr int STEP = EPI == TG_GATED ? 2 : 1;          // blocks of columns an output is made of
+#pragma nounroll
+        for (int i = 0; i < TMB; ++i) {
+            uint64_t which = 0;                                // bit 16 * j + e
+#pragma unroll
+            for (int ii = 0; ii < TMB; ++ii)
+#pragma unroll
+                for (int j = 0; j < TNB; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e)
+                        which |= static_cast<uint64_t>(ii == i && !__builtin_isfinite(acc[ii][j][e])) << (16 * (j / STEP) + e);
+            static_assert(TNB * 16 <= 64, "a bit a number");
+            for (; which; which &= which - 1) {
+                const int bit = __builtin_ctzll(which), j = bit / 16, m = row_of(i, bit % 16);
+                const int n = nt * (BN / STEP) + wn * (BN / WN / STEP) + 32 * j + (lane & 31);
+                if (m >= M || n >= cols) continue;
+                int row = m;
+                if constexpr (GROUPED)
+                    if (groups.rows) row = groups.rows[m];
+                const float* xk = x + static_cast<size_t>(row) * K + kbeg;
+                const float first = plain_dot(xk, w + static_cast<size_t>(n) * ldw + kbeg, kend - kbeg);
+                float v;
+                if constexpr (EPI == TG_GATED) v = act.value(first, plain_dot(xk, w + static_cast<size_t>(half + n) * ldw + kbeg, kend - kbeg));
+                else v = act.plain(first);
+                base[static_cast<size_t>(m) * cols + n] = v;
             }
         }
     }

@@ -76,6 +76,79 @@ def test_rows_that_are_not_finite_stay_so_and_touch_no_other(K):
     close(got[~bad.cuda()], x[~bad.cuda()], w)
 
 
+def same(got, want, rtol=1e-5):
+    """The same infinities with the same signs, NaN in the same places, the finite rest within rtol of its largest in a row."""
+    got, want = got.double().cpu(), want.double().cpu()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(torch.isinf(got) * torch.sign(got), torch.isinf(want) * torch.sign(want))
+    fine = torch.isfinite(want)
+    a, b = torch.where(fine, got, 0.0), torch.where(fine, want, 0.0)
+    assert bool(((a - b).abs() <= rtol * b.abs().amax(dim=1, keepdim=True)).all())
+
+
+def not_finite(M, N, Kd, seed=3, huge=True):
+    """Operands with infinities of both signs, NaN, zeros that meet an infinity and (``huge``) numbers near the type's
+    largest, whose bfloat16 is infinite; with the exact products, as float32 holds them."""
+    x, w = operands(M, N, Kd, seed=seed)
+    inf, nan = float("inf"), float("nan")
+    x[3, 5], x[70, 0], x[M - 1, Kd - 1], x[9, 8], x[9, 9] = inf, nan, -inf, inf, -inf
+    w[11, 2], w[N // 2 + 11, 7], w[N - 1, 3], w[41, 5] = -inf, inf, nan, 0.0
+    if huge:
+        x[20], x[21], w[40] = 3.4e38, 3.4e38 * torch.sign(x[21]), 1e-30
+    return x, w, (x.cpu().double() @ w.cpu().double().t()).float()
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("M,N,Kd", [(130, 300, 64), (300, 130, 132)])
+def test_what_is_not_finite_stays_what_a_float32_product_makes_of_it(K, tile, M, N, Kd):
+    x, w, z = not_finite(M, N, Kd)
+    same(K.split_gemm(x, w, plan=(tile, 1)), z)
+    # cut along K: the shares' sums, each as float32 holds it (two that overflow may cancel to NaN where one sum would not)
+    parts = K.split_gemm(x, w, plan=(tile, 2), addends=True)
+    per = -(-Kd // 32) * 16
+    for p, at in zip(parts, (0, per)):
+        same(p, (x[:, at:at + per].cpu().double() @ w[:, at:at + per].cpu().double().t()).float())
+    same(K.split_gemm(x, w, plan=(tile, 2)), parts[0] + parts[1])
+    same(K.split_gemm(x, w, squared=True, plan=(tile, 1)), torch.relu(z) ** 2)
+    same(K.split_gemm(x, w, squared=True, plan=(tile, 2)), torch.relu(parts[0] + parts[1]) ** 2)
+    for act in ("silu", "gelu_tanh"):
+        same(K.split_gemm(x, w, gated=act, plan=(tile, 1)), K.swiglu(z.cuda(), torch.empty(M, N // 2, device="cuda"), act), 1e-4)
+
+
+def test_feed_forwards_of_rows_that_are_not_finite(K):
+    """The same through the entry points, where the rule sends such products to these kernels."""
+    x, w, z = not_finite(300, 4096, 1024, huge=False)
+    calls = K.library_calls()
+    assert K.split_wins(x, w)
+    same(K.linear(x, w), z)
+    same(K.linear_relu2(x, K.Weight(w)), torch.relu(z) ** 2)
+    same(K.linear_swiglu(x, w), K.swiglu(z.cuda(), torch.empty(300, 2048, device="cuda")), 1e-4)
+    assert K.library_calls() == calls
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+def test_experts_of_tokens_that_are_not_finite(K, monkeypatch, tile):
+    """An infinity in a token, in an expert's rows: as all experts run as two float32 products would have it, but for the
+    experts that a token did not choose, which it does not meet."""
+    from nanoinfer_amd.kernels import tile as tiles
+    monkeypatch.setattr(tiles, "_grouped_plan", lambda *a: (0.0, tile))
+    T, d, ff, E, top = 150, 64, 36, 5, 2
+    g = torch.Generator().manual_seed(5)
+    x, up, down = torch.randn(T, d, generator=g), torch.randn(E * ff, d, generator=g), torch.randn(d, E * ff, generator=g)
+    chosen = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(T)]).int()
+    mix = torch.rand(T, top, generator=g) + 0.1
+    inf = float("inf")
+    x[4, 3], x[77, 0], x[149, 63], up[2 * ff + 5, 9], down[7, 3 * ff + 1] = inf, float("nan"), -inf, -inf, inf
+    want = torch.zeros(T, d, dtype=torch.float64)
+    for t in range(T):
+        for k in range(top):
+            e = int(chosen[t, k])
+            hid = mix[t, k].double() * torch.relu(up[e * ff:(e + 1) * ff].double() @ x[t].double()) ** 2
+            want[t] += (down[:, e * ff:(e + 1) * ff].double() * hid).sum(dim=1)
+    got = K.experts_grouped(x.cuda(), up.cuda(), down.cuda(), chosen.cuda(), mix.cuda(), E, lambda z, w: K.experts_act(z, w, ff, "relu2"))
+    same(got, want)
+
+
 def test_what_split_gemm_does_not_take(K):
     x, w = operands(70, 64, 64)
     for bad in (lambda: K.split_gemm(x[:, :62].contiguous(), w[:, :62].contiguous()), lambda: K.split_gemm(x.bfloat16(), w.bfloat16()),
