@@ -58,7 +58,7 @@ def split_wins(x: torch.Tensor, rows: torch.Tensor) -> bool:
 def split_gemm(x: torch.Tensor, rows: torch.Tensor, out: Optional[torch.Tensor] = None, gated: Optional[str] = None, squared: bool = False,
                plan: Optional[Tuple[int, int]] = None, addends: bool = False) -> torch.Tensor:
     """``x . rows^T`` for float32 ``x`` [M, K] and ``rows`` [N, K] by six bfloat16 products of the operands' three parts
-    (against 64 bits 0.9 times the error of the library's float32 product, less with shares).  ``gated``: an activation's
+    (against 64 bits 0.6 to 0.9 times the error of the library's float32 product for sums of 700 to 8,192 numbers).  ``gated``: an activation's
     name; ``rows`` is [gate; up] stacked and the result ``act(gate) * up`` [M, N / 2].  ``squared``: ``relu(.)^2``.
     ``plan``: another (tile, shares) than :func:`split_plan`'s.  ``addends``: where the product is cut along K its shares come
     back as they are, [shares, M, N], for a norm that adds them."""
