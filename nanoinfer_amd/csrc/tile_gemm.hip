@@ -555,13 +555,15 @@ NI_EXPORT int ni_tiled_gemm(const void* x, const void* w, void* out, int M, int 
     }
 }
 
-// out[i] = (relu of, squared,) the sum of `shares` times n float32 numbers, in their order
+// out[i] = (relu of, squared,) the sum of `shares` times n float32 numbers, in their order; four at a time where they and
+// `out` start at whole vectors of four
 NI_EXPORT int ni_add_shares(const void* parts, void* out, size_t n, int shares, int squared, int dtype, void* stream) {
     if (n == 0 || shares < 1) return static_cast<int>(hipErrorInvalidValue);
     GatedUnit act;
     act.squared = squared != 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const unsigned v = n % 4 == 0 ? 4 : 1, blocks = static_cast<unsigned>((n / v + 255) / 256);
+    const bool aligned = reinterpret_cast<uintptr_t>(parts) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % (dtype == 0 ? 16 : 8) == 0;
+    const unsigned v = n % 4 == 0 && aligned ? 4 : 1, blocks = static_cast<unsigned>((n / v + 255) / 256);
     const float* pf = static_cast<const float*>(parts);
     if (dtype == 0) {
         if (v == 4) add_shares_kernel<float, 4><<<blocks, 256, 0, s>>>(pf, static_cast<float*>(out), n, shares, act);
@@ -649,7 +651,8 @@ NI_EXPORT int ni_expert_lists(const void* chosen, const void* mix, int T, int to
 NI_EXPORT int ni_gather_entries(const void* y, const void* place, void* out, int T, int d, int top, void* stream) {
     if (T <= 0 || d <= 0 || top <= 0) return static_cast<int>(hipErrorInvalidValue);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (d % 4 == 0) gather_entries_kernel<4><<<dim3(T, (d / 4 + 255) / 256), 256, 0, s>>>((const float*)y, (const int32_t*)place, (float*)out, d, top);
+    const bool aligned = reinterpret_cast<uintptr_t>(y) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
+    if (d % 4 == 0 && aligned) gather_entries_kernel<4><<<dim3(T, (d / 4 + 255) / 256), 256, 0, s>>>((const float*)y, (const int32_t*)place, (float*)out, d, top);
     else gather_entries_kernel<1><<<dim3(T, (d + 255) / 256), 256, 0, s>>>((const float*)y, (const int32_t*)place, (float*)out, d, top);
     return NI_LAUNCH_RESULT();
 }

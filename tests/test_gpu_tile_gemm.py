@@ -194,6 +194,26 @@ def test_what_split_gemm_does_not_take(K):
     assert K.library_calls() == calls + 2
 
 
+@pytest.mark.parametrize("offset", [1, 2, 3])
+def test_results_that_start_at_any_number(K, offset):
+    """A caller's ``out`` need not start at 16 bytes: whole, added up from shares, and the experts' sum."""
+    x, w = operands(512, 1056, 2048)
+    aside = torch.full((512 * 1056 + 8,), 7.0, device="cuda")
+    for plan in ((1, 1), (1, 3)):
+        out = aside[offset:offset + 512 * 1056].view(512, 1056)
+        assert torch.equal(K.split_gemm(x, w, out, plan=plan), K.split_gemm(x, w, plan=plan))
+        assert bool((aside[:offset] == 7.0).all()) and bool((aside[offset + 512 * 1056:] == 7.0).all())
+    calls = K.library_calls()
+    assert K.linear(x, w, out=out).data_ptr() == out.data_ptr() and K.library_calls() == calls
+    g = torch.Generator().manual_seed(offset)
+    chosen = torch.stack([torch.randperm(5, generator=g)[:2] for _ in range(70)]).int().cuda()
+    tokens, up, down, mix = (torch.randn(s, generator=g).cuda() for s in ((70, 64), (5 * 36, 64), (64, 5 * 36), (70, 2)))
+    out = aside[offset:offset + 70 * 64].view(70, 64)
+    act = lambda z, weights: K.experts_act(z, weights, 36, "relu2")     # noqa: E731
+    assert torch.equal(K.experts_grouped(tokens, up, down, chosen, mix, 5, act, out=out), K.experts_grouped(tokens, up, down, chosen, mix, 5, act))
+    assert bool((aside[:offset] == 7.0).all())
+
+
 @pytest.mark.parametrize("T,d,ff,E,top,kind", [(1, 4, 4, 1, 1, "any"), (65, 36, 20, 5, 2, "any"), (300, 64, 132, 16, 4, "any"), (257, 68, 64, 7, 3, "one"),
                                                (130, 40, 36, 6, 2, "identity"), (1500, 128, 64, 16, 4, "any")])
 @pytest.mark.parametrize("tile", [0, 1, 2, 3])
