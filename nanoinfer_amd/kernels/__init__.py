@@ -1156,8 +1156,8 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
     output type) instead of a new tensor.  ``leave`` (with ``residual``, where :func:`leaves_scaled_ok`
     holds; ignored elsewhere): the norm that stands behind the stream; the product then runs whole and
     returns a :class:`ScaledInput` for that norm.  ``x`` may itself be a :class:`ScaledInput` where
-    :func:`takes_scaled_ok` holds.  ``addends``: a product of many rows may come back as float32 addends
-    [S, M, N] (its K range cut into S shares), for a norm that adds them to the stream itself."""
+    :func:`takes_scaled_ok` holds.  ``addends`` (ignored with ``out``): a product of many rows may come back as float32
+    addends [S, M, N] (its K range cut into S shares), for a norm that adds them to the stream itself."""
     rows, _ = _rows_and_tiles(weight)
     if out is not None and (isinstance(x, (NormedInput, ScaledInput)) or residual is not None):
         raise KernelError("out= goes with a plain product")
@@ -1196,6 +1196,7 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
     out_dtype = out_dtype or x.dtype
     if out is not None:
         _gpu(out, "out", out_dtype, (x.shape[0], rows.shape[0]))
+    addends = addends and out is None
     M, Kd = x.shape
     if skinny_wins(M, Kd, x.dtype, weight) if M <= SKINNY_MAX_ROWS else (
             skinny_deals(M, rows.shape[0], Kd, x.dtype, weight) and _plain(x) and (out is None or out.data_ptr() % 16 == 0)):

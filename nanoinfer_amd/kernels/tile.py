@@ -60,14 +60,15 @@ def split_gemm(x: torch.Tensor, rows: torch.Tensor, out: Optional[torch.Tensor] 
     """``x . rows^T`` for float32 ``x`` [M, K] and ``rows`` [N, K] by six bfloat16 products of the operands' three parts
     (against 64 bits 0.6 to 0.9 times the error of the library's float32 product for sums of 700 to 8,192 numbers).  ``gated``: an activation's
     name; ``rows`` is [gate; up] stacked and the result ``act(gate) * up`` [M, N / 2].  ``squared``: ``relu(.)^2``.
-    ``plan``: another (tile, shares) than :func:`split_plan`'s.  ``addends``: where the product is cut along K its shares come
-    back as they are, [shares, M, N], for a norm that adds them."""
+    ``plan``: another (tile, shares) than :func:`split_plan`'s.  ``addends`` (without ``out`` and activations): where the product is
+    cut along K its shares come back as they are, [shares, M, N], for a norm that adds them."""
     M, K = x.shape
     N = rows.shape[0]
     _gpu(x, "x", torch.float32)
     _gpu(rows, "w", torch.float32, (N, K))
     if gated is not None and (N % 2 or squared):
         raise KernelError("a gated product takes a stacked matrix and no other activation")
+    _addends_alone(addends, out, gated, squared)
     cols = N if gated is None else N // 2
     if K % 4 or x.data_ptr() % 16 or rows.data_ptr() % 16:
         raise KernelError(f"rows of {K} float32 elements at this address are not aligned to 16 bytes")
@@ -85,6 +86,11 @@ def split_gemm(x: torch.Tensor, rows: torch.Tensor, out: Optional[torch.Tensor] 
     if shares > 1:
         return parts if addends else _add_shares(parts, torch.float32, out, squared)
     return out
+
+
+def _addends_alone(addends: bool, out: Optional[torch.Tensor], gated: Optional[str], squared: bool) -> None:
+    if addends and (out is not None or gated is not None or squared):
+        raise KernelError("a product that leaves its addends has no out and no activation")
 
 
 def _add_shares(parts: torch.Tensor, dtype: torch.dtype, out: Optional[torch.Tensor], squared: bool) -> torch.Tensor:
@@ -155,6 +161,7 @@ def tiled_gemm(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None,
     _gpu(tiles, "tiles", torch.bfloat16)
     if gated is not None and (N % 32 or squared or out_dtype != torch.bfloat16):
         raise KernelError("a gated product takes a stacked matrix of whole tiles, no other activation, and gives bfloat16")
+    _addends_alone(addends, out, gated, squared)
     if K % 64 or N % 4 or x.data_ptr() % 16 or M * K >= 1 << 30 or (N + 15) * K >= 1 << 30 or tiles.numel() != (N + 15) // 16 * 16 * K:
         raise KernelError(f"tiled_gemm does not take [{M}, {K}] x [{N}, {K}]")
     cols = N if gated is None else N // 2

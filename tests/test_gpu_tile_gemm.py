@@ -180,6 +180,21 @@ def test_experts_of_tokens_that_are_not_finite(K, monkeypatch, tile):
     same(got, want)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_addends_go_with_nothing_else(K, dtype):
+    """A product that leaves its addends would leave an ``out`` unwritten and an activation undone: refused, and a linear
+    product with an ``out`` writes it."""
+    x, w = (t.to(dtype) for t in operands(300, 2048, 4096))
+    weight, out = K.Weight(w), torch.full((300, 2048), 7.0, device="cuda", dtype=dtype)
+    product = (lambda **k: K.split_gemm(x, w, plan=(1, 2), **k)) if dtype == torch.float32 else (lambda **k: K.tiled_gemm(x, weight, plan=(1, 2), **k))
+    assert product(addends=True).shape == (2, 300, 2048)
+    for more in ({"out": out}, {"squared": True}, {"gated": "silu"}):
+        with pytest.raises(K.KernelError):
+            product(addends=True, **more)
+    assert K.linear(x, weight, addends=True).dim() == 3
+    assert torch.equal(K.linear(x, weight, out=out, addends=True), K.linear(x, weight)) and torch.equal(out, K.linear(x, weight))
+
+
 def test_what_split_gemm_does_not_take(K):
     x, w = operands(70, 64, 64)
     for bad in (lambda: K.split_gemm(x[:, :62].contiguous(), w[:, :62].contiguous()), lambda: K.split_gemm(x.bfloat16(), w.bfloat16()),
