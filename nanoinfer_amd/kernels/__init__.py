@@ -598,7 +598,7 @@ def skinny_deals(M: int, N: int, K: int, dtype: torch.dtype, weight) -> bool:
     float32 [192, 512] at 100 rows 49 : 4.4, [1024, 192] at 256 rows 5.5 : 4.9, at 448 6.3 : 6.4, [1024, 512] at 100 rows
     6.5 : 4.8, at 160 6.7 : 7.0, [128, 2048] 7.3 : 8.9; bfloat16 [1024, 1024] at 256 rows 5.8 : 5.5, at 448 7.0 : 7.5,
     [16, 2048] at 1,500 rows 5.6 : 4.7, [1024, 2048] at 256 rows 7.6 : 7.5."""
-    if not (isinstance(weight, Weight) and weight.tiles is not None and K % (8 if dtype == torch.float32 else 16) == 0):
+    if not (isinstance(weight, Weight) and weight.tiles is not None and skinny_ok(1, K, dtype)):
         return False
     tiles = (N + 15) // 16
     if dtype == torch.float32:
@@ -672,8 +672,8 @@ def note_library_call() -> None:
 
 def skinny_ok(M: int, K: int, dtype: torch.dtype) -> bool:
     """Whether the hand-written skinny product takes this shape: at most 64 rows, rows of W that
-    split into whole 32-byte lane loads."""
-    return 0 < M <= SKINNY_MAX_ROWS and K % (8 if dtype == torch.float32 else 16) == 0
+    split into whole 32-byte lane loads, one of them at least (the kernels read the last piece of a row where others end)."""
+    return 0 < M <= SKINNY_MAX_ROWS and K > 0 and K % (8 if dtype == torch.float32 else 16) == 0
 
 
 def _tiles_per_group(n_out: int) -> int:

@@ -1,0 +1,16 @@
+"""The rules by which a product goes to a kernel here or to the library, without a GPU."""
+import pytest
+import torch
+
+from nanoinfer_amd import kernels as K
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M", [1, 20, 64, 65, 100, 512, 1000])
+@pytest.mark.parametrize("N,Kd", [(64, 0), (0, 64)])
+def test_products_over_nothing_are_the_librarys(dtype, M, N, Kd):
+    """No kernel here takes rows of no elements (it would read the last piece of a row that has none) or none of them."""
+    x, weight = torch.empty(M, Kd, dtype=dtype), K.Weight(torch.empty(N, Kd, dtype=dtype))
+    if Kd == 0:
+        assert not K.skinny_ok(M, Kd, dtype) and not K.skinny_wins(M, Kd, dtype, weight) and not K.skinny_deals(M, N, Kd, dtype, weight)
+    assert not K.tiled_wins(x, weight) and not K.tiled_wins(x, weight, gated=True) and not K.split_wins(x, weight.rows)
