@@ -143,7 +143,7 @@ def tiled_wins(x: torch.Tensor, weight, gated: bool = False) -> bool:
     M, K = x.shape
     N = weight.rows.shape[0]
     most = TILED_ROWS_GATED if gated and 2.0 * M * N * K <= 70e9 else TILED_ROWS
-    return (64 < M <= most and 0 < K and K % 64 == 0 and 0 < N and N % (32 if gated else 4) == 0 and (N + 15) * K < 1 << 30
+    return (64 < M <= most and 0 < K and K % 64 == 0 and 0 < N and N % (32 if gated else 4) == 0 and (N + 15) * K < 1 << 30 and M * K < 1 << 30
             and x.is_contiguous() and x.data_ptr() % 16 == 0)
 
 

@@ -14,3 +14,16 @@ def test_products_over_nothing_are_the_librarys(dtype, M, N, Kd):
     if Kd == 0:
         assert not K.skinny_ok(M, Kd, dtype) and not K.skinny_wins(M, Kd, dtype, weight) and not K.skinny_deals(M, N, Kd, dtype, weight)
     assert not K.tiled_wins(x, weight) and not K.tiled_wins(x, weight, gated=True) and not K.split_wins(x, weight.rows)
+
+
+def test_what_the_tiled_product_cannot_address_is_the_librarys():
+    """Bytes of x and of W are counted in 32 bits: what tiled_gemm refuses, the rule does not send there."""
+    class Stored:                                      # a matrix that is only looked at
+        tiles = torch.empty(0)
+
+        def __init__(self, N, Kd):
+            self.rows = torch.empty(N, Kd, dtype=torch.bfloat16, device="meta")
+
+    for M, N, Kd in ((1024, 32, 1 << 20), (512, 4, 1 << 21), (65, 1 << 14, 1 << 16)):
+        x = torch.empty(M, Kd, dtype=torch.bfloat16, device="meta")
+        assert not K.tiled_wins(x, Stored(N, Kd)) and not K.tiled_wins(x, Stored(N, Kd), gated=True)
