@@ -27,3 +27,13 @@ def test_what_the_tiled_product_cannot_address_is_the_librarys():
     for M, N, Kd in ((1024, 32, 1 << 20), (512, 4, 1 << 21), (65, 1 << 14, 1 << 16)):
         x = torch.empty(M, Kd, dtype=torch.bfloat16, device="meta")
         assert not K.tiled_wins(x, Stored(N, Kd)) and not K.tiled_wins(x, Stored(N, Kd), gated=True)
+
+
+def test_a_plan_is_made_once_for_64_rows():
+    """Steps of every number of rows weigh the tiles and shares of a product eight times up to 512 rows, not 448 times."""
+    from nanoinfer_amd.kernels import tile
+    for plan, made in ((K.tiled_plan, tile._tiled_plan), (K.split_plan, tile._split_plan), (lambda M, N, Kd: tile._grouped_plan(M, N, Kd, 7), tile._grouped_tiles)):
+        before = made.cache_info().misses
+        plans = [plan(M, 3075, 2047) for M in range(65, 513)]
+        assert made.cache_info().misses - before <= 8
+        assert plans[0] == plan(128, 3075, 2047) and plans[-1] == plan(449, 3075, 2047)
