@@ -383,11 +383,13 @@ NI_EXPORT int ni_split_gemm(const void* x, const void* w, void* out, int M, int 
 // all the time and no operand is held twice.  W is the A operand: a lane then has four neighbouring columns of a row
 // of y and stores them at once.
 //
-// Measured (us; the library's product, with SwiGLU its kernel too : this): 512 rows on [16384, 2048] with SwiGLU
-// 41.5 : 35.3, on [2048, 8192] 29.4 : 25.5, on [3072, 2048] 14.6 : 15.1, on [2048, 2048] 12.0 : 11.9; 128 rows
-// 21 : 16.5, 18.5 : 12.4, 12.8 : 8.3, 9.4 : 6.4.  Raising a wavefront's priority while it multiplies (s_setprio) was
-// worth 39.6 -> 34.2.  Past 512 rows (1,024 with SwiGLU) the library's 256 x 256 tiles are ahead (1.27 PFLOP/s at 2,048 rows
-// against 1.06).
+// Measured in recorded launches, every one with another W (us; the library's product, with SwiGLU its kernel too, o and down
+// with the norm behind them : this): 512 rows on [16384, 2048] with SwiGLU 43.9 : 41.1, on [2048, 8192] 39.1 : 33.5, on
+// [3072, 2048] 15.4 : 18.7, on [2048, 2048] 18.1 : 18.7; 128 rows 25.9 : 24.9, 25.6 : 19.6, 14.5 : 13.5, 15.5 : 11.9.  (With W
+// at hand from the launch before 35.3, 25.5, 15.1 and 11.9 without the norm at 512 rows: the first operands of W come from
+// memory a slab ahead, and that is what they wait for.)  Raising a wavefront's priority while it multiplies (s_setprio)
+// was worth 39.6 -> 34.2.  Where there are tiles enough for it the library's 256 x 256 ones are ahead (1.27 PFLOP/s at 2,048
+// rows against 1.06).
 template <int N> struct Num { static constexpr int value = N; };
 
 template <int WN, int TM, int TN, int MINW, int EPI, typename OUT>

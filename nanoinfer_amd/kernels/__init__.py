@@ -1205,7 +1205,7 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
         return skinny_gemm(x, weight, out)
     if out_dtype == torch.float32 and split_wins(x, rows):
         return split_gemm(x, rows, out, addends=addends)
-    if tiled_wins(x, weight) and (out is None or out.data_ptr() % 16 == 0):
+    if tiled_wins(x, weight, addends=addends) and (out is None or out.data_ptr() % 16 == 0):
         return tiled_gemm(x, weight, out_dtype, out, addends=addends)
     rows_t = weight.rows_t if isinstance(weight, Weight) else rows.t()
     global _library_calls

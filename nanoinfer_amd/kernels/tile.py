@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import math
 from typing import Optional, Tuple
 
 import torch
@@ -115,20 +116,29 @@ def _add_shares(parts: torch.Tensor, dtype: torch.dtype, out: Optional[torch.Ten
 
 # ---------------------------------------------------------------- bfloat16 on the re-tiled matrix
 
-# As SPLIT_TILES, for 64 columns of K, with the microseconds before the first and behind the last of them.  Fitted to sweeps
-# of 65 to 1,024 rows over the layer sizes of the 1B, 3B and 8B shapes: the plan taken is the best of all tiles and
-# shares or within 6 % of it in four cases of five, within 21 % in all.
-TILED_TILES = ((128, 256, 1, 0.87, 0.57, 7.4), (128, 128, 2, 1.02, 0.23, 5.8), (64, 128, 4, 1.23, 0.13, 4.8), (64, 64, 5, 0.98, 0.11, 4.1))
+# Tiles of the bfloat16 product: rows of x, rows of W, workgroups a compute unit holds, and in microseconds: before the
+# first and behind the last 64 columns of K, for 64 columns with one workgroup on a unit, what another on the same unit adds,
+# and how much of that comes at once when the first unit gets one more.  Fitted to sweeps of all tiles and shares at 65 to
+# 512 rows (with SwiGLU 1,024) over the layer sizes of the 1B, 3B and 8B shapes, recorded, every launch with another W, which
+# then comes from memory as it does in a step, o and down with the norm behind them: of 117 plans taken 116 are within 5 %
+# of the best and the last within 9.  (Fitted to one product launched over and over, its W at hand, as these figures were
+# before, the plans were 10 % above the best on average and up to 46.)
+TILED_TILES = ((128, 256, 1, 4.9, 1.02, 1.10, 0.45), (128, 128, 2, 5.3, 0.56, 0.50, 0.80), (64, 128, 4, 4.7, 0.48, 0.32, 0.85),
+               (64, 64, 5, 2.8, 0.385, 0.265, 0.25))
 
 
-def _tiled_cost(M: int, N: int, K: int, tile: int, shares: int, gated: bool, addends: bool) -> float:
-    bm, bn, held, loaded, alone, fixed = TILED_TILES[tile]
-    full, rest = divmod(-(-M // bm) * -(-N // bn) * shares, COMPUTE_UNITS * held)
-    per = -(-(K // 64) // shares)
-    cost = fixed + full * loaded * per + (alone + (loaded - alone) * rest / (COMPUTE_UNITS * held)) * per * (rest > 0)
-    cost = max(cost + (shares > 1) * shares * M * N * 4 / 8e6, 3.0 + N * K * 2 / 5e6)
-    if shares > 1:      # the shares are read again, by the norm behind them or by a kernel that adds them
-        cost += shares * M * N * 4 / 5e6 + (0.5 if addends else 3.0)
+def _tiled_cost(M: int, N: int, K: int, tile: int, shares: int, addends: bool) -> float:
+    bm, bn, held, fixed, one, more, jump = TILED_TILES[tile]
+    groups = -(-M // bm) * -(-N // bn) * shares
+    full, rest = divmod(groups, COMPUTE_UNITS * held)
+
+    def column(n: float) -> float:                     # 64 columns with n workgroups a unit
+        return one if n <= 1 else one + more * (n + jump * (math.ceil(n) - n) - 1)
+
+    cost = fixed + -(-(K // 64) // shares) * (full * column(held) + (column(rest / COMPUTE_UNITS) if rest else 0.0))
+    cost = max(cost, 3.0 + N * K * 2 / 5.5e6)
+    if shares > 1:      # the shares are written and read again, by the norm behind them or by a kernel that adds them
+        cost += shares * M * N * 4 / 3.3e6 + (0.1 if addends else 3.3)
     return cost
 
 
@@ -139,27 +149,49 @@ def tiled_plan(M: int, N: int, K: int, gated: bool = False, addends: bool = Fals
 
 @functools.lru_cache(maxsize=4096)
 def _tiled_plan(M: int, N: int, K: int, gated: bool, addends: bool) -> Tuple[int, int]:
-    return min((_tiled_cost(M, N, K, t, s, gated, addends), t, s) for t in range(3 if gated else 4)
+    return min((_tiled_cost(M, N, K, t, s, addends), t, s) for t in range(3 if gated else 4)
                for s in ((1,) if gated else (1, 2, 3, 4, 6, 8)) if s == 1 or K // s >= 256)[1:]
 
 
-TILED_ROWS = 512            # rows up to which the product on the re-tiled matrix beats the library's or ties with it
-TILED_ROWS_GATED = 1024     # the same with SwiGLU in the epilogue, up to 70 GFLOP
+TILED_ROWS = 512            # rows up to which products on the re-tiled matrix are made here
+TILED_ROWS_GATED = 1024     # the same with SwiGLU in the epilogue and few columns
 
 
-def tiled_wins(x: torch.Tensor, weight, gated: bool = False) -> bool:
-    """Whether a bfloat16 product goes to :func:`tiled_gemm`: from 65 rows (the skinny product's end) to 512, or 1,024 with
-    SwiGLU in the epilogue; beyond, the library's product is faster by itself (us, library : this, [16384, 2048] with
-    SwiGLU at 1,024 rows 73 : 66, at 2,048 120 : 130; [2048, 8192] at 512 rows 29 : 26, at 1,500 54 : 59).  Up to there it also costs
-    the host a launch of some 5 us in place of the library's 20, which is what a step launched kernel by kernel waits for."""
+def tiled_wins(x: torch.Tensor, weight, gated: bool = False, addends: bool = False) -> bool:
+    """Whether a bfloat16 product goes to :func:`tiled_gemm`, from 65 rows (the skinny product's end) to 512.  Measured as
+    ``TILED_TILES`` (us, library : this).  Its tiles are smaller than the library's: it is ahead where it is cut along K or its
+    tiles are at most one a compute unit, and behind where there are so many that the library's fill the chip as well.
+
+    Shares left to the norm (o and down of the three shapes): always.  [2048, 2048] at 65 / 256 / 512 rows 15.5 : 10.8,
+    16.1 : 14.3, 18.1 : 18.7; [2048, 8192] 25.2 : 18.2, 31.6 : 24.3, 39.1 : 33.5; [4096, 14336] 52.9 : 34.0, 67.1 : 52.6, 95.8 : 79.7.
+
+    SwiGLU in the epilogue: while the tiles are one a unit, of a large matrix to 128 rows.  [16384, 2048] at 65 / 256 / 512 rows
+    23.1 : 24.0, 34.0 : 25.8, 43.9 : 41.1, [28672, 4096] at 128 rows 61.7 : 59.6 and at 192 72.7 : 82.6.  More of them are up to a
+    third slower ([28672, 4096] at 512 rows 107 : 141, [16384, 3072] at 384 49.1 : 55.1).  To 1,024 rows where the smaller tiles do
+    ([4096, 2048] at 600 / 1,024 rows 26.3 : 21.6, 29.1 : 22.7; the large ones: [8192, 2048] at 767 35.4 : 40.7, [16384, 2048]
+    at 640 / 1,000 47.9 : 56.3, 70 : 75).
+
+    Plain: cut into three shares and more ([4096, 14336] at 173 / 512 rows 62.1 : 48.4, 92.8 : 78.0, [3072, 8192] at 118 / 356
+    27.7 : 22.2, 42.5 : 36.6), and to 256 rows while the tiles are one a unit ([6144, 4096] at 65 / 256 rows 23.1 : 19.0, 41.1 : 31.2;
+    at 263 / 512 28.8 : 36.2, 36.8 : 42.5).
+
+    Small matrices to 512 rows in every case, though the library may be up to 4 us ahead ([3072, 2048] at 131 / 343 / 512
+    rows 12.3 : 13.4, 14.6 : 15.7, 15.4 : 18.7, [5120, 3072] at 512 28.8 : 32.7, gated [16384, 2048] at 341 37.8 : 39.6): a launch here
+    costs the host 10 us, the library's 18, and 79 with a number of rows that it has not seen before, and a step of single
+    tokens beside a portion, launched kernel by kernel, waits for the host."""
     tiles = getattr(weight, "tiles", None)
     if x.dtype != torch.bfloat16 or tiles is None:
         return False
     M, K = x.shape
     N = weight.rows.shape[0]
-    most = TILED_ROWS_GATED if gated and 2.0 * M * N * K <= 70e9 else TILED_ROWS
-    return (64 < M <= most and 0 < K and K % 64 == 0 and 0 < N and N % (32 if gated else 4) == 0 and (N + 15) * K < 1 << 30 and M * K < 1 << 30
-            and x.is_contiguous() and x.data_ptr() % 16 == 0)
+    if not (64 < M <= TILED_ROWS_GATED and 0 < K and K % 64 == 0 and 0 < N and N % (32 if gated else 4) == 0 and (N + 15) * K < 1 << 30
+            and M * K < 1 << 30 and x.is_contiguous() and x.data_ptr() % 16 == 0):
+        return False
+    tile, shares = tiled_plan(M, N, K, gated, addends)
+    if M <= TILED_ROWS and (addends or shares >= 3 or N * K <= (1 << 25 if gated else 1 << 24)):
+        return True
+    most = 256 if not gated else 128 if N * K > 1 << 26 else TILED_ROWS if tile == 0 else TILED_ROWS_GATED
+    return M <= most and -(-M // TILED_TILES[tile][0]) * -(-N // TILED_TILES[tile][1]) * shares <= COMPUTE_UNITS
 
 
 def tiled_gemm(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None, out: Optional[torch.Tensor] = None, gated: Optional[str] = None,

@@ -37,3 +37,24 @@ def test_a_plan_is_made_once_for_64_rows():
         plans = [plan(M, 3075, 2047) for M in range(65, 513)]
         assert made.cache_info().misses - before <= 8
         assert plans[0] == plan(128, 3075, 2047) and plans[-1] == plan(449, 3075, 2047)
+
+
+@pytest.mark.parametrize("N,Kd,kind,here,there", [
+    (2048, 2048, "addends", (65, 512), (64, 513)), (4096, 14336, "addends", (65, 512), (513,)),      # shares left to the norm
+    (4096, 14336, "plain", (65, 320, 512), (513,)), (3072, 8192, "plain", (65, 356), (505, 512)),     # cut along K, or not often enough
+    (3072, 2048, "plain", (65, 300, 512), (513,)), (6144, 4096, "plain", (65, 256), (257, 320, 512)),
+    (16384, 2048, "gated", (65, 320, 512), (513, 640, 1024)), (16384, 3072, "gated", (65, 256, 512), (320, 384, 600)),
+    (28672, 4096, "gated", (65, 128), (129, 192, 512, 1024)), (4096, 2048, "gated", (65, 512, 600, 1024), (1025,)),
+    (8192, 2048, "gated", (512,), (701, 767))])
+def test_where_bfloat16_products_of_many_rows_go(N, Kd, kind, here, there):
+    """Both sides of the lines that the rule draws, at the sizes measured beside it; the plan is one that the kernel takes."""
+    class Stored:
+        tiles = torch.empty(0)
+        rows = torch.empty(N, Kd, dtype=torch.bfloat16, device="meta")
+
+    more = {kind: True} if kind != "plain" else {}
+    for M in here + there:
+        x = torch.empty(M, Kd, dtype=torch.bfloat16, device="meta")
+        assert K.tiled_wins(x, Stored(), **more) == (M in here), M
+        tile, shares = K.tiled_plan(M, N, Kd, kind == "gated", kind == "addends")
+        assert 0 <= tile < (3 if kind == "gated" else 4) and 1 <= shares <= (1 if kind == "gated" else 8) and (shares == 1 or Kd // shares >= 256)
