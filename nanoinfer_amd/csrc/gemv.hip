@@ -1239,7 +1239,8 @@ __global__ __launch_bounds__(GV_THREADS) void skinny_rows_kernel(const T* __rest
 }
 
 // Calls f with the number of rows of x its kernel is to be compiled for (TileSum): by the rows and the length of a row
-// alone, so that every kernel takes a product's sums in the same order.
+// alone, so that kernels with as many wavefronts take a product's sums in the same order, whatever the layout of W.  (A
+// normalising prologue that is not staged, as with four tiles a workgroup, keeps 16 x 16 at every number of rows.)
 #define EIGHT_COLS_ABOVE 1024      // elements of a row; also what four pieces a wavefront of a normalising prologue hold
 template <typename T, typename F>
 static void with_cols(int M, int K, F f) {

@@ -8,7 +8,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("M,N,Kd", [(65, 16, 16), (96, 17, 48), (97, 100, 192), (129, 256, 512), (256, 1000, 192), (700, 3, 96), (449, 1024, 160), (2049, 33, 64)])
 def test_dealt_rows_are_the_rows_alone(dtype, M, N, Kd):
-    """Every row gets bit for bit what it gets in a product of the 64 rows around it, whatever else is dealt out."""
+    """Every row gets bit for bit what it gets in a product of the 32 or 64 rows around it that a workgroup takes, whatever
+    else is dealt out (a rest of up to 16 rows alone goes to another kernel)."""
     from nanoinfer_amd import kernels as K
     g = torch.Generator().manual_seed(M)
     x, w = torch.randn(M, Kd, generator=g).cuda().to(dtype), K.Weight(torch.randn(N, Kd, generator=g).cuda().to(dtype))
@@ -24,6 +25,11 @@ def test_dealt_rows_are_the_rows_alone(dtype, M, N, Kd):
         if out_type == torch.bfloat16:
             bound = bound + 2.0 ** -8 * want.abs()
         assert bool(((out[:M].double() - want).abs() <= bound).all())
+        block = 32 if (N + 15) // 16 * ((M + 31) // 32) <= 256 else 64
+        for a in range(0, M - 16, block):
+            part = x[a:a + block].contiguous()
+            alone = K.skinny_gemm(part, w, torch.empty(part.shape[0], N, device="cuda", dtype=out_type))
+            assert torch.equal(out[a:min(a + block, M)], alone)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

@@ -1,5 +1,6 @@
 """Float32 products of four and of eight rows by 4 x 4 blocks: at the numbers of rows and lengths where the kernel changes,
-and that every kernel which takes such rows adds them up in the same order."""
+and that the kernels for a matrix as stored and re-tiled add such rows up in the same order where both have eight wavefronts
+(rows of fewer than 2,048 elements)."""
 import pytest
 import torch
 
@@ -14,15 +15,19 @@ def test_few_rows(M, N, Kd):
     x, w = torch.randn(M, Kd, generator=g).cuda(), torch.randn(N, Kd, generator=g).cuda()
     want = x.double() @ w.double().t()
     tol = 2 * (Kd + 16) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())     # every product and every sum rounded once
+    results = []
     for weight in (w, K.Weight(w)):
         out = torch.full((M + 1, N), 7.0, device="cuda")
         K.skinny_gemm(x, weight, out[:M])
+        results.append(out)
         assert bool(((out[:M].double() - want).abs() <= tol).all()) and bool((out[M] == 7.0).all())
         stream = torch.randn(M, N, generator=g).cuda()
         if isinstance(weight, K.Weight):
             h = stream.clone()
             K.skinny_gemm(x, weight, h, residual=True)
             assert bool(((h.double() - stream.double() - want).abs() <= tol + 2.0 ** -23 * h.double().abs()).all())
+    if Kd < 2048:
+        assert torch.equal(*results)
     if N % 32 == 0:
         gated = K.skinny_gemm(x, K.Weight(w), torch.empty(M, N // 2, device="cuda"), swiglu=True)
         a, b = want[:, :N // 2], want[:, N // 2:]
