@@ -8,7 +8,7 @@
 //     xl wh + xh wl + xm wm + xm wh + xh wm + xh wh,
 // each product exact and added up in float32 by the matrix cores.  |xm| is at most 2^-8 |x| and |xl| 2^-17 |x|, so the three
 // left out are at most 2^-24 of |x||w| and 2^-27.2 on average, no more than one float32 rounding.  (With xh cut off instead of
-// rounded, which is no faster, it was 2^-22 and 2^-25.2.)  Six bfloat16 instructions take 3/8 of the time of the float32 ones
+// rounded, which is up to 1.5 % faster, it was 2^-22 and 2^-25.2.)  Six bfloat16 instructions take 3/8 of the time of the float32 ones
 // they replace.  What is left of the error is the sums': against 64 bits, relative to the root of the sum of the squared
 // products, [512, 1024] with 1 / 16 / 256 numbers a row that are not zero 3.5e-8 / 1.6e-7 / 4.2e-7 where the library's float32
 // product has 2.5e-8 / 7.4e-8 / 2.9e-7; sums of 700 to 8,192 numbers 0.6 to 0.9 times the library's.
@@ -22,8 +22,9 @@
 //
 // What bounds it is the matrix cores under load: a workgroup alone works at a rate that on 256 units were 1.82 PFLOP/s
 // of bfloat16 products, all of them together reach 1.2 to 1.32 (the library's bfloat16 product of 8,192^3 1.41), as the
-// clock falls.  Measured against the library's float32 product (us): [512, 2048] x [16384, 2048] 271 -> 163, 1,999 rows
-// 936 -> 611 (220 TFLOP/s), 512 rows x [2048, 8192] 135 -> 94.  Tiles: the larger the tile, the fewer reads of LDS and
+// clock falls.  Measured against the library's float32 product, recorded, every launch with another W (us): 512 rows on
+// [16384, 2048] 259 : 172 (with SwiGLU 265 : 171), on [2048, 8192] 135 : 99, on [3072, 2048] 61 : 48, on [2048, 2048] 38 : 37;
+// 1,999 rows on [16384, 2048] 930 : 607 (221 TFLOP/s).  Tiles: the larger the tile, the fewer reads of LDS and
 // numbers taken apart a product; 256 x 256 runs at 220 TFLOP/s, 128 x 256 at 197, the smaller ones at 165 and fill the
 // chip where there are few rows.
 //

@@ -2,8 +2,12 @@
 on the host, that operand shapes, types and devices are what each kernel and its grid assume.
 
 There is no fallback: when a library cannot be built or loaded, or a tensor is not on the GPU,
-the call raises.  Matrix products that none of the kernels here takes or wins (over 512 bfloat16 rows, float32 ones of more
-than 64 rows and under 2.2 GFLOP) are the one thing taken from a library (``torch.matmul`` -> rocBLAS/hipBLASLt), as the reference takes its products from cuBLAS (src/op/kernels/cuda/matmul_kernel.cu:76-86).
+the call raises.  Matrix products that none of the kernels here takes or wins are the one thing taken from a library
+(``torch.matmul`` -> rocBLAS/hipBLASLt), as the reference takes its products from cuBLAS
+(src/op/kernels/cuda/matmul_kernel.cu:76-86): from 17 to 64 rows those that :func:`skinny_wins` leaves (float32 rows of more than
+2,048 elements, bfloat16 ones of more than 4,096 past 32 rows, matrices that are not re-tiled, as the vocabulary head); of more
+rows the bfloat16 ones that :func:`tiled_wins` leaves (past 512 rows nearly all) and the float32 ones under 2.2 GFLOP that
+:func:`skinny_deals` leaves; and inputs that are not one aligned run of memory.
 """
 from __future__ import annotations
 

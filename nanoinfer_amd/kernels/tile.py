@@ -59,9 +59,10 @@ def _split_plan(M: int, N: int, K: int, gated: bool) -> Tuple[int, int, float]:
 def split_wins(x: torch.Tensor, rows: torch.Tensor) -> bool:
     """Whether ``x . rows^T`` goes to the float32 product of :func:`split_gemm`: more rows than the skinny product takes
     and work enough to pay for its start (some 8 us from the first load to the first matrix instruction).  Measured in
-    recorded launches against the library's float32 product (us, library : this): 512 rows on [16384, 2048] 243 : 163,
-    on [2048, 8192] 135 : 94, on [3072, 2048] 58 : 46, on [2048, 2048] 39 : 38; 164 rows on [3072, 3072] 42 : 39, on
-    [3072, 2048] 28 : 30, on [2048, 2048] 20 : 26: the line lies at 2.2 GFLOP."""
+    recorded launches, each with another W, against the library's float32 product (us, library : this): 512 rows on
+    [16384, 2048] 259 : 172, on [2048, 8192] 135 : 99, on [3072, 2048] 61 : 48, on [2048, 2048] 38 : 37; 164 rows on [3072, 3072]
+    42 : 39, on [3072, 2048] 28 : 32, on [2048, 2048] 21 : 27; 256 rows on [3072, 2048] 40 : 34, on [2048, 2048] 22.5 : 28: the line
+    lies at 2.2 GFLOP."""
     M, K = x.shape
     return (x.dtype == torch.float32 and M > 64 and K % 4 == 0 and 2.0 * M * rows.shape[0] * K >= 2.2e9 and x.is_contiguous()
             and rows.is_contiguous() and x.data_ptr() % 16 == 0 and rows.data_ptr() % 16 == 0)
