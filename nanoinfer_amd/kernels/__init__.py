@@ -6,8 +6,8 @@ the call raises.  Matrix products that none of the kernels here takes or wins ar
 (``torch.matmul`` -> rocBLAS/hipBLASLt), as the reference takes its products from cuBLAS
 (src/op/kernels/cuda/matmul_kernel.cu:76-86): from 17 to 64 rows those that :func:`skinny_wins` leaves (float32 rows of more than
 2,048 elements, bfloat16 ones of more than 4,096 past 32 rows, matrices that are not re-tiled, as the vocabulary head); of more
-rows the bfloat16 ones that :func:`tiled_wins` leaves (past 512 rows nearly all) and the float32 ones under 2.2 GFLOP that
-:func:`skinny_deals` leaves; and inputs that are not one aligned run of memory.
+rows the bfloat16 ones that :func:`tiled_wins` leaves (past 512 rows nearly all) and the float32 ones under some 2.2 GFLOP that
+:func:`pair_wins`, :func:`split_wins` and :func:`skinny_deals` leave; and inputs that are not one aligned run of memory.
 """
 from __future__ import annotations
 
@@ -634,14 +634,19 @@ def tile_weight(w: torch.Tensor) -> torch.Tensor:
 
 class Weight:
     """A matrix [out, in] as the products want it: ``rows`` as stored (for the library product of
-    many rows) and, optionally, ``tiles`` in the order the skinny product streams it."""
+    many rows), optionally ``tiles`` in the order the skinny product streams it, and ``pairs``: a large float32 matrix
+    on the GPU as two halves a number for :func:`pair_gemm`."""
 
-    __slots__ = ("rows", "tiles", "rows_t")
+    __slots__ = ("rows", "tiles", "rows_t", "pairs")
 
-    def __init__(self, rows: torch.Tensor, tiled: bool = True):
+    def __init__(self, rows: torch.Tensor, tiled: bool = True, pairs: Optional[bool] = None):
         self.rows = rows
         self.rows_t = rows.t()        # the view the library product takes, made once
         self.tiles = tile_weight(rows) if tiled and rows.dtype in (torch.float32, torch.bfloat16) else None
+        self.pairs = None
+        if ((tiled if pairs is None else pairs) and rows.is_cuda and rows.dtype == torch.float32 and rows.is_contiguous() and rows.data_ptr() % 16 == 0
+                and pair_holds(*rows.shape)):
+            self.pairs = pair_weight(rows)
 
     @property
     def shape(self):
@@ -1148,7 +1153,7 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
            pending: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None, leave: Optional[NormSpec] = None,
            addends: bool = False):
     """``x . weight^T`` with ``weight`` stored [out, in].  Few rows go to the hand-written skinny
-    product, more of them to the tiled products (:func:`tiled_wins`, :func:`split_wins`), the rest to the library
+    product, more of them to the tiled products (:func:`tiled_wins`, :func:`pair_wins`, :func:`split_wins`), the rest to the library
     (rocBLAS/hipBLASLt; its reduced-precision matrix modes for float32 are switched off at import).
     ``out_dtype`` float32 keeps the float32 accumulators of a bfloat16 product.  ``x`` may be a
     :class:`NormedInput` where :func:`norm_prologue_ok` holds.  With ``residual`` (the float32
@@ -1207,6 +1212,8 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
         if out is None:
             out = torch.empty(M, rows.shape[0], dtype=out_dtype, device=x.device)
         return skinny_gemm(x, weight, out)
+    if out_dtype == torch.float32 and pair_wins(x, weight):
+        return pair_gemm(x, weight, out, addends=addends)
     if out_dtype == torch.float32 and split_wins(x, rows):
         return split_gemm(x, rows, out, addends=addends)
     if tiled_wins(x, weight, addends=addends) and (out is None or out.data_ptr() % 16 == 0):
@@ -1240,6 +1247,10 @@ def linear_swiglu(x, weight_gate_up, activation: str = "silu") -> torch.Tensor:
                                       and (M <= SKINNY_BEST_ROWS or inter % 16 == 0)):
         return skinny_gemm(x, weight_gate_up, out, swiglu=True, activation=activation)
     rows, _ = _rows_and_tiles(weight_gate_up)
+    if pair_wins(x, weight_gate_up):
+        if inter % 32 == 0 and pair_plan(M, 2 * inter, Kd, True)[2] <= pair_plan(M, 2 * inter, Kd)[2] + 4.0 + 12.0 * M * inter / 4e6:
+            return pair_gemm(x, weight_gate_up, out, gated=activation)
+        return swiglu(pair_gemm(x, weight_gate_up), out, activation)
     if split_wins(x, rows):
         # in one kernel, or cut along K with the SwiGLU kernel behind it (which moves 12 bytes an output at 4 TB/s)
         if split_plan(M, 2 * inter, Kd, True)[2] <= split_plan(M, 2 * inter, Kd)[2] + 4.0 + 12.0 * M * inter / 4e6:
@@ -1261,6 +1272,8 @@ def linear_relu2(x, weight) -> torch.Tensor:
         out = torch.empty(M, weight.shape[0], dtype=x.dtype, device=x.device)
         return skinny_gemm(x, weight, out, activation="relu2")
     rows, _ = _rows_and_tiles(weight)
+    if pair_wins(x, weight):
+        return pair_gemm(x, weight, squared=True)
     if split_wins(x, rows):
         return split_gemm(x, rows, squared=True)
     if tiled_wins(x, weight):
@@ -1278,7 +1291,7 @@ torch.backends.cuda.matmul.allow_tf32 = False
 torch.backends.cudnn.allow_tf32 = False
 
 # products of many rows on the matrix cores
-from .tile import (experts_grouped, experts_grouped_wins, split_gemm, split_plan, split_wins, tile_lib, tiled_gemm, tiled_plan,  # noqa: E402,F401
+from .tile import (experts_grouped, experts_grouped_wins, pair_gemm, pair_holds, pair_plan, pair_rows, pair_weight, pair_wins, split_gemm, split_plan, split_wins, tile_lib, tiled_gemm, tiled_plan,  # noqa: E402,F401
                    tiled_wins)
 # sums onto the residual stream, routed experts, the gated delta rule, attention with a bias by distance
 from .stream import (BIAS_ATTENTION_MFMA_FROM, DELTA_RUN_FROM, EXPERTS_FEW_ROWS, add_rmsnormed, add_vector,  # noqa: E402,F401

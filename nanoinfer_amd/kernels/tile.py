@@ -115,6 +115,125 @@ def _add_shares(parts: torch.Tensor, dtype: torch.dtype, out: Optional[torch.Ten
     return out
 
 
+# ---------------------------------------------------------------- float32 by three products in half precision
+
+# Tiles of the product in half precision: rows of x, rows of W, workgroups a compute unit holds, and in microseconds: what a
+# launch takes beside its steps, 16 columns of K with one workgroup alone on its unit and with all units full, and how late between the
+# two the time rises (the power of the share of the units that is taken).  Fitted to sweeps of all tiles and shares at 100 to
+# 2,000 rows over the layer sizes of the 1B, 3B and 8B shapes, recorded, every launch with another W: of 99 plans taken the
+# average is 2 % above the best and the worst 22.
+PAIR_TILES = ((128, 256, 1, 16.1, 0.447, 0.651, 4.2), (64, 256, 2, 12.4, 0.228, 0.729, 1.18), (128, 128, 2, 11.8, 0.278, 0.745, 1.25),
+              (64, 128, 3, 8.8, 0.115, 0.612, 1.06))
+
+
+def pair_lib() -> ctypes.CDLL:
+    return _load(_build.PAIR_GEMM)
+
+
+def _pair_cost(M: int, N: int, K: int, tile: int, shares: int, groups: int = 1) -> float:
+    """Microseconds of a product in half precision, by the figures above.  ``groups`` as for :func:`_split_cost`."""
+    bm, bn, held, fixed, alone, loaded, late = PAIR_TILES[tile]
+    tiles = -(-M // bm) if groups == 1 else M // bm + (groups + 1) // 2
+    full, rest = divmod(tiles * -(-N // bn) * shares, COMPUTE_UNITS * held)
+    steps = -(-K // (32 * shares)) * 2
+    cost = fixed + full * loaded * steps + ((alone + (loaded - alone) * (rest / (COMPUTE_UNITS * held)) ** late) * steps if rest else 0.0)
+    return max(cost, 3.0 + N * K * 4 / 5.5e6) + (shares * M * N * 4 / 4.6e6 if shares > 1 else 0.0)
+
+
+def pair_plan(M: int, N: int, K: int, gated: bool = False) -> Tuple[int, int, float]:
+    """(tile, shares, estimated microseconds) of :func:`pair_gemm`."""
+    return _pair_plan(_whole(M), N, K, gated)
+
+
+@functools.lru_cache(maxsize=4096)
+def _pair_plan(M: int, N: int, K: int, gated: bool) -> Tuple[int, int, float]:
+    cost, tile, shares = min((_pair_cost(M, N, K, t, s), t, s) for t in range(2 if gated else 4)
+                             for s in ((1,) if gated else (1, 2, 3, 4, 6, 8, 12)) if s == 1 or K // s >= 256)
+    return tile, shares, cost
+
+
+def pair_holds(N: int, K: int) -> bool:
+    """Whether a float32 matrix [N, K] is kept as pairs of halves beside its rows: one that :func:`pair_gemm` takes (whole
+    vectors of four, bytes counted in 31 bits) and that is large enough for a product of a few thousand rows to go there."""
+    return K % 4 == 0 and K >= 128 and N >= 32 and 1 << 18 <= N * K and (N + 31) * (K + 31) < 1 << 29
+
+
+def _pair_planes(rows: int, K: int, device) -> Tuple[torch.Tensor, torch.Tensor]:
+    return (torch.empty(rows * -(-K // 32) * 128, dtype=torch.uint8, device=device), torch.empty(rows, 2, dtype=torch.int32, device=device))
+
+
+def pair_weight(rows: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+    """The float32 matrix [N, K] as :func:`pair_gemm` reads it: its numbers as two halves each, scaled by a power of two a
+    row, and for every row int32 (that power, how many of its numbers are small beside its largest)."""
+    N, K = rows.shape
+    _gpu(rows, "w", torch.float32)
+    if K % 4 or rows.data_ptr() % 16 or (N + 31) * (K + 31) >= 1 << 29:
+        raise KernelError(f"pairs of halves are not made of a matrix [{N}, {K}] at this address")
+    planes, info = _pair_planes(-(-N // 32) * 32, K, rows.device)
+    _check(pair_lib().ni_pair_weight(_ptr(rows), _ptr(planes), _ptr(info), N, K, _stream()), "pair_weight")
+    return planes, info
+
+
+def pair_rows(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+    """The same of the rows of x [M, K], in another order and with the count of the numbers that are not small."""
+    M, K = x.shape
+    _gpu(x, "x", torch.float32)
+    if K % 4 or x.data_ptr() % 16 or M * (K + 31) >= 1 << 29:
+        raise KernelError(f"pairs of halves are not made of rows [{M}, {K}] at this address")
+    planes, info = _pair_planes(M, K, x.device)
+    _check(pair_lib().ni_pair_rows(_ptr(x), _ptr(planes), _ptr(info), M, K, _stream()), "pair_rows")
+    return planes, info
+
+
+# Operations from which a float32 product goes to pair_gemm.  Measured in recorded launches, each with another W and all its kernels
+# counted (us, library : this): [2048, 2048] at 256 / 400 / 800 rows (2.1 / 3.4 / 6.7 GFLOP) 22.8 : 26.0, 38.9 : 32.0, 65.7 : 42.9;
+# [3072, 2048] at 130 / 164 / 200 (1.6 / 2.1 / 2.5) 22.6 : 26.6, 30.6 : 27.5, 31.3 : 29.5; [4096, 1024] at 256 / 400 (2.1 / 3.4) 24.1 : 26.6,
+# 37.0 : 31.3; [3072, 3072] at 130 / 164 (2.5 / 3.1) 30.3 : 31.3, 42.0 : 32.2; [2048, 8192] at 65 / 130 (2.2 / 4.4) 42.6 : 40.0, 63.8 : 47.6.
+PAIR_FLOPS = 2.4e9
+
+
+def pair_wins(x: torch.Tensor, weight) -> bool:
+    """Whether a float32 product of more rows than the skinny product takes goes to :func:`pair_gemm`: a matrix that is kept as
+    pairs of halves and work enough to pay for the start and for the pass that makes pairs of x."""
+    if getattr(weight, "pairs", None) is None or x.dtype != torch.float32:
+        return False
+    M, K = x.shape
+    return (M > 64 and 2.0 * M * weight.rows.shape[0] * K >= PAIR_FLOPS and M * (K + 31) < 1 << 29 and x.is_contiguous()
+            and x.data_ptr() % 16 == 0)
+
+
+def pair_gemm(x: torch.Tensor, weight, out: Optional[torch.Tensor] = None, gated: Optional[str] = None, squared: bool = False,
+              plan: Optional[Tuple[int, int]] = None, addends: bool = False) -> torch.Tensor:
+    """``x . weight^T`` for float32 ``x`` [M, K] and a :class:`Weight` [N, K] that is kept as pairs of halves, by three products
+    in half precision.  The other arguments as for :func:`split_gemm`."""
+    M, K = x.shape
+    rows, pairs = weight.rows, weight.pairs
+    if pairs is None:
+        raise KernelError("this product takes a matrix that is kept as pairs of halves")
+    N = rows.shape[0]
+    _gpu(x, "x", torch.float32, (M, rows.shape[1]))
+    if gated is not None and (N % 64 or squared):
+        raise KernelError("a gated product takes a stacked matrix of halves of whole tiles of 32 and no other activation")
+    _addends_alone(addends, out, gated, squared)
+    cols = N if gated is None else N // 2
+    tile, shares = plan or pair_plan(M, N, K, gated is not None)[:2]
+    per = -(-K // (32 * shares)) * 32
+    shares = -(-K // per)                                   # no share is empty
+    planes, info = pair_rows(x)
+    if shares > 1:
+        parts = torch.empty(shares, M, N, dtype=torch.float32, device=x.device)
+    elif out is None:
+        out = torch.empty(M, cols, dtype=torch.float32, device=x.device)
+    if out is not None:
+        _gpu(out, "out", torch.float32, (M, cols))
+    _check(pair_lib().ni_pair_gemm(_ptr(planes), _ptr(info), _ptr(pairs[0]), _ptr(pairs[1]), _ptr(x), _ptr(rows), _ptr(parts if shares > 1 else out),
+                                   M, N, K, tile, shares, per, int(gated is not None), GATED_ACTIVATIONS[gated or "silu"],
+                                   int(squared and shares == 1), _stream()), "pair_gemm")
+    if shares > 1:
+        return parts if addends else _add_shares(parts, torch.float32, out, squared)
+    return out
+
+
 # ---------------------------------------------------------------- bfloat16 on the re-tiled matrix
 
 # Tiles of the bfloat16 product: rows of x, rows of W, workgroups a compute unit holds, and in microseconds: before the
@@ -243,55 +362,91 @@ def _grouped_tiles(places: int, N: int, K: int, groups: int) -> Tuple[float, int
     return min((_split_cost(places, N, K, t, 1, groups), t) for t in range(len(SPLIT_TILES)))
 
 
-def experts_grouped_wins(x: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor, top: int, experts: int) -> bool:
+def _grouped_pair_plan(places: int, N: int, K: int, groups: int) -> Tuple[float, int]:
+    return _grouped_pair_tiles(_whole(places), N, K, groups)
+
+
+@functools.lru_cache(maxsize=1024)
+def _grouped_pair_tiles(places: int, N: int, K: int, groups: int) -> Tuple[float, int]:
+    return min((_pair_cost(places, N, K, t, 1, groups), t) for t in range(len(PAIR_TILES)))
+
+
+def _experts_in_pairs(places: int, w_up, w_down, d: int, per: int, ff: int) -> bool:
+    """Whether both products of routed experts are made in half precision: matrices that are kept as pairs of halves, an
+    expert's rows of up whole tiles of 32 and its columns of down whole stages."""
+    return (getattr(w_up, "pairs", None) is not None and getattr(w_down, "pairs", None) is not None and d % 32 == 0 and ff % 32 == 0
+            and per % 32 == 0 and places * max(d, ff) < 1 << 29)
+
+
+def experts_grouped_wins(x: torch.Tensor, w_up, w_down, top: int, experts: int) -> bool:
     """Whether routed experts of float32 rows go expert by expert (:func:`experts_grouped`) instead of as two dense
-    products over all experts: by the estimates of :func:`split_plan`, with 25 us for the lists and the sums beside the
-    passes over the entries' rows.  1,500 rows of 2,048 elements, four of sixteen experts of 1,024: 290 us for the two products
-    against 960."""
+    products over all experts: by the estimates of :func:`split_plan` or :func:`pair_plan`, with 25 us for the lists and the sums
+    beside the passes over the entries' rows.  1,500 rows of 2,048 elements, four of sixteen experts of 1,024: 290 us for the two
+    products against 960 (in three parts)."""
+    up, down = getattr(w_up, "rows", w_up), getattr(w_down, "rows", w_down)
     M, d = x.shape
-    per, ff = w_up.shape[0] // experts, w_down.shape[1] // experts
-    if not (x.dtype == torch.float32 and d % 4 == 0 and ff % 4 == 0 and M * top < 1 << 24 and split_wins(x, w_up)
-            and w_down.is_contiguous() and w_down.data_ptr() % 16 == 0):
+    per, ff = up.shape[0] // experts, down.shape[1] // experts
+    if not (x.dtype == torch.float32 and d % 4 == 0 and ff % 4 == 0 and M * top < 1 << 24 and split_wins(x, up)
+            and down.is_contiguous() and down.data_ptr() % 16 == 0):
         return False
     places = M * top
-    grouped = _grouped_plan(places, per, d, experts)[0] + _grouped_plan(places, d, ff, experts)[0] + 25.0 + (12.0 * d + 4.0 * per) * places / 4e6
-    return grouped < split_plan(M, experts * per, d)[2] + split_plan(M, d, experts * ff)[2]
+    plan, whole = (_grouped_pair_plan, pair_plan) if _experts_in_pairs(places, w_up, w_down, d, per, ff) else (_grouped_plan, split_plan)
+    grouped = plan(places, per, d, experts)[0] + plan(places, d, ff, experts)[0] + 25.0 + (12.0 * d + 4.0 * per) * places / 4e6
+    return grouped < whole(M, experts * per, d)[2] + whole(M, d, experts * ff)[2]
 
 
-def experts_grouped(x: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor, chosen: torch.Tensor, mix: torch.Tensor, experts: int,
+def experts_grouped(x: torch.Tensor, w_up, w_down, chosen: torch.Tensor, mix: torch.Tensor, experts: int,
                     act, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The weighted sum of every row's chosen experts, float32 [T, d]: the entries (token, expert) are put in the order of
     their experts, each expert multiplies its own tokens' rows, and a token's results are added in the order in which it
-    chose.  ``w_up`` [E * per, d], ``w_down`` [d, E * ff]; ``act(up [entries, per], weights [entries, 1])`` gives the hidden
-    rows [entries, ff].  An index of E or more in ``chosen`` int32 [T, top] names an expert that is not among these."""
+    chose.  ``w_up`` [E * per, d], ``w_down`` [d, E * ff], tensors or :class:`Weight`; ``act(up [entries, per], weights [entries, 1])``
+    gives the hidden rows [entries, ff].  An index of E or more in ``chosen`` int32 [T, top] names an expert that is not among these."""
+    up_rows, down_rows = getattr(w_up, "rows", w_up), getattr(w_down, "rows", w_down)
     T, d = x.shape
     top, E = chosen.shape[1], experts
     places = T * top
-    if w_up.shape[0] % E or w_down.shape[1] % E:
+    if up_rows.shape[0] % E or down_rows.shape[1] % E:
         raise KernelError("the matrices are not whole experts")
-    per, ff = w_up.shape[0] // E, w_down.shape[1] // E
+    per, ff = up_rows.shape[0] // E, down_rows.shape[1] // E
     _gpu(x, "x", torch.float32)
-    _gpu(w_up, "w_up", torch.float32, (E * per, d))
-    _gpu(w_down, "w_down", torch.float32, (d, E * ff))
+    _gpu(up_rows, "w_up", torch.float32, (E * per, d))
+    _gpu(down_rows, "w_down", torch.float32, (d, E * ff))
     _gpu(chosen, "chosen", torch.int32, (T, top))
     _gpu(mix, "mix", torch.float32, (T, top))
-    if d % 4 or ff % 4 or any(t.data_ptr() % 16 for t in (x, w_up, w_down)):
+    if d % 4 or ff % 4 or any(t.data_ptr() % 16 for t in (x, up_rows, down_rows)):
         raise KernelError("rows of the experts' products are not aligned to 16 bytes")
+    pairs = _experts_in_pairs(places, w_up, w_down, d, per, ff)
     ints = torch.empty(E + 1 + 2 * places, dtype=torch.int32, device=x.device)
     offsets, rows, place = ints[:E + 1], ints[E + 1:E + 1 + places], ints[E + 1 + places:]
     weights = torch.empty(places, 1, dtype=torch.float32, device=x.device)
     lib = tile_lib()
     _check(lib.ni_expert_lists(_ptr(chosen), _ptr(mix), T, top, E, _ptr(offsets), _ptr(rows), _ptr(weights), _ptr(place), _stream()), "expert_lists")
     up = torch.empty(places, per, dtype=torch.float32, device=x.device)
-    _check(lib.ni_split_gemm_grouped(_ptr(x), _ptr(w_up), _ptr(up), places, per, d, _ptr(offsets), _ptr(rows), E, ctypes.c_size_t(per * d), d,
-                                     _grouped_plan(places, per, d, E)[1], _stream()), "experts_up")
+    if pairs:
+        _pair_grouped(x, w_up, up, offsets, rows, E, False)
+    else:
+        _check(lib.ni_split_gemm_grouped(_ptr(x), _ptr(up_rows), _ptr(up), places, per, d, _ptr(offsets), _ptr(rows), E, ctypes.c_size_t(per * d), d,
+                                         _grouped_plan(places, per, d, E)[1], _stream()), "experts_up")
     hidden = act(up, weights)
     _gpu(hidden, "hidden", torch.float32, (places, ff))
     y = torch.empty(places, d, dtype=torch.float32, device=x.device)
-    _check(lib.ni_split_gemm_grouped(_ptr(hidden), _ptr(w_down), _ptr(y), places, d, ff, _ptr(offsets), None, E, ctypes.c_size_t(ff), E * ff,
-                                     _grouped_plan(places, d, ff, E)[1], _stream()), "experts_down")
+    if pairs:
+        _pair_grouped(hidden, w_down, y, offsets, None, E, True)
+    else:
+        _check(lib.ni_split_gemm_grouped(_ptr(hidden), _ptr(down_rows), _ptr(y), places, d, ff, _ptr(offsets), None, E, ctypes.c_size_t(ff), E * ff,
+                                         _grouped_plan(places, d, ff, E)[1], _stream()), "experts_down")
     if out is None:
         out = torch.empty(T, d, dtype=torch.float32, device=x.device)
     _gpu(out, "out", torch.float32, (T, d))
     _check(lib.ni_gather_entries(_ptr(y), _ptr(place), _ptr(out), T, d, top, _stream()), "gather_entries")
     return out
+
+
+def _pair_grouped(x: torch.Tensor, weight, out: torch.Tensor, offsets: torch.Tensor, rows: Optional[torch.Tensor], experts: int, down: bool) -> None:
+    """``out[p] = x[rows[p]] . W_e^T`` for the places p of every expert's list; its rows of W behind the others' or (``down``) beside them."""
+    places, N = out.shape
+    K = x.shape[1]
+    planes, info = pair_rows(x)
+    _check(pair_lib().ni_pair_gemm_grouped(_ptr(planes), _ptr(info), _ptr(weight.pairs[0]), _ptr(weight.pairs[1]), _ptr(x), _ptr(weight.rows), _ptr(out),
+                                           places, N, K, _ptr(offsets), _ptr(rows), experts, int(down),
+                                           _grouped_pair_plan(places, N, K, experts)[1], _stream()), "pair_gemm_grouped")

@@ -77,7 +77,8 @@ class Runtime:
         """Bytes of device memory that the model's tensors take (every shared buffer once)."""
         seen, total = set(), 0
         for value in self.shared.values():
-            for t in (value if isinstance(value, tuple) else (getattr(value, "rows", value), getattr(value, "tiles", None))):
+            for t in (value if isinstance(value, tuple) else
+                      (getattr(value, "rows", value), getattr(value, "tiles", None), *(getattr(value, "pairs", None) or ()))):
                 if isinstance(t, torch.Tensor) and t.is_cuda and t.untyped_storage().data_ptr() not in seen:
                     seen.add(t.untyped_storage().data_ptr())
                     total += t.untyped_storage().nbytes()
@@ -92,16 +93,18 @@ class Runtime:
             self.shared[key] = t
         return t
 
-    def weight(self, name: str, cpu: torch.Tensor, tiled: bool = True):
+    def weight(self, name: str, cpu: torch.Tensor, tiled: bool = True, pairs: Optional[bool] = None):
         """A checkpoint matrix as a :class:`nanoinfer_amd.kernels.Weight`: its rows on the device in the
         compute type (shared with :meth:`matrix`) plus, when ``tiled``, the copy that the skinny
-        product of decoding streams."""
+        product of decoding streams, and, when ``pairs`` (where ``tiled`` if not said), a large float32 matrix as the
+        products of many rows take it."""
         from .. import kernels as K
+        pairs = (tiled if pairs is None else pairs) and self.tiled
         tiled = tiled and self.tiled
-        key = ("weight", name, self.dtype, tiled)
+        key = ("weight", name, self.dtype, tiled, pairs)
         w = self.shared.get(key)
         if w is None:
-            w = K.Weight(self.matrix(name, cpu), tiled=tiled)
+            w = K.Weight(self.matrix(name, cpu), tiled=tiled, pairs=pairs)
             self.shared[key] = w
         return w
 

@@ -471,9 +471,9 @@ class RoutedExperts(Part):
             raise ValueError(f"{self.top} experts cannot be chosen from {self.keep} of {self.groups} groups of {outputs}")
         self.w_router = rt.weight(names["router"], weights["router"])
         order = [k for e in range(self.E) for k in ((f"gate{e}", f"up{e}") if self.gated else (f"up{e}",))]
-        self.w_up = rt.weight("|".join(names[k] for k in order), torch.cat([weights[k] for k in order], dim=0), tiled=False)
+        self.w_up = rt.weight("|".join(names[k] for k in order), torch.cat([weights[k] for k in order], dim=0), tiled=False, pairs=True)
         self.w_down = rt.weight("|".join(names[f"down{e}"] for e in range(self.E)),
-                                torch.cat([weights[f"down{e}"] for e in range(self.E)], dim=1), tiled=False)
+                                torch.cat([weights[f"down{e}"] for e in range(self.E)], dim=1), tiled=False, pairs=True)
         self.shared = None
         if p.get("shared") is not None:
             self.shared = build_part("feed_forward", p["shared"], getattr(weights, "checkpoint", {}), rt)
@@ -492,8 +492,8 @@ class RoutedExperts(Part):
         if few:
             y = K.experts_few(x, self.w_up.rows, self.w_down.rows, chosen, mix, self.ff, self.activation, None if out is None else out[0],
                               limit=self.limit, slope=self.slope)
-        elif K.experts_grouped_wins(x, self.w_up.rows, self.w_down.rows, self.top, self.E):
-            y = K.experts_grouped(x, self.w_up.rows, self.w_down.rows, chosen, mix, self.E,
+        elif K.experts_grouped_wins(x, self.w_up, self.w_down, self.top, self.E):
+            y = K.experts_grouped(x, self.w_up, self.w_down, chosen, mix, self.E,
                                   lambda up, weights: K.experts_act(up, weights, self.ff, self.activation, self.limit, self.slope),
                                   out=None if out is None else out[0])
             if self.identity:

@@ -1,0 +1,199 @@
+"""The products of many float32 rows in half precision (``csrc/pair_gemm.hip``) alone: every tile at its edges, the rows and
+matrices that they hand on, the routed experts, and the error beside the other float32 products."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def K():
+    from nanoinfer_amd import kernels
+    return kernels
+
+
+class Held:
+    """A matrix as pairs of halves whatever its size (``Weight`` keeps the large ones so)."""
+
+    def __init__(self, K, rows):
+        self.rows, self.pairs = rows, K.pair_weight(rows)
+
+
+def operands(M, N, Kd, seed=0, spread=0):
+    g = torch.Generator().manual_seed(seed)
+    x, w = torch.randn(M, Kd, generator=g), torch.randn(N, Kd, generator=g)
+    if spread:      # rows of very different size, by powers of two
+        x *= 2.0 ** torch.randint(-spread, spread + 1, (M, 1), generator=g)
+        w *= 2.0 ** torch.randint(-spread, spread + 1, (N, 1), generator=g)
+    return x.cuda(), w.cuda()
+
+
+def error(got, x, w):
+    """Of all results together, in the root of the sum of the squared products."""
+    want = x.double() @ w.double().t()
+    return float(((got.double() - want) / ((x.double() ** 2) @ (w.double() ** 2).t()).sqrt()).pow(2).mean().sqrt())
+
+
+def bounded(got, x, w):
+    """The bound of a float32 sum: 6 K + 8 roundings of at most 2^-24 of sum |x||w| each (three parts; halves take fewer)."""
+    want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    return bool(((got.double() - want).abs() <= (6 * x.shape[1] + 8) * 2.0 ** -24 * size).all())
+
+
+# Sums of 100 to 2,048 numbers are off by 1e-7 to 3e-7; without any one of the three products by 1e-4 and more.  The roundings
+# of a sum, each of its size so far, grow together as the root of the number of addends beside the sum itself: longer
+# sums by that much more (8,192 numbers 5.8e-7).
+def whole(Kd):
+    return 2.0 ** -21 * max(1.0, (Kd / 2048) ** 0.5)
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("M,N,Kd,shares", [(1, 33, 128, 1), (63, 255, 132, 1), (64, 256, 160, 1), (65, 257, 192, 1), (129, 130, 100, 1),
+                                           (257, 513, 132, 1), (300, 258, 300, 2), (70, 77, 1036, 3), (256, 128, 2048, 8), (130, 40, 8196, 1)])
+def test_pair_gemm_at_the_edges_of_its_tiles(K, tile, M, N, Kd, shares):
+    x, w = operands(M, N, Kd, seed=M + N + Kd, spread=30)
+    out = torch.full((M + 1, N), 7.0, device="cuda")
+    K.pair_gemm(x, Held(K, w), out[:M], plan=(tile, shares))
+    assert bounded(out[:M], x, w) and error(out[:M], x, w) <= whole(Kd)
+    assert bool((out[M] == 7.0).all())                       # nothing behind the last row
+
+
+@pytest.mark.parametrize("tile", [0, 1])
+@pytest.mark.parametrize("M,inter", [(65, 32), (130, 96), (129, 160)])
+def test_pair_gemm_gated_and_squared(K, tile, M, inter):
+    x, w = operands(M, 2 * inter, 196, seed=inter)
+    held = Held(K, w)
+    z = K.pair_gemm(x, held, plan=(tile, 1))
+    for act in ("silu", "gelu_tanh"):
+        got = K.pair_gemm(x, held, gated=act, plan=(tile, 1))
+        assert torch.allclose(got, K.swiglu(z, torch.empty_like(got), act), rtol=1e-6, atol=0)
+    assert torch.equal(K.pair_gemm(x, held, squared=True, plan=(tile, 1)), torch.relu(z) ** 2)
+    parts = K.pair_gemm(x, held, plan=(3, 2), addends=True)
+    assert torch.equal(K.pair_gemm(x, held, squared=True, plan=(3, 2)), torch.relu(parts[0] + parts[1]) ** 2)
+
+
+@pytest.mark.parametrize("M,N,Kd", [(65, 16384, 2048), (512, 2048, 8192), (512, 3072, 3072), (1000, 2500, 700), (700, 1024, 2048), (512, 8192, 512)])
+def test_no_less_exact_than_in_three_parts_or_from_the_library(K, M, N, Kd):
+    x, w = operands(M, N, Kd)
+    weight = K.Weight(w)
+    assert K.pair_wins(x, weight)
+    calls = K.library_calls()
+    # no less exact is what is claimed; measured 0.43 of the other two where all are cut alike, 0.82 of a product in three parts
+    # that is cut along K where this one is not (shorter sums have fewer roundings)
+    got = error(K.linear(x, weight), x, w)
+    assert got <= error(K.split_gemm(x, w), x, w) and got <= error(torch.mm(x, w.t()), x, w)
+    g = K.linear_swiglu(x, weight)
+    want = torch.nn.functional.silu(x.double() @ w[:N // 2].double().t()) * (x.double() @ w[N // 2:].double().t())
+    assert float((g.double() - want).norm() / want.norm()) <= 1e-5
+    assert K.library_calls() == calls
+
+
+def left(x, w):
+    """Whether any tile may be made in halves, by the rule in 64 bits: big numbers against others."""
+    def big(t):
+        top = t.double().abs().amax(1, keepdim=True)
+        return (t.double().abs() >= 2.0 ** (torch.floor(torch.log2(top)) - 12)).sum(1)
+    return int(big(x).min()) - 64 < int((w.shape[1] - big(w)).max())
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("kind", ["few in x", "few in w", "an outlier against nothing", "many binades", "zeros in w", "short"])
+def test_what_halves_cannot_hold_is_made_in_three_parts(K, tile, kind):
+    """Such tiles are, bit for bit, what the product in three parts gives."""
+    M, N, Kd = 200, 270, 512
+    x, w = operands(M, N, Kd, seed=5)
+    if kind == "few in x":
+        x[77, 63:] = 0.0
+        x[77, 1::2] = 0.0
+    elif kind == "few in w":
+        w[100:] = torch.where(torch.arange(Kd, device="cuda") % 9 == 0, w[100:], 0.0)
+        x[:, ::9] = 0.0
+    elif kind == "an outlier against nothing":
+        x[:, 9], w[:, 9] = 1e13, 0.0
+    elif kind == "many binades":
+        x *= 2.0 ** torch.randint(-60, 1, (M, Kd), generator=torch.Generator().manual_seed(1)).cuda()
+        w *= 2.0 ** torch.randint(-60, 1, (N, Kd), generator=torch.Generator().manual_seed(2)).cuda()
+    elif kind == "zeros in w":
+        w[torch.rand(N, Kd, generator=torch.Generator().manual_seed(3)).cuda() < 0.7] = 0.0
+        x = torch.relu(x)
+    else:
+        x, w = x[:, :60].contiguous(), w[:, :60].contiguous()
+    assert left(x, w)
+    got = K.pair_gemm(x, Held(K, w), plan=(tile, 1))
+    assert bounded(got, x, w)
+    want = K.split_gemm(x, w, plan=(1, 1))
+    if kind not in ("few in x", "few in w"):                # there some tiles are made in halves
+        assert torch.equal(got, want)
+    else:
+        assert torch.equal(got[77], want[77]) if kind == "few in x" else torch.equal(got[:, 256:], want[:, 256:])
+
+
+def test_numbers_of_many_binades_against_dense_rows(K):
+    """A row of x may hold numbers that halves cannot, where a row of W holds none: within a float32 sum's bound."""
+    x, w = operands(300, 256, 2048, seed=8)
+    x *= 2.0 ** torch.randint(-36, 1, x.shape, generator=torch.Generator().manual_seed(1)).cuda()
+    x[::3] *= 2.0 ** -120           # down to numbers below the smallest normal one
+    assert not left(x, w)
+    got = K.pair_gemm(x, Held(K, w), plan=(0, 1))
+    assert bounded(got[1::3], x[1::3], w) and error(got[1::3], x[1::3], w) <= whole(2048)
+    lost = 2.0 ** -149              # the results' own last place there
+    want = x.double() @ w.double().t()
+    assert bool(((got.double() - want).abs() <= 1e-5 * (x.double().abs() @ w.double().abs().t()) + lost).all())
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+def test_what_is_not_finite_stays_what_a_float32_product_makes_of_it(K, tile):
+    M, N, Kd = 200, 300, 132
+    x, w = operands(M, N, Kd, seed=3)
+    inf, nan = float("inf"), float("nan")
+    x[3, 5], x[70, 0], x[M - 1, Kd - 1], x[9, 8], x[9, 9] = inf, nan, -inf, inf, -inf
+    w[11, 2], w[N // 2 + 11, 7], w[N - 1, 3], w[41, 5] = -inf, inf, nan, 0.0
+    x[20], x[21], w[40] = 3.4e38, 3.4e38 * torch.sign(x[21]), 1e-30
+    x[130:], x[150] = 0.0, inf
+    x[64:128:2], w[64:128] = 0.0, w[64:128]
+    want = (x.cpu().double() @ w.cpu().double().t()).float()
+    got = K.pair_gemm(x, Held(K, w), plan=(tile, 1)).cpu()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(torch.isinf(got) * torch.sign(got), torch.isinf(want) * torch.sign(want))
+    fine = torch.isfinite(want)
+    a, b = torch.where(fine, got, 0.0), torch.where(fine, want, 0.0)
+    assert bool(((a - b).abs() <= 1e-5 * b.abs().amax(dim=1, keepdim=True)).all())
+    zeros, bad = torch.zeros(130, Kd, device="cuda"), w.clone()
+    assert torch.equal(torch.isnan(K.pair_gemm(zeros, Held(K, bad), plan=(tile, 1))).cpu().any(0), ~torch.isfinite(w.cpu()).all(1))
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("T,d,ff,E,top,spoiled", [(150, 128, 64, 5, 2, False), (90, 160, 96, 3, 3, False), (64, 512, 128, 7, 1, True)])
+def test_experts_in_halves(K, monkeypatch, tile, T, d, ff, E, top, spoiled):
+    from nanoinfer_amd.kernels import tile as tiles
+    monkeypatch.setattr(tiles, "_grouped_pair_plan", lambda *a: (0.0, tile))
+    g = torch.Generator().manual_seed(T)
+    x, up, down = torch.randn(T, d, generator=g), torch.randn(E * ff, d, generator=g), torch.randn(d, E * ff, generator=g)
+    if spoiled:
+        x[5, 3:] = 0.0
+    chosen = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(T)]).int()
+    mix = torch.rand(T, top, generator=g) + 0.1
+    x, up, down, chosen, mix = (t.cuda() for t in (x, up, down, chosen, mix))
+    act = lambda z, w: K.experts_act(z, w, ff, "relu2")      # noqa: E731
+    got = K.experts_grouped(x, Held(K, up), Held(K, down), chosen, mix, E, act)
+    want = torch.zeros(T, d, dtype=torch.float64, device="cuda")
+    for k in range(top):
+        for e in range(E):
+            here = chosen[:, k] == e
+            hid = torch.relu(x[here].double() @ up[e * ff:(e + 1) * ff].double().t()) ** 2
+            want[here] += mix[here, k, None].double() * (hid @ down[:, e * ff:(e + 1) * ff].double().t())
+    assert float((got.double() - want).norm() / want.norm()) <= 1e-6
+    assert not torch.equal(got, torch.zeros_like(got))
+
+
+def test_what_pair_gemm_does_not_take(K):
+    x, w = operands(70, 64, 128)
+    held = Held(K, w)
+    bare = K.Weight(w)
+    assert bare.pairs is None and not K.pair_wins(x, bare) and not K.pair_wins(x, w)
+    for bad in (lambda: K.pair_gemm(x, bare), lambda: K.pair_gemm(x.bfloat16(), held), lambda: K.pair_gemm(x[:, :64].contiguous(), held),
+                lambda: K.pair_gemm(x.view(-1)[1:1 + 69 * 128].view(69, 128), held), lambda: K.pair_gemm(x.t().contiguous().t(), held),
+                lambda: K.pair_gemm(x, Held(K, w[:63].contiguous()), gated="silu"), lambda: K.pair_gemm(x, held, squared=True, addends=True),
+                lambda: K.pair_weight(w[:, :126].contiguous()), lambda: K.pair_rows(x.bfloat16())):
+        with pytest.raises(K.KernelError):
+            bad()
