@@ -343,6 +343,11 @@ def _heads_per_tile(group: int) -> int:
     return 16 if group >= 16 else 8 if group > 4 else 4 if group > 2 else 2 if group > 1 else 1
 
 
+@functools.lru_cache(maxsize=None)
+def _f32_tile_tokens(hd: int, group: int) -> int:
+    return int(attention_mfma_f32_lib(hd).ni_mfma_attention_f32_tile_tokens(group))
+
+
 def mfma_tile_tokens(hd: int, group: int, n_tokens: Optional[int] = None, kv_heads: int = 1,
                      dtype: torch.dtype = torch.bfloat16) -> int:
     """Tokens of one tile of the matrix-core attention kernel for ``group`` query heads per kv head.
@@ -355,7 +360,7 @@ def mfma_tile_tokens(hd: int, group: int, n_tokens: Optional[int] = None, kv_hea
     2,560 tokens 100.4 : 78.6, 3,072 tokens 117.2 : 95.3, 4,096 tokens 150.8 : 108.0).  Without ``n_tokens``:
     the smallest tile.  The float32 kernel has one tile size."""
     if dtype == torch.float32:
-        return int(attention_mfma_f32_lib(hd).ni_mfma_attention_f32_tile_tokens(int(group)))
+        return _f32_tile_tokens(hd, int(group))
     lib = attention_mfma_lib(hd)
     hpt = _heads_per_tile(group)
     blocks = 1
@@ -412,6 +417,54 @@ def build_q_tiles(q_start, q_len, context_len, tile_tokens: int):
     return [x for t in tiles for x in t]
 
 
+def _f32_blocks(n_tiles: int, kv_heads: int, group: int, nsplit: int, hd: int) -> int:
+    """Blocks of 16 rows that a wavefront of the float32 prompt kernel owns: one, with two workgroups a tile, while the chip
+    holds them all at once, else two (up to head size 64; above one, the only size)."""
+    hpt = _heads_per_tile(group)
+    return _blocks_of(n_tiles * kv_heads * ((group + hpt - 1) // hpt), nsplit, hd)
+
+
+def _blocks_of(items: int, nsplit: int, hd: int) -> int:
+    return 2 if hd <= 64 and 2 * items * nsplit > 2 * COMPUTE_UNITS else 1
+
+
+def _f32_cost(items: int, tokens: int, max_keys: int, hd: int, nsplit: int) -> float:
+    """Microseconds of the float32 prompt kernel and of the kernel that merges the runs, for ``items`` tiles (times kv heads) of a
+    portion of ``tokens`` tokens, the last of which walks ``max_keys`` keys, in ``nsplit`` runs: rounds of as many workgroups as the
+    chip holds (two a compute unit, one above head size 128), each with a start and so much a key, less where a workgroup has its
+    unit to itself.  Fitted at 60 to 2,048 tokens and contexts of 60 to 4,000 keys, head sizes 64 (32 heads on 8) and 128 (24
+    on 8): of 84 plans the average is 2 % above the best of all runs.  Measured, the runs of the rule before on the float32 instructions :
+    this kernel by this rule, us: head size 64, 60 tokens at 900 keys 24.1 : 17.9; 164 at 1,700 56.3 : 34.3; 256 at 256 / 1,024
+    22.6 : 16.8, 46.7 : 29.6; 512 at 512 / 1,024 / 1,536 / 4,096 46.5 : 30.5, 75.1 : 41.8, 101 : 53.7, 233 : 114; 1,024 at 1,024
+    94.2 : 55.6; 2,048 at 2,048 253 : 132; head size 128, 60 at 900 41.2 : 24.5; 164 at 1,700 104 : 53.0; 512 at 512 / 1,536 84.1 : 40.4,
+    202 : 95.0; 1,024 at 1,024 171 : 82.4; head size 256, 8 heads on 2, 1,024 at 1,024 132 : 70.9.  How the runs matter: 700 tokens at
+    1,400, head size 64, in two / three / four / five / eight 81 / 86 / 74 / 67 / 74 (with five, 880 workgroups take two rounds of 512)."""
+    two = _blocks_of(items, nsplit, hd) == 2
+    alone, shared, start = ((0.062, 0.092, 5.0) if two else (0.046, 0.068, 4.0)) if hd <= 64 else (0.085, 0.103, 4.0) if hd <= 128 else (0.12, 0.12, 4.0)
+    groups = items * nsplit * (2 if hd <= 64 and not two else 1)
+    held = 2 * COMPUTE_UNITS if hd <= 128 else COMPUTE_UNITS
+    longest = -(-max_keys // (32 * nsplit)) * 32
+    if groups <= COMPUTE_UNITS:
+        cost = longest * alone + start
+    elif groups <= held:                       # a long and a short one on a unit, the long one alone at its end
+        shortest = max(max_keys - tokens, 0) / nsplit
+        cost = shortest * shared + (longest - shortest) * alone + start
+    else:
+        full, rest = divmod(groups, held)
+        last = alone / shared
+        if rest > COMPUTE_UNITS:
+            last += (1.0 - last) * (rest - COMPUTE_UNITS) / COMPUTE_UNITS
+        cost = (full + (last if rest else 0.0)) * (max(max_keys - tokens / 2, max_keys / 2) / nsplit * shared + start)
+    rows = items * (128 if hd <= 64 else 64)
+    return cost + (3.5 + rows * nsplit * (hd + 2) * 8 / 6e6 if nsplit > 1 else 0.0)
+
+
+@functools.lru_cache(maxsize=4096)
+def _f32_runs(items: int, tokens: int, max_keys: int, hd: int) -> int:
+    """(From 256 keys on two runs are never more than 5 % behind one.)"""
+    return min(range(2, min(max_keys // 32, 16) + 1), key=lambda n: _f32_cost(items, tokens, max_keys, hd, n))
+
+
 def mfma_splits(n_tiles: int, kv_heads: int, group: int, max_keys: int, hd: int = 64,
                 dtype: torch.dtype = torch.bfloat16) -> int:
     """Into how many runs the matrix-core kernel cuts the keys of every tile.  Cutting costs a
@@ -423,26 +476,14 @@ def mfma_splits(n_tiles: int, kv_heads: int, group: int, max_keys: int, hd: int 
     a step with fewer tiles than the chip has compute units, into runs of 512 keys or more until
     every unit has one.
 
-    In float32 a key costs sixteen times the matrix instructions and the merge is the same, so a cut pays much sooner:
-    runs of 32 keys or more, up to two workgroups a compute unit, whose wavefronts then multiply while others take
-    exponentials (a workgroup alone on a unit leaves one wavefront on each matrix core).  A workgroup more than that
-    where two would be left uneven: three runs up to 256 tiles of head size 64 or less, two up to 512 tiles (1,024 of
-    small heads, whose workgroups are small).  Measured, uncut and by the rule above : by this one, us: head size 64,
-    8 kv heads, 60 tokens at 900 keys 77.9 : 24.8; 164 at 1,700 82.5 : 57.1; 256 at 256 / 1,024 27.5 : 23.2,
-    56.1 : 47.3; 512 at 512 / 1,024 / 1,536 / 4,096 49.6 : 46.4, 91.4 : 74.8, 132 : 102, 243 : 231; 1,024 at 1,024 95.6 : 90.0
-    (2,048 at 2,048: 255 uncut, 268 in two); head size 128, 60 at 900 138.5 : 41.7, 164 at 1,700 141.5 : 105.9, 512 at 1,536
-    234 : 198, 1,024 at 1,024 178.5 : 168.0 (in three 220); head size 32, one kv head, 32 at 500 keys 30.9 : 10.6; head size 256,
-    2 kv heads, 256 at 256 86.5 : 35.0, 1,024 at 1,024 185.8 : 129.5.  Under 256 keys the cut gains less than the launch of the
-    merge costs a host that is behind (32 tokens at 200 keys 16.2 : 10 us, but five prompts through a small model 7.2 : 7.4 ms)."""
+    In float32: by the estimate of :func:`_f32_cost`; not under 256 keys (32 tokens at 200 keys 16.2 us uncut, 10 cut, but five prompts
+    through a small model 7.2 ms uncut, 7.4 cut, which is the host's time)."""
+    if dtype == torch.float32 and max_keys < 256:
+        return 1            # a cut gains less than the launch of the merge costs a host that is behind
     hpt = _heads_per_tile(group)
     items = max(1, n_tiles * kv_heads * ((group + hpt - 1) // hpt))
     if dtype == torch.float32:
-        runs = 2 * COMPUTE_UNITS // items
-        if hd <= 64 and 1 <= runs <= 2 and (runs + 1) * items <= 3 * COMPUTE_UNITS:
-            runs += 1
-        if runs <= 1 and items > COMPUTE_UNITS and items <= (2 if hd > 48 else 4) * COMPUTE_UNITS:
-            runs = 2
-        return int(max(1, min(runs, max_keys // 32 if max_keys >= 256 else 1, 16)))
+        return _f32_runs(items, n_tiles * _f32_tile_tokens(hd, group), -(-int(max_keys) // 32) * 32, hd)
     many = min(1024 // items if items < 2 * COMPUTE_UNITS else 1, max_keys // 2048)
     few = min(COMPUTE_UNITS // items, max_keys // 512)
     return int(max(1, min(max(many, few), 16)))
@@ -499,7 +540,8 @@ def mfma_attention(qkv: torch.Tensor, kpool: torch.Tensor, vpool: torch.Tensor, 
         _check(attention_mfma_f32_lib(hd).ni_mfma_attention_f32(
             _ptr(qkv), qkv.shape[1], _ptr(kpool), _ptr(vpool), _ptr(block_table), block_table.shape[1], _ptr(tiles),
             tiles.shape[0], _ptr(out), _ptr(part_o), _ptr(part_ml), H, KVH, kpool.shape[2],
-            int(window) if window else 0, ctypes.c_float(scale), nsplit, _stream()), "mfma_attention (float32)")
+            int(window) if window else 0, ctypes.c_float(scale), nsplit, _f32_blocks(tiles.shape[0], KVH, H // KVH, nsplit, hd), _stream()),
+            "mfma_attention (float32)")
     else:
         _check(attention_mfma_lib(hd).ni_mfma_attention(
             _ptr(qkv), qkv.shape[1], _ptr(kpool), _ptr(vpool), _ptr(block_table), block_table.shape[1], _ptr(tiles),
