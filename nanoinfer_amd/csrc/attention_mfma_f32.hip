@@ -271,17 +271,6 @@ __device__ __forceinline__ void exact_tile(const TileArgs& a, const QTile& tile,
     }
 }
 
-// The exponential of a score less its reference (at most REF_SLACK), as exact as expf: the hardware's power of two (one
-// unit in the last place) with the rounding of its argument made good.  Minus infinity and what lies below the smallest
-// number give zero, NaN stays NaN.
-__device__ __forceinline__ float weight_of(float t) {
-    t = t < -110.f ? -110.f : t;
-    const float hi = t * 1.44269502f;
-    const float lo = fmaf(t, 1.92596299e-8f, fmaf(t, 1.44269502f, -hi));
-    const float e = __builtin_amdgcn_exp2f(hi);
-    return fmaf(e, lo * 0.693147182f, e);
-}
-
 // Eight float32 numbers as three times eight bfloat16 numbers that add up to them.
 struct Parts { uint4 p[3]; };
 __device__ __forceinline__ Parts parts8(const float* v) {
@@ -527,7 +516,7 @@ __device__ __forceinline__ bool parts_tile(const TileArgs& a, const QTile& tile,
                     float w[8];
 #pragma unroll
                     for (int j = 0; j < 8; ++j) {
-                        w[j] = weight_of(sc[j] - m_ref[c]);
+                        w[j] = exp_below(sc[j] - m_ref[c]);
                         if (!inner[c]) w[j] = sc[j] > 0.5f * NEG_BIG ? w[j] : 0.f;
                         l_lane[c] += w[j];
                     }

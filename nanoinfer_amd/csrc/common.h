@@ -265,6 +265,17 @@ __device__ __forceinline__ int token_by_length(const int32_t* __restrict__ posit
 #define RANKED_GROUPS 512
 #define RANKED_TOKENS 256
 
+// e^t for t that is hardly above zero (a score less its reference, a difference of logarithms), as exact as expf in two thirds of its
+// instructions: the hardware's power of two (one unit in the last place) with the rounding of its argument made good.  Minus
+// infinity and what lies below the smallest number give zero, NaN stays NaN.
+__device__ __forceinline__ float exp_below(float t) {
+    t = t < -110.f ? -110.f : t;
+    const float hi = t * 1.44269502f;
+    const float lo = fmaf(t, 1.92596299e-8f, fmaf(t, 1.44269502f, -hi));
+    const float e = __builtin_amdgcn_exp2f(hi);
+    return fmaf(e, lo * 0.693147182f, e);
+}
+
 // The bounds of hidden units.  NaN passes them (fmaxf and fminf would make it the bound: a number out of none).
 __device__ __forceinline__ float at_least(float v, float low) { return v < low ? low : v; }
 __device__ __forceinline__ float at_most(float v, float high) { return v > high ? high : v; }

@@ -52,8 +52,8 @@ __device__ __forceinline__ float softplus_f(float z) { return z > 20.f ? z : log
 // conv float32 [C, taps] with C = 2*G*dk + H*dv (the filters of q, k, v stacked).
 // state float32 [slots, state_stride]; the convolutions' inputs lie at conv_off as [taps - 1, C].
 // prep float32 [T, prep_cols]: q | k | v | beta [H] | g [H*dk] | gate [H*dv].
-// One workgroup a (token, unit): units 0 .. 2G-1 are the heads of q and of k (convolution, silu, unit norm),
-// units 2G .. 2G+H-1 the heads of v with that head's beta, decay and gate.
+// Units 0 .. 2G-1 are the heads of q and of k (convolution, silu, unit norm), units 2G .. 2G+H-1 the heads of v with that head's
+// beta, decay and gate.
 __device__ __forceinline__ float conv_at(const float* __restrict__ proj, const float* __restrict__ hist,
                                          const float* __restrict__ conv, int t, int i, int c, int C, int taps, int proj_cols) {
     float acc = 0.f;
@@ -66,58 +66,143 @@ __device__ __forceinline__ float conv_at(const float* __restrict__ proj, const f
     return acc;
 }
 
-__global__ void delta_prepare_kernel(const float* __restrict__ proj, const float* __restrict__ low,
+// One wavefront a unit of TOK tokens: nothing meets in LDS, and four tokens of a sequence read the rows that their filters share
+// once, all asked for together.  1,500 tokens of 16 heads of 128 (123 MB) took 65 us with a workgroup a token and unit, 43 now.
+template <int TOK>
+__global__ __launch_bounds__(256) void delta_prepare_kernel(const float* __restrict__ proj, const float* __restrict__ low,
                                      const float* __restrict__ conv, const float* __restrict__ a_log,
                                      const float* __restrict__ dt_bias, float* __restrict__ state,
                                      const int32_t* __restrict__ seq_of_token, const int32_t* __restrict__ q_start,
                                      const int32_t* __restrict__ state_slot, float* __restrict__ prep,
-                                     int G, int H, int dk, int dv, int taps, int proj_cols, size_t state_stride,
+                                     int T, int G, int H, int dk, int dv, int taps, int proj_cols, size_t state_stride,
                                      size_t conv_off, int log_decay, int move_on) {
-    __shared__ float scratch[16];
-    const int t = blockIdx.x, unit = blockIdx.y;
-    const int s = seq_of_token[t];
-    const int i = t - q_start[s];              // place of the token in its portion
+    const int lane = threadIdx.x & (WAVE - 1), unit = blockIdx.y;
     const int QK = 2 * G * dk, C = QK + H * dv;
     const int prep_cols = C + H + H * dk + H * dv;
-    float* hist = state + static_cast<size_t>(state_slot[s]) * state_stride + conv_off;
-    float* out = prep + static_cast<size_t>(t) * prep_cols;
-    // move_on: every sequence of the step brings one token, so the thread that has read a channel's last inputs is the
-    // only one that does, and moves them on itself (no kernel of its own for that)
-    auto moved = [&](int c) {
-        for (int j = 0; j + 2 < taps; ++j) hist[static_cast<size_t>(j) * C + c] = hist[static_cast<size_t>(j + 1) * C + c];
-        hist[static_cast<size_t>(taps - 2) * C + c] = proj[static_cast<size_t>(t) * proj_cols + c];
-    };
-    if (unit < 2 * G) {
-        // a head of q or of k: every thread keeps its channels (dk <= 256 = threads)
-        const int c = unit * dk + threadIdx.x;
-        float y = 0.f;
-        if (threadIdx.x < dk) {
-            const float z = conv_at(proj, hist, conv, t, i, c, C, taps, proj_cols);
-            y = z * (1.0f / (1.0f + expf(-z)));
-            if (move_on && taps > 1) moved(c);
+    const int first = (blockIdx.x * 4 + threadIdx.x / WAVE) * TOK;
+    if constexpr (TOK == 4) {
+        // four tokens of one sequence behind its first three, filters of four: the seven rows that they need, all asked for at once
+        if (first + 3 < T && taps == 4) {
+            const int s = __builtin_amdgcn_readfirstlane(seq_of_token[first]);
+            if (s == __builtin_amdgcn_readfirstlane(seq_of_token[first + 3]) && first - q_start[s] >= 3) {
+                const float* rows = proj + static_cast<size_t>(first) * proj_cols;
+                float* to = prep + static_cast<size_t>(first) * prep_cols;
+                const bool value = unit >= 2 * G;
+                const int h = unit - 2 * G, width = value ? dv : dk, c0 = value ? QK + h * dv : unit * dk;
+                auto filtered = [&](int c, float (&y)[4]) {
+                    float x[7], w[4];
+#pragma unroll
+                    for (int b = 0; b < 7; ++b) x[b] = rows[static_cast<ptrdiff_t>(b - 3) * proj_cols + c];
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) w[b] = conv[static_cast<size_t>(c) * 4 + b];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        float acc = 0.f;
+#pragma unroll
+                        for (int b = 0; b < 4; ++b) acc += w[b] * x[j + b];
+                        y[j] = silu_f(acc);
+                    }
+                };
+                if (!value) {
+                    float y[4][4], ss[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) {
+                        if (b * WAVE >= dk) break;
+                        const int at = lane + b * WAVE;
+                        filtered(c0 + min(at, dk - 1), y[b]);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) ss[j] += at < dk ? y[b][j] * y[b][j] : 0.f;
+                    }
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        ss[j] = (1.0f / sqrtf(wave_sum(ss[j]) + 1e-6f)) * (unit < G ? 1.0f / sqrtf(static_cast<float>(dk)) : 1.0f);
+#pragma unroll
+                    for (int b = 0; b < 4; ++b)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            if (lane + b * WAVE < dk) to[static_cast<size_t>(j) * prep_cols + c0 + lane + b * WAVE] = y[b][j] * ss[j];
+                    return;
+                }
+                const int wide = H * dk + H * dv;
+                const float* lows = low + static_cast<size_t>(first) * wide;
+                for (int at = lane; at < width; at += WAVE) {
+                    float y[4], gate[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) gate[j] = lows[static_cast<size_t>(j) * wide + H * dk + h * dv + at];
+                    filtered(c0 + at, y);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        to[static_cast<size_t>(j) * prep_cols + c0 + at] = y[j];
+                        to[static_cast<size_t>(j) * prep_cols + C + H + H * dk + h * dv + at] = sigmoid_f(gate[j]);
+                    }
+                }
+                const float rate = expf(a_log[h]);
+                for (int at = lane; at < dk; at += WAVE) {
+                    float z[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) z[j] = lows[static_cast<size_t>(j) * wide + h * dk + at];
+                    const float bias = dt_bias[h * dk + at];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const float lg = -rate * softplus_f(z[j] + bias);
+                        to[static_cast<size_t>(j) * prep_cols + C + H + h * dk + at] = log_decay ? lg : expf(lg);
+                    }
+                }
+                if (lane < 4) to[static_cast<size_t>(lane) * prep_cols + C + h] = sigmoid_f(rows[static_cast<size_t>(lane) * proj_cols + C + h]);
+                return;
+            }
         }
-        const float ss = block_sum(y * y, scratch);
-        const float inv = (1.0f / sqrtf(ss + 1e-6f)) * (unit < G ? 1.0f / sqrtf(static_cast<float>(dk)) : 1.0f);
-        if (threadIdx.x < dk) out[c] = y * inv;
-        return;
     }
-    const int h = unit - 2 * G;
-    const float* prow = proj + static_cast<size_t>(t) * proj_cols;
-    const float* lrow = low + static_cast<size_t>(t) * (H * dk + H * dv);
-    for (int j = threadIdx.x; j < dv; j += blockDim.x) {
-        const int c = QK + h * dv + j;
-        const float z = conv_at(proj, hist, conv, t, i, c, C, taps, proj_cols);
-        out[c] = z * (1.0f / (1.0f + expf(-z)));
-        if (move_on && taps > 1) moved(c);
-        out[C + H + H * dk + h * dv + j] = 1.0f / (1.0f + expf(-lrow[H * dk + h * dv + j]));
+    for (int j = 0; j < TOK; ++j) {
+        const int t = first + j;
+        if (t >= T) return;
+        const int s = seq_of_token[t];
+        const int i = t - q_start[s];              // place of the token in its portion
+        float* hist = state + static_cast<size_t>(state_slot[s]) * state_stride + conv_off;
+        float* out = prep + static_cast<size_t>(t) * prep_cols;
+        // move_on: every sequence of the step brings one token, so the lane that has read a channel's last inputs is the
+        // only one that does, and moves them on itself (no kernel of its own for that)
+        auto moved = [&](int c) {
+            for (int b = 0; b + 2 < taps; ++b) hist[static_cast<size_t>(b) * C + c] = hist[static_cast<size_t>(b + 1) * C + c];
+            hist[static_cast<size_t>(taps - 2) * C + c] = proj[static_cast<size_t>(t) * proj_cols + c];
+        };
+        if (unit < 2 * G) {
+            // a head of q or of k: every lane keeps its channels (dk <= 256)
+            float y[4], ss = 0.f;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const int at = lane + b * WAVE;
+                y[b] = 0.f;
+                if (at < dk) {
+                    const int c = unit * dk + at;
+                    y[b] = silu_f(conv_at(proj, hist, conv, t, i, c, C, taps, proj_cols));
+                    if (move_on && taps > 1) moved(c);
+                }
+                ss += y[b] * y[b];
+            }
+            ss = wave_sum(ss);
+            const float inv = (1.0f / sqrtf(ss + 1e-6f)) * (unit < G ? 1.0f / sqrtf(static_cast<float>(dk)) : 1.0f);
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+                if (lane + b * WAVE < dk) out[unit * dk + lane + b * WAVE] = y[b] * inv;
+            continue;
+        }
+        const int h = unit - 2 * G;
+        const float* prow = proj + static_cast<size_t>(t) * proj_cols;
+        const float* lrow = low + static_cast<size_t>(t) * (H * dk + H * dv);
+        for (int at = lane; at < dv; at += WAVE) {
+            const int c = QK + h * dv + at;
+            out[c] = silu_f(conv_at(proj, hist, conv, t, i, c, C, taps, proj_cols));
+            if (move_on && taps > 1) moved(c);
+            out[C + H + H * dk + h * dv + at] = sigmoid_f(lrow[H * dk + h * dv + at]);
+        }
+        const float rate = expf(a_log[h]);
+        for (int at = lane; at < dk; at += WAVE) {
+            const float lg = -rate * softplus_f(lrow[h * dk + at] + dt_bias[h * dk + at]);
+            out[C + H + h * dk + at] = log_decay ? lg : expf(lg);      // the chunked form sums logarithms
+        }
+        if (lane == 0) out[C + h] = sigmoid_f(prow[C + h]);
     }
-    const float rate = expf(a_log[h]);
-    for (int j = threadIdx.x; j < dk; j += blockDim.x) {
-        const float z = lrow[h * dk + j] + dt_bias[h * dk + j];
-        const float lg = -rate * (z > 20.f ? z : log1pf(expf(z)));
-        out[C + H + h * dk + j] = log_decay ? lg : expf(lg);      // the chunked form sums logarithms
-    }
-    if (threadIdx.x == 0) out[C + h] = 1.0f / (1.0f + expf(-prow[C + h]));
 }
 
 __global__ void conv_state_update_kernel(const float* __restrict__ proj, float* __restrict__ state,
@@ -240,10 +325,10 @@ delta_rule_kernel(const float* __restrict__ prep, float* __restrict__ state, con
 //     o_t = S0^T (e^{L_t} q_t) + sum_{s<=t} P_ts u_s,                        P_ts = sum_c q_t[c] k_s[c] e^{L_t[c] - L_s[c]}
 //     S_C = diag(e^{L_C}) S0 + sum_s (e^{L_C - L_s} k_s) u_s^T
 // Every exponent is a difference that is at most zero: nothing is divided by a decay, however small it gets.
-// A, P, the inverse Tm = (I + diag(beta) tril(A, -1))^-1 diag(beta) and the three scaled copies of k and q do not
-// depend on the memory: delta_chunk_prepare makes them for all runs of the step at once.  What is left for the
-// chain from run to run is five small matrix products,
-//     W = V - Kt S0;  U = Tm W;  O = Qt S0 + P U;  S <- diag(e^{L_C}) S0 + Kb^T U,
+// A, P, the inverse Tm = (I + diag(beta) tril(A, -1))^-1 diag(beta), its products with V and with Kt (the rows e^{L_t} k_t), and the
+// scaled copies of k and q do not depend on the memory: delta_chunk_prepare makes them for all runs of the step at once.  What is
+// left for the chain from run to run is
+//     U = Tm V - (Tm Kt) S0;  O = Qt S0 + P U;  S <- diag(e^{L_C}) S0 + Kb^T U,
 // which delta_chunk_scan does with v_mfma_f32_16x16x4_f32 (true 32-bit products and sums), one workgroup a
 // (sequence, head, sixteen value channels) with its [DK, 16] piece of S in the accumulators' layout for the whole
 // step.  A lane of that layout holds channels 4 (lane / 16) + r, r = 0..3, of each sixteen; as the second operand
@@ -254,13 +339,21 @@ delta_rule_kernel(const float* __restrict__ prep, float* __restrict__ state, con
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
 constexpr int RUN = 16;
 
-__host__ __device__ constexpr int chunk_floats(int dk) { return 3 * RUN * dk + 2 * RUN * RUN + dk; }
+// What is prepared for a run of tokens and a head, by place (floats): Tm Kt and Qt as [token][channel], Kb as [channel][token], P as
+// [token][token], e^{L_C}, and Tm V as [value channel][token], the channels filled up to sixteens.
+template <int DK> struct RunPlaces {
+    static constexpr int tk = 0, qt = RUN * DK, kb = 2 * RUN * DK, p = 3 * RUN * DK, dec = p + RUN * RUN, tv = dec + DK;
+};
+__host__ __device__ constexpr int chunk_floats(int dk, int dv) { return 3 * RUN * dk + RUN * RUN + dk + RUN * ((dv + RUN - 1) / RUN * RUN); }
 
 __global__ void __launch_bounds__(256)
 delta_chunk_prepare_kernel(const float* __restrict__ prep, float* __restrict__ chunks, const int32_t* __restrict__ q_start,
                            const int32_t* __restrict__ q_len, int G, int H, int dv) {
-    constexpr int DK = KPT * PARTS, LD = DK + 1;
-    __shared__ float Ls[RUN * LD], ks[RUN * LD], qs[RUN * LD], As[RUN * (RUN + 1)], betas[RUN];
+    constexpr int DK = KPT * PARTS, LD = DK + 4;
+    using At = RunPlaces<DK>;
+    __shared__ __attribute__((aligned(16))) float Ls[RUN * LD], ks[RUN * LD], qs[RUN * LD];
+    __shared__ float As[RUN * (RUN + 1)], betas[RUN];
+    __shared__ __attribute__((aligned(16))) float Tm[RUN * RUN];
     const int s = blockIdx.x, h = blockIdx.z;
     const int n = q_len[s], first = q_start[s];
     const int t0 = blockIdx.y * RUN;
@@ -269,7 +362,7 @@ delta_chunk_prepare_kernel(const float* __restrict__ prep, float* __restrict__ c
     const int QK = 2 * G * DK, C = QK + H * dv;
     const int prep_cols = C + H + H * DK + H * dv;
     const size_t slot = static_cast<size_t>(first / RUN + s + blockIdx.y);
-    float* out = chunks + (slot * H + h) * chunk_floats(DK);
+    float* out = chunks + (slot * H + h) * chunk_floats(DK, dv);
     const float* rows = prep + static_cast<size_t>(first + t0) * prep_cols;
     for (int e = threadIdx.x; e < RUN * DK; e += 256) {
         const int t = e / DK, c = e % DK;
@@ -289,29 +382,50 @@ delta_chunk_prepare_kernel(const float* __restrict__ prep, float* __restrict__ c
         }
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < RUN * DK; e += 256) {
-        const int t = e / DK, c = e % DK;
-        const float lt = Ls[t * LD + c], lc = Ls[(RUN - 1) * LD + c];
-        const float grow = expf(lt);
-        out[e] = grow * ks[t * LD + c];
-        out[RUN * DK + e] = grow * qs[t * LD + c];
-        out[2 * RUN * DK + e] = expf(lc - lt) * ks[t * LD + c];
-        if (t == RUN - 1) out[3 * RUN * DK + 2 * RUN * RUN + c] = grow;
-    }
+    // A and P: two neighbouring threads a pair j < t, half of the channels each; the last sixteen threads the diagonal of P
     {
-        const int t = threadIdx.x / RUN, j = threadIdx.x % RUN;
         float a = 0.f, p = 0.f;
-        if (j <= t) {
-            for (int c = 0; c < DK; ++c) {
-                const float w = expf(Ls[t * LD + c] - Ls[j * LD + c]) * ks[j * LD + c];
-                a += ks[t * LD + c] * w;
-                p += qs[t * LD + c] * w;
+        int t, j;
+        if (threadIdx.x < RUN * (RUN - 1)) {
+            const int pair = threadIdx.x / 2;
+            t = static_cast<int>((sqrtf(8.f * pair + 1.f) + 1.f) * 0.5f);       // pairs t (t - 1) / 2 .. are those of t
+            t -= t * (t - 1) / 2 > pair;
+            t += t * (t + 1) / 2 <= pair;
+            j = pair - t * (t - 1) / 2;
+            constexpr int HALF = DK / 2;
+            const float *lt = Ls + t * LD, *lj = Ls + j * LD, *kt = ks + t * LD, *kj = ks + j * LD, *qt = qs + t * LD;
+            for (int c = (threadIdx.x & 1) * HALF; c < ((threadIdx.x & 1) + 1) * HALF; c += 4) {
+                const float4 l0 = *reinterpret_cast<const float4*>(lt + c), l1 = *reinterpret_cast<const float4*>(lj + c);
+                const float4 k0 = *reinterpret_cast<const float4*>(kt + c), k1 = *reinterpret_cast<const float4*>(kj + c);
+                const float4 q0 = *reinterpret_cast<const float4*>(qt + c);
+                const float w[4] = {exp_below(l0.x - l1.x) * k1.x, exp_below(l0.y - l1.y) * k1.y, exp_below(l0.z - l1.z) * k1.z, exp_below(l0.w - l1.w) * k1.w};
+                a += k0.x * w[0]; a += k0.y * w[1]; a += k0.z * w[2]; a += k0.w * w[3];
+                p += q0.x * w[0]; p += q0.y * w[1]; p += q0.z * w[2]; p += q0.w * w[3];
             }
+            a += __shfl_xor(a, 1, WAVE);
+            p += __shfl_xor(p, 1, WAVE);
+            if ((threadIdx.x & 1) == 0) {
+                As[t * (RUN + 1) + j] = a;
+                out[At::p + t * RUN + j] = p;
+                out[At::p + j * RUN + t] = 0.f;
+            }
+        } else {
+            t = threadIdx.x - RUN * (RUN - 1);
+            for (int c = 0; c < DK; ++c) p += qs[t * LD + c] * ks[t * LD + c];
+            out[At::p + t * RUN + t] = p;
         }
-        As[t * (RUN + 1) + j] = j < t ? a : 0.f;
-        out[3 * RUN * DK + RUN * RUN + t * RUN + j] = j <= t ? p : 0.f;
     }
     __syncthreads();
+    // the scaled copies; what Kt needs stays where k was
+    for (int e = threadIdx.x; e < RUN * DK; e += 256) {
+        const int t = e / DK, c = e % DK;
+        const float lt = Ls[t * LD + c], lc = Ls[(RUN - 1) * LD + c], k = ks[t * LD + c];
+        const float grow = exp_below(lt);
+        out[At::qt + e] = grow * qs[t * LD + c];
+        ks[t * LD + c] = grow * k;
+        qs[t * LD + c] = exp_below(lc - lt) * k;
+        if (t == RUN - 1) out[At::dec + c] = grow;
+    }
     if (threadIdx.x < RUN) {
         // column j of (I + diag(beta) tril(A, -1))^-1 diag(beta), from the top down
         const int j = threadIdx.x;
@@ -324,31 +438,62 @@ delta_chunk_prepare_kernel(const float* __restrict__ prep, float* __restrict__ c
             x[t] = (t == j ? betas[j] : 0.f) - betas[t] * acc;
         }
 #pragma unroll
-        for (int t = 0; t < RUN; ++t) out[3 * RUN * DK + t * RUN + j] = x[t];
+        for (int t = 0; t < RUN; ++t) Tm[t * RUN + j] = x[t];
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < RUN * DK; e += 256) out[At::kb + e] = qs[e % RUN * LD + e / RUN];
+    // Tm Kt and Tm V: four tokens of a column a thread
+    const int dvp = (dv + RUN - 1) / RUN * RUN;
+    for (int e = threadIdx.x; e < 4 * (DK + dvp); e += 256) {
+        const bool key = e < 4 * DK;
+        const int part = key ? e / DK : (e - 4 * DK) / dvp, c = key ? e % DK : (e - 4 * DK) % dvp;
+        float sum[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (int r = 0; r < RUN; ++r) {
+            float x;
+            if (key) x = ks[r * LD + c];
+            else x = c < dv && t0 + r < n ? rows[static_cast<size_t>(r) * prep_cols + QK + h * dv + c] : 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sum[i] += Tm[(4 * part + i) * RUN + r] * x;
+        }
+        if (key) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) out[At::tk + (4 * part + i) * DK + c] = sum[i];
+        } else {
+            *reinterpret_cast<float4*>(out + At::tv + c * RUN + 4 * part) = make_float4(sum[0], sum[1], sum[2], sum[3]);
+        }
     }
 }
 
-// What a wavefront reads for one run of tokens: all of it is asked for one run ahead.
-template <int KTW> struct RunOperands {
-    float4 kt[KTW], qt[KTW], dec[KTW];   // rows (lane % 16) of Kt and Qt, channels 16 kt + 4 (lane / 16) + r; e^{L_C} of these
-    float kb[KTW][4];                    // Kb of token 4 (lane / 16) + r, channel 16 kt + lane % 16
-    float4 tm, p;                        // row (lane % 16) of Tm and of P, columns 4 (lane / 16) + r
-    floatx4_t v;                         // v of token 4 (lane / 16) + r, the lane's value channel
-};
-
 // The key channels of a (head, sixteen value channels) are dealt to SCAN_WAVES wavefronts, sixteen at a time: each
-// keeps its channels' rows of S and makes its share of Kt S0 and Qt S0.  The shares meet in LDS once a run (two
+// keeps its channels' rows of S and makes its share of (Tm Kt) S0 and Qt S0.  The shares of U meet in LDS once a run (two
 // buffers in turn, so one barrier a run is enough: a wavefront can be one run ahead of another, never two); every
-// wavefront then sums them in the same order, so all hold the same W and U, and moves its own rows of S on.
+// wavefront then sums them in the same order, so all hold the same U, and moves its own rows of S on.  The shares of O, with
+// a share of P U each, meet at the barrier of the run behind.
+//
+// What bounds it is the chain from run to run (128 workgroups for one prompt through 16 heads of 128 value channels): the
+// products with S, the meeting in LDS and the update of S.  So nothing else stands in it: Tm is multiplied in beforehand, sums
+// over channels go in two chains, the read-out fills the wait for the meeting, and the operands are asked for AHEAD runs
+// before their turn (they come from beyond the L2 of most XCDs, which takes longer than a run).  1,500 tokens of 16 heads
+// of 128 by 128 channels 145 -> 96 us (with operands at hand it takes 70, of which 25 matrix instructions a run are 31), while
+// delta_chunk_prepare, which has Tm's products to make now and does half as many exponentials, takes 45 -> 48.
 constexpr int scan_waves(int kt) { return kt % 4 == 0 ? 4 : kt % 2 == 0 ? 2 : 1; }
 
-__global__ void __launch_bounds__(64 * scan_waves(KPT * PARTS / RUN > 0 ? KPT * PARTS / RUN : 1))
-delta_chunk_scan_kernel(const float* __restrict__ prep, const float* __restrict__ chunks, float* __restrict__ state,
-                        const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len,
-                        const int32_t* __restrict__ state_slot, float* __restrict__ o, int G, int H, int dv,
+template <int KTW, int MINE> struct RunOperands {
+    floatx4_t tk[KTW], qt[KTW], kb[KTW], dec[KTW];   // rows (lane % 16) of Tm Kt and Qt, channels 16 kt + 4 (lane / 16) + r; Kb of channel
+                                                     // 16 kt + lane % 16, tokens 4 (lane / 16) + r; e^{L_C} of the lane's channels of S
+    floatx4_t tv;                                    // Tm V of tokens 4 (lane / 16) + r, the lane's value channel
+    float p[MINE];                                   // row (lane % 16) of P, columns 4 (lane / 16) + wave + waves * j
+};
+
+__global__ void __launch_bounds__(64 * scan_waves(KPT * PARTS / RUN > 0 ? KPT * PARTS / RUN : 1)) __attribute__((amdgpu_waves_per_eu(2)))
+delta_chunk_scan_kernel(const float* __restrict__ chunks, float* __restrict__ state, const int32_t* __restrict__ q_start,
+                        const int32_t* __restrict__ q_len, const int32_t* __restrict__ state_slot, float* __restrict__ o, int H, int dv,
                         size_t state_stride) {
-    constexpr int DK = KPT * PARTS, KT = DK / RUN > 0 ? DK / RUN : 1, SW = scan_waves(KT), KTW = KT / SW;
-    __shared__ float shares[2][SW][2][4][WAVE];
+    constexpr int DK = KPT * PARTS, KT = DK / RUN > 0 ? DK / RUN : 1, SW = scan_waves(KT), KTW = KT / SW, MINE = 4 / SW;
+    constexpr int AHEAD = KTW <= 2 ? 3 : 2;
+    using At = RunPlaces<DK>;
+    __shared__ floatx4_t ushare[2][SW][WAVE], oshare[2][SW][WAVE];
     const int s = blockIdx.x, h = blockIdx.y;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
     const int i = lane & 15, g4 = lane >> 4;
@@ -356,8 +501,6 @@ delta_chunk_scan_kernel(const float* __restrict__ prep, const float* __restrict_
     const bool live = col < dv;
     const int n = q_len[s], first = q_start[s];
     if (n <= 0) return;
-    const int QK = 2 * G * DK, C = QK + H * dv;
-    const int prep_cols = C + H + H * DK + H * dv;
     const int ch0 = wave * KTW * RUN;                  // the wavefront's first key channel
     float* S_mem = state + static_cast<size_t>(state_slot[s]) * state_stride + (static_cast<size_t>(h) * dv + (live ? col : 0)) * DK + ch0 + 4 * g4;
     floatx4_t S[KTW];
@@ -365,91 +508,97 @@ delta_chunk_scan_kernel(const float* __restrict__ prep, const float* __restrict_
     for (int kt = 0; kt < KTW; ++kt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) S[kt][r] = live ? S_mem[kt * RUN + r] : 0.f;
-    const float* base = chunks + (static_cast<size_t>(first / RUN + s) * H + h) * chunk_floats(DK);
-    const size_t per_run = static_cast<size_t>(H) * chunk_floats(DK);
-    const float* vcol = prep + static_cast<size_t>(first) * prep_cols + QK + h * dv + (live ? col : 0);
-
-    auto fetch = [&](RunOperands<KTW>& x, int run) {
-        const float* ch = base + per_run * run;
-        const int t0 = run * RUN;
+    const char* base = reinterpret_cast<const char*>(chunks + (static_cast<size_t>(first / RUN + s) * H + h) * chunk_floats(DK, dv));
+    const size_t per_run = static_cast<size_t>(H) * chunk_floats(DK, dv) * 4;
+    // bytes from a run's beginning, the lane's part in 32 bits
+    const uint32_t by_token = (i * DK + ch0 + 4 * g4) * 4, by_channel = ((ch0 + i) * RUN + 4 * g4) * 4, mine = (ch0 + 4 * g4) * 4;
+    const uint32_t by_value = (col * RUN + 4 * g4) * 4, by_p = (i * RUN + 4 * g4) * 4;
+    using Operands = RunOperands<KTW, MINE>;
+    auto fetch = [&](Operands& x, int run) {
+        const char* ch = base + per_run * run;
+        auto load = [&](int place, uint32_t lane_part, int more) { return *reinterpret_cast<const floatx4_t*>(ch + place * 4 + lane_part + more); };
 #pragma unroll
         for (int kt = 0; kt < KTW; ++kt) {
-            const int c = ch0 + kt * RUN;
-            x.kt[kt] = *reinterpret_cast<const float4*>(ch + i * DK + c + 4 * g4);
-            x.qt[kt] = *reinterpret_cast<const float4*>(ch + RUN * DK + i * DK + c + 4 * g4);
-            x.dec[kt] = *reinterpret_cast<const float4*>(ch + 3 * RUN * DK + 2 * RUN * RUN + c + 4 * g4);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) x.kb[kt][r] = ch[2 * RUN * DK + (4 * g4 + r) * DK + c + i];
+            x.tk[kt] = load(At::tk, by_token, kt * RUN * 4);
+            x.qt[kt] = load(At::qt, by_token, kt * RUN * 4);
+            x.kb[kt] = load(At::kb, by_channel, kt * RUN * RUN * 4);
+            x.dec[kt] = load(At::dec, mine, kt * RUN * 4);
         }
-        x.tm = *reinterpret_cast<const float4*>(ch + 3 * RUN * DK + i * RUN + 4 * g4);
-        x.p = *reinterpret_cast<const float4*>(ch + 3 * RUN * DK + RUN * RUN + i * RUN + 4 * g4);
+        x.tv = load(At::tv, by_value, 0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int tok = t0 + 4 * g4 + r;
-            x.v[r] = (live && tok < n) ? vcol[static_cast<size_t>(tok) * prep_cols] : 0.f;
+        for (int j = 0; j < MINE; ++j) x.p[j] = *reinterpret_cast<const float*>(ch + (At::p + wave + SW * j) * 4 + by_p);
+    };
+    // the shares of a run's read-out, once all wavefronts have left them; a wavefront stores the tokens 4 (lane / 16) + r with r its own
+    char* out = reinterpret_cast<char*>(o + static_cast<size_t>(first) * (H * dv) + h * dv);
+    const uint32_t by_out = (4 * g4 * H * dv + col) * 4;
+    auto read_out = [&](int run) {
+#pragma unroll
+        for (int j = 0; j < MINE; ++j) {
+            const int r = wave + SW * j, tok = run * RUN + 4 * g4 + r;
+            float val = 0.f;
+#pragma unroll
+            for (int w = 0; w < SW; ++w) val += reinterpret_cast<const float*>(&oshare[run & 1][w][lane])[r];
+            if (live && tok < n) *reinterpret_cast<float*>(out + static_cast<size_t>(run * RUN + r) * (H * dv) * 4 + by_out) = val;
         }
     };
-    auto at = [](const float4& f, int r) { return r == 0 ? f.x : r == 1 ? f.y : r == 2 ? f.z : f.w; };
-
     const int runs = (n + RUN - 1) / RUN;
-    RunOperands<KTW> cur, nxt;
-    fetch(cur, 0);
-    for (int run = 0; run < runs; ++run) {
-        if (run + 1 < runs) fetch(nxt, run + 1);
-        floatx4_t w = {0.f, 0.f, 0.f, 0.f}, out = {0.f, 0.f, 0.f, 0.f};
+    Operands ops[AHEAD];
 #pragma unroll
-        for (int kt = 0; kt < KTW; ++kt)
+    for (int j = 0; j < AHEAD; ++j) fetch(ops[j], min(j, runs - 1));
+    auto step = [&](Operands& x, int run) {
+        floatx4_t ua = {0.f, 0.f, 0.f, 0.f}, ub = {0.f, 0.f, 0.f, 0.f}, oa = ua, ob = ua;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                w = __builtin_amdgcn_mfma_f32_16x16x4f32(at(cur.kt[kt], r), S[kt][r], w, 0, 0, 0);
-                out = __builtin_amdgcn_mfma_f32_16x16x4f32(at(cur.qt[kt], r), S[kt][r], out, 0, 0, 0);
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int kt = 0; kt < KTW; ++kt) {
+                floatx4_t& to = kt & 1 ? ub : ua;
+                to = __builtin_amdgcn_mfma_f32_16x16x4f32(x.tk[kt][r], S[kt][r], to, 0, 0, 0);
             }
-        float (*mine)[2][4][WAVE] = shares[run & 1];
-        if constexpr (SW > 1) {
+        ushare[run & 1][wave][lane] = ua + ub;
+        __syncthreads();
+        floatx4_t theirs[SW];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                mine[wave][0][r][lane] = w[r];
-                mine[wave][1][r][lane] = out[r];
+        for (int w = 0; w < SW; ++w) theirs[w] = ushare[run & 1][w][lane];
+        __builtin_amdgcn_sched_barrier(0);
+        // (the wait for them is filled with the read-out from S)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int kt = 0; kt < KTW; ++kt) {
+                floatx4_t& to = kt & 1 ? ob : oa;
+                to = __builtin_amdgcn_mfma_f32_16x16x4f32(x.qt[kt][r], S[kt][r], to, 0, 0, 0);
             }
-            __syncthreads();
+        floatx4_t u = theirs[0];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                float sum = mine[0][0][r][lane];
+        for (int w = 1; w < SW; ++w) u += theirs[w];
+        u = x.tv - u;
 #pragma unroll
-                for (int j = 1; j < SW; ++j) sum += mine[j][0][r][lane];
-                w[r] = sum;
-            }
+        for (int kt = 0; kt < KTW; ++kt) S[kt] *= x.dec[kt];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int kt = 0; kt < KTW; ++kt) S[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.kb[kt][r], u[r], S[kt], 0, 0, 0);
+        if (run > 0) read_out(run - 1);
+#pragma unroll
+        for (int j = 0; j < MINE; ++j) {
+            float mine = u[SW * j];
+#pragma unroll
+            for (int w = 1; w < SW; ++w) mine = wave == w ? u[w + SW * j] : mine;
+            oa = __builtin_amdgcn_mfma_f32_16x16x4f32(x.p[j], mine, oa, 0, 0, 0);
         }
-        w = cur.v - w;
-        floatx4_t u = {0.f, 0.f, 0.f, 0.f};
+        oshare[run & 1][wave][lane] = oa + ob;
+        fetch(x, min(run + AHEAD, runs - 1));
+    };
+    int run = 0;
+    for (; run + AHEAD <= runs; run += AHEAD) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) u = __builtin_amdgcn_mfma_f32_16x16x4f32(at(cur.tm, r), w[r], u, 0, 0, 0);
-#pragma unroll
-        for (int kt = 0; kt < KTW; ++kt) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) S[kt][r] *= at(cur.dec[kt], r);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) S[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.kb[kt][r], u[r], S[kt], 0, 0, 0);
-        }
-        // the read-out: P U on top of the shares of Qt S0; a wavefront stores the tokens 4 (lane / 16) + r with r its own
-        floatx4_t pu = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int r = 0; r < 4; ++r) pu = __builtin_amdgcn_mfma_f32_16x16x4f32(at(cur.p, r), u[r], pu, 0, 0, 0);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            if (r % SW != wave) continue;
-            float val = pu[r];
-            if constexpr (SW > 1) {
-#pragma unroll
-                for (int j = 0; j < SW; ++j) val += mine[j][1][r][lane];
-            } else {
-                val += out[r];
-            }
-            const int tok = run * RUN + 4 * g4 + r;
-            if (live && tok < n) o[(static_cast<size_t>(first) + tok) * (H * dv) + h * dv + col] = val;
-        }
-        cur = nxt;
+        for (int j = 0; j < AHEAD; ++j) step(ops[j], run + j);
     }
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j)
+        if (run + j < runs) step(ops[j], run + j);
+    __syncthreads();
+    read_out(runs - 1);
     if (live) {
 #pragma unroll
         for (int kt = 0; kt < KTW; ++kt)
@@ -486,11 +635,13 @@ NI_EXPORT int ni_delta_prepare(const void* proj, const void* low, const void* co
     if (dk != KPT * PARTS) return -1;
     const int C = 2 * G * dk + H * dv;
     if (dk > 256) return -2;
-    const int widest = std::max(dk, std::min(dv, 256));
-    delta_prepare_kernel<<<dim3(T, 2 * G + H), (widest + 63) / 64 * 64, 0, stream>>>((const float*)proj, (const float*)low, (const float*)conv,
+    // a wavefront takes four tokens one after the other where that still fills the chip
+    const int tok = T >= 256 ? 4 : 1;
+    auto kernel = tok == 4 ? delta_prepare_kernel<4> : delta_prepare_kernel<1>;
+    kernel<<<dim3((T + 4 * tok - 1) / (4 * tok), 2 * G + H), 256, 0, stream>>>((const float*)proj, (const float*)low, (const float*)conv,
                                                   (const float*)a_log, (const float*)dt_bias, (float*)state,
                                                   (const int32_t*)seq_of_token, (const int32_t*)q_start,
-                                                  (const int32_t*)state_slot, (float*)prep, G, H, dk, dv, taps, proj_cols,
+                                                  (const int32_t*)state_slot, (float*)prep, T, G, H, dk, dv, taps, proj_cols,
                                                   state_stride, conv_off, log_decay, move_on);
     if (taps > 1 && !move_on) {
         dim3 grid(B, std::max(1, std::min(64, (C + 255) / 256)));
@@ -503,7 +654,7 @@ NI_EXPORT int ni_delta_prepare(const void* proj, const void* low, const void* co
 
 // floats of scratch that the chunked form needs per run of sixteen tokens and head (0: this key size has no such form);
 // a step of T tokens in B sequences has at most T / 16 + B + 1 run slots
-NI_EXPORT int ni_delta_run_floats() { return (KPT * PARTS) % RUN ? 0 : chunk_floats(KPT * PARTS); }
+NI_EXPORT int ni_delta_run_floats(int dv) { return (KPT * PARTS) % RUN ? 0 : chunk_floats(KPT * PARTS, dv); }
 
 // chunks: null for the token-by-token kernel (prep then holds the decays), else scratch for the chunked form
 // (prep then holds the decays' logarithms); max_q_len is the longest portion of the step
@@ -519,8 +670,8 @@ NI_EXPORT int ni_delta_rule(const void* prep, void* chunks, void* state, const v
             delta_chunk_prepare_kernel<<<dim3(B, runs, H), 256, 0, stream>>>((const float*)prep, (float*)chunks, (const int32_t*)q_start,
                                                                              (const int32_t*)q_len, G, H, dv);
             delta_chunk_scan_kernel<<<dim3(B, H, (dv + RUN - 1) / RUN), 64 * scan_waves(KPT * PARTS / RUN), 0, stream>>>(
-                (const float*)prep, (const float*)chunks, (float*)state, (const int32_t*)q_start, (const int32_t*)q_len,
-                (const int32_t*)state_slot, (float*)o, G, H, dv, state_stride);
+                (const float*)chunks, (float*)state, (const int32_t*)q_start, (const int32_t*)q_len, (const int32_t*)state_slot,
+                (float*)o, H, dv, state_stride);
         } else {
             return -3;
         }

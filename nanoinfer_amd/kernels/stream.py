@@ -482,7 +482,7 @@ def delta_rule(proj: torch.Tensor, low: torch.Tensor, conv: torch.Tensor, a_log:
     _need(0 <= max_q_len <= T, "max_q_len is larger than the step")
     _need(max_q_len != 1 or T == B, "a step of single tokens has one row a sequence")
     in_runs = max_q_len >= DELTA_RUN_FROM if runs is None else bool(runs)
-    run_floats = int(lib.ni_delta_run_floats()) if in_runs else 0
+    run_floats = int(lib.ni_delta_run_floats(int(dv))) if in_runs else 0
     _need(run_floats > 0 or not runs, f"the delta rule has no runs of sixteen for keys of {dk} channels")
     chunks = None
     if run_floats:
