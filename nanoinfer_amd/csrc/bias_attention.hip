@@ -719,14 +719,12 @@ __device__ __forceinline__ float groups4(float x, bool take_max) {
 // QS: 16-byte pieces of a lane's quarter of a query row at most (dk <= 64 QS); DVB: blocks of 16 value channels at most
 // (dv <= 16 DVB).  Both size arrays of registers, so the kernel is compiled for a few pairs of them.
 template <typename T, int QS, int DVB>
-__global__ void __launch_bounds__(WAVES * WAVE)
-bias_attention_mfma_kernel(const T* __restrict__ qkv, int row_stride, const T* __restrict__ kpool, const T* __restrict__ vpool,
-                           const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ tiles,
-                           const int32_t* __restrict__ positions, const float* __restrict__ bias, int distances,
-                           T* __restrict__ out, int H, int G, int dk, int dv, int page_size, float scale, float temp_coef,
-                           int temp_every, int heads_per_chunk, bool k_pieces, bool v_pieces, int window, int keep_first,
-                           float out_scale, const float* __restrict__ sink, ScoreForm form, float* __restrict__ partial, Gate gate) {
-    extern __shared__ __attribute__((aligned(16))) float lds[];
+__device__ __forceinline__ void mfma_rows(const T* __restrict__ qkv, int row_stride, const T* __restrict__ kpool, const T* __restrict__ vpool,
+                                          const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ tiles,
+                                          const int32_t* __restrict__ positions, const float* __restrict__ bias, int distances,
+                                          T* __restrict__ out, int H, int G, int dk, int dv, int page_size, float scale, float temp_coef,
+                                          int temp_every, int heads_per_chunk, bool k_pieces, bool v_pieces, int window, int keep_first,
+                                          float out_scale, const float* __restrict__ sink, ScoreForm form, float* __restrict__ partial, Gate gate, float* lds) {
     const int dkp = dk + 4, dvp = dv + 4;         // strides that spread the sixteen rows of a read over the banks
     // keys and values that are one pool (dv = dk) are staged once: the values are read from the keys' tile
     const bool one_pool = static_cast<const void*>(kpool) == static_cast<const void*>(vpool) && dk == dv;
@@ -875,6 +873,19 @@ bias_attention_mfma_kernel(const T* __restrict__ qkv, int row_stride, const T* _
                 st(orow + 16 * db + r, acc[db][r] * inv * gate.of(first_row + row / heads_here, head * dv + 16 * db + 4 * kg + r));
         }
     }
+}
+
+template <typename T, int QS, int DVB>
+__global__ void __launch_bounds__(WAVES * WAVE)
+bias_attention_mfma_kernel(const T* __restrict__ qkv, int row_stride, const T* __restrict__ kpool, const T* __restrict__ vpool,
+                           const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ tiles,
+                           const int32_t* __restrict__ positions, const float* __restrict__ bias, int distances,
+                           T* __restrict__ out, int H, int G, int dk, int dv, int page_size, float scale, float temp_coef,
+                           int temp_every, int heads_per_chunk, bool k_pieces, bool v_pieces, int window, int keep_first,
+                           float out_scale, const float* __restrict__ sink, ScoreForm form, float* __restrict__ partial, Gate gate) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    mfma_rows<T, QS, DVB>(qkv, row_stride, kpool, vpool, block_table, table_width, tiles, positions, bias, distances, out, H, G, dk, dv, page_size, scale, temp_coef, temp_every,
+                          heads_per_chunk, k_pieces, v_pieces, window, keep_first, out_scale, sink, form, partial, gate, lds);
 }
 
 // ------------------------------------------------------------------ prompt portions in bfloat16
@@ -1100,6 +1111,273 @@ bias_attention_bf16_kernel(const bf16_t* __restrict__ qkv, int row_stride, const
                 for (int r = 0; r < 4; ++r) o[r] *= gate.of(first_row + token, head * dv + 16 * db + 4 * kg + r);
             }
             store_packed<bf16_t, 4>(orow + 16 * db, o);
+        }
+    }
+}
+
+// ------------------------------------------------------------------ prompt portions in float32, in three parts
+// The same tiles for float32 queries, keys and values.  The float32 matrix instructions take sixteen times as long as bfloat16
+// ones, so every number is taken apart into three bfloat16 parts that add up to it (exactly, of 2^-110 and more) and six of the nine
+// products of two such sums are made: what is left out is at most 2^-24 of a product and 2^-27 on average.  Keys and values are split on their
+// way into LDS, 32 at a time, the queries once, a lane's eight weights in its registers; V^T is read by transposing
+// reads.  A row's weights are taken against a reference that moves only when its scores have risen far above it.  Rows, keys
+// and lanes are as in the bfloat16 kernel; the next keys are asked for before these are worked on, and their pages a step earlier.
+//
+// What bounds it is the vector unit: exponentials, splits, caps.  Measured, mfma_rows : this (us): 1,500 tokens, 32 heads of 64 on 8,
+// with a bias 302 : 154; 512 at 1,500 keys 242 : 127; 2,045 tokens, keys of 64 and values of 128 channels, two maps, capped, in chunks of
+// 1,024 741 : 275.
+//
+// An infinity less itself has no rest (nor has a number so large that it rounds to one): a tile with a result that is not finite is made
+// again by mfma_rows, which gives what a float32 product makes of such numbers.
+#define PART_KEYS 32
+#define PART_SLACK 5.545177444479562f      // e^5.545 = 2^8
+
+struct Parts { uint4 p[3]; };
+__device__ __forceinline__ Parts parts8(const float* v) {
+    uint32_t h[4], m[4], l[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        h[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
+        const float r0 = v[2 * i] - __uint_as_float(h[i] << 16), r1 = v[2 * i + 1] - __uint_as_float(h[i] & 0xffff0000u);
+        m[i] = pack_bf16x2(r0, r1);
+        l[i] = pack_bf16x2(r0 - __uint_as_float(m[i] << 16), r1 - __uint_as_float(m[i] & 0xffff0000u));
+    }
+    return Parts{{make_uint4(h[0], h[1], h[2], h[3]), make_uint4(m[0], m[1], m[2], m[3]), make_uint4(l[0], l[1], l[2], l[3])}};
+}
+// of six products of parts, the small ones first
+constexpr int PART_A[6] = {2, 0, 1, 1, 0, 0}, PART_B[6] = {0, 2, 1, 0, 1, 0};
+
+template <int KQ, int DVB> struct PartTile {
+    uint16_t k[3][PART_KEYS][32 * KQ + TILE_PAD], v[3][PART_KEYS][16 * DVB + TILE_PAD];
+};
+
+template <int KQ, int DVB>
+__global__ void __launch_bounds__(WAVES * WAVE, KQ > 4 || DVB > 8 ? 1 : 2)
+bias_attention_parts_kernel(const float* __restrict__ qkv, int row_stride, const float* __restrict__ kpool, const float* __restrict__ vpool,
+                            const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ tiles,
+                            const int32_t* __restrict__ positions, const float* __restrict__ bias, int distances,
+                            float* __restrict__ out, int H, int G, int dk, int dv, int page_size, float scale, float temp_coef,
+                            int temp_every, int heads_per_chunk, int window, int keep_first, float out_scale, const float* __restrict__ sink,
+                            ScoreForm form, float* __restrict__ partial, Gate gate) {
+    constexpr int KC = KQ > 1 ? KQ / 2 : 1, VC = DVB / 4, THREADS = WAVES * WAVE;
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    auto& at = *reinterpret_cast<PartTile<KQ, DVB>*>(lds);
+    const int tile = blockIdx.x, g = blockIdx.y, chunk = blockIdx.z;
+    const int seq = tiles[4 * tile], first_row = tiles[4 * tile + 1], n_tok = tiles[4 * tile + 2];
+    const int first_pos = positions[first_row];
+    const int group = H / G;
+    const int heads_here = std::min(heads_per_chunk, group - chunk * heads_per_chunk);
+    const int head0 = g * group + chunk * heads_per_chunk;
+    const int n_rows = n_tok * heads_here;        // row r = token r / heads_here, head r % heads_here
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int i = lane & 15, kg = lane >> 4;
+    const int kv = g / form.maps, kv_heads = G / form.maps, k_row = form.maps * dk;
+    const float* keys = kpool + (g % form.maps) * dk;
+    const float inv_cap = form.softcap > 0.f ? 1.0f / form.softcap : 0.f;
+
+    const int row = wave * 16 + i;
+    const bool valid = row < n_rows;
+    const int token = valid ? row / heads_here : 0;
+    const int pos = first_pos + token;
+    const int head = head0 + (valid ? row % heads_here : 0);
+    const int lo = first_seen(pos, window, form.chunk);
+    const int steps = temp_every > 0 ? (pos + 1) / temp_every : 0;
+    const float factor = scale * (1.0f + temp_coef * logf(static_cast<float>(steps) + 1.0f));
+    Parts qf[KQ];
+#pragma unroll
+    for (int kk = 0; kk < KQ; ++kk) {
+        const int c = 32 * kk + 8 * kg;
+        float v[8];
+        const bool have = valid && c < dk;
+        VecIO<float, 8>::load(qkv + static_cast<size_t>(first_row + token) * row_stride + head * dk + (have ? c : 0), v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = have ? v[e] : 0.f;
+        qf[kk] = parts8(v);
+    }
+    // the positions between which every row of this wavefront lies, and the last row's first key (the same for all its lanes)
+    const int wave_rows = std::min(16, n_rows - wave * 16);
+    const int wave_first = first_pos + (wave * 16) / heads_here;
+    const int wave_last = wave_rows > 0 ? first_pos + (wave * 16 + wave_rows - 1) / heads_here : -1;
+    const int wave_lo = first_seen(wave_last, window, form.chunk);
+    float m = -INFINITY, l_lane = 0.f;            // the row's reference; the sum of this lane's own weights
+    floatx4_t acc[DVB];
+#pragma unroll
+    for (int db = 0; db < DVB; ++db) acc[db] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    const int dvb = dv / 16;
+    const int last_pos = first_pos + n_tok - 1;
+    const int32_t* table = block_table + static_cast<size_t>(seq) * table_width;
+    const int k_pieces = dk / 8, v_pieces = dv / 8;
+    const int shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz(page_size) : -1;
+    auto page_of = [&](int key) { return shift >= 0 ? key >> shift : key / page_size; };
+    // a piece is eight numbers of a row; the pages of a thread's pieces (-1: no row to read), then the pieces themselves
+    auto look_up = [&](int k0, int pieces, auto& pages) {
+#pragma unroll
+        for (int u = 0; u < static_cast<int>(sizeof(pages) / sizeof(int)); ++u) {
+            const int j = (u * THREADS + tid) / pieces, key = k0 + j;
+            pages[u] = table[page_of(std::min(key, last_pos))];
+            if (j >= PART_KEYS || key > last_pos) pages[u] = -1;
+        }
+    };
+    struct Piece { float4 a, b; };
+    auto ask = [&](const float* pool, int pieces, int row_elems, int k0, const auto& pages, auto& regs) {
+#pragma unroll
+        for (int u = 0; u < static_cast<int>(sizeof(pages) / sizeof(int)); ++u) {
+            const int idx = u * THREADS + tid, j = idx / pieces, key = std::min(k0 + j, last_pos);
+            const float* from = pool + ((static_cast<size_t>(std::max(pages[u], 0)) * kv_heads + kv) * page_size + (key - page_of(key) * page_size)) * row_elems +
+                                (idx - j * pieces) * 8;
+            regs[u].a = *reinterpret_cast<const float4*>(from);
+            regs[u].b = *reinterpret_cast<const float4*>(from + 4);
+            if (pages[u] < 0) regs[u].a = regs[u].b = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    };
+    auto put = [&](auto& dst, int pieces, const auto& regs) {
+#pragma unroll
+        for (int u = 0; u < static_cast<int>(sizeof(regs) / sizeof(Piece)); ++u) {
+            const int idx = u * THREADS + tid, j = idx / pieces;
+            const float v[8] = {regs[u].a.x, regs[u].a.y, regs[u].a.z, regs[u].a.w, regs[u].b.x, regs[u].b.y, regs[u].b.z, regs[u].b.w};
+            const Parts x = parts8(v);
+            if (j < PART_KEYS) {
+#pragma unroll
+                for (int p = 0; p < 3; ++p) *reinterpret_cast<uint4*>(&dst[p][j][(idx - j * pieces) * 8]) = x.p[p];
+            }
+        }
+    };
+    if (dk < 32 * KQ) {                           // the channels that no key has meet zeros of the queries: they must be numbers
+        const int none = 32 * KQ - dk;
+        for (int e = tid; e < 3 * PART_KEYS * none; e += THREADS) at.k[e / (PART_KEYS * none)][e / none % PART_KEYS][dk + e % none] = 0;
+    }
+    const KeyWalk walk(first_pos, last_pos, window, keep_first, form.chunk);
+    const int count = 2 * walk.steps;             // halves of tiles of 64 keys; the last may lie behind the last key
+    auto first_key = [&](int v) { return walk.first_key(v >> 1) + (v & 1) * PART_KEYS; };
+    int k_page[KC], v_page[VC];
+    Piece kr[KC], vr[VC];
+    look_up(first_key(0), k_pieces, k_page);
+    look_up(first_key(0), v_pieces, v_page);
+    ask(keys, k_pieces, k_row, first_key(0), k_page, kr);
+    ask(vpool, v_pieces, dv, first_key(0), v_page, vr);
+    look_up(first_key(1), k_pieces, k_page);
+    look_up(first_key(1), v_pieces, v_page);
+    for (int v = 0; v < count; ++v) {
+        const int k0 = first_key(v);
+        __syncthreads();                          // the keys before these have been used by everyone
+        put(at.k, k_pieces, kr);
+        put(at.v, v_pieces, vr);
+        __syncthreads();
+        if (v + 1 < count) {
+            ask(keys, k_pieces, k_row, first_key(v + 1), k_page, kr);
+            ask(vpool, v_pieces, dv, first_key(v + 1), v_page, vr);
+            if (v + 2 < count) {
+                look_up(first_key(v + 2), k_pieces, k_page);
+                look_up(first_key(v + 2), v_pieces, v_page);
+            }
+        }
+        if (k0 > wave_last) continue;             // nothing here for this wavefront's rows (it still stages and waits)
+        float near[8];
+        if (bias) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int back = std::min(std::max(pos - (k0 + 16 * (e / 4) + 4 * kg + e % 4), 0), distances - 1);
+                near[e] = bias[static_cast<size_t>(back) * H + head];
+            }
+        }
+        floatx4_t sc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int kk = 0; kk < KQ; ++kk) {
+            if (32 * kk < dk) {
+                Parts kf[2];
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int p = 0; p < 3; ++p) kf[j].p[p] = *reinterpret_cast<const uint4*>(&at.k[p][16 * j + i][32 * kk + 8 * kg]);
+#pragma unroll
+                for (int n = 0; n < 6; ++n)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        sc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[j].p[PART_A[n]]),
+                                                                        __builtin_bit_cast(bf16x8_t, qf[kk].p[PART_B[n]]), sc[j], 0, 0, 0);
+            }
+        }
+        const bool edge = k0 + PART_KEYS - 1 > wave_first || k0 < wave_lo;      // some row of this wavefront does not see every key
+        float s[8], top = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            float x = sc[e / 4][e % 4] * factor;
+            if (bias) x += near[e];
+            if (form.softcap > 0.f) x = soft_capped(x, form.softcap, inv_cap);
+            if (edge && !(valid && key_seen(k0 + 16 * (e / 4) + 4 * kg + e % 4, pos, lo, keep_first))) x = -INFINITY;
+            s[e] = x;
+            top = fmaxf(top, x);
+        }
+        if (__any(top > m + PART_SLACK)) {        // a row whose scores have risen far above its reference: move it, rescale what was summed
+            top = groups4(top, true);
+            const bool move = top > m + PART_SLACK;
+            const float m_new = move ? top : m;
+            const float alpha = move ? expf(m - m_new) : 1.f;         // 0 at the row's first keys
+            m = m_new;
+            l_lane *= alpha;
+#pragma unroll
+            for (int db = 0; db < DVB; ++db) acc[db] *= alpha;
+        }
+        float w[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            w[e] = m > -INFINITY ? exp_below(s[e] - m) : s[e] != s[e] ? s[e] : 0.f;      // (NaN raises no maximum)
+            l_lane += w[e];
+        }
+        const Parts pf = parts8(w);
+#pragma unroll
+        for (int db = 0; db < DVB; ++db) {
+            if (db < dvb) {
+                bf16x8_t vf[3];
+#pragma unroll
+                for (int p = 0; p < 3; ++p) vf[p] = read_values_t(&at.v[p][0][0], 16 * DVB + TILE_PAD, 16 * db, i, kg);
+#pragma unroll
+                for (int n = 0; n < 6; ++n)
+                    acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[PART_A[n]], __builtin_bit_cast(bf16x8_t, pf.p[PART_B[n]]), acc[db], 0, 0, 0);
+            }
+        }
+    }
+    const float l = groups4(l_lane, false);
+    float zero = 0.f;
+    if (valid) {
+        zero = l * 0.f;
+#pragma unroll
+        for (int db = 0; db < DVB; ++db)
+            if (db < dvb) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) zero = fmaf(acc[db][r], 0.f, zero);
+            }
+    }
+    if (__syncthreads_or(!(zero == 0.f))) {
+        mfma_rows<float, 2 * KQ, DVB>(qkv, row_stride, kpool, vpool, block_table, table_width, tiles, positions, bias, distances, out, H, G, dk, dv, page_size,
+                                      scale, temp_coef, temp_every, heads_per_chunk, true, true, window, keep_first, out_scale, sink, form, partial, gate, lds);
+        return;
+    }
+    if (!valid) return;
+    if (partial) {              // an unfinished row, as a run of one
+        float* prow = partial + (static_cast<size_t>(first_row + token) * H + head) * (dv + 2);
+        if (kg == 0) { prow[0] = m; prow[1] = l; }
+#pragma unroll
+        for (int db = 0; db < DVB; ++db) {
+            if (db < dvb) {
+#pragma unroll
+                for (int r = 0; r < 4; r += 2)
+                    *reinterpret_cast<float2*>(prow + 2 + 16 * db + 4 * kg + r) = make_float2(acc[db][r], acc[db][r + 1]);
+            }
+        }
+        return;
+    }
+    float* orow = out + static_cast<size_t>(first_row + token) * (H * dv) + head * dv + 4 * kg;
+    float inv = out_scale / l;
+    if (sink) {                 // one more term in the denominator, as in the kernels above
+        const float sk = sink[head], M = fmaxf(m, sk), u = expf(m - M);
+        inv = out_scale * u / (l * u + expf(sk - M));
+    }
+#pragma unroll
+    for (int db = 0; db < DVB; ++db) {
+        if (db < dvb) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) orow[16 * db + r] = acc[db][r] * inv * gate.of(first_row + token, head * dv + 16 * db + 4 * kg + r);
         }
     }
 }
@@ -1591,6 +1869,23 @@ static void launch_bf16_values(const MfmaArgs& a, dim3 grid, hipStream_t stream)
     else launch_bf16<KQ, 16>(a, grid, stream);
 }
 
+template <int KQ, int DVB>
+static hipError_t launch_parts(const MfmaArgs& a, dim3 grid, size_t lds, hipStream_t stream) {
+    lds = std::max(lds, sizeof(PartTile<KQ, DVB>));
+    static size_t allowed = 48 * 1024;            // of this instance of the kernel
+    if (lds > allowed) {
+        const hipError_t err = hipFuncSetAttribute((const void*)bias_attention_parts_kernel<KQ, DVB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (err != hipSuccess) return err;
+        allowed = lds;
+    }
+    bias_attention_parts_kernel<KQ, DVB><<<grid, WAVES * WAVE, lds, stream>>>(
+        (const float*)a.qkv, a.row_stride, (const float*)a.kpool, (const float*)a.vpool, (const int32_t*)a.block_table, a.table_width,
+        (const int32_t*)a.tiles, (const int32_t*)a.positions, (const float*)a.bias, a.distances, (float*)a.out, a.H, a.G, a.dk, a.dv,
+        a.page_size, a.scale, a.temp_coef, a.temp_every, a.heads_per_chunk, a.window, a.keep_first, a.out_scale, (const float*)a.sink, a.form,
+        (float*)a.partial, a.gate);
+    return hipSuccess;
+}
+
 // tiles of up to 64 rows (tokens * heads of a chunk), no runs: for steps with portions of prompts
 NI_EXPORT int ni_bias_attention_mfma(const void* qkv, int row_stride, const void* kpool, const void* vpool, const void* block_table,
                                      int table_width, const void* tiles, int n_tiles, const void* positions, const void* bias,
@@ -1620,6 +1915,15 @@ NI_EXPORT int ni_bias_attention_mfma(const void* qkv, int row_stride, const void
         else if (dk <= 64) launch_bf16_values<2>(args, grid, stream);
         else if (dk <= 128) launch_bf16_values<4>(args, grid, stream);
         else launch_bf16_values<8>(args, grid, stream);
+        return NI_LAUNCH_RESULT();
+    }
+    // float32 rows in whole 16-byte pieces: in parts
+    if (dtype == 0 && k_pieces && v_pieces && row_stride % 4 == 0 && reinterpret_cast<uintptr_t>(qkv) % 16 == 0 && dk <= 128 && dv <= 256) {
+        if (dk <= 64) err = dv <= 64 ? launch_parts<2, 4>(args, grid, lds, stream) : dv <= 128 ? launch_parts<2, 8>(args, grid, lds, stream)
+                                                                                            : launch_parts<2, 16>(args, grid, lds, stream);
+        else err = dv <= 64 ? launch_parts<4, 4>(args, grid, lds, stream) : dv <= 128 ? launch_parts<4, 8>(args, grid, lds, stream)
+                                                                                    : launch_parts<4, 16>(args, grid, lds, stream);
+        if (err != hipSuccess) return (int)err;
         return NI_LAUNCH_RESULT();
     }
     // the smallest arrays of registers that hold these sizes
