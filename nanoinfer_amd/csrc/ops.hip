@@ -8,6 +8,7 @@
 //   * every entry point is extern "C", takes raw device pointers and a hipStream_t, and
 //     returns 0 or the hipError_t of its launch.  Shapes are checked by the host wrapper.
 #include "common.h"
+#include "pair_rows.h"
 
 #include <algorithm>
 
@@ -89,16 +90,19 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ h, const TP* __restrict__
 // The same for rows whose width is a multiple of four: a thread holds G groups of four consecutive
 // elements, so that every access is 16 bytes of float32 or 8 bytes of bfloat16 a lane and neighbouring
 // lanes touch neighbouring groups (a third of the instructions, and the memory system sees whole lines).
-template <typename TP, typename TO, int G>
+// HALVES (float32 rows of whole stages of 32 columns): the row is left as pairs of halves too (pair_rows.h), for the products behind
+// the norm.  It is at hand here; a pass of its own reads it again and is a launch more: 512 rows of 2,048 behind two addends 8.2 + 5.4 us
+// apart, 10.3 here; 1,500 rows 6.2 + 7.4 (that for each of two or three products) and 9.7.
+template <typename TP, typename TO, int G, bool HALVES = false>
 __global__ void add_rmsnorm_vec_kernel(float* __restrict__ h, const TP* __restrict__ pending, int addends, size_t addend_stride,
                                        const float* __restrict__ w, TO* __restrict__ out,
-                                       const int32_t* __restrict__ rows, int d, float eps) {
+                                       const int32_t* __restrict__ rows, int d, float eps, char* __restrict__ planes = nullptr,
+                                       int2* __restrict__ info = nullptr) {
     __shared__ float scratch[16];
     const int r = blockIdx.x;
     const size_t src = rows ? static_cast<size_t>(rows[r]) : static_cast<size_t>(r);
     float* hrow = h + src * d;
     const TP* prow = pending ? pending + src * d : nullptr;
-    const int groups = d / 4;
     float v[G][4], wv[G][4];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
@@ -156,8 +160,52 @@ __global__ void add_rmsnorm_vec_kernel(float* __restrict__ h, const TP* __restri
         if (at < d) {
             float y[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) y[e] = (v[g][e] * inv) * wv[g][e];
+            for (int e = 0; e < 4; ++e) v[g][e] = y[e] = (v[g][e] * inv) * wv[g][e];
             store_packed<TO, 4>(orow + at, y);
+        }
+    }
+    if constexpr (HALVES) {
+        __shared__ uint32_t tops[16];
+        __shared__ int bigs[16];
+        const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE, waves = blockDim.x / WAVE;
+        uint32_t top = 0;
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+            if ((threadIdx.x + g * blockDim.x) * 4 < d)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) top = max(top, __float_as_uint(v[g][e]) & 0x7fffffffu);
+#pragma unroll
+        for (int off = WAVE / 2; off > 0; off >>= 1) top = max(top, static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), off, WAVE)));
+        if (lane == 0) tops[wave] = top;
+        __syncthreads();
+        for (int i = 0; i < waves; ++i) top = max(top, tops[i]);
+        const int s = pair_scale(top);
+        char* prow_out = planes + static_cast<size_t>(r) * d * 4;
+        int big = 0;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const int at = (threadIdx.x + g * blockDim.x) * 4;
+            if (at < d) {
+                float u[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    u[e] = ldexpf(v[g][e], s);
+                    big += fabsf(u[e]) >= PAIR_BIG;
+                }
+                uint2 hh, ll;
+                pair_up(u, hh, ll);
+                *reinterpret_cast<uint2*>(prow_out + pair_place(at)) = hh;
+                *reinterpret_cast<uint2*>(prow_out + pair_place(at) + 32) = ll;
+            }
+        }
+#pragma unroll
+        for (int off = WAVE / 2; off > 0; off >>= 1) big += __shfl_xor(big, off, WAVE);
+        if (lane == 0) bigs[wave] = big;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            big = 0;
+            for (int i = 0; i < waves; ++i) big += bigs[i];
+            info[r] = pair_row_info(s, top, big);
         }
     }
 }
@@ -472,6 +520,21 @@ NI_EXPORT int ni_add_rmsnorm(void* h, const void* pending, int addends, int floa
     else
         launch_add_rmsnorm<bf16_t, bf16_t>((float*)h, (const bf16_t*)pending, addends, addend_stride, (const float*)w,
                                            (bf16_t*)out, (const int32_t*)rows, n_rows, d, eps, stream);
+    return NI_LAUNCH_RESULT();
+}
+
+// The same for float32 rows, all of them, that are left as pairs of halves as well: d in whole stages of 32 columns, everything
+// aligned to 16 bytes.
+NI_EXPORT int ni_add_rmsnorm_halves(void* h, const void* pending, int addends, size_t addend_stride, const void* w, void* out, void* planes,
+                                    void* info, int n_rows, int d, float eps, hipStream_t stream) {
+    constexpr int NV = 8;
+    if (n_rows <= 0) return 0;
+    if (d <= 0 || d % 32 || d > NV * 1024 || (pending && addends < 1) || !aligned_to(16, h, w) || !aligned_to(16, pending, out) ||
+        !aligned_to(16, planes) || (addends > 1 && addend_stride % 4))
+        return static_cast<int>(hipErrorInvalidValue);
+    const int threads = d <= NV * 64 ? 64 : d <= NV * 128 ? 128 : d <= NV * 256 ? 256 : d <= NV * 512 ? 512 : 1024;
+    add_rmsnorm_vec_kernel<float, float, NV / 4, true><<<n_rows, threads, 0, stream>>>(
+        (float*)h, (const float*)pending, addends, addend_stride, (const float*)w, (float*)out, nullptr, d, eps, (char*)planes, (int2*)info);
     return NI_LAUNCH_RESULT();
 }
 

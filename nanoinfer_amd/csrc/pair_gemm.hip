@@ -31,32 +31,12 @@
 // [16384, 2048] 643 : 380, on [4096, 14336] 1,105 : 574 (409 TFLOP/s); 100 rows on [16384, 2048] 103 : 64.  What bounds it is the clock
 // that the matrix cores hold: 256 workgroups of the largest tile take 0.68 us a step, eight 0.45 (of which the instructions are
 // 0.32), and with operands of ones, which switch less, 256 take 0.56.
+#include "pair_rows.h"
 #include "split_tile.h"
-#include <limits.h>
-
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 
 template <int N> struct Which { static constexpr int value = N; };
 
-#define PAIR_BIG 4.f            // scaled numbers of this size and more are big
 #define PAIR_TERMS 64           // products of big numbers that a result has at least
-
-// Eight scaled numbers as two planes of eight halves.
-__device__ __forceinline__ void pair8(const float* v, uint4& h, uint4& l) {
-    f16x8_t hv, lv;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        hv[i] = static_cast<_Float16>(v[i]);
-        lv[i] = static_cast<_Float16>((v[i] - static_cast<float>(hv[i])) * 4096.f);
-    }
-    h = __builtin_bit_cast(uint4, hv);
-    l = __builtin_bit_cast(uint4, lv);
-}
-
-// From the bits of a row's largest magnitude: the power of two that brings it to 2^14 .. 2^15.
-__device__ __forceinline__ int pair_scale(uint32_t top) {
-    return top == 0 || top >= 0x7f800000u ? 0 : 14 - ilogbf(__uint_as_float(top));
-}
 
 // eight numbers of a row from k on, zeros behind its end; K is a multiple of four
 __device__ __forceinline__ void load8(const float* __restrict__ row, int k, int K, float* v) {
@@ -110,8 +90,8 @@ __global__ __launch_bounds__(256) void pair_rows_kernel(const float* __restrict_
             big += fabsf(u[i]) >= PAIR_BIG;
         }
         uint4 h, l;
-        pair8(u, h, l);
-        char* p = to + (k >> 4) * 64 + ((k >> 3) & 1) * 16;
+        pair_up(u, h, l);
+        char* p = to + pair_place(k);
         *reinterpret_cast<uint4*>(p) = h;
         *reinterpret_cast<uint4*>(p + 32) = l;
     };
@@ -131,7 +111,7 @@ __global__ __launch_bounds__(256) void pair_rows_kernel(const float* __restrict_
     __syncthreads();
     if (tid == 0) {
         big = bigs[0] + bigs[1] + bigs[2] + bigs[3];
-        info[blockIdx.x] = make_int2(s, top == 0 ? INT_MAX : top >= 0x7f800000u ? -1 : big);
+        info[blockIdx.x] = pair_row_info(s, top, big);
     }
 }
 
@@ -172,7 +152,7 @@ __global__ __launch_bounds__(PAIR_WEIGHT_WAVES * WAVE) void pair_weight_kernel(c
             big += fabsf(v[i]) >= PAIR_BIG;
         }
         uint4 h, l;
-        pair8(v, h, l);
+        pair_up(v, h, l);
         *reinterpret_cast<uint4*>(to + static_cast<size_t>(t) * 2048) = h;
         *reinterpret_cast<uint4*>(to + static_cast<size_t>(t) * 2048 + 1024) = l;
     }

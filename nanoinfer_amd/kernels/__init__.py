@@ -1207,7 +1207,7 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
     output type) instead of a new tensor.  ``leave`` (with ``residual``, where :func:`leaves_scaled_ok`
     holds; ignored elsewhere): the norm that stands behind the stream; the product then runs whole and
     returns a :class:`ScaledInput` for that norm.  ``x`` may itself be a :class:`ScaledInput` where
-    :func:`takes_scaled_ok` holds.  ``addends`` (ignored with ``out``): a product of many rows may come back as float32
+    :func:`takes_scaled_ok` holds, or :class:`HalvedRows`.  ``addends`` (ignored with ``out``): a product of many rows may come back as float32
     addends [S, M, N] (its K range cut into S shares), for a norm that adds them to the stream itself."""
     rows, _ = _rows_and_tiles(weight)
     if out is not None and (isinstance(x, (NormedInput, ScaledInput)) or residual is not None):
@@ -1222,6 +1222,7 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
             raise KernelError("a normed input and a residual output in one product are not compiled")
         out = torch.empty(x.shape[0], rows.shape[0], dtype=x.dtype, device=x.device)
         return skinny_gemm(x, weight, out)
+    halved, x = x, rows_of(x)
     if not (x.is_cuda and rows.is_cuda):
         raise KernelError("linear needs GPU tensors")
     if not (x.dtype == rows.dtype):
@@ -1254,8 +1255,8 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
         if out is None:
             out = torch.empty(M, rows.shape[0], dtype=out_dtype, device=x.device)
         return skinny_gemm(x, weight, out)
-    if out_dtype == torch.float32 and pair_wins(x, weight):
-        return pair_gemm(x, weight, out, addends=addends)
+    if out_dtype == torch.float32 and pair_wins(halved, weight):
+        return pair_gemm(halved, weight, out, addends=addends)
     if out_dtype == torch.float32 and split_wins(x, rows):
         return split_gemm(x, rows, out, addends=addends)
     if tiled_wins(x, weight, addends=addends) and (out is None or out.data_ptr() % 16 == 0):
@@ -1277,8 +1278,9 @@ def swiglu_takes_scaled(M: int, K: int, dtype: torch.dtype, weight_gate_up) -> b
 def linear_swiglu(x, weight_gate_up, activation: str = "silu") -> torch.Tensor:
     """``silu(x . Wg^T) * (x . Wu^T)`` (or another of ``GATED_ACTIVATIONS``) for the stacked matrix [Wg; Wu]: fused into
     the product for few rows, product then the SwiGLU kernel for many.  ``x`` may be a :class:`NormedInput`, or a
-    :class:`ScaledInput` where :func:`swiglu_takes_scaled` holds."""
+    :class:`ScaledInput` where :func:`swiglu_takes_scaled` holds, or :class:`HalvedRows`."""
     inter = weight_gate_up.shape[0] // 2
+    halved, x = x, rows_of(x)
     out = torch.empty(x.shape[0], inter, dtype=x.dtype, device=x.device)
     if isinstance(x, ScaledInput) and not swiglu_takes_scaled(x.shape[0], x.shape[1], x.dtype, weight_gate_up):
         raise KernelError("this product cannot take a scaled input")
@@ -1289,10 +1291,10 @@ def linear_swiglu(x, weight_gate_up, activation: str = "silu") -> torch.Tensor:
                                       and (M <= SKINNY_BEST_ROWS or inter % 16 == 0)):
         return skinny_gemm(x, weight_gate_up, out, swiglu=True, activation=activation)
     rows, _ = _rows_and_tiles(weight_gate_up)
-    if pair_wins(x, weight_gate_up):
+    if pair_wins(halved, weight_gate_up):
         if inter % 32 == 0 and pair_plan(M, 2 * inter, Kd, True)[2] <= pair_plan(M, 2 * inter, Kd)[2] + 4.0 + 12.0 * M * inter / 4e6:
-            return pair_gemm(x, weight_gate_up, out, gated=activation)
-        return swiglu(pair_gemm(x, weight_gate_up), out, activation)
+            return pair_gemm(halved, weight_gate_up, out, gated=activation)
+        return swiglu(pair_gemm(halved, weight_gate_up), out, activation)
     if split_wins(x, rows):
         # in one kernel, or cut along K with the SwiGLU kernel behind it (which moves 12 bytes an output at 4 TB/s)
         if split_plan(M, 2 * inter, Kd, True)[2] <= split_plan(M, 2 * inter, Kd)[2] + 4.0 + 12.0 * M * inter / 4e6:
@@ -1309,13 +1311,14 @@ def linear_swiglu(x, weight_gate_up, activation: str = "silu") -> torch.Tensor:
 def linear_relu2(x, weight) -> torch.Tensor:
     """``relu(x . weight^T)^2`` in the type of ``x``: fused into the product for few rows, product then an elementwise kernel
     for many."""
+    halved, x = x, rows_of(x)
     M, Kd = x.shape
     if skinny_wins(M, Kd, x.dtype, weight) if M <= SKINNY_MAX_ROWS else (skinny_deals(M, weight.shape[0], Kd, x.dtype, weight) and _plain(x)):
         out = torch.empty(M, weight.shape[0], dtype=x.dtype, device=x.device)
         return skinny_gemm(x, weight, out, activation="relu2")
     rows, _ = _rows_and_tiles(weight)
-    if pair_wins(x, weight):
-        return pair_gemm(x, weight, squared=True)
+    if pair_wins(halved, weight):
+        return pair_gemm(halved, weight, squared=True)
     if split_wins(x, rows):
         return split_gemm(x, rows, squared=True)
     if tiled_wins(x, weight):
@@ -1333,8 +1336,9 @@ torch.backends.cuda.matmul.allow_tf32 = False
 torch.backends.cudnn.allow_tf32 = False
 
 # products of many rows on the matrix cores
-from .tile import (experts_grouped, experts_grouped_wins, pair_gemm, pair_holds, pair_plan, pair_rows, pair_weight, pair_wins, split_gemm, split_plan, split_wins, tile_lib, tiled_gemm, tiled_plan,  # noqa: E402,F401
-                   tiled_wins)
+from .tile import (HalvedRows, add_rmsnorm_halved, experts_grouped, experts_grouped_wins, pair_gemm, pair_holds, pair_plan,  # noqa: E402,F401
+                   pair_rows, pair_weight, pair_wins, rows_of, split_gemm, split_plan, split_wins, takes_halved, tile_lib, tiled_gemm,
+                   tiled_plan, tiled_wins)
 # sums onto the residual stream, routed experts, the gated delta rule, attention with a bias by distance
 from .stream import (BIAS_ATTENTION_MFMA_FROM, DELTA_RUN_FROM, EXPERTS_FEW_ROWS, add_rmsnormed, add_vector,  # noqa: E402,F401
                      bias_attention, bias_attention_lib, bias_attention_mfma, bias_attention_mfma_rows, bias_attention_rows, bias_attention_runs, bias_attention_bf16_tokens, bias_attention_token_runs, delta_rule, delta_rule_lib, embed_scaled, experts_act, experts_few,

@@ -10,7 +10,7 @@ from typing import Optional, Tuple
 import torch
 
 from ..csrc import build as _build
-from . import GATED_ACTIVATIONS, KernelError, _check, _gpu, _load, _ptr, _stream, dtype_code
+from . import GATED_ACTIVATIONS, KernelError, _check, _gpu, _load, _ptr, _stream, add_rmsnorm, core, dtype_code
 
 COMPUTE_UNITS = 256
 
@@ -185,33 +185,95 @@ def pair_rows(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     return planes, info
 
 
+class HalvedRows:
+    """Float32 rows ``x`` [M, K] that a norm also left as pairs of halves (``planes`` and ``info``, what :func:`pair_rows` makes of
+    them), for the products behind it.  A part that ``takes_halved`` is given one; whatever does not go to :func:`pair_gemm`
+    reads ``x``."""
+
+    __slots__ = ("x", "planes", "info")
+
+    def __init__(self, x: torch.Tensor, planes: torch.Tensor, info: torch.Tensor):
+        self.x, self.planes, self.info = x, planes, info
+
+    @property
+    def shape(self):
+        return self.x.shape
+
+    @property
+    def dtype(self):
+        return self.x.dtype
+
+    @property
+    def device(self):
+        return self.x.device
+
+
+def rows_of(x):
+    """The rows themselves of what may be :class:`HalvedRows`."""
+    return x.x if isinstance(x, HalvedRows) else x
+
+
+def _halves_of(x):
+    """(rows, planes, info) of rows or :class:`HalvedRows`."""
+    return (x.x, x.planes, x.info) if isinstance(x, HalvedRows) else (x, *pair_rows(x))
+
+
+def add_rmsnorm_halved(h: torch.Tensor, pending: Optional[torch.Tensor], weight: torch.Tensor, eps: float) -> HalvedRows:
+    """``h += pending`` and ``rmsnorm(h) * weight`` in float32, as rows and as pairs of halves.  ``pending`` [T, d] or [S, T, d]."""
+    T, d = h.shape
+    _gpu(h, "h", torch.float32)
+    _gpu(weight, "weight", torch.float32, (d,))
+    out = torch.empty(T, d, dtype=torch.float32, device=h.device)
+    addends = 1
+    if pending is not None:
+        addends = pending.shape[0] if pending.dim() == 3 else 1
+        _gpu(pending, "pending", torch.float32, (addends, T, d) if pending.dim() == 3 else (T, d))
+    if d % 32 or d > 8192 or T * (d + 31) >= 1 << 29 or any(t is not None and t.data_ptr() % 16 for t in (h, weight, pending)):
+        add_rmsnorm(h, pending, weight, eps, out)
+        return HalvedRows(out, *pair_rows(out))
+    planes, info = _pair_planes(T, d, h.device)
+    _check(core().ni_add_rmsnorm_halves(_ptr(h), _ptr(pending), addends, ctypes.c_size_t(T * d), _ptr(weight), _ptr(out), _ptr(planes), _ptr(info),
+                                        T, d, ctypes.c_float(eps), _stream()), "add_rmsnorm_halves")
+    return HalvedRows(out, planes, info)
+
+
 # Operations from which a float32 product goes to pair_gemm.  Measured in recorded launches, each with another W and all its kernels
 # counted (us, library : this): [2048, 2048] at 256 / 400 / 800 rows (2.1 / 3.4 / 6.7 GFLOP) 22.8 : 26.0, 38.9 : 32.0, 65.7 : 42.9;
 # [3072, 2048] at 130 / 164 / 200 (1.6 / 2.1 / 2.5) 22.6 : 26.6, 30.6 : 27.5, 31.3 : 29.5; [4096, 1024] at 256 / 400 (2.1 / 3.4) 24.1 : 26.6,
 # 37.0 : 31.3; [3072, 3072] at 130 / 164 (2.5 / 3.1) 30.3 : 31.3, 42.0 : 32.2; [2048, 8192] at 65 / 130 (2.2 / 4.4) 42.6 : 40.0, 63.8 : 47.6.
 PAIR_FLOPS = 2.4e9
+# The same where x comes as pairs of halves (:class:`HalvedRows`): the pass over x is 4 to 5 us of those figures, a norm that does its
+# work takes 2 more.  [3072, 2048] at 164 rows (2.1 GFLOP) 29.8 in the library, 22.3 here and 5.0 for its shares; at 130 (1.6) both would take 22.
+PAIR_FLOPS_HALVED = 2.0e9
 
 
-def pair_wins(x: torch.Tensor, weight) -> bool:
+def pair_wins(x, weight) -> bool:
     """Whether a float32 product of more rows than the skinny product takes goes to :func:`pair_gemm`: a matrix that is kept as
-    pairs of halves and work enough to pay for the start and for the pass that makes pairs of x."""
-    if getattr(weight, "pairs", None) is None or x.dtype != torch.float32:
-        return False
-    M, K = x.shape
-    return (M > 64 and 2.0 * M * weight.rows.shape[0] * K >= PAIR_FLOPS and M * (K + 31) < 1 << 29 and x.is_contiguous()
-            and x.data_ptr() % 16 == 0)
+    pairs of halves and work enough to pay for the start and for the pass that makes pairs of x (:class:`HalvedRows` need none)."""
+    rows = rows_of(x)
+    return _pair_sized(*x.shape, x.dtype, weight, PAIR_FLOPS if rows is x else PAIR_FLOPS_HALVED) and rows.is_contiguous() and rows.data_ptr() % 16 == 0
 
 
-def pair_gemm(x: torch.Tensor, weight, out: Optional[torch.Tensor] = None, gated: Optional[str] = None, squared: bool = False,
+def takes_halved(M: int, K: int, dtype: torch.dtype, weight) -> bool:
+    """Whether the product of M rows as :class:`HalvedRows` goes there."""
+    return _pair_sized(M, K, dtype, weight, PAIR_FLOPS_HALVED)
+
+
+def _pair_sized(M: int, K: int, dtype: torch.dtype, weight, flops: float) -> bool:
+    return (getattr(weight, "pairs", None) is not None and dtype == torch.float32 and M > 64
+            and 2.0 * M * weight.rows.shape[0] * K >= flops and M * (K + 31) < 1 << 29)
+
+
+def pair_gemm(x, weight, out: Optional[torch.Tensor] = None, gated: Optional[str] = None, squared: bool = False,
               plan: Optional[Tuple[int, int]] = None, addends: bool = False) -> torch.Tensor:
-    """``x . weight^T`` for float32 ``x`` [M, K] and a :class:`Weight` [N, K] that is kept as pairs of halves, by three products
-    in half precision.  The other arguments as for :func:`split_gemm`."""
+    """``x . weight^T`` for float32 ``x`` [M, K] (or :class:`HalvedRows`) and a :class:`Weight` [N, K] that is kept as pairs of
+    halves, by three products in half precision.  The other arguments as for :func:`split_gemm`."""
     M, K = x.shape
     rows, pairs = weight.rows, weight.pairs
     if pairs is None:
         raise KernelError("this product takes a matrix that is kept as pairs of halves")
     N = rows.shape[0]
-    _gpu(x, "x", torch.float32, (M, rows.shape[1]))
+    _gpu(rows_of(x), "x", torch.float32, (M, rows.shape[1]))
     if gated is not None and (N % 64 or squared):
         raise KernelError("a gated product takes a stacked matrix of halves of whole tiles of 32 and no other activation")
     _addends_alone(addends, out, gated, squared)
@@ -219,7 +281,7 @@ def pair_gemm(x: torch.Tensor, weight, out: Optional[torch.Tensor] = None, gated
     tile, shares = plan or pair_plan(M, N, K, gated is not None)[:2]
     per = -(-K // (32 * shares)) * 32
     shares = -(-K // per)                                   # no share is empty
-    planes, info = pair_rows(x)
+    x, planes, info = _halves_of(x)
     if shares > 1:
         parts = torch.empty(shares, M, N, dtype=torch.float32, device=x.device)
     elif out is None:
@@ -378,12 +440,13 @@ def _experts_in_pairs(places: int, w_up, w_down, d: int, per: int, ff: int) -> b
             and per % 32 == 0 and places * max(d, ff) < 1 << 29)
 
 
-def experts_grouped_wins(x: torch.Tensor, w_up, w_down, top: int, experts: int) -> bool:
+def experts_grouped_wins(x, w_up, w_down, top: int, experts: int) -> bool:
     """Whether routed experts of float32 rows go expert by expert (:func:`experts_grouped`) instead of as two dense
     products over all experts: by the estimates of :func:`split_plan` or :func:`pair_plan`, with 25 us for the lists and the sums
     beside the passes over the entries' rows.  1,500 rows of 2,048 elements, four of sixteen experts of 1,024: 290 us for the two
     products against 960 (in three parts)."""
     up, down = getattr(w_up, "rows", w_up), getattr(w_down, "rows", w_down)
+    x = rows_of(x)
     M, d = x.shape
     per, ff = up.shape[0] // experts, down.shape[1] // experts
     if not (x.dtype == torch.float32 and d % 4 == 0 and ff % 4 == 0 and M * top < 1 << 24 and split_wins(x, up)
@@ -395,13 +458,14 @@ def experts_grouped_wins(x: torch.Tensor, w_up, w_down, top: int, experts: int) 
     return grouped < whole(M, experts * per, d)[2] + whole(M, d, experts * ff)[2]
 
 
-def experts_grouped(x: torch.Tensor, w_up, w_down, chosen: torch.Tensor, mix: torch.Tensor, experts: int,
+def experts_grouped(x, w_up, w_down, chosen: torch.Tensor, mix: torch.Tensor, experts: int,
                     act, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The weighted sum of every row's chosen experts, float32 [T, d]: the entries (token, expert) are put in the order of
     their experts, each expert multiplies its own tokens' rows, and a token's results are added in the order in which it
     chose.  ``w_up`` [E * per, d], ``w_down`` [d, E * ff], tensors or :class:`Weight`; ``act(up [entries, per], weights [entries, 1])``
     gives the hidden rows [entries, ff].  An index of E or more in ``chosen`` int32 [T, top] names an expert that is not among these."""
     up_rows, down_rows = getattr(w_up, "rows", w_up), getattr(w_down, "rows", w_down)
+    halved, x = x, rows_of(x)
     T, d = x.shape
     top, E = chosen.shape[1], experts
     places = T * top
@@ -423,7 +487,7 @@ def experts_grouped(x: torch.Tensor, w_up, w_down, chosen: torch.Tensor, mix: to
     _check(lib.ni_expert_lists(_ptr(chosen), _ptr(mix), T, top, E, _ptr(offsets), _ptr(rows), _ptr(weights), _ptr(place), _stream()), "expert_lists")
     up = torch.empty(places, per, dtype=torch.float32, device=x.device)
     if pairs:
-        _pair_grouped(x, w_up, up, offsets, rows, E, False)
+        _pair_grouped(halved, w_up, up, offsets, rows, E, False)
     else:
         _check(lib.ni_split_gemm_grouped(_ptr(x), _ptr(up_rows), _ptr(up), places, per, d, _ptr(offsets), _ptr(rows), E, ctypes.c_size_t(per * d), d,
                                          _grouped_plan(places, per, d, E)[1], _stream()), "experts_up")
@@ -442,11 +506,11 @@ def experts_grouped(x: torch.Tensor, w_up, w_down, chosen: torch.Tensor, mix: to
     return out
 
 
-def _pair_grouped(x: torch.Tensor, weight, out: torch.Tensor, offsets: torch.Tensor, rows: Optional[torch.Tensor], experts: int, down: bool) -> None:
+def _pair_grouped(x, weight, out: torch.Tensor, offsets: torch.Tensor, rows: Optional[torch.Tensor], experts: int, down: bool) -> None:
     """``out[p] = x[rows[p]] . W_e^T`` for the places p of every expert's list; its rows of W behind the others' or (``down``) beside them."""
     places, N = out.shape
     K = x.shape[1]
-    planes, info = pair_rows(x)
+    x, planes, info = _halves_of(x)
     _check(pair_lib().ni_pair_gemm_grouped(_ptr(planes), _ptr(info), _ptr(weight.pairs[0]), _ptr(weight.pairs[1]), _ptr(x), _ptr(weight.rows), _ptr(out),
                                            places, N, K, _ptr(offsets), _ptr(rows), experts, int(down),
                                            _grouped_pair_plan(places, N, K, experts)[1], _stream()), "pair_gemm_grouped")

@@ -229,6 +229,11 @@ class GatedMLP(SwiGLU):
     def carries_addends(self, T: int, addends: int) -> bool:
         return False
 
+    def takes_halved(self, T: int) -> bool:
+        cls = type(self)
+        return (cls.forward is GatedMLP.forward and cls.hidden is GatedMLP.hidden
+                and K.takes_halved(T, self.w_gate_up.shape[1], self.rt.dtype, self.w_gate_up))
+
     def hidden(self, x) -> torch.Tensor:
         return K.linear_swiglu(x, self.w_gate_up, self.activation)
 

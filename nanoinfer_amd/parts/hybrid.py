@@ -16,7 +16,7 @@ import torch
 from .. import kernels as K
 from ..registry import register_part
 from .base import Block, CacheNeed, KVNeed, LayerCache, Part, StateNeed, WeightRequest
-from .standard import build_part
+from .standard import build_part, normed_rows, takes_halved
 
 
 def _pad16(n: int) -> int:
@@ -299,6 +299,10 @@ class BiasAttention(Part):
     def cache_need(self) -> CacheNeed:
         return CacheNeed(kv=KVNeed(self.G, self.dk, None, self.dv))
 
+    def takes_halved(self, T: int) -> bool:
+        """Whether ``forward`` takes, for T tokens, rows that are pairs of halves too, and its first product reads those."""
+        return type(self).forward is BiasAttention.forward and K.takes_halved(T, self.w_qkv.shape[1], self.rt.dtype, self.w_qkv)
+
     def forward(self, x, ctx, cache: LayerCache):
         qkv = K.linear(x, self.w_qkv)
         if cache.writes:
@@ -387,6 +391,10 @@ class ChannelDelta(Part):
 
     def cache_need(self) -> CacheNeed:
         return CacheNeed(state=StateNeed((self.state_size,), torch.float32))
+
+    def takes_halved(self, T: int) -> bool:
+        """Whether ``forward`` takes, for T tokens, rows that are pairs of halves too, and its first product reads those."""
+        return type(self).forward is ChannelDelta.forward and K.takes_halved(T, self.w_in.shape[1], self.rt.dtype, self.w_in)
 
     def forward(self, x, ctx, cache: LayerCache):
         if not cache.writes:
@@ -478,7 +486,12 @@ class RoutedExperts(Part):
         if p.get("shared") is not None:
             self.shared = build_part("feed_forward", p["shared"], getattr(weights, "checkpoint", {}), rt)
 
+    def takes_halved(self, T: int) -> bool:
+        """Whether ``forward`` takes, for T tokens, rows that are pairs of halves too, and a product of it may read those."""
+        return type(self).forward is RoutedExperts.forward and K.takes_halved(T, self.w_up.shape[1], self.rt.dtype, self.w_up)
+
     def forward(self, x, ctx):
+        halved, x = x, K.rows_of(x)
         T = x.shape[0]
         z = K.linear(x, self.w_router, out_dtype=torch.float32)
         few = T <= K.EXPERTS_FEW_ROWS
@@ -493,20 +506,20 @@ class RoutedExperts(Part):
             y = K.experts_few(x, self.w_up.rows, self.w_down.rows, chosen, mix, self.ff, self.activation, None if out is None else out[0],
                               limit=self.limit, slope=self.slope)
         elif K.experts_grouped_wins(x, self.w_up, self.w_down, self.top, self.E):
-            y = K.experts_grouped(x, self.w_up, self.w_down, chosen, mix, self.E,
+            y = K.experts_grouped(halved, self.w_up, self.w_down, chosen, mix, self.E,
                                   lambda up, weights: K.experts_act(up, weights, self.ff, self.activation, self.limit, self.slope),
                                   out=None if out is None else out[0])
             if self.identity:
                 K.identity_experts(x, mix_all, self.E, out[more])
         else:
-            act = K.experts_act(K.linear(x, self.w_up), mix_all, self.ff, self.activation, self.limit, self.slope)
+            act = K.experts_act(K.linear(halved, self.w_up), mix_all, self.ff, self.activation, self.limit, self.slope)
             y = K.linear(act, self.w_down, out_dtype=torch.float32, out=None if out is None else out[0])
             if self.identity:
                 K.identity_experts(x, mix_all, self.E, out[more])
         if out is None:
             return y
         if self.shared is not None:
-            K.linear(self.shared.hidden(x), self.shared.w_down, out_dtype=torch.float32, out=out[1])
+            K.linear(self.shared.hidden(halved if takes_halved(self.shared, T) else x), self.shared.w_down, out_dtype=torch.float32, out=out[1])
         return out
 
 
@@ -532,9 +545,14 @@ class ParallelBlock(Block):
 
     def forward(self, h, pending, ctx, cache: LayerCache):
         from .base import pending_for
-        n = self.norm.forward(h, pending_for(self.norm, pending, self.rt.dtype))
-        a = self.mixer.forward(n, ctx, cache)
-        f = self.ffn.forward(n, ctx) if "ffn" in self.roles else None
+        readers = [self.mixer] + ([self.ffn] if "ffn" in self.roles else [])
+        n = normed_rows(self.norm, h, pending_for(self.norm, pending, self.rt.dtype), readers)
+
+        def for_part(part):
+            return n if takes_halved(part, h.shape[0]) else K.rows_of(n)
+
+        a = self.mixer.forward(for_part(self.mixer), ctx, cache)
+        f = self.ffn.forward(for_part(self.ffn), ctx) if "ffn" in self.roles else None
         side = getattr(self, "side", None) if "side" in self.roles else None
         x = None
         if side is not None and self.rt.dtype != torch.float32:

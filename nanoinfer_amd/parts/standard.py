@@ -90,6 +90,14 @@ class RMSNorm(Part):
         out = torch.empty(n, self.size, dtype=self.rt.dtype, device=self.rt.device)
         return K.add_rmsnorm(h, pending, self.weight, self.eps, out, rows)
 
+    def forward_halved(self, h: torch.Tensor, pending: Optional[torch.Tensor]) -> "K.HalvedRows":
+        """``forward`` of all rows in float32, left as pairs of halves as well for products that take them."""
+        return K.add_rmsnorm_halved(h, pending, self.weight, self.eps)
+
+    def leaves_halved(self) -> bool:
+        """Whether ``forward_halved`` is what ``forward`` is."""
+        return type(self).forward is RMSNorm.forward and self.rt.dtype == torch.float32
+
     def as_deferred(self) -> "K.NormSpec":
         """Weight and eps of this norm, for a product onto the residual stream that can leave ``h * weight``
         and the rows' sums of squares behind (:class:`nanoinfer_amd.kernels.ScaledInput`): the product that
@@ -102,6 +110,20 @@ class RMSNorm(Part):
         """This norm of ``h`` as an input that a product can normalise itself; ``pending`` (float32
         addends [S, T, size] that ``h`` has not received) goes along for a part that ``carries_addends``."""
         return K.NormedInput(h, self.weight, self.eps, self.rt.dtype, pending)
+
+
+def normed_rows(norm, h: torch.Tensor, pending: Optional[torch.Tensor], parts):
+    """``norm.forward(h, pending)`` for all of ``parts``, as pairs of halves too where the norm can leave them and one of the
+    parts reads them.  Whichever does not gets the rows: ``K.rows_of`` of the result."""
+    leaves = getattr(norm, "leaves_halved", None)
+    if leaves is not None and leaves() and any(takes_halved(part, h.shape[0]) for part in parts):
+        return norm.forward_halved(h, pending)
+    return norm.forward(h, pending)
+
+
+def takes_halved(part, T: int) -> bool:
+    takes = getattr(part, "takes_halved", None)
+    return takes is not None and takes(T)
 
 
 # ------------------------------------------------------------------ position
@@ -326,6 +348,13 @@ class Attention(Part):
         return (type(self).output is Attention.output and self.adds_residual(T)
                 and K.leaves_scaled_ok(T, self.H * self.hd, self.rt.dtype, self.w_o))
 
+    def takes_halved(self, T: int) -> bool:
+        """Whether ``forward`` takes, for T tokens, rows that are pairs of halves too, and its first product reads those."""
+        cls = type(self)
+        return (cls.forward is Attention.forward and cls.project is Attention.project
+                and cls.project_rotate_write is Attention.project_rotate_write
+                and K.takes_halved(T, self.w_qkv.shape[1], self.rt.dtype, self.w_qkv))
+
     def project(self, x, ctx) -> torch.Tensor:
         """Stage 1: ``x`` [T, d] -> [T, (H + 2 KVH) * hd], the query heads, then the key heads, then the
         value heads, as projected."""
@@ -468,6 +497,12 @@ class SwiGLU(Part):
     def leaves_scaled(self, T: int) -> bool:
         return self.adds_residual(T) and K.leaves_scaled_ok(T, self.intermediate_size, self.rt.dtype, self.w_down)
 
+    def takes_halved(self, T: int) -> bool:
+        """Whether ``forward`` and ``hidden`` take, for T tokens, rows that are pairs of halves too, and the product reads those."""
+        cls = type(self)
+        return (cls.forward is SwiGLU.forward and cls.hidden is SwiGLU.hidden
+                and K.takes_halved(T, self.w_gate_up.shape[1], self.rt.dtype, self.w_gate_up))
+
     def hidden(self, x) -> torch.Tensor:
         """``silu(W_gate x) * (W_up x)``: what the down product takes (for a part that places that product's result itself)."""
         return K.linear_swiglu(x, self.w_gate_up)
@@ -536,7 +571,7 @@ class PreNormBlock(Block):
             if (carries is not None and getattr(norm, "takes_addends", False) and pending.dim() == 3
                     and pending.dtype == torch.float32 and carries(T, pending.shape[0])):
                 return prologue(h, pending)
-        return norm.forward(h, pending_for(norm, pending, self.rt.dtype))
+        return normed_rows(norm, h, pending_for(norm, pending, self.rt.dtype), (part,))
 
     @staticmethod
     def _deferred(norm, producer, consumer, T: int):

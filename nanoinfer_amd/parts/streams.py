@@ -93,6 +93,12 @@ class SquaredReluMLP(Part):
         self.w_down = rt.weight(names["down"], weights["down"])
         K.stream_lib()
 
+    def takes_halved(self, T: int) -> bool:
+        """Whether ``forward`` and ``hidden`` take, for T tokens, rows that are pairs of halves too, and the product reads those."""
+        cls = type(self)
+        return (cls.forward is SquaredReluMLP.forward and cls.hidden is SquaredReluMLP.hidden
+                and K.takes_halved(T, self.w_up.shape[1], self.rt.dtype, self.w_up))
+
     def hidden(self, x) -> torch.Tensor:
         """What the down product takes (for a part that places that product's result itself)."""
         return K.linear_relu2(x, self.w_up)

@@ -1,0 +1,87 @@
+"""The norm that leaves its rows as pairs of halves too (``ni_add_rmsnorm_halves``) against the norm and the pass over its rows, which
+it stands for, to the bit; and the products that read such rows."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def K():
+    from nanoinfer_amd import kernels
+    return kernels
+
+
+# one row and many; the fewest columns, every size of the workgroup, the most; widths that go the long way (no whole stages of 32
+# columns, too wide for the registers)
+@pytest.mark.parametrize("T,d", [(1, 32), (3, 512), (70, 544), (129, 1056), (130, 2048), (5, 4128), (2, 8192), (3, 2052), (2, 8224)])
+@pytest.mark.parametrize("addends", [None, 0, 1, 6])      # none, one [T, d], one and six [S, T, d]
+def test_rows_and_halves_are_those_of_the_two_passes(K, T, d, addends):
+    g = torch.Generator().manual_seed(T + d)
+    h = torch.randn(T, d, generator=g) * 2.0 ** torch.randint(-20, 20, (T, 1), generator=g)
+    w = torch.randn(d, generator=g)
+    if T > 2:
+        h[0] = 0.0                                         # a row of zeros, and rows that are no numbers
+        h[1, d - 1] = float("inf")
+        h[2, 0] = float("nan")
+    h, w = h.cuda(), w.cuda()
+    pending = None
+    if addends is not None:
+        pending = torch.randn(*((T, d) if addends == 0 else (addends, T, d)), generator=g).cuda()
+        if T > 2:
+            pending.view(-1, T, d)[:, 0] = 0.0
+    one, two = h.clone(), h.clone()
+    rows = K.add_rmsnorm(one, pending, w, 1e-5, torch.empty(T, d, device="cuda"))
+    planes, info = K.pair_rows(rows)
+    got = K.add_rmsnorm_halved(two, pending, w, 1e-5)
+    assert torch.equal(got.x.view(torch.int32), rows.view(torch.int32)) and torch.equal(one.view(torch.int32), two.view(torch.int32))
+    assert torch.equal(got.info, info)
+    finite = info[:, 1].cpu() >= 0                         # (the halves of a row with infinities are never read)
+    assert torch.equal(got.planes.view(torch.int32).view(T, -1)[finite], planes.view(torch.int32).view(T, -1)[finite])
+
+
+@pytest.mark.parametrize("T", [65, 600])       # (of [16384, 2048], from 65 rows on)
+def test_products_of_halved_rows_are_those_of_rows(K, T):
+    g = torch.Generator().manual_seed(T)
+    h, w = torch.randn(T, 2048, generator=g).cuda(), torch.ones(2048).cuda()
+    weight = K.Weight((torch.randn(16384, 2048, generator=g) / 45).cuda())
+    small = K.Weight((torch.randn(64, 2048, generator=g) / 45).cuda())       # goes to another product, which reads the rows
+    assert weight.pairs is not None and K.takes_halved(T, 2048, torch.float32, weight) and not K.takes_halved(T, 2048, torch.float32, small)
+    x = K.add_rmsnorm_halved(h, None, w, 1e-5)
+    for product in (K.linear, K.linear_swiglu, K.linear_relu2):
+        assert torch.equal(product(x, weight), product(x.x, weight))
+    assert torch.equal(K.linear(x, small), K.linear(x.x, small))
+
+
+def test_halved_rows_take_less_work_to_go_there(K):
+    g = torch.Generator().manual_seed(1)
+    weight = K.Weight((torch.randn(3072, 2048, generator=g) / 45).cuda())
+    x = K.add_rmsnorm_halved(torch.randn(164, 2048, generator=g).cuda(), None, torch.ones(2048, device="cuda"), 1e-5)
+    assert K.pair_wins(x, weight) and not K.pair_wins(x.x, weight)
+    assert torch.equal(K.linear(x, weight), K.pair_gemm(x.x, weight))
+
+
+def test_parts_say_which_rows_they_read(K):
+    """A layer that replaces a stage, and a part that knows nothing of halves, are given rows."""
+    from nanoinfer_amd.parts import standard
+
+    class Norm(standard.RMSNorm):
+        def forward(self, h, pending, rows=None):
+            return h
+
+    class Part:
+        pass
+
+    h = torch.zeros(600, 64, device="cuda")
+    norm = Norm.__new__(Norm)
+    norm.rt = type("Runtime", (), {"dtype": torch.float32})()
+    assert standard.normed_rows(norm, h, None, (Part(),)) is h
+    part = Part()
+    part.takes_halved = lambda T: True
+    assert standard.normed_rows(norm, h, None, (part,)) is h       # its forward is its own
+
+    class Projects(standard.Attention):
+        def project(self, x, ctx):
+            return None
+
+    assert not Projects.__new__(Projects).takes_halved(600)
