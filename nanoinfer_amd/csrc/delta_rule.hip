@@ -66,91 +66,145 @@ __device__ __forceinline__ float conv_at(const float* __restrict__ proj, const f
     return acc;
 }
 
-// One wavefront a unit of TOK tokens: nothing meets in LDS, and four tokens of a sequence read the rows that their filters share
-// once, all asked for together.  1,500 tokens of 16 heads of 128 (123 MB) took 65 us with a workgroup a token and unit, 43 now.
-template <int TOK>
-__global__ __launch_bounds__(256) void delta_prepare_kernel(const float* __restrict__ proj, const float* __restrict__ low,
+// A workgroup a token and unit, a thread a channel: for steps of few tokens, which wait for memory once and not once a group of
+// channels (twelve requests of 16 heads of 128 6.2 us, 9.3 by one wavefront a unit).
+__global__ void delta_prepare_token_kernel(const float* __restrict__ proj, const float* __restrict__ low,
                                      const float* __restrict__ conv, const float* __restrict__ a_log,
                                      const float* __restrict__ dt_bias, float* __restrict__ state,
                                      const int32_t* __restrict__ seq_of_token, const int32_t* __restrict__ q_start,
                                      const int32_t* __restrict__ state_slot, float* __restrict__ prep,
-                                     int T, int G, int H, int dk, int dv, int taps, int proj_cols, size_t state_stride,
+                                     int G, int H, int dk, int dv, int taps, int proj_cols, size_t state_stride,
                                      size_t conv_off, int log_decay, int move_on) {
+    __shared__ float scratch[16];
+    const int t = blockIdx.x, unit = blockIdx.y;
+    const int s = seq_of_token[t];
+    const int i = t - q_start[s];              // place of the token in its portion
+    const int QK = 2 * G * dk, C = QK + H * dv;
+    const int prep_cols = C + H + H * dk + H * dv;
+    float* hist = state + static_cast<size_t>(state_slot[s]) * state_stride + conv_off;
+    float* out = prep + static_cast<size_t>(t) * prep_cols;
+    // move_on: every sequence of the step brings one token, so the thread that has read a channel's last inputs is the
+    // only one that does, and moves them on itself (no kernel of its own for that)
+    auto moved = [&](int c) {
+        for (int j = 0; j + 2 < taps; ++j) hist[static_cast<size_t>(j) * C + c] = hist[static_cast<size_t>(j + 1) * C + c];
+        hist[static_cast<size_t>(taps - 2) * C + c] = proj[static_cast<size_t>(t) * proj_cols + c];
+    };
+    if (unit < 2 * G) {
+        // a head of q or of k: every thread keeps its channels (dk <= 256 = threads)
+        const int c = unit * dk + threadIdx.x;
+        float y = 0.f;
+        if (threadIdx.x < dk) {
+            const float z = conv_at(proj, hist, conv, t, i, c, C, taps, proj_cols);
+            y = silu_f(z);
+            if (move_on && taps > 1) moved(c);
+        }
+        const float ss = block_sum(y * y, scratch);
+        const float inv = (1.0f / sqrtf(ss + 1e-6f)) * (unit < G ? 1.0f / sqrtf(static_cast<float>(dk)) : 1.0f);
+        if (threadIdx.x < dk) out[c] = y * inv;
+        return;
+    }
+    const int h = unit - 2 * G;
+    const float* prow = proj + static_cast<size_t>(t) * proj_cols;
+    const float* lrow = low + static_cast<size_t>(t) * (H * dk + H * dv);
+    for (int j = threadIdx.x; j < dv; j += blockDim.x) {
+        const int c = QK + h * dv + j;
+        const float z = conv_at(proj, hist, conv, t, i, c, C, taps, proj_cols);
+        out[c] = silu_f(z);
+        if (move_on && taps > 1) moved(c);
+        out[C + H + H * dk + h * dv + j] = sigmoid_f(lrow[H * dk + h * dv + j]);
+    }
+    const float rate = expf(a_log[h]);
+    for (int j = threadIdx.x; j < dk; j += blockDim.x) {
+        const float z = lrow[h * dk + j] + dt_bias[h * dk + j];
+        const float lg = -rate * softplus_f(z);
+        out[C + H + h * dk + j] = log_decay ? lg : expf(lg);      // the chunked form sums logarithms
+    }
+    if (threadIdx.x == 0) out[C + h] = sigmoid_f(prow[C + h]);
+}
+
+// One wavefront a unit of four tokens: nothing meets in LDS, and four tokens of a sequence read the rows that their filters share
+// once, all asked for together.  1,500 tokens of 16 heads of 128 (123 MB) took 65 us with a workgroup a token and unit, 43 now.
+__global__ __launch_bounds__(256) void delta_prepare_kernel(const float* __restrict__ proj, const float* __restrict__ low,
+                                     const float* __restrict__ conv, const float* __restrict__ a_log,
+                                     const float* __restrict__ dt_bias, const float* __restrict__ state,
+                                     const int32_t* __restrict__ seq_of_token, const int32_t* __restrict__ q_start,
+                                     const int32_t* __restrict__ state_slot, float* __restrict__ prep,
+                                     int T, int G, int H, int dk, int dv, int taps, int proj_cols, size_t state_stride,
+                                     size_t conv_off, int log_decay) {
+    constexpr int TOK = 4;
     const int lane = threadIdx.x & (WAVE - 1), unit = blockIdx.y;
     const int QK = 2 * G * dk, C = QK + H * dv;
     const int prep_cols = C + H + H * dk + H * dv;
     const int first = (blockIdx.x * 4 + threadIdx.x / WAVE) * TOK;
-    if constexpr (TOK == 4) {
-        // four tokens of one sequence behind its first three, filters of four: the seven rows that they need, all asked for at once
-        if (first + 3 < T && taps == 4) {
-            const int s = __builtin_amdgcn_readfirstlane(seq_of_token[first]);
-            if (s == __builtin_amdgcn_readfirstlane(seq_of_token[first + 3]) && first - q_start[s] >= 3) {
-                const float* rows = proj + static_cast<size_t>(first) * proj_cols;
-                float* to = prep + static_cast<size_t>(first) * prep_cols;
-                const bool value = unit >= 2 * G;
-                const int h = unit - 2 * G, width = value ? dv : dk, c0 = value ? QK + h * dv : unit * dk;
-                auto filtered = [&](int c, float (&y)[4]) {
-                    float x[7], w[4];
+    // four tokens of one sequence behind its first three, filters of four: the seven rows that they need, all asked for at once
+    if (first + 3 < T && taps == 4) {
+        const int s = __builtin_amdgcn_readfirstlane(seq_of_token[first]);
+        if (s == __builtin_amdgcn_readfirstlane(seq_of_token[first + 3]) && first - q_start[s] >= 3) {
+            const float* rows = proj + static_cast<size_t>(first) * proj_cols;
+            float* to = prep + static_cast<size_t>(first) * prep_cols;
+            const bool value = unit >= 2 * G;
+            const int h = unit - 2 * G, width = value ? dv : dk, c0 = value ? QK + h * dv : unit * dk;
+            auto filtered = [&](int c, float (&y)[4]) {
+                float x[7], w[4];
 #pragma unroll
-                    for (int b = 0; b < 7; ++b) x[b] = rows[static_cast<ptrdiff_t>(b - 3) * proj_cols + c];
+                for (int b = 0; b < 7; ++b) x[b] = rows[static_cast<ptrdiff_t>(b - 3) * proj_cols + c];
 #pragma unroll
-                    for (int b = 0; b < 4; ++b) w[b] = conv[static_cast<size_t>(c) * 4 + b];
+                for (int b = 0; b < 4; ++b) w[b] = conv[static_cast<size_t>(c) * 4 + b];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        float acc = 0.f;
+                for (int j = 0; j < 4; ++j) {
+                    float acc = 0.f;
 #pragma unroll
-                        for (int b = 0; b < 4; ++b) acc += w[b] * x[j + b];
-                        y[j] = silu_f(acc);
-                    }
-                };
-                if (!value) {
-                    float y[4][4], ss[4] = {0.f, 0.f, 0.f, 0.f};
+                    for (int b = 0; b < 4; ++b) acc += w[b] * x[j + b];
+                    y[j] = silu_f(acc);
+                }
+            };
+            if (!value) {
+                float y[4][4], ss[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int b = 0; b < 4; ++b) {
-                        if (b * WAVE >= dk) break;
-                        const int at = lane + b * WAVE;
-                        filtered(c0 + min(at, dk - 1), y[b]);
+                for (int b = 0; b < 4; ++b) {
+                    if (b * WAVE >= dk) break;
+                    const int at = lane + b * WAVE;
+                    filtered(c0 + min(at, dk - 1), y[b]);
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) ss[j] += at < dk ? y[b][j] * y[b][j] : 0.f;
-                    }
+                    for (int j = 0; j < 4; ++j) ss[j] += at < dk ? y[b][j] * y[b][j] : 0.f;
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    ss[j] = (1.0f / sqrtf(wave_sum(ss[j]) + 1e-6f)) * (unit < G ? 1.0f / sqrtf(static_cast<float>(dk)) : 1.0f);
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        ss[j] = (1.0f / sqrtf(wave_sum(ss[j]) + 1e-6f)) * (unit < G ? 1.0f / sqrtf(static_cast<float>(dk)) : 1.0f);
-#pragma unroll
-                    for (int b = 0; b < 4; ++b)
-#pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            if (lane + b * WAVE < dk) to[static_cast<size_t>(j) * prep_cols + c0 + lane + b * WAVE] = y[b][j] * ss[j];
-                    return;
-                }
-                const int wide = H * dk + H * dv;
-                const float* lows = low + static_cast<size_t>(first) * wide;
-                for (int at = lane; at < width; at += WAVE) {
-                    float y[4], gate[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) gate[j] = lows[static_cast<size_t>(j) * wide + H * dk + h * dv + at];
-                    filtered(c0 + at, y);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        to[static_cast<size_t>(j) * prep_cols + c0 + at] = y[j];
-                        to[static_cast<size_t>(j) * prep_cols + C + H + H * dk + h * dv + at] = sigmoid_f(gate[j]);
-                    }
-                }
-                const float rate = expf(a_log[h]);
-                for (int at = lane; at < dk; at += WAVE) {
-                    float z[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) z[j] = lows[static_cast<size_t>(j) * wide + h * dk + at];
-                    const float bias = dt_bias[h * dk + at];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const float lg = -rate * softplus_f(z[j] + bias);
-                        to[static_cast<size_t>(j) * prep_cols + C + H + h * dk + at] = log_decay ? lg : expf(lg);
-                    }
-                }
-                if (lane < 4) to[static_cast<size_t>(lane) * prep_cols + C + h] = sigmoid_f(rows[static_cast<size_t>(lane) * proj_cols + C + h]);
+                        if (lane + b * WAVE < dk) to[static_cast<size_t>(j) * prep_cols + c0 + lane + b * WAVE] = y[b][j] * ss[j];
                 return;
             }
+            const int wide = H * dk + H * dv;
+            const float* lows = low + static_cast<size_t>(first) * wide;
+            for (int at = lane; at < width; at += WAVE) {
+                float y[4], gate[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) gate[j] = lows[static_cast<size_t>(j) * wide + H * dk + h * dv + at];
+                filtered(c0 + at, y);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    to[static_cast<size_t>(j) * prep_cols + c0 + at] = y[j];
+                    to[static_cast<size_t>(j) * prep_cols + C + H + H * dk + h * dv + at] = sigmoid_f(gate[j]);
+                }
+            }
+            const float rate = expf(a_log[h]);
+            for (int at = lane; at < dk; at += WAVE) {
+                float z[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) z[j] = lows[static_cast<size_t>(j) * wide + h * dk + at];
+                const float bias = dt_bias[h * dk + at];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float lg = -rate * softplus_f(z[j] + bias);
+                    to[static_cast<size_t>(j) * prep_cols + C + H + h * dk + at] = log_decay ? lg : expf(lg);
+                }
+            }
+            if (lane < 4) to[static_cast<size_t>(lane) * prep_cols + C + h] = sigmoid_f(rows[static_cast<size_t>(lane) * proj_cols + C + h]);
+            return;
         }
     }
     for (int j = 0; j < TOK; ++j) {
@@ -158,14 +212,8 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(const float* __restr
         if (t >= T) return;
         const int s = seq_of_token[t];
         const int i = t - q_start[s];              // place of the token in its portion
-        float* hist = state + static_cast<size_t>(state_slot[s]) * state_stride + conv_off;
+        const float* hist = state + static_cast<size_t>(state_slot[s]) * state_stride + conv_off;
         float* out = prep + static_cast<size_t>(t) * prep_cols;
-        // move_on: every sequence of the step brings one token, so the lane that has read a channel's last inputs is the
-        // only one that does, and moves them on itself (no kernel of its own for that)
-        auto moved = [&](int c) {
-            for (int b = 0; b + 2 < taps; ++b) hist[static_cast<size_t>(b) * C + c] = hist[static_cast<size_t>(b + 1) * C + c];
-            hist[static_cast<size_t>(taps - 2) * C + c] = proj[static_cast<size_t>(t) * proj_cols + c];
-        };
         if (unit < 2 * G) {
             // a head of q or of k: every lane keeps its channels (dk <= 256)
             float y[4], ss = 0.f;
@@ -176,7 +224,6 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(const float* __restr
                 if (at < dk) {
                     const int c = unit * dk + at;
                     y[b] = silu_f(conv_at(proj, hist, conv, t, i, c, C, taps, proj_cols));
-                    if (move_on && taps > 1) moved(c);
                 }
                 ss += y[b] * y[b];
             }
@@ -193,7 +240,6 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(const float* __restr
         for (int at = lane; at < dv; at += WAVE) {
             const int c = QK + h * dv + at;
             out[c] = silu_f(conv_at(proj, hist, conv, t, i, c, C, taps, proj_cols));
-            if (move_on && taps > 1) moved(c);
             out[C + H + H * dk + h * dv + at] = sigmoid_f(lrow[H * dk + h * dv + at]);
         }
         const float rate = expf(a_log[h]);
@@ -635,14 +681,20 @@ NI_EXPORT int ni_delta_prepare(const void* proj, const void* low, const void* co
     if (dk != KPT * PARTS) return -1;
     const int C = 2 * G * dk + H * dv;
     if (dk > 256) return -2;
-    // a wavefront takes four tokens one after the other where that still fills the chip
-    const int tok = T >= 256 ? 4 : 1;
-    auto kernel = tok == 4 ? delta_prepare_kernel<4> : delta_prepare_kernel<1>;
-    kernel<<<dim3((T + 4 * tok - 1) / (4 * tok), 2 * G + H), 256, 0, stream>>>((const float*)proj, (const float*)low, (const float*)conv,
-                                                  (const float*)a_log, (const float*)dt_bias, (float*)state,
+    if (T >= 256 && !move_on) {                 // a wavefront takes four tokens where that still fills the chip
+        delta_prepare_kernel<<<dim3((T + 15) / 16, 2 * G + H), 256, 0, stream>>>((const float*)proj, (const float*)low, (const float*)conv,
+                                                  (const float*)a_log, (const float*)dt_bias, (const float*)state,
                                                   (const int32_t*)seq_of_token, (const int32_t*)q_start,
                                                   (const int32_t*)state_slot, (float*)prep, T, G, H, dk, dv, taps, proj_cols,
+                                                  state_stride, conv_off, log_decay);
+    } else {
+        const int widest = std::max(dk, std::min(dv, 256));
+        delta_prepare_token_kernel<<<dim3(T, 2 * G + H), (widest + 63) / 64 * 64, 0, stream>>>((const float*)proj, (const float*)low, (const float*)conv,
+                                                  (const float*)a_log, (const float*)dt_bias, (float*)state,
+                                                  (const int32_t*)seq_of_token, (const int32_t*)q_start,
+                                                  (const int32_t*)state_slot, (float*)prep, G, H, dk, dv, taps, proj_cols,
                                                   state_stride, conv_off, log_decay, move_on);
+    }
     if (taps > 1 && !move_on) {
         dim3 grid(B, std::max(1, std::min(64, (C + 255) / 256)));
         conv_state_update_kernel<<<grid, 256, 0, stream>>>((const float*)proj, (float*)state, (const int32_t*)q_start,
