@@ -899,10 +899,15 @@ bias_attention_mfma_kernel(const T* __restrict__ qkv, int row_stride, const T* _
 //   O^T[dim, row] += V^T . P^T   over 32 keys at a time: the k index of a lane's eight numbers is key 4 kg + e of either
 //                    sixteen, where its own scores are; V^T is read from the tile [key][channel] by transposing reads
 //
-// A workgroup asks for the next tile's keys and values before it works on this one.  KQ: 32-channel pieces of a key, DVB:
-// blocks of 16 value channels, at most; the registers are held to what lets two to four wavefronts share a SIMD, where the
-// sizes allow (left alone the compiler takes accumulation registers besides, and one wavefront fewer fits: 176 instead of
-// 128 us at keys of 64 and values of 128 channels).
+// A workgroup asks for the next tile's keys and values before it works on this one, and for the pages of the tile behind that;
+// pieces without a row become zeros when they are put into LDS (where they are asked for it would wait for all of them).  What
+// bounds it is the chain of instructions of a wavefront (scores, maximum, exponentials, products), so nothing in it branches between
+// blocks of channels or keys: their reads and products overlap.  KQ: 32-channel pieces of a key, DVB: blocks of 16 value channels,
+// at most; the registers are held to what lets two or three wavefronts share a SIMD without spills, where the sizes allow (keys of
+// 64 and values of 128 channels: two a SIMD 60.6 us, three with 12 spilled registers 65.5).  Measured with pages looked up, divided
+// and waited for between the tiles : now (us): 2,045 tokens, keys of 64 and values of 128 channels, 32 heads on 8 of two maps, capped,
+// in chunks of 1,024 124 : 62; 512 of them 65 : 36; 1,500 tokens, 32 heads of 64 on 8 with a bias 122 : 55, 512 of them 104 : 48; 2,000
+// tokens, 16 heads of 128 on 4 164 : 89, with a window of 512 63 : 43; 1,000 tokens, keys of 192, 16 heads 123 : 60; 96 / 160 81 : 69.
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef short shortx4_t __attribute__((ext_vector_type(4)));
 #define TILE_PAD 8             // elements of padding of a staged row: the rows of a read fall on different banks
@@ -917,8 +922,8 @@ __device__ __forceinline__ bf16x8_t read_values_t(const uint16_t* tile, int row_
     return __builtin_bit_cast(bf16x8_t, make_uint4(a.x, a.y, b.x, b.y));
 }
 
-template <int KQ, int DVB>
-__global__ void __launch_bounds__(WAVES * WAVE, KQ > 4 ? 1 : DVB == 4 ? 4 - KQ / 4 : DVB == 8 ? 3 : 2)
+template <int KQ, int DVB, bool POW2>
+__global__ void __launch_bounds__(WAVES * WAVE, KQ > 4 ? 1 : DVB == 4 ? 3 : 2)
 bias_attention_bf16_kernel(const bf16_t* __restrict__ qkv, int row_stride, const bf16_t* __restrict__ kpool, const bf16_t* __restrict__ vpool,
                            const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ tiles,
                            const int32_t* __restrict__ positions, const float* __restrict__ bias, int distances, bf16_t* __restrict__ out,
@@ -929,7 +934,8 @@ bias_attention_bf16_kernel(const bf16_t* __restrict__ qkv, int row_stride, const
     constexpr int KROW = 32 * KQ + TILE_PAD, VROW = 16 * DVB + TILE_PAD, VP = DVB / 2;
     __shared__ __attribute__((aligned(16))) uint16_t Ks[KEYS * KROW];
     __shared__ __attribute__((aligned(16))) uint16_t Vs[KEYS * VROW];
-    const int tile = blockIdx.x, g = blockIdx.y, chunk = blockIdx.z;
+    // kv heads fastest: the longest tiles of all heads start first, and with eight heads each has the L2 of one die
+    const int tile = blockIdx.x / G, g = blockIdx.x - tile * G, chunk = blockIdx.z;
     const int seq = tiles[4 * tile], first_row = tiles[4 * tile + 1], n_tok = tiles[4 * tile + 2];
     const int first_pos = positions[first_row];
     const int group = H / G;
@@ -949,8 +955,9 @@ bias_attention_bf16_kernel(const bf16_t* __restrict__ qkv, int row_stride, const
     const int lo = first_seen(pos, window, form.chunk);
     const int steps = temp_every > 0 ? (pos + 1) / temp_every : 0;
     const float factor = scale * (1.0f + temp_coef * logf(static_cast<float>(steps) + 1.0f));
-    // a capped score, in units of log2: cap log2e tanh(s / cap) = c - 2 c / (2^(s 2 log2e / cap) + 1)
-    const float cap2 = form.softcap * LOG2E, cap_in = form.softcap > 0.f ? 2.0f * LOG2E / form.softcap : 0.f;
+    // scores in units of log2; a capped one: cap log2e tanh(s / cap) = c - 2 c / (2^(s 2 log2e / cap) + 1)
+    const float cap2 = form.softcap * LOG2E, unit = form.softcap > 0.f ? 2.0f * LOG2E / form.softcap : LOG2E;
+    const float factor2 = factor * unit;
     uint4 qf[KQ];
 #pragma unroll
     for (int kk = 0; kk < KQ; ++kk) {
@@ -963,7 +970,7 @@ bias_attention_bf16_kernel(const bf16_t* __restrict__ qkv, int row_stride, const
     const int wave_first = first_pos + (wave * 16) / heads_here;
     const int wave_last = wave_rows > 0 ? first_pos + (wave * 16 + wave_rows - 1) / heads_here : -1;
     const int wave_lo = first_seen(wave_last, window, form.chunk);
-    float m = -INFINITY, l = 0.f;                 // the maximum in units of log2
+    float m = -INFINITY, l_lane = 0.f;            // the row's reference in units of log2; the sum of this lane's own weights
     floatx4_t acc[DVB];
 #pragma unroll
     for (int db = 0; db < DVB; ++db) acc[db] = floatx4_t{0.f, 0.f, 0.f, 0.f};
@@ -971,68 +978,102 @@ bias_attention_bf16_kernel(const bf16_t* __restrict__ qkv, int row_stride, const
     const int last_pos = first_pos + n_tok - 1;
     const int32_t* table = block_table + static_cast<size_t>(seq) * table_width;
     const int k_pieces = dk / 8, v_pieces = dv / 8;
+    const int shift = __builtin_ctz(page_size);
+    auto page_of = [&](int key) { return POW2 ? key >> shift : key / page_size; };
+    auto slot_of = [&](int key) { return POW2 ? key & (page_size - 1) : key % page_size; };
+    // a piece is eight numbers of a row: piece u of this thread is piece `c` of key `j` of a tile, the same in every tile
     uint4 kr[KQ], vr[VP];
-    auto ask_pool = [&](const bf16_t* pool, int pieces, int row_elems, int k0, auto& regs, auto count) {
+    int k_at[KQ], v_at[VP], k_page[KQ], v_page[VP];      // j << 16 | 8 c
+    uint32_t k_none = 0u, v_none = 0u;            // the pieces of the tile in kr and vr that have no row: zeros
+    auto place = [&](int pieces, auto& at) {
 #pragma unroll
-        for (int u = 0; u < decltype(count)::value; ++u) {
-            const int idx = u * (WAVES * WAVE) + tid, j = idx / pieces, key = k0 + j;
-            regs[u] = make_uint4(0u, 0u, 0u, 0u);
-            if (j < KEYS && key <= last_pos) {
-                const int page = table[key / page_size];
-                if (page >= 0)
-                    regs[u] = *reinterpret_cast<const uint4*>(pool + ((static_cast<size_t>(page) * kv_heads + kv) * page_size + key % page_size) *
-                                                                         row_elems + (idx - j * pieces) * 8);
-            }
-        }
-    };
-    auto put_tile = [&](uint16_t* dst, int row_elems, int pieces, const auto& regs, auto count) {
-#pragma unroll
-        for (int u = 0; u < decltype(count)::value; ++u) {
+        for (int u = 0; u < static_cast<int>(sizeof(at) / sizeof(int)); ++u) {
             const int idx = u * (WAVES * WAVE) + tid, j = idx / pieces;
-            if (j < KEYS) *reinterpret_cast<uint4*>(dst + j * row_elems + (idx - j * pieces) * 8) = regs[u];
+            at[u] = j << 16 | (idx - j * pieces) * 8;
         }
     };
-    using KCount = std::integral_constant<int, KQ>;
-    using VCount = std::integral_constant<int, VP>;
+    // the pages of the thread's pieces (-1: no row to read), then the pieces themselves
+    auto look_up = [&](int k0, const auto& at, auto& pages) {
+#pragma unroll
+        for (int u = 0; u < static_cast<int>(sizeof(pages) / sizeof(int)); ++u) {
+            const int j = at[u] >> 16, key = k0 + j;
+            pages[u] = table[page_of(std::min(key, last_pos))];
+            if (j >= KEYS || key > last_pos) pages[u] = -1;
+        }
+    };
+    auto ask = [&](const bf16_t* pool, int row_elems, int k0, const auto& at, const auto& pages, uint32_t& none, auto& regs) {
+        none = 0u;
+#pragma unroll
+        for (int u = 0; u < static_cast<int>(sizeof(pages) / sizeof(int)); ++u) {
+            const int key = std::min(k0 + (at[u] >> 16), last_pos);
+            const size_t row = (static_cast<size_t>(std::max(pages[u], 0)) * kv_heads + kv) * page_size + slot_of(key);
+            regs[u] = *reinterpret_cast<const uint4*>(pool + row * row_elems + (at[u] & 0xffff));
+            none |= pages[u] < 0 ? 1u << u : 0u;
+        }
+    };
+    auto put = [&](uint16_t* dst, int row_elems, const auto& at, uint32_t none, auto& regs) {
+        if (__any(none != 0u)) {                  // (not where they are asked for: that would wait for them)
+#pragma unroll
+            for (int u = 0; u < static_cast<int>(sizeof(regs) / sizeof(uint4)); ++u)
+                if (none >> u & 1u) regs[u] = make_uint4(0u, 0u, 0u, 0u);
+        }
+#pragma unroll
+        for (int u = 0; u < static_cast<int>(sizeof(regs) / sizeof(uint4)); ++u)
+            if (at[u] >> 16 < KEYS) *reinterpret_cast<uint4*>(dst + (at[u] >> 16) * row_elems + (at[u] & 0xffff)) = regs[u];
+    };
     if (dk < 32 * KQ) {                           // the channels that no key has meet zeros of the queries: they must be numbers
         for (int e = tid; e < KEYS * (32 * KQ - dk); e += WAVES * WAVE) Ks[e / (32 * KQ - dk) * KROW + dk + e % (32 * KQ - dk)] = 0;
     }
     const KeyWalk walk(first_pos, last_pos, window, keep_first, form.chunk);
-    ask_pool(kpool, k_pieces, k_row, walk.first_key(0), kr, KCount{});
-    ask_pool(vpool, v_pieces, dv, walk.first_key(0), vr, VCount{});
+    place(k_pieces, k_at);
+    place(v_pieces, v_at);
+    look_up(walk.first_key(0), k_at, k_page);
+    look_up(walk.first_key(0), v_at, v_page);
+    ask(kpool, k_row, walk.first_key(0), k_at, k_page, k_none, kr);
+    ask(vpool, dv, walk.first_key(0), v_at, v_page, v_none, vr);
+    look_up(walk.first_key(1), k_at, k_page);
+    look_up(walk.first_key(1), v_at, v_page);
     for (int v = 0; v < walk.steps; ++v) {
         const int k0 = walk.first_key(v);
         __syncthreads();                          // the tile before this one has been used by everyone
-        put_tile(Ks, KROW, k_pieces, kr, KCount{});
-        put_tile(Vs, VROW, v_pieces, vr, VCount{});
+        put(Ks, KROW, k_at, k_none, kr);
+        put(Vs, VROW, v_at, v_none, vr);
         __syncthreads();
         if (v + 1 < walk.steps) {
-            ask_pool(kpool, k_pieces, k_row, walk.first_key(v + 1), kr, KCount{});
-            ask_pool(vpool, v_pieces, dv, walk.first_key(v + 1), vr, VCount{});
+            ask(kpool, k_row, walk.first_key(v + 1), k_at, k_page, k_none, kr);
+            ask(vpool, dv, walk.first_key(v + 1), v_at, v_page, v_none, vr);
+            look_up(walk.first_key(v + 2), k_at, k_page);
+            look_up(walk.first_key(v + 2), v_at, v_page);
         }
         if (k0 > wave_last) continue;             // nothing here for this wavefront's rows (it still stages and waits)
+        float near[KEYS / 4];
+        if (bias) {
+#pragma unroll
+            for (int e = 0; e < KEYS / 4; ++e) {
+                const int back = std::min(std::max(pos - (k0 + 16 * (e / 4) + 4 * kg + e % 4), 0), distances - 1);
+                near[e] = bias[static_cast<size_t>(back) * H + head];
+            }
+        }
         floatx4_t sc[KEYS / 16];
 #pragma unroll
-        for (int j = 0; j < KEYS / 16; ++j) {
-            sc[j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < KEYS / 16; ++j) sc[j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int kk = 0; kk < KQ; ++kk)
-                if (32 * kk < dk)
+        for (int kk = 0; kk < KQ; ++kk)
+            if (kk < 2 || 64 * (kk / 2) < dk) {
+#pragma unroll
+                for (int j = 0; j < KEYS / 16; ++j)
                     sc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                         __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(Ks + (16 * j + i) * KROW + 32 * kk + 8 * kg)),
                         __builtin_bit_cast(bf16x8_t, qf[kk]), sc[j], 0, 0, 0);
-        }
+            }
         float top = -INFINITY;
 #pragma unroll
         for (int j = 0; j < KEYS / 16; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                float s = sc[j][r] * factor;
-                if (bias) {
-                    const int back = std::min(std::max(pos - (k0 + 16 * j + 4 * kg + r), 0), distances - 1);
-                    s += bias[static_cast<size_t>(back) * H + head];
-                }
-                s = form.softcap > 0.f ? cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(s * cap_in) + 1.0f) : s * LOG2E;
+                float s = sc[j][r] * factor2;
+                if (bias) s = fmaf(near[4 * j + r], unit, s);
+                if (form.softcap > 0.f) s = cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(s) + 1.0f);
                 sc[j][r] = s;
             }
         if (k0 + KEYS - 1 > wave_first || k0 < wave_lo) {      // some row of this wavefront does not see every key of the tile
@@ -1046,42 +1087,51 @@ bias_attention_bf16_kernel(const bf16_t* __restrict__ qkv, int row_stride, const
         for (int j = 0; j < KEYS / 16; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) top = fmaxf(top, sc[j][r]);
-        top = groups4(top, true);
-        const float m_new = fmaxf(m, top);
-        const float m_ref = m_new > -INFINITY ? m_new : 0.f;   // a row whose keys all lie elsewhere: weights 2^-inf = 0
-        const float alpha = __builtin_amdgcn_exp2f(m - m_ref); // 0 at the row's first keys
-        float sum = 0.f;
+        if (__any(top > m)) {                     // a row's maximum rose: rescale what was summed (its largest weight is 1, which is exact in halves)
+            const float m_new = fmaxf(m, groups4(top, true));
+            const float alpha = m_new > m ? __builtin_amdgcn_exp2f(m - m_new) : 1.f;      // 0 at the row's first keys
+            m = m_new;
+            l_lane *= alpha;
+#pragma unroll
+            for (int db = 0; db < DVB; ++db) acc[db] *= alpha;
+        }
+        const float m_ref = m > -INFINITY ? m : 0.f;           // a row whose keys all lie elsewhere: weights 2^-inf = 0
         uint32_t hi[KEYS / 16][2], rest[KEYS / 16][2];         // the weights of a sixteen as pairs: upper halves, what they leave
 #pragma unroll
         for (int j = 0; j < KEYS / 16; ++j)
 #pragma unroll
             for (int r = 0; r < 4; r += 2) {
                 const float p0 = __builtin_amdgcn_exp2f(sc[j][r] - m_ref), p1 = __builtin_amdgcn_exp2f(sc[j][r + 1] - m_ref);
-                sum += p0 + p1;
+                l_lane += p0 + p1;
                 const uint32_t u0 = __float_as_uint(p0), u1 = __float_as_uint(p1);
                 hi[j][r / 2] = (u0 >> 16) | (u1 & 0xffff0000u);
                 rest[j][r / 2] = pack_bf16x2(p0 - __uint_as_float(u0 & 0xffff0000u), p1 - __uint_as_float(u1 & 0xffff0000u));
             }
-        l = l * alpha + groups4(sum, false);
-        m = m_new;
-        const bool moved = __any(alpha != 1.f);                // no row's maximum rose: the sums stay as they are
+        // four blocks of channels at a time, no branch between them: their chains of products and reads overlap (what a block
+        // past the last channel multiplies stays in its own sums, which nobody stores)
 #pragma unroll
-        for (int db = 0; db < DVB; ++db) {
-            if (db < dvb) {
-                floatx4_t a = acc[db];
-                if (moved) a = a * alpha;
+        for (int d4 = 0; d4 < DVB; d4 += 4) {
+            if (d4 == 0 || d4 < dvb) {
 #pragma unroll
                 for (int jj = 0; jj < KEYS / 32; ++jj) {
-                    const bf16x8_t vt = read_values_t(Vs + 32 * jj * VROW, VROW, 16 * db, i, kg);
-                    a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        vt, __builtin_bit_cast(bf16x8_t, make_uint4(hi[2 * jj][0], hi[2 * jj][1], hi[2 * jj + 1][0], hi[2 * jj + 1][1])), a, 0, 0, 0);
-                    a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        vt, __builtin_bit_cast(bf16x8_t, make_uint4(rest[2 * jj][0], rest[2 * jj][1], rest[2 * jj + 1][0], rest[2 * jj + 1][1])), a, 0, 0, 0);
+                    bf16x8_t vt[4];
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) vt[d] = read_values_t(Vs + 32 * jj * VROW, VROW, 16 * (d4 + d), i, kg);
+#pragma unroll
+                    for (int d = 0; d < 4; ++d)
+                        acc[d4 + d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            vt[d], __builtin_bit_cast(bf16x8_t, make_uint4(hi[2 * jj][0], hi[2 * jj][1], hi[2 * jj + 1][0], hi[2 * jj + 1][1])),
+                            acc[d4 + d], 0, 0, 0);
+#pragma unroll
+                    for (int d = 0; d < 4; ++d)
+                        acc[d4 + d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            vt[d], __builtin_bit_cast(bf16x8_t, make_uint4(rest[2 * jj][0], rest[2 * jj][1], rest[2 * jj + 1][0], rest[2 * jj + 1][1])),
+                            acc[d4 + d], 0, 0, 0);
                 }
-                acc[db] = a;
             }
         }
     }
+    const float l = groups4(l_lane, false);
     if (!valid) return;
     if (partial) {              // an unfinished row, as a run of one
         float* prow = partial + (static_cast<size_t>(first_row + token) * H + head) * (dv + 2);
@@ -1219,7 +1269,8 @@ bias_attention_parts_kernel(const float* __restrict__ qkv, int row_stride, const
         }
     };
     struct Piece { float4 a, b; };
-    auto ask = [&](const float* pool, int pieces, int row_elems, int k0, const auto& pages, auto& regs) {
+    auto ask = [&](const float* pool, int pieces, int row_elems, int k0, const auto& pages, uint32_t& none, auto& regs) {
+        none = 0u;
 #pragma unroll
         for (int u = 0; u < static_cast<int>(sizeof(pages) / sizeof(int)); ++u) {
             const int idx = u * THREADS + tid, j = idx / pieces, key = std::min(k0 + j, last_pos);
@@ -1227,10 +1278,15 @@ bias_attention_parts_kernel(const float* __restrict__ qkv, int row_stride, const
                                 (idx - j * pieces) * 8;
             regs[u].a = *reinterpret_cast<const float4*>(from);
             regs[u].b = *reinterpret_cast<const float4*>(from + 4);
-            if (pages[u] < 0) regs[u].a = regs[u].b = make_float4(0.f, 0.f, 0.f, 0.f);
+            none |= pages[u] < 0 ? 1u << u : 0u;
         }
     };
-    auto put = [&](auto& dst, int pieces, const auto& regs) {
+    auto put = [&](auto& dst, int pieces, uint32_t none, auto& regs) {
+        if (__any(none != 0u)) {                  // (not where they are asked for: that would wait for them)
+#pragma unroll
+            for (int u = 0; u < static_cast<int>(sizeof(regs) / sizeof(Piece)); ++u)
+                if (none >> u & 1u) regs[u].a = regs[u].b = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
 #pragma unroll
         for (int u = 0; u < static_cast<int>(sizeof(regs) / sizeof(Piece)); ++u) {
             const int idx = u * THREADS + tid, j = idx / pieces;
@@ -1251,21 +1307,22 @@ bias_attention_parts_kernel(const float* __restrict__ qkv, int row_stride, const
     auto first_key = [&](int v) { return walk.first_key(v >> 1) + (v & 1) * PART_KEYS; };
     int k_page[KC], v_page[VC];
     Piece kr[KC], vr[VC];
+    uint32_t k_none = 0u, v_none = 0u;            // the pieces in kr and vr that have no row: zeros
     look_up(first_key(0), k_pieces, k_page);
     look_up(first_key(0), v_pieces, v_page);
-    ask(keys, k_pieces, k_row, first_key(0), k_page, kr);
-    ask(vpool, v_pieces, dv, first_key(0), v_page, vr);
+    ask(keys, k_pieces, k_row, first_key(0), k_page, k_none, kr);
+    ask(vpool, v_pieces, dv, first_key(0), v_page, v_none, vr);
     look_up(first_key(1), k_pieces, k_page);
     look_up(first_key(1), v_pieces, v_page);
     for (int v = 0; v < count; ++v) {
         const int k0 = first_key(v);
         __syncthreads();                          // the keys before these have been used by everyone
-        put(at.k, k_pieces, kr);
-        put(at.v, v_pieces, vr);
+        put(at.k, k_pieces, k_none, kr);
+        put(at.v, v_pieces, v_none, vr);
         __syncthreads();
         if (v + 1 < count) {
-            ask(keys, k_pieces, k_row, first_key(v + 1), k_page, kr);
-            ask(vpool, v_pieces, dv, first_key(v + 1), v_page, vr);
+            ask(keys, k_pieces, k_row, first_key(v + 1), k_page, k_none, kr);
+            ask(vpool, v_pieces, dv, first_key(v + 1), v_page, v_none, vr);
             if (v + 2 < count) {
                 look_up(first_key(v + 2), k_pieces, k_page);
                 look_up(first_key(v + 2), v_pieces, v_page);
@@ -1325,15 +1382,20 @@ bias_attention_parts_kernel(const float* __restrict__ qkv, int row_stride, const
             l_lane += w[e];
         }
         const Parts pf = parts8(w);
+        // two blocks of channels at a time, no branch between them: their chains of products and reads overlap
 #pragma unroll
-        for (int db = 0; db < DVB; ++db) {
-            if (db < dvb) {
-                bf16x8_t vf[3];
+        for (int d2 = 0; d2 < DVB; d2 += 2) {
+            if (d2 < dvb) {
+                bf16x8_t vf[2][3];
 #pragma unroll
-                for (int p = 0; p < 3; ++p) vf[p] = read_values_t(&at.v[p][0][0], 16 * DVB + TILE_PAD, 16 * db, i, kg);
+                for (int d = 0; d < 2; ++d)
+#pragma unroll
+                    for (int p = 0; p < 3; ++p) vf[d][p] = read_values_t(&at.v[p][0][0], 16 * DVB + TILE_PAD, 16 * (d2 + d), i, kg);
 #pragma unroll
                 for (int n = 0; n < 6; ++n)
-                    acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[PART_A[n]], __builtin_bit_cast(bf16x8_t, pf.p[PART_B[n]]), acc[db], 0, 0, 0);
+#pragma unroll
+                    for (int d = 0; d < 2; ++d)
+                        acc[d2 + d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[d][PART_A[n]], __builtin_bit_cast(bf16x8_t, pf.p[PART_B[n]]), acc[d2 + d], 0, 0, 0);
             }
         }
     }
@@ -1855,7 +1917,8 @@ static hipError_t launch_mfma(const MfmaArgs& a, dim3 grid, size_t lds, hipStrea
 
 template <int KQ, int DVB>
 static void launch_bf16(const MfmaArgs& a, dim3 grid, hipStream_t stream) {
-    bias_attention_bf16_kernel<KQ, DVB><<<grid, WAVES * WAVE, 0, stream>>>(
+    auto kernel = (a.page_size & (a.page_size - 1)) == 0 ? bias_attention_bf16_kernel<KQ, DVB, true> : bias_attention_bf16_kernel<KQ, DVB, false>;
+    kernel<<<dim3(grid.x * grid.y, 1, grid.z), WAVES * WAVE, 0, stream>>>(
         (const bf16_t*)a.qkv, a.row_stride, (const bf16_t*)a.kpool, (const bf16_t*)a.vpool, (const int32_t*)a.block_table, a.table_width,
         (const int32_t*)a.tiles, (const int32_t*)a.positions, (const float*)a.bias, a.distances, (bf16_t*)a.out, a.H, a.G, a.dk, a.dv,
         a.page_size, a.scale, a.temp_coef, a.temp_every, a.heads_per_chunk, a.window, a.keep_first, a.out_scale, (const float*)a.sink, a.form,
