@@ -164,8 +164,15 @@ __device__ __forceinline__ floatx4_t row_sum_step(const uint4& pf, floatx4_t l) 
 // (Where the registers allow two wavefronts a SIMD, asking for them also makes the compiler keep the
 // accumulators in ordinary vector registers: with a whole register file to itself it parks them in
 // the accumulation registers, which the vector unit cannot multiply, and copies them to and fro.)
-template <int CB, bool POW2>
-__global__ __launch_bounds__(MA_WAVES * WAVE) __attribute__((amdgpu_waves_per_eu(HEAD_DIM * CB <= 128 ? 2 : 1)))
+//
+// GROUPS = 2: eight wavefronts, two groups of four, own one tile; each group walks one half of the tile's
+// steps with staged tiles of its own, and the second hands its (maximum, sum, output) to the first through
+// LDS.  A wavefront alone on a SIMD waits for LDS and its own chain of instructions (0.6 us for a step of
+// 32 keys, two blocks of rows, head size 64; two together take 0.73), and the last tiles of a prompt, its
+// longest, used to run alone.  2,048 tokens at 2,048 keys, 32 heads on 8: 42.6 -> 39.4 us, of which 33 pairs
+// of steps are 24 and the start and end of two tiles 14; 512 at 2,048 28.3 -> 23.4, 1,700 at 1,700 54.3 -> 39.6.
+template <int CB, bool POW2, int GROUPS>
+__global__ __launch_bounds__(GROUPS * MA_WAVES * WAVE) __attribute__((amdgpu_waves_per_eu(HEAD_DIM * CB <= 128 ? 2 : 1)))
 void mfma_attention_kernel(
     const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ kpool, const bf16_t* __restrict__ vpool,
     const int32_t* __restrict__ block_table, int table_stride, const QTile* __restrict__ tiles,
@@ -178,8 +185,14 @@ void mfma_attention_kernel(
     constexpr int DT = HD / 16;              // 16-wide tiles of the head dimension in the output
     constexpr int VROW = HD + VPAD;
     constexpr int KROW = HD + KPAD;
-    __shared__ __attribute__((aligned(16))) uint16_t ksm[2][KSTEP][KROW];  // K of a step: [key][dim]
-    __shared__ __attribute__((aligned(16))) uint16_t vs[2][KSTEP][VROW];   // V of a step, as it lies in the cache: [key][dim]
+    __shared__ __attribute__((aligned(16))) uint16_t ksm_all[GROUPS][2][KSTEP][KROW];  // K of a step: [key][dim]
+    __shared__ __attribute__((aligned(16))) uint16_t vs_all[GROUPS][2][KSTEP][VROW];   // V of a step, as it lies in the cache: [key][dim]
+    // what the second group hands over, as its lanes hold it: the same lane of the first group takes it
+    __shared__ __attribute__((aligned(16))) floatx4_t meet_o[GROUPS > 1 ? MA_WAVES * CB * DT : 1][WAVE];
+    __shared__ float2 meet_ml[GROUPS > 1 ? MA_WAVES * CB : 1][WAVE];
+    const int group = GROUPS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / MA_THREADS) : 0;
+    auto& ksm = ksm_all[group];
+    auto& vs = vs_all[group];
 
     // The launch has as many workgroups as the chip holds at once, and the tiles come sorted by the
     // number of keys they have to walk, longest first.  Workgroup w takes tiles w, 2P-1-w, 2P+w, ...
@@ -200,7 +213,7 @@ void mfma_attention_kernel(
         const int g = blockIdx.y / chunks;
         const int chunk = blockIdx.y % chunks;
 
-        const int tid = threadIdx.x;
+        const int tid = threadIdx.x % MA_THREADS;                 // within the group
         const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;      // the same in every lane: say so
         const int r = lane % 16, kg = lane / 16;
 
@@ -230,11 +243,15 @@ void mfma_attention_kernel(
         const int kend = tile.pos0 + tile.ntok;
         const int kbeg = (window > 0 ? max(0, tile.pos0 + 1 - window) : 0) / KSTEP * KSTEP;
         const int nsteps_all = (kend - kbeg + KSTEP - 1) / KSTEP;
-        // a split (blockIdx.z) takes a contiguous run of steps
+        // a split (blockIdx.z) takes a contiguous run of steps, a group its half of the run.  All groups pass the same
+        // number of barriers: `nsteps` is the first group's count, `own` this one's, which may be less or none (such a
+        // group looks at the addresses of the last step, where there are keys, and multiplies nothing).
         const int per_split = (nsteps_all + nsplit - 1) / nsplit;
-        const int s_begin = blockIdx.z * per_split;
-        const int nsteps = max(0, min(nsteps_all, s_begin + per_split) - s_begin);
-        const int kfirst = kbeg + s_begin * KSTEP;
+        const int run_begin = blockIdx.z * per_split;
+        const int run_end = max(run_begin, min(nsteps_all, run_begin + per_split));
+        const int nsteps = (run_end - run_begin + GROUPS - 1) / GROUPS;
+        const int s_begin = run_begin + group * nsteps;
+        const int own = max(0, min(run_end, s_begin + nsteps) - s_begin);
         const float scale2 = scale * LOG2E;
 
         const int32_t* table = block_table + static_cast<size_t>(tile.seq) * table_stride;
@@ -245,7 +262,8 @@ void mfma_attention_kernel(
         // inside the loop would have to be waited for before its rows can be asked for, and that
         // wait, being in order, would drain every row load still in flight.
         constexpr int TBL_MAX = 1024;
-        __shared__ __attribute__((aligned(16))) int32_t tbl[TBL_MAX];
+        __shared__ __attribute__((aligned(16))) int32_t tbl_all[GROUPS][TBL_MAX];
+        int32_t* tbl = tbl_all[group];
         int key_lo = 0, key_hi = 0, lp0 = 0;              // keys of the current segment, and its first page
         // the first key any row of the tile may read: keys before it (the steps start at a multiple of
         // KSTEP) may lie in pages that a window has passed and given back, and are never loaded
@@ -332,10 +350,12 @@ void mfma_attention_kernel(
         u32x4_t kr[DEPTH][PER_THREAD];
         u32x4_t vr[DEPTH][PER_THREAD];
         for (int seg0 = 0; seg0 < nsteps;) {
-            key_lo = kfirst + seg0 * KSTEP;
+            key_lo = kbeg + min(s_begin + seg0, nsteps_all - 1) * KSTEP;
             lp0 = page_of(key_lo);
-            const int seg_steps = min(nsteps - seg0, ((lp0 + TBL_MAX) * page_size - key_lo) / KSTEP);
-            key_hi = min(key_lo + seg_steps * KSTEP, kend) - 1;
+            // (TBL_MAX - 1 pages hold the keys of this many steps wherever in a page the first one lies)
+            const int seg_steps = min(nsteps - seg0, (TBL_MAX - 1) * page_size / KSTEP / 4 * 4);
+            const int own_steps = GROUPS > 1 ? max(0, min(own - seg0, seg_steps)) : seg_steps;
+            key_hi = min(key_lo + max(own_steps, 1) * KSTEP, kend) - 1;
             __syncthreads();                   // nobody still reads the previous segment's table or staged tiles
             for (int i = tid; i <= page_of(key_hi) - lp0; i += MA_THREADS) tbl[i] = table[lp0 + i];
             __syncthreads();
@@ -370,7 +390,7 @@ void mfma_attention_kernel(
                     bool act[CB], inner[CB], any_act = INTERIOR, all_inner = true;
 #pragma unroll
                     for (int c = 0; c < CB; ++c) {
-                        act[c] = INTERIOR || (blk_ok[c] && ks <= blk_pmax[c]);
+                        act[c] = INTERIOR || (blk_ok[c] && ks <= blk_pmax[c] && (GROUPS == 1 || s < own_steps));
                         inner[c] = INTERIOR || (act[c] && ks >= blk_lo_max[c] && ks + KSTEP - 1 <= blk_pmin[c]);
                         any_act = any_act || act[c];
                         all_inner = all_inner && inner[c];
@@ -481,7 +501,7 @@ void mfma_attention_kernel(
                 load_at(at_next, knext, vnext);
             };
             // the steps [in_lo, in_hi) of the segment, whole turns of the ring, are interior for this wavefront
-            int in_lo = seg_steps, in_hi = seg_steps;
+            int in_lo = own_steps, in_hi = own_steps;
             {
                 bool every = true;
                 int lo_max = 0, p_min = blk_pmin[0];
@@ -494,7 +514,7 @@ void mfma_attention_kernel(
                 const int first = lo_max > key_lo ? (lo_max - key_lo + KSTEP - 1) / KSTEP : 0;       // ks >= lo_max
                 const int past = p_min - (KSTEP - 1) >= key_lo ? (p_min - (KSTEP - 1) - key_lo) / KSTEP + 1 : 0;   // ks + 31 <= p_min
                 const int a = (first + DEPTH - 1) / DEPTH * DEPTH;
-                const int b = min(past, seg_steps);
+                const int b = min(past, own_steps);
                 if (every && b - a >= DEPTH) { in_lo = a; in_hi = a + (b - a) / DEPTH * DEPTH; }
             }
             for (int s0 = 0; s0 < seg_steps; s0 += DEPTH) {
@@ -511,6 +531,29 @@ void mfma_attention_kernel(
             seg0 += seg_steps;
         }
 
+        if constexpr (GROUPS > 1) {
+            // (the next tile's writes here lie behind the barriers of its steps)
+            if (group == 1) {
+#pragma unroll
+                for (int c = 0; c < CB; ++c) {
+                    meet_ml[wave * CB + c][lane] = make_float2(m_run[c], l_run[c][0]);
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt) meet_o[(wave * CB + c) * DT + dt][lane] = o[c][dt];
+                }
+            }
+            __syncthreads();
+            if (group == 1) continue;
+#pragma unroll
+            for (int c = 0; c < CB; ++c) {
+                const float2 other = meet_ml[wave * CB + c][lane];
+                const float m = fmaxf(m_run[c], other.x);
+                const float mine = __builtin_amdgcn_exp2f(m_run[c] - m), theirs = __builtin_amdgcn_exp2f(other.x - m);
+                m_run[c] = m;
+                l_run[c] = l_run[c] * mine + other.y * theirs;
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) o[c][dt] = o[c][dt] * mine + meet_o[(wave * CB + c) * DT + dt][lane] * theirs;
+            }
+        }
 #pragma unroll
         for (int c = 0; c < CB; ++c) {
             const float l = l_run[c][0];
@@ -784,11 +827,11 @@ NI_EXPORT int ni_mfma_attention_tile_tokens(int group, int blocks) {
 NI_EXPORT int ni_mfma_attention(const void* q, int q_stride, const void* kpool, const void* vpool, const void* block_table,
                                 int table_stride, const void* tiles, int n_tiles, void* out, void* part_o, void* part_ml,
                                 int H, int KVH, int page_size, int window, float scale, int nsplit, int blocks,
-                                hipStream_t stream) {
+                                int groups, hipStream_t stream) {
     if (n_tiles <= 0) return 0;
     if (H % KVH != 0 || page_size < 1 || nsplit < 1 || nsplit > 64 || !(scale > 0.f)) return -1;
     if (nsplit > 1 && (!part_o || !part_ml)) return -2;
-    if (blocks < 1 || blocks > MA_MAX_BLOCKS) return -3;
+    if (blocks < 1 || blocks > MA_MAX_BLOCKS || groups < 1 || groups > (HEAD_DIM <= 128 ? 2 : 1)) return -3;
     const int G = H / KVH;
     const int hpt = heads_per_tile(G);
     int hpt_shift = 0;
@@ -801,15 +844,15 @@ NI_EXPORT int ni_mfma_attention(const void* q, int q_stride, const void* kpool, 
     const int per_tile = KVH * chunks * nsplit;
     // As many workgroups as the chip holds at once (asked of the runtime once per kernel), each walking
     // through its share of the sorted tiles.
-#define MA_LAUNCH(CB_)                                                                                              \
+#define MA_LAUNCH(CB_, GROUPS_)                                                                                              \
     {                                                                                                               \
-        auto kernel = pow2 ? mfma_attention_kernel<CB_, true> : mfma_attention_kernel<CB_, false>;                 \
+        auto kernel = pow2 ? mfma_attention_kernel<CB_, true, GROUPS_> : mfma_attention_kernel<CB_, false, GROUPS_>; \
         static int slots[2] = {0, 0}, units[2] = {0, 0};                                                            \
         if (slots[pow2] == 0) {                                                                                     \
             int dev = 0, cus = 0, per_cu = 0;                                                                       \
             if (hipGetDevice(&dev) != hipSuccess ||                                                                 \
                 hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||            \
-                hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, MA_WAVES * WAVE, 0) != hipSuccess ||  \
+                hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, GROUPS_ * MA_WAVES * WAVE, 0) != hipSuccess || \
                 cus < 1 || per_cu < 1)                                                                              \
                 return -4;                                                                                          \
             units[pow2] = cus;                                                                                      \
@@ -825,14 +868,18 @@ NI_EXPORT int ni_mfma_attention(const void* q, int q_stride, const void* kpool, 
         }                                                                                                           \
         const int in_x = (n_tiles + rounds - 1) / rounds;                                                           \
         dim3 grid(in_x, KVH * chunks, nsplit);                                                                      \
-        kernel<<<grid, MA_WAVES * WAVE, 0, stream>>>(                                                               \
+        kernel<<<grid, GROUPS_ * MA_WAVES * WAVE, 0, stream>>>(                                                               \
             (const bf16_t*)q, q_stride, (const bf16_t*)kpool, (const bf16_t*)vpool, (const int32_t*)block_table,   \
             table_stride, (const QTile*)tiles, n_tiles, (bf16_t*)out, (float*)part_o, (float*)part_ml, H, KVH,     \
             page_size, page_shift, hpt_shift, window, scale, nsplit);                                               \
     }
-    if (blocks == 1) MA_LAUNCH(1)
+    if (blocks == 1 && groups == 1) MA_LAUNCH(1, 1)
+#if HEAD_DIM <= 128
+    else if (blocks == 1) MA_LAUNCH(1, 2)
+#endif
 #if HEAD_DIM <= 64
-    else MA_LAUNCH(2)
+    else if (groups == 1) MA_LAUNCH(2, 1)
+    else MA_LAUNCH(2, 2)
 #endif
 #undef MA_LAUNCH
     return NI_LAUNCH_RESULT();

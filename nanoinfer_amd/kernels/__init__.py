@@ -404,6 +404,43 @@ def mfma_plan(hd: int, group: int, kv_heads: int, n_tokens: int, max_q_len: int,
     return small, None
 
 
+def mfma_group_plan(hd: int, group: int, kv_heads: int, n_tokens: int, max_q_len: int, max_keys: int, dtype: torch.dtype = torch.bfloat16):
+    """``(tile_tokens, nsplit)`` where the bfloat16 prompt kernel takes eight wavefronts a tile, two groups of four that walk one
+    half of its keys each, instead of :func:`mfma_plan`'s four; else None.  A workgroup then has a compute unit to itself and keeps
+    two wavefronts a SIMD busy to the end, which pays for one portion without a window whose tiles leave a unit one workgroup, or
+    whose long tiles outlast the short ones (``max_keys`` rounded up to a power of two, as there).  Measured, that plan : this one,
+    us, 32 heads on 8:
+    one block of rows and no more than a tile (times runs) for each of the 256 units, from 512 keys on, up to eight times the
+    portion (or 2,048): head size 64, 512 tokens at 512 / 1,024 / 1,536 / 2,048 / 3,072 / 4,096 / 6,000 keys 11.6 : 11.0, 17.9 : 15.3, 25.9 : 19.5,
+    28.3 : 23.4, 33.7 : 31.6, 39.0 : 39.8, 50.5 : 54.8; 256 at 256 / 1,024 / 2,048 / 4,096 8.3 : 8.5, 16.3 : 14.7, 22.1 : 19.9, 28.7 : 28.3; 128 at
+    2,000 17.4 : 16.2.  Head size 96, 512 at 768 / 4,096 20.2 : 17.8, 66.1 : 60.5; 128 (24 on 8), 512 at 512 / 1,024 / 2,048 / 8,192
+    17.9 : 18.8, 29.0 : 27.7, 49.7 : 42.5, 140 : 132, 256 at 1,024 / 4,096 24.6 : 26.7, 55.4 : 50.3.
+    Two blocks, one tile a unit, keys at least twice the portion: 1,024 at 2,048 / 4,096 34.8 : 33.0, 63.5 : 55.3 (700 tokens at 1,400, where
+    176 tiles leave units idle, 27.0 : 30.1).  Two blocks, 1.4 to 3 tiles a unit, long and short ones in turn by one workgroup, keys
+    no more than twice the portion: 1,500 at 1,500 35.2 : 32.6, 1,700 54.3 : 39.6, 1,999 42.6 : 39.0, 3,000 82.3 : 76.7, 2,048 at 4,096 / 6,000
+    86.6 : 84.9, 127 : 133 (four tiles a unit, 4,096 at 4,096, 109 : 119; four portions of 300 at 700 26.7 : 29.6)."""
+    if dtype != torch.bfloat16 or n_tokens != max_q_len or not 32 < hd <= 128:
+        return None
+    small = mfma_tile_tokens(hd, group)
+    hpt = _heads_per_tile(group)
+    per_tile = kv_heads * ((group + hpt - 1) // hpt)
+    bound = max(256, 1 << max(0, int(max_keys) - 1).bit_length())
+    one = -(-n_tokens // small) * per_tile
+    if one <= COMPUTE_UNITS:
+        nsplit = max(1, min(COMPUTE_UNITS // one, bound // 640, 16))
+        if hd <= 64:
+            return (small, nsplit) if 512 <= bound <= max(8 * n_tokens, 2048) else None
+        return (small, nsplit) if bound >= 1024 and 2 * nsplit * one > COMPUTE_UNITS else None
+    if hd > 64:
+        return None
+    two = n_tokens // (2 * small) * per_tile
+    if 7 * COMPUTE_UNITS < 8 * two <= 8 * COMPUTE_UNITS and bound >= 2 * n_tokens:
+        return 2 * small, 1
+    if 14 * COMPUTE_UNITS <= 10 * two <= 30 * COMPUTE_UNITS and bound <= 2 * n_tokens + 2 * small:
+        return 2 * small, 1
+    return None
+
+
 def build_q_tiles(q_start, q_len, context_len, tile_tokens: int):
     """Cut the portions of a step (host lists: first row, length, context after the step) into
     tiles of at most ``tile_tokens`` tokens: flat list of (sequence, first row, tokens, first position),
@@ -492,15 +529,18 @@ def mfma_splits(n_tiles: int, kv_heads: int, group: int, max_keys: int, hd: int 
 def mfma_attention(qkv: torch.Tensor, kpool: torch.Tensor, vpool: torch.Tensor, block_table: torch.Tensor,
                    tiles: torch.Tensor, out: torch.Tensor, H: int, KVH: int, hd: int, scale: float,
                    window: Optional[int], nsplit: int = 1, workspace: Optional[torch.Tensor] = None,
-                   tile_tokens: Optional[int] = None) -> torch.Tensor:
+                   tile_tokens: Optional[int] = None, groups: int = 1) -> torch.Tensor:
     """Attention of prompt portions on the matrix cores, in bfloat16 or in true float32 (a kernel
     each).  ``tiles`` is int32 [n, 4] from :func:`build_q_tiles` with ``tile_tokens`` tokens a tile (a
     size that :func:`mfma_tile_tokens` gives for the type; default: its smallest); the pools already
     hold the keys and values of every position of the step.  ``workspace`` (float32,
-    ``T*H*nsplit*(hd+2)`` elements) is needed when ``nsplit > 1``."""
+    ``T*H*nsplit*(hd+2)`` elements) is needed when ``nsplit > 1``.  ``groups`` (bfloat16, head sizes up to 128): 1 or 2
+    groups of four wavefronts that share out a tile's keys (:func:`mfma_group_plan`)."""
     T = qkv.shape[0]
     dtype = qkv.dtype
     _gpu(qkv, "qkv")
+    if not (groups == 1 or (groups == 2 and dtype == torch.bfloat16 and hd <= 128)):
+        raise KernelError(f"mfma_attention has no {groups} groups of wavefronts at head size {hd} in {dtype}")
     if not (mfma_attention_ok(dtype, hd)):
         raise KernelError(f"mfma_attention does not take {dtype} with head size {hd}")
     if not (H >= 1 and KVH >= 1 and H % KVH == 0):
@@ -546,7 +586,7 @@ def mfma_attention(qkv: torch.Tensor, kpool: torch.Tensor, vpool: torch.Tensor, 
         _check(attention_mfma_lib(hd).ni_mfma_attention(
             _ptr(qkv), qkv.shape[1], _ptr(kpool), _ptr(vpool), _ptr(block_table), block_table.shape[1], _ptr(tiles),
             tiles.shape[0], _ptr(out), _ptr(part_o), _ptr(part_ml), H, KVH, kpool.shape[2],
-            int(window) if window else 0, ctypes.c_float(scale), nsplit, blocks, _stream()), "mfma_attention")
+            int(window) if window else 0, ctypes.c_float(scale), nsplit, blocks, groups, _stream()), "mfma_attention")
     if nsplit > 1:
         _check(attention_lib(hd).ni_merge_splits(_ptr(part_o), _ptr(part_ml), _ptr(out), T, H, nsplit,
                                                  dtype_code(out.dtype), _stream()), "merge_splits")

@@ -390,14 +390,16 @@ class Attention(Part):
             # prompt portions: tiles of tokens on the matrix cores (a recorded step has them only if
             # it was recorded with them)
             max_keys = ctx.max_context if self.window is None else min(ctx.max_context, self.window + ctx.max_q_len)
-            tile_tokens, nsplit = K.mfma_plan(self.hd, self.H // self.KVH, self.KVH, T, ctx.max_q_len, max_keys, dtype)
+            plan = None if self.window is not None else K.mfma_group_plan(self.hd, self.H // self.KVH, self.KVH, T, ctx.max_q_len, max_keys, dtype)
+            groups = 1 if plan is None else 2
+            tile_tokens, nsplit = plan or K.mfma_plan(self.hd, self.H // self.KVH, self.KVH, T, ctx.max_q_len, max_keys, dtype)
             tiles = ctx.q_tiles(tile_tokens)
         if tiles is not None:
             if nsplit is None:
                 nsplit = K.mfma_splits(tiles.shape[0], self.KVH, self.H // self.KVH, max_keys, self.hd, dtype)
             ws = ctx.workspace(T * self.H * nsplit * (self.hd + 2)) if nsplit > 1 else None
             K.mfma_attention(qkv, cache.kpool, cache.vpool, cache.block_table, tiles, out, self.H, self.KVH, self.hd,
-                             self.scale, self.window, nsplit, ws, tile_tokens)
+                             self.scale, self.window, nsplit, ws, tile_tokens, groups)
             return out
         # single tokens and short portions, token by token
         max_keys = ctx.max_context if self.window is None else min(ctx.max_context, self.window)
