@@ -170,7 +170,7 @@ __device__ __forceinline__ floatx4_t row_sum_step(const uint4& pf, floatx4_t l) 
 // LDS.  A wavefront alone on a SIMD waits for LDS and its own chain of instructions (0.6 us for a step of
 // 32 keys, two blocks of rows, head size 64; two together take 0.73), and the last tiles of a prompt, its
 // longest, used to run alone.  2,048 tokens at 2,048 keys, 32 heads on 8: 42.6 -> 39.4 us, of which 33 pairs
-// of steps are 24 and the start and end of two tiles 14; 512 at 2,048 28.3 -> 23.4, 1,700 at 1,700 54.3 -> 39.6.
+// of steps are 24 and the start and end of two tiles 14; 512 at 1,024 17.9 -> 15.3, 1,700 at 1,700 54.3 -> 39.6.
 template <int CB, bool POW2, int GROUPS>
 __global__ __launch_bounds__(GROUPS * MA_WAVES * WAVE) __attribute__((amdgpu_waves_per_eu(HEAD_DIM * CB <= 128 ? 2 : 1)))
 void mfma_attention_kernel(

@@ -411,15 +411,18 @@ def mfma_group_plan(hd: int, group: int, kv_heads: int, n_tokens: int, max_q_len
     whose long tiles outlast the short ones (``max_keys`` rounded up to a power of two, as there).  Measured, that plan : this one,
     us, 32 heads on 8:
     one block of rows and no more than a tile (times runs) for each of the 256 units, from 512 keys on, up to eight times the
-    portion (or 2,048): head size 64, 512 tokens at 512 / 1,024 / 1,536 / 2,048 / 3,072 / 4,096 / 6,000 keys 11.6 : 11.0, 17.9 : 15.3, 25.9 : 19.5,
-    28.3 : 23.4, 33.7 : 31.6, 39.0 : 39.8, 50.5 : 54.8; 256 at 256 / 1,024 / 2,048 / 4,096 8.3 : 8.5, 16.3 : 14.7, 22.1 : 19.9, 28.7 : 28.3; 128 at
-    2,000 17.4 : 16.2.  Head size 96, 512 at 768 / 4,096 20.2 : 17.8, 66.1 : 60.5; 128 (24 on 8), 512 at 512 / 1,024 / 2,048 / 8,192
+    portion (or 2,048): head size 64, 512 tokens at 512 / 1,024 keys 11.6 : 11.0, 17.9 : 15.3; 256 at 256 / 1,024 / 2,048 8.3 : 8.5, 16.3 : 14.7,
+    22.1 : 19.9; 128 at 2,000 17.4 : 16.2.  (Where :func:`mfma_plan` cuts the keys of tiles of two blocks, that stays: 256 at 4,096
+    28.7 : 28.3, 512 at 4,096 / 6,000 39.0 : 39.8, 50.5 : 54.8; 512 at 1,536 / 2,048 / 3,072, 25.9 : 19.5, 28.3 : 23.4, 33.7 : 31.6, stay with it
+    too, the only portions that bring those runs and their merge through the engine.)  Head size 96, 512 at 768 / 4,096 20.2 : 17.8, 66.1 : 60.5; 128 (24 on 8), 512 at 512 / 1,024 / 2,048 / 8,192
     17.9 : 18.8, 29.0 : 27.7, 49.7 : 42.5, 140 : 132, 256 at 1,024 / 4,096 24.6 : 26.7, 55.4 : 50.3.
     Two blocks, one tile a unit, keys at least twice the portion: 1,024 at 2,048 / 4,096 34.8 : 33.0, 63.5 : 55.3 (700 tokens at 1,400, where
     176 tiles leave units idle, 27.0 : 30.1).  Two blocks, 1.4 to 3 tiles a unit, long and short ones in turn by one workgroup, keys
     no more than twice the portion: 1,500 at 1,500 35.2 : 32.6, 1,700 54.3 : 39.6, 1,999 42.6 : 39.0, 3,000 82.3 : 76.7, 2,048 at 4,096 / 6,000
     86.6 : 84.9, 127 : 133 (four tiles a unit, 4,096 at 4,096, 109 : 119; four portions of 300 at 700 26.7 : 29.6)."""
     if dtype != torch.bfloat16 or n_tokens != max_q_len or not 32 < hd <= 128:
+        return None
+    if mfma_plan(hd, group, kv_heads, n_tokens, max_q_len, max_keys)[1] is not None:
         return None
     small = mfma_tile_tokens(hd, group)
     hpt = _heads_per_tile(group)

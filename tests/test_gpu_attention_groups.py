@@ -70,8 +70,8 @@ def test_one_workgroup_for_a_long_and_a_short_tile():
 def test_the_rule():
     from nanoinfer_amd import kernels as K
     plan = K.mfma_group_plan
-    assert plan(64, 4, 8, 512, 512, 512) == (16, 1) == plan(64, 4, 8, 512, 512, 4096)
-    assert plan(64, 4, 8, 512, 512, 4097) is None and plan(64, 4, 8, 256, 256, 256) is None
+    assert plan(64, 4, 8, 512, 512, 512) == (16, 1) == plan(64, 4, 8, 512, 512, 1024)
+    assert plan(64, 4, 8, 512, 512, 1100) is None and plan(64, 4, 8, 256, 256, 256) is None
     assert plan(64, 4, 8, 256, 256, 2048) == (16, 2) and plan(64, 4, 8, 1024, 1024, 1024) is None
     assert plan(64, 4, 8, 1024, 1024, 2048) == (32, 1) == plan(64, 4, 8, 1999, 1999, 1999) == plan(64, 4, 8, 3000, 3000, 3000)
     assert plan(64, 4, 8, 4096, 4096, 4096) is None and plan(64, 4, 8, 2048, 2048, 6000) is None
