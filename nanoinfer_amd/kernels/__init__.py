@@ -416,13 +416,11 @@ def mfma_group_plan(hd: int, group: int, kv_heads: int, n_tokens: int, max_q_len
     28.7 : 28.3, 512 at 4,096 / 6,000 39.0 : 39.8, 50.5 : 54.8; 512 at 1,536 / 2,048 / 3,072, 25.9 : 19.5, 28.3 : 23.4, 33.7 : 31.6, stay with it
     too, the only portions that bring those runs and their merge through the engine.)  Head size 96, 512 at 768 / 4,096 20.2 : 17.8, 66.1 : 60.5; 128 (24 on 8), 512 at 512 / 1,024 / 2,048 / 8,192
     17.9 : 18.8, 29.0 : 27.7, 49.7 : 42.5, 140 : 132, 256 at 1,024 / 4,096 24.6 : 26.7, 55.4 : 50.3.
-    Two blocks, one tile a unit, keys at least twice the portion: 1,024 at 2,048 / 4,096 34.8 : 33.0, 63.5 : 55.3 (700 tokens at 1,400, where
+    Two blocks, one tile a unit, keys twice to four times the portion: 1,024 at 2,048 / 4,096 34.8 : 33.0, 63.5 : 55.3 (700 tokens at 1,400, where
     176 tiles leave units idle, 27.0 : 30.1).  Two blocks, 1.4 to 3 tiles a unit, long and short ones in turn by one workgroup, keys
     no more than twice the portion: 1,500 at 1,500 35.2 : 32.6, 1,700 54.3 : 39.6, 1,999 42.6 : 39.0, 3,000 82.3 : 76.7, 2,048 at 4,096 / 6,000
     86.6 : 84.9, 127 : 133 (four tiles a unit, 4,096 at 4,096, 109 : 119; four portions of 300 at 700 26.7 : 29.6)."""
     if dtype != torch.bfloat16 or n_tokens != max_q_len or not 32 < hd <= 128:
-        return None
-    if mfma_plan(hd, group, kv_heads, n_tokens, max_q_len, max_keys)[1] is not None:
         return None
     small = mfma_tile_tokens(hd, group)
     hpt = _heads_per_tile(group)
@@ -430,6 +428,8 @@ def mfma_group_plan(hd: int, group: int, kv_heads: int, n_tokens: int, max_q_len
     bound = max(256, 1 << max(0, int(max_keys) - 1).bit_length())
     one = -(-n_tokens // small) * per_tile
     if one <= COMPUTE_UNITS:
+        if mfma_plan(hd, group, kv_heads, n_tokens, max_q_len, max_keys)[1] is not None:
+            return None
         nsplit = max(1, min(COMPUTE_UNITS // one, bound // 640, 16))
         if hd <= 64:
             return (small, nsplit) if 512 <= bound <= max(8 * n_tokens, 2048) else None
@@ -437,7 +437,7 @@ def mfma_group_plan(hd: int, group: int, kv_heads: int, n_tokens: int, max_q_len
     if hd > 64:
         return None
     two = n_tokens // (2 * small) * per_tile
-    if 7 * COMPUTE_UNITS < 8 * two <= 8 * COMPUTE_UNITS and bound >= 2 * n_tokens:
+    if 7 * COMPUTE_UNITS < 8 * two <= 8 * COMPUTE_UNITS and 2 * n_tokens <= bound <= 4 * n_tokens + 8 * small:
         return 2 * small, 1
     if 14 * COMPUTE_UNITS <= 10 * two <= 30 * COMPUTE_UNITS and bound <= 2 * n_tokens + 2 * small:
         return 2 * small, 1

@@ -74,6 +74,7 @@ def test_the_rule():
     assert plan(64, 4, 8, 512, 512, 1100) is None and plan(64, 4, 8, 256, 256, 256) is None
     assert plan(64, 4, 8, 256, 256, 2048) == (16, 2) and plan(64, 4, 8, 1024, 1024, 1024) is None
     assert plan(64, 4, 8, 1024, 1024, 2048) == (32, 1) == plan(64, 4, 8, 1999, 1999, 1999) == plan(64, 4, 8, 3000, 3000, 3000)
+    assert plan(64, 4, 8, 1024, 1024, 4096) == (32, 1) and plan(64, 4, 8, 1024, 1024, 4097) is None
     assert plan(64, 4, 8, 4096, 4096, 4096) is None and plan(64, 4, 8, 2048, 2048, 6000) is None
     assert plan(64, 4, 8, 512, 481, 1100) is None                    # several portions in the step
     assert plan(128, 3, 8, 512, 512, 512) is None and plan(128, 3, 8, 512, 512, 2048) == (16, 1)
