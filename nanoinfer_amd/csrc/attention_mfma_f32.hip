@@ -79,6 +79,7 @@ struct TileArgs {
 };
 
 constexpr int TBL_MAX = 1024;                       // pages of a sequence that a workgroup looks up at a time
+constexpr int PKEYS = 32;                           // keys of a step in three parts; a run of keys is whole steps
 
 // One block of 16 rows a wavefront (of the `blocks` it owns) on the float32 instructions.  The k index of an MFMA is only a
 // label: lane group kg of MFMA j takes dim kg*HD/4 + j of K and Q; of the second product the weight of key 4*kg + i is register i
@@ -130,16 +131,15 @@ __device__ __forceinline__ void exact_tile(const TileArgs& a, const QTile& tile,
     const int blk_pmax = tile.pos0 + min(tile.ntok, tb0 + tok_per_block) - 1;
     const int blk_lo_max = window > 0 ? max(0, blk_pmax + 1 - window) : 0;
 
-    // key range of the workgroup, walked in steps of KSTEP from a multiple of KSTEP; only keys
-    // tile_lo..kend-1 are read from the cache (all of them the sequence's own, none given back)
+    // key range of the workgroup, walked in steps of KSTEP: the same run of PKEYS at a time as in parts_tile, since the other runs
+    // of these rows may have been made there; only keys tile_lo..kend-1 are read from the cache (all of them the
+    // sequence's own, none given back)
     const int kend = tile.pos0 + tile.ntok;
     const int tile_lo = window > 0 ? max(0, tile.pos0 + 1 - window) : 0;
-    const int kbeg = tile_lo / KSTEP * KSTEP;
-    const int nsteps_all = (kend - kbeg + KSTEP - 1) / KSTEP;
-    const int per_split = (nsteps_all + nsplit - 1) / nsplit;
-    const int s_begin = blockIdx.z * per_split;
-    const int nsteps = max(0, min(nsteps_all, s_begin + per_split) - s_begin);
-    const int kfirst = kbeg + s_begin * KSTEP;
+    const int kbeg = tile_lo / PKEYS * PKEYS;
+    const int per_split = ((kend - kbeg + PKEYS - 1) / PKEYS + nsplit - 1) / nsplit;
+    const int kfirst = kbeg + blockIdx.z * per_split * PKEYS;
+    const int nsteps = (max(0, min(kend - kfirst, per_split * PKEYS)) + KSTEP - 1) / KSTEP;
 
     const int32_t* table = block_table + static_cast<size_t>(tile.seq) * table_stride;
     auto page_of = [&](int key) { return POW2 ? (key >> page_shift) : key / page_size; };
@@ -291,7 +291,6 @@ __device__ __forceinline__ floatx4_t times(const uint4& a, const uint4& b, float
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
-constexpr int PKEYS = 32;                                   // keys of a step
 constexpr int PSLOTS = HEAD_DIM <= 64 ? 2 : 1;              // steps that LDS holds
 struct PartLds {
     uint16_t k[PSLOTS][3][PKEYS][HEAD_DIM + 8], v[PSLOTS][3][PKEYS][HEAD_DIM + 8];

@@ -107,3 +107,17 @@ def test_weights_far_below_the_reference_keep_their_places():
     # a weight e^t is off by (|t| + 4) roundings of itself; over weights that fall by e^0.9 a key, numerator and denominator, that
     # is 2 (1 + 4) of the largest value, and a few for the sums
     assert float((got - want).abs().max()) <= 16 * 2.0 ** -24 * float(v.abs().max())
+
+
+@pytest.mark.parametrize("hd,nsplit", [(256, 2), (256, 3), (160, 3), (128, 3)])
+def test_one_run_of_keys_is_made_again(hd, nsplit):
+    """The run with a value too large for a bfloat16 goes to the float32 instructions, the others do not: together they have every
+    key once, also where those take fewer keys a step."""
+    H, KVH, T, keys = 2, 1, 17, 120
+    q, k, v = operands(hd, H, KVH, T, keys, hd)
+    v[3, 0, 8] = 3.4e38
+    want = plain(q, k, v, T, hd ** -0.5)
+    got = attention(hd, H, KVH, q, k, v, T, nsplit, hd ** -0.5)
+    assert torch.allclose(got[:, :, 8].double(), want[:, :, 8], rtol=1e-5)
+    others = [c for c in range(hd) if c != 8]
+    assert float((got[:, :, others].double() - want[:, :, others]).abs().max()) <= 1e-5
