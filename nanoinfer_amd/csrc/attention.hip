@@ -270,7 +270,7 @@ __global__ void merge_splits_kernel(const float* __restrict__ part_o, const floa
     constexpr bool FAST = sizeof(T) == 2;
     const int t = blockIdx.x, h = blockIdx.y;
     const size_t p0 = (static_cast<size_t>(t) * H + h) * nsplit;
-    float M = NEG_BIG;
+    float M = -INFINITY;        // (a run without keys leaves a finite maximum, and zeros)
     for (int s = 0; s < nsplit; ++s) M = fmaxf(M, part_ml[(p0 + s) * 2]);
     for (int dim = threadIdx.x; dim < HEAD_DIM; dim += blockDim.x) {
         float Lsum = 0.f, O = 0.f;

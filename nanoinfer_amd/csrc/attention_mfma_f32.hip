@@ -49,6 +49,10 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 // reference is moved and the output rescaled (e^5.545 = 2^8).  Softmax is the same whatever the
 // reference, as long as numerator and denominator share it.
 #define REF_SLACK 5.545177444479562f
+// A row's reference before its first score.  A key that a row does not see scores minus infinity, and its weight against this or any
+// later reference is zero by itself: keys are told apart by their places, never by their scores, so that NaN and infinities
+// reach the sums whichever step they lie in.
+#define LOWEST (-3.4028234663852886e38f)
 
 struct QTile { int32_t seq, row0, ntok, pos0; };   // tokens row0..row0+ntok-1 of the batch, positions pos0..
 
@@ -162,7 +166,7 @@ __device__ __forceinline__ void exact_tile(const TileArgs& a, const QTile& tile,
         for (int j = 0; j < QK; ++j) qf[j] = 0.f;
     }
 
-    float m_ref = NEG_BIG, l_lane = 0.f;       // the row's reference; the sum of this lane's own weights
+    float m_ref = LOWEST, l_lane = 0.f;       // the row's reference; the sum of this lane's own weights
     floatx4_t o[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db) o[db] = floatx4_t{0.f, 0.f, 0.f, 0.f};
@@ -207,7 +211,7 @@ __device__ __forceinline__ void exact_tile(const TileArgs& a, const QTile& tile,
                     }
                 }
                 float sc[HALVES][4];
-                float lane_max = NEG_BIG;
+                float lane_max = -INFINITY;
 #pragma unroll
                 for (int t = 0; t < HALVES; ++t)
 #pragma unroll
@@ -215,7 +219,7 @@ __device__ __forceinline__ void exact_tile(const TileArgs& a, const QTile& tile,
                         float v = st[t][i];
                         if (!inner) {
                             const int key = ks + t * 16 + kg * 4 + i;
-                            v = (row_ok && key <= pos && key >= row_lo) ? v : NEG_BIG;
+                            v = (row_ok && key <= pos && key >= row_lo) ? v : -INFINITY;
                         }
                         sc[t][i] = v;
                         lane_max = fmaxf(lane_max, v);
@@ -223,7 +227,7 @@ __device__ __forceinline__ void exact_tile(const TileArgs& a, const QTile& tile,
                 // 2. a row whose scores have risen far above its reference: move it, rescale what was summed
                 if (__any(lane_max - REF_SLACK > m_ref)) {
                     const float mx = lanes4(lane_max, true);
-                    const bool move = mx > 0.5f * NEG_BIG && mx > m_ref + REF_SLACK;
+                    const bool move = mx > m_ref + REF_SLACK;
                     const float m_new = move ? mx : m_ref;
                     const float corr = move ? expf(m_ref - m_new) : 1.0f;
                     m_ref = m_new;
@@ -236,8 +240,7 @@ __device__ __forceinline__ void exact_tile(const TileArgs& a, const QTile& tile,
                 for (int t = 0; t < HALVES; ++t)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        float p = expf(sc[t][i] - m_ref);
-                        if (!inner) p = sc[t][i] > 0.5f * NEG_BIG ? p : 0.f;
+                        const float p = expf(sc[t][i] - m_ref);
                         l_lane += p;
                         float va[DB];
                         VecIO<float, DB>::load(&vb[t * 16 + kg * 4 + i][r * DB], va);
@@ -262,7 +265,7 @@ __device__ __forceinline__ void exact_tile(const TileArgs& a, const QTile& tile,
             const size_t p = (static_cast<size_t>(tile.row0 + tt) * H + head) * nsplit + blockIdx.z;
             if (kg == 0) { part_ml[p * 2] = m_ref; part_ml[p * 2 + 1] = l; }
             VecIO<float, QK>::store(part_o + p * HD + kg * QK, vals);
-        } else if (l > 0.f) {
+        } else {
             const float inv = 1.0f / l;
 #pragma unroll
             for (int j = 0; j < QK; ++j) vals[j] *= inv;
@@ -379,7 +382,7 @@ __device__ __forceinline__ bool parts_tile(const TileArgs& a, const QTile& tile,
     floatx4_t o[CB][DT];
 #pragma unroll
     for (int c = 0; c < CB; ++c) {
-        m_ref[c] = NEG_BIG;
+        m_ref[c] = LOWEST;
         l_lane[c] = 0.f;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) o[c][dt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
@@ -487,7 +490,7 @@ __device__ __forceinline__ bool parts_tile(const TileArgs& a, const QTile& tile,
                 Parts pf[CB];
 #pragma unroll
                 for (int c = 0; c < CB; ++c) {
-                    float sc[8], lane_max = NEG_BIG;
+                    float sc[8], lane_max = -INFINITY;
 #pragma unroll
                     for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -495,7 +498,7 @@ __device__ __forceinline__ bool parts_tile(const TileArgs& a, const QTile& tile,
                             float v = st[c][t][i];
                             if (!inner[c]) {
                                 const int key = ks + t * 16 + kg * 4 + i;
-                                v = (row_ok[c] && act[c] && key <= pos[c] && key >= row_lo[c]) ? v : NEG_BIG;
+                                v = (row_ok[c] && act[c] && key <= pos[c] && key >= row_lo[c]) ? v : -INFINITY;
                             }
                             sc[t * 4 + i] = v;
                             lane_max = fmaxf(lane_max, v);
@@ -503,7 +506,7 @@ __device__ __forceinline__ bool parts_tile(const TileArgs& a, const QTile& tile,
                     // 2. a row whose scores have risen far above its reference: move it, rescale what was summed
                     if (__any(lane_max - REF_SLACK > m_ref[c])) {
                         const float mx = lanes4(lane_max, true);
-                        const bool move = mx > 0.5f * NEG_BIG && mx > m_ref[c] + REF_SLACK;
+                        const bool move = mx > m_ref[c] + REF_SLACK;
                         const float m_new = move ? mx : m_ref[c];
                         const float corr = move ? expf(m_ref[c] - m_new) : 1.0f;
                         m_ref[c] = m_new;
@@ -516,7 +519,6 @@ __device__ __forceinline__ bool parts_tile(const TileArgs& a, const QTile& tile,
 #pragma unroll
                     for (int j = 0; j < 8; ++j) {
                         w[j] = exp_below(sc[j] - m_ref[c]);
-                        if (!inner[c]) w[j] = sc[j] > 0.5f * NEG_BIG ? w[j] : 0.f;
                         l_lane[c] += w[j];
                     }
                     pf[c] = parts8(w);
@@ -566,7 +568,7 @@ __device__ __forceinline__ bool parts_tile(const TileArgs& a, const QTile& tile,
             if (kg == 0) { a.part_ml[p * 2] = m_ref[c]; a.part_ml[p * 2 + 1] = l[c]; }
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<floatx4_t*>(a.part_o + p * HD + dt * 16 + kg * 4) = o[c][dt];
-        } else if (l[c] > 0.f) {
+        } else {
             const float inv = 1.0f / l[c];
             float* to = a.out + static_cast<size_t>(tile.row0 + tt[c]) * a.H * HD + static_cast<size_t>(head) * HD + kg * 4;
 #pragma unroll
