@@ -532,7 +532,9 @@ void mfma_attention_kernel(
         }
 
         if constexpr (GROUPS > 1) {
-            // (the next tile's writes here lie behind the barriers of its steps)
+            // The second group may be a tile ahead of the first one's reads below: the barriers of its steps lie between them
+            // and these writes, and where a tile's run has no steps (all of its groups know that) one that stands here.
+            if (nsteps == 0) __syncthreads();
             if (group == 1) {
 #pragma unroll
                 for (int c = 0; c < CB; ++c) {

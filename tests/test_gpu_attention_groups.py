@@ -67,6 +67,14 @@ def test_one_workgroup_for_a_long_and_a_short_tile():
     assert run(((1530, 1530),), 32, 8, 64, 16, 2, 1, None, 5) <= 0.0
 
 
+@pytest.mark.parametrize("hd,H,KVH,blocks", [(64, 32, 8, 1), (64, 32, 8, 2), (128, 24, 8, 1)])
+def test_runs_without_keys_behind_runs_with_keys(hd, H, KVH, blocks):
+    """More tiles than the chip holds workgroups, cut into more runs than the short ones have steps: a workgroup goes from a long
+    tile to one that is empty for it while its first group may still be taking over the long one's sums."""
+    portions = tuple((80, 80 + 640 * (s % 2)) for s in range(16))
+    assert run(portions, H, KVH, hd, 16, blocks, 8, None, 11) <= 0.0
+
+
 def test_the_rule():
     from nanoinfer_amd import kernels as K
     plan = K.mfma_group_plan
