@@ -16,8 +16,12 @@
 // that at most, no more than K 2^-24 sum |x||w|: the bound of a float32 sum.  And with few addends the sum's roundings do not
 // hide the halves': one product alone is off by 7e-8, 3.5e-8 in three parts.  So a tile in which some row of x has not at least
 // PAIR_TERMS (64) more big numbers than some row of W has others is made by the six bfloat16 products (split_tile.h), by the
-// same workgroup after its main loop; infinities and NaN count as no big number at all and end there too.  That takes such a tile
-// three times as long.  Normal deviates have one number in 2,900 that is not big, squared ReLU leaves half of them: neither gets there.
+// same workgroup instead of its main loop; infinities and NaN count as no big number at all and end there too.  Normal
+// deviates have one number in 2,900 that is not big, squared ReLU leaves half of them: neither gets there; a row of which one number
+// is 30,000 times the rest does.  What is known of the rows is asked for before anything else and looked at while the first stages are on
+// their way, which costs nothing.  Measured, no such row : one in the first tile : one in every tile : all by tile_gemm.hip (us): 512 rows on
+// [16384, 2048] with SwiGLU 107 : 198 : 215 : 177 (looked at behind the main loop 110 : 248 : 292), on [2048, 8192] 71 : 117 : 127 : 105,
+// 100 rows on [16384, 2048] 63 : 115 : 115 : 95, 2,000 rows there 368 : 496 : 771 : 620.
 //
 // Both operands come as halves: W once, when it is loaded, in the order of the lanes (pair_weight_kernel); x by a pass of its own
 // (pair_rows_kernel, 3.5 to 8 us for 100 to 2,000 rows of 2,048).  A workgroup is four wavefronts side by side, one on each matrix core
@@ -180,6 +184,11 @@ __global__ __launch_bounds__(256, MINB) void pair_gemm_kernel(const char* __rest
     __shared__ __attribute__((aligned(16))) char lds[LDS];
     __shared__ int few, many;
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    if (tid == 0) {
+        few = INT_MAX;
+        many = 0;
+    }
+    __syncthreads();
     const int t = tile_of_block(blockIdx.x, mtiles * ntiles);
     int m0 = (t % mtiles) * BM, ldw = K, rows = M, wtile = 0, wrow = 0, wstep = 0;
     const int nt = t / mtiles;
@@ -321,10 +330,6 @@ __global__ __launch_bounds__(256, MINB) void pair_gemm_kernel(const char* __rest
         at1 = at2;
         at2 = first;
     };
-    if (tid == 0) {
-        few = INT_MAX;
-        many = 0;
-    }
     // (in the order of the loop, so that what waits for the rows of x there does not wait for W)
     Rows first, second;
     fetch(first, sbeg);
@@ -333,9 +338,18 @@ __global__ __launch_bounds__(256, MINB) void pair_gemm_kernel(const char* __rest
     fetch(xs[1], sbeg + 3);
 #pragma unroll
     for (int r = 0; r < R - 1; ++r) weights(wreg[r], 2 * sbeg + r);
+    // is there a result that these products may not be exact enough for
+    if (tid < BM) atomicMin(&few, mine_x.y);
+#pragma unroll
+    for (int c = 0; c < (BN + 255) / 256; ++c)
+        if (tid + c * 256 < BN) atomicMax(&many, mine_w[c].y);
     put(first, at0);
     put(second, at1);
     __syncthreads();
+    if (few - PAIR_TERMS < many) {
+        split_tile<BM, BN, SWM, 4 / SWM, true, EPI, GROUPED>(x, w, out, M, N, K, m0, nt, share, kbeg, kend, ldw, groups.rows, act, lds);
+        return;
+    }
     if constexpr (AHEAD) read(xf[0], at0, 0);
     int s = sbeg;
     for (; s + 2 <= send; s += 2) {
@@ -344,23 +358,13 @@ __global__ __launch_bounds__(256, MINB) void pair_gemm_kernel(const char* __rest
     }
     if (s < send) stage(Which<0>{}, s);
 
-    // is there a result that these products may not be exact enough for
-    if (tid < BM) atomicMin(&few, mine_x.y);
     int* wexp = reinterpret_cast<int*>(lds);
     int* xexp = wexp + BN;
 #pragma unroll
     for (int c = 0; c < (BN + 255) / 256; ++c)
-        if (tid + c * 256 < BN) {
-            atomicMax(&many, mine_w[c].y);
-            wexp[tid + c * 256] = mine_w[c].x;
-        }
+        if (tid + c * 256 < BN) wexp[tid + c * 256] = mine_w[c].x;
     if (tid < BM) xexp[tid] = mine_x.x;
     __syncthreads();
-    if (few - PAIR_TERMS < many) {
-        __syncthreads();
-        split_tile<BM, BN, SWM, 4 / SWM, true, EPI, GROUPED>(x, w, out, M, N, K, m0, nt, share, kbeg, kend, ldw, groups.rows, act, lds);
-        return;
-    }
     const int cols = EPI == TG_GATED ? half : N;
     float* base = out + static_cast<size_t>(share) * rows * cols;
 #pragma unroll

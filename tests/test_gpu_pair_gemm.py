@@ -197,3 +197,27 @@ def test_what_pair_gemm_does_not_take(K):
                 lambda: K.pair_weight(w[:, :126].contiguous()), lambda: K.pair_rows(x.bfloat16())):
         with pytest.raises(K.KernelError):
             bad()
+
+
+def test_tiles_in_three_parts_do_not_pay_for_the_halves_first(K):
+    """A row with one number far above the rest in every tile: the product is the one in three parts, on larger tiles than that
+    would choose and so up to 1.25 times as long; with the loop of the halves before it it took 1.7 times."""
+    M, N, Kd = 512, 16384, 2048
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn(M, Kd, generator=g, device="cuda")
+    x[::32, 7] = 1e6
+    weights = [K.Weight(torch.randn(N, Kd, generator=g, device="cuda")) for _ in range(3)]
+    halved = K.HalvedRows(x, *K.pair_rows(x))
+
+    def elapsed(call):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for w in weights * 4:
+            call(w)
+        b.record()
+        b.synchronize()
+        return a.elapsed_time(b)
+
+    times = [(elapsed(lambda w: K.pair_gemm(halved, w)), elapsed(lambda w: K.split_gemm(x, w.rows))) for _ in range(12)][3:]
+    pair, split = (sorted(t)[len(t) // 2] for t in zip(*times))
+    assert pair <= 1.45 * split, f"{pair} ms against {split}"
