@@ -52,7 +52,9 @@ def build_parser() -> argparse.ArgumentParser:
     ap.add_argument("--max-decode-run", type=int, default=8,
                     help="decode steps run back to back on one scheduling decision (requests without a repetition penalty)")
     ap.add_argument("--one-weight-copy", action="store_true",
-                    help="keep every layer matrix once on the device (no re-tiled copy for decode steps: less memory, slower decoding)")
+                    help="keep every layer matrix once on the device (no re-tiled copies: less memory, slower steps)")
+    ap.add_argument("--no-pair-copies", action="store_true",
+                    help="do not keep large float32 matrices as pairs of halves too (less memory, slower prompts)")
     ap.add_argument("--json", action="store_true", help="print the generated ids as one JSON line per request")
     return ap
 
@@ -81,7 +83,7 @@ def main(argv: List[str] = None) -> int:
                        num_cache_blocks=args.num_cache_blocks, max_num_batched_tokens=args.max_num_batched_tokens,
                        max_model_len=args.max_model_len, max_decode_run=args.max_decode_run, dtype=_DTYPES[args.dtype],
                        kv_cache_bytes=None if args.kv_cache_gb is None else int(args.kv_cache_gb * (1 << 30)),
-                       one_weight_copy=args.one_weight_copy)
+                       one_weight_copy=args.one_weight_copy, pair_copies=not args.no_pair_copies)
     print(f"Model: {model_dir}  dtype: {args.dtype}", file=sys.stderr)
     t0 = time.perf_counter()
     engine = Engine(model_dir, cfg, ignore_eos=args.ignore_eos)

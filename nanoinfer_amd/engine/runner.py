@@ -215,6 +215,11 @@ class _Gpu:
         return int(torch.cuda.memory_reserved())
 
     @staticmethod
+    def free_bytes() -> int:
+        """Device memory that nobody holds, and what the allocator holds without using it."""
+        return int(torch.cuda.mem_get_info()[0] + torch.cuda.memory_reserved() - torch.cuda.memory_allocated())
+
+    @staticmethod
     def draw(logits, work, view: "DrawView", ones, zeros, out, uses_top_k: bool, uses_top_p: bool) -> torch.Tensor:
         """One token per row of ``logits`` into ``out`` by the sampling kernels, without a repetition penalty
         (``ones``: a penalty of 1 per row; ``zeros``: the empty lists of penalised tokens)."""
@@ -269,30 +274,32 @@ class ModelRunner:
     def __init__(self, model_dir: str, dtype: str = "bfloat16", page_size: int = 16, max_tokens: int = 4096,
                  max_requests: int = 64, device: Optional[torch.device] = None, use_graphs: bool = True,
                  warm_up: bool = True, max_step_tokens: Optional[int] = None, kv_cache_bytes: Optional[int] = None,
-                 graph_memory_bytes: Optional[int] = None, one_weight_copy: bool = False):
+                 graph_memory_bytes: Optional[int] = None, one_weight_copy: bool = False, pair_copies: bool = True):
         arch, config, spec = read_model_folder(model_dir)
         tensors = load_tensors(model_dir, spec)
         self._setup(spec, tensors, dtype, page_size, max_tokens, max_requests, device, use_graphs, warm_up,
                     max_step_tokens, kv_cache_bytes, graph_memory_bytes, arch=arch, config=config,
-                    one_weight_copy=one_weight_copy)
+                    one_weight_copy=one_weight_copy, pair_copies=pair_copies)
 
     @classmethod
     def from_spec(cls, spec, tensors: Dict[str, torch.Tensor], dtype: str = "bfloat16", page_size: int = 16,
                   max_tokens: int = 4096, max_requests: int = 64, device: Optional[torch.device] = None,
                   use_graphs: bool = True, warm_up: bool = False, max_step_tokens: Optional[int] = None,
                   kv_cache_bytes: Optional[int] = None, graph_memory_bytes: Optional[int] = None,
-                  one_weight_copy: bool = False) -> "ModelRunner":
+                  one_weight_copy: bool = False, pair_copies: bool = True) -> "ModelRunner":
         """A runner over a model given as data (a :class:`~nanoinfer_amd.config.spec.ModelSpec`) and its
         tensors by checkpoint name (CPU tensors), without a folder: the same model, cache manager and
         step function.  The tensors are checked against what the parts of the spec ask for."""
         from ..weights.loader import check_tensors
         self = cls.__new__(cls)
         self._setup(spec, check_tensors(spec, tensors), dtype, page_size, max_tokens, max_requests, device, use_graphs,
-                    warm_up, max_step_tokens, kv_cache_bytes, graph_memory_bytes, one_weight_copy=one_weight_copy)
+                    warm_up, max_step_tokens, kv_cache_bytes, graph_memory_bytes, one_weight_copy=one_weight_copy,
+                    pair_copies=pair_copies)
         return self
 
     def _setup(self, spec, tensors, dtype, page_size, max_tokens, max_requests, device, use_graphs, warm_up,
-               max_step_tokens, kv_cache_bytes, graph_memory_bytes, arch=None, config=None, one_weight_copy=False) -> None:
+               max_step_tokens, kv_cache_bytes, graph_memory_bytes, arch=None, config=None, one_weight_copy=False,
+               pair_copies=True) -> None:
         self.device = device or K.require_gpu()
         torch_dtype = {"bfloat16": torch.bfloat16, "bf16": torch.bfloat16,
                        "float32": torch.float32, "fp32": torch.float32}.get(dtype)
@@ -301,7 +308,8 @@ class ModelRunner:
         self.dtype = torch_dtype
         self.arch, self.config, self.spec = arch, config, spec
         # the products of decode steps stream a re-tiled copy of every layer matrix beside the rows that the
-        # library's product of prompt portions reads; ``one_weight_copy`` does without it (a slower decode step)
+        # products of prompt portions read, and large float32 matrices one more for those (``pair_copies``, where memory
+        # allows); ``one_weight_copy`` does without either (slower steps)
         self.rt = Runtime(torch_dtype, self.device, tiled=not one_weight_copy)
         el = 2 if torch_dtype == torch.bfloat16 else 4
         self.checkpoint_bytes = sum(t.numel() * (el if t.dim() > 1 else 4) for t in tensors.values())
@@ -319,6 +327,8 @@ class ModelRunner:
         self.cache = KVCacheManager(self.model.cache_needs(), self.page_size, num_pages, max_requests,
                                     dtype=torch_dtype, device=self.device, max_step_tokens=self.max_step_tokens,
                                     scatter_pages=True)   # requests of equal length would else hold runs at regular distances
+        if pair_copies and torch_dtype == torch.float32 and self.device.type == "cuda":
+            self.rt.hold_pairs(self.gpu.free_bytes())
         self.vocab_size = self.spec.vocab_size
         self.max_positions = self.model.max_positions
         self.eos_token_ids = tuple(self.spec.eos_token_ids)

@@ -101,10 +101,11 @@ class EngineConfig:
     max_model_len: Optional[int] = None  # longest request (prompt + generated); None: what model and pool allow
     max_decode_run: int = 8           # decode steps run back to back on one scheduling decision (1: never more than one)
     admission_headroom: int = 1       # pages left free for every request already running when another is admitted
-    one_weight_copy: bool = False     # keep every layer matrix once on the device (no re-tiled copy for decode steps: slower)
+    one_weight_copy: bool = False     # keep every layer matrix once on the device (no re-tiled copies: slower)
     graph_memory_bytes: Optional[int] = None  # device memory that recorded steps may hold together (None: the runner's default)
     dtype: str = "bfloat16"
     seed: int = 0
+    pair_copies: bool = True          # keep large float32 matrices as pairs of halves too, where memory allows (faster prompts)
 
     def validate(self) -> None:
         for name in ("max_batch_size", "max_sequences", "prefill_chunk_size", "block_size", "num_cache_blocks",

@@ -729,9 +729,18 @@ class Weight:
         self.rows_t = rows.t()        # the view the library product takes, made once
         self.tiles = tile_weight(rows) if tiled and rows.dtype in (torch.float32, torch.bfloat16) else None
         self.pairs = None
-        if ((tiled if pairs is None else pairs) and rows.is_cuda and rows.dtype == torch.float32 and rows.is_contiguous() and rows.data_ptr() % 16 == 0
-                and pair_holds(*rows.shape)):
-            self.pairs = pair_weight(rows)
+        if tiled if pairs is None else pairs:
+            self.hold_pairs()
+
+    def pair_bytes(self) -> int:
+        """Device memory that :meth:`hold_pairs` takes (0: this matrix is not held so)."""
+        rows = self.rows
+        holds = rows.is_cuda and rows.dtype == torch.float32 and rows.is_contiguous() and rows.data_ptr() % 16 == 0 and pair_holds(*rows.shape)
+        return pair_weight_bytes(*rows.shape) if holds else 0
+
+    def hold_pairs(self) -> None:
+        if self.pair_bytes():
+            self.pairs = pair_weight(self.rows)
 
     @property
     def shape(self):
@@ -1380,7 +1389,7 @@ torch.backends.cudnn.allow_tf32 = False
 
 # products of many rows on the matrix cores
 from .tile import (HalvedRows, add_rmsnorm_halved, experts_grouped, experts_grouped_wins, pair_gemm, pair_holds, pair_plan,  # noqa: E402,F401
-                   pair_rows, pair_weight, pair_wins, rows_of, split_gemm, split_plan, split_wins, takes_halved, tile_lib, tiled_gemm,
+                   pair_rows, pair_weight, pair_weight_bytes, pair_wins, rows_of, split_gemm, split_plan, split_wins, takes_halved, tile_lib, tiled_gemm,
                    tiled_plan, tiled_wins)
 # sums onto the residual stream, routed experts, the gated delta rule, attention with a bias by distance
 from .stream import (BIAS_ATTENTION_MFMA_FROM, DELTA_RUN_FROM, EXPERTS_FEW_ROWS, add_rmsnormed, add_vector,  # noqa: E402,F401

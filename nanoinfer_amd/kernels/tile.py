@@ -162,6 +162,12 @@ def _pair_planes(rows: int, K: int, device) -> Tuple[torch.Tensor, torch.Tensor]
     return (torch.empty(rows * -(-K // 32) * 128, dtype=torch.uint8, device=device), torch.empty(rows, 2, dtype=torch.int32, device=device))
 
 
+def pair_weight_bytes(N: int, K: int) -> int:
+    """Bytes of what :func:`pair_weight` makes of a matrix [N, K]: as many as the matrix, and eight a row."""
+    rows = -(-N // 32) * 32
+    return rows * (-(-K // 32) * 128 + 8)
+
+
 def pair_weight(rows: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """The float32 matrix [N, K] as :func:`pair_gemm` reads it: its numbers as two halves each, scaled by a power of two a
     row, and for every row int32 (that power, how many of its numbers are small beside its largest)."""
