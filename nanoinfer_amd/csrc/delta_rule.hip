@@ -532,12 +532,16 @@ template <int KTW, int MINE> struct RunOperands {
     float p[MINE];                                   // row (lane % 16) of P, columns 4 (lane / 16) + wave + waves * j
 };
 
-__global__ void __launch_bounds__(64 * scan_waves(KPT * PARTS / RUN > 0 ? KPT * PARTS / RUN : 1)) __attribute__((amdgpu_waves_per_eu(2)))
+constexpr int SCAN_TILES = KPT * PARTS / RUN > 0 ? KPT * PARTS / RUN : 1, SCAN_WAVES = scan_waves(SCAN_TILES);
+
+// (Three wavefronts a SIMD hold the operands of two runs up to two sixteens of channels each.  With two and three runs ahead one portion
+// of 1,500 tokens takes as long, 94 us, and steps of many requests more: 300 tokens beside 40 single ones 73.6 us, now 67.6.)
+__global__ void __launch_bounds__(64 * SCAN_WAVES) __attribute__((amdgpu_waves_per_eu(SCAN_TILES / SCAN_WAVES <= 2 ? 3 : 2)))
 delta_chunk_scan_kernel(const float* __restrict__ chunks, float* __restrict__ state, const int32_t* __restrict__ q_start,
                         const int32_t* __restrict__ q_len, const int32_t* __restrict__ state_slot, float* __restrict__ o, int H, int dv,
                         size_t state_stride) {
-    constexpr int DK = KPT * PARTS, KT = DK / RUN > 0 ? DK / RUN : 1, SW = scan_waves(KT), KTW = KT / SW, MINE = 4 / SW;
-    constexpr int AHEAD = KTW <= 2 ? 3 : 2;
+    constexpr int DK = KPT * PARTS, SW = SCAN_WAVES, KTW = SCAN_TILES / SW, MINE = 4 / SW;
+    constexpr int AHEAD = 2;
     using At = RunPlaces<DK>;
     __shared__ floatx4_t ushare[2][SW][WAVE], oshare[2][SW][WAVE];
     const int s = blockIdx.x, h = blockIdx.y;
@@ -589,9 +593,7 @@ delta_chunk_scan_kernel(const float* __restrict__ chunks, float* __restrict__ st
     };
     const int runs = (n + RUN - 1) / RUN;
     Operands ops[AHEAD];
-#pragma unroll
-    for (int j = 0; j < AHEAD; ++j) fetch(ops[j], min(j, runs - 1));
-    auto step = [&](Operands& x, int run) {
+    auto step = [&](auto more, Operands& x, int run) {
         floatx4_t ua = {0.f, 0.f, 0.f, 0.f}, ub = {0.f, 0.f, 0.f, 0.f}, oa = ua, ob = ua;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
@@ -633,16 +635,29 @@ delta_chunk_scan_kernel(const float* __restrict__ chunks, float* __restrict__ st
             oa = __builtin_amdgcn_mfma_f32_16x16x4f32(x.p[j], mine, oa, 0, 0, 0);
         }
         oshare[run & 1][wave][lane] = oa + ob;
-        fetch(x, min(run + AHEAD, runs - 1));
+        if constexpr (decltype(more)::value) fetch(x, min(run + AHEAD, runs - 1));
     };
-    int run = 0;
-    for (; run + AHEAD <= runs; run += AHEAD) {
+    if (runs <= AHEAD) {
+        // single tokens and short portions: their runs' operands once (asked for as in the loop, the last one's AHEAD times more, 8
+        // single tokens beside 60 took 31 us, 200 beside 60 500; now 19 and 213)
 #pragma unroll
-        for (int j = 0; j < AHEAD; ++j) step(ops[j], run + j);
+        for (int j = 0; j < AHEAD; ++j)
+            if (j < runs) fetch(ops[j], j);
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j)
+            if (j < runs) step(std::false_type{}, ops[j], j);
+    } else {
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j) fetch(ops[j], j);
+        int run = 0;
+        for (; run + AHEAD <= runs; run += AHEAD) {
+#pragma unroll
+            for (int j = 0; j < AHEAD; ++j) step(std::true_type{}, ops[j], run + j);
+        }
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j)
+            if (run + j < runs) step(std::false_type{}, ops[j], run + j);
     }
-#pragma unroll
-    for (int j = 0; j < AHEAD; ++j)
-        if (run + j < runs) step(ops[j], run + j);
     __syncthreads();
     read_out(runs - 1);
     if (live) {
@@ -681,7 +696,10 @@ NI_EXPORT int ni_delta_prepare(const void* proj, const void* low, const void* co
     if (dk != KPT * PARTS) return -1;
     const int C = 2 * G * dk + H * dv;
     if (dk > 256) return -2;
-    if (T >= 256 && !move_on) {                 // a wavefront takes four tokens where that still fills the chip
+    // A wavefront takes four tokens where that still fills the chip and most groups of four lie in one sequence: 16 heads of 128, one
+    // portion of 256 / 481 / 700 / 1,500 tokens (a token a workgroup : this) 15.3 : 17.6, 24.2 : 23.3, 32.6 : 27.3, 63.0 : 41.4; 300 beside 40
+    // single tokens 18.6 : 24.9, 481 beside 31 25.8 : 41.9, 16 portions of 20 17.8 : 22.3.
+    if (T >= 448 && T >= 64 * B && !move_on) {
         delta_prepare_kernel<<<dim3((T + 15) / 16, 2 * G + H), 256, 0, stream>>>((const float*)proj, (const float*)low, (const float*)conv,
                                                   (const float*)a_log, (const float*)dt_bias, (const float*)state,
                                                   (const int32_t*)seq_of_token, (const int32_t*)q_start,
@@ -721,7 +739,7 @@ NI_EXPORT int ni_delta_rule(const void* prep, void* chunks, void* state, const v
             const int runs = (max_q_len + RUN - 1) / RUN;
             delta_chunk_prepare_kernel<<<dim3(B, runs, H), 256, 0, stream>>>((const float*)prep, (float*)chunks, (const int32_t*)q_start,
                                                                              (const int32_t*)q_len, G, H, dv);
-            delta_chunk_scan_kernel<<<dim3(B, H, (dv + RUN - 1) / RUN), 64 * scan_waves(KPT * PARTS / RUN), 0, stream>>>(
+            delta_chunk_scan_kernel<<<dim3(B, H, (dv + RUN - 1) / RUN), 64 * SCAN_WAVES, 0, stream>>>(
                 (const float*)chunks, (float*)state, (const int32_t*)q_start, (const int32_t*)q_len, (const int32_t*)state_slot,
                 (float*)o, H, dv, state_stride);
         } else {

@@ -1,4 +1,4 @@
-"""The delta rule over steps of 256 tokens and more, whose rows are prepared four tokens at a time where a sequence allows it."""
+"""The delta rule over many tokens of many short and some longer sequences."""
 import pytest
 import torch
 
