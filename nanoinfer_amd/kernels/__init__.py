@@ -77,13 +77,15 @@ def _ptr(t: Optional[torch.Tensor]) -> ctypes.c_void_p:
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
 
 
 def _stream() -> ctypes.c_void_p:
-    """The current stream of the current device as the kernels' launch argument (the raw handle is
-    asked for directly: building a Stream object costs more than a small kernel's launch)."""
+    """The current stream of the current device as the kernels' launch argument (the raw handles are
+    asked for directly: building a Stream object costs more than a small kernel's launch, and a step asks a hundred times;
+    whoever launches has tensors on the GPU, so that the runtime is there)."""
     if _raw_stream is not None:
-        return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
+        return ctypes.c_void_p(_raw_stream(_device()))
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
@@ -720,15 +722,15 @@ def tile_weight(w: torch.Tensor) -> torch.Tensor:
 class Weight:
     """A matrix [out, in] as the products want it: ``rows`` as stored (for the library product of
     many rows), optionally ``tiles`` in the order the skinny product streams it, and ``pairs``: a large float32 matrix
-    on the GPU as two halves a number for :func:`pair_gemm`."""
+    on the GPU as two halves a number for :func:`pair_gemm` (``pair_lines``: from how many rows on)."""
 
-    __slots__ = ("rows", "tiles", "rows_t", "pairs")
+    __slots__ = ("rows", "tiles", "rows_t", "pairs", "pair_lines")
 
     def __init__(self, rows: torch.Tensor, tiled: bool = True, pairs: Optional[bool] = None):
         self.rows = rows
         self.rows_t = rows.t()        # the view the library product takes, made once
         self.tiles = tile_weight(rows) if tiled and rows.dtype in (torch.float32, torch.bfloat16) else None
-        self.pairs = None
+        self.pairs = self.pair_lines = None
         if tiled if pairs is None else pairs:
             self.hold_pairs()
 
@@ -740,7 +742,7 @@ class Weight:
 
     def hold_pairs(self) -> None:
         if self.pair_bytes():
-            self.pairs = pair_weight(self.rows)
+            self.pairs, self.pair_lines = pair_weight(self.rows), pair_lines(*self.rows.shape)
 
     @property
     def shape(self):
@@ -1274,7 +1276,9 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
             raise KernelError("a normed input and a residual output in one product are not compiled")
         out = torch.empty(x.shape[0], rows.shape[0], dtype=x.dtype, device=x.device)
         return skinny_gemm(x, weight, out)
-    halved, x = x, rows_of(x)
+    halved = x
+    if type(x) is HalvedRows:
+        x = x.x
     if not (x.is_cuda and rows.is_cuda):
         raise KernelError("linear needs GPU tensors")
     if not (x.dtype == rows.dtype):
@@ -1332,7 +1336,9 @@ def linear_swiglu(x, weight_gate_up, activation: str = "silu") -> torch.Tensor:
     the product for few rows, product then the SwiGLU kernel for many.  ``x`` may be a :class:`NormedInput`, or a
     :class:`ScaledInput` where :func:`swiglu_takes_scaled` holds, or :class:`HalvedRows`."""
     inter = weight_gate_up.shape[0] // 2
-    halved, x = x, rows_of(x)
+    halved = x
+    if type(x) is HalvedRows:
+        x = x.x
     out = torch.empty(x.shape[0], inter, dtype=x.dtype, device=x.device)
     if isinstance(x, ScaledInput) and not swiglu_takes_scaled(x.shape[0], x.shape[1], x.dtype, weight_gate_up):
         raise KernelError("this product cannot take a scaled input")
@@ -1363,7 +1369,9 @@ def linear_swiglu(x, weight_gate_up, activation: str = "silu") -> torch.Tensor:
 def linear_relu2(x, weight) -> torch.Tensor:
     """``relu(x . weight^T)^2`` in the type of ``x``: fused into the product for few rows, product then an elementwise kernel
     for many."""
-    halved, x = x, rows_of(x)
+    halved = x
+    if type(x) is HalvedRows:
+        x = x.x
     M, Kd = x.shape
     if skinny_wins(M, Kd, x.dtype, weight) if M <= SKINNY_MAX_ROWS else (skinny_deals(M, weight.shape[0], Kd, x.dtype, weight) and _plain(x)):
         out = torch.empty(M, weight.shape[0], dtype=x.dtype, device=x.device)
@@ -1388,8 +1396,8 @@ torch.backends.cuda.matmul.allow_tf32 = False
 torch.backends.cudnn.allow_tf32 = False
 
 # products of many rows on the matrix cores
-from .tile import (HalvedRows, add_rmsnorm_halved, experts_grouped, experts_grouped_wins, pair_gemm, pair_holds, pair_plan,  # noqa: E402,F401
-                   pair_rows, pair_weight, pair_weight_bytes, pair_wins, rows_of, split_gemm, split_plan, split_wins, takes_halved, tile_lib, tiled_gemm,
+from .tile import (HalvedRows, add_rmsnorm_halved, experts_grouped, experts_grouped_wins, pair_gemm, pair_holds, pair_lines,  # noqa: E402,F401
+                   pair_plan, pair_rows, pair_weight, pair_weight_bytes, pair_wins, rows_of, split_gemm, split_plan, split_wins, takes_halved, tile_lib, tiled_gemm,
                    tiled_plan, tiled_wins)
 # sums onto the residual stream, routed experts, the gated delta rule, attention with a bias by distance
 from .stream import (BIAS_ATTENTION_MFMA_FROM, DELTA_RUN_FROM, EXPERTS_FEW_ROWS, add_rmsnormed, add_vector,  # noqa: E402,F401

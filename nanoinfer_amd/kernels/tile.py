@@ -10,7 +10,7 @@ from typing import Optional, Tuple
 import torch
 
 from ..csrc import build as _build
-from . import GATED_ACTIVATIONS, KernelError, _check, _gpu, _load, _ptr, _stream, add_rmsnorm, core, dtype_code
+from . import GATED_ACTIVATIONS, SKINNY_MAX_ROWS, KernelError, _check, _gpu, _load, _ptr, _stream, add_rmsnorm, core, dtype_code
 
 COMPUTE_UNITS = 256
 
@@ -234,7 +234,8 @@ def add_rmsnorm_halved(h: torch.Tensor, pending: Optional[torch.Tensor], weight:
     if pending is not None:
         addends = pending.shape[0] if pending.dim() == 3 else 1
         _gpu(pending, "pending", torch.float32, (addends, T, d) if pending.dim() == 3 else (T, d))
-    if d % 32 or d > 8192 or T * (d + 31) >= 1 << 29 or any(t is not None and t.data_ptr() % 16 for t in (h, weight, pending)):
+    if (d % 32 or d > 8192 or T * (d + 31) >= 1 << 29
+            or (h.data_ptr() | weight.data_ptr() | (0 if pending is None else pending.data_ptr())) % 16):
         add_rmsnorm(h, pending, weight, eps, out)
         return HalvedRows(out, *pair_rows(out))
     planes, info = _pair_planes(T, d, h.device)
@@ -251,23 +252,44 @@ PAIR_FLOPS = 2.4e9
 # The same where x comes as pairs of halves (:class:`HalvedRows`): the pass over x is 4 to 5 us of those figures, a norm that does its
 # work takes 2 more.  [3072, 2048] at 164 rows (2.1 GFLOP) 29.8 in the library, 22.3 here and 5.0 for its shares; at 130 (1.6) both would take 22.
 PAIR_FLOPS_HALVED = 2.0e9
+# Steps of fewer rows than this are a portion beside running requests, launched one by one by a host that takes as long as their
+# kernels: a launch and two allocations more (10 to 15 us of it) cost what the kernels gain.  Rows of more than 8,192 numbers the
+# pass over x reads twice: [2048, 16384] at 69 rows (4.6 GFLOP) 44.7 in three parts, 45.5 here and 10.0 for the pass.  Steps of 68 / 96 /
+# 118 tokens, all products in three parts or from the library : by the lines above alone : by these (us): the 1B shape 2,828 : 2,745 : 2,652,
+# 3,114 : 2,970 : 2,876, 3,080 : 2,968 : 2,838; the 3B shape 6,845 : 6,349 : 6,279, 7,551 : 7,065 : 6,931, 7,422 : 6,923 : 6,778; 69 / 84 / 97 / 119 of
+# a hybrid with routed experts 2,406 : 2,587 : 2,475, 2,496 : 2,595 : 2,471, 2,576 : 2,599 : 2,468, 2,644 : 2,594 : 2,517;
+# recorded prompts of 66 / 100 / 127 tokens, the 1B shape, 2,520 : 2,336 : 2,318, 2,725 : 2,613 : 2,522, 2,808 : 2,717 : 2,531.
+PAIR_FEW_ROWS = 128
+PAIR_FLOPS_FEW = 4.3e9
+PAIR_FLOPS_FEW_LONG = 7.5e9
 
 
 def pair_wins(x, weight) -> bool:
     """Whether a float32 product of more rows than the skinny product takes goes to :func:`pair_gemm`: a matrix that is kept as
     pairs of halves and work enough to pay for the start and for the pass that makes pairs of x (:class:`HalvedRows` need none)."""
-    rows = rows_of(x)
-    return _pair_sized(*x.shape, x.dtype, weight, PAIR_FLOPS if rows is x else PAIR_FLOPS_HALVED) and rows.is_contiguous() and rows.data_ptr() % 16 == 0
+    lines = getattr(weight, "pair_lines", None)
+    if lines is None:
+        return False
+    halved = type(x) is HalvedRows
+    rows = x.x if halved else x
+    return (lines[halved] <= rows.shape[0] <= lines[2] and rows.dtype == torch.float32 and rows.is_contiguous()
+            and rows.data_ptr() % 16 == 0)
 
 
 def takes_halved(M: int, K: int, dtype: torch.dtype, weight) -> bool:
     """Whether the product of M rows as :class:`HalvedRows` goes there."""
-    return _pair_sized(M, K, dtype, weight, PAIR_FLOPS_HALVED)
+    lines = getattr(weight, "pair_lines", None)
+    return lines is not None and lines[1] <= M <= lines[2] and dtype == torch.float32
 
 
-def _pair_sized(M: int, K: int, dtype: torch.dtype, weight, flops: float) -> bool:
-    return (getattr(weight, "pairs", None) is not None and dtype == torch.float32 and M > 64
-            and 2.0 * M * weight.rows.shape[0] * K >= flops and M * (K + 31) < 1 << 29)
+def pair_lines(N: int, K: int) -> Tuple[int, int, int]:
+    """For a matrix [N, K] that is kept as pairs of halves: the rows of x, as they are and as :class:`HalvedRows`, from which a product
+    goes to :func:`pair_gemm`, and the most that it takes."""
+    def rows(flops):
+        return max(SKINNY_MAX_ROWS + 1, math.ceil(flops / (2 * N * K)))
+
+    few = rows(PAIR_FLOPS_FEW if K <= 8192 else PAIR_FLOPS_FEW_LONG)
+    return (few if few < PAIR_FEW_ROWS else max(PAIR_FEW_ROWS, rows(PAIR_FLOPS)), rows(PAIR_FLOPS_HALVED), ((1 << 29) - 1) // (K + 31))
 
 
 def pair_gemm(x, weight, out: Optional[torch.Tensor] = None, gated: Optional[str] = None, squared: bool = False,
@@ -461,7 +483,8 @@ def experts_grouped_wins(x, w_up, w_down, top: int, experts: int) -> bool:
     places = M * top
     plan, whole = (_grouped_pair_plan, pair_plan) if _experts_in_pairs(places, w_up, w_down, d, per, ff) else (_grouped_plan, split_plan)
     grouped = plan(places, per, d, experts)[0] + plan(places, d, ff, experts)[0] + 25.0 + (12.0 * d + 4.0 * per) * places / 4e6
-    return grouped < whole(M, experts * per, d)[2] + whole(M, d, experts * ff)[2]
+    # (some five launches more, which a host that is behind pays for: see PAIR_FEW_ROWS)
+    return grouped + (40.0 if M < PAIR_FEW_ROWS else 0.0) < whole(M, experts * per, d)[2] + whole(M, d, experts * ff)[2]
 
 
 def experts_grouped(x, w_up, w_down, chosen: torch.Tensor, mix: torch.Tensor, experts: int,

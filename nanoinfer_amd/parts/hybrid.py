@@ -549,7 +549,7 @@ class ParallelBlock(Block):
         n = normed_rows(self.norm, h, pending_for(self.norm, pending, self.rt.dtype), readers)
 
         def for_part(part):
-            return n if takes_halved(part, h.shape[0]) else K.rows_of(n)
+            return n if type(n) is not K.HalvedRows or takes_halved(part, h.shape[0]) else n.x
 
         a = self.mixer.forward(for_part(self.mixer), ctx, cache)
         f = self.ffn.forward(for_part(self.ffn), ctx) if "ffn" in self.roles else None

@@ -115,9 +115,13 @@ class RMSNorm(Part):
 def normed_rows(norm, h: torch.Tensor, pending: Optional[torch.Tensor], parts):
     """``norm.forward(h, pending)`` for all of ``parts``, as pairs of halves too where the norm can leave them and one of the
     parts reads them.  Whichever does not gets the rows: ``K.rows_of`` of the result."""
-    leaves = getattr(norm, "leaves_halved", None)
-    if leaves is not None and leaves() and any(takes_halved(part, h.shape[0]) for part in parts):
-        return norm.forward_halved(h, pending)
+    T = h.shape[0]
+    if T > K.SKINNY_MAX_ROWS:
+        leaves = getattr(norm, "leaves_halved", None)
+        if leaves is not None and leaves():
+            for part in parts:
+                if takes_halved(part, T):
+                    return norm.forward_halved(h, pending)
     return norm.forward(h, pending)
 
 
