@@ -503,12 +503,17 @@ def _f32_cost(items: int, tokens: int, max_keys: int, hd: int, nsplit: int) -> f
 
 @functools.lru_cache(maxsize=4096)
 def _f32_runs(items: int, tokens: int, max_keys: int, hd: int) -> int:
-    """(From 256 keys on two runs are never more than 5 % behind one.)"""
+    """Two runs or more where the chip holds the tiles in one or two rounds: beside one run there never more than 2 us behind.  With more
+    tiles than that a cut only adds its merge and its scratch: 32 heads of 64 on 8, in one : two runs, us, 2,048 tokens at 2,048 keys (512
+    items) 142 : 136, 4,096 at 4,096 (1,024) 393 : 439, 8,192 at 8,192 1,526 : 1,616; 24 of 128 on 8, 1,024 at 1,024 (512) 92 : 85, 2,048 at 2,048
+    (1,024) 239 : 264, 8,192 at 8,192 3,607 : 3,749."""
+    if items >= 4 * COMPUTE_UNITS:
+        return 1
     return min(range(2, min(max_keys // 32, 16) + 1), key=lambda n: _f32_cost(items, tokens, max_keys, hd, n))
 
 
 def mfma_splits(n_tiles: int, kv_heads: int, group: int, max_keys: int, hd: int = 64,
-                dtype: torch.dtype = torch.bfloat16) -> int:
+                dtype: torch.dtype = torch.bfloat16, alone: bool = True) -> int:
     """Into how many runs the matrix-core kernel cuts the keys of every tile.  Cutting costs a
     second kernel that merges the runs, and float32 partial results in between: a step with many
     tiles is cut only into runs of 2,048 keys or more, up to about a thousand workgroups (measured
@@ -519,8 +524,11 @@ def mfma_splits(n_tiles: int, kv_heads: int, group: int, max_keys: int, hd: int 
     every unit has one.
 
     In float32: by the estimate of :func:`_f32_cost`; not under 256 keys (32 tokens at 200 keys 16.2 us uncut, 10 cut, but five prompts
-    through a small model 7.2 ms uncut, 7.4 cut, which is the host's time)."""
-    if dtype == torch.float32 and max_keys < 256:
+    through a small model 7.2 ms uncut, 7.4 cut, which is the host's time), nor under 512 up to head size 64 where the portion is not
+    ``alone`` in its step: such steps are launched one by one.  8 single tokens beside 40 / 60 / 100 / 300 / 481, 240 keys before them, 1B shape,
+    us a step, uncut : cut: 2,160 : 2,312, 2,792 : 2,885, 2,908 : 2,893, 4,474 : 4,462, 5,192 : 5,272; beside 60 behind 500 keys 2,975 : 2,885.  (Head
+    size 128, 3B shape: 60 / 160 / 300 / 481 6,478 : 6,296, 7,805 : 7,724, 10,604 : 10,628, 12,542 : 12,333.)"""
+    if dtype == torch.float32 and (max_keys < 256 or (not alone and max_keys < 512 and hd <= 64)):
         return 1            # a cut gains less than the launch of the merge costs a host that is behind
     hpt = _heads_per_tile(group)
     items = max(1, n_tiles * kv_heads * ((group + hpt - 1) // hpt))

@@ -400,10 +400,7 @@ class Attention(Part):
             tiles = ctx.q_tiles(tile_tokens)
         if tiles is not None:
             if nsplit is None:
-                # (short float32 portions beside others: the host, which launches such steps one by one, pays more for the merge:
-                # 8 tokens beside 60 at 300 keys, 1B shape, 2,951 us a step with runs, 2,819 without)
-                lone = T == ctx.max_q_len or dtype != torch.float32 or max_keys >= 512
-                nsplit = K.mfma_splits(tiles.shape[0], self.KVH, self.H // self.KVH, max_keys, self.hd, dtype) if lone else 1
+                nsplit = K.mfma_splits(tiles.shape[0], self.KVH, self.H // self.KVH, max_keys, self.hd, dtype, T == ctx.max_q_len)
             ws = ctx.workspace(T * self.H * nsplit * (self.hd + 2)) if nsplit > 1 else None
             K.mfma_attention(qkv, cache.kpool, cache.vpool, cache.block_table, tiles, out, self.H, self.KVH, self.hd,
                              self.scale, self.window, nsplit, ws, tile_tokens, groups)
