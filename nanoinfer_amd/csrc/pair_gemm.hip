@@ -19,9 +19,10 @@
 // same workgroup instead of its main loop; infinities and NaN count as no big number at all and end there too.  Normal
 // deviates have one number in 2,900 that is not big, squared ReLU leaves half of them: neither gets there; a row of which one number
 // is 30,000 times the rest does.  What is known of the rows is asked for before anything else and looked at while the first stages are on
-// their way, which costs nothing.  Measured, no such row : one in the first tile : one in every tile : all by tile_gemm.hip (us): 512 rows on
-// [16384, 2048] with SwiGLU 107 : 198 : 215 : 177 (looked at behind the main loop 110 : 248 : 292), on [2048, 8192] 71 : 117 : 127 : 105,
-// 100 rows on [16384, 2048] 63 : 115 : 115 : 95, 2,000 rows there 368 : 496 : 771 : 620.
+// their way: a maximum over each wavefront in registers and four numbers in LDS (by atomics there it takes 3 us).  Measured, no such
+// row : one in the first tile : one in every tile : all by tile_gemm.hip (us): 512 rows on [16384, 2048] with SwiGLU 110 : 191 : 206 : 178
+// (looked at behind the main loop 107 : 249 : 290), on [2048, 8192] 69 : 111 : 121 : 103, on [2048, 2048] 25 : 37 : 37 : 38, 100 rows on
+// [16384, 2048] 59 : 110 : 110 : 93, 2,000 rows there 355 : 478 : 760 : 610.
 //
 // Both operands come as halves: W once, when it is loaded, in the order of the lanes (pair_weight_kernel); x by a pass of its own
 // (pair_rows_kernel, 3.5 to 8 us for 100 to 2,000 rows of 2,048).  A workgroup is four wavefronts side by side, one on each matrix core
@@ -31,8 +32,8 @@
 // operands of a step are read during the step before (not where two workgroups share a unit and the registers do).
 //
 // Measured, recorded, every launch with another W, without the pass over x (us; six bfloat16 products : this): 512 rows on
-// [16384, 2048] with SwiGLU 179 : 101, on [2048, 8192] 101 : 62, on [3072, 2048] 48 : 31, on [2048, 2048] 37 : 22; 2,000 rows on
-// [16384, 2048] 643 : 380, on [4096, 14336] 1,105 : 574 (409 TFLOP/s); 100 rows on [16384, 2048] 103 : 64.  What bounds it is the clock
+// [16384, 2048] with SwiGLU 178 : 110, on [2048, 8192] 103 : 69, on [3072, 2048] 48 : 34, on [2048, 2048] 38 : 25; 2,000 rows on
+// [16384, 2048] 610 : 355 (378 TFLOP/s); 100 rows on [16384, 2048] 93 : 59; 200 rows on [3072, 2048] 32 : 21.  What bounds it is the clock
 // that the matrix cores hold: 256 workgroups of the largest tile take 0.68 us a step, eight 0.45 (of which the instructions are
 // 0.32), and with operands of ones, which switch less, 256 take 0.56.
 #include "pair_rows.h"
@@ -166,6 +167,18 @@ __global__ __launch_bounds__(PAIR_WEIGHT_WAVES * WAVE) void pair_weight_kernel(c
         info[n0 + tid] = make_int2(s, top == 0 ? 0 : top >= 0x7f800000u ? INT_MAX : K - bigs[tid]);
 }
 
+// The largest of a wavefront's numbers, in every lane.
+__device__ __forceinline__ int wave_max(int v) {
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x128, 0xf, 0xf, false));       // of a row of sixteen lanes: row_ror:8, :4, :2, :1
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x124, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x122, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x121, 0xf, 0xf, false));
+    const auto a = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    v = max(static_cast<int>(a[0]), static_cast<int>(a[1]));
+    const auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return max(static_cast<int>(b[0]), static_cast<int>(b[1]));
+}
+
 // What tells the groups' rows of W apart, beside Groups.
 struct PairGroups {
     int tiles;      // tiles of 32 rows of W from one group's to the next
@@ -182,13 +195,8 @@ __global__ __launch_bounds__(256, MINB) void pair_gemm_kernel(const char* __rest
     constexpr int ROWB = 128 + 16, SLAB = BM * ROWB, CX = BM * 8 / 256;
     constexpr int LDS = SplitLds<BM, BN>::BYTES > 3 * SLAB ? SplitLds<BM, BN>::BYTES : 3 * SLAB;
     __shared__ __attribute__((aligned(16))) char lds[LDS];
-    __shared__ int few, many;
+    __shared__ __attribute__((aligned(16))) int few_of[4], many_of[4];       // of every wavefront
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-    if (tid == 0) {
-        few = INT_MAX;
-        many = 0;
-    }
-    __syncthreads();
     const int t = tile_of_block(blockIdx.x, mtiles * ntiles);
     int m0 = (t % mtiles) * BM, ldw = K, rows = M, wtile = 0, wrow = 0, wstep = 0;
     const int nt = t / mtiles;
@@ -339,13 +347,21 @@ __global__ __launch_bounds__(256, MINB) void pair_gemm_kernel(const char* __rest
 #pragma unroll
     for (int r = 0; r < R - 1; ++r) weights(wreg[r], 2 * sbeg + r);
     // is there a result that these products may not be exact enough for
-    if (tid < BM) atomicMin(&few, mine_x.y);
+    int few = mine_x.y, many = mine_w[0].y;
 #pragma unroll
-    for (int c = 0; c < (BN + 255) / 256; ++c)
-        if (tid + c * 256 < BN) atomicMax(&many, mine_w[c].y);
+    for (int c = 1; c < (BN + 255) / 256; ++c) many = max(many, mine_w[c].y);
+    few = -wave_max(-few);
+    many = wave_max(many);
+    if (lane == 0) {
+        few_of[wave] = few;
+        many_of[wave] = many;
+    }
     put(first, at0);
     put(second, at1);
     __syncthreads();
+    const int4 f = *reinterpret_cast<const int4*>(few_of), m = *reinterpret_cast<const int4*>(many_of);
+    few = __builtin_amdgcn_readfirstlane(min(min(f.x, f.y), min(f.z, f.w)));
+    many = __builtin_amdgcn_readfirstlane(max(max(m.x, m.y), max(m.z, m.w)));
     if (few - PAIR_TERMS < many) {
         split_tile<BM, BN, SWM, 4 / SWM, true, EPI, GROUPED>(x, w, out, M, N, K, m0, nt, share, kbeg, kend, ldw, groups.rows, act, lds);
         return;
