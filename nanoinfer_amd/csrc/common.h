@@ -266,8 +266,10 @@ __device__ __forceinline__ int token_by_length(const int32_t* __restrict__ posit
 #define RANKED_TOKENS 256
 
 // e^t for t that is hardly above zero (a score less its reference, a difference of logarithms), as exact as expf in two thirds of its
-// instructions: the hardware's power of two (one unit in the last place) with the rounding of its argument made good.  Minus
-// infinity and what lies below the smallest number give zero, NaN stays NaN.
+// instructions: e^t = 2^(t log2 e) by the hardware's power of two (one unit in the last place), its argument as a sum of two float32
+// numbers (log2 e as two of them, the product's rounding by a fused multiply-add: a compensated product), and 2^(hi + lo) =
+// 2^hi (1 + lo ln 2) to first order, lo being at most a rounding of hi.  Minus infinity and what lies below the smallest number
+// give zero, NaN stays NaN.
 __device__ __forceinline__ float exp_below(float t) {
     t = t < -110.f ? -110.f : t;
     const float hi = t * 1.44269502f;

@@ -733,8 +733,9 @@ def bias_attention_mfma(qkv: torch.Tensor, kpool: torch.Tensor, vpool: torch.Ten
                         softcap: Optional[float] = None, chunk: Optional[int] = None, maps: int = 1,
                         workspace: Optional[torch.Tensor] = None, gate=None) -> torch.Tensor:
     """:func:`bias_attention` for steps with portions of prompts: tiles of up to 64 rows (tokens * heads of a chunk),
-    both products on the float32 matrix instructions, the same formula and the same 32-bit softmax; no runs.  ``out``
-    None: the rows are left in ``workspace`` (float32, T * H * (dv + 2)) unfinished, as runs of one."""
+    both products on the bfloat16 matrix instructions (a float32 number, and a weight beside bfloat16 values, as the bfloat16 numbers that
+    add up to it; rows that do not come in whole 16-byte pieces, and float32 keys of more than 128 channels, on the float32 ones), the same
+    formula and the same 32-bit softmax; no runs.  ``out`` None: the rows are left in ``workspace`` (float32, T * H * (dv + 2)) unfinished, as runs of one."""
     T, width = qkv.shape
     pages, G, ps, dk, dv = _map_sizes(kpool, vpool, maps)
     _gpu(qkv, "qkv")
