@@ -1,0 +1,260 @@
+// Products of many bfloat16 rows, y[M, N] = x[M, K] . W[N, K]^T, both operands as stored, with SwiGLU or squared ReLU in the epilogue.
+//
+// x and W go from memory straight into LDS (sixteen bytes a lane) and from there into the matrix cores' registers; no operand waits in
+// registers for LDS.  A stage is 64 columns of K: 128 bytes of a row, one line.  (With 32 columns a stage, half a line a row, a compute
+// unit takes in 69 GB/s whatever the source, with whole lines 137: a 256 x 256 tile 131 -> 116 us.)  Rows lie in LDS without gaps, as
+// such a load leaves them; which of a row's eight pieces of sixteen bytes stands where is turned round by the row's number when it is
+// asked for (wide_swizzle), so that the sixteen lanes that LDS serves at once meet no bank twice (counted: none).
+//
+// LDS is rings of stages, DX of x and DW of W.  While a half of a stage (32 columns) is multiplied the operands of the next half are
+// read, in a second set of registers; when a wavefront has read a stage it waits until its own loads of the next one have
+// landed, meets the others, and only then are the stage's places asked for anew: one barrier a stage, and loads have DX - 1 stages
+// and more to arrive.  x goes first, W a stage further ahead where LDS has room for it (two stages of each, 256 x 256 tiles: 5 % slower): W
+// comes from memory, x mostly from the caches.  Every ring slot is an array of its own, by which the compiler knows that a read does
+// not wait for loads into the others.
+//
+// The rows of x are taken in groups of WIDE_GROUP tiles, whose workgroups run on one die and share the lines of W in its L2; every
+// group begins at another stage of K, so that of two dies that need the same W one asks memory for the half that the other finds in
+// the memory-side cache: a unit has some 48 KB of lines on their way, 60 GB/s from memory and 115 from that cache
+// ([2048, 8192] at 1,536 rows 66 -> 55 us, [3072, 2048] at 1,999 30.6 -> 27.5; groups of eight tiles 62, of two as fast, but 21 us
+// for [2048, 2048] at 1,999 rows instead of 18).
+//
+// W is the first operand, and MFMA row 4 g + e of a block stands for row 16 g + 4 (block mod 4) + e of the tile's 64: a lane then holds sixteen
+// neighbouring columns of a row of y and stores whole vectors.  With SwiGLU a wavefront's blocks are half gate rows, half the up rows of
+// the same outputs.  Eight wavefronts, two a matrix core: given the whole register file (four wavefronts) the compiler moves
+// accumulators between its halves.  v_mfma_f32_16x16x32 instead of 32x32x16: 114 -> 107 us for [16384, 2048] at 1,999 rows, as the clock holds
+// 1.92 instead of 1.82 GHz.
+//
+// Measured (us, the library's product and the SwiGLU kernel : this; kernels/tile.py has more): [16384, 2048] with SwiGLU at 512 / 1,024 / 1,999 / 4,096 rows
+// 44 : 36, 68 : 58, 121 : 111, 239 : 211; [2048, 8192] at 1,999 70 : 62.  What bounds the large ones is the clock that the chip
+// holds: matrix cores busy 64 % of the time at 1.9 GHz (the library's 65 % at 1.96; with operands of ones, which switch less, 2.3 GHz and
+// 88 us); without its loads the same kernel takes 103.  A prompt of 1,999 tokens of the 1B shape 5,170 -> 4,630 us.
+#include "split_tile.h"
+
+template <int N> struct Index { static constexpr int value = N; };
+
+// sixteen bytes a lane from memory straight into LDS: lane l's land at `to` + 16 l, `to` the same in all lanes
+__device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t from, char* to, int lane_at, int at) {
+    typedef __attribute__((address_space(3))) char lds_char;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)(lds_char*)to, 16, lane_at, at, 0, 0);
+}
+
+// Which piece of sixteen bytes of row r stands where the row's piece 0 would.
+__device__ __forceinline__ int wide_swizzle(int r) { return (r & 2) << 1 | ((r >> 4 ^ r >> 5) & 1) << 1 | (r >> 4 & 1); }
+
+#define WIDE_GROUP 4            // tiles of x side by side
+
+template <int ROWS> struct WideSlot { char b[ROWS * 128]; };
+
+template <int BM, int BN, int WM, int WN, int DX, int DW, int EPI, typename OUT>
+__global__ __launch_bounds__(WM * WN * WAVE, 2) void wide_gemm_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                                                                            OUT* __restrict__ out, int M, int N, int K, int mtiles,
+                                                                            int ntiles, GatedUnit act) {
+    constexpr int NW = WM * WN, TM = BM / WM / 16, TN = BN / WN / 16;
+    constexpr int CX = BM / 8 / NW, CW = BN / 8 / NW, ALL = CX + CW;            // loads a wavefront and stage
+    static_assert((TM % 4 == 0 || TM == 2) && TN % 4 == 0 && BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "whole groups of 64 rows, whole loads a wavefront");
+    static_assert(DX >= 2 && DW >= DX && DW <= 5, "slots");
+    __shared__ __attribute__((aligned(1024))) WideSlot<BM> x0, x1, x2, x3, x4;
+    __shared__ __attribute__((aligned(1024))) WideSlot<BN> w0, w1, w2, w3, w4;
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int wm = wave / WN, wn = wave % WN;
+    const int t = tile_of_block(blockIdx.x, mtiles * ntiles);
+    const int g = t / (WIDE_GROUP * ntiles), gm = min(WIDE_GROUP, mtiles - g * WIDE_GROUP), rem = t - g * WIDE_GROUP * ntiles;
+    const int m0 = (g * WIDE_GROUP + rem % gm) * BM, nt = rem / gm;
+    const int steps = K / 64;
+    const int turn = g * (steps / ((mtiles + WIDE_GROUP - 1) / WIDE_GROUP));          // the stage that this group begins with
+    const int half = N / 2;
+    // where the columns of block j and lane group q of a wavefront start: GB blocks stand side by side in a lane's run
+    constexpr int GB = EPI == TG_GATED && TN == 4 ? 2 : 4;
+    auto column = [](int j, int q) { return j / GB * GB * 16 + q * GB * 4 + j % GB * 4; };
+    const auto xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(x), 0, M * K * 2, 0x00020000);
+    const auto wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(w), 0, N * K * 2, 0x00020000);
+    int xsrc[CX], wsrc[CW];
+#pragma unroll
+    for (int c = 0; c < CX; ++c) {
+        const int r = (wave + c * NW) * 8 + (lane >> 3);
+        xsrc[c] = min(m0 + r, M - 1) * K * 2 + ((lane & 7) ^ wide_swizzle(r)) * 16;
+    }
+#pragma unroll
+    for (int c = 0; c < CW; ++c) {
+        const int r = (wave + c * NW) * 8 + (lane >> 3);
+        int n;
+        if constexpr (EPI == TG_GATED) {       // gate rows are the first half of a wavefront's blocks, the up rows of the same outputs the other
+            const int wv = r / (TN * 16), b = r / 64 % (TN / 4) * 4 + (r >> 2 & 3);
+            n = b / (TN / 2) * half + min(nt * (BN / 2) + wv * (TN * 8) + column(b % (TN / 2), r >> 4 & 3) + (r & 3), half - 1);
+        } else {
+            n = min(nt * BN + r, N - 1);
+        }
+        wsrc[c] = n * K * 2 + ((lane & 7) ^ wide_swizzle(r)) * 16;
+    }
+    floatx4_t acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    auto xslot = [&](auto I) -> WideSlot<BM>& {
+        constexpr int i = decltype(I)::value % DX;
+        if constexpr (i == 0) return x0;
+        else if constexpr (i == 1) return x1;
+        else if constexpr (i == 2) return x2;
+        else if constexpr (i == 3) return x3;
+        else return x4;
+    };
+    auto wslot = [&](auto I) -> WideSlot<BN>& {
+        constexpr int i = decltype(I)::value % DW;
+        if constexpr (i == 0) return w0;
+        else if constexpr (i == 1) return w1;
+        else if constexpr (i == 2) return w2;
+        else if constexpr (i == 3) return w3;
+        else return w4;
+    };
+    // loads FROM to TO of the batch that may go out when stage s (in slots I) has been read: x of stage s + DX, then W of stage s + DW
+    auto fetch = [&](auto I, int s, auto FROM, auto TO) {
+        WideSlot<BM>& xs = xslot(I);
+        WideSlot<BN>& ws = wslot(I);
+        auto columns = [&](int s) {
+            const int at = min(s, steps - 1) + turn;
+            return (at - (at >= steps ? steps : 0)) * 128;
+        };
+        const int xat = columns(s + DX), wat = columns(s + DW);
+#pragma unroll
+        for (int c = decltype(FROM)::value; c < decltype(TO)::value; ++c) {
+            if (c < CX) load_to_lds(xr, xs.b + (wave + c * NW) * 1024, xsrc[c < CX ? c : 0], xat);
+            else load_to_lds(wr, ws.b + (wave + (c - CX) * NW) * 1024, wsrc[c < CX ? 0 : c - CX], wat);
+        }
+    };
+    struct Frags { bf16x8_t x[TM], w[TN]; };
+    Frags f[2];
+    const int row = (lane >> 2 & 3) * 16 + (lane & 3);
+    const int xblock = wm * TM;                                // this wavefront's first sixteen rows
+    int xo[2], wo[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int at = ((k * 4 + (lane >> 4)) ^ wide_swizzle(row)) * 16;
+        xo[k] = (xblock / 4 * 64 + xblock % 4 * 4 + row) * 128 + at;
+        wo[k] = (wn * TN * 16 + row) * 128 + at;
+    }
+    auto read = [&](Frags& fr, auto I, int k) {
+        const WideSlot<BM>& xs = xslot(I);
+        const WideSlot<BN>& ws = wslot(I);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) fr.x[i] = *reinterpret_cast<const bf16x8_t*>(xs.b + xo[k] + (i / 4) * 8192 + (i % 4) * 512);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) fr.w[j] = *reinterpret_cast<const bf16x8_t*>(ws.b + wo[k] + (j / 4) * 8192 + (j % 4) * 512);
+    };
+    auto multiply = [&](const Frags& fr) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fr.w[j], fr.x[i], acc[i][j], 0, 0, 0);
+    };
+    // between the products: the reads of the next operands, one every second, and LOADS loads
+    auto paced = [&](auto LOADS) {
+        constexpr int L = decltype(LOADS)::value;
+#pragma unroll
+        for (int q = 0; q < TM * TN; ++q) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (TM * TN < 2 * (TM + TN) || (q % 2 == 0 && q / 2 < TM + TN)) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            if (q * L / (TM * TN) != (q + 1) * L / (TM * TN)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // loads that may still be on their way when the next stage is read: all that were asked for after its last one
+    constexpr int WAITX = CW + (DX - 2) * ALL, WAITW = (DW - 2) * ALL, WAIT = WAITX < WAITW ? WAITX : WAITW;
+    constexpr int FIRST = (ALL + 1) / 2;
+    // (inside a half of a stage the compiler may order loads as it likes)
+    static_assert(DX == DW || FIRST == CX, "batches are counted whole, or x in the first half of a stage and W in the second");
+    auto stage = [&](auto I, int s) {
+        constexpr int i = decltype(I)::value;
+        read(f[1], I, 1);
+        fetch(Index<i + DX * DW - 1>{}, s - 1, Index<FIRST>{}, Index<ALL>{});
+        multiply(f[0]);
+        paced(Index<ALL - FIRST>{});
+        // this wavefront has read the stage, and its loads of the next one have landed; behind the barrier, every wavefront's
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(WAIT) : "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        read(f[0], Index<i + 1>{}, 0);
+        fetch(I, s, Index<0>{}, Index<FIRST>{});
+        multiply(f[1]);
+        paced(Index<FIRST>{});
+    };
+    // what stages before the first one would have asked for, in their order
+    auto ahead = [&](auto B) {
+        constexpr int b = decltype(B)::value;                  // stages before the first
+        constexpr int last = b == 1 ? FIRST : ALL;
+        if constexpr (b <= DX) fetch(Index<DX * DW - b>{}, -b, Index<0>{}, Index<(last < CX ? last : CX)>{});
+        if constexpr (b <= DW) fetch(Index<DX * DW - b>{}, -b, Index<CX>{}, Index<(last < CX ? CX : last)>{});
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    ahead(Index<5>{});
+    ahead(Index<4>{});
+    ahead(Index<3>{});
+    ahead(Index<2>{});
+    ahead(Index<1>{});
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(WAIT + FIRST) : "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    read(f[0], Index<0>{}, 0);
+    constexpr int PERIOD = DX == DW ? DX : DX * DW;
+    int s = 0;
+    for (; s + PERIOD <= steps; s += PERIOD) {
+#define WIDE_STAGE(i) if constexpr (i < PERIOD) stage(Index<i>{}, s + i);
+        WIDE_STAGE(0) WIDE_STAGE(1) WIDE_STAGE(2) WIDE_STAGE(3) WIDE_STAGE(4) WIDE_STAGE(5)
+#undef WIDE_STAGE
+    }
+#define WIDE_STAGE(i) if constexpr (i + 1 < PERIOD) if (s + i < steps) stage(Index<i>{}, s + i);
+    WIDE_STAGE(0) WIDE_STAGE(1) WIDE_STAGE(2) WIDE_STAGE(3) WIDE_STAGE(4)
+#undef WIDE_STAGE
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // (loads of stages behind the last: they land before the wavefront ends)
+
+    const int cols = EPI == TG_GATED ? half : N;
+    constexpr int OT = EPI == TG_GATED ? TN / 2 : TN;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const int m = m0 + (xblock + i) / 4 * 64 + (xblock + i) % 4 * 4 + row;
+        if (m >= M) continue;
+#pragma unroll
+        for (int j = 0; j < OT; j += GB) {
+            const int n = nt * (BN * OT / TN) + wn * OT * 16 + column(j, lane >> 4);
+            if (n >= cols) continue;
+            float v[GB * 4];
+#pragma unroll
+            for (int e = 0; e < GB * 4; ++e)
+                v[e] = EPI == TG_GATED ? act.rough(acc[i][j + e / 4][e % 4], acc[i][j + e / 4 + TN - OT][e % 4]) : act.plain(acc[i][j + e / 4][e % 4]);
+            OUT* to = out + static_cast<size_t>(m) * cols + n;
+            constexpr int V = 16 / sizeof(OUT);
+#pragma unroll
+            for (int e = 0; e < GB * 4; e += V) store_packed<OUT, V>(to + e, v + e);
+        }
+    }
+}
+
+template <int BM, int BN, int WM, int WN, int DX, int DW>
+static int launch_wide(const bf16_t* x, const bf16_t* w, void* out, int M, int N, int K, int gated, int f32, GatedUnit act, hipStream_t stream) {
+    const int cols = gated ? N / 2 : N, each = gated ? BN / 2 : BN, mt = (M + BM - 1) / BM, nt = (cols + each - 1) / each;
+    constexpr int T = WM * WN * WAVE;
+    if (gated) wide_gemm_kernel<BM, BN, WM, WN, DX, DW, TG_GATED, bf16_t><<<mt * nt, T, 0, stream>>>(x, w, static_cast<bf16_t*>(out), M, N, K, mt, nt, act);
+    else if (f32) wide_gemm_kernel<BM, BN, WM, WN, DX, DW, TG_STORE, float><<<mt * nt, T, 0, stream>>>(x, w, static_cast<float*>(out), M, N, K, mt, nt, act);
+    else wide_gemm_kernel<BM, BN, WM, WN, DX, DW, TG_STORE, bf16_t><<<mt * nt, T, 0, stream>>>(x, w, static_cast<bf16_t*>(out), M, N, K, mt, nt, act);
+    return NI_LAUNCH_RESULT();
+}
+
+// tile: 0 = 256 x 256, 1 = 128 x 256, 2 = 256 x 128, 3 and 4 = 128 x 128 (rows of x, rows of W; of 4 a unit holds two).  f32: float32 results
+NI_EXPORT int ni_wide_gemm(const void* x, const void* w, void* out, int M, int N, int K, int tile, int gated, int f32, int activation, int squared, void* stream) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 64 || N % (gated ? 32 : 16) || (gated && (f32 || squared)) || static_cast<long>(M) * K >= 1l << 30 ||
+        static_cast<long>(N) * K >= 1l << 30 || reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w) % 16 || reinterpret_cast<uintptr_t>(out) % 16)
+        return static_cast<int>(hipErrorInvalidValue);
+    GatedUnit act = GatedUnit::of(activation);
+    act.squared = squared != 0;
+    const bf16_t *xb = static_cast<const bf16_t*>(x), *wb = static_cast<const bf16_t*>(w);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    switch (tile) {
+        case 0: return launch_wide<256, 256, 2, 4, 2, 3>(xb, wb, out, M, N, K, gated, f32, act, s);
+        case 1: return launch_wide<128, 256, 2, 4, 3, 3>(xb, wb, out, M, N, K, gated, f32, act, s);
+        case 2: return launch_wide<256, 128, 4, 2, 3, 3>(xb, wb, out, M, N, K, gated, f32, act, s);
+        case 3: return launch_wide<128, 128, 4, 2, 5, 5>(xb, wb, out, M, N, K, gated, f32, act, s);
+        case 4: return launch_wide<128, 128, 2, 2, 2, 3>(xb, wb, out, M, N, K, gated, f32, act, s);
+        default: return static_cast<int>(hipErrorInvalidValue);
+    }
+}

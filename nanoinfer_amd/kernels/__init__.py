@@ -6,7 +6,7 @@ the call raises.  Matrix products that none of the kernels here takes or wins ar
 (``torch.matmul`` -> rocBLAS/hipBLASLt), as the reference takes its products from cuBLAS
 (src/op/kernels/cuda/matmul_kernel.cu:76-86): from 17 to 64 rows those that :func:`skinny_wins` leaves (float32 rows of more than
 2,048 elements, bfloat16 ones of more than 4,096 past 32 rows, matrices that are not re-tiled, as the vocabulary head); of more
-rows the bfloat16 ones that :func:`tiled_wins` leaves (past 512 rows nearly all) and the float32 ones under some 2.2 GFLOP that
+rows the bfloat16 ones that :func:`tiled_wins` and :func:`wide_wins` leave and the float32 ones under some 2.2 GFLOP that
 :func:`pair_wins`, :func:`split_wins` and :func:`skinny_deals` leave; and inputs that are not one aligned run of memory.
 """
 from __future__ import annotations
@@ -1257,7 +1257,7 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
            pending: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None, leave: Optional[NormSpec] = None,
            addends: bool = False):
     """``x . weight^T`` with ``weight`` stored [out, in].  Few rows go to the hand-written skinny
-    product, more of them to the tiled products (:func:`tiled_wins`, :func:`pair_wins`, :func:`split_wins`), the rest to the library
+    product, more of them to the tiled products (:func:`tiled_wins`, :func:`wide_wins`, :func:`pair_wins`, :func:`split_wins`), the rest to the library
     (rocBLAS/hipBLASLt; its reduced-precision matrix modes for float32 are switched off at import).
     ``out_dtype`` float32 keeps the float32 accumulators of a bfloat16 product.  ``x`` may be a
     :class:`NormedInput` where :func:`norm_prologue_ok` holds.  With ``residual`` (the float32
@@ -1325,6 +1325,8 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
         return split_gemm(x, rows, out, addends=addends)
     if tiled_wins(x, weight, addends=addends) and (out is None or out.data_ptr() % 16 == 0):
         return tiled_gemm(x, weight, out_dtype, out, addends=addends)
+    if wide_wins(x, rows) and (out is None or out.data_ptr() % 16 == 0):
+        return wide_gemm(x, rows, out_dtype, out)
     rows_t = weight.rows_t if isinstance(weight, Weight) else rows.t()
     global _library_calls
     _library_calls += 1
@@ -1366,6 +1368,8 @@ def linear_swiglu(x, weight_gate_up, activation: str = "silu") -> torch.Tensor:
         if split_plan(M, 2 * inter, Kd, True)[2] <= split_plan(M, 2 * inter, Kd)[2] + 4.0 + 12.0 * M * inter / 4e6:
             return split_gemm(x, rows, out, gated=activation)
         return swiglu(split_gemm(x, rows), out, activation)
+    if wide_wins(x, rows, gated=True):
+        return wide_gemm(x, rows, out=out, gated=activation)
     if tiled_wins(x, weight_gate_up, gated=True):
         return tiled_gemm(x, weight_gate_up, out=out, gated=activation)
     global _library_calls
@@ -1391,6 +1395,8 @@ def linear_relu2(x, weight) -> torch.Tensor:
         return split_gemm(x, rows, squared=True)
     if tiled_wins(x, weight):
         return tiled_gemm(x, weight, squared=True)
+    if wide_wins(x, rows):
+        return wide_gemm(x, rows, squared=True)
     return experts_act(linear(x, weight), None, weight.shape[0], "relu2")
 
 
@@ -1406,7 +1412,7 @@ torch.backends.cudnn.allow_tf32 = False
 # products of many rows on the matrix cores
 from .tile import (HalvedRows, add_rmsnorm_halved, experts_grouped, experts_grouped_wins, pair_gemm, pair_holds, pair_lines,  # noqa: E402,F401
                    pair_plan, pair_rows, pair_weight, pair_weight_bytes, pair_wins, rows_of, split_gemm, split_plan, split_wins, takes_halved, tile_lib, tiled_gemm,
-                   tiled_plan, tiled_wins)
+                   tiled_plan, tiled_wins, wide_gemm, wide_plan, wide_wins)
 # sums onto the residual stream, routed experts, the gated delta rule, attention with a bias by distance
 from .stream import (BIAS_ATTENTION_MFMA_FROM, DELTA_RUN_FROM, EXPERTS_FEW_ROWS, add_rmsnormed, add_vector,  # noqa: E402,F401
                      bias_attention, bias_attention_lib, bias_attention_mfma, bias_attention_mfma_rows, bias_attention_rows, bias_attention_runs, bias_attention_bf16_tokens, bias_attention_token_runs, delta_rule, delta_rule_lib, embed_scaled, experts_act, experts_few,

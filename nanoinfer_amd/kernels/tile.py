@@ -441,6 +441,103 @@ def tiled_gemm(x: torch.Tensor, weight, out_dtype: Optional[torch.dtype] = None,
     return out
 
 
+# ---------------------------------------------------------------- bfloat16, many rows, both operands as stored
+
+# Tiles of the product of csrc/wide_gemm.hip: rows of x, rows of W, workgroups a compute unit holds, and in microseconds: what a launch takes
+# beside its steps, 64 columns of K with one workgroup alone on its unit and with all units full, and how late between the two the
+# time rises (the power of the share of the units that is taken).  Fitted to sweeps of all tiles at 192 to 4,096 rows over the layer
+# sizes of the 1B, 3B and 8B shapes and smaller matrices, recorded, every launch with another W: of the plans taken the average is
+# 1 % above the best, the worst 30 (tiles that just outnumber the units).
+WIDE_TILES = ((256, 256, 1, 8.7, 1.055, 1.509, 2.5), (128, 256, 1, 5.1, 0.633, 0.858, 3.4), (256, 128, 1, 5.0, 0.618, 0.853, 3.0),
+              (128, 128, 1, 4.0, 0.320, 0.521, 1.4), (128, 128, 2, 3.8, 0.368, 0.942, 1.2))
+
+
+def wide_lib() -> ctypes.CDLL:
+    return _load(_build.WIDE_GEMM)
+
+
+def _wide_cost(M: int, N: int, K: int, tile: int) -> float:
+    """Microseconds of a product with this tile, by the figures above."""
+    bm, bn, held, fixed, alone, loaded, late = WIDE_TILES[tile]
+    full, rest = divmod(-(-M // bm) * -(-N // bn), COMPUTE_UNITS * held)
+    return fixed + K // 64 * (full * loaded + (alone + (loaded - alone) * (rest / (COMPUTE_UNITS * held)) ** late if rest else 0.0))
+
+
+def wide_plan(M: int, N: int, K: int, gated: bool = False) -> Tuple[int, float]:
+    """(tile, estimated microseconds) of :func:`wide_gemm`.  The largest tile and the one of which a unit holds two are for the product whose
+    epilogue makes gate and up one output: where a plain product would take them the library's is ahead ([4096, 4096] at 3,000 rows
+    87 : 78 us, [6144, 4096] at 1,999 88 : 84; [3072, 2048] at 1,300 and 1,600 26.6 : 23.5, 27.2 : 23.7)."""
+    return _wide_plan(_whole(M), N, K, gated)
+
+
+@functools.lru_cache(maxsize=4096)
+def _wide_plan(M: int, N: int, K: int, gated: bool) -> Tuple[int, float]:
+    cost, tile = min((_wide_cost(M, N, K, t), t) for t in (range(len(WIDE_TILES)) if gated else (1, 2, 3)))
+    return tile, cost
+
+
+WIDE_ROWS_GATED = 257       # rows from which a product with SwiGLU goes there, and a plain one, and to how many a plain one does
+WIDE_ROWS = 513
+WIDE_ROWS_LAST = 2048
+WIDE_FLOPS = 2e9            # operations of the smallest plain product that was measured ([2048, 1024] at 600 rows: 10.8 us in the library, 9.5 here)
+
+
+def wide_wins(x: torch.Tensor, rows: torch.Tensor, gated: bool = False) -> bool:
+    """Whether the bfloat16 product ``x . rows^T`` goes to :func:`wide_gemm`: where it is estimated to take no longer than the library's
+    product (with the SwiGLU kernel behind it): 5 to 8 us, 1 us for 1.33 GFLOP, and where its tiles are few 1.5 us for 1,024 elements of K (plain
+    products with 15 % more, by which few tiles are estimated too high).  Measured in recorded launches, each with another W (us, library : this; cards differ by 10 %):
+
+    SwiGLU in the epilogue, from 257 rows: [16384, 2048] at 400 / 512 / 900 / 1,024 / 1,300 / 1,600 / 1,999 / 3,000 / 4,096 rows 41 : 34,
+    44 : 36, 64 : 58, 68 : 58, 99 : 90, 113 : 102, 121 : 111, 183 : 157, 239 : 211 (the tiled product 37 at 400 and 39 at 512 rows),
+    [16384, 3072] at 512 / 1,024 / 1,999 62 : 52, 95 : 79, 172 : 152, [28672, 4096] at 512 / 1,999 108 : 102, 391 : 373, [4096, 2048] at
+    600 / 1,024 / 1,999 25 : 17, 29 : 21, 42 : 31.  Not where the tiles just outnumber the units ([16384, 2048] at 600 rows 49 : 56,
+    [16384, 3072] 67 : 74), and to 512 rows only on its larger tiles (a small matrix, [4096, 2048] at 512 rows, takes 19 in the smallest, 16 by
+    the tiled product); to 256 rows the tiled product is as fast or faster (26 : 28).
+
+    Plain, from 513 rows (the tiled product's end) to 2,048: [2048, 8192] at 1,024 / 1,600 / 1,999 50 : 58, 66 : 58, 70 : 62, [2048, 2048] at
+    768 / 1,150 / 1,600 / 1,999 13.3 : 14.8, 19.7 : 15.8, 20.1 : 17.3, 21.2 : 18 to 22, [3072, 2048] at 1,024 / 1,300 / 1,999 20.9 : 16.0,
+    23.5 : 26.6, 28.0 : 27.2, [4096, 4096] at 1,024 / 1,999 41 : 36, 59 : 57, [4096, 14336] at 1,300 / 1,999 157 : 171, 194 : 185.  With more rows
+    the tiles are as many as the library's larger ones, which then win ([3072, 2048] at 3,000 37 : 45, [2048, 8192] at 2,500 83 : 87)."""
+    if x.dtype != torch.bfloat16 or rows.dtype != torch.bfloat16 or x.dim() != 2 or rows.dim() != 2:
+        return False
+    M, K = x.shape
+    N = rows.shape[0]
+    if not ((WIDE_ROWS_GATED <= M if gated else WIDE_ROWS <= M <= WIDE_ROWS_LAST) and 0 < K and K % 64 == 0 and 0 < N and N % (32 if gated else 16) == 0
+            and N * K < 1 << 30 and M * K < 1 << 30 and x.is_contiguous() and rows.is_contiguous() and x.data_ptr() % 16 == 0 and rows.data_ptr() % 16 == 0):
+        return False
+    tile, cost = wide_plan(M, N, K, gated)
+    library = M * N * K / 0.665e9
+    if gated:
+        return (M >= WIDE_ROWS or tile < 3) and cost <= 12.0 + library + 3.0 * M * N / 4.6e6
+    return 2.0 * M * N * K >= WIDE_FLOPS and cost <= 1.15 * (5.0 + library + 1.5e-3 * K)
+
+
+def wide_gemm(x: torch.Tensor, rows: torch.Tensor, out_dtype: Optional[torch.dtype] = None, out: Optional[torch.Tensor] = None, gated: Optional[str] = None,
+              squared: bool = False, tile: Optional[int] = None) -> torch.Tensor:
+    """``x . rows^T`` for bfloat16 ``x`` [M, K] and ``rows`` [N, K] as stored, in bfloat16 or (``out_dtype``) float32.  ``gated`` and ``squared`` as for
+    :func:`split_gemm`.  ``tile``: another than :func:`wide_plan`'s."""
+    M, K = x.shape
+    N = rows.shape[0]
+    out_dtype = out_dtype or x.dtype
+    _gpu(x, "x", torch.bfloat16)
+    _gpu(rows, "w", torch.bfloat16, (N, K))
+    if gated is not None and (N % 32 or squared or out_dtype != torch.bfloat16):
+        raise KernelError("a gated product takes a stacked matrix of whole tiles, no other activation, and gives bfloat16")
+    if K % 64 or K == 0 or N % 16 or N == 0 or M == 0 or x.data_ptr() % 16 or rows.data_ptr() % 16 or M * K >= 1 << 30 or N * K >= 1 << 30:
+        raise KernelError(f"wide_gemm does not take [{M}, {K}] x [{N}, {K}]")
+    cols = N if gated is None else N // 2
+    if out is None:
+        out = torch.empty(M, cols, dtype=out_dtype, device=x.device)
+    _gpu(out, "out", out_dtype, (M, cols))
+    if out.data_ptr() % 16:
+        raise KernelError("out is not aligned to 16 bytes")
+    if tile is None:
+        tile = wide_plan(M, N, K, gated is not None)[0]
+    _check(wide_lib().ni_wide_gemm(_ptr(x), _ptr(rows), _ptr(out), M, N, K, tile, int(gated is not None), int(out_dtype == torch.float32),
+                                   GATED_ACTIVATIONS[gated or "silu"], int(squared), _stream()), "wide_gemm")
+    return out
+
+
 # ---------------------------------------------------------------- routed experts
 
 def _grouped_plan(places: int, N: int, K: int, groups: int) -> Tuple[float, int]:

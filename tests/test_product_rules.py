@@ -58,3 +58,19 @@ def test_where_bfloat16_products_of_many_rows_go(N, Kd, kind, here, there):
         assert K.tiled_wins(x, Stored(), **more) == (M in here), M
         tile, shares = K.tiled_plan(M, N, Kd, kind == "gated", kind == "addends")
         assert 0 <= tile < (3 if kind == "gated" else 4) and 1 <= shares <= (1 if kind == "gated" else 8) and (shares == 1 or Kd // shares >= 256)
+
+
+@pytest.mark.parametrize("N,Kd,gated,here,there", [
+    (16384, 2048, True, (400, 512, 900, 1024, 1999, 4096), (256, 600)), (4096, 2048, True, (600, 1024, 1999), (512,)),
+    (2048, 8192, False, (1600, 1999, 2048), (512, 1024, 2049)), (2048, 2048, False, (1024, 1600, 1999), (512, 640, 2049)),
+    (3072, 2048, False, (1024, 1999), (512, 1300, 1600, 3000)), (2040, 2048, False, (), (1999,)), (2048, 2080, False, (), (1999,)),
+    (16, 1 << 27, False, (), (1024,)), (1 << 25, 64, True, (), (1024,))])
+def test_where_bfloat16_products_of_many_rows_on_the_stored_matrix_go(N, Kd, gated, here, there):
+    """Both sides of the lines; what the kernel refuses (columns that are no whole vectors, bytes past 31 bits) the rule does not send there."""
+    rows = torch.empty(N, Kd, dtype=torch.bfloat16, device="meta")
+    for M in here + there:
+        assert K.wide_wins(torch.empty(M, Kd, dtype=torch.bfloat16, device="meta"), rows, gated) == (M in here), M
+    x = torch.empty(1024, Kd, device="meta")
+    assert not K.wide_wins(x, rows, gated) and not K.wide_wins(x, rows.float(), gated)
+    if Kd < 1 << 20:
+        assert not K.wide_wins(torch.empty(Kd, 1024, dtype=torch.bfloat16, device="meta").t(), rows, gated)
