@@ -386,6 +386,76 @@ __global__ void rope_kv_write_vec_kernel(T* __restrict__ qkv, const int32_t* __r
     }
 }
 
+// The same for a product that was cut along K: its shares' float32 sums [S][T][(H + 2 KVH) * hd] are added in their order, rotated and
+// stored, the queries in rows of their own.  One pass instead of two (512 rows of the 1B shape in float32, four shares of 6 MB: 6.3 us for a
+// kernel that adds them and 5.5 for the one above, 7.4 here): bound by the shares, which the caches hold.  Dims in vectors of four.
+// SHARES: how many, known to the compiler, so that all are asked for at once; 0: `S`.
+template <typename T, int SHARES>
+__global__ __launch_bounds__(256) void rope_kv_write_shares_kernel(const float* __restrict__ parts, int S, T* __restrict__ q, const int32_t* __restrict__ positions,
+                                                                   const float* __restrict__ cos_t, const float* __restrict__ sin_t,
+                                                                   const int32_t* __restrict__ slot_mapping, T* __restrict__ kpool,
+                                                                   T* __restrict__ vpool, int H, int KVH, int hd, int rot, int page_size) {
+    constexpr int V = 4;
+    const int t = blockIdx.x, half = rot / 2;
+    const size_t width = static_cast<size_t>(H + 2 * KVH) * hd, share = gridDim.x * width;
+    const float* row = parts + t * width;
+    const int pos = positions[t];
+    const int slot = slot_mapping ? slot_mapping[t] : -1;
+    const int page = slot >= 0 ? slot / page_size : 0, off = slot >= 0 ? slot % page_size : 0;
+    const int stored = H + (slot >= 0 ? 2 * KVH : 0);                  // heads that go somewhere
+    const int rot_vecs = half / V, pass_vecs = (hd - rot) / V, head_vecs = hd / V;
+    const int turned = min(stored, H + KVH), n_rot = turned * rot_vecs, n_pass = turned * pass_vecs;
+    auto sum = [&](int at, float* v) {
+        VecIO<float, V>::load(row + at, v);
+        if constexpr (SHARES > 0) {
+            float u[SHARES][V];
+#pragma unroll
+            for (int p = 1; p < SHARES; ++p) VecIO<float, V>::load(row + p * share + at, u[p]);
+#pragma unroll
+            for (int p = 1; p < SHARES; ++p)
+#pragma unroll
+                for (int e = 0; e < V; ++e) v[e] += u[p][e];
+        } else {
+            for (int p = 1; p < S; ++p) {
+                float u[V];
+                VecIO<float, V>::load(row + p * share + at, u);
+#pragma unroll
+                for (int e = 0; e < V; ++e) v[e] += u[e];
+            }
+        }
+    };
+    auto place = [&](int head) {
+        if (head < H) return q + (static_cast<size_t>(t) * H + head) * hd;
+        const int g = head < H + KVH ? head - H : head - H - KVH;
+        return (head < H + KVH ? kpool : vpool) + ((static_cast<size_t>(page) * KVH + g) * page_size + off) * hd;
+    };
+    for (int item = threadIdx.x; item < n_rot + n_pass + (stored - turned) * head_vecs; item += 256) {
+        if (item < n_rot) {
+            const int head = item / rot_vecs, j = (item % rot_vecs) * V;
+            float x0[V], x1[V], cs[V], sn[V], y0[V], y1[V];
+            sum(head * hd + j, x0);
+            sum(head * hd + j + half, x1);
+            VecIO<float, V>::load(cos_t + static_cast<size_t>(pos) * half + j, cs);
+            VecIO<float, V>::load(sin_t + static_cast<size_t>(pos) * half + j, sn);
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                y0[e] = x0[e] * cs[e] - x1[e] * sn[e];
+                y1[e] = x0[e] * sn[e] + x1[e] * cs[e];
+            }
+            T* dst = place(head);
+            store_packed<T, V>(dst + j, y0);
+            store_packed<T, V>(dst + j + half, y1);
+        } else {
+            const bool pass = item < n_rot + n_pass;
+            const int k = item - n_rot - (pass ? 0 : n_pass), vecs = pass ? pass_vecs : head_vecs;
+            const int head = k / vecs + (pass ? 0 : H + KVH), dim = (k % vecs) * V + (pass ? rot : 0);
+            float v[V];
+            sum(head * hd + dim, v);
+            store_packed<T, V>(place(head) + dim, v);
+        }
+    }
+}
+
 // The same, 16 bytes of gate and of up per thread (rows whose width is a multiple of V elements).
 // The bfloat16 instantiation takes the exponential with the hardware's exp2: its error is far
 // below the rounding of the stored result.
@@ -573,6 +643,29 @@ NI_EXPORT int ni_rope_kv_write(void* qkv, const void* positions, const void* cos
                                                             (const float*)cos_t, (const float*)sin_t,
                                                             (const int32_t*)slot_mapping, (bf16_t*)kpool,
                                                             (bf16_t*)vpool, H, KVH, hd, rot, page_size);
+    return NI_LAUNCH_RESULT();
+}
+
+// parts: float32 [shares][T][(H + 2 KVH) * hd]; q [T, H * hd] and the pools in `dtype`
+NI_EXPORT int ni_rope_kv_write_shares(const void* parts, int shares, void* q, const void* positions, const void* cos_t, const void* sin_t,
+                                      const void* slot_mapping, void* kpool, void* vpool, int T, int H, int KVH, int hd, int rot, int page_size, int dtype,
+                                      hipStream_t stream) {
+    if (T <= 0 || shares < 1 || H <= 0 || KVH <= 0 || hd <= 0 || hd % 4 || rot < 0 || rot > hd || rot % 8 || page_size <= 0 || (rot && (!cos_t || !sin_t)) ||
+        (slot_mapping && (!kpool || !vpool)) || !aligned_to(16, parts, q, cos_t) || !aligned_to(16, sin_t, kpool, vpool))
+        return static_cast<int>(hipErrorInvalidValue);
+    auto launch = [&](auto kernel, auto* qt, auto* kp, auto* vp) {
+        kernel<<<T, 256, 0, stream>>>((const float*)parts, shares, qt, (const int32_t*)positions, (const float*)cos_t, (const float*)sin_t,
+                                      (const int32_t*)slot_mapping, kp, vp, H, KVH, hd, rot, page_size);
+    };
+    auto typed = [&](auto* qt, auto* kp, auto* vp) {
+        using E = std::remove_pointer_t<decltype(qt)>;
+        if (shares == 2) launch(rope_kv_write_shares_kernel<E, 2>, qt, kp, vp);
+        else if (shares == 3) launch(rope_kv_write_shares_kernel<E, 3>, qt, kp, vp);
+        else if (shares == 4) launch(rope_kv_write_shares_kernel<E, 4>, qt, kp, vp);
+        else launch(rope_kv_write_shares_kernel<E, 0>, qt, kp, vp);
+    };
+    if (dtype == 0) typed((float*)q, (float*)kpool, (float*)vpool);
+    else typed((bf16_t*)q, (bf16_t*)kpool, (bf16_t*)vpool);
     return NI_LAUNCH_RESULT();
 }
 

@@ -33,6 +33,7 @@
 // that are not finite are therefore worked out again from the float32 operands (plain_dot), each by the lane that holds
 // it, and are what a float32 product gives: infinities with their sign, NaN where there is no answer.  Finite results
 // pay one multiplication; 1,999 rows on [16384, 2048] take 0.63 ms, 0.95 with an infinity in one row, 38 with one in every row.
+#include "rope_store.h"
 #include "split_tile.h"
 
 template <int BM, int BN, int WM, int WN, bool AHEAD, int EPI, bool GROUPED>
@@ -145,7 +146,7 @@ template <int N> struct Num { static constexpr int value = N; };
 template <int WN, int TM, int TN, int MINW, int EPI, typename OUT>
 __global__ __launch_bounds__(WN * WAVE, MINW) void tiled_gemm_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                                     OUT* __restrict__ out, int M, int N, int K, int per,
-                                                                    int mtiles, int ntiles, GatedUnit act) {
+                                                                    int mtiles, int ntiles, GatedUnit act, RopeStore rope) {
     constexpr int THREADS = WN * WAVE, BM = TM * 16, BNT = WN * TN;      // BNT: tiles of W a workgroup
     constexpr int ROWB = 128 + 16, SLAB = BM * ROWB;
     constexpr int CX = BM * 8 / THREADS;
@@ -173,6 +174,10 @@ __global__ __launch_bounds__(WN * WAVE, MINW) void tiled_gemm_kernel(const bf16_
         if constexpr (EPI == TG_GATED) {       // the first half of a wave's tiles are gate rows, the other half the up rows of the same outputs
             const int o = min(nt * (BNT / 2) + wave * (TN / 2) + j % (TN > 1 ? TN / 2 : 1), all / 2 - 1);
             n = (j / (TN > 1 ? TN / 2 : 1)) * (all / 2) + o;
+        } else if constexpr (EPI == TG_ROPE) { // a wave's two tiles are sixteen dims of a head's first half and the ones half a head behind them
+            static_assert(TN == 2, "a pair of tiles a wave");
+            const int o = min(nt * (BNT / 2) + wave, all / 2 - 1), pairs = rope.hd / 32;
+            n = o / pairs * 2 * pairs + o % pairs + j * pairs;
         } else {
             n = min(nt * BNT + wave * TN + j, all - 1);
         }
@@ -247,6 +252,25 @@ __global__ __launch_bounds__(WN * WAVE, MINW) void tiled_gemm_kernel(const bf16_
     if (p < pend) piece(Num<0>{}, p);
     if (p + 1 < pend) piece(Num<1>{}, p + 1);
 
+    if constexpr (EPI == TG_ROPE) {
+        const int o = nt * (BNT / 2) + wave, pairs = rope.hd / 32;
+        if (o >= all / 2) return;
+        int pos[TM], slot[TM];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int m = min(m0 + i * 16 + (lane & 15), M - 1);
+            pos[i] = rope.positions[m];
+            slot[i] = rope.slots ? rope.slots[m] : -1;
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int m = m0 + i * 16 + (lane & 15);
+            if (m >= M) continue;
+            const float a[4] = {acc[i][0][0], acc[i][0][1], acc[i][0][2], acc[i][0][3]}, b[4] = {acc[i][1][0], acc[i][1][1], acc[i][1][2], acc[i][1][3]};
+            rope.put<4>(m, pos[i], slot[i], o / pairs, o % pairs * 16 + (lane >> 4) * 4, a, b);
+        }
+        return;
+    }
     const int cols = EPI == TG_GATED ? N / 2 : N;
     OUT* base = out + static_cast<size_t>(share) * M * cols;
 #pragma unroll
@@ -274,15 +298,15 @@ static int launch_tiled(const bf16_t* x, const bf16_t* w, void* out, int M, int 
     if (epi == TG_GATED) {
         if constexpr (TN > 1) {
             const int nt = (tiles / 2 + BNT / 2 - 1) / (BNT / 2);
-            tiled_gemm_kernel<WN, TM, TN, MINW, TG_GATED, bf16_t><<<dim3(mt * nt), T, 0, stream>>>(x, w, static_cast<bf16_t*>(out), M, N, K, per, mt, nt, act);
+            tiled_gemm_kernel<WN, TM, TN, MINW, TG_GATED, bf16_t><<<dim3(mt * nt), T, 0, stream>>>(x, w, static_cast<bf16_t*>(out), M, N, K, per, mt, nt, act, RopeStore{});
             return NI_LAUNCH_RESULT();
         }
         return static_cast<int>(hipErrorInvalidValue);
     }
     const int nt = (tiles + BNT - 1) / BNT;
     const dim3 grid(mt * nt, shares);
-    if (f32) tiled_gemm_kernel<WN, TM, TN, MINW, TG_STORE, float><<<grid, T, 0, stream>>>(x, w, static_cast<float*>(out), M, N, K, per, mt, nt, act);
-    else tiled_gemm_kernel<WN, TM, TN, MINW, TG_STORE, bf16_t><<<grid, T, 0, stream>>>(x, w, static_cast<bf16_t*>(out), M, N, K, per, mt, nt, act);
+    if (f32) tiled_gemm_kernel<WN, TM, TN, MINW, TG_STORE, float><<<grid, T, 0, stream>>>(x, w, static_cast<float*>(out), M, N, K, per, mt, nt, act, RopeStore{});
+    else tiled_gemm_kernel<WN, TM, TN, MINW, TG_STORE, bf16_t><<<grid, T, 0, stream>>>(x, w, static_cast<bf16_t*>(out), M, N, K, per, mt, nt, act, RopeStore{});
     return NI_LAUNCH_RESULT();
 }
 
@@ -303,6 +327,36 @@ NI_EXPORT int ni_tiled_gemm(const void* x, const void* w, void* out, int M, int 
         case 1: return launch_tiled<4, 8, 2, 2>(xb, wb, out, M, N, K, shares, per, gated, f32, act, s);
         case 2: return launch_tiled<4, 4, 2, 4>(xb, wb, out, M, N, K, shares, per, gated, f32, act, s);
         case 3: return launch_tiled<4, 4, 1, 4>(xb, wb, out, M, N, K, shares, per, gated, f32, act, s);
+        default: return static_cast<int>(hipErrorInvalidValue);
+    }
+}
+
+template <int WN, int TM, int MINW>
+static int launch_tiled_rope(const bf16_t* x, const bf16_t* w, int M, int N, int K, const RopeStore& rope, hipStream_t stream) {
+    constexpr int BM = TM * 16;
+    const int mt = (M + BM - 1) / BM, nt = (N / 32 + WN - 1) / WN;
+    tiled_gemm_kernel<WN, TM, 2, MINW, TG_ROPE, bf16_t><<<dim3(mt * nt), WN * WAVE, 0, stream>>>(x, w, static_cast<bf16_t*>(nullptr), M, N, K, K / 64, mt, nt, GatedUnit{}, rope);
+    return NI_LAUNCH_RESULT();
+}
+
+// The product with the re-tiled stacked matrix [q; k; v] of (H + 2 KVH) heads of hd (whole pairs of 16): rotated queries to q, keys and values to
+// the pools.  tile: 0, 1 or 2 of ni_tiled_gemm
+NI_EXPORT int ni_tiled_qkv_rope(const void* x, const void* w, void* q, const void* positions, const void* cos_t, const void* sin_t, const void* slots, void* kpool,
+                                void* vpool, int M, int K, int H, int KVH, int hd, int page_size, int tile, void* stream) {
+    const long N = (H + 2l * KVH) * hd;
+    if (M <= 0 || K <= 0 || K % 64 || H <= 0 || KVH <= 0 || hd <= 0 || hd % 32 || page_size <= 0 || static_cast<long>(M) * K >= 1l << 30 || (N + 15) * K >= 1l << 30 ||
+        !q || !positions || !cos_t || !sin_t || (slots && (!kpool || !vpool)) ||
+        (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(kpool) | reinterpret_cast<uintptr_t>(vpool) |
+         reinterpret_cast<uintptr_t>(cos_t) | reinterpret_cast<uintptr_t>(sin_t)) % 16)
+        return static_cast<int>(hipErrorInvalidValue);
+    const RopeStore rope{(const int32_t*)positions, (const float*)cos_t, (const float*)sin_t, (const int32_t*)slots, (bf16_t*)q, (bf16_t*)kpool, (bf16_t*)vpool,
+                         H, KVH, hd, page_size};
+    const bf16_t *xb = static_cast<const bf16_t*>(x), *wb = static_cast<const bf16_t*>(w);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    switch (tile) {
+        case 0: return launch_tiled_rope<8, 8, 2>(xb, wb, M, static_cast<int>(N), K, rope, s);
+        case 1: return launch_tiled_rope<4, 8, 2>(xb, wb, M, static_cast<int>(N), K, rope, s);
+        case 2: return launch_tiled_rope<4, 4, 4>(xb, wb, M, static_cast<int>(N), K, rope, s);
         default: return static_cast<int>(hipErrorInvalidValue);
     }
 }

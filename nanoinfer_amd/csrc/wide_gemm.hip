@@ -29,6 +29,7 @@
 // 44 : 36, 68 : 58, 121 : 111, 239 : 211; [2048, 8192] at 1,999 70 : 62.  What bounds the large ones is the clock that the chip
 // holds: matrix cores busy 64 % of the time at 1.9 GHz (the library's 65 % at 1.96; with operands of ones, which switch less, 2.3 GHz and
 // 88 us); without its loads the same kernel takes 103.  A prompt of 1,999 tokens of the 1B shape 5,170 -> 4,630 us.
+#include "rope_store.h"
 #include "split_tile.h"
 
 template <int N> struct Index { static constexpr int value = N; };
@@ -49,7 +50,7 @@ template <int ROWS> struct WideSlot { char b[ROWS * 128]; };
 template <int BM, int BN, int WM, int WN, int DX, int DW, int EPI, typename OUT>
 __global__ __launch_bounds__(WM * WN * WAVE, 2) void wide_gemm_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                                             OUT* __restrict__ out, int M, int N, int K, int mtiles,
-                                                                            int ntiles, GatedUnit act) {
+                                                                            int ntiles, GatedUnit act, RopeStore rope) {
     constexpr int NW = WM * WN, TM = BM / WM / 16, TN = BN / WN / 16;
     constexpr int CX = BM / 8 / NW, CW = BN / 8 / NW, ALL = CX + CW;            // loads a wavefront and stage
     static_assert((TM % 4 == 0 || TM == 2) && TN % 4 == 0 && BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "whole groups of 64 rows, whole loads a wavefront");
@@ -65,7 +66,7 @@ __global__ __launch_bounds__(WM * WN * WAVE, 2) void wide_gemm_kernel(const bf16
     const int turn = g * (steps / ((mtiles + WIDE_GROUP - 1) / WIDE_GROUP));          // the stage that this group begins with
     const int half = N / 2;
     // where the columns of block j and lane group q of a wavefront start: GB blocks stand side by side in a lane's run
-    constexpr int GB = EPI == TG_GATED && TN == 4 ? 2 : 4;
+    constexpr int GB = EPI == TG_ROPE || (EPI == TG_GATED && TN == 4) ? 2 : 4;
     auto column = [](int j, int q) { return j / GB * GB * 16 + q * GB * 4 + j % GB * 4; };
     const auto xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(x), 0, M * K * 2, 0x00020000);
     const auto wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(w), 0, N * K * 2, 0x00020000);
@@ -82,6 +83,9 @@ __global__ __launch_bounds__(WM * WN * WAVE, 2) void wide_gemm_kernel(const bf16
         if constexpr (EPI == TG_GATED) {       // gate rows are the first half of a wavefront's blocks, the up rows of the same outputs the other
             const int wv = r / (TN * 16), b = r / 64 % (TN / 4) * 4 + (r >> 2 & 3);
             n = b / (TN / 2) * half + min(nt * (BN / 2) + wv * (TN * 8) + column(b % (TN / 2), r >> 4 & 3) + (r & 3), half - 1);
+        } else if constexpr (EPI == TG_ROPE) { // 64 columns are 32 neighbouring dims of a head's first half and the 32 half a head behind them
+            const int set = min(nt * (BN / 64) + r / 64, N / 64 - 1), sets = rope.hd / 64, b = r >> 2 & 3;
+            n = set / sets * rope.hd + b / 2 * (rope.hd / 2) + set % sets * 32 + column(b % 2, r >> 4 & 3) + (r & 3);
         } else {
             n = min(nt * BN + r, N - 1);
         }
@@ -208,6 +212,32 @@ __global__ __launch_bounds__(WM * WN * WAVE, 2) void wide_gemm_kernel(const bf16
 #undef WIDE_STAGE
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // (loads of stages behind the last: they land before the wavefront ends)
 
+    if constexpr (EPI == TG_ROPE) {
+        static_assert(TN == 4, "64 columns a wavefront");
+        const int set = nt * (BN / 64) + wn, sets = rope.hd / 64;
+        if (set >= N / 64) return;
+        const int head = set / sets, d = set % sets * 32 + column(0, lane >> 4);
+        int pos[TM], slot[TM];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int m = min(m0 + (xblock + i) / 4 * 64 + (xblock + i) % 4 * 4 + row, M - 1);
+            pos[i] = rope.positions[m];
+            slot[i] = rope.slots ? rope.slots[m] : -1;
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int m = m0 + (xblock + i) / 4 * 64 + (xblock + i) % 4 * 4 + row;
+            if (m >= M) continue;
+            float a[8], b[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                a[e] = acc[i][e / 4][e % 4];
+                b[e] = acc[i][2 + e / 4][e % 4];
+            }
+            rope.put<8>(m, pos[i], slot[i], head, d, a, b);
+        }
+        return;
+    }
     const int cols = EPI == TG_GATED ? half : N;
     constexpr int OT = EPI == TG_GATED ? TN / 2 : TN;
 #pragma unroll
@@ -231,30 +261,52 @@ __global__ __launch_bounds__(WM * WN * WAVE, 2) void wide_gemm_kernel(const bf16
 }
 
 template <int BM, int BN, int WM, int WN, int DX, int DW>
-static int launch_wide(const bf16_t* x, const bf16_t* w, void* out, int M, int N, int K, int gated, int f32, GatedUnit act, hipStream_t stream) {
-    const int cols = gated ? N / 2 : N, each = gated ? BN / 2 : BN, mt = (M + BM - 1) / BM, nt = (cols + each - 1) / each;
+static int launch_wide(const bf16_t* x, const bf16_t* w, void* out, int M, int N, int K, int epi, int f32, GatedUnit act, const RopeStore& rope, hipStream_t stream) {
+    const int cols = epi == TG_GATED ? N / 2 : N, each = epi == TG_GATED ? BN / 2 : BN, mt = (M + BM - 1) / BM, nt = (cols + each - 1) / each;
     constexpr int T = WM * WN * WAVE;
-    if (gated) wide_gemm_kernel<BM, BN, WM, WN, DX, DW, TG_GATED, bf16_t><<<mt * nt, T, 0, stream>>>(x, w, static_cast<bf16_t*>(out), M, N, K, mt, nt, act);
-    else if (f32) wide_gemm_kernel<BM, BN, WM, WN, DX, DW, TG_STORE, float><<<mt * nt, T, 0, stream>>>(x, w, static_cast<float*>(out), M, N, K, mt, nt, act);
-    else wide_gemm_kernel<BM, BN, WM, WN, DX, DW, TG_STORE, bf16_t><<<mt * nt, T, 0, stream>>>(x, w, static_cast<bf16_t*>(out), M, N, K, mt, nt, act);
+    if (epi == TG_GATED) {
+        wide_gemm_kernel<BM, BN, WM, WN, DX, DW, TG_GATED, bf16_t><<<mt * nt, T, 0, stream>>>(x, w, static_cast<bf16_t*>(out), M, N, K, mt, nt, act, rope);
+        return NI_LAUNCH_RESULT();
+    }
+    if constexpr (DX == 2) return static_cast<int>(hipErrorInvalidValue);      // (the tiles that only products with SwiGLU take)
+    else if (epi == TG_ROPE) wide_gemm_kernel<BM, BN, WM, WN, DX, DW, TG_ROPE, bf16_t><<<mt * nt, T, 0, stream>>>(x, w, static_cast<bf16_t*>(out), M, N, K, mt, nt, act, rope);
+    else if (f32) wide_gemm_kernel<BM, BN, WM, WN, DX, DW, TG_STORE, float><<<mt * nt, T, 0, stream>>>(x, w, static_cast<float*>(out), M, N, K, mt, nt, act, rope);
+    else wide_gemm_kernel<BM, BN, WM, WN, DX, DW, TG_STORE, bf16_t><<<mt * nt, T, 0, stream>>>(x, w, static_cast<bf16_t*>(out), M, N, K, mt, nt, act, rope);
     return NI_LAUNCH_RESULT();
 }
 
-// tile: 0 = 256 x 256, 1 = 128 x 256, 2 = 256 x 128, 3 and 4 = 128 x 128 (rows of x, rows of W; of 4 a unit holds two).  f32: float32 results
-NI_EXPORT int ni_wide_gemm(const void* x, const void* w, void* out, int M, int N, int K, int tile, int gated, int f32, int activation, int squared, void* stream) {
-    if (M <= 0 || N <= 0 || K <= 0 || K % 64 || N % (gated ? 32 : 16) || (gated && (f32 || squared)) || static_cast<long>(M) * K >= 1l << 30 ||
-        static_cast<long>(N) * K >= 1l << 30 || reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w) % 16 || reinterpret_cast<uintptr_t>(out) % 16)
+static int launch_wide_tile(int tile, const void* x, const void* w, void* out, int M, int N, int K, int epi, int f32, GatedUnit act, const RopeStore& rope,
+                            void* stream) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 64 || static_cast<long>(M) * K >= 1l << 30 || static_cast<long>(N) * K >= 1l << 30 ||
+        reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w) % 16 || reinterpret_cast<uintptr_t>(out) % 16)
         return static_cast<int>(hipErrorInvalidValue);
-    GatedUnit act = GatedUnit::of(activation);
-    act.squared = squared != 0;
     const bf16_t *xb = static_cast<const bf16_t*>(x), *wb = static_cast<const bf16_t*>(w);
     hipStream_t s = static_cast<hipStream_t>(stream);
     switch (tile) {
-        case 0: return launch_wide<256, 256, 2, 4, 2, 3>(xb, wb, out, M, N, K, gated, f32, act, s);
-        case 1: return launch_wide<128, 256, 2, 4, 3, 3>(xb, wb, out, M, N, K, gated, f32, act, s);
-        case 2: return launch_wide<256, 128, 4, 2, 3, 3>(xb, wb, out, M, N, K, gated, f32, act, s);
-        case 3: return launch_wide<128, 128, 4, 2, 5, 5>(xb, wb, out, M, N, K, gated, f32, act, s);
-        case 4: return launch_wide<128, 128, 2, 2, 2, 3>(xb, wb, out, M, N, K, gated, f32, act, s);
+        case 0: return launch_wide<256, 256, 2, 4, 2, 3>(xb, wb, out, M, N, K, epi, f32, act, rope, s);
+        case 1: return launch_wide<128, 256, 2, 4, 3, 3>(xb, wb, out, M, N, K, epi, f32, act, rope, s);
+        case 2: return launch_wide<256, 128, 4, 2, 3, 3>(xb, wb, out, M, N, K, epi, f32, act, rope, s);
+        case 3: return launch_wide<128, 128, 4, 2, 5, 5>(xb, wb, out, M, N, K, epi, f32, act, rope, s);
+        case 4: return launch_wide<128, 128, 2, 2, 2, 3>(xb, wb, out, M, N, K, epi, f32, act, rope, s);
         default: return static_cast<int>(hipErrorInvalidValue);
     }
+}
+
+// tile: 1 = 128 x 256, 2 = 256 x 128, 3 = 128 x 128 (rows of x, rows of W), gated also 0 = 256 x 256, 4 = 128 x 128, two a unit.  f32: float32 results
+NI_EXPORT int ni_wide_gemm(const void* x, const void* w, void* out, int M, int N, int K, int tile, int gated, int f32, int activation, int squared, void* stream) {
+    if (N % (gated ? 32 : 16) || (gated && (f32 || squared))) return static_cast<int>(hipErrorInvalidValue);
+    GatedUnit act = GatedUnit::of(activation);
+    act.squared = squared != 0;
+    return launch_wide_tile(tile, x, w, out, M, N, K, gated ? TG_GATED : TG_STORE, f32, act, RopeStore{}, stream);
+}
+
+// The product with the stacked matrix [q; k; v] of (H + 2 KVH) heads of hd (whole sets of 64): rotated queries to q, keys and values to the pools
+NI_EXPORT int ni_wide_qkv_rope(const void* x, const void* w, void* q, const void* positions, const void* cos_t, const void* sin_t, const void* slots, void* kpool,
+                               void* vpool, int M, int K, int H, int KVH, int hd, int page_size, int tile, void* stream) {
+    if (H <= 0 || KVH <= 0 || hd <= 0 || hd % 64 || page_size <= 0 || !q || !positions || !cos_t || !sin_t || (slots && (!kpool || !vpool)) ||
+        (reinterpret_cast<uintptr_t>(kpool) | reinterpret_cast<uintptr_t>(vpool) | reinterpret_cast<uintptr_t>(cos_t) | reinterpret_cast<uintptr_t>(sin_t)) % 16)
+        return static_cast<int>(hipErrorInvalidValue);
+    const RopeStore rope{(const int32_t*)positions, (const float*)cos_t, (const float*)sin_t, (const int32_t*)slots, (bf16_t*)q, (bf16_t*)kpool, (bf16_t*)vpool,
+                         H, KVH, hd, page_size};
+    return launch_wide_tile(tile, x, w, q, M, (H + 2 * KVH) * hd, K, TG_ROPE, 0, GatedUnit{}, rope, stream);
 }

@@ -190,6 +190,42 @@ def rope_kv_write(qkv: torch.Tensor, positions: torch.Tensor, cos: Optional[torc
                                    dtype_code(qkv.dtype), _stream()), "rope_kv_write")
 
 
+def rope_kv_write_shares(parts: torch.Tensor, positions: torch.Tensor, cos: Optional[torch.Tensor], sin: Optional[torch.Tensor],
+                         slot_mapping: Optional[torch.Tensor], kpool: Optional[torch.Tensor], vpool: Optional[torch.Tensor], H: int, KVH: int, hd: int,
+                         dtype: torch.dtype) -> torch.Tensor:
+    """:func:`rope_kv_write` of the sum of a product's float32 shares ``parts`` [S, T, (H+2KVH)*hd]: the rotated queries [T, H*hd] in ``dtype``,
+    which the pools have too."""
+    S, T, N = parts.shape
+    _gpu(parts, "parts", torch.float32, (S, T, (H + 2 * KVH) * hd))
+    _gpu(positions, "positions", torch.int32, (T,))
+    rot = 0
+    if cos is not None:
+        rot = 2 * cos.shape[1]
+        _gpu(cos, "cos", torch.float32)
+        _gpu(sin, "sin", torch.float32, cos.shape)
+    if rot > hd or not rope_shares_ok(hd, rot):
+        raise KernelError(f"the rotation of a product's shares does not take heads of {hd}, of which {rot} are rotated")
+    page_size = 1
+    if slot_mapping is not None:
+        _gpu(slot_mapping, "slot_mapping", torch.int32, (T,))
+        if kpool is None or vpool is None:
+            raise KernelError("a slot mapping needs both pools")
+        _gpu(kpool, "kpool", dtype)
+        _gpu(vpool, "vpool", dtype, kpool.shape)
+        if not (kpool.dim() == 4 and kpool.shape[1] == KVH and kpool.shape[3] == hd):
+            raise KernelError(f"pool must be [pages, {KVH}, page_size, {hd}], is {tuple(kpool.shape)}")
+        page_size = kpool.shape[2]
+    q = torch.empty(T, H * hd, dtype=dtype, device=parts.device)
+    _check(core().ni_rope_kv_write_shares(_ptr(parts), S, _ptr(q), _ptr(positions), _ptr(cos), _ptr(sin), _ptr(slot_mapping), _ptr(kpool), _ptr(vpool),
+                                          T, H, KVH, hd, rot, page_size, dtype_code(dtype), _stream()), "rope_kv_write_shares")
+    return q
+
+
+def rope_shares_ok(hd: int, rot: int) -> bool:
+    """Whether :func:`rope_kv_write_shares` takes heads of ``hd``, of which ``rot`` dims are rotated: vectors of four."""
+    return hd % 4 == 0 and rot % 8 == 0
+
+
 GATED_ACTIVATIONS = {"silu": 0, "gelu_tanh": 1}      # what a gated feed-forward may do to its gate
 
 
@@ -1411,7 +1447,7 @@ torch.backends.cudnn.allow_tf32 = False
 
 # products of many rows on the matrix cores
 from .tile import (HalvedRows, add_rmsnorm_halved, experts_grouped, experts_grouped_wins, pair_gemm, pair_holds, pair_lines,  # noqa: E402,F401
-                   pair_plan, pair_rows, pair_weight, pair_weight_bytes, pair_wins, rows_of, split_gemm, split_plan, split_wins, takes_halved, tile_lib, tiled_gemm,
+                   pair_plan, pair_rows, pair_weight, pair_weight_bytes, pair_wins, qkv_rope, qkv_rope_plan, rows_of, split_gemm, split_plan, split_wins, takes_halved, tile_lib, tiled_gemm,
                    tiled_plan, tiled_wins, wide_gemm, wide_plan, wide_wins)
 # sums onto the residual stream, routed experts, the gated delta rule, attention with a bias by distance
 from .stream import (BIAS_ATTENTION_MFMA_FROM, DELTA_RUN_FROM, EXPERTS_FEW_ROWS, add_rmsnormed, add_vector,  # noqa: E402,F401

@@ -558,6 +558,83 @@ def _grouped_pair_tiles(places: int, N: int, K: int, groups: int) -> Tuple[float
     return min((_pair_cost(places, N, K, t, 1, groups), t) for t in range(len(PAIR_TILES)))
 
 
+# ---------------------------------------------------------------- bfloat16, [q; k; v] with rotation and the cache's pages behind it
+
+ROPE_PASS = 3.5, 2.2e-3      # microseconds of the kernel that rotates and stores: a launch, and a row (4.3 at 512 rows, 7.9 at 1,999, the 1B shape)
+
+
+@functools.lru_cache(maxsize=4096)
+def _qkv_rope_plan(M: int, N: int, K: int, hd: int, tiled: bool) -> Optional[Tuple[bool, int]]:
+    """(whether on the re-tiled matrix, tile) of :func:`qkv_rope`, or None where the product and a kernel behind it are estimated to be faster."""
+    ahead = ROPE_PASS[0] + ROPE_PASS[1] * M
+    if M <= TILED_ROWS:
+        if not tiled:
+            return None
+        cost, tile = min((_tiled_cost(M, N, K, t, 1, False), t) for t in range(3))
+        return (True, tile) if cost <= _tiled_cost(M, N, K, *_tiled_plan(M, N, K, False, False), False) + ahead else None
+    if hd % 64 or 2.0 * M * N * K < WIDE_FLOPS:
+        return None
+    tile, cost = _wide_plan(M, N, K, False)
+    return (False, tile) if cost <= 1.15 * (5.0 + M * N * K / 0.665e9 + 1.5e-3 * K) + ahead else None
+
+
+def qkv_rope_plan(x, weight, hd: int, rotary_dim: int) -> Optional[Tuple[bool, int]]:
+    """How the product of more than 64 bfloat16 rows with the stacked matrix [q; k; v] rotates and stores in its epilogue (:func:`qkv_rope`), None where
+    it does not: heads rotated whole, of whole tiles, and a product that :func:`tiled_wins` sends to the re-tiled matrix or that the
+    one on the stored matrix makes in the time of the library's and the rotating kernel's.  Measured in recorded launches, each with
+    another W (us, product and kernel : this): see the two kernels."""
+    if not isinstance(x, torch.Tensor) or x.dtype != torch.bfloat16 or x.dim() != 2 or hd % 32 or rotary_dim != hd:
+        return None
+    M, K = x.shape
+    rows = getattr(weight, "rows", None)
+    if M <= SKINNY_MAX_ROWS or rows is None or rows.dtype != torch.bfloat16 or not (x.is_contiguous() and x.data_ptr() % 16 == 0):
+        return None
+    N = rows.shape[0]
+    if K == 0 or K % 64 or N == 0 or N % hd or M * K >= 1 << 30 or (N + 15) * K >= 1 << 30:
+        return None
+    if M <= TILED_ROWS:
+        if not tiled_wins(x, weight):
+            return None
+    elif not (rows.is_contiguous() and rows.data_ptr() % 16 == 0):
+        return None
+    return _qkv_rope_plan(_whole(M), N, K, hd, getattr(weight, "tiles", None) is not None)
+
+
+def qkv_rope(x: torch.Tensor, weight, positions: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, slot_mapping: Optional[torch.Tensor],
+             kpool: Optional[torch.Tensor], vpool: Optional[torch.Tensor], H: int, KVH: int, hd: int, plan: Tuple[bool, int]) -> torch.Tensor:
+    """``x . weight^T`` for many bfloat16 rows and the stacked matrix [q; k; v]: returns the rotated queries [M, H * hd]; rotated keys and
+    plain values go into the pools ([pages, KVH, page_size, hd]) at ``slot_mapping`` (below zero, or absent: not stored).  ``plan`` as
+    :func:`qkv_rope_plan` gives it."""
+    M, K = x.shape
+    on_tiles, tile = plan
+    rows, tiles = weight.rows, weight.tiles
+    _gpu(x, "x", torch.bfloat16)
+    _gpu(rows, "w_qkv", torch.bfloat16, ((H + 2 * KVH) * hd, K))
+    _gpu(positions, "positions", torch.int32, (M,))
+    _gpu(cos, "cos", torch.float32)
+    _gpu(sin, "sin", torch.float32, cos.shape)
+    N = rows.shape[0]
+    matrix = tiles if on_tiles else rows
+    if (hd % (32 if on_tiles else 64) or 2 * cos.shape[1] != hd or K == 0 or K % 64 or M * K >= 1 << 30 or (N + 15) * K >= 1 << 30 or matrix is None
+            or (on_tiles and tiles.numel() != N * K) or (x.data_ptr() | matrix.data_ptr() | cos.data_ptr() | sin.data_ptr()) % 16):
+        raise KernelError(f"qkv_rope does not take [{M}, {K}] x [{N}, {K}] with heads of {hd}, of which {2 * cos.shape[1]} are rotated")
+    page_size = 1
+    if slot_mapping is not None:
+        _gpu(slot_mapping, "slot_mapping", torch.int32, (M,))
+        if kpool is None or vpool is None:
+            raise KernelError("a slot mapping needs both pools")
+        _gpu(kpool, "kpool", torch.bfloat16)
+        _gpu(vpool, "vpool", torch.bfloat16, kpool.shape)
+        if not (kpool.dim() == 4 and kpool.shape[1] == KVH and kpool.shape[3] == hd) or (kpool.data_ptr() | vpool.data_ptr()) % 16:
+            raise KernelError(f"pool must be [pages, {KVH}, page_size, {hd}] at a multiple of 16 bytes, is {tuple(kpool.shape)}")
+        page_size = kpool.shape[2]
+    q = torch.empty(M, H * hd, dtype=torch.bfloat16, device=x.device)
+    launch = tile_lib().ni_tiled_qkv_rope if on_tiles else wide_lib().ni_wide_qkv_rope
+    _check(launch(_ptr(x), _ptr(matrix), _ptr(q), _ptr(positions), _ptr(cos), _ptr(sin), _ptr(slot_mapping), _ptr(kpool), _ptr(vpool), M, K, H, KVH, hd,
+                  page_size, tile, _stream()), "qkv_rope")
+    return q
+
+
 def _experts_in_pairs(places: int, w_up, w_down, d: int, per: int, ff: int) -> bool:
     """Whether both products of routed experts are made in half precision: matrices that are kept as pairs of halves, an
     expert's rows of up whole tiles of 32 and its columns of down whole stages."""

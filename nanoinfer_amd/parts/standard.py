@@ -374,13 +374,32 @@ class Attention(Part):
         return qkv
 
     def project_rotate_write(self, x, ctx, cache: LayerCache) -> torch.Tensor:
-        """Stages 1 and 2: by one kernel where few rows allow it and neither stage has been replaced."""
+        """Stages 1 and 2: by one kernel where the number of rows allows it and neither stage has been replaced."""
         T = x.shape[0]
-        if self._fused_projection(T, x.shape[1], x.dtype):
+        if T > K.SKINNY_MAX_ROWS:
+            cls = type(self)
+            if cls.project is Attention.project and cls.rotate_and_write is Attention.rotate_and_write:
+                return self._project_many(x, ctx, cache)
+        elif self._fused_projection(T, x.shape[1], x.dtype):
             cos, sin = self.position.tables()
             return K.skinny_qkv_rope(x, self.w_qkv, ctx.positions, cos, sin, cache.slot_mapping if cache.writes else None,
                                      cache.kpool, cache.vpool, self.H, self.KVH, self.hd)
         return self.rotate_and_write(self.project(x, ctx), ctx, cache)
+
+    def _project_many(self, x, ctx, cache: LayerCache) -> torch.Tensor:
+        """The same for many rows: in the product's epilogue where that is compiled and no slower, or in the pass that adds the shares of
+        a product that was cut along K."""
+        tables = self.position.tables()
+        cos, sin = tables if tables is not None else (None, None)
+        slots = cache.slot_mapping if cache.writes else None
+        rot = 0 if cos is None else 2 * cos.shape[1]
+        plan = K.qkv_rope_plan(x, self.w_qkv, self.hd, rot)
+        if plan is not None:
+            return K.qkv_rope(x, self.w_qkv, ctx.positions, cos, sin, slots, cache.kpool, cache.vpool, self.H, self.KVH, self.hd, plan)
+        qkv = K.linear(x, self.w_qkv, addends=K.rope_shares_ok(self.hd, rot))
+        if qkv.dim() == 3:
+            return K.rope_kv_write_shares(qkv, ctx.positions, cos, sin, slots, cache.kpool, cache.vpool, self.H, self.KVH, self.hd, x.dtype)
+        return self.rotate_and_write(qkv, ctx, cache)
 
     def attend(self, qkv: torch.Tensor, ctx, cache: LayerCache, leave_runs: bool = False):
         """Stage 3: every query of ``qkv`` over the keys and values of its sequence in the cache, up to its own

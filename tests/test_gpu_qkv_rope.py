@@ -1,0 +1,107 @@
+"""The products of many bfloat16 rows that rotate queries and keys and store keys and values in their epilogue, against the product
+and the rotating kernel one behind the other."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def K():
+    from nanoinfer_amd import kernels
+    return kernels
+
+
+# rows at the edges of tiles; heads whose halves are one, two and four blocks of a wavefront's columns; a last tile of columns that is not
+# whole; slots that are left out, and none at all
+@pytest.mark.parametrize("plan", [(True, 0), (True, 1), (True, 2), (False, 1), (False, 2), (False, 3)])
+@pytest.mark.parametrize("M,Kd,H,KVH,hd,page", [(65, 64, 1, 1, 64, 16), (129, 128, 6, 2, 64, 5), (300, 192, 3, 1, 128, 16), (257, 320, 2, 1, 192, 7),
+                                                (1100, 128, 4, 4, 64, 16), (200, 64, 5, 5, 32, 16)])
+def test_rotated_and_stored_as_by_the_kernel_behind_the_product(K, plan, M, Kd, H, KVH, hd, page):
+    if not plan[0] and hd % 64:
+        pytest.skip("on the stored matrix: heads of whole 64")
+    g = torch.Generator().manual_seed(M + hd)
+    N = (H + 2 * KVH) * hd
+    x, w = torch.randn(M, Kd, generator=g).bfloat16().cuda(), torch.randn(N, Kd, generator=g).bfloat16().cuda()
+    weight = K.Weight(w)
+    angle = torch.rand(2000, hd // 2, generator=g) * 6.28
+    cos, sin = angle.cos().cuda(), angle.sin().cuda()
+    positions = torch.randint(0, 2000, (M,), generator=g, dtype=torch.int32).cuda()
+    pages = M // page + 3
+    slots = torch.randperm(pages * page, generator=g)[:M].to(torch.int32)
+    slots[3] = -1
+    slots = slots.cuda()
+    sums = x.double() @ w.double().t()
+    size = (x.double().abs() @ w.double().abs().t()).view(M, H + 2 * KVH, 2, hd // 2)
+    heads = sums.view(M, H + 2 * KVH, 2, hd // 2)
+    c, s = cos.double()[positions.long()][:, None], sin.double()[positions.long()][:, None]
+    turned = torch.stack((heads[:, :, 0] * c - heads[:, :, 1] * s, heads[:, :, 0] * s + heads[:, :, 1] * c), dim=2)
+    want = torch.cat((turned[:, :H + KVH], heads[:, H + KVH:]), dim=1).reshape(M, H + 2 * KVH, hd)
+    # K roundings of a sum, three of the rotation, one to bfloat16
+    off = ((Kd + 12) * 2.0 ** -24 * size.sum(2, keepdim=True).expand_as(size)).reshape(M, H + 2 * KVH, hd) + 2.0 ** -8 * want.abs()
+    kept = slots >= 0
+    at = slots[kept].long()
+
+    def check(q, kpool, vpool):
+        assert bool(((q.double().view(M, H, hd) - want[:, :H]).abs() <= off[:, :H]).all())
+        for pool, first in ((kpool, H), (vpool, H + KVH)):
+            got = pool.permute(0, 2, 1, 3).reshape(-1, KVH, hd)[at].double()
+            assert bool(((got - want[kept, first:first + KVH]).abs() <= off[kept, first:first + KVH]).all())
+            untouched = torch.ones(pages * page, dtype=torch.bool, device="cuda")
+            untouched[at] = False
+            assert bool((pool.permute(0, 2, 1, 3).reshape(-1, KVH, hd)[untouched] == 7.0).all())
+
+    kpool, vpool = (torch.full((pages, KVH, page, hd), 7.0, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    q = K.qkv_rope(x, weight, positions, cos, sin, slots, kpool, vpool, H, KVH, hd, plan)
+    check(q, kpool, vpool)
+    assert torch.equal(K.qkv_rope(x, weight, positions, cos, sin, None, None, None, H, KVH, hd, plan), q)
+    kpool, vpool = (torch.full((pages, KVH, page, hd), 7.0, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    behind = K.wide_gemm(x, w) if N % 16 == 0 else None          # the product and the kernel behind it, within one rounding more
+    K.rope_kv_write(behind, positions, cos, sin, slots, kpool, vpool, H, KVH, hd)
+    assert bool(((behind[:, :H * hd].double().view(M, H, hd) - want[:, :H]).abs() <= off[:, :H] + 2.0 ** -8 * sums.abs().max()).all())
+
+
+def test_what_it_does_not_take(K):
+    x, weight = torch.zeros(100, 64, device="cuda", dtype=torch.bfloat16), K.Weight(torch.zeros(3 * 96, 64, device="cuda", dtype=torch.bfloat16))
+    pos, half = torch.zeros(100, device="cuda", dtype=torch.int32), torch.zeros(8, 48, device="cuda")
+    K.qkv_rope(x, weight, pos, half, half, None, None, None, 1, 1, 96, (True, 2))
+    pool = torch.zeros(8, 1, 16, 96, device="cuda", dtype=torch.bfloat16)
+    for bad in (lambda: K.qkv_rope(x, weight, pos, half, half, None, None, None, 1, 1, 96, (False, 3)),                # heads of 96 on the stored matrix
+                lambda: K.qkv_rope(x, weight, pos, half[:, :32].contiguous(), half[:, :32].contiguous(), None, None, None, 1, 1, 96, (True, 2)),
+                lambda: K.qkv_rope(x, weight, pos, half, half, None, None, None, 2, 1, 96, (True, 2)),
+                lambda: K.qkv_rope(x, weight, pos, half, half, pos, pool, None, 1, 1, 96, (True, 2)),
+                lambda: K.qkv_rope(x, weight, pos, half, half, pos, pool.float(), pool, 1, 1, 96, (True, 2)),
+                lambda: K.qkv_rope(x, weight, pos, half, half, None, None, None, 1, 1, 96, (True, 3))):
+        with pytest.raises(K.KernelError):
+            bad()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,S,H,KVH,hd,rot,page", [(1, 1, 1, 1, 64, 64, 16), (67, 2, 6, 2, 64, 64, 5), (130, 3, 3, 1, 80, 48, 16), (70, 4, 2, 2, 20, 8, 16), (65, 2, 4, 2, 64, 0, 7), (66, 6, 2, 1, 64, 64, 16)])
+def test_the_shares_of_a_cut_product_added_rotated_and_stored(K, dtype, T, S, H, KVH, hd, rot, page):
+    """In float32 bit for bit what adding them in their order and the rotating kernel make."""
+    g = torch.Generator().manual_seed(T + hd)
+    parts = torch.randn(S, T, (H + 2 * KVH) * hd, generator=g).cuda()
+    cos = sin = None
+    if rot:
+        angle = torch.rand(300, rot // 2, generator=g) * 6.28
+        cos, sin = angle.cos().cuda(), angle.sin().cuda()
+    positions = torch.randint(0, 300, (T,), generator=g, dtype=torch.int32).cuda()
+    pages = T // page + 3
+    slots = torch.randperm(pages * page, generator=g)[:T].to(torch.int32)
+    slots[T // 2] = -1
+    slots = slots.cuda()
+    pools = [torch.full((pages, KVH, page, hd), 7.0, device="cuda", dtype=dtype) for _ in range(2)]
+    q = K.rope_kv_write_shares(parts, positions, cos, sin, slots, *pools, H, KVH, hd, dtype)
+    whole = parts[0].clone()
+    for p in range(1, S):
+        whole += parts[p]
+    want = [torch.full((pages, KVH, page, hd), 7.0, device="cuda") for _ in range(2)]
+    K.rope_kv_write(whole, positions, cos, sin, slots, *want, H, KVH, hd)
+    for got, true in ((q, whole[:, :H * hd].contiguous()), *zip(pools, want)):
+        assert torch.equal(got, true.to(dtype))                # both round to nearest
+    assert torch.equal(K.rope_kv_write_shares(parts, positions, cos, sin, None, None, None, H, KVH, hd, dtype), q)
+    for bad in (lambda: K.rope_kv_write_shares(parts[:, :, :-4], positions, cos, sin, None, None, None, H, KVH, hd, dtype),
+                lambda: K.rope_kv_write_shares(parts, positions, cos, sin, slots, pools[0], None, H, KVH, hd, dtype)):
+        with pytest.raises(K.KernelError):
+            bad()
