@@ -59,29 +59,14 @@ __device__ __forceinline__ uint32_t top_bits(const float* v, uint32_t top) {
     return top;
 }
 
-// Rows of x: a workgroup a row, C chunks of eight numbers a thread in registers (C = 0: read twice).
+// A row's numbers, C chunks of eight a thread (C = 0: read again), and its thread's part of the row's largest bits, as pairs of halves; by a
+// workgroup of 256.
 template <int C>
-__global__ __launch_bounds__(256) void pair_rows_kernel(const float* __restrict__ x, char* __restrict__ planes, int2* __restrict__ info, int K) {
+__device__ __forceinline__ void row_to_pairs(float (&v)[C ? C : 1][8], uint32_t top, const float* __restrict__ row, int K, char* __restrict__ to,
+                                             int2* __restrict__ info) {
     __shared__ uint32_t tops[4];
     __shared__ int bigs[4];
     const int kp = (K + 31) & ~31, tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE;
-    const float* row = x + static_cast<size_t>(blockIdx.x) * K;
-    char* to = planes + static_cast<size_t>(blockIdx.x) * kp * 4;
-    float v[C ? C : 1][8];
-    uint32_t top = 0;
-    if constexpr (C) {
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            const int k = (tid + c * 256) * 8;
-            load8(row, k, K, v[c]);
-            top = top_bits(v[c], top);
-        }
-    } else {
-        for (int k = tid * 8; k < K; k += 2048) {
-            load8(row, k, K, v[0]);
-            top = top_bits(v[0], top);
-        }
-    }
 #pragma unroll
     for (int off = WAVE / 2; off > 0; off >>= 1) top = max(top, static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), off, WAVE)));
     if (lane == 0) tops[wave] = top;
@@ -117,8 +102,68 @@ __global__ __launch_bounds__(256) void pair_rows_kernel(const float* __restrict_
     __syncthreads();
     if (tid == 0) {
         big = bigs[0] + bigs[1] + bigs[2] + bigs[3];
-        info[blockIdx.x] = pair_row_info(s, top, big);
+        *info = pair_row_info(s, top, big);
     }
+}
+
+// Rows of x: a workgroup a row, C chunks of eight numbers a thread in registers (C = 0: read twice).
+template <int C>
+__global__ __launch_bounds__(256) void pair_rows_kernel(const float* __restrict__ x, char* __restrict__ planes, int2* __restrict__ info, int K) {
+    const int kp = (K + 31) & ~31, tid = threadIdx.x;
+    const float* row = x + static_cast<size_t>(blockIdx.x) * K;
+    float v[C ? C : 1][8];
+    uint32_t top = 0;
+    if constexpr (C) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int k = (tid + c * 256) * 8;
+            load8(row, k, K, v[c]);
+            top = top_bits(v[c], top);
+        }
+    } else {
+        for (int k = tid * 8; k < kp; k += 2048) {
+            load8(row, k, K, v[0]);
+            top = top_bits(v[0], top);
+        }
+    }
+    row_to_pairs<C>(v, top, row, K, planes + static_cast<size_t>(blockIdx.x) * kp * 4, info + blockIdx.x);
+}
+
+// Rows of x that are the merged key runs of an attention (what merge_splits_kernel of attention.hip makes of them, in the same order), and
+// the same as pairs: a workgroup a token, C chunks of eight dims a thread.  part_o [T, H, runs, hd], part_ml [T, H, runs, 2] (maximum, sum).
+template <int C>
+__global__ __launch_bounds__(256) void merge_pair_rows_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml, float* __restrict__ x,
+                                                              char* __restrict__ planes, int2* __restrict__ info, int H, int hd, int runs) {
+    const int K = H * hd, kp = (K + 31) & ~31, t = blockIdx.x;
+    float* row = x + static_cast<size_t>(t) * K;
+    float v[C][8];
+    uint32_t top = 0;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int k = (threadIdx.x + c * 256) * 8;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[c][e] = 0.f;
+        if (k < K) {
+            const size_t p0 = (static_cast<size_t>(t) * H + k / hd) * runs;
+            const int dim = k % hd;
+            float M = -INFINITY, L = 0.f;
+            for (int s = 0; s < runs; ++s) M = fmaxf(M, part_ml[(p0 + s) * 2]);
+#pragma unroll 4
+            for (int s = 0; s < runs; ++s) {
+                const float f = expf(part_ml[(p0 + s) * 2] - M);
+                float u[8];
+                VecIO<float, 8>::load(part_o + (p0 + s) * hd + dim, u);
+                L += part_ml[(p0 + s) * 2 + 1] * f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[c][e] += u[e] * f;
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[c][e] /= L;
+            VecIO<float, 8>::store(row + k, v[c]);
+        }
+        top = top_bits(v[c], top);
+    }
+    row_to_pairs<C>(v, top, row, K, planes + static_cast<size_t>(t) * kp * 4, info + t);
 }
 
 // Rows of W: a workgroup 32 rows, in the order in which the product's wavefronts take them: [tile of 32 rows][16 columns]
@@ -460,6 +505,22 @@ NI_EXPORT int ni_pair_rows(const void* x, void* planes, void* info, int M, int K
     else if (K <= 4096) pair_rows_kernel<2><<<M, 256, 0, s>>>(xf, p, i, K);
     else if (K <= 8192) pair_rows_kernel<4><<<M, 256, 0, s>>>(xf, p, i, K);
     else pair_rows_kernel<0><<<M, 256, 0, s>>>(xf, p, i, K);
+    return NI_LAUNCH_RESULT();
+}
+
+// hd a multiple of eight, H * hd at most 8,192; x [T, H * hd] takes the merged rows themselves
+NI_EXPORT int ni_merge_pair_rows(const void* part_o, const void* part_ml, void* x, void* planes, void* info, int T, int H, int hd, int runs, void* stream) {
+    if (T <= 0 || H <= 0 || hd <= 0 || hd % 8 || static_cast<long>(H) * hd > 8192 || runs < 1 || (reinterpret_cast<uintptr_t>(part_o) | reinterpret_cast<uintptr_t>(x)) % 16)
+        return static_cast<int>(hipErrorInvalidValue);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const float *po = static_cast<const float*>(part_o), *ml = static_cast<const float*>(part_ml);
+    float* xf = static_cast<float*>(x);
+    char* p = static_cast<char*>(planes);
+    int2* i = static_cast<int2*>(info);
+    const int K = H * hd;
+    if (K <= 2048) merge_pair_rows_kernel<1><<<T, 256, 0, s>>>(po, ml, xf, p, i, H, hd, runs);
+    else if (K <= 4096) merge_pair_rows_kernel<2><<<T, 256, 0, s>>>(po, ml, xf, p, i, H, hd, runs);
+    else merge_pair_rows_kernel<4><<<T, 256, 0, s>>>(po, ml, xf, p, i, H, hd, runs);
     return NI_LAUNCH_RESULT();
 }
 

@@ -578,13 +578,14 @@ def mfma_splits(n_tiles: int, kv_heads: int, group: int, max_keys: int, hd: int 
 def mfma_attention(qkv: torch.Tensor, kpool: torch.Tensor, vpool: torch.Tensor, block_table: torch.Tensor,
                    tiles: torch.Tensor, out: torch.Tensor, H: int, KVH: int, hd: int, scale: float,
                    window: Optional[int], nsplit: int = 1, workspace: Optional[torch.Tensor] = None,
-                   tile_tokens: Optional[int] = None, groups: int = 1) -> torch.Tensor:
+                   tile_tokens: Optional[int] = None, groups: int = 1, halves: bool = False):
     """Attention of prompt portions on the matrix cores, in bfloat16 or in true float32 (a kernel
     each).  ``tiles`` is int32 [n, 4] from :func:`build_q_tiles` with ``tile_tokens`` tokens a tile (a
     size that :func:`mfma_tile_tokens` gives for the type; default: its smallest); the pools already
     hold the keys and values of every position of the step.  ``workspace`` (float32,
     ``T*H*nsplit*(hd+2)`` elements) is needed when ``nsplit > 1``.  ``groups`` (bfloat16, head sizes up to 128): 1 or 2
-    groups of four wavefronts that share out a tile's keys (:func:`mfma_group_plan`)."""
+    groups of four wavefronts that share out a tile's keys (:func:`mfma_group_plan`).  ``halves``: where float32 key runs are merged the
+    result comes back as pairs of halves too (:class:`HalvedRows`), for a product that reads those."""
     T = qkv.shape[0]
     dtype = qkv.dtype
     _gpu(qkv, "qkv")
@@ -636,6 +637,8 @@ def mfma_attention(qkv: torch.Tensor, kpool: torch.Tensor, vpool: torch.Tensor, 
             _ptr(qkv), qkv.shape[1], _ptr(kpool), _ptr(vpool), _ptr(block_table), block_table.shape[1], _ptr(tiles),
             tiles.shape[0], _ptr(out), _ptr(part_o), _ptr(part_ml), H, KVH, kpool.shape[2],
             int(window) if window else 0, ctypes.c_float(scale), nsplit, blocks, groups, _stream()), "mfma_attention")
+    if nsplit > 1 and halves and merge_pair_rows_ok(T, H, hd, part_o, out):
+        return merge_pair_rows(part_o, part_ml, out, H, hd, nsplit)
     if nsplit > 1:
         _check(attention_lib(hd).ni_merge_splits(_ptr(part_o), _ptr(part_ml), _ptr(out), T, H, nsplit,
                                                  dtype_code(out.dtype), _stream()), "merge_splits")
@@ -1446,7 +1449,7 @@ torch.backends.cuda.matmul.allow_tf32 = False
 torch.backends.cudnn.allow_tf32 = False
 
 # products of many rows on the matrix cores
-from .tile import (HalvedRows, add_rmsnorm_halved, experts_grouped, experts_grouped_wins, pair_gemm, pair_holds, pair_lines,  # noqa: E402,F401
+from .tile import (HalvedRows, add_rmsnorm_halved, merge_pair_rows, merge_pair_rows_ok, experts_grouped, experts_grouped_wins, pair_gemm, pair_holds, pair_lines,  # noqa: E402,F401
                    pair_plan, pair_rows, pair_weight, pair_weight_bytes, pair_wins, qkv_rope, qkv_rope_plan, rows_of, split_gemm, split_plan, split_wins, takes_halved, tile_lib, tiled_gemm,
                    tiled_plan, tiled_wins, wide_gemm, wide_plan, wide_wins)
 # sums onto the residual stream, routed experts, the gated delta rule, attention with a bias by distance

@@ -244,6 +244,26 @@ def add_rmsnorm_halved(h: torch.Tensor, pending: Optional[torch.Tensor], weight:
     return HalvedRows(out, planes, info)
 
 
+def merge_pair_rows_ok(T: int, H: int, hd: int, part_o: torch.Tensor, out: torch.Tensor) -> bool:
+    """Whether :func:`merge_pair_rows` takes rows of ``H`` heads of ``hd``: they wait in registers, eight numbers a thread and chunk."""
+    return (out.dtype == torch.float32 and T > 0 and hd % 8 == 0 and H * hd <= 8192 and T * (H * hd + 31) < 1 << 29
+            and (part_o.data_ptr() | out.data_ptr()) % 16 == 0)
+
+
+def merge_pair_rows(part_o: torch.Tensor, part_ml: torch.Tensor, out: torch.Tensor, H: int, hd: int, runs: int) -> HalvedRows:
+    """The key runs of an attention, ``part_o`` float32 [T, H, runs, hd] with (maximum, sum) in ``part_ml`` [T, H, runs, 2], merged into ``out``
+    [T, H * hd] and left as pairs of halves as well."""
+    T = out.shape[0]
+    _gpu(out, "out", torch.float32, (T, H * hd))
+    _gpu(part_o, "part_o", torch.float32)
+    _gpu(part_ml, "part_ml", torch.float32)
+    if part_o.numel() != T * H * runs * hd or part_ml.numel() != T * H * runs * 2 or not merge_pair_rows_ok(T, H, hd, part_o, out):
+        raise KernelError(f"{runs} runs of {H} heads of {hd} are not merged into pairs of halves")
+    planes, info = _pair_planes(T, H * hd, out.device)
+    _check(pair_lib().ni_merge_pair_rows(_ptr(part_o), _ptr(part_ml), _ptr(out), _ptr(planes), _ptr(info), T, H, hd, runs, _stream()), "merge_pair_rows")
+    return HalvedRows(out, planes, info)
+
+
 # Operations from which a float32 product goes to pair_gemm.  Measured in recorded launches, each with another W and all its kernels
 # counted (us, library : this): [2048, 2048] at 256 / 400 / 800 rows (2.1 / 3.4 / 6.7 GFLOP) 22.8 : 26.0, 38.9 : 32.0, 65.7 : 42.9;
 # [3072, 2048] at 130 / 164 / 200 (1.6 / 2.1 / 2.5) 22.6 : 26.6, 30.6 : 27.5, 31.3 : 29.5; [4096, 1024] at 256 / 400 (2.1 / 3.4) 24.1 : 26.6,
@@ -538,26 +558,6 @@ def wide_gemm(x: torch.Tensor, rows: torch.Tensor, out_dtype: Optional[torch.dty
     return out
 
 
-# ---------------------------------------------------------------- routed experts
-
-def _grouped_plan(places: int, N: int, K: int, groups: int) -> Tuple[float, int]:
-    return _grouped_tiles(_whole(places), N, K, groups)
-
-
-@functools.lru_cache(maxsize=1024)
-def _grouped_tiles(places: int, N: int, K: int, groups: int) -> Tuple[float, int]:
-    return min((_split_cost(places, N, K, t, 1, groups), t) for t in range(len(SPLIT_TILES)))
-
-
-def _grouped_pair_plan(places: int, N: int, K: int, groups: int) -> Tuple[float, int]:
-    return _grouped_pair_tiles(_whole(places), N, K, groups)
-
-
-@functools.lru_cache(maxsize=1024)
-def _grouped_pair_tiles(places: int, N: int, K: int, groups: int) -> Tuple[float, int]:
-    return min((_pair_cost(places, N, K, t, 1, groups), t) for t in range(len(PAIR_TILES)))
-
-
 # ---------------------------------------------------------------- bfloat16, [q; k; v] with rotation and the cache's pages behind it
 
 ROPE_PASS = 3.5, 2.2e-3      # microseconds of the kernel that rotates and stores: a launch, and a row (4.3 at 512 rows, 7.9 at 1,999, the 1B shape)
@@ -633,6 +633,26 @@ def qkv_rope(x: torch.Tensor, weight, positions: torch.Tensor, cos: torch.Tensor
     _check(launch(_ptr(x), _ptr(matrix), _ptr(q), _ptr(positions), _ptr(cos), _ptr(sin), _ptr(slot_mapping), _ptr(kpool), _ptr(vpool), M, K, H, KVH, hd,
                   page_size, tile, _stream()), "qkv_rope")
     return q
+
+
+# ---------------------------------------------------------------- routed experts
+
+def _grouped_plan(places: int, N: int, K: int, groups: int) -> Tuple[float, int]:
+    return _grouped_tiles(_whole(places), N, K, groups)
+
+
+@functools.lru_cache(maxsize=1024)
+def _grouped_tiles(places: int, N: int, K: int, groups: int) -> Tuple[float, int]:
+    return min((_split_cost(places, N, K, t, 1, groups), t) for t in range(len(SPLIT_TILES)))
+
+
+def _grouped_pair_plan(places: int, N: int, K: int, groups: int) -> Tuple[float, int]:
+    return _grouped_pair_tiles(_whole(places), N, K, groups)
+
+
+@functools.lru_cache(maxsize=1024)
+def _grouped_pair_tiles(places: int, N: int, K: int, groups: int) -> Tuple[float, int]:
+    return min((_pair_cost(places, N, K, t, 1, groups), t) for t in range(len(PAIR_TILES)))
 
 
 def _experts_in_pairs(places: int, w_up, w_down, d: int, per: int, ff: int) -> bool:

@@ -404,7 +404,8 @@ class Attention(Part):
     def attend(self, qkv: torch.Tensor, ctx, cache: LayerCache, leave_runs: bool = False):
         """Stage 3: every query of ``qkv`` over the keys and values of its sequence in the cache, up to its own
         position (inside the window, if there is one).  Returns ``out`` [T, H * hd]; or, with ``leave_runs``
-        where the key ranges were cut into runs that the output product can merge itself, ``(workspace, runs)``."""
+        where the key ranges were cut into runs that the output product can merge itself, ``(workspace, runs)``, or the rows as pairs of
+        halves too (:class:`nanoinfer_amd.kernels.HalvedRows`) where it reads those."""
         T = qkv.shape[0]
         dtype = qkv.dtype
         out = torch.empty(T, self.H * self.hd, dtype=dtype, device=qkv.device)
@@ -421,9 +422,9 @@ class Attention(Part):
             if nsplit is None:
                 nsplit = K.mfma_splits(tiles.shape[0], self.KVH, self.H // self.KVH, max_keys, self.hd, dtype, T == ctx.max_q_len)
             ws = ctx.workspace(T * self.H * nsplit * (self.hd + 2)) if nsplit > 1 else None
-            K.mfma_attention(qkv, cache.kpool, cache.vpool, cache.block_table, tiles, out, self.H, self.KVH, self.hd,
-                             self.scale, self.window, nsplit, ws, tile_tokens, groups)
-            return out
+            halves = leave_runs and K.takes_halved(T, self.H * self.hd, dtype, self.w_o)
+            return K.mfma_attention(qkv, cache.kpool, cache.vpool, cache.block_table, tiles, out, self.H, self.KVH, self.hd,
+                                    self.scale, self.window, nsplit, ws, tile_tokens, groups, halves)
         # single tokens and short portions, token by token
         max_keys = ctx.max_context if self.window is None else min(ctx.max_context, self.window)
         on_matrix_cores = K.mfma_token_ok(dtype, self.hd)

@@ -85,3 +85,37 @@ def test_parts_say_which_rows_they_read(K):
             return None
 
     assert not Projects.__new__(Projects).takes_halved(600)
+
+
+# widths of every size of the workgroup's chunks, and one that is no whole stage of 32 columns; one run and many; runs without a key (sum
+# and rows zero, a finite maximum) and rows that are no numbers
+@pytest.mark.parametrize("T,H,hd,runs", [(1, 1, 64, 1), (70, 32, 64, 4), (3, 24, 128, 3), (66, 5, 80, 2), (2, 3, 24, 7), (65, 32, 256, 5)])
+def test_merged_runs_and_their_halves_are_those_of_the_two_passes(K, T, H, hd, runs):
+    g = torch.Generator().manual_seed(T + hd)
+    part_o = torch.randn(T, H, runs, hd, generator=g) * 2.0 ** torch.randint(-10, 10, (T, 1, 1, 1), generator=g)
+    part_ml = torch.rand(T, H, runs, 2, generator=g) * 20 + 0.1
+    if runs > 1:
+        part_o[0, 0, 1], part_ml[0, 0, 1] = 0.0, torch.tensor([-1e30, 0.0])
+    if T > 2:
+        part_o[1] = 0.0
+        part_o[2, H - 1, runs - 1, hd - 1] = float("nan")
+    part_o, part_ml = part_o.cuda(), part_ml.cuda()
+    rows = torch.empty(T, H * hd, device="cuda")
+    if hd % 16 == 0:
+        K._check(K.attention_lib(hd).ni_merge_splits(K._ptr(part_o), K._ptr(part_ml), K._ptr(rows), T, H, runs, 0, K._stream()), "merge_splits")
+    got = K.merge_pair_rows(part_o.view(-1), part_ml.view(-1), torch.empty(T, H * hd, device="cuda"), H, hd, runs)
+    if hd % 16 == 0:
+        assert torch.equal(got.x.view(torch.int32), rows.view(torch.int32))
+    weight = torch.exp(part_ml[..., :1].double() - part_ml[..., :1].double().amax(2, keepdim=True))
+    below = (part_ml[..., 1:].double() * weight).sum(2)
+    want, size = (((v * weight).sum(2) / below).view(T, H * hd) for v in (part_o.double(), part_o.double().abs()))
+    sure = torch.isfinite(want)                            # (an exponential off by two places, a rounding or two a run)
+    assert bool(((got.x.double() - want).abs()[sure] <= (2 * runs + 8) * 2.0 ** -23 * size[sure]).all())
+    planes, info = K.pair_rows(got.x)
+    assert torch.equal(got.info, info)
+    finite = info[:, 1].cpu() >= 0
+    assert torch.equal(got.planes.view(torch.int32).view(T, -1)[finite], planes.view(torch.int32).view(T, -1)[finite])
+    for bad in (lambda: K.merge_pair_rows(part_o.view(-1)[:-8], part_ml.view(-1), got.x, H, hd, runs),
+                lambda: K.merge_pair_rows(part_o.view(-1), part_ml.view(-1), got.x[:, :-8].contiguous(), H, hd, runs)):
+        with pytest.raises(K.KernelError):
+            bad()
