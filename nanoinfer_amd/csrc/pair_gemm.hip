@@ -19,30 +19,40 @@
 // same workgroup instead of its main loop; infinities and NaN count as no big number at all and end there too.  Normal
 // deviates have one number in 2,900 that is not big, squared ReLU leaves half of them: neither gets there; a row of which one number
 // is 30,000 times the rest does.  What is known of the rows is asked for before anything else and looked at while the first stages are on
-// their way: a maximum over each wavefront in registers and four numbers in LDS (by atomics there it takes 3 us).  Measured, no such
-// row : one in the first tile : one in every tile : all by tile_gemm.hip (us): 512 rows on [16384, 2048] with SwiGLU 110 : 191 : 206 : 178
-// (looked at behind the main loop 107 : 249 : 290), on [2048, 8192] 69 : 111 : 121 : 103, on [2048, 2048] 25 : 37 : 37 : 38, 100 rows on
-// [16384, 2048] 59 : 110 : 110 : 93, 2,000 rows there 355 : 478 : 760 : 610.
+// their way: a maximum over each wavefront in registers and a number of each in LDS (by atomics there it takes 3 us).  Measured, no such
+// row : one in the first tile : one in every tile : all by tile_gemm.hip (us): 512 rows on [16384, 2048] with SwiGLU 84 : 164 : 181 : 173,
+// on [2048, 8192] 53 : 97 : 103 : 91, on [2048, 2048] 16 : 39 : 40 : 31, 100 rows on [16384, 2048] 53 : 115 : 113 : 98, 2,000 rows
+// there 343 : 591 : 715 : 628.
 //
 // Both operands come as halves: W once, when it is loaded, in the order of the lanes (pair_weight_kernel); x by a pass of its own
-// (pair_rows_kernel, 3.5 to 8 us for 100 to 2,000 rows of 2,048).  A workgroup is four wavefronts side by side, one on each matrix core
-// where the tile is largest, each with TN tiles of 32 rows of W and all 32 TM rows of x.  W goes from memory into registers three
-// steps (of 16 columns) ahead of its turn and never through LDS: no two wavefronts share a row of it.  x comes in stages of 32
-// columns through three slots of LDS; a stage's rows are loaded four stages ahead and written two ahead, and AHEAD the
-// operands of a step are read during the step before (not where two workgroups share a unit and the registers do).
+// (pair_rows_kernel, 3.5 to 8 us for 100 to 2,000 rows of 2,048) or by what makes x.  Both go from memory straight into LDS, without a
+// register, in stages of 32 columns: 128 bytes of a row of x, whole lines (pieces of 64 bytes come at half the rate), their
+// 16-byte pieces in another order for every second row, so that the reads meet no bank twice; W in the order that it is stored in,
+// which the reads take as it is.  A ring holds three or four stages; of the one being multiplied the slots are asked for anew
+// as soon as it is in registers, one barrier a stage.  A stage is three rounds of TM x TN products, low by high, high by
+// low, high by high: what a round needs is read during the round before, so that no product waits for LDS.  Where the registers are
+// there, high by high has two sums that take the stages in turn: shorter sums have fewer roundings, so that a plan of half as many
+// shares is no less exact (512 rows on [2048, 2048] in four shares 1.708e-7, in two with two sums 1.706e-7).  Eight wavefronts, two on a matrix core, where the tile has the work for them:
+// with four of them and 512 registers each the compiler keeps sums in accumulation registers and copies them (64 x 256: 110 us of
+// 105).  The products are of 16 x 16, which draw less power than 32 x 32: the clock is 5 % higher.  Groups of PAIR_GROUP tiles of x share
+// the tiles of W that they read from an L2; every group begins with another stage, so that what one die asks of memory first the next
+// finds in the cache on the memory's side.
 //
-// Measured, recorded, every launch with another W, without the pass over x (us; six bfloat16 products : this): 512 rows on
-// [16384, 2048] with SwiGLU 178 : 110, on [2048, 8192] 103 : 69, on [3072, 2048] 48 : 34, on [2048, 2048] 38 : 25; 2,000 rows on
-// [16384, 2048] 610 : 355 (378 TFLOP/s); 100 rows on [16384, 2048] 93 : 59; 200 rows on [3072, 2048] 32 : 21.  What bounds it is the clock
-// that the matrix cores hold: 256 workgroups of the largest tile take 0.68 us a step, eight 0.45 (of which the instructions are
-// 0.32), and with operands of ones, which switch less, 256 take 0.56.  By counters, 2,048 rows on [16384, 2048]: 1.81 GHz, matrix cores busy
-// 61 % of the cycles; 512 workgroups of the smallest tile: 2.30 GHz and 35 %.
+// Measured, recorded, every launch with another W, without the pass over x (us; six bfloat16 products : W in registers a stage of 16
+// columns ahead, 32 x 32 products, four wavefronts : this): 512 rows on [16384, 2048] with SwiGLU 173 : 98 : 85, on [2048, 8192]
+// 91 : 60 : 50, on [3072, 2048] 42 : 29 : 25, on [2048, 2048] 31 : 19 : 16; 1,500 rows on [2048, 8192] 150 : 125 (the second and this); 2,000 rows
+// on [16384, 2048] 628 : 360 : 307 (437 TFLOP/s); 100 rows on [16384, 2048] 98 : 60 : 53; 200 rows on [3072, 2048] 28 : 20 : 17.  What
+// bounds it is the clock that the matrix cores hold: by counters, 2,048 rows on [16384, 2048], they are busy 71 % of the cycles at
+// 1.76 GHz (W in registers: 61 % at 1.81), 192 workgroups of the largest tile 47 % at 2.2 GHz; no bank conflicts.
+#include "lds_load.h"
 #include "pair_rows.h"
 #include "split_tile.h"
 
-template <int N> struct Which { static constexpr int value = N; };
 
 #define PAIR_TERMS 64           // products of big numbers that a result has at least
+#define PAIR_GROUP 4            // tiles of x side by side
+
+template <int ROWS> struct Slot { char b[ROWS * 128]; };
 
 // eight numbers of a row from k on, zeros behind its end; K is a multiple of four
 __device__ __forceinline__ void load8(const float* __restrict__ row, int k, int K, float* v) {
@@ -231,23 +241,27 @@ struct PairGroups {
     int steps;      // 16 columns from one group's to the next
 };
 
-template <int TM, int TN, int SWM, int MINB, bool AHEAD, int EPI, bool GROUPED>
-__global__ __launch_bounds__(256, MINB) void pair_gemm_kernel(const char* __restrict__ xp, const int2* __restrict__ xinfo, const char* __restrict__ wp,
-                                                              const int2* __restrict__ winfo, const float* __restrict__ x,
-                                                              const float* __restrict__ w, float* __restrict__ out, int M, int N, int K,
-                                                              int kper, int wsteps, int mtiles, int ntiles, GatedUnit act, Groups groups,
-                                                              PairGroups apart) {
-    constexpr int BM = 32 * TM, BN = 128 * TN, R = 4;      // R: sixteens of columns of W in registers
-    constexpr int ROWB = 128 + 16, SLAB = BM * ROWB, CX = BM * 8 / 256;
-    constexpr int LDS = SplitLds<BM, BN>::BYTES > 3 * SLAB ? SplitLds<BM, BN>::BYTES : 3 * SLAB;
-    __shared__ __attribute__((aligned(16))) char lds[LDS];
-    __shared__ __attribute__((aligned(16))) int few_of[4], many_of[4];       // of every wavefront
+template <int BM, int BN, int WM, int WN, int D, int EPI, bool GROUPED>
+__global__ __launch_bounds__(WM * WN * WAVE, 2) void pair_gemm_kernel(const char* __restrict__ xp, const int2* __restrict__ xinfo, const char* __restrict__ wp,
+                                                                     const int2* __restrict__ winfo, const float* __restrict__ x,
+                                                                     const float* __restrict__ w, float* __restrict__ out, int M, int N, int K,
+                                                                     int kper, int wsteps, int mtiles, int ntiles, GatedUnit act, Groups groups,
+                                                                     PairGroups apart) {
+    constexpr int NW = WM * WN, THREADS = NW * WAVE, TM = BM / WM / 16, TN = BN / WN / 16;
+    constexpr int CX = BM / 8 / NW, CW = BN / 8 / NW, ALL = CX + CW;            // loads a wavefront and stage
+    constexpr int SUMS = BM * BN <= 16384 ? 2 : 1;                                   // of high by high, stages in turn
+    static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0 && BN <= THREADS && (EPI != TG_GATED || TN == 4) && TN % 2 == 0, "whole loads a wavefront");
+    __shared__ __attribute__((aligned(1024))) Slot<BM> x0, x1, x2, x3;
+    __shared__ __attribute__((aligned(1024))) Slot<BN> w0, w1, w2, w3;
+    __shared__ __attribute__((aligned(16))) int few_of[NW], many_of[NW];     // of every wavefront
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int wm = wave / WN, wn = wave % WN;
     const int t = tile_of_block(blockIdx.x, mtiles * ntiles);
-    int m0 = (t % mtiles) * BM, ldw = K, rows = M, wtile = 0, wrow = 0, wstep = 0;
-    const int nt = t / mtiles;
+    const int g = t / (PAIR_GROUP * ntiles), gm = min(PAIR_GROUP, mtiles - g * PAIR_GROUP), rem = t - g * PAIR_GROUP * ntiles;
+    const int mt = g * PAIR_GROUP + rem % gm, nt = rem / gm;
+    int m0 = mt * BM, ldw = K, rows = M, wtile = 0, wrow = 0, wstep = 0;
     if constexpr (GROUPED) {
-        int tile = t % mtiles, e = 0, begin = 0, end = 0;
+        int tile = mt, e = 0, begin = 0, end = 0;
         for (; e < groups.count; ++e) {
             begin = groups.offsets[e];
             end = groups.offsets[e + 1];
@@ -266,7 +280,8 @@ __global__ __launch_bounds__(256, MINB) void pair_gemm_kernel(const char* __rest
     }
     const int share = blockIdx.y;
     const int kbeg = share * kper, kend = min(K, kbeg + kper), half = N / 2;
-    const int sbeg = kbeg / 32, send = (kend + 31) / 32, rowb = ((K + 31) & ~31) * 4;
+    const int first = kbeg / 32, steps = (kend + 31) / 32 - first, rowb = ((K + 31) & ~31) * 4;
+    const int turn = g * (steps / ((mtiles + PAIR_GROUP - 1) / PAIR_GROUP));         // the stage that this group begins with
 
     auto row_at = [&](int m) {
         m = min(m, M - 1);
@@ -274,182 +289,191 @@ __global__ __launch_bounds__(256, MINB) void pair_gemm_kernel(const char* __rest
             if (groups.rows) m = groups.rows[m];
         return m;
     };
+    // tile of 32 rows of W at place q of the workgroup's: with SwiGLU a wavefront's two are gate rows and the up rows of the same outputs
+    auto tile_at = [&](int q) {
+        if constexpr (EPI == TG_GATED) return (q & 1) * (half / 32) + min(nt * (BN / 64) + q / 2, half / 32 - 1);
+        else return min(nt * (BN / 32) + q, (N + 31) / 32 - 1);
+    };
     // what the rows and columns of this tile were scaled by, and how many big numbers they have: waits in registers
-    int2 mine_x = make_int2(0, INT_MAX), mine_w[(BN + 255) / 256];
+    int2 mine_x = make_int2(0, INT_MAX), mine_w = make_int2(0, 0);
     if (tid < BM) mine_x = xinfo[row_at(m0 + tid)];
-#pragma unroll
-    for (int c = 0; c < (BN + 255) / 256; ++c) {
-        const int r = tid + c * 256;
-        mine_w[c] = make_int2(0, 0);
-        if (r < BN) {
-            int n;
-            if constexpr (EPI == TG_GATED) n = ((r >> 5) & 1) * half + min(nt * (BN / 2) + (r / 64) * 32 + (r & 31), half - 1);
-            else n = min(nt * BN + r, N - 1);
-            mine_w[c] = winfo[wrow + n];
-        }
-    }
-    // x: 16 bytes a thread and chunk, eight neighbouring threads a row's 32 columns
+    if (tid < BN) mine_w = winfo[wrow + min(tile_at(tid / 32) * 32 + (tid & 31), N - 1)];
     const auto xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(xp), 0, INT_MAX, 0x00020000);
-    int xsrc[CX], xdst[CX];
+    const auto wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(wp), 0, INT_MAX, 0x00020000);
+    int xsrc[CX], wsrc[CW];
 #pragma unroll
     for (int c = 0; c < CX; ++c) {
-        const int i = tid + c * 256, r = i >> 3;
-        xsrc[c] = row_at(m0 + r) * rowb + (i & 7) * 16;
-        xdst[c] = r * ROWB + (i & 7) * 16;
+        const int r = (wave + c * NW) * 8 + (lane >> 3);
+        xsrc[c] = row_at(m0 + r) * rowb + ((lane & 7) ^ (r >> 1 & 7)) * 16;
     }
-    // W: two planes of a lane's eight numbers for every tile of 32 rows and 16 columns
-    int wsrc[TN];
-    const auto wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(wp), 0, INT_MAX, 0x00020000);
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-        int tile;
-        if constexpr (EPI == TG_GATED) tile = (j & 1) * (half / 32) + min((nt * 4 + wave) * (TN / 2) + j / 2, half / 32 - 1);
-        else tile = min((nt * 4 + wave) * TN + j, (N + 31) / 32 - 1);
-        wsrc[j] = ((wtile + tile) * wsteps + wstep) * 2048;
+    for (int c = 0; c < CW; ++c) {
+        const int q = wave + c * NW;                          // a quarter of a tile's 32 columns
+        wsrc[c] = ((wtile + tile_at(q / 4)) * wsteps + wstep) * 2048 + q % 4 * 1024 + lane * 16;
     }
-    struct Rows { u32x4_t v[CX]; };
-    struct Cols { u32x4_t v[TN][2]; };
-    struct Frags { f16x8_t v[2][TM]; };
-    Rows xs[2];
-    Cols wreg[R];
-    Frags xf[AHEAD ? 2 : 1];
-    floatx16_t acc[TM][TN], low[TM][TN];
+    floatx4_t acc[SUMS][TM][TN], low[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = low[i][j][e] = 0.f;
-
-    auto fetch = [&](Rows& r, int s) {
-        const int at = min(s, send - 1) * 128;
-#pragma unroll
-        for (int c = 0; c < CX; ++c) r.v[c] = __builtin_amdgcn_raw_buffer_load_b128(xr, xsrc[c], at, 0);
+        for (int j = 0; j < TN; ++j) acc[0][i][j] = acc[SUMS - 1][i][j] = low[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    auto xslot = [&](auto I) -> Slot<BM>& {
+        constexpr int i = decltype(I)::value % D;
+        if constexpr (i == 0) return x0;
+        else if constexpr (i == 1) return x1;
+        else if constexpr (i == 2) return x2;
+        else return x3;
     };
-    auto put = [&](const Rows& r, int slot) {
-#pragma unroll
-        for (int c = 0; c < CX; ++c) *reinterpret_cast<u32x4_t*>(lds + slot + xdst[c]) = r.v[c];
+    auto wslot = [&](auto I) -> Slot<BN>& {
+        constexpr int i = decltype(I)::value % D;
+        if constexpr (i == 0) return w0;
+        else if constexpr (i == 1) return w1;
+        else if constexpr (i == 2) return w2;
+        else return w3;
     };
-    auto weights = [&](Cols& r, int step) {               // sixteen columns: step counts from K's beginning
-        const int at = min(step, 2 * send - 1) * 2048;
+    // loads FROM to TO of stage s, into slots I
+    auto fetch = [&](auto I, int s, auto FROM, auto TO) {
+        Slot<BM>& xs = xslot(I);
+        Slot<BN>& ws = wslot(I);
+        int at = min(s, steps - 1) + turn;
+        at = first + at - (at >= steps ? steps : 0);
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int p = 0; p < 2; ++p) r.v[j][p] = __builtin_amdgcn_raw_buffer_load_b128(wr, lane * 16 + p * 1024, wsrc[j] + at, 0);
-    };
-    const int xoff = (lane & 31) * ROWB + (lane >> 5) * 16;
-    auto read = [&](Frags& f, int slot, int which) {
-#pragma unroll
-        for (int p = 0; p < 2; ++p)
-#pragma unroll
-            for (int i = 0; i < TM; ++i) f.v[p][i] = *reinterpret_cast<const f16x8_t*>(lds + slot + xoff + i * 32 * ROWB + which * 64 + p * 32);
-    };
-    auto multiply = [&](const Frags& a, const Cols& b) {
-#pragma unroll
-        for (int p = 0; p < 3; ++p) {                     // high by low, low by high, high by high
-            constexpr int PA[3] = {0, 1, 0}, PB[3] = {1, 0, 0};
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    floatx16_t& to = p < 2 ? low[i][j] : acc[i][j];
-                    to = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.v[PA[p]][i], __builtin_bit_cast(f16x8_t, b.v[j][PB[p]]), to, 0, 0, 0);
-                }
+        for (int c = decltype(FROM)::value; c < decltype(TO)::value; ++c) {
+            if (c < CX) load_to_lds(xr, xs.b + (wave + c * NW) * 1024, xsrc[c < CX ? c : 0], at * 128);
+            else load_to_lds(wr, ws.b + (wave + (c - CX) * NW) * 1024, wsrc[c < CX ? 0 : c - CX], at * 4096);
         }
     };
-    int at0 = 0, at1 = SLAB, at2 = 2 * SLAB;              // the slots of this stage, the next and the one behind it
-    // 32 columns: their rows of x are in LDS, and the next 32; the ones behind are written, those behind them loaded
-    auto stage = [&](auto B, int s) {
-        constexpr int b = decltype(B)::value;
-        put(xs[b], at2);
-        fetch(xs[b], s + 4);
-        weights(wreg[(2 * b + 3) % R], 2 * s + 3);
-        if constexpr (AHEAD) read(xf[1], at0, 1);
-        else read(xf[0], at0, 0);
-        multiply(xf[0], wreg[2 * b]);
-        weights(wreg[2 * b], 2 * s + 4);
-        if constexpr (AHEAD) read(xf[0], at1, 0);
-        else read(xf[0], at0, 1);
-        multiply(xf[AHEAD ? 1 : 0], wreg[2 * b + 1]);
+    f16x8_t xh[TM], xl[TM], wl[TN], wh[2][TN];
+    const int r = lane & 15, kg = lane >> 4;
+    const int xo = ((wm * TM * 16 + r) * 128) + (((kg & 1) + (kg >> 1) * 4) ^ (r >> 1)) * 16;        // low halves two pieces on
+    const int wo = wn * TN * 2048 + (kg >> 1) * 2048 + (kg & 1) * 512 + r * 16;                      // 1 KB on
+    auto read_x = [&](f16x8_t (&f)[TM], auto I, int low_half) {
+        const Slot<BM>& xs = xslot(I);
 #pragma unroll
-        for (int g = 0; g < 6 * TM * TN; ++g) {
+        for (int i = 0; i < TM; ++i) f[i] = *reinterpret_cast<const f16x8_t*>(xs.b + (low_half ? xo ^ 32 : xo) + i * 2048);
+    };
+    auto read_w = [&](f16x8_t (&f)[TN], auto I, int low_half) {
+        const Slot<BN>& ws = wslot(I);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) f[j] = *reinterpret_cast<const f16x8_t*>(ws.b + wo + low_half * 1024 + j / 2 * 4096 + j % 2 * 256);
+    };
+    auto multiply = [&](floatx4_t (&to)[TM][TN], const f16x8_t (&fx)[TM], const f16x8_t (&fw)[TN]) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) to[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fw[j], fx[i], to[i][j], 0, 0, 0);
+    };
+    // between the products: READS reads of operands, one behind each, and LOADS loads
+    auto paced = [&](auto READS, auto LOADS) {
+        constexpr int R = decltype(READS)::value, L = decltype(LOADS)::value, MF = TM * TN;
+#pragma unroll
+        for (int q = 0; q < MF; ++q) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+            if (q < R) __builtin_amdgcn_sched_group_barrier(0x100, R > MF && q == 0 ? R - MF + 1 : 1, 0);
+            if (q * L / MF != (q + 1) * L / MF) __builtin_amdgcn_sched_group_barrier(0x020, L > MF ? 2 : 1, 0);
         }
-        __syncthreads();
-        const int first = at0;
-        at0 = at1;
-        at1 = at2;
-        at2 = first;
+        __builtin_amdgcn_sched_barrier(0);
     };
-    // (in the order of the loop, so that what waits for the rows of x there does not wait for W)
-    Rows first, second;
-    fetch(first, sbeg);
-    fetch(second, sbeg + 1);
-    fetch(xs[0], sbeg + 2);
-    fetch(xs[1], sbeg + 3);
-#pragma unroll
-    for (int r = 0; r < R - 1; ++r) weights(wreg[r], 2 * sbeg + r);
+    constexpr int L1 = (ALL + 2) / 3, L2 = L1 + (ALL + 1) / 3;
+    // A stage: low by high, high by low, high by high.  What the first needs is in registers; during it the rest of the stage is read, then the
+    // stage's slots are asked for anew and the first operands of the next stage read.
+    auto stage = [&](auto I, int s) {
+        constexpr int i = decltype(I)::value;
+        read_x(xh, I, 0);
+        read_w(wl, I, 1);
+        fetch(Index<i + D - 1>{}, s + D - 1, Index<L2>{}, Index<ALL>{});
+        multiply(low, xl, wh[i & 1]);
+        paced(Index<TM + TN>{}, Index<ALL - L2>{});
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((D - 2) * ALL) : "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        read_x(xl, Index<i + 1>{}, 1);
+        fetch(I, s + D, Index<0>{}, Index<L1>{});
+        multiply(low, xh, wl);
+        paced(Index<TM>{}, Index<L1>{});
+        read_w(wh[(i + 1) & 1], Index<i + 1>{}, 0);
+        fetch(I, s + D, Index<L1>{}, Index<L2>{});
+        multiply(acc[i % SUMS], xh, wh[i & 1]);
+        paced(Index<TN>{}, Index<L2 - L1>{});
+    };
+    fetch(Index<0>{}, 0, Index<0>{}, Index<ALL>{});
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(Index<1>{}, 1, Index<0>{}, Index<ALL>{});
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (D > 3) fetch(Index<2>{}, 2, Index<0>{}, Index<ALL>{});
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(Index<D - 1>{}, D - 1, Index<0>{}, Index<L2>{});
+    __builtin_amdgcn_sched_barrier(0);
     // is there a result that these products may not be exact enough for
-    int few = mine_x.y, many = mine_w[0].y;
-#pragma unroll
-    for (int c = 1; c < (BN + 255) / 256; ++c) many = max(many, mine_w[c].y);
-    few = -wave_max(-few);
-    many = wave_max(many);
+    const int few_here = -wave_max(-mine_x.y), many_here = wave_max(mine_w.y);
     if (lane == 0) {
-        few_of[wave] = few;
-        many_of[wave] = many;
+        few_of[wave] = few_here;
+        many_of[wave] = many_here;
     }
-    put(first, at0);
-    put(second, at1);
-    __syncthreads();
-    const int4 f = *reinterpret_cast<const int4*>(few_of), m = *reinterpret_cast<const int4*>(many_of);
-    few = __builtin_amdgcn_readfirstlane(min(min(f.x, f.y), min(f.z, f.w)));
-    many = __builtin_amdgcn_readfirstlane(max(max(m.x, m.y), max(m.z, m.w)));
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((D - 2) * ALL + L2) : "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    int few = few_of[0], many = many_of[0];
+#pragma unroll
+    for (int v = 1; v < NW; ++v) {
+        few = min(few, few_of[v]);
+        many = max(many, many_of[v]);
+    }
+    few = __builtin_amdgcn_readfirstlane(few);
+    many = __builtin_amdgcn_readfirstlane(many);
     if (few - PAIR_TERMS < many) {
-        split_tile<BM, BN, SWM, 4 / SWM, true, EPI, GROUPED>(x, w, out, M, N, K, m0, nt, share, kbeg, kend, ldw, groups.rows, act, lds);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();                                      // nothing is on its way into the slots, which hold the slabs now
+        constexpr int SNW = BM * 4 / WAVE < NW ? BM * 4 / WAVE : NW, SWN = BN / 64 < SNW ? BN / 64 : SNW, SWM = SNW / SWN;
+        if (wave >= SNW) return;                              // (64 rows are work for four wavefronts; barriers wait for those that are left)
+        split_tile<BM, BN, SWM, SWN, true, EPI, GROUPED>(x, w, out, M, N, K, m0, nt, share, kbeg, kend, ldw, groups.rows, act,
+                                                         SplitSlabs{{x0.b, x1.b}, {w0.b, w1.b}});
         return;
     }
-    if constexpr (AHEAD) read(xf[0], at0, 0);
-    int s = sbeg;
-    for (; s + 2 <= send; s += 2) {
-        stage(Which<0>{}, s);
-        stage(Which<1>{}, s + 1);
+    read_x(xl, Index<0>{}, 1);
+    read_w(wh[0], Index<0>{}, 0);
+    constexpr int PERIOD = D % 2 ? 2 * D : D;
+    int s = 0;
+    for (; s + PERIOD <= steps; s += PERIOD) {
+#define PAIR_STAGE(i) if constexpr (i < PERIOD) stage(Index<i>{}, s + i);
+        PAIR_STAGE(0) PAIR_STAGE(1) PAIR_STAGE(2) PAIR_STAGE(3) PAIR_STAGE(4) PAIR_STAGE(5)
+#undef PAIR_STAGE
     }
-    if (s < send) stage(Which<0>{}, s);
-
-    int* wexp = reinterpret_cast<int*>(lds);
-    int* xexp = wexp + BN;
-#pragma unroll
-    for (int c = 0; c < (BN + 255) / 256; ++c)
-        if (tid + c * 256 < BN) wexp[tid + c * 256] = mine_w[c].x;
+#define PAIR_STAGE(i) if constexpr (i + 1 < PERIOD) if (s + i < steps) stage(Index<i>{}, s + i);
+    PAIR_STAGE(0) PAIR_STAGE(1) PAIR_STAGE(2) PAIR_STAGE(3) PAIR_STAGE(4)
+#undef PAIR_STAGE
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    int *xexp = reinterpret_cast<int*>(x0.b), *wexp = reinterpret_cast<int*>(w0.b);
     if (tid < BM) xexp[tid] = mine_x.x;
+    if (tid < BN) wexp[tid] = mine_w.x;
     __syncthreads();
     const int cols = EPI == TG_GATED ? half : N;
     float* base = out + static_cast<size_t>(share) * rows * cols;
+    const bool vectors = cols % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
+    constexpr int OT = EPI == TG_GATED ? 2 : TN;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
+        const int mr = (wm * TM + i) * 16 + r, m = m0 + mr;
+        if (m >= M) continue;
+        const int sx = xexp[mr];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int r = 32 * i + 8 * (e / 4) + 4 * (lane >> 5) + (e & 3), m = m0 + r;
-            if (m >= M) continue;
-            const int sx = xexp[r];
-            auto value = [&](int j) { return ldexpf(fmaf(low[i][j][e], 1.f / 4096.f, acc[i][j][e]), -(sx + wexp[(wave * TN + j) * 32 + (lane & 31)])); };
-            if constexpr (EPI == TG_GATED) {
+        for (int j = 0; j < OT; ++j) {
+            const int n = EPI == TG_GATED ? (nt * (BN / 64) + wn) * 32 + j * 16 + kg * 4 : nt * BN + (wn * TN + j) * 16 + kg * 4;
+            if (n >= cols) continue;
+            auto value = [&](int block, int e) {
+                const float high = SUMS == 1 ? acc[0][i][block][e] : acc[0][i][block][e] + acc[SUMS - 1][i][block][e];
+                return ldexpf(fmaf(low[i][block][e], 1.f / 4096.f, high), -(sx + wexp[(wn * TN + block) * 16 + kg * 4 + e]));
+            };
+            float v[4];
 #pragma unroll
-                for (int j = 0; j < TN; j += 2) {
-                    const int n = ((nt * 4 + wave) * (TN / 2) + j / 2) * 32 + (lane & 31);
-                    if (n < cols) base[static_cast<size_t>(m) * cols + n] = act.value(value(j), value(j + 1));
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    const int n = ((nt * 4 + wave) * TN + j) * 32 + (lane & 31);
-                    if (n < cols) base[static_cast<size_t>(m) * cols + n] = act.plain(value(j));
-                }
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (EPI == TG_GATED) v[e] = act.value(value(j, e), value(j + 2, e));
+                else v[e] = act.plain(value(j, e));
             }
+            float* to = base + static_cast<size_t>(m) * cols + n;
+            if (vectors) VecIO<float, 4>::store(to, v);
+            else
+                for (int e = 0; e < 4 && n + e < cols; ++e) to[e] = v[e];
         }
     }
 }
@@ -469,16 +493,15 @@ struct PairArgs {
     hipStream_t stream;
 };
 
-template <int TM, int TN, int SWM, int MINB, bool AHEAD> static int launch_pair(const PairArgs& a) {
-    constexpr int BM = 32 * TM, BN = 128 * TN;
+template <int BM, int BN, int WM, int WN, int D> static int launch_pair(const PairArgs& a) {
     const int cols = a.gated ? a.N / 2 : a.N, per = a.gated ? BN / 2 : BN;
     const int mt = a.grouped ? a.M / BM + a.groups.count : (a.M + BM - 1) / BM, nt = (cols + per - 1) / per;
     const dim3 grid(mt * nt, a.shares);
-#define PAIR_LAUNCH(EPI, GROUPED) pair_gemm_kernel<TM, TN, SWM, MINB, AHEAD, EPI, GROUPED><<<grid, 256, 0, a.stream>>>(a.xp, a.xinfo, a.wp, a.winfo, a.x, a.w, \
+#define PAIR_LAUNCH(EPI, GROUPED) pair_gemm_kernel<BM, BN, WM, WN, D, EPI, GROUPED><<<grid, WM * WN * WAVE, 0, a.stream>>>(a.xp, a.xinfo, a.wp, a.winfo, a.x, a.w, \
         a.out, a.M, a.N, a.K, a.kper, a.wsteps, mt, nt, a.act, a.groups, a.apart)
     if (a.grouped) PAIR_LAUNCH(TG_STORE, true);
     else if (a.gated) {
-        if constexpr (TN % 2 == 0) PAIR_LAUNCH(TG_GATED, false);
+        if constexpr (BN == 256) PAIR_LAUNCH(TG_GATED, false);
         else return static_cast<int>(hipErrorInvalidValue);
     } else PAIR_LAUNCH(TG_STORE, false);
 #undef PAIR_LAUNCH
@@ -487,10 +510,10 @@ template <int TM, int TN, int SWM, int MINB, bool AHEAD> static int launch_pair(
 
 static int launch_pair_tile(int tile, const PairArgs& a) {
     switch (tile) {
-        case 0: return launch_pair<4, 2, 2, 1, true>(a);
-        case 1: return launch_pair<2, 2, 1, 2, false>(a);
-        case 2: return launch_pair<4, 1, 2, 2, false>(a);
-        case 3: return launch_pair<2, 1, 2, 3, true>(a);
+        case 0: return launch_pair<128, 256, 2, 4, 3>(a);
+        case 1: return launch_pair<64, 256, 2, 4, 3>(a);
+        case 2: return launch_pair<128, 128, 4, 2, 4>(a);
+        case 3: return launch_pair<64, 128, 2, 2, 3>(a);
         default: return static_cast<int>(hipErrorInvalidValue);
     }
 }

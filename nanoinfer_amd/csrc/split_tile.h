@@ -69,18 +69,26 @@ struct Groups {
     int ldw;                     // numbers from one row of W to the next
 };
 
-template <int BM, int BN> struct SplitLds { static constexpr int BYTES = 2 * (BM + BN) * (3 * 16 * 2 + 16); };
+// Two slabs in LDS: a row takes SPLIT_ROWB bytes, the rows of x and of W of a slab stand apart.
+#define SPLIT_ROWB (3 * 16 * 2 + 16)
+template <int BM, int BN> struct SplitLds { static constexpr int BYTES = 2 * (BM + BN) * SPLIT_ROWB; };
+struct SplitSlabs {
+    char *x[2], *w[2];
+    template <int BM, int BN> static __device__ __forceinline__ SplitSlabs in(char* lds) {      // SplitLds<BM, BN>::BYTES
+        constexpr int SLAB = (BM + BN) * SPLIT_ROWB;
+        return SplitSlabs{{lds, lds + SLAB}, {lds + BM * SPLIT_ROWB, lds + SLAB + BM * SPLIT_ROWB}};
+    }
+};
 
 // The tile whose first row (place) is m0 and whose columns are the nt-th BN, over the K range kbeg to kend of share `share`.
-// M: one behind the last row of the tile's group; K: numbers from one row of x to the next.  lds: SplitLds<BM, BN>::BYTES.
+// M: one behind the last row of the tile's group; K: numbers from one row of x to the next.
 template <int BM, int BN, int WM, int WN, bool AHEAD, int EPI, bool GROUPED>
 __device__ __forceinline__ void split_tile(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ out, int M, int N,
                                            int K, int m0, int nt, int share, int kbeg, int kend, int ldw, const int32_t* __restrict__ rows,
-                                           const GatedUnit& act, char* lds) {
+                                           const GatedUnit& act, const SplitSlabs& slabs) {
     constexpr int THREADS = WM * WN * WAVE;
     constexpr int BK = 16;
-    constexpr int ROWB = 3 * BK * 2 + 16;               // bytes of a row of a slab
-    constexpr int SLAB = (BM + BN) * ROWB;
+    constexpr int ROWB = SPLIT_ROWB;
     constexpr int TMB = BM / WM / 32, TNB = BN / WN / 32;
     constexpr int CPR = BK / 4;                         // chunks of four numbers a row
     constexpr int CA = BM * CPR / THREADS, CB = BN * CPR / THREADS, CH = CA + CB;
@@ -110,7 +118,7 @@ __device__ __forceinline__ void split_tile(const float* __restrict__ x, const fl
                 n = min(nt * BN + r, N - 1);
             }
             src[c] = w + static_cast<size_t>(n) * ldw;
-            dst[c] = (BM + r) * ROWB + kc * 2;
+            dst[c] = r * ROWB + kc * 2;
         }
     }
     struct Raw { float4 v[CH]; };
@@ -124,21 +132,21 @@ __device__ __forceinline__ void split_tile(const float* __restrict__ x, const fl
         uint2 h, m, l;
         split3(s.v[c], h, m, l);
         if (k0 + kc >= kend) h = m = l = make_uint2(0, 0);
-        char* p = lds + buf + dst[c];
+        char* p = (c < CA ? slabs.x[buf] : slabs.w[buf]) + dst[c];
         *reinterpret_cast<uint2*>(p) = h;
         *reinterpret_cast<uint2*>(p + BK * 2) = m;
         *reinterpret_cast<uint2*>(p + BK * 4) = l;
     };
     const int wm = wave / WN, wn = wave % WN;
     const int aoff = (wm * (BM / WM) + (lane & 31)) * ROWB + (lane >> 5) * 16;
-    const int boff = (BM + wn * (BN / WN) + (lane & 31)) * ROWB + (lane >> 5) * 16;
+    const int boff = (wn * (BN / WN) + (lane & 31)) * ROWB + (lane >> 5) * 16;
     auto read = [&](Frags& f, int buf) {
 #pragma unroll
         for (int p = 2; p >= 0; --p) {
 #pragma unroll
-            for (int i = 0; i < TMB; ++i) f.a[p][i] = *reinterpret_cast<const bf16x8_t*>(lds + buf + aoff + 32 * i * ROWB + p * BK * 2);
+            for (int i = 0; i < TMB; ++i) f.a[p][i] = *reinterpret_cast<const bf16x8_t*>(slabs.x[buf] + aoff + 32 * i * ROWB + p * BK * 2);
 #pragma unroll
-            for (int j = 0; j < TNB; ++j) f.b[p][j] = *reinterpret_cast<const bf16x8_t*>(lds + buf + boff + 32 * j * ROWB + p * BK * 2);
+            for (int j = 0; j < TNB; ++j) f.b[p][j] = *reinterpret_cast<const bf16x8_t*>(slabs.w[buf] + boff + 32 * j * ROWB + p * BK * 2);
         }
     };
     floatx16_t acc[TMB][TNB];
@@ -183,7 +191,7 @@ __device__ __forceinline__ void split_tile(const float* __restrict__ x, const fl
     for (int c = 0; c < CH; ++c) put(r0, c, 0, kbeg);
     if constexpr (AHEAD) {
 #pragma unroll
-        for (int c = 0; c < CH; ++c) put(r1, c, SLAB, kbeg + BK);
+        for (int c = 0; c < CH; ++c) put(r1, c, 1, kbeg + BK);
         fetch(r0, kbeg + 2 * BK);
         fetch(r1, kbeg + 3 * BK);
     } else {
@@ -194,14 +202,14 @@ __device__ __forceinline__ void split_tile(const float* __restrict__ x, const fl
         read(f0, 0);
         __syncthreads();
         for (int k0 = kbeg; k0 < kend; k0 += 2 * BK) {      // (a slab past the end is zeros)
-            step(k0, f0, f1, r0, SLAB, 0);
-            step(k0 + BK, f1, f0, r1, 0, SLAB);
+            step(k0, f0, f1, r0, 1, 0);
+            step(k0 + BK, f1, f0, r1, 0, 1);
         }
     } else {
         for (int k0 = kbeg; k0 < kend; k0 += 2 * BK) {
             read(f0, 0);
-            step(k0 - BK, f0, f0, r1, 0, SLAB);
-            read(f0, SLAB);
+            step(k0 - BK, f0, f0, r1, 0, 1);
+            read(f0, 1);
             step(k0, f0, f0, r0, 0, 0);
         }
     }

@@ -61,7 +61,7 @@ __global__ __launch_bounds__(WM * WN * WAVE) void split_gemm_kernel(const float*
     }
     const int share = blockIdx.y;
     const int kbeg = share * kper, kend = min(K, kbeg + kper);
-    split_tile<BM, BN, WM, WN, AHEAD, EPI, GROUPED>(x, w, out, M, N, K, m0, nt, share, kbeg, kend, ldw, groups.rows, act, lds);
+    split_tile<BM, BN, WM, WN, AHEAD, EPI, GROUPED>(x, w, out, M, N, K, m0, nt, share, kbeg, kend, ldw, groups.rows, act, SplitSlabs::in<BM, BN>(lds));
 }
 
 // out[i] = the sum of the shares' n numbers, in their order; V at a time (n is a multiple of V).

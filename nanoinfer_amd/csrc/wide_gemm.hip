@@ -29,16 +29,9 @@
 // 44 : 36, 68 : 58, 121 : 111, 239 : 211; [2048, 8192] at 1,999 70 : 62.  What bounds the large ones is the clock that the chip
 // holds: matrix cores busy 64 % of the time at 1.9 GHz (the library's 65 % at 1.96; with operands of ones, which switch less, 2.3 GHz and
 // 88 us); without its loads the same kernel takes 103.  A prompt of 1,999 tokens of the 1B shape 5,170 -> 4,630 us.
+#include "lds_load.h"
 #include "rope_store.h"
 #include "split_tile.h"
-
-template <int N> struct Index { static constexpr int value = N; };
-
-// sixteen bytes a lane from memory straight into LDS: lane l's land at `to` + 16 l, `to` the same in all lanes
-__device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t from, char* to, int lane_at, int at) {
-    typedef __attribute__((address_space(3))) char lds_char;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)(lds_char*)to, 16, lane_at, at, 0, 0);
-}
 
 // Which piece of sixteen bytes of row r stands where the row's piece 0 would.
 __device__ __forceinline__ int wide_swizzle(int r) { return (r & 2) << 1 | ((r >> 4 ^ r >> 5) & 1) << 1 | (r >> 4 & 1); }

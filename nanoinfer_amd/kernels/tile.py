@@ -119,11 +119,11 @@ def _add_shares(parts: torch.Tensor, dtype: torch.dtype, out: Optional[torch.Ten
 
 # Tiles of the product in half precision: rows of x, rows of W, workgroups a compute unit holds, and in microseconds: what a
 # launch takes beside its steps, 16 columns of K with one workgroup alone on its unit and with all units full, and how late between the
-# two the time rises (the power of the share of the units that is taken).  Fitted to sweeps of all tiles and shares at 100 to
-# 2,000 rows over the layer sizes of the 1B, 3B and 8B shapes, recorded, every launch with another W: of 99 plans taken the
-# average is 2 % above the best and the worst 22.
-PAIR_TILES = ((128, 256, 1, 16.1, 0.447, 0.651, 4.2), (64, 256, 2, 12.4, 0.228, 0.729, 1.18), (128, 128, 2, 11.8, 0.278, 0.745, 1.25),
-              (64, 128, 3, 8.8, 0.115, 0.612, 1.06))
+# two the time rises (the power of the share of the units that is taken).  Fitted to sweeps of all tiles and shares at 96 to
+# 2,048 rows over the layer sizes of the 1B, 3B and 8B shapes, on two cards, recorded, every launch with another W: of 162 plans taken the
+# average is 1 % above the best and the worst 12.
+PAIR_TILES = ((128, 256, 1, 10.8, 0.401, 0.562, 4.48), (64, 256, 1, 9.9, 0.276, 0.330, 6.72), (128, 128, 1, 10.9, 0.219, 0.309, 4.98),
+              (64, 128, 2, 9.4, 0.084, 0.437, 1.59))
 
 
 def pair_lib() -> ctypes.CDLL:

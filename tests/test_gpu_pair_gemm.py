@@ -58,6 +58,22 @@ def test_pair_gemm_at_the_edges_of_its_tiles(K, tile, M, N, Kd, shares):
     assert bool((out[M] == 7.0).all())                       # nothing behind the last row
 
 
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 7, 13])
+def test_pair_gemm_with_few_stages(K, tile, steps):
+    """A share of fewer stages than the ring has, and of every remainder behind its rounds; groups of rows of x that begin with other
+    stages than the first; results that no vector can be stored to."""
+    M, N, shares = 1100, 258, 3
+    x, w = operands(M, N, 32 * steps * shares, seed=steps)
+    held = Held(K, w)
+    got = K.pair_gemm(x, held, plan=(tile, shares))
+    assert bounded(got, x, w) and error(got, x, w) <= whole(x.shape[1])
+    buffer = torch.full((M * N + 2,), 7.0, device="cuda")
+    got = K.pair_gemm(x, held, buffer[1:-1].view(M, N), plan=(tile, 1))
+    assert bounded(got, x, w) and error(got, x, w) <= whole(x.shape[1])
+    assert float(buffer[0]) == float(buffer[-1]) == 7.0
+
+
 @pytest.mark.parametrize("tile", [0, 1])
 @pytest.mark.parametrize("M,inter", [(65, 32), (130, 96), (129, 160)])
 def test_pair_gemm_gated_and_squared(K, tile, M, inter):
