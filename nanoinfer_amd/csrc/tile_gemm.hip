@@ -34,6 +34,7 @@
 // it, and are what a float32 product gives: infinities with their sign, NaN where there is no answer.  Finite results
 // pay one multiplication; 1,999 rows on [16384, 2048] take 0.63 ms, 0.95 with an infinity in one row, 38 with one in every row.
 #include "rope_store.h"
+#include "row_stores.h"
 #include "split_tile.h"
 
 template <int BM, int BN, int WM, int WN, bool AHEAD, int EPI, bool GROUPED>
@@ -191,6 +192,16 @@ __global__ __launch_bounds__(WN * WAVE, MINW) void tiled_gemm_kernel(const bf16_
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    int pos[TM], slot[TM];                                     // of the rows, with the rotation: long there when they are needed (512 rows on
+                                                               // [3072, 2048] 16.6 -> 15.8 us, with the angles of all rows asked for together)
+    if constexpr (EPI == TG_ROPE) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int m = min(m0 + i * 16 + (lane & 15), M - 1);
+            pos[i] = rope.positions[m];
+            slot[i] = rope.slots ? rope.slots[m] : -1;
+        }
+    }
     auto fetch = [&](int p) {
         const int at = min(p, pend - 1) * 128;
 #pragma unroll
@@ -255,37 +266,47 @@ __global__ __launch_bounds__(WN * WAVE, MINW) void tiled_gemm_kernel(const bf16_
     if constexpr (EPI == TG_ROPE) {
         const int o = nt * (BNT / 2) + wave, pairs = rope.hd / 32;
         if (o >= all / 2) return;
-        int pos[TM], slot[TM];
+        const int head = o / pairs, d = o % pairs * 16 + (lane >> 4) * 4;
+        RopeStore::Angles<4> t[TM];                            // of all rows, asked for together, behind one wait
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            const int m = min(m0 + i * 16 + (lane & 15), M - 1);
-            pos[i] = rope.positions[m];
-            slot[i] = rope.slots ? rope.slots[m] : -1;
-        }
+        for (int i = 0; i < TM; ++i)
+            if (rope.rotates(head)) t[i] = rope.angles<4>(pos[i], d);
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
             const int m = m0 + i * 16 + (lane & 15);
             if (m >= M) continue;
             const float a[4] = {acc[i][0][0], acc[i][0][1], acc[i][0][2], acc[i][0][3]}, b[4] = {acc[i][1][0], acc[i][1][1], acc[i][1][2], acc[i][1][3]};
-            rope.put<4>(m, pos[i], slot[i], o / pairs, o % pairs * 16 + (lane >> 4) * 4, a, b);
+            bf16_t* to = rope.place(m, slot[i], head);
+            if (!to) continue;
+            if (rope.rotates(head)) rope.turned<4>(to, d, a, b, t[i]);
+            else rope.plain<4>(to, d, a, b);
         }
         return;
     }
     const int cols = EPI == TG_GATED ? N / 2 : N;
     OUT* base = out + static_cast<size_t>(share) * M * cols;
+    constexpr int OT = EPI == TG_GATED && TN > 1 ? TN / 2 : TN, RUN = OT % 2 ? 1 : 2;      // RUN: stores that leave a row together
+    struct __attribute__((aligned(4 * sizeof(OUT)))) Four { OUT v[4]; };
+    const bool upper = RUN == 2 && (lane & 8);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-        const int m = m0 + i * 16 + (lane & 15);
-        if (m >= M) continue;
-        constexpr int OT = EPI == TG_GATED && TN > 1 ? TN / 2 : TN;
+        const int m = m0 + i * 16 + (RUN == 2 ? lane & 7 : lane & 15);
 #pragma unroll
-        for (int j = 0; j < OT; ++j) {
-            const int n = (nt * (BNT * OT / TN) + wave * OT + j) * 16 + (lane >> 4) * 4;
+        for (int j = 0; j < OT; j += RUN) {
+            const int n = (nt * (BNT * OT / TN) + wave * OT + j + upper) * 16 + (lane >> 4) * 4;
+            Four o[RUN];
+#pragma unroll
+            for (int k = 0; k < RUN; ++k) {
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = EPI == TG_GATED ? act.rough(acc[i][j + k][e], acc[i][j + k + TN - OT][e]) : act.plain(acc[i][j + k][e]);
+                store_packed<OUT, 4>(o[k].v, v);
+            }
+            if constexpr (RUN == 2) rows_together(o[0], o[1], upper);
             if (n >= cols) continue;
-            float v[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = EPI == TG_GATED ? act.rough(acc[i][j][e], acc[i][j + TN - OT][e]) : act.plain(acc[i][j][e]);
-            store_packed<OUT, 4>(base + static_cast<size_t>(m) * cols + n, v);
+            for (int k = 0; k < RUN; ++k)
+                if (m + 8 * k < M) *reinterpret_cast<Four*>(base + static_cast<size_t>(m + 8 * k) * cols + n) = o[k];
         }
     }
 }

@@ -484,15 +484,15 @@ def _wide_cost(M: int, N: int, K: int, tile: int) -> float:
 
 
 def wide_plan(M: int, N: int, K: int, gated: bool = False) -> Tuple[int, float]:
-    """(tile, estimated microseconds) of :func:`wide_gemm`.  The largest tile and the one of which a unit holds two are for the product whose
-    epilogue makes gate and up one output: where a plain product would take them the library's is ahead ([4096, 4096] at 3,000 rows
-    87 : 78 us, [6144, 4096] at 1,999 88 : 84; [3072, 2048] at 1,300 and 1,600 26.6 : 23.5, 27.2 : 23.7)."""
+    """(tile, estimated microseconds) of :func:`wide_gemm`.  The tile of which a unit holds two is for the product whose epilogue makes
+    gate and up one output: where a plain product would take it the library's is ahead ([3072, 2048] at 1,300 and 1,600 rows
+    26.6 : 23.5 us, 27.2 : 23.7)."""
     return _wide_plan(_whole(M), N, K, gated)
 
 
 @functools.lru_cache(maxsize=4096)
 def _wide_plan(M: int, N: int, K: int, gated: bool) -> Tuple[int, float]:
-    cost, tile = min((_wide_cost(M, N, K, t), t) for t in (range(len(WIDE_TILES)) if gated else (1, 2, 3)))
+    cost, tile = min((_wide_cost(M, N, K, t), t) for t in range(len(WIDE_TILES) if gated else 4))
     return tile, cost
 
 
@@ -505,7 +505,7 @@ WIDE_FLOPS = 2e9            # operations of the smallest plain product that was 
 def wide_wins(x: torch.Tensor, rows: torch.Tensor, gated: bool = False) -> bool:
     """Whether the bfloat16 product ``x . rows^T`` goes to :func:`wide_gemm`: where it is estimated to take no longer than the library's
     product (with the SwiGLU kernel behind it): 5 to 8 us, 1 us for 1.33 GFLOP, and where its tiles are few 1.5 us for 1,024 elements of K (plain
-    products with 15 % more, by which few tiles are estimated too high).  Measured in recorded launches, each with another W (us, library : this; cards differ by 10 %):
+    products of no more tiles than units with 15 % more, by which few tiles are estimated too high; not the largest tile).  Measured in recorded launches, each with another W (us, library : this; cards differ by 10 %):
 
     SwiGLU in the epilogue, from 257 rows: [16384, 2048] at 400 / 512 / 900 / 1,024 / 1,300 / 1,600 / 1,999 / 3,000 / 4,096 rows 41 : 34,
     44 : 36, 64 : 58, 68 : 58, 99 : 90, 113 : 102, 121 : 111, 183 : 157, 239 : 211 (the tiled product 37 at 400 and 39 at 512 rows),
@@ -514,10 +514,12 @@ def wide_wins(x: torch.Tensor, rows: torch.Tensor, gated: bool = False) -> bool:
     [16384, 3072] 67 : 74), and to 512 rows only on its larger tiles (a small matrix, [4096, 2048] at 512 rows, takes 19 in the smallest, 16 by
     the tiled product); to 256 rows the tiled product is as fast or faster (26 : 28).
 
-    Plain, from 513 rows (the tiled product's end) to 2,048: [2048, 8192] at 1,024 / 1,600 / 1,999 50 : 58, 66 : 58, 70 : 62, [2048, 2048] at
-    768 / 1,150 / 1,600 / 1,999 13.3 : 14.8, 19.7 : 15.8, 20.1 : 17.3, 21.2 : 18 to 22, [3072, 2048] at 1,024 / 1,300 / 1,999 20.9 : 16.0,
-    23.5 : 26.6, 28.0 : 27.2, [4096, 4096] at 1,024 / 1,999 41 : 36, 59 : 57, [4096, 14336] at 1,300 / 1,999 157 : 171, 194 : 185.  With more rows
-    the tiles are as many as the library's larger ones, which then win ([3072, 2048] at 3,000 37 : 45, [2048, 8192] at 2,500 83 : 87)."""
+    Plain, from 513 rows (the tiled product's end) to 2,048: [2048, 8192] at 1,024 / 1,600 / 2,045 50 : 58, 66 : 58, 70 : 63, [2048, 2048] at
+    800 / 1,300 / 1,600 / 2,045 15.4 : 14.8, 20.6 : 15.9, 20.7 : 17.1, 21.6 : 18.4, [3072, 2048] at 1,024 / 1,300 / 2,045 20.6 : 16.3,
+    24.1 : 24.3, 28.4 : 26.4, [4096, 4096] at 1,024 / 2,045 40.7 : 35.5, 59.1 : 56.1; the results in float32, [2048, 2048] at 2,045 23.4 : 20.6,
+    [3072, 2048] 28.7 : 29.0, [4096, 2048] 37.6 : 33.5, [8192, 2048] 64.2 : 57.5.  More tiles than units end in a round that few of them fill, where the
+    library takes other tiles ([6144, 2048] at 2,045 48 : 55, [8192, 2048] at 1,600 49 : 56); with more rows its larger ones win ([3072, 2048] at
+    3,000 37 : 45, [2048, 8192] at 2,500 83 : 87)."""
     if x.dtype != torch.bfloat16 or rows.dtype != torch.bfloat16 or x.dim() != 2 or rows.dim() != 2:
         return False
     M, K = x.shape
@@ -529,7 +531,9 @@ def wide_wins(x: torch.Tensor, rows: torch.Tensor, gated: bool = False) -> bool:
     library = M * N * K / 0.665e9
     if gated:
         return (M >= WIDE_ROWS or tile < 3) and cost <= 12.0 + library + 3.0 * M * N / 4.6e6
-    return 2.0 * M * N * K >= WIDE_FLOPS and cost <= 1.15 * (5.0 + library + 1.5e-3 * K)
+    bm, bn = WIDE_TILES[tile][:2]
+    slack = 1.15 if tile and -(-M // bm) * -(-N // bn) <= COMPUTE_UNITS else 1.0
+    return 2.0 * M * N * K >= WIDE_FLOPS and cost <= slack * (5.0 + library + 1.5e-3 * K)
 
 
 def wide_gemm(x: torch.Tensor, rows: torch.Tensor, out_dtype: Optional[torch.dtype] = None, out: Optional[torch.Tensor] = None, gated: Optional[str] = None,

@@ -14,7 +14,7 @@ def K():
 
 # rows at the edges of tiles; heads whose halves are one, two and four blocks of a wavefront's columns; a last tile of columns that is not
 # whole; slots that are left out, and none at all
-@pytest.mark.parametrize("plan", [(True, 0), (True, 1), (True, 2), (False, 1), (False, 2), (False, 3)])
+@pytest.mark.parametrize("plan", [(True, 0), (True, 1), (True, 2), (False, 0), (False, 1), (False, 2), (False, 3)])
 @pytest.mark.parametrize("M,Kd,H,KVH,hd,page", [(65, 64, 1, 1, 64, 16), (129, 128, 6, 2, 64, 5), (300, 192, 3, 1, 128, 16), (257, 320, 2, 1, 192, 7),
                                                 (1100, 128, 4, 4, 64, 16), (200, 64, 5, 5, 32, 16)])
 def test_rotated_and_stored_as_by_the_kernel_behind_the_product(K, plan, M, Kd, H, KVH, hd, page):
