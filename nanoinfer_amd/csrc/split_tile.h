@@ -51,7 +51,7 @@ __device__ __forceinline__ void split3(const float4 a, uint2& h, uint2& m, uint2
 // What a workgroup's operands wait for.  AHEAD: the operands of a slab are read from LDS while the slab before is
 // multiplied, in a second set of registers (a product of 32 workgroups 121 -> 113 us); the largest tile has no room for
 // that set and reads them when their slab begins.
-enum { TG_STORE = 0, TG_GATED = 1, TG_ROPE = 2 };       // TG_ROPE: products of bfloat16 rows alone (rope_store.h)
+enum { TG_STORE = 0, TG_GATED = 1, TG_ROPE = 2, TG_STREAM = 3 };       // the last two: products of bfloat16 rows alone (rope_store.h, row_norm.h)
 
 // EPI TG_STORE: out[share][m][n] (shares > 1: float32 sums of every share).  TG_GATED: W is [gate; up] stacked, N its
 // rows; blocks of 32 columns of a tile come from the two halves in turn, so that a lane holds gate and up of the same

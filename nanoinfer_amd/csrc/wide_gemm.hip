@@ -31,6 +31,7 @@
 // 88 us); without its loads the same kernel takes 103.  A prompt of 1,999 tokens of the 1B shape 5,170 -> 4,630 us.
 #include "lds_load.h"
 #include "rope_store.h"
+#include "row_norm.h"
 #include "row_stores.h"
 #include "split_tile.h"
 
@@ -41,10 +42,10 @@ __device__ __forceinline__ int wide_swizzle(int r) { return (r & 2) << 1 | ((r >
 
 template <int ROWS> struct WideSlot { char b[ROWS * 128]; };
 
-template <int BM, int BN, int WM, int WN, int DX, int DW, int EPI, typename OUT>
+template <int BM, int BN, int WM, int WN, int DX, int DW, int EPI, typename OUT, bool NORMED>
 __global__ __launch_bounds__(WM * WN * WAVE, 2) void wide_gemm_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                                             OUT* __restrict__ out, int M, int N, int K, int mtiles,
-                                                                            int ntiles, GatedUnit act, RopeStore rope) {
+                                                                            int ntiles, GatedUnit act, RopeStore rope, StreamStore stream, RowNorm norm) {
     constexpr int NW = WM * WN, TM = BM / WM / 16, TN = BN / WN / 16;
     constexpr int CX = BM / 8 / NW, CW = BN / 8 / NW, ALL = CX + CW;            // loads a wavefront and stage
     static_assert((TM % 4 == 0 || TM == 2) && TN % 4 == 0 && BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "whole groups of 64 rows, whole loads a wavefront");
@@ -187,11 +188,14 @@ __global__ __launch_bounds__(WM * WN * WAVE, 2) void wide_gemm_kernel(const bf16
         if constexpr (b <= DW) fetch(Index<DX * DW - b>{}, -b, Index<CX>{}, Index<(last < CX ? CX : last)>{});
         __builtin_amdgcn_sched_barrier(0);
     };
+    RowSquares<BM, NW * WAVE> squares;
+    if constexpr (NORMED) squares.ask(norm, m0, M, tid);
     ahead(Index<5>{});
     ahead(Index<4>{});
     ahead(Index<3>{});
     ahead(Index<2>{});
     ahead(Index<1>{});
+    const float factor = NORMED ? squares.factor(norm, K) : 1.f;
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(WAIT + FIRST) : "memory");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
@@ -207,6 +211,75 @@ __global__ __launch_bounds__(WM * WN * WAVE, 2) void wide_gemm_kernel(const bf16
     WIDE_STAGE(0) WIDE_STAGE(1) WIDE_STAGE(2) WIDE_STAGE(3) WIDE_STAGE(4)
 #undef WIDE_STAGE
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // (loads of stages behind the last: they land before the wavefront ends)
+
+    auto factor_of = [&](int i) {                              // of this lane's row of block i
+        if constexpr (NORMED) return reinterpret_cast<const float*>(x0.b)[(xblock + i) / 4 * 64 + (xblock + i) % 4 * 4 + row];
+        else return 1.f;
+    };
+    if constexpr (NORMED) {
+        __syncthreads();                                       // nobody reads or fills the ring any more
+        constexpr int EACH = NW * WAVE / BM;
+        if (tid % EACH == 0) reinterpret_cast<float*>(x0.b)[tid / EACH] = factor;
+        __syncthreads();
+    }
+    if constexpr (EPI == TG_STREAM) {
+        static_assert(TN == 4, "64 columns a wavefront, a part of a row's sum of squares");
+        // lane by lane what rows_together leaves it: four columns of blocks j and j + 1 of a row and of the one 32 further on
+        const int side = lane & 8 ? 16 : 0;
+        auto stream_n = [&](int j) { return nt * BN + (wn * TN + j) * 16 + side + (lane >> 4) * 4; };
+        float4 weight[TN / 2];
+#pragma unroll
+        for (int j = 0; j < TN; j += 2)
+            weight[j / 2] = stream.next ? *reinterpret_cast<const float4*>(stream.weight + min(stream_n(j), N - 4)) : make_float4(0.f, 0.f, 0.f, 0.f);
+        const bool here = nt * BN + wn * 64 < N;              // N is whole sets of 64
+        auto row_at = [&](int i, int k) { return m0 + (xblock + i) / 4 * 64 + (xblock + i) % 4 * 4 + (row & 31) + 32 * k; };
+        // what the stream holds, GROUP blocks of rows at a time: no load behind a store that it waits for
+        constexpr int GROUP = TM < 4 ? TM : 4;
+        float4 before[GROUP][TN];
+        auto load = [&](int i0) {
+#pragma unroll
+            for (int i = 0; i < GROUP; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    before[i][j] = *reinterpret_cast<const float4*>(stream.h + static_cast<size_t>(min(row_at(i0 + i, j & 1), M - 1)) * N + min(stream_n(j & ~1), N - 4));
+        };
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            if (i % GROUP == 0) load(i);
+            float sum[2] = {0.f, 0.f};
+            uint2 next[2][TN / 2];
+#pragma unroll
+            for (int j = 0; j < TN; j += 2) {
+                float4 o[2];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) o[k] = make_float4(acc[i][j + k][0], acc[i][j + k][1], acc[i][j + k][2], acc[i][j + k][3]);
+                rows_together(o[0], o[1], side != 0);
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const float4 b = before[i % GROUP][j + k], w4 = weight[j / 2];
+                    const float4 v = make_float4(b.x + o[k].x, b.y + o[k].y, b.z + o[k].z, b.w + o[k].w);
+                    sum[k] += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
+                    if (here && row_at(i, k) < M) *reinterpret_cast<float4*>(stream.h + static_cast<size_t>(row_at(i, k)) * N + stream_n(j)) = v;
+                    next[k][j / 2] = make_uint2(pack_bf16x2(v.x * w4.x, v.y * w4.y), pack_bf16x2(v.z * w4.z, v.w * w4.w));
+                }
+            }
+            if (stream.next) {
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    // lane groups 0 and 2 give their four columns of the second pair of blocks for the next group's of the first: eight side by side
+                    const auto lo = __builtin_amdgcn_permlane16_swap(next[k][0].x, next[k][1].x, false, false);
+                    const auto hi = __builtin_amdgcn_permlane16_swap(next[k][0].y, next[k][1].y, false, false);
+                    sum[k] += __shfl_xor(sum[k], 8, WAVE);
+                    sum[k] += __shfl_xor(sum[k], 16, WAVE);
+                    sum[k] += __shfl_xor(sum[k], 32, WAVE);
+                    const int m = row_at(i, k), n = nt * BN + wn * 64 + (lane >> 4 & 1) * 32 + side + (lane >> 5) * 8;
+                    if (here && m < M) *reinterpret_cast<uint4*>(stream.next + static_cast<size_t>(m) * N + n) = make_uint4(lo[0], hi[0], lo[1], hi[1]);
+                    if (here && m < M && (lane >> 3) == k) stream.ss[static_cast<size_t>(m) * (N / 64) + nt * (BN / 64) + wn] = sum[k];
+                }
+            }
+        }
+        return;
+    }
 
     if constexpr (EPI == TG_ROPE) {
         static_assert(TN == 4, "64 columns a wavefront");
@@ -230,6 +303,11 @@ __global__ __launch_bounds__(WM * WN * WAVE, 2) void wide_gemm_kernel(const bf16
                 a[e] = acc[i][e / 4][e % 4];
                 b[e] = acc[i][2 + e / 4][e % 4];
             }
+            if constexpr (NORMED) {
+                const float f = factor_of(i);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) a[e] *= f, b[e] *= f;
+            }
             bf16_t* to = rope.place(m, slots[i], head);
             if (!to) continue;
             if (rope.rotates(head)) rope.turned<8>(to, d, a, b, rope.angles<8>(pos[i], d));
@@ -244,6 +322,7 @@ __global__ __launch_bounds__(WM * WN * WAVE, 2) void wide_gemm_kernel(const bf16
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
         const int m = m0 + (xblock + i) / 4 * 64 + (xblock + i) % 4 * 4 + (RUN == 2 ? row & 31 : row);
+        const float f = factor_of(i);
 #pragma unroll
         for (int j = 0; j < OT; j += RUN * GB) {
             const int n = nt * (BN * OT / TN) + wn * OT * 16 + column(upper ? j + GB : j, lane >> 4);
@@ -254,7 +333,8 @@ __global__ __launch_bounds__(WM * WN * WAVE, 2) void wide_gemm_kernel(const bf16
 #pragma unroll
                 for (int e = 0; e < GB * 4; ++e) {
                     const int b = j + k * GB + e / 4;
-                    v[e] = EPI == TG_GATED ? act.rough(acc[i][b][e % 4], acc[i][b + TN - OT][e % 4]) : act.plain(acc[i][b][e % 4]);
+                    if constexpr (EPI == TG_GATED && NORMED) v[e] = act.rough(acc[i][b][e % 4] * f, acc[i][b + TN - OT][e % 4] * f);
+                    else v[e] = EPI == TG_GATED ? act.rough(acc[i][b][e % 4], acc[i][b + TN - OT][e % 4]) : act.plain(acc[i][b][e % 4]);
                 }
                 store_packed<OUT, GB * 4>(reinterpret_cast<OUT*>(&o[k]), v);
             }
@@ -267,53 +347,100 @@ __global__ __launch_bounds__(WM * WN * WAVE, 2) void wide_gemm_kernel(const bf16
     }
 }
 
-template <int BM, int BN, int WM, int WN, int DX, int DW>
-static int launch_wide(const bf16_t* x, const bf16_t* w, void* out, int M, int N, int K, int epi, int f32, GatedUnit act, const RopeStore& rope, hipStream_t stream) {
-    const int cols = epi == TG_GATED ? N / 2 : N, each = epi == TG_GATED ? BN / 2 : BN, mt = (M + BM - 1) / BM, nt = (cols + each - 1) / each;
-    constexpr int T = WM * WN * WAVE;
+struct WideArgs {
+    const bf16_t *x, *w;
+    void* out;
+    int M, N, K, f32;
+    GatedUnit act;
+    RopeStore rope;
+    StreamStore stream;
+    RowNorm norm;
+};
+
+template <int BM, int BN, int WM, int WN, int DX, int DW> static int launch_wide(int epi, const WideArgs& a, hipStream_t stream) {
+    const int cols = epi == TG_GATED ? a.N / 2 : a.N, each = epi == TG_GATED ? BN / 2 : BN, mt = (a.M + BM - 1) / BM, nt = (cols + each - 1) / each;
+#define WIDE_LAUNCH(EPI, OUT, NORMED) wide_gemm_kernel<BM, BN, WM, WN, DX, DW, EPI, OUT, NORMED><<<mt * nt, WM * WN * WAVE, 0, stream>>>(a.x, a.w, \
+        static_cast<OUT*>(a.out), a.M, a.N, a.K, mt, nt, a.act, a.rope, a.stream, a.norm)
     if (epi == TG_GATED) {
-        wide_gemm_kernel<BM, BN, WM, WN, DX, DW, TG_GATED, bf16_t><<<mt * nt, T, 0, stream>>>(x, w, static_cast<bf16_t*>(out), M, N, K, mt, nt, act, rope);
+        if (a.norm.ss) WIDE_LAUNCH(TG_GATED, bf16_t, true);
+        else WIDE_LAUNCH(TG_GATED, bf16_t, false);
         return NI_LAUNCH_RESULT();
     }
     if constexpr (DX == 2 && BM == 128) return static_cast<int>(hipErrorInvalidValue);      // (a tile that only products with SwiGLU take)
-    else if (epi == TG_ROPE) wide_gemm_kernel<BM, BN, WM, WN, DX, DW, TG_ROPE, bf16_t><<<mt * nt, T, 0, stream>>>(x, w, static_cast<bf16_t*>(out), M, N, K, mt, nt, act, rope);
-    else if (f32) wide_gemm_kernel<BM, BN, WM, WN, DX, DW, TG_STORE, float><<<mt * nt, T, 0, stream>>>(x, w, static_cast<float*>(out), M, N, K, mt, nt, act, rope);
-    else wide_gemm_kernel<BM, BN, WM, WN, DX, DW, TG_STORE, bf16_t><<<mt * nt, T, 0, stream>>>(x, w, static_cast<bf16_t*>(out), M, N, K, mt, nt, act, rope);
+    else if (epi == TG_ROPE && a.norm.ss) WIDE_LAUNCH(TG_ROPE, bf16_t, true);
+    else if (epi == TG_ROPE) WIDE_LAUNCH(TG_ROPE, bf16_t, false);
+    else if (epi == TG_STREAM) WIDE_LAUNCH(TG_STREAM, float, false);
+    else if (a.f32) WIDE_LAUNCH(TG_STORE, float, false);
+    else WIDE_LAUNCH(TG_STORE, bf16_t, false);
+#undef WIDE_LAUNCH
     return NI_LAUNCH_RESULT();
 }
 
-static int launch_wide_tile(int tile, const void* x, const void* w, void* out, int M, int N, int K, int epi, int f32, GatedUnit act, const RopeStore& rope,
-                            void* stream) {
-    if (M <= 0 || N <= 0 || K <= 0 || K % 64 || static_cast<long>(M) * K >= 1l << 30 || static_cast<long>(N) * K >= 1l << 30 ||
-        reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w) % 16 || reinterpret_cast<uintptr_t>(out) % 16)
+static int launch_wide_tile(int tile, int epi, const WideArgs& a, void* stream) {
+    if (a.M <= 0 || a.N <= 0 || a.K <= 0 || a.K % 64 || static_cast<long>(a.M) * a.K >= 1l << 30 || static_cast<long>(a.N) * a.K >= 1l << 30 ||
+        (reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.w) | reinterpret_cast<uintptr_t>(a.out)) % 16 ||
+        (a.norm.ss && (a.norm.parts <= 0 || a.norm.parts % 4 || a.norm.parts > 64 || reinterpret_cast<uintptr_t>(a.norm.ss) % 16)))
         return static_cast<int>(hipErrorInvalidValue);
-    const bf16_t *xb = static_cast<const bf16_t*>(x), *wb = static_cast<const bf16_t*>(w);
     hipStream_t s = static_cast<hipStream_t>(stream);
     switch (tile) {
-        case 0: return launch_wide<256, 256, 2, 4, 2, 3>(xb, wb, out, M, N, K, epi, f32, act, rope, s);
-        case 1: return launch_wide<128, 256, 2, 4, 3, 3>(xb, wb, out, M, N, K, epi, f32, act, rope, s);
-        case 2: return launch_wide<256, 128, 4, 2, 3, 3>(xb, wb, out, M, N, K, epi, f32, act, rope, s);
-        case 3: return launch_wide<128, 128, 4, 2, 5, 5>(xb, wb, out, M, N, K, epi, f32, act, rope, s);
-        case 4: return launch_wide<128, 128, 2, 2, 2, 3>(xb, wb, out, M, N, K, epi, f32, act, rope, s);
+        case 0: return launch_wide<256, 256, 2, 4, 2, 3>(epi, a, s);
+        case 1: return launch_wide<128, 256, 2, 4, 3, 3>(epi, a, s);
+        case 2: return launch_wide<256, 128, 4, 2, 3, 3>(epi, a, s);
+        case 3: return launch_wide<128, 128, 4, 2, 5, 5>(epi, a, s);
+        case 4: return launch_wide<128, 128, 2, 2, 2, 3>(epi, a, s);
         default: return static_cast<int>(hipErrorInvalidValue);
     }
 }
 
-// tile: 1 = 128 x 256, 2 = 256 x 128, 3 = 128 x 128 (rows of x, rows of W), gated also 0 = 256 x 256, 4 = 128 x 128, two a unit.  f32: float32 results
-NI_EXPORT int ni_wide_gemm(const void* x, const void* w, void* out, int M, int N, int K, int tile, int gated, int f32, int activation, int squared, void* stream) {
-    if (N % (gated ? 32 : 16) || (gated && (f32 || squared))) return static_cast<int>(hipErrorInvalidValue);
-    GatedUnit act = GatedUnit::of(activation);
-    act.squared = squared != 0;
-    return launch_wide_tile(tile, x, w, out, M, N, K, gated ? TG_GATED : TG_STORE, f32, act, RopeStore{}, stream);
+// tile: 0 = 256 x 256, 1 = 128 x 256, 2 = 256 x 128, 3 = 128 x 128 (rows of x, rows of W), gated also 4 = 128 x 128, two a unit.  f32: float32
+// results.  ss (gated; or null): the rows' sums of squares in `parts` parts, by whose root mean square with eps the rows of x are divided
+NI_EXPORT int ni_wide_gemm(const void* x, const void* w, void* out, int M, int N, int K, int tile, int gated, int f32, int activation, int squared, const void* ss,
+                           int parts, float eps, void* stream) {
+    if (N % (gated ? 32 : 16) || (gated && (f32 || squared)) || (ss && !gated)) return static_cast<int>(hipErrorInvalidValue);
+    WideArgs a{};
+    a.x = static_cast<const bf16_t*>(x);
+    a.w = static_cast<const bf16_t*>(w);
+    a.out = out;
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    a.f32 = f32;
+    a.act = GatedUnit::of(activation);
+    a.act.squared = squared != 0;
+    a.norm = RowNorm{static_cast<const float*>(ss), parts, eps};
+    return launch_wide_tile(tile, gated ? TG_GATED : TG_STORE, a, stream);
+}
+
+// h [M, N] += x . w^T; with `next` (and the weight of the norm that follows) next = h * weight and ss [M, N / 64] the sums of h^2
+NI_EXPORT int ni_wide_stream(const void* x, const void* w, void* h, const void* weight, void* next, void* ss, int M, int N, int K, int tile, void* stream) {
+    if (N % 64 || !h || (next && (!weight || !ss)) || (reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(next)) % 16)
+        return static_cast<int>(hipErrorInvalidValue);
+    WideArgs a{};
+    a.x = static_cast<const bf16_t*>(x);
+    a.w = static_cast<const bf16_t*>(w);
+    a.out = h;
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    a.stream = StreamStore{static_cast<float*>(h), static_cast<const float*>(weight), static_cast<bf16_t*>(next), static_cast<float*>(ss)};
+    return launch_wide_tile(tile, TG_STREAM, a, stream);
 }
 
 // The product with the stacked matrix [q; k; v] of (H + 2 KVH) heads of hd (whole sets of 64): rotated queries to q, keys and values to the pools
 NI_EXPORT int ni_wide_qkv_rope(const void* x, const void* w, void* q, const void* positions, const void* cos_t, const void* sin_t, const void* slots, void* kpool,
-                               void* vpool, int M, int K, int H, int KVH, int hd, int page_size, int tile, void* stream) {
+                               void* vpool, int M, int K, int H, int KVH, int hd, int page_size, int tile, const void* ss, int parts, float eps, void* stream) {
     if (H <= 0 || KVH <= 0 || hd <= 0 || hd % 64 || page_size <= 0 || !q || !positions || !cos_t || !sin_t || (slots && (!kpool || !vpool)) ||
         (reinterpret_cast<uintptr_t>(kpool) | reinterpret_cast<uintptr_t>(vpool) | reinterpret_cast<uintptr_t>(cos_t) | reinterpret_cast<uintptr_t>(sin_t)) % 16)
         return static_cast<int>(hipErrorInvalidValue);
-    const RopeStore rope{(const int32_t*)positions, (const float*)cos_t, (const float*)sin_t, (const int32_t*)slots, (bf16_t*)q, (bf16_t*)kpool, (bf16_t*)vpool,
-                         H, KVH, hd, page_size};
-    return launch_wide_tile(tile, x, w, q, M, (H + 2 * KVH) * hd, K, TG_ROPE, 0, GatedUnit{}, rope, stream);
+    WideArgs a{};
+    a.x = static_cast<const bf16_t*>(x);
+    a.w = static_cast<const bf16_t*>(w);
+    a.out = q;
+    a.M = M;
+    a.N = (H + 2 * KVH) * hd;
+    a.K = K;
+    a.rope = RopeStore{(const int32_t*)positions, (const float*)cos_t, (const float*)sin_t, (const int32_t*)slots, (bf16_t*)q, (bf16_t*)kpool, (bf16_t*)vpool,
+                       H, KVH, hd, page_size};
+    a.norm = RowNorm{static_cast<const float*>(ss), parts, eps};
+    return launch_wide_tile(tile, TG_ROPE, a, stream);
 }

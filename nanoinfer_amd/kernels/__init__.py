@@ -1313,6 +1313,15 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
     rows, _ = _rows_and_tiles(weight)
     if out is not None and (isinstance(x, (NormedInput, ScaledInput)) or residual is not None):
         raise KernelError("out= goes with a plain product")
+    if residual is not None and x.shape[0] > SKINNY_MAX_ROWS:
+        if not isinstance(x, torch.Tensor) or pending is not None or not (wide_stream_ok(*x.shape, x.dtype, weight) and _plain(x)):
+            raise KernelError("the residual epilogue does not take this product")
+        if leave is None:
+            wide_stream(x, rows, residual)
+            return None
+        if not wide_leaves_ok(*x.shape, x.dtype, weight):
+            raise KernelError("this product cannot leave a norm's input")
+        return ScaledInput(*wide_stream(x, rows, residual, leave.weight), leave)
     if isinstance(x, ScaledInput):
         if residual is not None or not takes_scaled_ok(x.shape[0], x.shape[1], x.dtype, weight):
             raise KernelError("this product cannot take a scaled input")
@@ -1376,7 +1385,9 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
 
 def swiglu_takes_scaled(M: int, K: int, dtype: torch.dtype, weight_gate_up) -> bool:
     """Whether :func:`linear_swiglu` can take a :class:`ScaledInput` of M rows: the fused skinny product on a
-    re-tiled stacked matrix whose halves start on tile boundaries."""
+    re-tiled stacked matrix whose halves start on tile boundaries, or many rows on the stored one."""
+    if M > SKINNY_MAX_ROWS:
+        return DEFER_NORMS and isinstance(weight_gate_up, Weight) and M >= WIDE_ROWS and dtype == torch.bfloat16 and wide_takes(M, K, weight_gate_up.rows, True)
     return takes_scaled_ok(M, K, dtype, weight_gate_up) and (weight_gate_up.shape[0] // 2) % 16 == 0
 
 
@@ -1389,8 +1400,11 @@ def linear_swiglu(x, weight_gate_up, activation: str = "silu") -> torch.Tensor:
     if type(x) is HalvedRows:
         x = x.x
     out = torch.empty(x.shape[0], inter, dtype=x.dtype, device=x.device)
-    if isinstance(x, ScaledInput) and not swiglu_takes_scaled(x.shape[0], x.shape[1], x.dtype, weight_gate_up):
-        raise KernelError("this product cannot take a scaled input")
+    if isinstance(x, ScaledInput):
+        if not swiglu_takes_scaled(x.shape[0], x.shape[1], x.dtype, weight_gate_up):
+            raise KernelError("this product cannot take a scaled input")
+        if x.shape[0] > SKINNY_MAX_ROWS:
+            return wide_gemm(x, weight_gate_up.rows, out=out, gated=activation)
     # (past 16 rows only a matrix whose halves start on tile boundaries is streamed re-tiled)
     M, Kd = x.shape
     if isinstance(x, NormedInput) or ((skinny_wins(M, Kd, x.dtype, weight_gate_up) if M <= SKINNY_MAX_ROWS else
@@ -1451,7 +1465,7 @@ torch.backends.cudnn.allow_tf32 = False
 # products of many rows on the matrix cores
 from .tile import (HalvedRows, add_rmsnorm_halved, merge_pair_rows, merge_pair_rows_ok, experts_grouped, experts_grouped_wins, pair_gemm, pair_holds, pair_lines,  # noqa: E402,F401
                    pair_plan, pair_rows, pair_weight, pair_weight_bytes, pair_wins, qkv_rope, qkv_rope_plan, rows_of, split_gemm, split_plan, split_wins, takes_halved, tile_lib, tiled_gemm,
-                   tiled_plan, tiled_wins, wide_gemm, wide_plan, wide_wins)
+                   tiled_plan, tiled_wins, wide_gemm, wide_leaves_ok, wide_plan, wide_rope_plan, wide_stream, wide_stream_ok, wide_takes, wide_wins, WIDE_ROWS)
 # sums onto the residual stream, routed experts, the gated delta rule, attention with a bias by distance
 from .stream import (BIAS_ATTENTION_MFMA_FROM, DELTA_RUN_FROM, EXPERTS_FEW_ROWS, add_rmsnormed, add_vector,  # noqa: E402,F401
                      bias_attention, bias_attention_lib, bias_attention_mfma, bias_attention_mfma_rows, bias_attention_rows, bias_attention_runs, bias_attention_bf16_tokens, bias_attention_token_runs, delta_rule, delta_rule_lib, embed_scaled, experts_act, experts_few,

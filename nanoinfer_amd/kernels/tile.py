@@ -520,12 +520,16 @@ def wide_wins(x: torch.Tensor, rows: torch.Tensor, gated: bool = False) -> bool:
     [3072, 2048] 28.7 : 29.0, [4096, 2048] 37.6 : 33.5, [8192, 2048] 64.2 : 57.5.  More tiles than units end in a round that few of them fill, where the
     library takes other tiles ([6144, 2048] at 2,045 48 : 55, [8192, 2048] at 1,600 49 : 56); with more rows its larger ones win ([3072, 2048] at
     3,000 37 : 45, [2048, 8192] at 2,500 83 : 87)."""
-    if x.dtype != torch.bfloat16 or rows.dtype != torch.bfloat16 or x.dim() != 2 or rows.dim() != 2:
+    return (x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous() and x.data_ptr() % 16 == 0 and wide_takes(*x.shape, rows, gated))
+
+
+def wide_takes(M: int, K: int, rows: torch.Tensor, gated: bool = False) -> bool:
+    """The same of M aligned rows of K elements."""
+    if rows.dtype != torch.bfloat16 or rows.dim() != 2:
         return False
-    M, K = x.shape
     N = rows.shape[0]
     if not ((WIDE_ROWS_GATED <= M if gated else WIDE_ROWS <= M <= WIDE_ROWS_LAST) and 0 < K and K % 64 == 0 and 0 < N and N % (32 if gated else 16) == 0
-            and N * K < 1 << 30 and M * K < 1 << 30 and x.is_contiguous() and rows.is_contiguous() and x.data_ptr() % 16 == 0 and rows.data_ptr() % 16 == 0):
+            and N * K < 1 << 30 and M * K < 1 << 30 and rows.is_contiguous() and rows.data_ptr() % 16 == 0):
         return False
     tile, cost = wide_plan(M, N, K, gated)
     library = M * N * K / 0.665e9
@@ -536,13 +540,60 @@ def wide_wins(x: torch.Tensor, rows: torch.Tensor, gated: bool = False) -> bool:
     return 2.0 * M * N * K >= WIDE_FLOPS and cost <= slack * (5.0 + library + 1.5e-3 * K)
 
 
-def wide_gemm(x: torch.Tensor, rows: torch.Tensor, out_dtype: Optional[torch.dtype] = None, out: Optional[torch.Tensor] = None, gated: Optional[str] = None,
+def wide_stream_ok(M: int, K: int, dtype: torch.dtype, weight) -> bool:
+    """Whether the product of M rows of K elements onto the residual stream goes to :func:`wide_stream`."""
+    rows = getattr(weight, "rows", None)
+    return rows is not None and M >= WIDE_ROWS and dtype == torch.bfloat16 and rows.shape[0] % 64 == 0 and wide_takes(M, K, rows)
+
+
+def wide_leaves_ok(M: int, K: int, dtype: torch.dtype, weight) -> bool:
+    """Whether that product can leave the next norm's input half done: rows of 256 to 4,096 elements, whose sums of squares come in whole
+    vectors of parts of 64 columns."""
+    return wide_stream_ok(M, K, dtype, weight) and weight.rows.shape[0] % 256 == 0 and weight.rows.shape[0] <= 4096
+
+
+def wide_stream(x: torch.Tensor, rows: torch.Tensor, h: torch.Tensor, weight: Optional[torch.Tensor] = None, tile: Optional[int] = None):
+    """``h += x . rows^T`` for bfloat16 ``x`` and ``rows`` and the float32 stream ``h``.  With the ``weight`` [N] of the norm behind it
+    (``h * weight`` in bfloat16, the sums of ``h^2`` over 64 columns at a time [M, N / 64]) are returned."""
+    M, K = x.shape
+    N = rows.shape[0]
+    _gpu(x, "x", torch.bfloat16)
+    _gpu(rows, "w", torch.bfloat16, (N, K))
+    _gpu(h, "h", torch.float32, (M, N))
+    if K % 64 or K == 0 or N % 64 or N == 0 or M == 0 or (x.data_ptr() | rows.data_ptr() | h.data_ptr()) % 16 or M * K >= 1 << 30 or N * K >= 1 << 30:
+        raise KernelError(f"wide_stream does not take [{M}, {K}] x [{N}, {K}]")
+    following = ss = None
+    if weight is not None:
+        _gpu(weight, "norm weight", torch.float32, (N,))
+        if weight.data_ptr() % 16:
+            raise KernelError("the norm's weight is not aligned to 16 bytes")
+        following = torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
+        ss = torch.empty(M, N // 64, dtype=torch.float32, device=x.device)
+    _check(wide_lib().ni_wide_stream(_ptr(x), _ptr(rows), _ptr(h), _ptr(weight), _ptr(following), _ptr(ss), M, N, K,
+                                     wide_plan(M, N, K)[0] if tile is None else tile, _stream()), "wide_stream")
+    return following, ss
+
+
+def _row_norm(x, M: int, K: int):
+    """(rows, sums of squares, parts, eps) of what a product of many rows is given: rows, or a :class:`ScaledInput`."""
+    if isinstance(x, torch.Tensor):
+        return x, None, 0, ctypes.c_float(0.0)
+    _gpu(x.ss, "sums of squares", torch.float32)
+    if x.ss.dim() != 2 or x.ss.shape[0] != M or not 0 < x.ss.shape[1] <= 64 or x.ss.shape[1] % 4 or x.ss.data_ptr() % 16:
+        raise KernelError(f"sums of squares {tuple(x.ss.shape)} of {M} rows")
+    return x.x, x.ss, int(x.ss.shape[1]), ctypes.c_float(x.norm.eps)
+
+
+def wide_gemm(x, rows: torch.Tensor, out_dtype: Optional[torch.dtype] = None, out: Optional[torch.Tensor] = None, gated: Optional[str] = None,
               squared: bool = False, tile: Optional[int] = None) -> torch.Tensor:
     """``x . rows^T`` for bfloat16 ``x`` [M, K] and ``rows`` [N, K] as stored, in bfloat16 or (``out_dtype``) float32.  ``gated`` and ``squared`` as for
-    :func:`split_gemm`.  ``tile``: another than :func:`wide_plan`'s."""
+    :func:`split_gemm`.  ``tile``: another than :func:`wide_plan`'s.  With ``gated`` ``x`` may be a :class:`ScaledInput`."""
     M, K = x.shape
     N = rows.shape[0]
     out_dtype = out_dtype or x.dtype
+    x, ss, parts, eps = _row_norm(x, M, K)
+    if ss is not None and gated is None:
+        raise KernelError("the plain product does not take a scaled input")
     _gpu(x, "x", torch.bfloat16)
     _gpu(rows, "w", torch.bfloat16, (N, K))
     if gated is not None and (N % 32 or squared or out_dtype != torch.bfloat16):
@@ -558,7 +609,7 @@ def wide_gemm(x: torch.Tensor, rows: torch.Tensor, out_dtype: Optional[torch.dty
     if tile is None:
         tile = wide_plan(M, N, K, gated is not None)[0]
     _check(wide_lib().ni_wide_gemm(_ptr(x), _ptr(rows), _ptr(out), M, N, K, tile, int(gated is not None), int(out_dtype == torch.float32),
-                                   GATED_ACTIVATIONS[gated or "silu"], int(squared), _stream()), "wide_gemm")
+                                   GATED_ACTIVATIONS[gated or "silu"], int(squared), _ptr(ss), parts, eps, _stream()), "wide_gemm")
     return out
 
 
@@ -587,7 +638,9 @@ def qkv_rope_plan(x, weight, hd: int, rotary_dim: int) -> Optional[Tuple[bool, i
     it does not: heads rotated whole, of whole tiles, and a product that :func:`tiled_wins` sends to the re-tiled matrix or that the
     one on the stored matrix makes in the time of the library's and the rotating kernel's.  Measured in recorded launches, each with
     another W (us, product and kernel : this): see the two kernels."""
-    if not isinstance(x, torch.Tensor) or x.dtype != torch.bfloat16 or x.dim() != 2 or hd % 32 or rotary_dim != hd:
+    if not isinstance(x, torch.Tensor):
+        return wide_rope_plan(*x.shape, x.dtype, weight, hd, rotary_dim) if hasattr(x, "ss") else None
+    if x.dtype != torch.bfloat16 or x.dim() != 2 or hd % 32 or rotary_dim != hd:
         return None
     M, K = x.shape
     rows = getattr(weight, "rows", None)
@@ -599,19 +652,33 @@ def qkv_rope_plan(x, weight, hd: int, rotary_dim: int) -> Optional[Tuple[bool, i
     if M <= TILED_ROWS:
         if not tiled_wins(x, weight):
             return None
-    elif not (rows.is_contiguous() and rows.data_ptr() % 16 == 0):
-        return None
+    else:
+        return wide_rope_plan(M, K, x.dtype, weight, hd, rotary_dim)
     return _qkv_rope_plan(_whole(M), N, K, hd, getattr(weight, "tiles", None) is not None)
 
 
-def qkv_rope(x: torch.Tensor, weight, positions: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, slot_mapping: Optional[torch.Tensor],
+def wide_rope_plan(M: int, K: int, dtype: torch.dtype, weight, hd: int, rotary_dim: int) -> Optional[Tuple[bool, int]]:
+    """:func:`qkv_rope_plan` of M aligned rows past those of the tiled product, also where they are a :class:`ScaledInput`."""
+    rows = getattr(weight, "rows", None)
+    if rows is None or dtype != torch.bfloat16 or rows.dtype != torch.bfloat16 or M <= TILED_ROWS or hd % 64 or rotary_dim != hd:
+        return None
+    N = rows.shape[0]
+    if (K == 0 or K % 64 or N == 0 or N % hd or M * K >= 1 << 30 or (N + 15) * K >= 1 << 30 or not rows.is_contiguous() or rows.data_ptr() % 16):
+        return None
+    return _qkv_rope_plan(_whole(M), N, K, hd, False)
+
+
+def qkv_rope(x, weight, positions: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, slot_mapping: Optional[torch.Tensor],
              kpool: Optional[torch.Tensor], vpool: Optional[torch.Tensor], H: int, KVH: int, hd: int, plan: Tuple[bool, int]) -> torch.Tensor:
     """``x . weight^T`` for many bfloat16 rows and the stacked matrix [q; k; v]: returns the rotated queries [M, H * hd]; rotated keys and
     plain values go into the pools ([pages, KVH, page_size, hd]) at ``slot_mapping`` (below zero, or absent: not stored).  ``plan`` as
-    :func:`qkv_rope_plan` gives it."""
+    :func:`qkv_rope_plan` gives it.  On the stored matrix ``x`` may be a :class:`ScaledInput`."""
     M, K = x.shape
     on_tiles, tile = plan
     rows, tiles = weight.rows, weight.tiles
+    x, ss, parts, eps = _row_norm(x, M, K)
+    if ss is not None and on_tiles:
+        raise KernelError("the product with the re-tiled matrix does not take a scaled input")
     _gpu(x, "x", torch.bfloat16)
     _gpu(rows, "w_qkv", torch.bfloat16, ((H + 2 * KVH) * hd, K))
     _gpu(positions, "positions", torch.int32, (M,))
@@ -633,9 +700,9 @@ def qkv_rope(x: torch.Tensor, weight, positions: torch.Tensor, cos: torch.Tensor
             raise KernelError(f"pool must be [pages, {KVH}, page_size, {hd}] at a multiple of 16 bytes, is {tuple(kpool.shape)}")
         page_size = kpool.shape[2]
     q = torch.empty(M, H * hd, dtype=torch.bfloat16, device=x.device)
-    launch = tile_lib().ni_tiled_qkv_rope if on_tiles else wide_lib().ni_wide_qkv_rope
+    launch, norm = (tile_lib().ni_tiled_qkv_rope, ()) if on_tiles else (wide_lib().ni_wide_qkv_rope, (_ptr(ss), parts, eps))
     _check(launch(_ptr(x), _ptr(matrix), _ptr(q), _ptr(positions), _ptr(cos), _ptr(sin), _ptr(slot_mapping), _ptr(kpool), _ptr(vpool), M, K, H, KVH, hd,
-                  page_size, tile, _stream()), "qkv_rope")
+                  page_size, tile, *norm, _stream()), "qkv_rope")
     return q
 
 

@@ -328,6 +328,8 @@ class Attention(Part):
     def adds_residual(self, T: int) -> bool:
         """Whether ``forward`` can take ``residual=h`` for T tokens: its output then goes into the residual
         stream without a kernel for the sum (added by the product itself, or left as float32 addends)."""
+        if T > K.SKINNY_MAX_ROWS:
+            return K.FUSE_NORMS and type(self).output is Attention.output and K.wide_stream_ok(T, self.H * self.hd, self.rt.dtype, self.w_o)
         return K.FUSE_NORMS and K.residual_epilogue_ok(T, self.H * self.hd, self.rt.dtype, self.w_o)
 
     def carries_addends(self, T: int, addends: int) -> bool:
@@ -343,12 +345,19 @@ class Attention(Part):
         """Whether ``forward`` takes, for T tokens, the input that the product before the norm left half done
         (a :class:`nanoinfer_amd.kernels.ScaledInput`): its first product divides by the rows' root mean squares."""
         d = self.w_qkv.shape[1]
+        if T > K.SKINNY_MAX_ROWS:
+            cls, tables = type(self), self.position.tables()
+            return (K.DEFER_NORMS and tables is not None and cls.forward is Attention.forward and cls.project is Attention.project
+                    and cls.project_rotate_write is Attention.project_rotate_write and cls.rotate_and_write is Attention.rotate_and_write
+                    and K.wide_rope_plan(T, d, self.rt.dtype, self.w_qkv, self.hd, 2 * tables[0].shape[1]) is not None)
         return (type(self).project is Attention.project and K.takes_scaled_ok(T, d, self.rt.dtype, self.w_qkv)
                 and (self._fused_projection(T, d, self.rt.dtype) or type(self).rotate_and_write is Attention.rotate_and_write))
 
     def leaves_scaled(self, T: int) -> bool:
         """Whether ``forward``, given ``residual=h`` and ``leave`` (the next norm's weight and eps), returns
         that norm's input half done for T tokens."""
+        if T > K.SKINNY_MAX_ROWS:
+            return K.DEFER_NORMS and self.adds_residual(T) and K.wide_leaves_ok(T, self.H * self.hd, self.rt.dtype, self.w_o)
         return (type(self).output is Attention.output and self.adds_residual(T)
                 and K.leaves_scaled_ok(T, self.H * self.hd, self.rt.dtype, self.w_o))
 
@@ -509,6 +518,8 @@ class SwiGLU(Part):
                 and K.norm_prologue_ok(T, d, self.rt.dtype, self.w_gate_up))
 
     def adds_residual(self, T: int) -> bool:
+        if T > K.SKINNY_MAX_ROWS:
+            return K.FUSE_NORMS and type(self).forward is SwiGLU.forward and K.wide_stream_ok(T, self.intermediate_size, self.rt.dtype, self.w_down)
         return K.FUSE_NORMS and K.residual_epilogue_ok(T, self.intermediate_size, self.rt.dtype, self.w_down)
 
     def carries_addends(self, T: int, addends: int) -> bool:
@@ -518,9 +529,13 @@ class SwiGLU(Part):
                 and K.residual_takes_addends(T, self.intermediate_size, self.rt.dtype, self.w_down))
 
     def takes_scaled(self, T: int) -> bool:
+        if T > K.SKINNY_MAX_ROWS and not (type(self).forward is SwiGLU.forward and type(self).hidden is SwiGLU.hidden):
+            return False
         return K.swiglu_takes_scaled(T, self.w_gate_up.shape[1], self.rt.dtype, self.w_gate_up)
 
     def leaves_scaled(self, T: int) -> bool:
+        if T > K.SKINNY_MAX_ROWS:
+            return K.DEFER_NORMS and self.adds_residual(T) and K.wide_leaves_ok(T, self.intermediate_size, self.rt.dtype, self.w_down)
         return self.adds_residual(T) and K.leaves_scaled_ok(T, self.intermediate_size, self.rt.dtype, self.w_down)
 
     def takes_halved(self, T: int) -> bool:

@@ -74,3 +74,15 @@ def test_where_bfloat16_products_of_many_rows_on_the_stored_matrix_go(N, Kd, gat
     assert not K.wide_wins(x, rows, gated) and not K.wide_wins(x, rows.float(), gated)
     if Kd < 1 << 20:
         assert not K.wide_wins(torch.empty(Kd, 1024, dtype=torch.bfloat16, device="meta").t(), rows, gated)
+
+
+@pytest.mark.parametrize("N,Kd,M,adds,leaves", [(2048, 2048, 1999, True, True), (2048, 8192, 1999, True, True), (2048, 2048, 1100, True, True), (2048, 8192, 1100, False, False),
+                                                (2048, 2048, 512, False, False), (2048, 2048, 2049, False, False), (4160, 2048, 1200, True, False), (3136, 4096, 1024, True, False), (2064, 2048, 1999, False, False)])
+def test_which_products_go_onto_the_stream_in_their_epilogue(N, Kd, M, adds, leaves):
+    """Those that go to the product on the stored matrix at all; sums of squares are left in whole vectors of parts of 64 columns, at most 64."""
+    class Stored:
+        tiles = torch.empty(0)
+        rows = torch.empty(N, Kd, dtype=torch.bfloat16, device="meta")
+
+    assert K.wide_stream_ok(M, Kd, torch.bfloat16, Stored()) == adds and K.wide_leaves_ok(M, Kd, torch.bfloat16, Stored()) == leaves
+    assert not K.wide_stream_ok(M, Kd, torch.float32, Stored()) and not K.wide_stream_ok(M, Kd, torch.bfloat16, Stored.rows)
