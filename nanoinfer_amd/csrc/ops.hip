@@ -556,6 +556,13 @@ NI_EXPORT int ni_embedding(const void* ids, const void* table, void* out, int T,
     return NI_LAUNCH_RESULT();
 }
 
+// Whether the norm of rows of d numbers takes a vector of four a thread instead of two: more wavefronts a row to wait with, half the
+// chain in each.  Two : one (us, rows of 2,048 in bfloat16): 17 rows 3.7 : 3.2, 64 with four addends 3.8 : 3.3, 512 6.9 : 6.3, 2,045 19.2 : 18.2,
+// of 3,072 at 17 / 512 / 2,045 rows 3.6 : 3.4, 5.6 : 5.5, 16.4 : 15.7; past 4,096 a workgroup has no more threads.  Float32 rows may be left as pairs
+// of halves too, which keeps a thread at work: of 2,048 at 164 / 512 / 1,024 rows 5.4 : 4.7, 9.1 : 8.7, 13.2 : 13.0, but 1,500 12.1 : 13.0, and of 3,072
+// at 512 8.1 : 8.7 (the norm that leaves none goes by the same line: the same bits).
+static bool one_vector_a_thread(int d, int n_rows, bool float32) { return float32 ? d <= 2048 && n_rows <= 1024 : d <= 4096; }
+
 template <typename TP, typename TO>
 static void launch_add_rmsnorm(float* h, const TP* pending, int addends, size_t addend_stride, const float* w, TO* out,
                                const int32_t* rows, int n_rows, int d, float eps, hipStream_t stream) {
@@ -564,6 +571,10 @@ static void launch_add_rmsnorm(float* h, const TP* pending, int addends, size_t 
         const int threads = d <= NV * 64 ? 64 : d <= NV * 128 ? 128 : d <= NV * 256 ? 256 : d <= NV * 512 ? 512 : 1024;
         if (d % 4 == 0 && aligned_to(16, h, w) && aligned_to(4 * sizeof(TP), pending) && aligned_to(4 * sizeof(TO), out) &&
             (addends <= 1 || addend_stride % 4 == 0)) {
+            if (one_vector_a_thread(d, n_rows, sizeof(TO) == 4)) {
+                add_rmsnorm_vec_kernel<TP, TO, 1><<<n_rows, (d / 4 + WAVE - 1) / WAVE * WAVE, 0, stream>>>(h, pending, addends, addend_stride, w, out, rows, d, eps);
+                return;
+            }
             add_rmsnorm_vec_kernel<TP, TO, NV / 4><<<n_rows, threads, 0, stream>>>(h, pending, addends, addend_stride, w, out,
                                                                                   rows, d, eps);
             return;
@@ -603,7 +614,10 @@ NI_EXPORT int ni_add_rmsnorm_halves(void* h, const void* pending, int addends, s
         !aligned_to(16, planes) || (addends > 1 && addend_stride % 4))
         return static_cast<int>(hipErrorInvalidValue);
     const int threads = d <= NV * 64 ? 64 : d <= NV * 128 ? 128 : d <= NV * 256 ? 256 : d <= NV * 512 ? 512 : 1024;
-    add_rmsnorm_vec_kernel<float, float, NV / 4, true><<<n_rows, threads, 0, stream>>>(
+    if (one_vector_a_thread(d, n_rows, true))
+        add_rmsnorm_vec_kernel<float, float, 1, true><<<n_rows, (d / 4 + WAVE - 1) / WAVE * WAVE, 0, stream>>>(
+            (float*)h, (const float*)pending, addends, addend_stride, (const float*)w, (float*)out, nullptr, d, eps, (char*)planes, (int2*)info);
+    else add_rmsnorm_vec_kernel<float, float, NV / 4, true><<<n_rows, threads, 0, stream>>>(
         (float*)h, (const float*)pending, addends, addend_stride, (const float*)w, (float*)out, nullptr, d, eps, (char*)planes, (int2*)info);
     return NI_LAUNCH_RESULT();
 }

@@ -119,3 +119,20 @@ def test_merged_runs_and_their_halves_are_those_of_the_two_passes(K, T, H, hd, r
                 lambda: K.merge_pair_rows(part_o.view(-1), part_ml.view(-1), got.x[:, :-8].contiguous(), H, hd, runs)):
         with pytest.raises(K.KernelError):
             bad()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,d", [(9, 4), (9, 252), (9, 260), (1024, 2048), (1025, 2048), (3, 2052), (3, 4096), (3, 4100)])
+def test_a_norm_on_both_sides_of_a_vector_a_thread(K, dtype, T, d):
+    """Against 64 bits: a sum of d squares (at most d + 2 roundings), the root and the division, two products, and one rounding to the type."""
+    g = torch.Generator().manual_seed(T + d)
+    h, w, parts = torch.randn(T, d, generator=g), torch.randn(d, generator=g), torch.randn(5, T, d, generator=g)
+    hd = h.cuda()
+    out = K.add_rmsnorm(hd, parts.cuda(), w.cuda(), 1e-5, torch.empty(T, d, device="cuda", dtype=dtype))
+    stream = h
+    for p in parts:
+        stream = stream + p                                    # in their order
+    assert torch.equal(hd.cpu(), stream)
+    want = stream.double() * ((stream.double() ** 2).mean(1, keepdim=True) + 1e-5).rsqrt() * w.double()
+    off = ((d + 2) / 2 + 5) * 2.0 ** -24 + (2.0 ** -8 if dtype == torch.bfloat16 else 0.0)
+    assert bool(((out.cpu().double() - want).abs() <= off * want.abs() + 1e-30).all())
