@@ -1314,9 +1314,11 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
     if out is not None and (isinstance(x, (NormedInput, ScaledInput)) or residual is not None):
         raise KernelError("out= goes with a plain product")
     if residual is not None and x.shape[0] > SKINNY_MAX_ROWS:
-        if not isinstance(x, torch.Tensor) or pending is not None or not (wide_stream_ok(*x.shape, x.dtype, weight) and _plain(x)):
+        if not isinstance(x, torch.Tensor) or pending is not None or not wide_stream_ok(*x.shape, x.dtype, weight):
             raise KernelError("the residual epilogue does not take this product")
-        if leave is None:
+        if not _plain(x):
+            x = x.clone(memory_format=torch.contiguous_format)
+        if leave is None or leave.weight.data_ptr() % 16:      # (the norm behind it then runs as a kernel of its own)
             wide_stream(x, rows, residual)
             return None
         if not wide_leaves_ok(*x.shape, x.dtype, weight):

@@ -1,4 +1,4 @@
-"""Python face of the kernels in ``csrc/tile_gemm.hip``: products of many rows on the matrix cores, and the rules by
+"""Python face of the kernels in ``csrc/tile_gemm.hip``, ``pair_gemm.hip`` and ``wide_gemm.hip``: products of many rows on the matrix cores, and the rules by
 which a product goes there, how it is cut into tiles and shares, and where the library's product stays."""
 from __future__ import annotations
 

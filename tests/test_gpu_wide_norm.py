@@ -88,6 +88,19 @@ def test_what_they_do_not_take(K):
             bad()
 
 
+def test_rows_and_weights_that_are_not_aligned(K):
+    """Rows with a stride, or off sixteen bytes, are copied; a norm's weight off them leaves the norm to its kernel."""
+    M, N, Kd = 1999, 2048, 2048
+    wide, w = draw(M, Kd + 8, seed=1).bfloat16().cuda(), K.Weight(draw(N, Kd, seed=2).bfloat16().cuda())
+    flat = draw(M * Kd + 1, seed=3).bfloat16().cuda()
+    weight = draw(N + 1, seed=4).cuda()
+    for x in (wide[:, :Kd], flat[1:].view(M, Kd)):
+        a, b = torch.zeros(M, N, device="cuda"), torch.zeros(M, N, device="cuda")
+        left = K.linear(x, w, residual=a, leave=K.NormSpec(weight[:N], 1e-5))
+        assert K.linear(x.clone(memory_format=torch.contiguous_format), w, residual=b, leave=K.NormSpec(weight[1:], 1e-5)) is None
+        assert torch.equal(a, b) and torch.equal(left.x, (a * weight[:N]).bfloat16())
+
+
 def test_a_prompt_with_its_norms_in_halves(K, monkeypatch):
     """A prompt of 1,700 tokens at the 1B layer sizes in one portion, launched and recorded, against the plain implementation; every
     product onto the stream but the last one leaves the next norm's input, and the products behind those take it."""
