@@ -120,19 +120,28 @@ def _add_shares(parts: torch.Tensor, dtype: torch.dtype, out: Optional[torch.Ten
 # Tiles of the product in half precision: rows of x, rows of W, workgroups a compute unit holds, and in microseconds: what a
 # launch takes beside its steps, 16 columns of K with one workgroup alone on its unit and with all units full, and how late between the
 # two the time rises (the power of the share of the units that is taken).  Fitted to sweeps of all tiles and shares at 96 to
-# 2,048 rows over the layer sizes of the 1B, 3B and 8B shapes, on two cards, recorded, every launch with another W: of 162 plans taken the
+# 2,048 rows over the layer sizes of the 1B, 3B and 8B shapes, on two cards, recorded, every launch with another W: of 162 plans taken by time alone the
 # average is 1 % above the best and the worst 12.
 PAIR_TILES = ((128, 256, 1, 10.8, 0.401, 0.562, 4.48), (64, 256, 1, 9.9, 0.276, 0.330, 6.72), (128, 128, 1, 10.9, 0.219, 0.309, 4.98),
               (64, 128, 2, 9.4, 0.084, 0.437, 1.59))
+PAIR_SUMS = (1, 2, 2, 2)        # sums that a share's large products are added in (SUMS of the kernel)
+# The same figures of a layout with one sum a share, W in registers and 32 x 32 products.  Its plans say how many partial sums a result is made of
+# at least: the fewer there are the longer each is, and every addition is rounded.  Rms error beside the rows' norms, with that layout's
+# plan : by time alone : with as many sums (1e-7): 700 rows on [2048, 2048] 1.71 : 2.21 : 1.71, 1,300 on
+# [2048, 8192] 3.43 : 4.15 : 2.53, 2,048 on [5120, 3072] 2.22 : 2.64 : 2.22, 600 on [16384, 3072] 2.22 : 2.64 : 2.22, 448 on [6144, 4096] 2.51 : 3.00 :
+# 1.91; of 54 products and 18 with SwiGLU none is above the first by more than 0.2 %.  One plan in 70 is another by this, estimated to be 2 %
+# slower on average and 4 at worst.
+PAIR_SUM_TILES = ((128, 256, 1, 16.1, 0.447, 0.651, 4.2), (64, 256, 2, 12.4, 0.228, 0.729, 1.18), (128, 128, 2, 11.8, 0.278, 0.745, 1.25),
+                  (64, 128, 3, 8.8, 0.115, 0.612, 1.06))
 
 
 def pair_lib() -> ctypes.CDLL:
     return _load(_build.PAIR_GEMM)
 
 
-def _pair_cost(M: int, N: int, K: int, tile: int, shares: int, groups: int = 1) -> float:
+def _pair_cost(M: int, N: int, K: int, tile: int, shares: int, groups: int = 1, tiles_of=PAIR_TILES) -> float:
     """Microseconds of a product in half precision, by the figures above.  ``groups`` as for :func:`_split_cost`."""
-    bm, bn, held, fixed, alone, loaded, late = PAIR_TILES[tile]
+    bm, bn, held, fixed, alone, loaded, late = tiles_of[tile]
     tiles = -(-M // bm) if groups == 1 else M // bm + (groups + 1) // 2
     full, rest = divmod(tiles * -(-N // bn) * shares, COMPUTE_UNITS * held)
     steps = -(-K // (32 * shares)) * 2
@@ -145,10 +154,16 @@ def pair_plan(M: int, N: int, K: int, gated: bool = False) -> Tuple[int, int, fl
     return _pair_plan(_whole(M), N, K, gated)
 
 
+def _pair_shares(K: int, shares: int) -> int:
+    """How many of ``shares`` shares of whole stages of 32 columns are not empty."""
+    return -(-K // (-(-K // (32 * shares)) * 32))
+
+
 @functools.lru_cache(maxsize=4096)
 def _pair_plan(M: int, N: int, K: int, gated: bool) -> Tuple[int, int, float]:
-    cost, tile, shares = min((_pair_cost(M, N, K, t, s), t, s) for t in range(2 if gated else 4)
-                             for s in ((1,) if gated else (1, 2, 3, 4, 6, 8, 12)) if s == 1 or K // s >= 256)
+    plans = [(t, s) for t in range(2 if gated else 4) for s in ((1,) if gated else (1, 2, 3, 4, 6, 8, 12)) if s == 1 or K // s >= 256]
+    sums = _pair_shares(K, min((_pair_cost(M, N, K, t, s, 1, PAIR_SUM_TILES), t, s) for t, s in plans)[2])
+    cost, tile, shares = min((_pair_cost(M, N, K, t, s), t, s) for t, s in plans if _pair_shares(K, s) * PAIR_SUMS[t] >= sums)
     return tile, shares, cost
 
 

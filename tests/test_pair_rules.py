@@ -39,3 +39,13 @@ def test_experts_of_few_rows_stay_together(pairs):
         up, down = up.rows, down.rows
     wins = [K.experts_grouped_wins(rows(M, 2048, False), up, down, 4, 16) for M in (65, 96, 127, 300, 1500)]
     assert wins == [False, False, False, True, True]
+
+
+@pytest.mark.parametrize("M,N,Kd,sums", [(700, 2048, 2048, 4), (1300, 2048, 8192, 3), (1999, 5120, 3072, 3), (2048, 5120, 3072, 3), (600, 16384, 3072, 3),
+                                         (448, 6144, 4096, 3), (192, 8192, 2048, 4), (1300, 2048, 4096, 3), (1000, 1536, 1536, 3), (512, 2048, 2048, 4)])
+def test_of_how_many_partial_sums_a_result_is_made(M, N, Kd, sums):
+    """A plan does not make its sums longer, each of their additions rounded, than plans did when a share was one sum: shares that are not empty, and the
+    sums that the tile has for each of them."""
+    tile, shares = K.pair_plan(M, N, Kd)[:2]
+    per = -(-Kd // (32 * shares)) * 32
+    assert -(-Kd // per) * (1 if tile == 0 else 2) >= sums
