@@ -389,7 +389,8 @@ __global__ void rope_kv_write_vec_kernel(T* __restrict__ qkv, const int32_t* __r
 // The same for a product that was cut along K: its shares' float32 sums [S][T][(H + 2 KVH) * hd] are added in their order, rotated and
 // stored, the queries in rows of their own.  One pass instead of two (512 rows of the 1B shape in float32, four shares of 6 MB: 6.3 us for a
 // kernel that adds them and 5.5 for the one above, 7.4 here): bound by the shares, which the caches hold.  Dims in vectors of four.
-// SHARES: how many, known to the compiler, so that all are asked for at once; 0: `S`.
+// SHARES: how many, known to the compiler, so that all are asked for at once; 0: `S`, by fours.  Six shares of 65 rows of [5120, 3072] in bfloat16, the
+// product counted: 16.3 us, 21.8 where each waited for the one before; a kernel that adds them and the one above 18.6.
 template <typename T, int SHARES>
 __global__ __launch_bounds__(256) void rope_kv_write_shares_kernel(const float* __restrict__ parts, int S, T* __restrict__ q, const int32_t* __restrict__ positions,
                                                                    const float* __restrict__ cos_t, const float* __restrict__ sin_t,
@@ -416,7 +417,18 @@ __global__ __launch_bounds__(256) void rope_kv_write_shares_kernel(const float* 
 #pragma unroll
                 for (int e = 0; e < V; ++e) v[e] += u[p][e];
         } else {
-            for (int p = 1; p < S; ++p) {
+            constexpr int EACH = 4;
+            int p = 1;
+            for (; p + EACH <= S; p += EACH) {
+                float u[EACH][V];
+#pragma unroll
+                for (int i = 0; i < EACH; ++i) VecIO<float, V>::load(row + (p + i) * share + at, u[i]);
+#pragma unroll
+                for (int i = 0; i < EACH; ++i)
+#pragma unroll
+                    for (int e = 0; e < V; ++e) v[e] += u[i][e];
+            }
+            for (; p < S; ++p) {
                 float u[V];
                 VecIO<float, V>::load(row + p * share + at, u);
 #pragma unroll
@@ -676,6 +688,10 @@ NI_EXPORT int ni_rope_kv_write_shares(const void* parts, int shares, void* q, co
         if (shares == 2) launch(rope_kv_write_shares_kernel<E, 2>, qt, kp, vp);
         else if (shares == 3) launch(rope_kv_write_shares_kernel<E, 3>, qt, kp, vp);
         else if (shares == 4) launch(rope_kv_write_shares_kernel<E, 4>, qt, kp, vp);
+        else if (shares == 6) launch(rope_kv_write_shares_kernel<E, 6>, qt, kp, vp);
+        else if (shares == 8) launch(rope_kv_write_shares_kernel<E, 8>, qt, kp, vp);
+        else if (shares == 10) launch(rope_kv_write_shares_kernel<E, 10>, qt, kp, vp);
+        else if (shares == 12) launch(rope_kv_write_shares_kernel<E, 12>, qt, kp, vp);
         else launch(rope_kv_write_shares_kernel<E, 0>, qt, kp, vp);
     };
     if (dtype == 0) typed((float*)q, (float*)kpool, (float*)vpool);

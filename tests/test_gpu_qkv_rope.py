@@ -105,3 +105,21 @@ def test_the_shares_of_a_cut_product_added_rotated_and_stored(K, dtype, T, S, H,
                 lambda: K.rope_kv_write_shares(parts, positions, cos, sin, slots, pools[0], None, H, KVH, hd, dtype)):
         with pytest.raises(K.KernelError):
             bad()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("S", [5, 8, 10, 12, 13])
+def test_as_many_shares_as_plans_have(K, dtype, S):
+    """The numbers of shares that are compiled and their neighbours, whose places in a sum differ by bits where one is left out or taken twice."""
+    T, H, KVH, hd = 70, 3, 1, 64
+    g = torch.Generator().manual_seed(S)
+    parts, angle = torch.randn(S, T, (H + 2 * KVH) * hd, generator=g).cuda(), torch.rand(T, hd // 2, generator=g) * 6.28
+    cos, sin, at = angle.cos().cuda(), angle.sin().cuda(), torch.arange(T, dtype=torch.int32).cuda()
+    pools, want = ([torch.zeros(5, KVH, 16, hd, device="cuda", dtype=t) for _ in range(2)] for t in (dtype, torch.float32))
+    q = K.rope_kv_write_shares(parts, at, cos, sin, at, *pools, H, KVH, hd, dtype)
+    whole = parts[0].clone()
+    for p in range(1, S):
+        whole += parts[p]
+    K.rope_kv_write(whole, at, cos, sin, at, *want, H, KVH, hd)
+    for got, true in ((q, whole[:, :H * hd].contiguous()), *zip(pools, want)):
+        assert torch.equal(got, true.to(dtype))
