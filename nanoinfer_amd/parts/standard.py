@@ -405,7 +405,7 @@ class Attention(Part):
         plan = K.qkv_rope_plan(x, self.w_qkv, self.hd, rot)
         if plan is not None:
             return K.qkv_rope(x, self.w_qkv, ctx.positions, cos, sin, slots, cache.kpool, cache.vpool, self.H, self.KVH, self.hd, plan)
-        qkv = K.linear(x, self.w_qkv, addends=K.rope_shares_ok(self.hd, rot))
+        qkv = K.linear(x, self.w_qkv, addends=K.qkv_shares_ok(x, self.w_qkv, self.hd, rot))
         if qkv.dim() == 3:
             return K.rope_kv_write_shares(qkv, ctx.positions, cos, sin, slots, cache.kpool, cache.vpool, self.H, self.KVH, self.hd, x.dtype)
         return self.rotate_and_write(qkv, ctx, cache)

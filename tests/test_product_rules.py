@@ -99,3 +99,20 @@ def test_where_products_of_many_rows_rotate_and_store(N, Kd, hd, here, there):
     for M in here + there:
         plan = K.qkv_rope_plan(torch.empty(M, Kd, dtype=torch.bfloat16, device="meta"), Stored(), hd, hd)
         assert plan == K.wide_rope_plan(M, Kd, torch.bfloat16, Stored(), hd, hd) and (plan is not None) == (M in here), M
+
+
+@pytest.mark.parametrize("N,Kd,hd,whole,shares,inside", [(5120, 3072, 128, (), (65, 256, 300, 384), (400, 512)), (6144, 4096, 128, (300, 400, 512), (65, 256, 352, 384), ()),
+                                                         (3072, 2048, 64, (300, 320), (65, 192, 224, 256), (352, 512)), (2048, 2048, 64, (300, 384, 512), (65, 256), ()),
+                                                         (2560, 2048, 128, (300, 384), (65, 256), (400, 512)), (1536, 1024, 64, (), (65, 128), (160, 512))])
+def test_where_stacked_products_of_65_to_512_rows_rotate_and_store(N, Kd, hd, whole, shares, inside):
+    """In a kernel behind the product, in the pass that adds its shares, or in its epilogue: whichever was measured to be fastest, or as fast."""
+    class Stored:
+        tiles = torch.empty(0)
+        rows = torch.empty(N, Kd, dtype=torch.bfloat16, device="meta")
+
+    for M in whole + shares + inside:
+        x = torch.empty(M, Kd, dtype=torch.bfloat16, device="meta")
+        assert (K.qkv_rope_plan(x, Stored(), hd, hd) is not None) == (M in inside), M
+        assert M in inside or K.qkv_shares_ok(x, Stored(), hd, hd) == (M in shares), M
+    assert not K.qkv_shares_ok(x, Stored(), 36, 36) and not K.qkv_shares_ok(x, Stored.rows, hd, hd)
+    assert K.qkv_shares_ok(torch.empty(300, Kd), Stored(), hd, hd)
