@@ -1375,7 +1375,7 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
         return split_gemm(x, rows, out, addends=addends)
     if tiled_wins(x, weight, addends=addends) and (out is None or out.data_ptr() % 16 == 0):
         return tiled_gemm(x, weight, out_dtype, out, addends=addends)
-    if wide_wins(x, rows) and (out is None or out.data_ptr() % 16 == 0):
+    if wide_wins(x, rows, to="float32" if out_dtype == torch.float32 else "bfloat16") and (out is None or out.data_ptr() % 16 == 0):
         return wide_gemm(x, rows, out_dtype, out)
     rows_t = weight.rows_t if isinstance(weight, Weight) else rows.t()
     global _library_calls

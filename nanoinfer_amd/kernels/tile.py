@@ -517,28 +517,39 @@ WIDE_ROWS_LAST = 2048
 WIDE_FLOPS = 2e9            # operations of the smallest plain product that was measured ([2048, 1024] at 600 rows: 10.8 us in the library, 9.5 here)
 
 
-def wide_wins(x: torch.Tensor, rows: torch.Tensor, gated: bool = False) -> bool:
+# How much longer than the library's product a plain one on each tile may be estimated to take, by where its results go: few tiles are estimated too
+# high, the larger ones less so, the largest too low.  Of 289 products (17 matrices, 520 to 2,048 rows) those taken with 15 % for all but the largest
+# were up to 13 % behind: [5120, 3072] at 1,024 rows 40.5 : 42.3 us, to float32 39.5 : 44.7, [8192, 4096] at 700 49.4 : 53.7, at 2,048 92.0 : 96.4 on the largest,
+# whose float32 results are ahead of the library's ([8192, 2048] at 2,048 64.2 : 58.0).  With these [2048, 8192] at 1,400 is, by 4 %.  Onto the stream none was:
+# a kernel less behind it.
+WIDE_SLACK = {"bfloat16": (0.9, 1.08, 1.08, 1.15), "float32": (1.0, 1.0, 1.0, 1.15), "stream": (1.0, 1.15, 1.15, 1.15)}
+
+
+def wide_wins(x: torch.Tensor, rows: torch.Tensor, gated: bool = False, to: str = "bfloat16") -> bool:
     """Whether the bfloat16 product ``x . rows^T`` goes to :func:`wide_gemm`: where it is estimated to take no longer than the library's
     product (with the SwiGLU kernel behind it): 5 to 8 us, 1 us for 1.33 GFLOP, and where its tiles are few 1.5 us for 1,024 elements of K (plain
-    products of no more tiles than units with 15 % more, by which few tiles are estimated too high; not the largest tile).  Measured in recorded launches, each with another W (us, library : this; cards differ by 10 %):
+    products of no more tiles than units by ``WIDE_SLACK``; past 8,192 elements of K, where the library is faster than that, 3 % at most).  ``to``: where
+    the results go, a key of that table.  Measured in recorded launches, each with another W (us, library : this; cards differ by 10 %):
 
     SwiGLU in the epilogue, from 257 rows: [16384, 2048] at 400 / 512 / 900 / 1,024 / 1,300 / 1,600 / 1,999 / 3,000 / 4,096 rows 41 : 34,
     44 : 36, 64 : 58, 68 : 58, 99 : 90, 113 : 102, 121 : 111, 183 : 157, 239 : 211 (the tiled product 37 at 400 and 39 at 512 rows),
     [16384, 3072] at 512 / 1,024 / 1,999 62 : 52, 95 : 79, 172 : 152, [28672, 4096] at 512 / 1,999 108 : 102, 391 : 373, [4096, 2048] at
     600 / 1,024 / 1,999 25 : 17, 29 : 21, 42 : 31.  Not where the tiles just outnumber the units ([16384, 2048] at 600 rows 49 : 56,
-    [16384, 3072] 67 : 74), and to 512 rows only on its larger tiles (a small matrix, [4096, 2048] at 512 rows, takes 19 in the smallest, 16 by
+    [16384, 3072] 67 : 74), and to 512 rows only on its larger tiles, the one of 128 x 256 with matrices that the tiled product would take
+    ([16384, 3072] at 300 / 350 rows 45 : 48, 48 : 51; a small matrix, [4096, 2048] at 512 rows, takes 19 in the smallest, 16 by
     the tiled product); to 256 rows the tiled product is as fast or faster (26 : 28).
 
     Plain, from 513 rows (the tiled product's end) to 2,048: [2048, 8192] at 1,024 / 1,600 / 2,045 50 : 58, 66 : 58, 70 : 63, [2048, 2048] at
     800 / 1,300 / 1,600 / 2,045 15.4 : 14.8, 20.6 : 15.9, 20.7 : 17.1, 21.6 : 18.4, [3072, 2048] at 1,024 / 1,300 / 2,045 20.6 : 16.3,
     24.1 : 24.3, 28.4 : 26.4, [4096, 4096] at 1,024 / 2,045 40.7 : 35.5, 59.1 : 56.1; the results in float32, [2048, 2048] at 2,045 23.4 : 20.6,
     [3072, 2048] 28.7 : 29.0, [4096, 2048] 37.6 : 33.5, [8192, 2048] 64.2 : 57.5.  More tiles than units end in a round that few of them fill, where the
-    library takes other tiles ([6144, 2048] at 2,045 48 : 55, [8192, 2048] at 1,600 49 : 56); with more rows its larger ones win ([3072, 2048] at
+    library takes other tiles ([6144, 2048] at 2,045 48 : 55, [8192, 2048] at 1,600 49 : 56), and rows of 14,336 elements are slower here
+    ([4096, 14336] at 900 / 1,300 / 1,400 116 : 122, 154 : 170, 152 : 174, but at 1,700 194 : 177); with more rows its larger ones win ([3072, 2048] at
     3,000 37 : 45, [2048, 8192] at 2,500 83 : 87)."""
-    return (x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous() and x.data_ptr() % 16 == 0 and wide_takes(*x.shape, rows, gated))
+    return (x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous() and x.data_ptr() % 16 == 0 and wide_takes(*x.shape, rows, gated, to))
 
 
-def wide_takes(M: int, K: int, rows: torch.Tensor, gated: bool = False) -> bool:
+def wide_takes(M: int, K: int, rows: torch.Tensor, gated: bool = False, to: str = "bfloat16") -> bool:
     """The same of M aligned rows of K elements."""
     if rows.dtype != torch.bfloat16 or rows.dim() != 2:
         return False
@@ -549,16 +560,20 @@ def wide_takes(M: int, K: int, rows: torch.Tensor, gated: bool = False) -> bool:
     tile, cost = wide_plan(M, N, K, gated)
     library = M * N * K / 0.665e9
     if gated:
-        return (M >= WIDE_ROWS or tile < 3) and cost <= 12.0 + library + 3.0 * M * N / 4.6e6
+        return (M >= WIDE_ROWS or tile in (0, 2) or (tile == 1 and N * K <= 1 << 25)) and cost <= 12.0 + library + 3.0 * M * N / 4.6e6
     bm, bn = WIDE_TILES[tile][:2]
-    slack = 1.15 if tile and -(-M // bm) * -(-N // bn) <= COMPUTE_UNITS else 1.0
+    slack = WIDE_SLACK[to][tile]
+    if -(-M // bm) * -(-N // bn) > COMPUTE_UNITS:
+        slack = min(slack, 1.0)
+    if K > 8192:
+        slack = min(slack, 1.03)
     return 2.0 * M * N * K >= WIDE_FLOPS and cost <= slack * (5.0 + library + 1.5e-3 * K)
 
 
 def wide_stream_ok(M: int, K: int, dtype: torch.dtype, weight) -> bool:
     """Whether the product of M rows of K elements onto the residual stream goes to :func:`wide_stream`."""
     rows = getattr(weight, "rows", None)
-    return rows is not None and M >= WIDE_ROWS and dtype == torch.bfloat16 and rows.shape[0] % 64 == 0 and wide_takes(M, K, rows)
+    return rows is not None and M >= WIDE_ROWS and dtype == torch.bfloat16 and rows.shape[0] % 64 == 0 and wide_takes(M, K, rows, to="stream")
 
 
 def wide_leaves_ok(M: int, K: int, dtype: torch.dtype, weight) -> bool:
