@@ -329,7 +329,8 @@ class Attention(Part):
         """Whether ``forward`` can take ``residual=h`` for T tokens: its output then goes into the residual
         stream without a kernel for the sum (added by the product itself, or left as float32 addends)."""
         if T > K.SKINNY_MAX_ROWS:
-            return K.FUSE_NORMS and type(self).output is Attention.output and K.wide_stream_ok(T, self.H * self.hd, self.rt.dtype, self.w_o)
+            return (K.FUSE_NORMS and type(self).forward is Attention.forward and type(self).output is Attention.output
+                    and K.wide_stream_ok(T, self.H * self.hd, self.rt.dtype, self.w_o))
         return K.FUSE_NORMS and K.residual_epilogue_ok(T, self.H * self.hd, self.rt.dtype, self.w_o)
 
     def carries_addends(self, T: int, addends: int) -> bool:

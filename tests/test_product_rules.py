@@ -128,3 +128,21 @@ def test_where_stacked_products_of_65_to_512_rows_rotate_and_store(N, Kd, hd, wh
         assert M in inside or K.qkv_shares_ok(x, Stored(), hd, hd) == (M in shares), M
     assert not K.qkv_shares_ok(x, Stored(), 36, 36) and not K.qkv_shares_ok(x, Stored.rows, hd, hd)
     assert K.qkv_shares_ok(torch.empty(300, Kd), Stored(), hd, hd)
+
+
+@pytest.mark.parametrize("stage", ["forward", "output"])
+def test_a_replaced_stage_of_attention_is_given_no_stream_of_many_rows(stage):
+    """Past the skinny products' rows a class that has its own ``forward`` or ``output``, which may know of no ``residual``, is run without one."""
+    from types import SimpleNamespace
+
+    from nanoinfer_amd.parts.standard import Attention
+
+    def part(cls):
+        p = cls.__new__(cls)
+        p.H, p.hd, p.rt = 32, 64, SimpleNamespace(dtype=torch.bfloat16)
+        p.w_o = SimpleNamespace(tiles=None, rows=torch.empty(2048, 2048, dtype=torch.bfloat16, device="meta"))
+        return p
+
+    assert part(Attention).adds_residual(1999) and part(Attention).leaves_scaled(1999)
+    own = part(type("Own", (Attention,), {stage: lambda self, x, ctx, cache: x}))
+    assert not own.adds_residual(1999) and not own.leaves_scaled(1999)
