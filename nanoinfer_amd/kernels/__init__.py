@@ -1300,29 +1300,27 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
     (rocBLAS/hipBLASLt; its reduced-precision matrix modes for float32 are switched off at import).
     ``out_dtype`` float32 keeps the float32 accumulators of a bfloat16 product.  ``x`` may be a
     :class:`NormedInput` where :func:`norm_prologue_ok` holds.  With ``residual`` (the float32
-    residual stream, where :func:`residual_epilogue_ok` holds) the product is added into it and
+    residual stream, where :func:`residual_epilogue_ok` holds, or :func:`wide_stream_ok` of many rows) the product is added into it and
     nothing is returned, or (17 to 64 rows on a matrix of few tiles, :func:`skinny_ksplit`) it is
     returned as float32 addends [S, M, N] that the next norm adds to the stream.  ``pending``: addends
     that ``residual`` has not received yet and that the product brings in with it (where
     :func:`residual_takes_addends` holds).  ``out``: where a plain product is to be written ([M, N] of the
-    output type) instead of a new tensor.  ``leave`` (with ``residual``, where :func:`leaves_scaled_ok`
-    holds; ignored elsewhere): the norm that stands behind the stream; the product then runs whole and
-    returns a :class:`ScaledInput` for that norm.  ``x`` may itself be a :class:`ScaledInput` where
+    output type) instead of a new tensor.  ``leave`` (with ``residual``, where :func:`leaves_scaled_ok`, of many rows
+    :func:`wide_leaves_ok`, holds; ignored elsewhere): the norm that stands behind the stream; the product then runs whole and
+    returns a :class:`ScaledInput` for that norm.  ``x`` may itself be a :class:`ScaledInput` of few rows where
     :func:`takes_scaled_ok` holds, or :class:`HalvedRows`.  ``addends`` (ignored with ``out``): a product of many rows may come back as float32
     addends [S, M, N] (its K range cut into S shares), for a norm that adds them to the stream itself."""
     rows, _ = _rows_and_tiles(weight)
     if out is not None and (isinstance(x, (NormedInput, ScaledInput)) or residual is not None):
         raise KernelError("out= goes with a plain product")
     if residual is not None and x.shape[0] > SKINNY_MAX_ROWS:
-        if not isinstance(x, torch.Tensor) or pending is not None or not wide_stream_ok(*x.shape, x.dtype, weight):
+        if not isinstance(x, torch.Tensor) or x.dim() != 2 or pending is not None or not wide_stream_ok(*x.shape, x.dtype, weight):
             raise KernelError("the residual epilogue does not take this product")
         if not _plain(x):
             x = x.clone(memory_format=torch.contiguous_format)
-        if leave is None or leave.weight.data_ptr() % 16:      # (the norm behind it then runs as a kernel of its own)
-            wide_stream(x, rows, residual)
+        if leave is None or leave.weight.data_ptr() % 16 or not wide_leaves_ok(*x.shape, x.dtype, weight):
+            wide_stream(x, rows, residual)                     # (the norm behind it then runs as a kernel of its own)
             return None
-        if not wide_leaves_ok(*x.shape, x.dtype, weight):
-            raise KernelError("this product cannot leave a norm's input")
         return ScaledInput(*wide_stream(x, rows, residual, leave.weight), leave)
     if isinstance(x, ScaledInput):
         if residual is not None or not takes_scaled_ok(x.shape[0], x.shape[1], x.dtype, weight):

@@ -146,3 +146,14 @@ def test_a_replaced_stage_of_attention_is_given_no_stream_of_many_rows(stage):
     assert part(Attention).adds_residual(1999) and part(Attention).leaves_scaled(1999)
     own = part(type("Own", (Attention,), {stage: lambda self, x, ctx, cache: x}))
     assert not own.adds_residual(1999) and not own.leaves_scaled(1999)
+
+
+def test_a_norm_whose_input_a_product_cannot_leave_is_ignored(monkeypatch):
+    """As with few rows: 4,160 columns are 65 parts of sums of squares, more than the product behind takes; the sum onto the stream goes out alone."""
+    went = []
+    monkeypatch.setattr(K, "wide_stream", lambda *a, **k: went.append((len(a), k)) or (None, None))
+    x, w, h = torch.empty(1200, 2048, dtype=torch.bfloat16), K.Weight(torch.empty(4160, 2048, dtype=torch.bfloat16), tiled=False), torch.empty(1200, 4160)
+    assert K.linear(x, w, residual=h, leave=K.NormSpec(torch.empty(4160), 1e-5)) is None and went == [(3, {})]
+    for bad in (x.view(1, 1200, 2048).expand(65, 1200, 2048), x[:, :64]):
+        with pytest.raises(K.KernelError):
+            K.linear(bad, w, residual=h)
