@@ -215,10 +215,22 @@ def rope_kv_write_shares(parts: torch.Tensor, positions: torch.Tensor, cos: Opti
         if not (kpool.dim() == 4 and kpool.shape[1] == KVH and kpool.shape[3] == hd):
             raise KernelError(f"pool must be [pages, {KVH}, page_size, {hd}], is {tuple(kpool.shape)}")
         page_size = kpool.shape[2]
+    if _off_vectors(kpool, vpool, cos, sin):
+        rows = parts[0].clone()
+        for p in range(1, S):
+            rows += parts[p]
+        rows = rows.to(dtype)
+        rope_kv_write(rows, positions, cos, sin, slot_mapping, kpool, vpool, H, KVH, hd)
+        return rows[:, :H * hd].contiguous()
     q = torch.empty(T, H * hd, dtype=dtype, device=parts.device)
     _check(core().ni_rope_kv_write_shares(_ptr(parts), S, _ptr(q), _ptr(positions), _ptr(cos), _ptr(sin), _ptr(slot_mapping), _ptr(kpool), _ptr(vpool),
                                           T, H, KVH, hd, rot, page_size, dtype_code(dtype), _stream()), "rope_kv_write_shares")
     return q
+
+
+def _off_vectors(*tensors: Optional[torch.Tensor]) -> bool:
+    """Whether any of them starts off sixteen bytes, as views into a buffer of a program's own may: kernels with wide accesses do not take it."""
+    return any(t is not None and t.data_ptr() % 16 for t in tensors)
 
 
 def rope_shares_ok(hd: int, rot: int) -> bool:

@@ -10,7 +10,7 @@ from typing import Optional, Tuple
 import torch
 
 from ..csrc import build as _build
-from . import GATED_ACTIVATIONS, SKINNY_MAX_ROWS, KernelError, _check, _gpu, _load, _ptr, _stream, add_rmsnorm, core, dtype_code, rope_shares_ok
+from . import GATED_ACTIVATIONS, SKINNY_MAX_ROWS, KernelError, _check, _gpu, _load, _off_vectors, _ptr, _stream, add_rmsnorm, core, dtype_code, rope_kv_write, rope_shares_ok
 
 COMPUTE_UNITS = 256
 
@@ -726,6 +726,7 @@ def qkv_rope(x, weight, positions: torch.Tensor, cos: torch.Tensor, sin: torch.T
     plain values go into the pools ([pages, KVH, page_size, hd]) at ``slot_mapping`` (below zero, or absent: not stored).  ``plan`` as
     :func:`qkv_rope_plan` gives it.  On the stored matrix ``x`` may be a :class:`ScaledInput`."""
     M, K = x.shape
+    given = x
     on_tiles, tile = plan
     rows, tiles = weight.rows, weight.tiles
     x, ss, parts, eps = _row_norm(x, M, K)
@@ -739,7 +740,7 @@ def qkv_rope(x, weight, positions: torch.Tensor, cos: torch.Tensor, sin: torch.T
     N = rows.shape[0]
     matrix = tiles if on_tiles else rows
     if (hd % (32 if on_tiles else 64) or 2 * cos.shape[1] != hd or K == 0 or K % 64 or M * K >= 1 << 30 or (N + 15) * K >= 1 << 30 or matrix is None
-            or (on_tiles and tiles.numel() != N * K) or (x.data_ptr() | matrix.data_ptr() | cos.data_ptr() | sin.data_ptr()) % 16):
+            or (on_tiles and tiles.numel() != N * K) or (x.data_ptr() | matrix.data_ptr()) % 16):
         raise KernelError(f"qkv_rope does not take [{M}, {K}] x [{N}, {K}] with heads of {hd}, of which {2 * cos.shape[1]} are rotated")
     page_size = 1
     if slot_mapping is not None:
@@ -748,9 +749,17 @@ def qkv_rope(x, weight, positions: torch.Tensor, cos: torch.Tensor, sin: torch.T
             raise KernelError("a slot mapping needs both pools")
         _gpu(kpool, "kpool", torch.bfloat16)
         _gpu(vpool, "vpool", torch.bfloat16, kpool.shape)
-        if not (kpool.dim() == 4 and kpool.shape[1] == KVH and kpool.shape[3] == hd) or (kpool.data_ptr() | vpool.data_ptr()) % 16:
-            raise KernelError(f"pool must be [pages, {KVH}, page_size, {hd}] at a multiple of 16 bytes, is {tuple(kpool.shape)}")
+        if not (kpool.dim() == 4 and kpool.shape[1] == KVH and kpool.shape[3] == hd):
+            raise KernelError(f"pool must be [pages, {KVH}, page_size, {hd}], is {tuple(kpool.shape)}")
         page_size = kpool.shape[2]
+    if _off_vectors(cos, sin):
+        cos, sin = cos.clone(), sin.clone()
+    if slot_mapping is not None and _off_vectors(kpool, vpool):
+        # keys and values to pages of one token, and from there as the kernel behind a product stores them
+        whole = [torch.empty(M, KVH, 1, hd, dtype=torch.bfloat16, device=given.device) for _ in range(2)]
+        q = qkv_rope(given, weight, positions, cos, sin, torch.arange(M, dtype=torch.int32, device=given.device), *whole, H, KVH, hd, plan)
+        rope_kv_write(torch.cat([q, *(t.view(M, -1) for t in whole)], dim=1), positions, None, None, slot_mapping, kpool, vpool, H, KVH, hd)
+        return q
     q = torch.empty(M, H * hd, dtype=torch.bfloat16, device=x.device)
     launch, norm = (tile_lib().ni_tiled_qkv_rope, ()) if on_tiles else (wide_lib().ni_wide_qkv_rope, (_ptr(ss), parts, eps))
     _check(launch(_ptr(x), _ptr(matrix), _ptr(q), _ptr(positions), _ptr(cos), _ptr(sin), _ptr(slot_mapping), _ptr(kpool), _ptr(vpool), M, K, H, KVH, hd,

@@ -123,3 +123,44 @@ def test_as_many_shares_as_plans_have(K, dtype, S):
     K.rope_kv_write(whole, at, cos, sin, at, *want, H, KVH, hd)
     for got, true in ((q, whole[:, :H * hd].contiguous()), *zip(pools, want)):
         assert torch.equal(got, true.to(dtype))
+
+
+def off_vectors(t):
+    """The same numbers four bytes behind a multiple of sixteen, as a view into a program's own buffer may stand."""
+    by = 4 // t.element_size()
+    flat = torch.zeros(t.numel() + by, dtype=t.dtype, device=t.device)
+    flat[by:] = t.reshape(-1)
+    return flat[by:].view(t.shape)
+
+
+@pytest.mark.parametrize("pools_off,tables_off", [(True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("kind", ["tiled", "stored", "shares", "shares float32"])
+def test_pools_and_tables_off_sixteen_bytes(K, kind, pools_off, tables_off):
+    """They were taken by the rotating kernel behind a product, and are by what stands in its place; queries are the same, keys and values up to the one
+    rounding more of a kernel behind rounded rows."""
+    M, Kd, H, KVH, hd = 300, 256, 3, 1, 64
+    dtype = torch.float32 if "float32" in kind else torch.bfloat16
+    g = torch.Generator().manual_seed(3)
+    x, w = torch.randn(M, Kd, generator=g).bfloat16().cuda(), torch.randn((H + 2 * KVH) * hd, Kd, generator=g).bfloat16().cuda()
+    parts, angle = torch.randn(3, M, (H + 2 * KVH) * hd, generator=g).cuda(), torch.rand(M, hd // 2, generator=g) * 6.28
+    tables, at = (angle.cos().cuda(), angle.sin().cuda()), torch.arange(M, dtype=torch.int32).cuda()
+    at[5] = -1
+    made = []
+    for off in (False, True):
+        pools = [torch.full((20, KVH, 16, hd), 7.0, device="cuda", dtype=dtype) for _ in range(2)]
+        cos, sin = (off_vectors(t) for t in tables) if off and tables_off else tables
+        pools = [off_vectors(p) for p in pools] if off and pools_off else pools
+        positions = torch.arange(M, dtype=torch.int32).cuda()
+        if kind.startswith("shares"):
+            q = K.rope_kv_write_shares(parts, positions, cos, sin, at, *pools, H, KVH, hd, dtype)
+        else:
+            q = K.qkv_rope(x, K.Weight(w), positions, cos, sin, at, *pools, H, KVH, hd, (kind == "tiled", 2 if kind == "tiled" else 3))
+        made.append((q, *pools))
+    for one, other in zip(*made):
+        if kind.startswith("shares"):
+            # a c - b s with either product inside the sum's rounding: apart by at most 2^-23 (|a c| + |b s|) <= 2^-22 of the row's largest, as the rotation
+            # leaves a pair's length; in bfloat16 the rounded row is rotated (2^-8 of it), and the result rounded once more
+            off = 2.0 ** -22 if dtype == torch.float32 else 2.0 ** -6
+            assert bool(((one.float() - other.float()).abs() <= off * one.float().abs().amax(-1, keepdim=True)).all())
+        else:
+            assert torch.equal(one, other)
