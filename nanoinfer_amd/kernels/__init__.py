@@ -1328,6 +1328,10 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
     if residual is not None and x.shape[0] > SKINNY_MAX_ROWS:
         if not isinstance(x, torch.Tensor) or x.dim() != 2 or pending is not None or not wide_stream_ok(*x.shape, x.dtype, weight):
             raise KernelError("the residual epilogue does not take this product")
+        if residual.data_ptr() % 16:                           # (no whole vectors: the sum is made behind the product)
+            _gpu(residual, "residual", torch.float32, (x.shape[0], rows.shape[0]))
+            residual += linear(x, weight, torch.float32)
+            return None
         if not _plain(x):
             x = x.clone(memory_format=torch.contiguous_format)
         if leave is None or leave.weight.data_ptr() % 16 or not wide_leaves_ok(*x.shape, x.dtype, weight):

@@ -121,3 +121,17 @@ def test_a_prompt_with_its_norms_in_halves(K, monkeypatch):
         assert left[:2 * layers] == [4] * (2 * layers - 1) + [3]
         runner.release(0)
         assert_close(got, plain_logits(folder, tokens, "bfloat16")[at], "bfloat16", f"graphs {graphs}")
+
+
+def test_a_stream_that_is_not_aligned(K):
+    """Off sixteen bytes there are no whole vectors to add to: the product goes out alone, and nothing is left for the norm."""
+    M, N, Kd = 1999, 2048, 2048
+    x, w = draw(M, Kd, seed=1).bfloat16().cuda(), K.Weight(draw(N, Kd, seed=2).bfloat16().cuda())
+    h, a = torch.zeros(M * N + 1, device="cuda")[1:].view(M, N), torch.zeros(M, N, device="cuda")
+    for t in (h, a):
+        t.copy_(draw(M, N, seed=3))
+    assert K.linear(x, w, residual=h, leave=K.NormSpec(torch.ones(N, device="cuda"), 1e-5)) is None
+    K.linear(x, w, residual=a)
+    assert torch.equal(h, a)
+    with pytest.raises(K.KernelError):
+        K.linear(x, w, residual=h.bfloat16())
