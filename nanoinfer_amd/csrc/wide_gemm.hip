@@ -163,7 +163,7 @@ __global__ __launch_bounds__(WM * WN * WAVE, 2) void wide_gemm_kernel(const bf16
     // loads that may still be on their way when the next stage is read: all that were asked for after its last one
     constexpr int WAITX = CW + (DX - 2) * ALL, WAITW = (DW - 2) * ALL, WAIT = WAITX < WAITW ? WAITX : WAITW;
     constexpr int FIRST = (ALL + 1) / 2;
-    // (inside a half of a stage the compiler may order loads as it likes)
+    // (inside a half of a stage the compiler may order loads as it likes, and before the first stage inside a batch)
     static_assert(DX == DW || FIRST == CX, "batches are counted whole, or x in the first half of a stage and W in the second");
     auto stage = [&](auto I, int s) {
         constexpr int i = decltype(I)::value;
@@ -185,6 +185,7 @@ __global__ __launch_bounds__(WM * WN * WAVE, 2) void wide_gemm_kernel(const bf16
         constexpr int b = decltype(B)::value;                  // stages before the first
         constexpr int last = b == 1 ? FIRST : ALL;
         if constexpr (b <= DX) fetch(Index<DX * DW - b>{}, -b, Index<0>{}, Index<(last < CX ? last : CX)>{});
+        if constexpr (DX != DW) __builtin_amdgcn_sched_barrier(0);     // (x and W of different stages: the wait below counts x's first)
         if constexpr (b <= DW) fetch(Index<DX * DW - b>{}, -b, Index<CX>{}, Index<(last < CX ? CX : last)>{});
         __builtin_amdgcn_sched_barrier(0);
     };
