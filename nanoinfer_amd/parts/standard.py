@@ -329,7 +329,7 @@ class Attention(Part):
         """Whether ``forward`` can take ``residual=h`` for T tokens: its output then goes into the residual
         stream without a kernel for the sum (added by the product itself, or left as float32 addends)."""
         if T > K.SKINNY_MAX_ROWS:
-            return (K.FUSE_NORMS and type(self).forward is Attention.forward and type(self).output is Attention.output
+            return (self.rt.dtype == torch.bfloat16 and K.FUSE_NORMS and type(self).forward is Attention.forward and type(self).output is Attention.output
                     and K.wide_stream_ok(T, self.H * self.hd, self.rt.dtype, self.w_o))
         return K.FUSE_NORMS and K.residual_epilogue_ok(T, self.H * self.hd, self.rt.dtype, self.w_o)
 
@@ -347,6 +347,8 @@ class Attention(Part):
         (a :class:`nanoinfer_amd.kernels.ScaledInput`): its first product divides by the rows' root mean squares."""
         d = self.w_qkv.shape[1]
         if T > K.SKINNY_MAX_ROWS:
+            if self.rt.dtype != torch.bfloat16:
+                return False
             cls, tables = type(self), self.position.tables()
             return (K.DEFER_NORMS and tables is not None and cls.forward is Attention.forward and cls.project is Attention.project
                     and cls.project_rotate_write is Attention.project_rotate_write and cls.rotate_and_write is Attention.rotate_and_write
@@ -403,7 +405,7 @@ class Attention(Part):
         cos, sin = tables if tables is not None else (None, None)
         slots = cache.slot_mapping if cache.writes else None
         rot = 0 if cos is None else 2 * cos.shape[1]
-        plan = K.qkv_rope_plan(x, self.w_qkv, self.hd, rot)
+        plan = K.qkv_rope_plan(x, self.w_qkv, self.hd, rot) if x.dtype == torch.bfloat16 else None
         if plan is not None:
             return K.qkv_rope(x, self.w_qkv, ctx.positions, cos, sin, slots, cache.kpool, cache.vpool, self.H, self.KVH, self.hd, plan)
         qkv = K.linear(x, self.w_qkv, addends=K.qkv_shares_ok(x, self.w_qkv, self.hd, rot))
@@ -432,7 +434,7 @@ class Attention(Part):
             if nsplit is None:
                 nsplit = K.mfma_splits(tiles.shape[0], self.KVH, self.H // self.KVH, max_keys, self.hd, dtype, T == ctx.max_q_len)
             ws = ctx.workspace(T * self.H * nsplit * (self.hd + 2)) if nsplit > 1 else None
-            halves = leave_runs and K.takes_halved(T, self.H * self.hd, dtype, self.w_o)
+            halves = nsplit > 1 and leave_runs and K.takes_halved(T, self.H * self.hd, dtype, self.w_o)
             return K.mfma_attention(qkv, cache.kpool, cache.vpool, cache.block_table, tiles, out, self.H, self.KVH, self.hd,
                                     self.scale, self.window, nsplit, ws, tile_tokens, groups, halves)
         # single tokens and short portions, token by token
@@ -520,7 +522,7 @@ class SwiGLU(Part):
 
     def adds_residual(self, T: int) -> bool:
         if T > K.SKINNY_MAX_ROWS:
-            return K.FUSE_NORMS and type(self).forward is SwiGLU.forward and K.wide_stream_ok(T, self.intermediate_size, self.rt.dtype, self.w_down)
+            return self.rt.dtype == torch.bfloat16 and K.FUSE_NORMS and type(self).forward is SwiGLU.forward and K.wide_stream_ok(T, self.intermediate_size, self.rt.dtype, self.w_down)
         return K.FUSE_NORMS and K.residual_epilogue_ok(T, self.intermediate_size, self.rt.dtype, self.w_down)
 
     def carries_addends(self, T: int, addends: int) -> bool:
@@ -530,7 +532,7 @@ class SwiGLU(Part):
                 and K.residual_takes_addends(T, self.intermediate_size, self.rt.dtype, self.w_down))
 
     def takes_scaled(self, T: int) -> bool:
-        if T > K.SKINNY_MAX_ROWS and not (type(self).forward is SwiGLU.forward and type(self).hidden is SwiGLU.hidden):
+        if T > K.SKINNY_MAX_ROWS and not (self.rt.dtype == torch.bfloat16 and type(self).forward is SwiGLU.forward and type(self).hidden is SwiGLU.hidden):
             return False
         return K.swiglu_takes_scaled(T, self.w_gate_up.shape[1], self.rt.dtype, self.w_gate_up)
 

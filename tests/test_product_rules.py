@@ -157,3 +157,20 @@ def test_a_norm_whose_input_a_product_cannot_leave_is_ignored(monkeypatch):
     for bad in (x.view(1, 1200, 2048).expand(65, 1200, 2048), x[:, :64]):
         with pytest.raises(K.KernelError):
             K.linear(bad, w, residual=h)
+
+
+def test_float32_steps_ask_nothing_that_is_for_bfloat16(monkeypatch):
+    """A step of more than 64 float32 tokens is launched kernel by kernel by a host that takes longer than they do: what its type decides it asks no rule."""
+    from types import SimpleNamespace
+
+    from nanoinfer_amd.parts.standard import Attention, SwiGLU
+
+    for name in ("wide_stream_ok", "wide_rope_plan", "wide_leaves_ok", "wide_takes", "swiglu_takes_scaled"):
+        monkeypatch.setattr(K, name, lambda *a, **k: pytest.fail("asked"))
+    w = SimpleNamespace(rows=torch.empty(192, 192), shape=(192, 192), tiles=None)
+    for cls in (Attention, SwiGLU):
+        part = cls.__new__(cls)
+        part.rt, part.H, part.hd, part.intermediate_size = SimpleNamespace(dtype=torch.float32), 6, 32, 192
+        part.w_o = part.w_qkv = part.w_gate_up = part.w_down = w
+        part.position = SimpleNamespace(tables=lambda: pytest.fail("asked"))
+        assert not part.adds_residual(100) and not part.takes_scaled(100) and not part.leaves_scaled(100)
