@@ -55,10 +55,20 @@ def test_rotated_and_stored_as_by_the_kernel_behind_the_product(K, plan, M, Kd, 
     q = K.qkv_rope(x, weight, positions, cos, sin, slots, kpool, vpool, H, KVH, hd, plan)
     check(q, kpool, vpool)
     assert torch.equal(K.qkv_rope(x, weight, positions, cos, sin, None, None, None, H, KVH, hd, plan), q)
-    kpool, vpool = (torch.full((pages, KVH, page, hd), 7.0, device="cuda", dtype=torch.bfloat16) for _ in range(2))
-    behind = K.wide_gemm(x, w) if N % 16 == 0 else None          # the product and the kernel behind it, within one rounding more
-    K.rope_kv_write(behind, positions, cos, sin, slots, kpool, vpool, H, KVH, hd)
-    assert bool(((behind[:, :H * hd].double().view(M, H, hd) - want[:, :H]).abs() <= off[:, :H] + 2.0 ** -8 * sums.abs().max()).all())
+    # the product and the kernel behind it: its rows are rounded before they are rotated (2^-9 of a pair's two), both results are rounded (2^-9 each of
+    # no more than the pair's two), and the sums' order may be another
+    pools = [torch.full((pages, KVH, page, hd), 7.0, device="cuda", dtype=torch.bfloat16) for _ in range(2)]
+    behind = K.wide_gemm(x, w)
+    K.rope_kv_write(behind, positions, cos, sin, slots, *pools, H, KVH, hd)
+    pair = heads.abs().sum(2, keepdim=True).expand_as(heads).reshape(M, H + 2 * KVH, hd)
+    apart = 2 * (off - 2.0 ** -8 * want.abs()) + 2.0 ** -7 * pair
+    assert bool(((behind[:, :H * hd].double().view(M, H, hd) - q.double().view(M, H, hd)).abs() <= apart[:, :H]).all())
+    for one, other, first in ((kpool, pools[0], H), (vpool, pools[1], H + KVH)):
+        one, other = (t.permute(0, 2, 1, 3).reshape(-1, KVH, hd) for t in (one, other))
+        assert bool(((one[at].double() - other[at].double()).abs() <= apart[kept, first:first + KVH]).all())
+        untouched = torch.ones(pages * page, dtype=torch.bool, device="cuda")
+        untouched[at] = False
+        assert torch.equal(one[untouched], other[untouched])
 
 
 def test_what_it_does_not_take(K):
