@@ -30,9 +30,10 @@
 // 16-byte pieces in another order for every second row, so that the reads meet no bank twice; W in the order that it is stored in,
 // which the reads take as it is.  A ring holds three or four stages; of the one being multiplied the slots are asked for anew
 // as soon as it is in registers, one barrier a stage.  A stage is three rounds of TM x TN products, low by high, high by
-// low, high by high: what a round needs is read during the round before, so that no product waits for LDS.  Where the registers are
+// low, high by high: what a round needs is read during the round before, so that no product waits for LDS.  (In the stages left over
+// behind the loop, four of 64 in threes, the compiler waits for more loads than it has to.)  Where the registers are
 // there, high by high has two sums that take the stages in turn: shorter sums have fewer roundings, so that a plan of half as many
-// shares is no less exact (512 rows on [2048, 2048] in four shares 1.708e-7, in two with two sums 1.706e-7).  Eight wavefronts, two on a matrix core, where the tile has the work for them:
+// shares is no less exact (512 rows on [2048, 2048] in four shares 1.708e-7, in two with two sums 1.706e-7; kernels/tile.py keeps count).  Eight wavefronts, two on a matrix core, where the tile has the work for them:
 // with four of them and 512 registers each the compiler keeps sums in accumulation registers and copies them (64 x 256: 110 us of
 // 105).  The products are of 16 x 16, which draw less power than 32 x 32: the clock is 5 % higher.  Groups of PAIR_GROUP tiles of x share
 // the tiles of W that they read from an L2; every group begins with another stage, so that what one die asks of memory first the next

@@ -10,8 +10,9 @@
 // read, in a second set of registers; when a wavefront has read a stage it waits until its own loads of the next one have
 // landed, meets the others, and only then are the stage's places asked for anew: one barrier a stage, and loads have DX - 1 stages
 // and more to arrive.  x goes first, W a stage further ahead where LDS has room for it (two stages of each, 256 x 256 tiles: 5 % slower): W
-// comes from memory, x mostly from the caches.  Every ring slot is an array of its own, by which the compiler knows that a read does
-// not wait for loads into the others.
+// comes from memory, x mostly from the caches.  Every ring slot is an array of its own, by which the compiler knows that a read in the loop
+// does not wait for loads into the others.  (In the stages left over behind it, where ways join, it waits for more than it has to: two of 32 stages on
+// 256 x 256 tiles with 2,048 columns.)
 //
 // The rows of x are taken in groups of WIDE_GROUP tiles, whose workgroups run on one die and share the lines of W in its L2; every
 // group begins at another stage of K, so that of two dies that need the same W one asks memory for the half that the other finds in
@@ -26,9 +27,11 @@
 // 1.92 instead of 1.82 GHz.
 //
 // Measured (us, the library's product and the SwiGLU kernel : this; kernels/tile.py has more): [16384, 2048] with SwiGLU at 512 / 1,024 / 1,999 / 4,096 rows
-// 44 : 36, 68 : 58, 121 : 111, 239 : 211; [2048, 8192] at 1,999 70 : 62.  What bounds the large ones is the clock that the chip
-// holds: matrix cores busy 64 % of the time at 1.9 GHz (the library's 65 % at 1.96; with operands of ones, which switch less, 2.3 GHz and
-// 88 us); without its loads the same kernel takes 103.  A prompt of 1,999 tokens of the 1B shape 5,170 -> 4,630 us.
+// 44 : 36, 68 : 58, 121 : 111, 239 : 211; [2048, 8192] at 1,999 70 : 62.  Of [16384, 2048] at 1,999 rows the library's product alone takes 105: what is ahead is the
+// epilogue.  Its loop runs at 1.42 PFLOP/s (kernels/tile.py: 1.509 us for 64 columns with all units at work), the launch at 1.2, and 1.1 to 1.2 inside a prompt: two rounds of
+// one workgroup a unit, whose first loads and stores nothing covers.  In the loop it is the clock: alone, matrix cores busy 64 % of the time at 1.9 GHz
+// (the library's 65 % at 1.96; with operands of ones, which switch less, 2.3 GHz and 88 us; without its loads the same kernel takes 103), in a prompt of 2,048
+// tokens 57 % at 1.99.  A prompt of 1,999 tokens of the 1B shape 5,170 -> 4,630 us.
 #include "lds_load.h"
 #include "rope_store.h"
 #include "row_norm.h"

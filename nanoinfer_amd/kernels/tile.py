@@ -571,7 +571,12 @@ def wide_takes(M: int, K: int, rows: torch.Tensor, gated: bool = False, to: str 
 
 
 def wide_stream_ok(M: int, K: int, dtype: torch.dtype, weight) -> bool:
-    """Whether the product of M rows of K elements onto the residual stream goes to :func:`wide_stream`."""
+    """Whether the product of M rows of K elements onto the residual stream goes to :func:`wide_stream`: by the line of a plain product with more slack,
+    as a norm kernel behind it is not launched, or reads one operand less.  Measured (us, the library's product and a norm : this, its norm left half
+    done : this and a norm): [2048, 2048] at 1,024 / 1,600 / 2,048 rows 21.4 : 19.0 : 21.3, 28.7 : 21.4 : 25.5, 31.7 : 23.7 : 28.4, [2048, 8192] at 1,600 / 2,048 74.4 : 62.0 :
+    65.6, 81.3 : 66.9 : 71.5, [3072, 3072] at 1,024 / 2,048 37.3 : 32.0 : 36.2, 55.3 : 47.5 : 53.8, [4096, 4096] at 800 / 2,048 47.8 : 38.1 : 43.0, 78.0 : 64.5 : 74.1.  The line
+    leaves out some that are ahead ([2048, 2048] at 800 20.2 : 18.9, [2048, 8192] at 1,300 62.8 : 59.4, [3072, 3072] at 800 / 1,300 35.6 : 31.2, 49.3 : 45.1, [4096, 4096] at
+    600 42.4 : 36.2) with those that are not ([2048, 8192] at 600 / 1,024 46.4 : 60.6, 55.8 : 61.0, [3072, 8192] at 1,300 84.9 : 92.8)."""
     rows = getattr(weight, "rows", None)
     return rows is not None and M >= WIDE_ROWS and dtype == torch.bfloat16 and rows.shape[0] % 64 == 0 and wide_takes(M, K, rows, to="stream")
 
