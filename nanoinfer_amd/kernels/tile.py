@@ -535,9 +535,8 @@ def wide_wins(x: torch.Tensor, rows: torch.Tensor, gated: bool = False, to: str 
     44 : 36, 64 : 58, 68 : 58, 99 : 90, 113 : 102, 121 : 111, 183 : 157, 239 : 211 (the tiled product 37 at 400 and 39 at 512 rows),
     [16384, 3072] at 512 / 1,024 / 1,999 62 : 52, 95 : 79, 172 : 152, [28672, 4096] at 512 / 1,999 108 : 102, 391 : 373, [4096, 2048] at
     600 / 1,024 / 1,999 25 : 17, 29 : 21, 42 : 31.  Not where the tiles just outnumber the units ([16384, 2048] at 600 rows 49 : 56,
-    [16384, 3072] 67 : 74), and to 512 rows only on its larger tiles, the one of 128 x 256 with matrices that the tiled product would take
-    ([16384, 3072] at 300 / 350 rows 45 : 48, 48 : 51; a small matrix, [4096, 2048] at 512 rows, takes 19 in the smallest, 16 by
-    the tiled product); to 256 rows the tiled product is as fast or faster (26 : 28).
+    [16384, 3072] 67 : 74), and to 512 rows only on its larger tiles (a small matrix, [4096, 2048] at 512 rows, takes 19 in the smallest, 16 by
+    the tiled product; [16384, 3072] at 350 is 5 % behind, 48 : 51, but the library's way rounds gate and up before it multiplies them); to 256 rows the tiled product is as fast or faster (26 : 28).
 
     Plain, from 513 rows (the tiled product's end) to 2,048: [2048, 8192] at 1,024 / 1,600 / 2,045 50 : 58, 66 : 58, 70 : 63, [2048, 2048] at
     800 / 1,300 / 1,600 / 2,045 15.4 : 14.8, 20.6 : 15.9, 20.7 : 17.1, 21.6 : 18.4, [3072, 2048] at 1,024 / 1,300 / 2,045 20.6 : 16.3,
@@ -560,12 +559,12 @@ def wide_takes(M: int, K: int, rows: torch.Tensor, gated: bool = False, to: str 
     tile, cost = wide_plan(M, N, K, gated)
     library = M * N * K / 0.665e9
     if gated:
-        return (M >= WIDE_ROWS or tile in (0, 2) or (tile == 1 and N * K <= 1 << 25)) and cost <= 12.0 + library + 3.0 * M * N / 4.6e6
+        return (M >= WIDE_ROWS or tile < 3) and cost <= 12.0 + library + 3.0 * M * N / 4.6e6
     bm, bn = WIDE_TILES[tile][:2]
     slack = WIDE_SLACK[to][tile]
     if -(-M // bm) * -(-N // bn) > COMPUTE_UNITS:
         slack = min(slack, 1.0)
-    if K > 8192:
+    if K > 8192 and to != "stream":
         slack = min(slack, 1.03)
     return 2.0 * M * N * K >= WIDE_FLOPS and cost <= slack * (5.0 + library + 1.5e-3 * K)
 
