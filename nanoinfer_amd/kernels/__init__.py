@@ -1480,7 +1480,7 @@ torch.backends.cudnn.allow_tf32 = False
 
 # products of many rows on the matrix cores
 from .tile import (HalvedRows, add_rmsnorm_halved, merge_pair_rows, merge_pair_rows_ok, experts_grouped, experts_grouped_wins, pair_gemm, pair_holds, pair_lines,  # noqa: E402,F401
-                   pair_plan, pair_rows, pair_weight, pair_weight_bytes, pair_wins, qkv_rope, qkv_rope_plan, qkv_shares_ok, rows_of, split_gemm, split_plan, split_wins, takes_halved, tile_lib, tiled_gemm,
+                   pair_plan, pair_rows, pair_weight, pair_weight_bytes, pair_wins, qkv_rope, qkv_rope_plan, qkv_whole, rows_of, split_gemm, split_plan, split_wins, takes_halved, tile_lib, tiled_gemm,
                    tiled_plan, tiled_wins, wide_gemm, wide_leaves_ok, wide_plan, wide_rope_plan, wide_stream, wide_stream_ok, wide_takes, wide_wins, WIDE_ROWS)
 # sums onto the residual stream, routed experts, the gated delta rule, attention with a bias by distance
 from .stream import (BIAS_ATTENTION_MFMA_FROM, DELTA_RUN_FROM, EXPERTS_FEW_ROWS, add_rmsnormed, add_vector,  # noqa: E402,F401

@@ -10,7 +10,7 @@ from typing import Optional, Tuple
 import torch
 
 from ..csrc import build as _build
-from . import GATED_ACTIVATIONS, SKINNY_MAX_ROWS, KernelError, _check, _gpu, _load, _off_vectors, _ptr, _stream, add_rmsnorm, core, dtype_code, rope_kv_write, rope_shares_ok
+from . import GATED_ACTIVATIONS, SKINNY_MAX_ROWS, KernelError, _check, _gpu, _load, _off_vectors, _ptr, _stream, add_rmsnorm, core, dtype_code, rope_kv_write
 
 COMPUTE_UNITS = 256
 
@@ -662,8 +662,9 @@ def _qkv_rope_plan(M: int, N: int, K: int, hd: int, tiled: bool) -> Optional[Tup
             return None
         cost, tile = min((_tiled_cost(M, N, K, t, 1, False), t) for t in range(3))
         t, shares = _tiled_plan(M, N, K, False, False)
-        behind = _tiled_cost(M, N, K, t, 1, False) + ahead if shares == 1 else _tiled_cost(M, N, K, t, shares, True) + ROPE_SHARES_PASS
-        return (True, tile) if cost <= behind else None
+        if shares == 1:                    # (small matrices are estimated a third too high)
+            return (True, tile) if M > 256 and N * K <= 1 << 22 or cost <= _tiled_cost(M, N, K, t, 1, False) + ahead else None
+        return (True, tile) if cost <= _tiled_cost(M, N, K, t, shares, True) + ROPE_SHARES_PASS else None
     if hd % 64 or 2.0 * M * N * K < WIDE_FLOPS:
         return None
     tile, cost = _wide_plan(M, N, K, False)
@@ -699,19 +700,13 @@ def qkv_rope_plan(x, weight, hd: int, rotary_dim: int) -> Optional[Tuple[bool, i
     return _qkv_rope_plan(_whole(M), N, K, hd, getattr(weight, "tiles", None) is not None)
 
 
-def qkv_shares_ok(x, weight, hd: int, rotary_dim: int) -> bool:
-    """Whether the product of many rows with the stacked matrix [q; k; v], where it does not rotate itself, is asked for its shares
-    (:func:`rope_kv_write_shares`): float32 ones, and in bfloat16 those on the re-tiled matrix, past 256 rows only where they would be cut without
-    that.  A plan that cuts just because whatever is behind adds the shares pays where that would run in any case, as a norm does; the rotating kernel
-    takes as long over a whole product.  Measured (us, product and kernel : this): cut without it, [5120, 3072] at 128 / 256 / 384 rows 21.4 : 19.3,
-    25.6 : 22.7, 30.0 : 26.5, [6144, 4096] at 128 / 256 25.6 : 23.8, 34.3 : 31.6, [3072, 2048] at 65 / 192 14.4 : 12.0, 18.1 : 15.3; only with it,
-    [3072, 2048] at 224 / 256 / 320 17.6 : 16.6, 17.6 : 17.5, 17.9 : 17.4, [2560, 2048] at 256 / 320 17.1 : 15.1, 17.3 : 18.0, [2048, 2048] at 384 / 512
-    14.5 : 15.3, 15.0 : 17.9; by the library, [6144, 4096] at 320 / 512 34.2 : 37.6, 40.8 : 46.9."""
-    if not rope_shares_ok(hd, rotary_dim):
-        return False
-    if x.dtype != torch.bfloat16:
-        return True
-    return tiled_wins(x, weight) and (x.shape[0] <= 256 or tiled_plan(x.shape[0], weight.rows.shape[0], x.shape[1])[1] > 1)
+def qkv_whole(x, weight) -> bool:
+    """Whether the product of 65 to 512 bfloat16 rows with the stacked matrix [q; k; v], where it does not rotate itself, is made whole, with float32
+    results for the pass that rounds once (:func:`rope_kv_write_shares` of one share), instead of cut into shares for it: where :func:`tiled_wins`
+    would leave it to the library if nothing behind it added shares.  Cutting pays where that is done in any case or the tiles fill no chip;
+    [6144, 4096] at 320 / 400 / 448 / 512 rows (us, shares : this) 37.1 : 35.6, 44.3 : 39.7, 45.5 : 40.8, 46.8 : 42.6 (rounded rows and the rotating kernel 34.4, 35.7, 37.3,
+    41.0), but cut without that, at 352 / 384, 37.9 : 41.9, 38.9 : 42.0, as [5120, 3072] at 256 / 384 22.7 : 36.4, 26.3 : 28.8."""
+    return x.dtype == torch.bfloat16 and tiled_wins(x, weight, addends=True) and not tiled_wins(x, weight)
 
 
 def wide_rope_plan(M: int, K: int, dtype: torch.dtype, weight, hd: int, rotary_dim: int) -> Optional[Tuple[bool, int]]:

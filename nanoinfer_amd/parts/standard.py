@@ -399,8 +399,8 @@ class Attention(Part):
         return self.rotate_and_write(self.project(x, ctx), ctx, cache)
 
     def _project_many(self, x, ctx, cache: LayerCache) -> torch.Tensor:
-        """The same for many rows: in the product's epilogue where that is compiled and no slower, or in the pass that adds the shares of
-        a product that was cut along K."""
+        """The same for many rows: in the product's epilogue where that is compiled and about as fast, or in the pass that adds the shares of
+        a product that was cut along K, or takes float32 results."""
         tables = self.position.tables()
         cos, sin = tables if tables is not None else (None, None)
         slots = cache.slot_mapping if cache.writes else None
@@ -408,7 +408,11 @@ class Attention(Part):
         plan = K.qkv_rope_plan(x, self.w_qkv, self.hd, rot) if x.dtype == torch.bfloat16 else None
         if plan is not None:
             return K.qkv_rope(x, self.w_qkv, ctx.positions, cos, sin, slots, cache.kpool, cache.vpool, self.H, self.KVH, self.hd, plan)
-        qkv = K.linear(x, self.w_qkv, addends=K.qkv_shares_ok(x, self.w_qkv, self.hd, rot))
+        shares = K.rope_shares_ok(self.hd, rot)
+        if shares and K.qkv_whole(x, self.w_qkv):
+            qkv = K.linear(x, self.w_qkv, out_dtype=torch.float32).unsqueeze(0)
+        else:
+            qkv = K.linear(x, self.w_qkv, addends=shares)
         if qkv.dim() == 3:
             return K.rope_kv_write_shares(qkv, ctx.positions, cos, sin, slots, cache.kpool, cache.vpool, self.H, self.KVH, self.hd, x.dtype)
         return self.rotate_and_write(qkv, ctx, cache)

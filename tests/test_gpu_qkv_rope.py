@@ -174,3 +174,29 @@ def test_pools_and_tables_off_sixteen_bytes(K, kind, pools_off, tables_off):
             assert bool(((one.float() - other.float()).abs() <= off * one.float().abs().amax(-1, keepdim=True)).all())
         else:
             assert torch.equal(one, other)
+
+
+@pytest.mark.parametrize("M,H,KVH,hd,Kd,way", [(320, 32, 8, 128, 4096, "whole"), (352, 32, 8, 128, 4096, "shares"), (257, 16, 8, 64, 2048, "inside"), (256, 16, 8, 64, 2048, "shares")])
+def test_whichever_way_a_layer_takes_rounds_once(K, M, H, KVH, hd, Kd, way):
+    """Past 64 rows a layer's queries, keys and values are sums in float32, rotated, and rounded once, by the epilogue as by the pass behind a product."""
+    from types import SimpleNamespace
+
+    from nanoinfer_amd.parts.standard import Attention
+    g = torch.Generator().manual_seed(M)
+    x, w = torch.randn(M, Kd, generator=g).bfloat16().cuda(), (torch.randn((H + 2 * KVH) * hd, Kd, generator=g) * Kd ** -0.5).bfloat16().cuda()
+    weight, angle = K.Weight(w), torch.rand(M, hd // 2, generator=g) * 6.28
+    cos, sin, at = angle.cos().cuda(), angle.sin().cuda(), torch.arange(M, dtype=torch.int32).cuda()
+    assert ("inside" if K.qkv_rope_plan(x, weight, hd, hd) else "whole" if K.qkv_whole(x, weight) else "shares") == way
+    part = Attention.__new__(Attention)
+    part.H, part.KVH, part.hd, part.w_qkv, part.position = H, KVH, hd, weight, SimpleNamespace(tables=lambda: (cos, sin))
+    pools = [torch.zeros(M // 16 + 1, KVH, 16, hd, device="cuda", dtype=torch.bfloat16) for _ in range(2)]
+    cache = SimpleNamespace(writes=True, slot_mapping=at, kpool=pools[0], vpool=pools[1])
+    q = part._project_many(x, SimpleNamespace(positions=at), cache)
+    sums, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    heads, c, s = sums.view(M, H + 2 * KVH, 2, hd // 2), cos.double()[:, None], sin.double()[:, None]
+    turned = torch.stack((heads[:, :, 0] * c - heads[:, :, 1] * s, heads[:, :, 0] * s + heads[:, :, 1] * c), dim=2)
+    want = torch.cat((turned[:, :H + KVH], heads[:, H + KVH:]), dim=1).reshape(M, H + 2 * KVH, hd)
+    got = torch.cat((q.view(M, H, hd), *(p.permute(0, 2, 1, 3).reshape(-1, KVH, hd)[:M] for p in pools)), dim=1).double()
+    # K roundings of a sum and three of the rotation in float32, one to bfloat16
+    off = (Kd + 12) * 2.0 ** -24 * size.view(M, H + 2 * KVH, 2, hd // 2).sum(2, keepdim=True).expand(-1, -1, 2, -1).reshape(M, H + 2 * KVH, hd) + 2.0 ** -8 * want.abs()
+    assert bool(((got - want).abs() <= off).all())
