@@ -1464,7 +1464,7 @@ def linear_relu2(x, weight) -> torch.Tensor:
         return split_gemm(x, rows, squared=True)
     if tiled_wins(x, weight):
         return tiled_gemm(x, weight, squared=True)
-    if wide_wins(x, rows):
+    if wide_wins(x, rows, to="epilogue"):
         return wide_gemm(x, rows, squared=True)
     return experts_act(linear(x, weight), None, weight.shape[0], "relu2")
 

@@ -77,8 +77,8 @@ def test_where_bfloat16_products_of_many_rows_on_the_stored_matrix_go(N, Kd, gat
 
 
 @pytest.mark.parametrize("N,Kd,to,here,there", [
-    (5120, 3072, "bfloat16", (600, 1200), (1024,)), (5120, 3072, "float32", (600,), (1024,)), (5120, 3072, "stream", (600, 1024, 1200), ()),
-    (8192, 4096, "bfloat16", (1024,), (700, 2048)), (4096, 14336, "bfloat16", (1700, 2048), (900, 1300, 1400)), (4096, 14336, "stream", (900, 1300, 2048), ()),
+    (5120, 3072, "bfloat16", (600, 1200), (1024,)), (5120, 3072, "float32", (600,), (1024,)), (5120, 3072, "epilogue", (600, 1024, 1200), ()),
+    (8192, 4096, "bfloat16", (1024,), (700, 2048)), (4096, 14336, "bfloat16", (1700, 2048), (900, 1300, 1400)), (4096, 14336, "epilogue", (900, 1300, 2048), ()),
     (8192, 2048, "bfloat16", (1024,), (2048,)), (8192, 2048, "float32", (2048,), (700,)), (2048, 2048, "float32", (1300, 2048), ()),
     (16384, 3072, "gated", (350, 400, 512), (300,)), (16384, 2048, "gated", (300, 350, 512), ())])
 def test_no_products_on_the_stored_matrix_where_the_librarys_are_faster(N, Kd, to, here, there):
@@ -173,3 +173,11 @@ def test_float32_steps_ask_nothing_that_is_for_bfloat16(monkeypatch):
         part.w_o = part.w_qkv = part.w_gate_up = part.w_down = w
         part.position = SimpleNamespace(tables=lambda: pytest.fail("asked"))
         assert not part.adds_residual(100) and not part.takes_scaled(100) and not part.leaves_scaled(100)
+
+
+def test_squares_are_of_sums_that_were_not_rounded(monkeypatch):
+    """The product whose epilogue squares goes by the line of those, not by a plain one's, whose rounded results a kernel would square."""
+    monkeypatch.setattr(K, "wide_gemm", lambda x, rows, **k: k)
+    x, w = torch.empty(1024, 3072, dtype=torch.bfloat16), K.Weight(torch.empty(5120, 3072, dtype=torch.bfloat16), tiled=False)
+    assert not K.wide_wins(x, w.rows) and K.wide_wins(x, w.rows, to="epilogue")
+    assert K.linear_relu2(x, w) == {"squared": True}
