@@ -129,8 +129,9 @@ PAIR_SUMS = (1, 2, 2, 2)        # sums that a share's large products are added i
 # at least: the fewer there are the longer each is, and every addition is rounded.  Rms error beside the rows' norms, with that layout's
 # plan : by time alone : with as many sums (1e-7): 700 rows on [2048, 2048] 1.71 : 2.21 : 1.71, 1,300 on
 # [2048, 8192] 3.43 : 4.15 : 2.53, 2,048 on [5120, 3072] 2.22 : 2.64 : 2.22, 600 on [16384, 3072] 2.22 : 2.64 : 2.22, 448 on [6144, 4096] 2.51 : 3.00 :
-# 1.91; of 54 products and 18 with SwiGLU none is above the first by more than 0.2 %.  One plan in 70 is another by this, estimated to be 2 %
-# slower on average and 4 at worst.
+# 1.91; of 54 products and 18 with SwiGLU none is above the first by more than 0.2 %.  One plan in 70 is another by this: with the norm behind it that
+# adds the shares 1 to 5 % slower (us, by time alone : so: 700 rows on [2048, 2048] 31.0 : 31.5, 2,000 on [5120, 3072] 222 : 234, 400 on [6144, 4096] 86.6 : 90.1), where a
+# kernel has to add them up to 24 % (1,000 on [1536, 1536] 18.9 : 23.5, 700 on [2048, 2048] 23.6 : 27.2).
 PAIR_SUM_TILES = ((128, 256, 1, 16.1, 0.447, 0.651, 4.2), (64, 256, 2, 12.4, 0.228, 0.729, 1.18), (128, 128, 2, 11.8, 0.278, 0.745, 1.25),
                   (64, 128, 3, 8.8, 0.115, 0.612, 1.06))
 
