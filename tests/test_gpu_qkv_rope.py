@@ -200,3 +200,36 @@ def test_whichever_way_a_layer_takes_rounds_once(K, M, H, KVH, hd, Kd, way):
     # K roundings of a sum and three of the rotation in float32, one to bfloat16
     off = (Kd + 12) * 2.0 ** -24 * size.view(M, H + 2 * KVH, 2, hd // 2).sum(2, keepdim=True).expand(-1, -1, 2, -1).reshape(M, H + 2 * KVH, hd) + 2.0 ** -8 * want.abs()
     assert bool(((got - want).abs() <= off).all())
+
+
+@pytest.mark.parametrize("M", [257, 320, 400, 512])
+def test_float32_results_of_the_library_recorded(K, M):
+    """The library's product with float32 results and the pass behind it in a graph: every replay, with other work between, is what they give launched."""
+    H, KVH, hd, Kd = 32, 8, 128, 4096
+    g = torch.Generator().manual_seed(M)
+    x, w = torch.randn(M, Kd, generator=g).bfloat16().cuda(), K.Weight((torch.randn((H + 2 * KVH) * hd, Kd, generator=g) * Kd ** -0.5).bfloat16().cuda())
+    angle, at = torch.rand(M, hd // 2, generator=g) * 6.28, torch.arange(M, dtype=torch.int32).cuda()
+    cos, sin = angle.cos().cuda(), angle.sin().cuda()
+    pools = [torch.zeros(M // 16 + 1, KVH, 16, hd, device="cuda", dtype=torch.bfloat16) for _ in range(2)]
+
+    def run():
+        return K.rope_kv_write_shares(K.linear(x, w, torch.float32).unsqueeze(0), at, cos, sin, at, *pools, H, KVH, hd, torch.bfloat16)
+
+    def stored():
+        return [p.permute(0, 2, 1, 3).reshape(-1, KVH, hd)[:M].clone() for p in pools]
+
+    assert K.qkv_whole(x, w)
+    want = [run(), *stored()]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        q = run()
+    for turn in range(4):
+        for t in (q, *pools):
+            t.fill_(float(turn))
+        K.linear(x, w)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for got, true in zip((q, *stored()), want):
+            assert torch.equal(got, true)
