@@ -1,4 +1,5 @@
-// Attention of prompt portions over the paged key/value cache on the matrix cores of gfx950.
+// Attention of prompt portions over the paged key/value cache on the matrix cores of gfx950.  (mfma_attention_kernel; head sizes 64 and 128
+// with pages of sixteen tokens and more take the kernel of attention_prompt.h.)
 // bfloat16 only; compiled once per head size (-DHEAD_DIM=n, a multiple of 16 up to 256; the kernel for
 // single tokens takes the multiples of 32 among them).
 //
@@ -591,53 +592,34 @@ void mfma_attention_kernel(
 #define DEC_WAVES (HEAD_DIM <= 128 ? 4 : 2)
 #if !HEAD_HALF
 
-// (Asked for four wavefronts a SIMD at head size 64, the compiler fits the kernel into 122 registers instead of 148
-// without spilling, and a compute unit holds four workgroups instead of three: 11.5 -> 10.8 us at batch 8.)
-template <bool POW2>
-__global__ __launch_bounds__(DEC_WAVES * WAVE) __attribute__((amdgpu_waves_per_eu(HEAD_DIM <= 64 ? 4 : 2)))
-void mfma_decode_kernel(
-    const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ kpool, const bf16_t* __restrict__ vpool,
-    const int32_t* __restrict__ block_table, int table_stride, const int32_t* __restrict__ seq_of_token,
-    const int32_t* __restrict__ positions, bf16_t* __restrict__ out, float* __restrict__ part_o,
-    float* __restrict__ part_ml, int H, int KVH, int page_size, int page_shift, int window, float scale, int nsplit) {
+// One token's heads `chunk * heads` .. of kv head g (this lane's row: head hh of the group), keys of run `split` of nsplit; `vs` and `sm_ml` are
+// LDS of the whole workgroup, `tbl` has room for TBL_MAX page numbers.
+#define DEC_VROW (HEAD_DIM + VPAD)
+template <bool POW2, int TBL_MAX>
+__device__ __forceinline__ void attend_token(
+    const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ kpool, const bf16_t* __restrict__ vpool, const int32_t* __restrict__ block_table,
+    int table_stride, bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml, int H, int KVH, int page_size, int page_shift,
+    int window, float scale, int nsplit, int split, int t, int seq, int pos, int G, int g, int chunk, int heads, uint16_t (*vs)[KSTEP][DEC_VROW],
+    float (*sm_ml)[16][2], int32_t* tbl) {
     constexpr int HD = HEAD_DIM;
     constexpr int NW = DEC_WAVES;
     constexpr int THREADS = NW * WAVE;
     constexpr int KK = HD / 32;
     constexpr int DT = HD / 16;
-    constexpr int VROW = HD + VPAD;
-    __shared__ __attribute__((aligned(16))) uint16_t vs[NW][KSTEP][VROW];  // per wavefront: V of its step, [key][dim]
-    __shared__ float sm_ml[NW][16][2];
+    constexpr int VROW = DEC_VROW;
     static_assert(KSTEP * VROW * 2 >= 16 * HD * 4, "a wavefront's V tile is reused for its 16 x HD partial output");
-
-    // Uncut key ranges of many tokens: the chip holds the grid two workgroups a compute unit, u and u + half the grid,
-    // which is the same x in the lower and the upper half of y.  In the order of their contexts, longest first, the upper
-    // half takes the tokens from the far end: a long and a short one on every unit (64 requests of 175 to 2,100 tokens in
-    // no order 41 -> 33 us, in order 31.6).
-    constexpr int TBL_MAX = 1024;
-    __shared__ __attribute__((aligned(16))) int32_t tbl[TBL_MAX];
-    int t = (gridDim.z == 1 && gridDim.y > 1 && 2 * blockIdx.y >= gridDim.y) ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
-    if (gridDim.z == 1 && gridDim.y > 1 && gridDim.x > 1 && gridDim.x <= RANKED_TOKENS && gridDim.x * gridDim.y <= RANKED_GROUPS)
-        t = token_by_length(positions, gridDim.x, t, tbl);
-    const int G = H / KVH;
-    const int chunks = (G + 15) / 16;
-    const int g = blockIdx.y / chunks;
-    const int chunk = blockIdx.y % chunks;
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;      // the same in every lane: say so
     const int r = lane % 16, kg = lane / 16;
-    const int hh = chunk * 16 + r;                   // this lane's row: a query head of the group
-    const bool row_ok = hh < G;
+    const int hh = chunk * heads + r;                // this lane's row: a query head of the group
+    const bool row_ok = hh < G && r < heads;
     const int head = g * G + hh;
-
-    const int pos = positions[t];
-    const int seq = seq_of_token[t];
     const int hi = pos + 1;
     const int lo = window > 0 ? max(0, hi - window) : 0;
     const int kbeg = lo / KSTEP * KSTEP;
     const int nsteps_all = (hi - kbeg + KSTEP - 1) / KSTEP;
     const int per_split = (nsteps_all + nsplit - 1) / nsplit;
-    const int s_begin = blockIdx.z * per_split;
+    const int s_begin = split * per_split;
     const int nsteps = max(0, min(nsteps_all, s_begin + per_split) - s_begin);
     const int kfirst = kbeg + s_begin * KSTEP;
     const float scale2 = scale * LOG2E;
@@ -779,7 +761,7 @@ void mfma_decode_kernel(
     for (int dt = 0; dt < DT; ++dt)
         *reinterpret_cast<float4*>(so + r * HD + dt * 16 + kg * 4) = make_float4(o[dt][0], o[dt][1], o[dt][2], o[dt][3]);
     __syncthreads();
-    const int rows = min(16, G - chunk * 16);
+    const int rows = min(heads, G - chunk * heads);
     for (int idx = tid; idx < rows * HD; idx += THREADS) {
         const int row = idx / HD, dim = idx % HD;
         float M = sm_ml[0][row][0];
@@ -792,18 +774,50 @@ void mfma_decode_kernel(
             Lsum += sm_ml[w][row][1] * f;
             O += reinterpret_cast<const float*>(&vs[w][0][0])[row * HD + dim] * f;
         }
-        const int h = g * G + chunk * 16 + row;
+        const int h = g * G + chunk * heads + row;
         if (nsplit == 1) {
             st(out + static_cast<size_t>(t) * H * HD + static_cast<size_t>(h) * HD + dim, O / Lsum);
         } else {
-            const size_t p = (static_cast<size_t>(t) * H + h) * nsplit + blockIdx.z;
+            const size_t p = (static_cast<size_t>(t) * H + h) * nsplit + split;
             part_o[p * HD + dim] = O;
             if (dim == 0) { part_ml[p * 2] = M * LN2; part_ml[p * 2 + 1] = Lsum; }     // the merge kernel works in base e
         }
     }
 }
 
+
+// (Asked for four wavefronts a SIMD at head size 64, the compiler fits the kernel into 122 registers instead of 148
+// without spilling, and a compute unit holds four workgroups instead of three: 11.5 -> 10.8 us at batch 8.)
+template <bool POW2>
+__global__ __launch_bounds__(DEC_WAVES * WAVE) __attribute__((amdgpu_waves_per_eu(HEAD_DIM <= 64 ? 4 : 2)))
+void mfma_decode_kernel(
+    const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ kpool, const bf16_t* __restrict__ vpool,
+    const int32_t* __restrict__ block_table, int table_stride, const int32_t* __restrict__ seq_of_token,
+    const int32_t* __restrict__ positions, bf16_t* __restrict__ out, float* __restrict__ part_o,
+    float* __restrict__ part_ml, int H, int KVH, int page_size, int page_shift, int window, float scale, int nsplit) {
+    __shared__ __attribute__((aligned(16))) uint16_t vs[DEC_WAVES][KSTEP][DEC_VROW];  // per wavefront: V of its step, [key][dim]
+    __shared__ float sm_ml[DEC_WAVES][16][2];
+
+    // Uncut key ranges of many tokens: the chip holds the grid two workgroups a compute unit, u and u + half the grid,
+    // which is the same x in the lower and the upper half of y.  In the order of their contexts, longest first, the upper
+    // half takes the tokens from the far end: a long and a short one on every unit (64 requests of 175 to 2,100 tokens in
+    // no order 41 -> 33 us, in order 31.6).
+    constexpr int TBL_MAX = 1024;
+    __shared__ __attribute__((aligned(16))) int32_t tbl[TBL_MAX];
+    int t = (gridDim.z == 1 && gridDim.y > 1 && 2 * blockIdx.y >= gridDim.y) ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
+    if (gridDim.z == 1 && gridDim.y > 1 && gridDim.x > 1 && gridDim.x <= RANKED_TOKENS && gridDim.x * gridDim.y <= RANKED_GROUPS)
+        t = token_by_length(positions, gridDim.x, t, tbl);
+    const int G = H / KVH;
+    const int chunks = (G + 15) / 16;
+    attend_token<POW2, TBL_MAX>(q, q_stride, kpool, vpool, block_table, table_stride, out, part_o, part_ml, H, KVH, page_size, page_shift, window, scale,
+                                nsplit, blockIdx.z, t, seq_of_token[t], positions[t], G, blockIdx.y / chunks, blockIdx.y % chunks, 16, vs, sm_ml, tbl);
+}
+
 #endif   // !HEAD_HALF
+
+#if HEAD_DIM == 64 || HEAD_DIM == 128
+#include "attention_prompt.h"
+#endif
 
 NI_EXPORT int ni_mfma_attention_head_dim() { return HEAD_DIM; }
 
@@ -844,36 +858,50 @@ NI_EXPORT int ni_mfma_attention(const void* q, int q_stride, const void* kpool, 
     int page_shift = 0;
     while (pow2 && (1 << page_shift) < page_size) ++page_shift;
     const int per_tile = KVH * chunks * nsplit;
-    // As many workgroups as the chip holds at once (asked of the runtime once per kernel), each walking
-    // through its share of the sorted tiles.
-#define MA_LAUNCH(CB_, GROUPS_)                                                                                              \
-    {                                                                                                               \
-        auto kernel = pow2 ? mfma_attention_kernel<CB_, true, GROUPS_> : mfma_attention_kernel<CB_, false, GROUPS_>; \
-        static int slots[2] = {0, 0}, units[2] = {0, 0};                                                            \
-        if (slots[pow2] == 0) {                                                                                     \
-            int dev = 0, cus = 0, per_cu = 0;                                                                       \
-            if (hipGetDevice(&dev) != hipSuccess ||                                                                 \
-                hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||            \
-                hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, GROUPS_ * MA_WAVES * WAVE, 0) != hipSuccess || \
-                cus < 1 || per_cu < 1)                                                                              \
-                return -4;                                                                                          \
-            units[pow2] = cus;                                                                                      \
-            slots[pow2] = cus * per_cu;                                                                             \
-        }                                                                                                           \
-        /* with no more tiles than the chip holds workgroups every tile gets one (the kernel pairs them over the */  \
-        /* compute units); else two rounds pair long tiles with short ones, or more, as few as fit the chip:      */  \
-        /* three rounds leave more workgroups on the chip than four, and their shares differ by less than a tile  */  \
-        int rounds = 1;                                                                                             \
-        if (n_tiles * per_tile > slots[pow2]) {                                                                     \
-            rounds = 2;                                                                                             \
-            while ((n_tiles + rounds - 1) / rounds * per_tile > slots[pow2] && rounds < n_tiles) rounds += 1;       \
-        }                                                                                                           \
-        const int in_x = (n_tiles + rounds - 1) / rounds;                                                           \
-        dim3 grid(in_x, KVH * chunks, nsplit);                                                                      \
-        kernel<<<grid, GROUPS_ * MA_WAVES * WAVE, 0, stream>>>(                                                               \
-            (const bf16_t*)q, q_stride, (const bf16_t*)kpool, (const bf16_t*)vpool, (const int32_t*)block_table,   \
-            table_stride, (const QTile*)tiles, n_tiles, (bf16_t*)out, (float*)part_o, (float*)part_ml, H, KVH,     \
-            page_size, page_shift, hpt_shift, window, scale, nsplit);                                               \
+    // A workgroup for every tile where the chip holds that many (the kernels then pair tiles over the compute units); else two rounds of
+    // workgroups pair long tiles with short ones, or more, as few as fit the chip: three rounds leave more workgroups on the chip than
+    // four, and their shares differ by less than a tile.
+    auto grid_for = [&](const void* kernel, int threads, int& held, dim3& grid) {
+        if (held == 0) {                 // asked of the runtime once per kernel
+            int dev = 0, cus = 0, per_cu = 0;
+            if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+                hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0) != hipSuccess || cus < 1 || per_cu < 1)
+                return false;
+            held = cus * per_cu;
+        }
+        int rounds = 1;
+        if (n_tiles * per_tile > held) {
+            rounds = 2;
+            while ((n_tiles + rounds - 1) / rounds * per_tile > held && rounds < n_tiles) rounds += 1;
+        }
+        grid = dim3((n_tiles + rounds - 1) / rounds, KVH * chunks, nsplit);
+        return true;
+    };
+    dim3 grid;
+#if HEAD_DIM == 64 || HEAD_DIM == 128
+#define MA_LAUNCH_PROMPT(CB_, GROUPS_)                                                                                         \
+    if (pow2 && page_size >= 1024 / HEAD_DIM) { /* (a wavefront's rows of a stage lie in one page) */                        \
+        static int held = 0;                                                                                                   \
+        if (!grid_for(reinterpret_cast<const void*>(prompt_attention_kernel<CB_, GROUPS_>), GROUPS_ * MA_WAVES * WAVE, held, grid)) return -4; \
+        prompt_attention_kernel<CB_, GROUPS_><<<grid, GROUPS_ * MA_WAVES * WAVE, 0, stream>>>(                                 \
+            (const bf16_t*)q, q_stride, (const bf16_t*)kpool, (const bf16_t*)vpool, (const int32_t*)block_table, table_stride, \
+            (const QTile*)tiles, n_tiles, (bf16_t*)out, (float*)part_o, (float*)part_ml, H, KVH, G, chunks, page_shift, hpt_shift, \
+            window, scale, nsplit);                                                                                            \
+        return NI_LAUNCH_RESULT();                                                                                             \
+    }
+#else
+#define MA_LAUNCH_PROMPT(CB_, GROUPS_)
+#endif
+#define MA_LAUNCH(CB_, GROUPS_)                                                                                                \
+    {                                                                                                                          \
+        MA_LAUNCH_PROMPT(CB_, GROUPS_)                                                                                         \
+        static int held[2] = {0, 0};                                                                                           \
+        auto kernel = pow2 ? mfma_attention_kernel<CB_, true, GROUPS_> : mfma_attention_kernel<CB_, false, GROUPS_>;           \
+        if (!grid_for(reinterpret_cast<const void*>(kernel), GROUPS_ * MA_WAVES * WAVE, held[pow2], grid)) return -4;          \
+        kernel<<<grid, GROUPS_ * MA_WAVES * WAVE, 0, stream>>>(                                                                \
+            (const bf16_t*)q, q_stride, (const bf16_t*)kpool, (const bf16_t*)vpool, (const int32_t*)block_table,               \
+            table_stride, (const QTile*)tiles, n_tiles, (bf16_t*)out, (float*)part_o, (float*)part_ml, H, KVH,                 \
+            page_size, page_shift, hpt_shift, window, scale, nsplit);                                                          \
     }
     if (blocks == 1 && groups == 1) MA_LAUNCH(1, 1)
 #if HEAD_DIM <= 128
@@ -883,6 +911,7 @@ NI_EXPORT int ni_mfma_attention(const void* q, int q_stride, const void* kpool, 
     else if (groups == 1) MA_LAUNCH(2, 1)
     else MA_LAUNCH(2, 2)
 #endif
+#undef MA_LAUNCH_PROMPT
 #undef MA_LAUNCH
     return NI_LAUNCH_RESULT();
 }

@@ -1,0 +1,105 @@
+"""The bfloat16 prompt attention of head sizes 64 and 128 against 64 bits of the same rounded numbers: where its stages, sets and pages end,
+single tokens beside portions, scores that rise far above a row's first ones (the tile is made again), key ranges past the page numbers in LDS."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def worst_excess(portions, H, KVH, hd, ps, blocks=1, groups=1, nsplit=1, window=None, seed=0, plant=None):
+    """``portions``: (tokens, keys) of every sequence.  The largest excess over the bound of rounded weights."""
+    from nanoinfer_amd import kernels as K
+    g = torch.Generator().manual_seed(seed)
+    T = sum(n for n, _ in portions)
+    counts = [(keys + ps - 1) // ps for _, keys in portions]
+    order = torch.randperm(sum(counts) + 1, generator=g)
+    kp, vp = (torch.full((len(order), KVH, ps, hd), float("nan"), dtype=torch.bfloat16) for _ in range(2))      # a page of nobody's is no number
+    table = torch.full((len(portions), max(counts)), -1, dtype=torch.int32)
+    starts = [sum(n for n, _ in portions[:s]) for s in range(len(portions))]
+    q = torch.randn(T, H, hd, generator=g).bfloat16()
+    keys_of, at = [], 0
+    for s, (n, keys) in enumerate(portions):
+        k, v = (torch.randn(keys, KVH, hd, generator=g).bfloat16() for _ in range(2))
+        if plant is not None:
+            plant(q[starts[s]:starts[s] + n], k, v)
+        keys_of.append((k, v))
+        mine, at = order[at:at + counts[s]], at + counts[s]
+        table[s, :counts[s]] = mine.int()
+        for pool, t in ((kp, k), (vp, v)):
+            padded = torch.full((counts[s] * ps, KVH, hd), float("nan"), dtype=torch.bfloat16)
+            padded[:keys] = t
+            pool[mine] = padded.view(counts[s], ps, KVH, hd).permute(0, 2, 1, 3)
+    tile = K.mfma_tile_tokens(hd, H // KVH) * blocks
+    tiles = torch.tensor(K.build_q_tiles(starts, [n for n, _ in portions], [c for _, c in portions], tile), dtype=torch.int32).view(-1, 4).cuda()
+    qkv = torch.zeros(T, (H + 2 * KVH) * hd, dtype=torch.bfloat16)
+    qkv[:, :H * hd] = q.reshape(T, H * hd)
+    out = torch.full((T + 1, H * hd), 7.0, device="cuda", dtype=torch.bfloat16)
+    ws = torch.empty(T * H * nsplit * (hd + 2), device="cuda")
+    K.mfma_attention(qkv.cuda(), kp.cuda(), vp.cuda(), table.cuda(), tiles, out[:T], H, KVH, hd, hd ** -0.5, window, nsplit, ws, tile, groups)
+    assert bool((out[T] == 7.0).all())
+    got, worst = out[:T].view(T, H, hd).cpu().double(), -1.0
+    for s, (n, keys) in enumerate(portions):
+        k, v = keys_of[s]
+        for t in sorted({0, 1, n // 2, n - 2, n - 1} & set(range(n))):
+            p = keys - n + t
+            lo = 0 if window is None else max(0, p + 1 - window)
+            for h in range(H):
+                kv = h // (H // KVH)
+                w = torch.softmax((k[lo:p + 1, kv].double() @ q[starts[s] + t, h].double()) * hd ** -0.5, 0)
+                want = w @ v[lo:p + 1, kv].double()
+                here = got[starts[s] + t, h]
+                same = (here == want) | (here.isnan() & want.isnan())        # (infinities, where some are planted)
+                # weights rounded to 8 bits, in the sum as well; the result's rounding; a score's 2^-24 a product
+                biggest = float(v[lo:p + 1, kv].double().nan_to_num(0.0, 0.0, 0.0).abs().max())
+                excess = torch.where(same, torch.full_like(want, -1.0), (here - want).abs() - 2.0 ** -8 * biggest - 2.0 ** -8 * want.abs() - 1e-3)
+                assert not bool(excess.isnan().any())
+                worst = max(worst, float(excess.max()))
+    return worst
+
+
+@pytest.mark.parametrize("hd,H,KVH,blocks,groups", [(64, 4, 1, 1, 1), (64, 8, 2, 2, 1), (64, 4, 1, 2, 2), (64, 5, 1, 1, 2), (128, 3, 1, 1, 1), (128, 4, 2, 1, 2)])
+@pytest.mark.parametrize("portions,ps", [
+    (((1, 1),), 16), (((31, 31), (33, 64), (2, 65)), 16), (((63, 63),), 32), (((64, 64), (65, 65)), 64), (((40, 127), (9, 129)), 16),
+    (((17, 191), (1, 192), (1, 193), (1, 7)), 16), (((130, 500),), 256), (((20, 20480 + 40),), 16)])
+def test_ends_of_stages_and_pages(hd, H, KVH, blocks, groups, portions, ps):
+    assert worst_excess(portions, H, KVH, hd, ps, blocks, groups, seed=hd + blocks) <= 0.0
+
+
+def test_more_pages_than_their_numbers_in_lds():
+    assert worst_excess(((9, 50000),), 4, 1, 64, 16) <= 0.0
+
+
+@pytest.mark.parametrize("hd,H,KVH", [(64, 8, 2), (64, 20, 1), (128, 6, 2)])
+@pytest.mark.parametrize("window,nsplit", [(None, 1), (40, 1), (None, 3)])
+def test_single_tokens_beside_a_portion(hd, H, KVH, window, nsplit):
+    portions = ((70, 70),) + tuple((1, keys) for keys in (1, 31, 32, 33, 128, 129, 700)) + ((2, 300),)
+    assert worst_excess(portions, H, KVH, hd, 16, nsplit=nsplit, window=window, seed=3) <= 0.0
+
+
+@pytest.mark.parametrize("hd,blocks,groups", [(64, 1, 1), (64, 2, 1), (64, 2, 2), (128, 1, 1), (128, 1, 2)])
+@pytest.mark.parametrize("nsplit,rise", [(1, 3.0), (1, 20.0), (2, 20.0)])
+def test_scores_that_rise_late(hd, blocks, groups, nsplit, rise):
+    """Keys behind the first ones that every query likes by e^(rise * sqrt(hd)) more: with 3 the weights stay in range, with 20 none is."""
+    def plant(q, k, v):
+        q[..., 0] = 8.0
+        k[..., 0] = -1.0
+        k[100::37, :, 0] = rise * hd ** 0.5 / 8.0
+    assert worst_excess(((150, 400), (60, 60)), 4, 2, hd, 16, blocks, groups, nsplit, seed=5, plant=plant) <= 0.0
+
+
+@pytest.mark.parametrize("groups", [1, 2])
+def test_values_that_are_not_finite(groups):
+    """An infinity in one dim of one value is in that dim of every row that reads it and nowhere else; a value near the largest number stays one."""
+    def plant(q, k, v):
+        q[..., 0] = 0.0
+        v[40, :, 3] = float("inf")
+        v[70, :, 9] = 2.0 ** 126
+    assert worst_excess(((150, 400),), 4, 2, 64, 16, 1, groups, seed=6, plant=plant) <= 2.0 ** -8 * 2.0 ** 126
+
+
+def test_a_workgroup_goes_from_a_tile_that_is_made_again_to_the_next():
+    def plant(q, k, v):
+        q[..., 0] = 8.0
+        k[:, :, 0] = 0.0
+        k[1000::701, :, 0] = 20.0
+    assert worst_excess(((1530, 1530),), 32, 8, 64, 16, 2, 2, seed=7, plant=plant) <= 0.0
