@@ -28,7 +28,10 @@
 //
 // Measured (us, the library's product and the SwiGLU kernel : this; kernels/tile.py has more): [16384, 2048] with SwiGLU at 512 / 1,024 / 1,999 / 4,096 rows
 // 44 : 36, 68 : 58, 121 : 111, 239 : 211; [2048, 8192] at 1,999 70 : 62.  Of [16384, 2048] at 1,999 rows the library's product alone takes 105: what is ahead is the
-// epilogue.  Its loop runs at 1.42 PFLOP/s (kernels/tile.py: 1.509 us for 64 columns with all units at work), the launch at 1.2, and 1.1 to 1.2 inside a prompt: two rounds of
+// epilogue.  17 to 64 rows on a head of [128256, 2048], where W streams from memory once and 64 rows of x from the caches for every tile: tiles of 64 x 128, two a
+// unit so that one's start and stores go beside the other's stages, 118.8 us at 32 rows and 127.9 at 64 (the library's 125.1 and 133.8; tiles of 64 x 256 in rings of three
+// or four slots 124 and 135); on longer rows 64 x 256 ([128256, 3072] 144.6 and 154.7, the library's 162.1 and 181.4).
+// Its loop runs at 1.42 PFLOP/s (kernels/tile.py: 1.509 us for 64 columns with all units at work), the launch at 1.2, and 1.1 to 1.2 inside a prompt: two rounds of
 // one workgroup a unit, whose first loads and stores nothing covers.  In the loop it is the clock: alone, matrix cores busy 64 % of the time at 1.9 GHz
 // (the library's 65 % at 1.96; with operands of ones, which switch less, 2.3 GHz and 88 us; without its loads the same kernel takes 103), in a prompt of 2,048
 // tokens 57 % at 1.99.  A prompt of 1,999 tokens of the 1B shape 5,170 -> 4,630 us.
@@ -365,6 +368,12 @@ template <int BM, int BN, int WM, int WN, int DX, int DW> static int launch_wide
     const int cols = epi == TG_GATED ? a.N / 2 : a.N, each = epi == TG_GATED ? BN / 2 : BN, mt = (a.M + BM - 1) / BM, nt = (cols + each - 1) / each;
 #define WIDE_LAUNCH(EPI, OUT, NORMED) wide_gemm_kernel<BM, BN, WM, WN, DX, DW, EPI, OUT, NORMED><<<mt * nt, WM * WN * WAVE, 0, stream>>>(a.x, a.w, \
         static_cast<OUT*>(a.out), a.M, a.N, a.K, mt, nt, a.act, a.rope, a.stream, a.norm)
+    if constexpr (BM == 64) {                                 // (few rows of plain products)
+        if (epi != TG_STORE) return static_cast<int>(hipErrorInvalidValue);
+        if (a.f32) WIDE_LAUNCH(TG_STORE, float, false);
+        else WIDE_LAUNCH(TG_STORE, bf16_t, false);
+        return NI_LAUNCH_RESULT();
+    } else {
     if (epi == TG_GATED) {
         if (a.norm.ss) WIDE_LAUNCH(TG_GATED, bf16_t, true);
         else WIDE_LAUNCH(TG_GATED, bf16_t, false);
@@ -376,8 +385,9 @@ template <int BM, int BN, int WM, int WN, int DX, int DW> static int launch_wide
     else if (epi == TG_STREAM) WIDE_LAUNCH(TG_STREAM, float, false);
     else if (a.f32) WIDE_LAUNCH(TG_STORE, float, false);
     else WIDE_LAUNCH(TG_STORE, bf16_t, false);
-#undef WIDE_LAUNCH
     return NI_LAUNCH_RESULT();
+    }
+#undef WIDE_LAUNCH
 }
 
 static int launch_wide_tile(int tile, int epi, const WideArgs& a, void* stream) {
@@ -392,12 +402,14 @@ static int launch_wide_tile(int tile, int epi, const WideArgs& a, void* stream) 
         case 2: return launch_wide<256, 128, 4, 2, 3, 3>(epi, a, s);
         case 3: return launch_wide<128, 128, 4, 2, 5, 5>(epi, a, s);
         case 4: return launch_wide<128, 128, 2, 2, 2, 3>(epi, a, s);
+        case 5: return launch_wide<64, 128, 2, 2, 3, 3>(epi, a, s);
+        case 6: return launch_wide<64, 256, 2, 4, 3, 3>(epi, a, s);
         default: return static_cast<int>(hipErrorInvalidValue);
     }
 }
 
-// tile: 0 = 256 x 256, 1 = 128 x 256, 2 = 256 x 128, 3 = 128 x 128 (rows of x, rows of W), gated also 4 = 128 x 128, two a unit.  f32: float32
-// results.  ss (gated; or null): the rows' sums of squares in `parts` parts, by whose root mean square with eps the rows of x are divided
+// tile: 0 = 256 x 256, 1 = 128 x 256, 2 = 256 x 128, 3 = 128 x 128 (rows of x, rows of W), gated also 4 = 128 x 128, two a unit, plain also
+// 5 = 64 x 128, two a unit, and 6 = 64 x 256.  f32: float32 results.  ss (gated; or null): the rows' sums of squares in `parts` parts, by whose root mean square with eps the rows of x are divided
 NI_EXPORT int ni_wide_gemm(const void* x, const void* w, void* out, int M, int N, int K, int tile, int gated, int f32, int activation, int squared, const void* ss,
                            int parts, float eps, void* stream) {
     if (N % (gated ? 32 : 16) || (gated && (f32 || squared)) || (ss && !gated)) return static_cast<int>(hipErrorInvalidValue);

@@ -4,8 +4,8 @@ on the host, that operand shapes, types and devices are what each kernel and its
 There is no fallback: when a library cannot be built or loaded, or a tensor is not on the GPU,
 the call raises.  Matrix products that none of the kernels here takes or wins are the one thing taken from a library
 (``torch.matmul`` -> rocBLAS/hipBLASLt), as the reference takes its products from cuBLAS
-(src/op/kernels/cuda/matmul_kernel.cu:76-86): from 17 to 64 rows those that :func:`skinny_wins` leaves (float32 rows of more than
-2,048 elements, bfloat16 ones of more than 4,096 past 32 rows, matrices that are not re-tiled, as the vocabulary head); of more
+(src/op/kernels/cuda/matmul_kernel.cu:76-86): from 17 to 64 rows those that :func:`skinny_wins` and :func:`wide_few_wins` leave (float32 rows of more than
+2,048 elements, bfloat16 ones of more than 4,096 past 32 rows, matrices that are not re-tiled, but for a bfloat16 vocabulary head); of more
 rows the bfloat16 ones that :func:`tiled_wins` and :func:`wide_wins` leave and the float32 ones under some 2.2 GFLOP that
 :func:`pair_wins`, :func:`split_wins` and :func:`skinny_deals` leave; and inputs that are not one aligned run of memory.
 """
@@ -1383,6 +1383,9 @@ def linear(x, weight, out_dtype: Optional[torch.dtype] = None, residual: Optiona
         if out is None:
             out = torch.empty(M, rows.shape[0], dtype=out_dtype, device=x.device)
         return skinny_gemm(x, weight, out)
+    if (M <= SKINNY_MAX_ROWS and out_dtype == torch.float32 and x.dtype == torch.bfloat16 and wide_few_wins(M, Kd, rows) and _plain(x)
+            and (out is None or out.data_ptr() % 16 == 0)):
+        return wide_gemm(x, rows, out_dtype, out, tile=wide_few_tile(Kd))
     if out_dtype == torch.float32 and pair_wins(halved, weight):
         return pair_gemm(halved, weight, out, addends=addends)
     if out_dtype == torch.float32 and split_wins(x, rows):
@@ -1481,7 +1484,7 @@ torch.backends.cudnn.allow_tf32 = False
 # products of many rows on the matrix cores
 from .tile import (HalvedRows, add_rmsnorm_halved, merge_pair_rows, merge_pair_rows_ok, experts_grouped, experts_grouped_wins, pair_gemm, pair_holds, pair_lines,  # noqa: E402,F401
                    pair_plan, pair_rows, pair_weight, pair_weight_bytes, pair_wins, qkv_rope, qkv_rope_plan, qkv_whole, rows_of, split_gemm, split_plan, split_wins, takes_halved, tile_lib, tiled_gemm,
-                   tiled_plan, tiled_wins, wide_gemm, wide_leaves_ok, wide_plan, wide_rope_plan, wide_stream, wide_stream_ok, wide_takes, wide_wins, WIDE_ROWS)
+                   tiled_plan, tiled_wins, wide_few_tile, wide_few_wins, wide_gemm, wide_leaves_ok, wide_plan, wide_rope_plan, wide_stream, wide_stream_ok, wide_takes, wide_wins, WIDE_ROWS)
 # sums onto the residual stream, routed experts, the gated delta rule, attention with a bias by distance
 from .stream import (BIAS_ATTENTION_MFMA_FROM, DELTA_RUN_FROM, EXPERTS_FEW_ROWS, add_rmsnormed, add_vector,  # noqa: E402,F401
                      bias_attention, bias_attention_lib, bias_attention_mfma, bias_attention_mfma_rows, bias_attention_rows, bias_attention_runs, bias_attention_bf16_tokens, bias_attention_token_runs, delta_rule, delta_rule_lib, embed_scaled, experts_act, experts_few,

@@ -572,6 +572,24 @@ def wide_takes(M: int, K: int, rows: torch.Tensor, gated: bool = False, to: str 
     return 2.0 * M * N * K >= WIDE_FLOPS and cost <= slack * (5.0 + library + 1.5e-3 * K)
 
 
+WIDE_FEW_COLUMNS = 32000
+
+
+def wide_few_wins(M: int, K: int, rows: torch.Tensor) -> bool:
+    """Whether 17 to 64 plain bfloat16 rows go to :func:`wide_gemm` on a matrix as stored, as the head over the vocabulary is, with float32 results: from as
+    many columns and in the lengths of row measured, where the library streams the matrix no faster (us, library : this, 24 / 32 / 48 / 64 rows: [128256, 2048]
+    123.2 : 117.1, 125.1 : 118.8, 128.8 : 121.6, 133.8 : 127.9; [128256, 3072] 159 : 142, 162 : 145, 171 : 151, 181 : 155; [128256, 4096] 204 : 195, 207 : 198,
+    216 : 197, 219 : 199; [32000, 2048] 22.7 : 22.3, 22.8 : 22.4, 25.3 : 22.8, 24.2 : 23.5)."""
+    N = rows.shape[0]
+    return (16 < M <= 64 and N >= WIDE_FEW_COLUMNS and 2048 <= K <= 4096 and K % 64 == 0 and N % 16 == 0 and N * K < 1 << 30
+            and rows.dtype == torch.bfloat16 and rows.dim() == 2 and rows.is_contiguous() and rows.data_ptr() % 16 == 0)
+
+
+def wide_few_tile(K: int) -> int:
+    """Its tile: two workgroups a unit (64 x 128) on rows of 2,048 elements, one of twice the columns on longer ones."""
+    return 5 if K <= 2048 else 6
+
+
 def wide_stream_ok(M: int, K: int, dtype: torch.dtype, weight) -> bool:
     """Whether the product of M rows of K elements onto the residual stream goes to :func:`wide_stream`: by the line of a plain product with more slack,
     as a norm kernel behind it is not launched, or reads one operand less.  Measured (us, the library's product and a norm : this, its norm left half
