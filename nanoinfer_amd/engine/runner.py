@@ -189,6 +189,25 @@ class _RecordedStep:
     held_bytes: int = 0                  # device memory the recording holds (what the allocator's reserve grew by)
 
 
+_streams: Dict[tuple, "torch.cuda.Stream"] = {}
+
+
+class _Event(torch.cuda.Event):
+    """An event whose ``record()`` finds the current stream by its raw handle: asking torch for the stream's object takes longer than
+    recording (4.4 us together), and a step of single kernels records two or three."""
+
+    def record(self, stream=None) -> None:
+        if stream is None and K._raw_stream is not None:
+            device = K._device()
+            key = device, K._raw_stream(device)
+            stream = _streams.get(key)
+            if stream is None:
+                if len(_streams) >= 256:
+                    _streams.clear()
+                stream = _streams[key] = torch.cuda.current_stream()
+        super().record(stream) if stream is not None else super().record()
+
+
 class _Gpu:
     """What recording a step needs from the device besides the model: kept apart so that the
     runner's host side (tables, books, the order of runs while a step is recorded) can be driven
@@ -204,7 +223,7 @@ class _Gpu:
 
     @staticmethod
     def event():
-        return torch.cuda.Event()
+        return _Event()
 
     @staticmethod
     def argmax(logits: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -472,7 +491,10 @@ class ModelRunner:
         context length, state slot | the draw's table, if ``draw_rows`` (int32 [4 B]) is given]."""
         ps = self.page_size
         i32 = np.int32
+        # neighbouring entries of one token share one array (``few``): five small numpy calls an entry, each about a microsecond, were
+        # 0.2 ms of a step of 31 of them beside a prompt's portion, whose launches keep the GPU waiting for the host
         token_ids, positions, seq_of_token = [], [], []
+        few: List[tuple] = []                                  # (token, position, sequence)
         logit_rows: List[int] = []
         row = 0
         host = ctx._host
@@ -484,9 +506,16 @@ class ModelRunner:
             host["q_len"].append(n)
             host["context_len"].append(done + n)
             host["state_slot"].append(self.cache.state_slot(e.request))
-            token_ids.append(np.asarray(e.tokens, dtype=i32))
-            positions.append(np.arange(done, done + n, dtype=i32))
-            seq_of_token.append(np.full(n, si, dtype=i32))
+            if n == 1:
+                few.append((e.tokens[0], done, si))
+            if few and (n > 1 or si + 1 == len(entries)):
+                for pieces_of, values in zip((token_ids, positions, seq_of_token), np.array(few, dtype=i32).T):
+                    pieces_of.append(values)
+                few = []
+            if n > 1:
+                token_ids.append(np.asarray(e.tokens, dtype=i32))
+                positions.append(np.arange(done, done + n, dtype=i32))
+                seq_of_token.append(np.full(n, si, dtype=i32))
             for w in e.want:
                 logit_rows.append(row + int(w))
             row += n
@@ -503,13 +532,26 @@ class ModelRunner:
             width = table_width or max(len(t) for t in tables)
             block_table = np.full((B, width), -1, dtype=i32)
             off_slot = at
-            for b, (table, pos) in enumerate(zip(tables, positions)):
+            slots: List[int] = []                              # of neighbouring entries of one token
+            for b, (table, n, total) in enumerate(zip(tables, host["q_len"], host["context_len"])):
                 block_table[b, :len(table)] = table
-                pages = block_table[b, pos // ps]
-                if (pages < 0).any():
-                    p = int(pos[int(np.argmax(pages < 0))])
-                    raise StepError(f"request {entries[b].request!r}: position {p} lies in a page already given back")
-                pieces.append(pages * ps + pos % ps)
+                first = total - n
+                if n == 1:
+                    page = table[first // ps] if first // ps < len(table) else -1
+                    gone = 0 if page < 0 else None
+                    slots.append(page * ps + first % ps)
+                else:
+                    if slots:
+                        pieces.append(np.array(slots, dtype=i32))
+                        slots = []
+                    pos = np.arange(first, total, dtype=i32)
+                    pages = block_table[b, pos // ps]
+                    gone = int(np.argmax(pages < 0)) if (pages < 0).any() else None
+                    pieces.append(pages * ps + pos % ps)
+                if gone is not None:
+                    raise StepError(f"request {entries[b].request!r}: position {first + gone} lies in a page already given back")
+            if slots:
+                pieces.append(np.array(slots, dtype=i32))
             at += row
             pieces.append(block_table.reshape(-1))
             layout.append((off_slot, at, width))

@@ -102,7 +102,7 @@ def _gpu(t: torch.Tensor, name: str, dtype=None, shape=None) -> None:
         raise KernelError(f"{name} must be contiguous")
     if dtype is not None and t.dtype != dtype:
         raise KernelError(f"{name} must be {dtype}, is {t.dtype}")
-    if shape is not None and tuple(t.shape) != tuple(shape):
+    if shape is not None and t.shape != shape and tuple(t.shape) != tuple(shape):
         raise KernelError(f"{name} must have shape {tuple(shape)}, has {tuple(t.shape)}")
 
 
@@ -398,6 +398,7 @@ def _f32_tile_tokens(hd: int, group: int) -> int:
     return int(attention_mfma_f32_lib(hd).ni_mfma_attention_f32_tile_tokens(group))
 
 
+@functools.lru_cache(maxsize=4096)       # (every layer of a step asks the same)
 def mfma_tile_tokens(hd: int, group: int, n_tokens: Optional[int] = None, kv_heads: int = 1,
                      dtype: torch.dtype = torch.bfloat16) -> int:
     """Tokens of one tile of the matrix-core attention kernel for ``group`` query heads per kv head.
@@ -424,6 +425,7 @@ def mfma_tile_tokens(hd: int, group: int, n_tokens: Optional[int] = None, kv_hea
     return int(lib.ni_mfma_attention_tile_tokens(int(group), blocks))
 
 
+@functools.lru_cache(maxsize=4096)       # (every layer of a step asks the same)
 def mfma_plan(hd: int, group: int, kv_heads: int, n_tokens: int, max_q_len: int, max_keys: int,
               dtype: torch.dtype = torch.bfloat16):
     """Tile size and number of key runs for the matrix-core attention of a step of ``n_tokens``
@@ -454,6 +456,7 @@ def mfma_plan(hd: int, group: int, kv_heads: int, n_tokens: int, max_q_len: int,
     return small, None
 
 
+@functools.lru_cache(maxsize=4096)       # (every layer of a step asks the same)
 def mfma_group_plan(hd: int, group: int, kv_heads: int, n_tokens: int, max_q_len: int, max_keys: int, dtype: torch.dtype = torch.bfloat16):
     """``(tile_tokens, nsplit)`` where the bfloat16 prompt kernel takes eight wavefronts a tile, two groups of four that walk one
     half of its keys each, instead of :func:`mfma_plan`'s four; else None.  A workgroup then has a compute unit to itself and keeps
@@ -560,6 +563,7 @@ def _f32_runs(items: int, tokens: int, max_keys: int, hd: int) -> int:
     return min(range(2, min(max_keys // 32, 16) + 1), key=lambda n: _f32_cost(items, tokens, max_keys, hd, n))
 
 
+@functools.lru_cache(maxsize=4096)       # (every layer of a step asks the same)
 def mfma_splits(n_tiles: int, kv_heads: int, group: int, max_keys: int, hd: int = 64,
                 dtype: torch.dtype = torch.bfloat16, alone: bool = True) -> int:
     """Into how many runs the matrix-core kernel cuts the keys of every tile.  Cutting costs a

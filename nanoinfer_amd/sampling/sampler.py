@@ -64,7 +64,8 @@ class Sampler:
                            [p.repetition_penalty for p in params],
                            [uniform_from_counter(max(p.seed, 0), c) for p, c in zip(params, counters)]], dtype=np.float32)
         ints = np.array([p.top_k if p.use_top_k() else 0 for p in params] + pen_off + (pen_ids or [0]), dtype=np.int32)
-        packed = torch.from_numpy(np.concatenate([floats.reshape(-1).view(np.int32), ints])).to(self.device)
+        # (from pinned memory: from ordinary memory the copy would wait for the forward, and the draw's launches with it)
+        packed = torch.from_numpy(np.concatenate([floats.reshape(-1).view(np.int32), ints])).pin_memory().to(self.device, non_blocking=True)
         as_float = packed[: 4 * R].view(torch.float32)
         temperature, top_p, penalty, uniform = (as_float[i * R:(i + 1) * R] for i in range(4))
         top_k = packed[4 * R: 5 * R]
