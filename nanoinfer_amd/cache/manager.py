@@ -259,6 +259,11 @@ class KVCacheManager:
         return self.num_pages * self.page_size if not self.groups else 1 << 60
 
     # ---------------------------------------------------------------- changes
+    def _clear(self, slot: int) -> None:
+        """Zero a slot's states, all layers' together (one by one they were eight launches of 4 to 5 us for a hybrid of eight layers)."""
+        if self.state:
+            torch._foreach_zero_([t[slot] for t in self.state.values()])
+
     def reserve(self, request: Hashable, total_tokens: int) -> bool:
         """Make room for the request's tokens ``0..total_tokens-1`` in every group; a request seen
         for the first time also gets its state slot.  All or nothing: ``False`` leaves everything
@@ -270,8 +275,7 @@ class KVCacheManager:
             return False
         if not known:
             slot = self.slots.take(request)
-            for cid, t in self.state.items():
-                t[slot].zero_()
+            self._clear(slot)
             for g in self.groups:
                 g.tables[request] = []
         for g in self.groups:
@@ -306,8 +310,7 @@ class KVCacheManager:
             needs.append(per)
         for r in new:
             slot = self.slots.take(r)
-            for cid, t in self.state.items():
-                t[slot].zero_()
+            self._clear(slot)
             for g in self.groups:
                 g.tables[r] = []
         for g, per in zip(self.groups, needs):

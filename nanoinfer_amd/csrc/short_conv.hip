@@ -4,8 +4,10 @@
 // A step brings, for every sequence b, the rows q_start[b] .. q_start[b] + q_len[b] - 1 (consecutive tokens of that
 // sequence).  Inputs before a portion's first row come from the sequence's tail, [(taps - 1)][channels] float32 (the
 // oldest first; zeros for a new sequence) at float `tail_off` of the row state_slot[b] of `state`.  A step of single
-// tokens (`single`: one row a sequence) moves the tail on in the kernel that reads it; for longer portions
-// conv_move_tail_kernel does so in a launch of its own, after every row has been read.
+// tokens (`single`: one row a sequence) moves the tail on in the kernel that reads it.  So does a step of one sequence whose first
+// taps - 1 rows, the only ones that read the tail, lie in one thread's block of rows (TailMove::Alone); for other portions
+// conv_move_tail_kernel does so in a launch of its own, after every row has been read (4.2 to 5.5 us a launch, all latency:
+// 2,045 tokens through eight layers with twelve convolutions 3,123 us with it, 3,081 without and with all states cleared in one launch).
 //
 //   input_conv        x[t] = u[t] + conv(u)[t]: what a sublayer reads of the stream
 //   add_norm_conv     h += rmsnorm(y) * w * mult, and (single tokens) the input convolution of the layer behind it
@@ -33,6 +35,13 @@ struct StepRows {
     }
 };
 
+// who moves a sequence's tail on: a launch of its own behind the step's rows, the thread of a single token, or the thread that has the
+// first rows of a step's one sequence
+enum class TailMove { Behind, Single, Alone };
+static TailMove tail_move(bool single, int B, int block, int taps) {
+    return single ? TailMove::Single : B == 1 && block >= taps - 1 ? TailMove::Alone : TailMove::Behind;
+}
+
 // the filtered input at row t (place r in its portion), channel c of `channels`
 __device__ __forceinline__ float conv_at(const float* __restrict__ u, int stride, const float* __restrict__ w, const float* tail,
                                          int t, int r, int c, int channels, int taps) {
@@ -52,18 +61,25 @@ __device__ __forceinline__ void move_tail_one(float* tail, int c, int channels, 
     if (taps > 1) tail[static_cast<size_t>(taps - 2) * channels + c] = input;
 }
 
+// N channels' columns of the tail after a portion of n rows that begins at row `first`
+template <int N>
+__device__ __forceinline__ void move_tail_rows(const float* __restrict__ u, int stride, float* tail, int first, int n, int c, int channels, int taps) {
+    const int keep = taps - 1;
+    for (int j = 0; j < keep; ++j) {              // ascending: what is read lies at or above what has been written
+        const int idx = n - keep + j;             // place in the portion of the input that ends up at j
+        float v[N];
+        if (idx >= 0) VecIO<float, N>::load(u + static_cast<size_t>(first + idx) * stride + c, v);
+        else VecIO<float, N>::load(tail + static_cast<size_t>(keep + idx) * channels + c, v);
+        VecIO<float, N>::store(tail + static_cast<size_t>(j) * channels + c, v);
+    }
+}
+
 // the last taps - 1 inputs of every sequence of the step, the oldest first; a thread moves one channel's column
 __global__ void conv_move_tail_kernel(const float* __restrict__ u, int stride, StepRows rows, int channels, int taps, int B) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.y;
     if (c >= channels || b >= B) return;
-    const int n = rows.q_len[b], keep = taps - 1;
-    if (n <= 0) return;
-    float* tail = rows.tail(b);
-    for (int j = 0; j < keep; ++j) {              // ascending: what is read lies at or above what has been written
-        const int idx = n - keep + j;             // place in the portion of the input that ends up at j
-        tail[static_cast<size_t>(j) * channels + c] = idx >= 0 ? u[static_cast<size_t>(rows.q_start[b] + idx) * stride + c]
-                                                               : tail[static_cast<size_t>(keep + idx) * channels + c];
-    }
+    const int n = rows.q_len[b];
+    if (n > 0) move_tail_rows<1>(u, stride, rows.tail(b), rows.q_start[b], n, c, channels, taps);
 }
 
 static void launch_move_tail(const float* u, int stride, const StepRows& rows, int channels, int taps, int B, hipStream_t stream) {
@@ -80,7 +96,7 @@ static void launch_move_tail(const float* u, int stride, const StepRows& rows, i
 template <typename T, bool PIECES, int TOKENS>
 __global__ void __launch_bounds__(256)
 input_conv_kernel(const float* __restrict__ h, const float* __restrict__ w, StepRows rows, T* __restrict__ x, int Tn, int d, int taps,
-                  int per_row, size_t total, bool single) {
+                  int per_row, size_t total, TailMove move) {
     constexpr int N = PIECES ? 4 : 1;
     const size_t at = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (at >= total) return;
@@ -129,11 +145,12 @@ input_conv_kernel(const float* __restrict__ h, const float* __restrict__ w, Step
         }
         if constexpr (PIECES) store_packed<T, 4>(x + static_cast<size_t>(t) * d + c, acc);
         else st(x + static_cast<size_t>(t) * d + c, acc[0]);
-        if (single) {        // this thread alone reads and writes its channels' columns of the tail
+        if (move == TailMove::Single) {        // this thread alone reads and writes its channels' columns of the tail
 #pragma unroll
             for (int e = 0; e < N; ++e) move_tail_one(tail, c + e, d, taps, own[tt][e]);
         }
     }
+    if (move == TailMove::Alone && t0 == 0) move_tail_rows<N>(h, d, rows.tail(0), rows.q_start[0], rows.q_len[0], c, d, taps);      // (as above)
 }
 
 static bool whole_pieces(int d, const StepRows& rows, const void* a, const void* b) {
@@ -152,21 +169,23 @@ NI_EXPORT int ni_input_conv(const void* h, const void* w, void* state, size_t st
                         (float*)state, state_stride, tail_off};
     const bool pieces = whole_pieces(d, rows, h, x);
     const int per_row = pieces ? d / 4 : d;
+    TailMove move = TailMove::Behind;
     auto launch = [&](auto* out, auto piece_tag, auto tokens_tag) {
         constexpr int TOKENS = decltype(tokens_tag)::value;
         const size_t threads = static_cast<size_t>((T + TOKENS - 1) / TOKENS) * per_row;
         input_conv_kernel<std::remove_pointer_t<decltype(out)>, decltype(piece_tag)::value, TOKENS><<<blocks_of(threads, 256), 256, 0, stream>>>(
-            (const float*)h, (const float*)w, rows, out, T, d, taps, per_row, threads, single != 0);
+            (const float*)h, (const float*)w, rows, out, T, d, taps, per_row, threads, move = tail_move(single != 0, B, TOKENS, taps));
     };
     auto run = [&](auto* out) {
         using One = std::integral_constant<int, 1>;
         using Four = std::integral_constant<int, 4>;
-        if (pieces) T >= 256 ? launch(out, std::true_type{}, Four{}) : launch(out, std::true_type{}, One{});
+        // (one sequence in blocks of four from 64 rows on: the fewer threads cost less than the launch behind them)
+        if (pieces) T >= 256 || (B == 1 && T >= 64) ? launch(out, std::true_type{}, Four{}) : launch(out, std::true_type{}, One{});
         else launch(out, std::false_type{}, One{});
     };
     if (dtype == 0) run((float*)x);
     else run((bf16_t*)x);
-    if (!single) launch_move_tail((const float*)h, d, rows, d, taps, B, stream);
+    if (move == TailMove::Behind) launch_move_tail((const float*)h, d, rows, d, taps, B, stream);
     return NI_LAUNCH_RESULT();
 }
 
@@ -378,7 +397,7 @@ __global__ void __launch_bounds__(256)
 qkv_conv_kernel(const float* __restrict__ proj, int row_stride, const int32_t* __restrict__ positions,
                 const int32_t* __restrict__ slot_mapping, const float* __restrict__ filters, const float* __restrict__ wq,
                 const float* __restrict__ wk, float eps, const float* __restrict__ freq, StepRows rows, T* __restrict__ q_out,
-                T* __restrict__ kpool, T* __restrict__ vpool, int Tn, QkvForm f, bool single) {
+                T* __restrict__ kpool, T* __restrict__ vpool, int Tn, QkvForm f, TailMove move) {
     static_assert(UPW == 1 || NP == 1, "a unit of two a wavefront has one pair a lane");
     __shared__ float cos_of[TB * CONV_PAIRS], sin_of[TB * CONV_PAIRS];
     const int t0 = blockIdx.x * TB, n_tok = min(TB, Tn - t0);
@@ -476,7 +495,7 @@ qkv_conv_kernel(const float* __restrict__ proj, int row_stride, const int32_t* _
                         y[tt][p][e] = in[p][e] ? conv_at(proj, row_stride, filters, tail, t, r, c0 + c + e, channels, taps) : 0.f;
                     }
                 }
-                if (single && filters) {          // this lane alone reads and writes its channels' columns of the tail
+                if (move == TailMove::Single && filters) {          // this lane alone reads and writes its channels' columns of the tail
                     if constexpr (TAPS > 1) {     // the window holds what the tail is to hold
 #pragma unroll
                         for (int j = 0; j < TAPS - 1; ++j)
@@ -484,6 +503,23 @@ qkv_conv_kernel(const float* __restrict__ proj, int row_stride, const int32_t* _
                     } else {
                         if (in[p][0]) move_tail_one(tail, c0 + c, channels, taps, own[0]);
                         if (in[p][1]) move_tail_one(tail, c0 + c + 1, channels, taps, own[1]);
+                    }
+                }
+            }
+        }
+        if constexpr (TAPS > 1 && TB >= TAPS - 1) {
+            if (move == TailMove::Alone && t0 == 0 && filters) {          // (as above: the only rows that read the tail are this block's)
+                float* tail = rows.tail(0);
+                const int end = rows.q_start[0] + rows.q_len[0], keep = min(TAPS - 1, rows.q_len[0]);
+#pragma unroll
+                for (int j = 0; j < TAPS - 1; ++j) {                      // (ascending: what is read lies above what has been written)
+                    const float* from = j >= TAPS - 1 - keep ? proj + static_cast<size_t>(end - (TAPS - 1) + j) * row_stride
+                                                             : tail + static_cast<size_t>(j + keep) * channels;
+#pragma unroll
+                    for (int p = 0; p < NP; ++p) {
+                        float v[2];
+                        load_two<PAIRS>(from + c0 + 2 * sub + 128 * p, in[p], v);
+                        store_two<PAIRS>(tail + static_cast<size_t>(j) * channels + c0 + 2 * sub + 128 * p, in[p], v[0], v[1]);
                     }
                 }
             }
@@ -540,11 +576,12 @@ qkv_conv_kernel(const float* __restrict__ proj, int row_stride, const int32_t* _
 
 struct QkvArgs {
     const float* proj; int row_stride; const int32_t *positions, *slot_mapping; const float *filters, *wq, *wk; float eps;
-    const float* freq; StepRows rows; void *q_out, *kpool, *vpool; int T; QkvForm f; bool single;
+    const float* freq; StepRows rows; void *q_out, *kpool, *vpool; int T, B; QkvForm f; bool single;
 };
 
 template <typename T, int TAPS, int TB>
-static bool launch_qkv(const QkvArgs& a, hipStream_t stream) {
+static bool launch_qkv(const QkvArgs& a, TailMove& move, hipStream_t stream) {
+    move = tail_move(a.single, a.B, TAPS > 1 ? TB : 0, a.f.taps);      // (without a number of taps of its own the kernel has no block)
     const int blocks = (a.T + TB - 1) / TB;
     // every row, unit and tail starts at an even element, and the addresses are aligned to pairs
     auto even = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 8 == 0; };
@@ -559,7 +596,7 @@ static bool launch_qkv(const QkvArgs& a, hipStream_t stream) {
         const dim3 grid(blocks, std::max(1, std::min(most, (1536 + blocks - 1) / blocks)));
         qkv_conv_kernel<T, TAPS, TB, NP, UPW, decltype(pair_tag)::value><<<grid, 256, 0, stream>>>(
             a.proj, a.row_stride, a.positions, a.slot_mapping, a.filters, a.wq, a.wk, a.eps, a.freq, a.rows, (T*)a.q_out, (T*)a.kpool,
-            (T*)a.vpool, a.T, a.f, a.single);
+            (T*)a.vpool, a.T, a.f, move);
     };
     auto run = [&](auto np, auto upw) {
         if (pairs) { go(np, upw, std::true_type{}); return true; }
@@ -575,11 +612,13 @@ static bool launch_qkv(const QkvArgs& a, hipStream_t stream) {
 }
 
 template <typename T>
-static void launch_qkv_any(const QkvArgs& a, hipStream_t stream) {
+static TailMove launch_qkv_any(const QkvArgs& a, hipStream_t stream) {
     const bool few = a.T < 64;        // few tokens: a row a workgroup, spread over the units
+    TailMove move;
     if (a.filters && a.f.taps == 4 && reinterpret_cast<uintptr_t>(a.filters) % 16 == 0 &&
-        (few ? launch_qkv<T, 4, 1>(a, stream) : launch_qkv<T, 4, 8>(a, stream))) return;
-    few ? launch_qkv<T, 0, 1>(a, stream) : launch_qkv<T, 0, 8>(a, stream);
+        (few ? launch_qkv<T, 4, 1>(a, move, stream) : launch_qkv<T, 4, 8>(a, move, stream))) return move;
+    few ? launch_qkv<T, 0, 1>(a, move, stream) : launch_qkv<T, 0, 8>(a, move, stream);
+    return move;
 }
 
 // filters float32 [channels, taps] or null; state and tail_off: see StepRows (channels of the tail: q | k | v)
@@ -597,10 +636,9 @@ NI_EXPORT int ni_qkv_conv(const void* proj, int row_stride, const void* position
     const StepRows rows{(const int32_t*)seq_of_token, (const int32_t*)q_start, (const int32_t*)q_len, (const int32_t*)state_slot,
                         (float*)state, state_stride, tail_off};
     const QkvArgs a{(const float*)proj, row_stride, (const int32_t*)positions, (const int32_t*)slot_mapping, (const float*)filters,
-                    (const float*)wq, (const float*)wk, eps, (const float*)freq, rows, q_out, kpool, vpool, T,
+                    (const float*)wq, (const float*)wk, eps, (const float*)freq, rows, q_out, kpool, vpool, T, B,
                     QkvForm{H, G, maps, dk, dv, rot, taps, page_size}, single != 0};
-    if (dtype == 0) launch_qkv_any<float>(a, stream);
-    else launch_qkv_any<bf16_t>(a, stream);
-    if (filters && !single) launch_move_tail((const float*)proj, row_stride, rows, channels, taps, B, stream);
+    const TailMove move = dtype == 0 ? launch_qkv_any<float>(a, stream) : launch_qkv_any<bf16_t>(a, stream);
+    if (filters && move == TailMove::Behind) launch_move_tail((const float*)proj, row_stride, rows, channels, taps, B, stream);
     return NI_LAUNCH_RESULT();
 }
