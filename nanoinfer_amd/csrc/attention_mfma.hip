@@ -1,5 +1,5 @@
 // Attention of prompt portions over the paged key/value cache on the matrix cores of gfx950.  (mfma_attention_kernel; head sizes 64 and 128
-// with pages of sixteen tokens and more take the kernel of attention_prompt.h.)
+// mostly take the kernel of attention_prompt.h: takes_prompt_kernel.)
 // bfloat16 only; compiled once per head size (-DHEAD_DIM=n, a multiple of 16 up to 256; the kernel for
 // single tokens takes the multiples of 32 among them).
 //
@@ -879,8 +879,11 @@ NI_EXPORT int ni_mfma_attention(const void* q, int q_stride, const void* kpool, 
     };
     dim3 grid;
 #if HEAD_DIM == 64 || HEAD_DIM == 128
+    // The kernel of attention_prompt.h: a wavefront's rows of a stage lie in one page, and what goes straight into LDS starts at sixteen bytes.
+    auto whole = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+    const bool takes_prompt_kernel = pow2 && page_size >= 1024 / HEAD_DIM && whole(kpool) && whole(vpool);
 #define MA_LAUNCH_PROMPT(CB_, GROUPS_)                                                                                         \
-    if (pow2 && page_size >= 1024 / HEAD_DIM) { /* (a wavefront's rows of a stage lie in one page) */                        \
+    if (takes_prompt_kernel) {                                                                                                 \
         static int held = 0;                                                                                                   \
         if (!grid_for(reinterpret_cast<const void*>(prompt_attention_kernel<CB_, GROUPS_>), GROUPS_ * MA_WAVES * WAVE, held, grid)) return -4; \
         prompt_attention_kernel<CB_, GROUPS_><<<grid, GROUPS_ * MA_WAVES * WAVE, 0, stream>>>(                                 \

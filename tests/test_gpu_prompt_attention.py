@@ -6,8 +6,9 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def worst_excess(portions, H, KVH, hd, ps, blocks=1, groups=1, nsplit=1, window=None, seed=0, plant=None):
-    """``portions``: (tokens, keys) of every sequence.  The largest excess over the bound of rounded weights."""
+def worst_excess(portions, H, KVH, hd, ps, blocks=1, groups=1, nsplit=1, window=None, seed=0, plant=None, off=0):
+    """``portions``: (tokens, keys) of every sequence.  The largest excess over the bound of rounded weights.  ``off``: elements by which the pools start
+    behind an allocation's first byte."""
     from nanoinfer_amd import kernels as K
     g = torch.Generator().manual_seed(seed)
     T = sum(n for n, _ in portions)
@@ -35,7 +36,8 @@ def worst_excess(portions, H, KVH, hd, ps, blocks=1, groups=1, nsplit=1, window=
     qkv[:, :H * hd] = q.reshape(T, H * hd)
     out = torch.full((T + 1, H * hd), 7.0, device="cuda", dtype=torch.bfloat16)
     ws = torch.empty(T * H * nsplit * (hd + 2), device="cuda")
-    K.mfma_attention(qkv.cuda(), kp.cuda(), vp.cuda(), table.cuda(), tiles, out[:T], H, KVH, hd, hd ** -0.5, window, nsplit, ws, tile, groups)
+    kp, vp = (torch.cat([p.new_zeros(off), p.view(-1)]).cuda()[off:].view(p.shape) for p in (kp, vp))
+    K.mfma_attention(qkv.cuda(), kp, vp, table.cuda(), tiles, out[:T], H, KVH, hd, hd ** -0.5, window, nsplit, ws, tile, groups)
     assert bool((out[T] == 7.0).all())
     got, worst = out[:T].view(T, H, hd).cpu().double(), -1.0
     for s, (n, keys) in enumerate(portions):
@@ -63,6 +65,13 @@ def worst_excess(portions, H, KVH, hd, ps, blocks=1, groups=1, nsplit=1, window=
     (((17, 191), (1, 192), (1, 193), (1, 7)), 16), (((130, 500),), 256), (((20, 20480 + 40),), 16)])
 def test_ends_of_stages_and_pages(hd, H, KVH, blocks, groups, portions, ps):
     assert worst_excess(portions, H, KVH, hd, ps, blocks, groups, seed=hd + blocks) <= 0.0
+
+
+@pytest.mark.parametrize("hd,H,KVH,groups", [(64, 4, 1, 1), (64, 4, 1, 2), (128, 3, 1, 1)])
+@pytest.mark.parametrize("off", [1, 4])
+def test_pools_off_sixteen_bytes(hd, H, KVH, groups, off):
+    """Views into a program's own buffers: what goes straight into LDS would start between sixteen bytes, so that another kernel takes them."""
+    assert worst_excess(((17, 191), (1, 193), (40, 40)), H, KVH, hd, 16, 1, groups, seed=off, off=off) <= 0.0
 
 
 def test_more_pages_than_their_numbers_in_lds():
