@@ -194,7 +194,6 @@ void prompt_attention_kernel(
     constexpr int SLOT = sizeof(Stage), LAST_SLOT = (PA_RING - 1) * SLOT;
     const uint32_t ring_at = lds_address(&ring[group][0]) + wave * LOADS * 1024;
     int slot_in = 0, slot_out = 0, ahead = 0;                // bytes into the ring; stages asked for and not taken yet
-    const uint32_t stride = static_cast<uint32_t>(KVH) * ROW << page_shift;      // bytes of a page
     const char *k_pool = reinterpret_cast<const char*>(kpool) - 1024, *v_pool = reinterpret_cast<const char*>(vpool) - 1024;
     int page = 0, from = 0;
     bool asks = false;                                       // there are rows to be asked for: of `page`, from key `from` on
@@ -214,11 +213,12 @@ void prompt_attention_kernel(
         }
     };
     auto ask = [&]() {
-        // from the page's first byte to where key 0 would lie
-        const int back = ((g << page_shift) + (from & (page_size - 1)) - from) * ROW;
-        const size_t at = static_cast<size_t>(static_cast<uint32_t>(max(uniform(page), 0))) * stride + back;
+        // the first row of the group's in the pool: its number fits 32 bits (the host checks the pool's size), and the lanes count from there
+        const uint32_t row = ((static_cast<uint32_t>(max(uniform(page), 0)) * KVH + g) << page_shift) + (from & (page_size - 1));
+        const size_t at = static_cast<size_t>(row) * ROW;
         const uint32_t to = ring_at + slot_in;
-        const int key0 = min(max(in.key + line, in.lo), in.last), key1 = min(max(in.key + line + CHUNK, in.lo), in.last);
+        const int key = in.key - from, lo = in.lo - from, last = in.last - from;
+        const int key0 = min(max(key + line, lo), last), key1 = min(max(key + line + CHUNK, lo), last);
         // (the pools' addresses are 1,024 bytes before them, and so much is in the lanes' places: a load that lands so much further on reads there)
         load_rows_to_lds(k_pool + at, v_pool + at, to, to + KEYS * ROW, key0 * ROW + piece_k[0], key1 * ROW + piece_k[1], key0 * ROW + piece_v[0],
                          key1 * ROW + piece_v[1]);

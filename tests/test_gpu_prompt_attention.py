@@ -78,6 +78,37 @@ def test_more_pages_than_their_numbers_in_lds():
     assert worst_excess(((9, 50000),), 4, 1, 64, 16) <= 0.0
 
 
+@pytest.mark.parametrize("hd,groups", [(64, 1), (64, 2), (128, 1), (128, 2)])
+def test_keys_further_than_two_gigabytes(hd, groups):
+    """A sequence whose key rows, one behind the other, would pass 2^31 bytes: the few pages behind that hold the keys that count, the others are the
+    same 64 pages over and over."""
+    from nanoinfer_amd import kernels as K
+    ps, H, n, few = 256, 2, 40, 3
+    far = (1 << 31) // (2 * hd) // ps                           # the first page past it
+    keys = (far + few) * ps
+    g = torch.Generator().manual_seed(hd)
+    kp, vp = (torch.randn(64 + few, 1, ps, hd, generator=g).bfloat16() for _ in range(2))
+    q = torch.randn(n, H, hd, generator=g).bfloat16()
+    q[..., 0], kp[..., 0] = 8.0, 0.0
+    kp[64:, :, 5::16, 0] = 24.0 * hd ** 0.5 / 8.0               # e^24 of the others, of which there are e^16
+    table = torch.cat([torch.arange(far) % 64, 64 + torch.arange(few)]).int().view(1, -1).cuda()
+    qkv = torch.zeros(n, (H + 2) * hd, dtype=torch.bfloat16)
+    qkv[:, :H * hd] = q.reshape(n, H * hd)
+    tile, nsplit = K.mfma_tile_tokens(hd, H), 16
+    tiles = torch.tensor(K.build_q_tiles([0], [n], [keys], tile), dtype=torch.int32).view(-1, 4).cuda()
+    out, ws = torch.empty(n, H * hd, device="cuda", dtype=torch.bfloat16), torch.empty(n * H * nsplit * (hd + 2), device="cuda")
+    K.mfma_attention(qkv.cuda(), kp.cuda(), vp.cuda(), table, tiles, out, H, 1, hd, hd ** -0.5, None, nsplit, ws, tile, groups)
+    k, v = (p[:, 0].reshape(-1, hd).double() for p in (kp, vp))
+    for t in (0, n - 1):
+        rows = keys - n + t + 1
+        times = torch.cat([torch.full((64 * ps,), float(far // 64)) + (torch.arange(64 * ps) < far % 64 * ps), (torch.arange(few * ps) < rows - far * ps).double()])
+        for h in range(H):
+            w = times * torch.exp((k @ q[t, h].double()) * hd ** -0.5 - 24.0)
+            want = w @ v / w.sum()
+            here = out[t].view(H, hd)[h].cpu().double()
+            assert float(((here - want).abs() - 2.0 ** -8 * float(v.abs().max()) - 2.0 ** -8 * want.abs()).max()) <= 1e-3
+
+
 @pytest.mark.parametrize("hd,H,KVH", [(64, 8, 2), (64, 20, 1), (128, 6, 2)])
 @pytest.mark.parametrize("window,nsplit", [(None, 1), (40, 1), (None, 3)])
 def test_single_tokens_beside_a_portion(hd, H, KVH, window, nsplit):
