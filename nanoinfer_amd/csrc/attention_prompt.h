@@ -2,7 +2,7 @@
 // same tiles, blocks, groups, rows and products as mfma_attention_kernel there, which the other head sizes and pages keep.  What is different:
 //
 // Keys and values go from memory straight into LDS, a page's rows by one wavefront, whose page number and addresses are scalars: no vector
-// instruction works out where rows lie (sixteen a set of 32 keys before) and no row waits in registers, which leaves 165 of them instead of 253.
+// instruction works out where rows lie (sixteen a set of 32 keys there) and no row waits in registers (219 of them at most, 253 there).
 // Stages go through a ring of three slots; the next tile's first ones are asked for while this one's last are multiplied.
 //
 // Inside the key range of all its rows a set of 32 keys is not looked at for scores that rise above the row's reference (four maxima, a
@@ -11,7 +11,9 @@
 // workgroup makes the tile again with a look at every set (references that move, as in the other kernel; windows always take that way).
 //
 // The scores of a set are taken while the set before it gets its weights (at head size 128 a step of 32 keys is 25 % faster by it), so that the
-// matrix cores work beside the vector unit's exponentials.
+// matrix cores work beside the vector unit's exponentials.  At the ends of a walk, and where scores are looked at, head size 64 takes a stage's two
+// sets side by side: one at a time, short walks were slower than mfma_attention_kernel's (128 tokens at 228 keys 7.5 us there, 8.4 one at a time, 7.6
+// side by side; 16 heads on 16, 256 at 256 7.4, 8.6, 7.7; 512 at 512 10.1, 10.5, 9.6).
 //
 // What bounds it: at long key ranges neither of the two (matrix cores busy 41 %, the vector unit 50 % of the cycles, two wavefronts a SIMD with
 // a chain of instructions each); in one prompt of 2,000 tokens starts and ends: of 79,000 cycles of a workgroup's two tiles 9,000 pass before the first
@@ -302,16 +304,20 @@ void prompt_attention_kernel(
                     o[c][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vf[dt]), __builtin_bit_cast(bf16x8_t, pf[c]), o[c][dt], 0, 0, 0);
             }
         };
-        // Any set, with a look at how far its scores rise (key0: this lane's first key of it):
-        auto any_set = [&](const char* k, const char* v, int key0) {
-            floatx4_t sc[CB][2];
-            scores(k, sc);
-            float raw[CB][8], lane_max[CB];
+        // n neighbouring sets of a stage, with a look at how far their scores rise (key0: this lane's first key of them):
+        auto any_sets = [&](auto N, const char* k, const char* v, int key0) {
+            constexpr int n = decltype(N)::value;
+            floatx4_t sc[n][CB][2];
+#pragma unroll
+            for (int s = 0; s < n; ++s) scores(k + s * KSTEP * ROW, sc[s]);
+            float raw[n][CB][8], lane_max[CB];
             bool risen = false;
 #pragma unroll
             for (int c = 0; c < CB; ++c) {
                 const int lo = window > 0 ? hi[c] + 1 - window : 0;
-                lane_max[c] = mask_scores<true>(sc[c], key0, lo, hi[c], true, raw[c]);
+                lane_max[c] = NEG_BIG;
+#pragma unroll
+                for (int s = 0; s < n; ++s) lane_max[c] = fmaxf(lane_max[c], mask_scores<true>(sc[s][c], key0 + s * KSTEP, lo, hi[c], true, raw[s][c]));
                 risen = risen || above_reference(lane_max[c], scale2, m_run[c]);
             }
             if (__any(risen)) {
@@ -323,10 +329,13 @@ void prompt_attention_kernel(
                     for (int dt = 0; dt < DT; ++dt) o[c][dt] *= corr;
                 }
             }
-            uint4 pf[CB];
+            uint4 pf[n][CB];
 #pragma unroll
-            for (int c = 0; c < CB; ++c) pf[c] = weights<true>(raw[c], scale2, m_run[c]);
-            add_values(v, pf);
+            for (int s = 0; s < n; ++s)
+#pragma unroll
+                for (int c = 0; c < CB; ++c) pf[s][c] = weights<true>(raw[s][c], scale2, m_run[c]);
+#pragma unroll
+            for (int s = 0; s < n; ++s) add_values(v + s * KSTEP * ROW, pf[s]);
             if (!primed) {
                 bool cold = safe;
 #pragma unroll
@@ -334,34 +343,40 @@ void prompt_attention_kernel(
                 primed = !__any(cold);
             }
         };
-        // Without a window: a tile's first set, from whose largest scores the rows take their references, and one with keys behind some rows' positions.
-        auto edge_set = [&](const char* k, const char* v, int key0) {
-            floatx4_t sc[CB][2];
-            scores(k, sc);
+        // Without a window: a tile's first sets, from the largest scores of the first of which the rows take their references, and those with keys
+        // behind some rows' positions.
+        auto edge_sets = [&](auto N, const char* k, const char* v, int key0) {
+            constexpr int n = decltype(N)::value;
+            floatx4_t sc[n][CB][2];
+#pragma unroll
+            for (int s = 0; s < n; ++s) scores(k + s * KSTEP * ROW, sc[s]);
             if (!primed) {
 #pragma unroll
                 for (int c = 0; c < CB; ++c) {
-                    float mx = fmaxf(sc[c][0][0], sc[c][1][0]);
+                    float mx = fmaxf(sc[0][c][0][0], sc[0][c][1][0]);
 #pragma unroll
-                    for (int i = 1; i < 4; ++i) mx = fmaxf(mx, fmaxf(sc[c][0][i], sc[c][1][i]));
+                    for (int i = 1; i < 4; ++i) mx = fmaxf(mx, fmaxf(sc[0][c][0][i], sc[0][c][1][i]));
                     m_run[c] = row_max4(mx) * scale2;
                 }
                 primed = true;
             }
-            uint4 pf[CB];
+            uint4 pf[n][CB];
 #pragma unroll
-            for (int c = 0; c < CB; ++c) {
-                float w[8];
+            for (int s = 0; s < n; ++s)
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    w[i] = __builtin_amdgcn_exp2f(fmaf(sc[c][i / 4][i % 4], scale2, -m_run[c]));
-                    w[i] = key0 + i / 4 * 16 + i % 4 <= hi[c] ? w[i] : 0.f;
+                for (int c = 0; c < CB; ++c) {
+                    float w[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        w[i] = __builtin_amdgcn_exp2f(fmaf(sc[s][c][i / 4][i % 4], scale2, -m_run[c]));
+                        w[i] = key0 + s * KSTEP + i / 4 * 16 + i % 4 <= hi[c] ? w[i] : 0.f;
+                    }
+                    pf[s][c] = make_uint4(pack_bf16x2(w[0], w[1]), pack_bf16x2(w[2], w[3]), pack_bf16x2(w[4], w[5]), pack_bf16x2(w[6], w[7]));
                 }
-                pf[c] = make_uint4(pack_bf16x2(w[0], w[1]), pack_bf16x2(w[2], w[3]), pack_bf16x2(w[4], w[5]), pack_bf16x2(w[6], w[7]));
-            }
-            add_values(v, pf);
+#pragma unroll
+            for (int s = 0; s < n; ++s) add_values(v + s * KSTEP * ROW, pf[s]);
         };
-        // One whose keys lie inside the range of every row, once every row has a reference: its scores have been taken, and those of the set
+        // A set whose keys lie inside the range of every row, once every row has a reference: its scores have been taken, and those of the set
         // behind it (whose rows start at k) are, while it gets its weights and its values.
         floatx4_t sc[2][CB][2];
         auto inner_set = [&](auto P, const char* k, const char* v) {
@@ -414,9 +429,17 @@ void prompt_attention_kernel(
             } else {
                 const char* k = here + j % SUB * SET;
                 const int key0 = cur.first + j * KSTEP + kg * 4;
-                if (!safe && window <= 0 && (primed || (j == 0 && in_hi > 0))) edge_set(k, k + VALUES, key0);
-                else any_set(k, k + VALUES, key0);
-                ++j;
+                // (both sets of a stage side by side: one alone is a chain of instructions that nothing covers)
+                const bool look = safe || window > 0 || !(primed || (j == 0 && in_hi > 0));
+                if (SUB == 2 && j % SUB == 0 && j + 1 < own) {
+                    if (look) any_sets(Index<SUB>{}, k, k + VALUES, key0);
+                    else edge_sets(Index<SUB>{}, k, k + VALUES, key0);
+                    j += 2;
+                } else {
+                    if (look) any_sets(Index<1>{}, k, k + VALUES, key0);
+                    else edge_sets(Index<1>{}, k, k + VALUES, key0);
+                    ++j;
+                }
             }
         }
         while (met < cur.stages) meet();

@@ -67,6 +67,13 @@ def test_ends_of_stages_and_pages(hd, H, KVH, blocks, groups, portions, ps):
     assert worst_excess(portions, H, KVH, hd, ps, blocks, groups, seed=hd + blocks) <= 0.0
 
 
+@pytest.mark.parametrize("hd,H,KVH,blocks", [(64, 4, 1, 1), (64, 4, 1, 2), (64, 3, 3, 1), (128, 3, 1, 1)])
+@pytest.mark.parametrize("window,nsplit", [(1, 1), (31, 1), (64, 1), (65, 1), (200, 1), (200, 2), (1000, 1)])
+def test_windows(hd, H, KVH, blocks, window, nsplit):
+    """Windows that start and end at and beside stages and sets, rows whose window starts inside the tile's first ones, and one longer than the keys."""
+    assert worst_excess(((130, 500), (33, 33), (64, 128)), H, KVH, hd, 16, blocks, nsplit=nsplit, window=window, seed=window) <= 0.0
+
+
 @pytest.mark.parametrize("hd,H,KVH,groups", [(64, 4, 1, 1), (64, 4, 1, 2), (128, 3, 1, 1)])
 @pytest.mark.parametrize("off", [1, 4])
 def test_pools_off_sixteen_bytes(hd, H, KVH, groups, off):
