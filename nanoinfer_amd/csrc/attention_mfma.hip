@@ -881,7 +881,13 @@ NI_EXPORT int ni_mfma_attention(const void* q, int q_stride, const void* kpool, 
 #if HEAD_DIM == 64 || HEAD_DIM == 128
     // The kernel of attention_prompt.h: a wavefront's rows of a stage lie in one page, and what goes straight into LDS starts at sixteen bytes.
     auto whole = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-    const bool takes_prompt_kernel = pow2 && page_size >= 1024 / HEAD_DIM && whole(kpool) && whole(vpool);
+    // At head size 64 tiles of one block over short windows stay with mfma_attention_kernel while the chip holds them in one round, and those whose
+    // windows are cut into runs: every set is an edge there, or the merge waits (us, that kernel : the other one, 32 heads on 8: 100 and 512 tokens, window 30,
+    // 6.4 : 6.7, 6.1 : 6.7; 128 8.0 : 8.5, 7.9 : 8.3; 300 9.5 : 10.2, 10.3 : 10.2; 512 12.2 : 12.1, 12.1 : 11.8; 16 on 16, 1,999 tokens, 30 / 128 / 300 9.0 : 9.6,
+    // 12.0 : 11.8, 16.8 : 16.1; in two runs, 512 tokens, 512 / 1,024 14.5 : 15.5, 17.2 : 18.1).
+    const bool short_walks = HEAD_DIM == 64 && window > 0 && blocks == 1 &&
+                             (nsplit > 1 || n_tiles * per_tile <= (window <= 128 ? 512 : window < 512 ? 256 : 0));
+    const bool takes_prompt_kernel = pow2 && page_size >= 1024 / HEAD_DIM && whole(kpool) && whole(vpool) && !short_walks;
 #define MA_LAUNCH_PROMPT(CB_, GROUPS_)                                                                                         \
     if (takes_prompt_kernel) {                                                                                                 \
         static int held = 0;                                                                                                   \
