@@ -6,9 +6,13 @@
 // Stages go through a ring of three slots; the next tile's first ones are asked for while this one's last are multiplied.
 //
 // Inside the key range of all its rows a set of 32 keys is not looked at for scores that rise above the row's reference (four maxima, a
-// comparison and a branch a block before): the reference is the largest score of the tile's first set, and float32 holds sums of weights up
-// to 2^40 of it as exactly as any.  What leaves that range, or is not finite, is seen in the sums at the end of the tile, and the whole
-// workgroup makes the tile again with a look at every set (references that move, as in the other kernel; windows always take that way).
+// comparison and a branch a block there): the reference is the largest score of the tile's first set (with a window: of its first sets), and
+// float32 holds sums of weights up to 2^100 of it as exactly as any (an exponent of 100 is rounded by 2^-18 of the weight, which keeps eight
+// bits; what such a sum is merged with and loses lies 2^-26 below it).  What leaves that range, or is not finite, is seen in the sums at the
+// end of the tile, and the whole workgroup makes the tile again with a look at every set (references that move, as in the other kernel).
+// That costs a second, slower walk, for scores that rise by 69 (natural units) above a first set's, or values that are no numbers.  Where it happens
+// to every tile, mfma_attention_kernel : this without it : with it, us: 1,999 tokens at head size 64 39 : 37 : 77, at 128 80 : 60 : 139; 2,048 at 8,192
+// 188 : 161 : 408, 420 : 335 : 892.  (A limit of 2^40 had sent scores that rise by 28 that way, which differ no more in their error against 64 bits.)
 //
 // The scores of a set are taken while the set before it gets its weights (at head size 128 a step of 32 keys is 25 % faster by it), so that the
 // matrix cores work beside the vector unit's exponentials.  At the ends of a walk, and where scores are looked at, head size 64 takes a stage's two
@@ -456,7 +460,7 @@ void prompt_attention_kernel(
                     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
                         for (int i = 0; i < 4; ++i) zero = fmaf(o[c][dt][i], 0.f, zero);
-                    bad = bad || (hi[c] >= 0 && !(l_run[c][0] < 0x1p40f && zero == 0.f));
+                    bad = bad || (hi[c] >= 0 && !(l_run[c][0] < 0x1p100f && zero == 0.f));
                 }
             }
             again[round & 1][group * MA_WAVES + wave] = __any(bad);
