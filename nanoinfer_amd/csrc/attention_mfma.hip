@@ -146,8 +146,8 @@ __device__ __forceinline__ uint4 weights(const float (&raw)[8], float scale2, fl
         float p0 = __builtin_amdgcn_exp2f(fmaf(raw[2 * j], scale2, -m_ref));
         float p1 = __builtin_amdgcn_exp2f(fmaf(raw[2 * j + 1], scale2, -m_ref));
         if constexpr (MASKED) {
-            p0 = raw[2 * j] > 0.5f * NEG_BIG ? p0 : 0.f;
-            p1 = raw[2 * j + 1] > 0.5f * NEG_BIG ? p1 : 0.f;
+            p0 = raw[2 * j] <= 0.5f * NEG_BIG ? 0.f : p0;      // (a score that is no number stays one that is none)
+            p1 = raw[2 * j + 1] <= 0.5f * NEG_BIG ? 0.f : p1;
         }
         pw[j] = pack_bf16x2(p0, p1);
     }
@@ -569,7 +569,7 @@ void mfma_attention_kernel(
                 for (int dt = 0; dt < DT; ++dt)
                     *reinterpret_cast<float4*>(part_o + p * HD + dt * 16 + kg * 4) =
                         make_float4(o[c][dt][0], o[c][dt][1], o[c][dt][2], o[c][dt][3]);
-            } else if (l > 0.f) {
+            } else if (l != 0.f) {            // (no number too, so that the row is none and not what the memory held)
                 const float inv = 1.0f / l;
                 bf16_t* dst = out + static_cast<size_t>(tile.row0 + tt[c]) * H * HD + static_cast<size_t>(head) * HD;
 #pragma unroll

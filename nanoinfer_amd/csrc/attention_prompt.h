@@ -517,7 +517,7 @@ void prompt_attention_kernel(
 #pragma unroll
                     for (int dt = 0; dt < MINE; ++dt)
                         *reinterpret_cast<float4*>(part_o + p * HD + dim0 + dt * 16) = make_float4(done[dt][0], done[dt][1], done[dt][2], done[dt][3]);
-                } else if (l > 0.f) {
+                } else if (l != 0.f) {                           // (no number too, so that the row is none and not what the memory held)
                     const float inv = 1.0f / l;
                     bf16_t* dst = out + static_cast<size_t>(row) * H * HD + static_cast<size_t>(head_) * HD + dim0;
 #pragma unroll

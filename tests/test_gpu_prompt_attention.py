@@ -166,6 +166,18 @@ def test_values_that_are_not_finite(groups):
     assert worst_excess(((150, 400),), 4, 2, 64, 16, 1, groups, seed=6, plant=plant) <= 0.0
 
 
+@pytest.mark.parametrize("hd,blocks,groups,ps,window,nsplit", [
+    (64, 1, 1, 16, None, 1), (64, 1, 2, 16, None, 1), (64, 2, 2, 16, None, 1), (64, 1, 2, 16, None, 2), (128, 1, 1, 16, None, 1), (128, 1, 2, 16, None, 2),
+    (64, 2, 1, 16, 700, 1), (128, 1, 1, 16, 700, 1), (64, 1, 1, 5, None, 1), (64, 2, 2, 5, None, 1), (64, 1, 1, 5, 30, 1), (48, 1, 1, 16, None, 1)])
+@pytest.mark.parametrize("at", [3, 440, 860])
+def test_a_key_that_is_no_number(hd, blocks, groups, ps, window, nsplit, at):
+    """Every row that reads it is no number either, the others (before it, past their window, of the other key head) are what they are without it."""
+    def plant(q, k, v):
+        if len(k) > at:
+            k[at, 0, 7] = float("nan")
+    assert worst_excess(((150, 900), (60, 60), (1, 500)), 4, 2, hd, ps, blocks, groups, nsplit, window, seed=9, plant=plant) <= 0.0
+
+
 @pytest.mark.parametrize("blocks,groups", [(1, 1), (2, 1), (2, 2)])
 def test_a_workgroup_goes_from_a_tile_that_is_made_again_to_the_next(blocks, groups):
     assert worst_excess(((1530, 1530),), 32, 8, 64, 16, blocks, groups, seed=7, plant=planted(120.0, 1000, 701)) <= 0.0
