@@ -42,7 +42,8 @@ __device__ __forceinline__ void load_rows_to_lds(const char* k, const char* v, u
     asm volatile(
         "s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %4, %0\n\tglobal_load_lds_dwordx4 %5, %0 offset:1024\n\t"
         "s_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %6, %1\n\tglobal_load_lds_dwordx4 %7, %1 offset:1024"
-        ::"s"(k), "s"(v), "s"(k_to), "s"(v_to), "v"(k0), "v"(k1), "v"(v0), "v"(v1));
+        ::"s"(k), "s"(v), "s"(k_to), "s"(v_to), "v"(k0), "v"(k1), "v"(v0), "v"(v1)
+        : "m0");
 }
 
 // A barrier that waits for LDS only, not for loads on their way
