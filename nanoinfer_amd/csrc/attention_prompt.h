@@ -3,7 +3,8 @@
 //
 // Keys and values go from memory straight into LDS, a page's rows by one wavefront, whose page number and addresses are scalars: no vector
 // instruction works out where rows lie (sixteen a set of 32 keys there) and no row waits in registers (219 of them at most, 253 there).
-// Stages go through a ring of three slots; the next tile's first ones are asked for while this one's last are multiplied.
+// Stages go through a ring of three slots: the one whose scores are taken, the one before it, whose values are still read, and one on its way (two where
+// a walk starts); the next tile's first are asked for while this one's last are multiplied.
 //
 // Inside the key range of all its rows a set of 32 keys is not looked at for scores that rise above the row's reference (four maxima, a
 // comparison and a branch a block there): the reference is the largest score of the tile's first set (with a window: of its first sets), and
@@ -33,7 +34,7 @@
 #pragma once
 #include "lds_load.h"
 
-#define PA_RING 3          // stages of keys and values in LDS: one that is multiplied, two on their way
+#define PA_RING 3          // stages of keys and values in LDS: the current one, the one before it and one on its way
 
 // 2 KB of K and 2 KB of V straight into LDS at k_to and v_to, sixteen bytes a lane: lane l brings the bytes at lane offset k0 (and k1, 1,024 bytes
 // further on, where they also land).  Addresses in scalar registers are the same in all lanes.  (In assembly: behind the builtin every read of
@@ -234,14 +235,14 @@ void prompt_attention_kernel(
         ++ahead;
         slot_in = slot_in == LAST_SLOT ? 0 : slot_in + SLOT;
     };
-    auto fill = [&]() {                                      // two stages on their way, if there are any, and the next to ask for
+    auto fill = [&]() {                                      // where nobody reads the ring: two stages on their way, if there are any, and the next to ask for
         find();
         while (ahead < 2 && asks) {
             ask();
             find();
         }
     };
-    // this wavefront's loads of the next stage to take have landed
+    // this wavefront's loads of the next stage to take have landed (a stage behind it is on its way only where a walk starts)
     auto landed = [&]() {
         if (ahead > 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LOADS) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

@@ -64,7 +64,8 @@ def worst_excess(portions, H, KVH, hd, ps, blocks=1, groups=1, nsplit=1, window=
 @pytest.mark.parametrize("hd,H,KVH,blocks,groups", [(64, 4, 1, 1, 1), (64, 8, 2, 2, 1), (64, 4, 1, 2, 2), (64, 5, 1, 1, 2), (128, 3, 1, 1, 1), (128, 4, 2, 1, 2)])
 @pytest.mark.parametrize("portions,ps", [
     (((1, 1),), 16), (((31, 31), (33, 64), (2, 65)), 16), (((63, 63),), 32), (((64, 64), (65, 65)), 64), (((40, 127), (9, 129)), 16),
-    (((17, 191), (1, 192), (1, 193), (1, 7)), 16), (((130, 500),), 256), (((20, 20480 + 40),), 16)])
+    (((17, 191), (1, 192), (1, 193), (1, 7)), 16), (((130, 500),), 256), (((20, 20480 + 40),), 16),
+    (((31, 31), (33, 64), (2, 65), (1, 9)), 8), (((40, 127), (9, 129), (70, 500)), 8)])
 def test_ends_of_stages_and_pages(hd, H, KVH, blocks, groups, portions, ps):
     assert worst_excess(portions, H, KVH, hd, ps, blocks, groups, seed=hd + blocks) <= 0.0
 
