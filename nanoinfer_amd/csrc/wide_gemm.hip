@@ -29,8 +29,8 @@
 // Measured (us, the library's product and the SwiGLU kernel : this; kernels/tile.py has more): [16384, 2048] with SwiGLU at 512 / 1,024 / 1,999 / 4,096 rows
 // 44 : 36, 68 : 58, 121 : 111, 239 : 211; [2048, 8192] at 1,999 70 : 62.  Of [16384, 2048] at 1,999 rows the library's product alone takes 105: what is ahead is the
 // epilogue.  17 to 64 rows on a head of [128256, 2048], where W streams from memory once and 64 rows of x from the caches for every tile: tiles of 64 x 128, two a
-// unit so that one's start and stores go beside the other's stages, 118.8 us at 32 rows and 127.9 at 64 (the library's 125.1 and 133.8; tiles of 64 x 256 in rings of three
-// or four slots 124 and 135); on longer rows 64 x 256 ([128256, 3072] 144.6 and 154.7, the library's 162.1 and 181.4).
+// unit so that one's start and stores go beside the other's stages, 115.8 us at 32 rows and 124.1 at 64 (the library's 120.9 and 130.6; tiles of 64 x 256 119.5
+// and 129.6); on rows of 2,304 to 3,584 elements 64 x 256 ([128256, 3072] 150.7 and 160.7, the library's 167.7 and 184.9).
 // Its loop runs at 1.42 PFLOP/s (kernels/tile.py: 1.509 us for 64 columns with all units at work), the launch at 1.2, and 1.1 to 1.2 inside a prompt: two rounds of
 // one workgroup a unit, whose first loads and stores nothing covers.  In the loop it is the clock: alone, matrix cores busy 64 % of the time at 1.9 GHz
 // (the library's 65 % at 1.96; with operands of ones, which switch less, 2.3 GHz and 88 us; without its loads the same kernel takes 103), in a prompt of 2,048

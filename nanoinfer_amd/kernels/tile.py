@@ -573,21 +573,36 @@ def wide_takes(M: int, K: int, rows: torch.Tensor, gated: bool = False, to: str 
 
 
 WIDE_FEW_COLUMNS = 32000
+WIDE_FEW_ROUND = 65536       # columns that the chip holds tiles of at once: two tiles of 128 a unit, or one of 256
 
 
 def wide_few_wins(M: int, K: int, rows: torch.Tensor) -> bool:
-    """Whether 17 to 64 plain bfloat16 rows go to :func:`wide_gemm` on a matrix as stored, as the head over the vocabulary is, with float32 results: from as
-    many columns and in the lengths of row measured, where the library streams the matrix no faster (us, library : this, 24 / 32 / 48 / 64 rows: [128256, 2048]
-    123.2 : 117.1, 125.1 : 118.8, 128.8 : 121.6, 133.8 : 127.9; [128256, 3072] 159 : 142, 162 : 145, 171 : 151, 181 : 155; [128256, 4096] 204 : 195, 207 : 198,
-    216 : 197, 219 : 199; [32000, 2048] 22.7 : 22.3, 22.8 : 22.4, 25.3 : 22.8, 24.2 : 23.5)."""
+    """Whether 17 to 64 plain bfloat16 rows go to :func:`wide_gemm` on a matrix as stored, as the head over the vocabulary is, with float32 results: where
+    the tiles fill their rounds, as far as the library does no better.  Measured with matrices that the caches do not hold (us, library : this, 17 / 32 / 64 rows):
+    rows of 2,048: 32,000 columns 30.9 : 31.1, 31.0 : 31.2, 32.4 : 32.2; 36,864 39.9 : 43.4, 40.7 : 45.1, 41.9 : 47.1; 49,152 49.3 : 47.9, 50.0 : 48.5, 53.9 : 51.2;
+    128,256 118.5 : 112.2, 120.9 : 115.8, 130.6 : 124.1.  4,096: 32,000 61.3 : 63.0, 61.8 : 63.6, 63.8 : 64.3; 66,560 122.5 : 134.1, 125.1 : 135.8, 131.1 : 144.6; 128,256
+    202.5 : 203.8, 208.4 : 209.6, 223.9 : 223.1; 131,072 234.8 : 191.7, 241.8 : 195.5, 254.3 : 204.3.  3,072: 32,000 38.9 : 52.2, 39.3 : 54.1, 40.6 : 58.4; 65,536
+    76.2 : 75.4, 79.0 : 79.0, 83.5 : 84.4; 66,560 131.0 : 105.6, 130.6 : 109.6, 92.1 : 120.3; 100,352 191.9 : 118.6, 192.4 : 123.1, 153.5 : 133.5; 128,256 161.3 : 144.7,
+    167.7 : 150.7, 184.9 : 160.7.  3,584: 151,936 249.6 : 213.5, 261.9 : 217.9, 224.7 : 232.9."""
     N = rows.shape[0]
-    return (16 < M <= 64 and N >= WIDE_FEW_COLUMNS and 2048 <= K <= 4096 and K % 64 == 0 and N % 16 == 0 and N * K < 1 << 30
-            and rows.dtype == torch.bfloat16 and rows.dim() == 2 and rows.is_contiguous() and rows.data_ptr() % 16 == 0)
+    if not (16 < M <= 64 and N >= WIDE_FEW_COLUMNS and 2048 <= K <= 4096 and K % 64 == 0 and N % 16 == 0 and N * K < 1 << 30
+            and rows.dtype == torch.bfloat16 and rows.dim() == 2 and rows.is_contiguous() and rows.data_ptr() % 16 == 0):
+        return False
+    if K == 2048:
+        return N <= 32768 or N >= 49152
+    rounds, last = divmod(N - 1, WIDE_FEW_ROUND)       # full rounds, and the last column of the round behind them
+    if K == 4096:
+        return N >= 49152 and (rounds != 1 or last >= 24576)
+    if last >= 49151:
+        return True
+    # a round that is not full: up to 32 rows the library is far behind
+    return rounds >= 1 and (M <= 32 or last >= 32767) if K <= 3072 else rounds >= 2 and M <= 32 and last < 32767
 
 
 def wide_few_tile(K: int) -> int:
-    """Its tile: two workgroups a unit (64 x 128) on rows of 2,048 elements, one of twice the columns on longer ones."""
-    return 5 if K <= 2048 else 6
+    """Its tile: two workgroups a unit (64 x 128) on rows of 2,048 or 4,096 elements, one of twice the columns on those between (us, 64 x 128 : 64 x 256 on 128,256
+    columns at 32 rows: 2,048 115.8 : 119.5, 2,560 133.7 : 128.9, 3,072 154.0 : 150.7, 3,584 174.4 : 170.7, 4,096 209.6 : 226.9)."""
+    return 5 if K in (2048, 4096) else 6
 
 
 def wide_stream_ok(M: int, K: int, dtype: torch.dtype, weight) -> bool:
