@@ -179,8 +179,9 @@ NI_EXPORT int ni_input_conv(const void* h, const void* w, void* state, size_t st
     auto run = [&](auto* out) {
         using One = std::integral_constant<int, 1>;
         using Four = std::integral_constant<int, 4>;
-        // (one sequence in blocks of four from 64 rows on: the fewer threads cost less than the launch behind them)
-        if (pieces) T >= 256 || (B == 1 && T >= 64) ? launch(out, std::true_type{}, Four{}) : launch(out, std::true_type{}, One{});
+        // (one sequence in blocks of four from 64 rows on where that moves its tail: the fewer threads cost less than the launch behind them.  100 / 200 rows of
+        // 2,048 channels, four taps 6.7 -> 6.2 us, 8.5 -> 6.2; with seven, whose tail takes that launch, blocks of four are 11.5 and 11.6 for 8.0 and 10.0)
+        if (pieces) T >= 256 || (T >= 64 && tail_move(single != 0, B, 4, taps) == TailMove::Alone) ? launch(out, std::true_type{}, Four{}) : launch(out, std::true_type{}, One{});
         else launch(out, std::false_type{}, One{});
     };
     if (dtype == 0) run((float*)x);
