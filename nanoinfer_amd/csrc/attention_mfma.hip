@@ -171,7 +171,8 @@ __device__ __forceinline__ floatx4_t row_sum_step(const uint4& pf, floatx4_t l) 
 // LDS.  A wavefront alone on a SIMD waits for LDS and its own chain of instructions (0.6 us for a step of
 // 32 keys, two blocks of rows, head size 64; two together take 0.73), and the last tiles of a prompt, its
 // longest, used to run alone.  2,048 tokens at 2,048 keys, 32 heads on 8: 42.6 -> 39.4 us, of which 33 pairs
-// of steps are 24 and the start and end of two tiles 14; 512 at 1,024 17.9 -> 15.3, 1,700 at 1,700 54.3 -> 39.6.
+// of steps are 24 and the start and end of two tiles 14; 512 at 1,024 17.9 -> 15.3, 1,700 at 1,700 54.3 -> 39.6.  (Of this kernel; at head size 64
+// most such portions take the other one now, for which kernels/__init__.py has figures.)
 template <int CB, bool POW2, int GROUPS>
 __global__ __launch_bounds__(GROUPS * MA_WAVES * WAVE) __attribute__((amdgpu_waves_per_eu(HEAD_DIM * CB <= 128 ? 2 : 1)))
 void mfma_attention_kernel(
@@ -821,9 +822,10 @@ void mfma_decode_kernel(
 
 NI_EXPORT int ni_mfma_attention_head_dim() { return HEAD_DIM; }
 
-// Blocks of 16 rows that a wavefront can own at this head size.  Registers set the limit: two
+// Blocks of 16 rows that a wavefront can own at this head size.  Registers set the limit: in mfma_attention_kernel two
 // blocks at head size 128, or four at 64, fit only with the accumulators parked in the accumulation
-// registers and one wavefront a SIMD, and were slower than one block in every case measured.
+// registers and one wavefront a SIMD, and were slower than one block in every case measured.  (The kernel of attention_prompt.h has 216 registers
+// with one block of head size 128; two were not tried.)
 #define MA_MAX_BLOCKS (HEAD_DIM <= 64 ? 2 : 1)
 NI_EXPORT int ni_mfma_attention_max_blocks() { return MA_MAX_BLOCKS; }
 

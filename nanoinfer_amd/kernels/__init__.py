@@ -407,8 +407,8 @@ def mfma_tile_tokens(hd: int, group: int, n_tokens: Optional[int] = None, kv_hea
     but fewer tiles fill the chip less evenly (the kernel pairs long tiles with short ones, in a workgroup
     or over the two workgroups of a compute unit): two blocks are taken where a step of ``n_tokens``
     tokens still has one and a half such tiles for every compute unit (measured at head size 64, one
-    block : two blocks in us: 1,024 tokens 19.8 : 24.0, 1,536 tokens 41.8 : 37.0, 2,048 tokens 44.2 : 43.2,
-    2,560 tokens 100.4 : 78.6, 3,072 tokens 117.2 : 95.3, 4,096 tokens 150.8 : 108.0).  Without ``n_tokens``:
+    block : two blocks in us: 1,024 tokens 17.9 : 20.1, 1,536 tokens 29.9 : 31.2, 2,048 tokens 37.0 : 36.1,
+    2,560 tokens 62.4 : 58.6, 3,072 tokens 76.0 : 67.8, 4,096 tokens 120.6 : 91.5).  Without ``n_tokens``:
     the smallest tile.  The float32 kernel has one tile size."""
     if dtype == torch.float32:
         return _f32_tile_tokens(hd, int(group))
@@ -436,8 +436,8 @@ def mfma_plan(hd: int, group: int, kv_heads: int, n_tokens: int, max_q_len: int,
     keys before it at least as many as its own, judged from ``max_keys`` rounded up to a power of
     two so that a recorded step and its eager twin decide alike): its tiles are then of like length
     and need no pairing, and cutting their keys into runs of 512 or more fills the chip (measured at
-    head size 64: 512 tokens at context 2,048 take 36.8 us with one block and no cut, 30.8 with two
-    blocks and four runs; at context 4,096 68.4 and 45.7)."""
+    head size 64: 512 tokens at context 4,096 take 46.0 us with one block and no cut, 36.0 with two
+    blocks and four runs; at context 2,048, where the kernel before needed the cut too, 25.0 and 27.3)."""
     if dtype == torch.float32:
         return mfma_tile_tokens(hd, group, dtype=dtype), None
     small = mfma_tile_tokens(hd, group)
@@ -464,15 +464,16 @@ def mfma_group_plan(hd: int, group: int, kv_heads: int, n_tokens: int, max_q_len
     whose long tiles outlast the short ones (``max_keys`` rounded up to a power of two, as there).  Measured, that plan : this one,
     us, 32 heads on 8:
     one block of rows and no more than a tile (times runs) for each of the 256 units, from 512 keys on, up to eight times the
-    portion (or 2,048): head size 64, 512 tokens at 512 / 1,024 keys 11.6 : 11.0, 17.9 : 15.3; 256 at 256 / 1,024 / 2,048 8.3 : 8.5, 16.3 : 14.7,
-    22.1 : 19.9; 128 at 2,000 17.4 : 16.2.  (Where :func:`mfma_plan` cuts the keys of tiles of two blocks, that stays: 256 at 4,096
-    28.7 : 28.3, 512 at 4,096 / 6,000 39.0 : 39.8, 50.5 : 54.8; 512 at 1,536 / 2,048 / 3,072, 25.9 : 19.5, 28.3 : 23.4, 33.7 : 31.6, stay with it
-    too, the only portions that bring those runs and their merge through the engine.)  Head size 96, 512 at 768 / 4,096 20.2 : 17.8, 66.1 : 60.5; 128 (24 on 8), 512 at 512 / 1,024 / 2,048 / 8,192
-    17.9 : 18.8, 29.0 : 27.7, 49.7 : 42.5, 140 : 132, 256 at 1,024 / 4,096 24.6 : 26.7, 55.4 : 50.3.
-    Two blocks, one tile a unit, keys twice to four times the portion: 1,024 at 2,048 / 4,096 34.8 : 33.0, 63.5 : 55.3 (700 tokens at 1,400, where
-    176 tiles leave units idle, 27.0 : 30.1).  Two blocks, 1.4 to 3 tiles a unit, long and short ones in turn by one workgroup, keys
-    no more than twice the portion: 1,500 at 1,500 35.2 : 32.6, 1,700 54.3 : 39.6, 1,999 42.6 : 39.0, 3,000 82.3 : 76.7, 2,048 at 4,096 / 6,000
-    86.6 : 84.9, 127 : 133 (four tiles a unit, 4,096 at 4,096, 109 : 119; four portions of 300 at 700 26.7 : 29.6)."""
+    portion (or 2,048): head size 64, 512 tokens at 512 / 1,024 keys 10.1 : 9.8, 15.6 : 13.6; 256 at 256 / 1,024 / 2,048 7.6 : 7.6, 16.2 : 13.0,
+    21.2 : 19.7; 128 at 2,000 16.9 : 16.8.  (Where :func:`mfma_plan` cuts the keys of tiles of two blocks, that stays: 256 at 4,096
+    27.3 : 27.1, 512 at 4,096 / 6,000 36.8 : 36.0, 45.7 : 47.9; 512 at 1,536 / 2,048 / 3,072, 24.9 : 16.9, 26.7 : 21.1, 30.8 : 28.1, stay with it
+    too, the only portions that bring those runs and their merge through the engine.)  Head size 96 (mfma_attention_kernel), 512 at 768 / 4,096 20.2 : 17.8,
+    66.1 : 60.5; 128 (24 on 8), 512 at 512 / 1,024 / 2,048 / 8,192 15.5 : 14.1, 25.4 : 21.3, 43.0 : 33.7, 118 : 113, 256 at 1,024 / 4,096 21.8 : 20.1, 48.8 : 39.5
+    (512 at 512 and 256 at 1,024 are not taken: with that kernel they were no faster).
+    Two blocks, one tile a unit, keys twice to four times the portion: 1,024 at 2,048 / 4,096 30.9 : 28.6, 56.8 : 47.9 (700 tokens at 1,400, where
+    176 tiles leave units idle, 22.6 : 21.1).  Two blocks, 1.4 to 3 tiles a unit, long and short ones in turn by one workgroup, keys
+    no more than twice the portion: 1,500 at 1,500 29.1 : 28.0, 1,700 36.9 : 31.2, 1,999 35.5 : 33.6, 3,000 66.4 : 64.1, 2,048 at 4,096 / 6,000
+    72.4 : 71.2, 109 : 110 (four tiles a unit, 4,096 at 4,096, 89.8 : 99.9; four portions of 300 at 700 23.0 : 24.7)."""
     if dtype != torch.bfloat16 or n_tokens != max_q_len or not 32 < hd <= 128:
         return None
     small = mfma_tile_tokens(hd, group)
@@ -570,8 +571,8 @@ def mfma_splits(n_tiles: int, kv_heads: int, group: int, max_keys: int, hd: int 
     second kernel that merges the runs, and float32 partial results in between: a step with many
     tiles is cut only into runs of 2,048 keys or more, up to about a thousand workgroups (measured
     for portions of 512 tokens at contexts of 512 to 8,192), and not at all once it has two tiles for
-    every compute unit (2,048 tokens in tiles of 32 at contexts of 4,096 / 8,192 / 32,768: 88 / 180 / 721 us
-    uncut, 99 / 192 / 741 in two runs; 1,024 tokens, one tile a unit: 75 / 142 uncut, 64 / 114 in two);
+    every compute unit (2,048 tokens in tiles of 32 at contexts of 4,096 / 8,192 / 32,768: 76 / 151 / 603 us
+    uncut, 89 / 164 / 619 in two runs; 1,024 tokens, one tile a unit, at 4,096 / 8,192: 58 / 108 uncut, 56 / 94 in two);
     a step with fewer tiles than the chip has compute units, into runs of 512 keys or more until
     every unit has one.
 
