@@ -17,20 +17,21 @@
 //
 // The scores of a set are taken while the set before it gets its weights (at head size 128 a step of 32 keys is 25 % faster by it), so that the
 // matrix cores work beside the vector unit's exponentials.  At the ends of a walk, and where scores are looked at, head size 64 takes a stage's two
-// sets side by side: one at a time, short walks were slower than mfma_attention_kernel's (128 tokens at 228 keys 7.5 us there, 8.4 one at a time, 7.6
-// side by side; 16 heads on 16, 256 at 256 7.4, 8.6, 7.7; 512 at 512 10.1, 10.5, 9.6).
+// sets side by side: one at a time, short walks were slower than mfma_attention_kernel's (128 tokens at 228 keys 7.5 us there, 8.4 one at a time, 7.5
+// side by side; 16 heads on 16, 256 at 256 7.4, 8.6, 7.7; 512 at 512 10.2, 10.5, 9.6).
 //
 // What bounds it: at long key ranges neither of the two (matrix cores busy 41 %, the vector unit 50 % of the cycles, two wavefronts a SIMD with
-// a chain of instructions each); in one prompt of 2,000 tokens starts and ends: of 79,000 cycles of a workgroup's two tiles 9,000 pass before the first
-// keys are there, 8,000 between the tiles, 5,000 behind the last.
+// a chain of instructions each); in one prompt of 2,000 tokens starts and ends: of 79,000 cycles of a workgroup's two tiles 9,000 passed before the first
+// keys were there, 8,000 between the tiles, 5,000 behind the last (75,000 in all with a stage's sets side by side).
 //
-// Measured, mfma_attention_kernel : this, us: 32 heads of 64 on 8, 512 tokens at 512 / 1,024 keys 10.5 : 10.4, 15.3 : 14.3; 700 at 700 16.6 : 14.7; 1,024 at
-// 1,024 / 4,096 19.4 : 17.9, 55.8 : 51.7; 1,999 at 1,999 40.5 : 37.6; 4,096 at 4,096 114.6 : 98.3; 2,048 at 8,192 / 32,768 171.9 : 146.1, 692.7 : 588.8;
-// 24 of 128 on 8, 256 at 256 11.9 : 10.4; 512 at 512 / 2,048 18.1 : 15.4, 43.1 : 33.8; 1,999 at 1,999 80.8 : 60.9; 2,048 at 8,192 415.8 : 309.9.
+// Measured, mfma_attention_kernel : this, us: 32 heads of 64 on 8, 512 tokens at 512 / 1,024 keys 10.5 : 9.6, 14.9 : 13.2; 700 at 700 16.3 : 13.9; 1,024 at
+// 1,024 / 4,096 18.5 : 16.6, 54.6 : 48.2; 1,999 at 1,999 38.3 : 33.8; 4,096 at 4,096 106.4 : 88.5; 2,048 at 8,192 / 32,768 170.7 : 142.8, 689.4 : 575.5;
+// 24 of 128 on 8, 256 at 256 11.9 : 10.3; 512 at 512 / 2,048 17.3 : 14.9, 41.8 : 32.1; 1,999 at 1,999 75.1 : 54.5; 2,048 at 8,192 423.7 : 305.5.  Behind it
+// by 2 to 4 % are few tokens of head size 64 at 1,500 to 2,000 keys in runs (100 at 2,000 15.6 : 16.0) and 256 of 16 heads on 16 (7.4 : 7.7).
 //
 // A single token beside the portions of a step walked its keys by one wavefront of four, as long as the portions' tiles: its four wavefronts
 // now share them out as in the kernel for single tokens (attend_token), where it has a workgroup to itself.  481 tokens beside 31 with 100 to 1,100
-// keys 18.8 : 14.6 us.
+// keys 18.6 : 14.4 us.
 #pragma once
 #include "lds_load.h"
 
